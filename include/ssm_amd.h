@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define SSM_AMD_ABI_VERSION 8
+#define SSM_AMD_ABI_VERSION 9
 
 typedef enum ssm_status {
   SSM_OK = 0,
@@ -750,6 +750,9 @@ typedef struct ssm_norm_bwd_args {
   int32_t rows, hidden;
   int32_t x_dtype, residual_dtype;
   int32_t is_rms, prenorm;
+  const void *grad_residual_out; /* (rows, hidden) gradient of residual_out, or NULL: added to dx, and to dresidual
+                                    when prenorm */
+  int32_t grad_residual_out_dtype;
 } ssm_norm_bwd_args;
 
 size_t ssm_norm_bwd_workspace_bytes(int rows, int hidden);

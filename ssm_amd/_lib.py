@@ -19,7 +19,7 @@ import os
 # SSM_AMD_LIB points the binding at another build of the same C ABI.
 LIB_PATH = Path(os.environ.get("SSM_AMD_LIB") or
                 Path(__file__).resolve().parent / "lib" / "libssm_amd.so")
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 SSM_F32, SSM_BF16, SSM_F16 = 0, 1, 2
 PROJ_DN, PROJ_BDN, PROJ_BGNL = 0, 1, 2
@@ -275,7 +275,7 @@ class NormBwdArgs(C.Structure):
         ("dx", _vp), ("dresidual", _vp), ("dweight", _vp), ("dbias", _vp),
         ("workspace", _vp), ("workspace_bytes", C.c_size_t),
         ("rows", _i32), ("hidden", _i32), ("x_dtype", _i32), ("residual_dtype", _i32),
-        ("is_rms", _i32), ("prenorm", _i32),
+        ("is_rms", _i32), ("prenorm", _i32), ("grad_residual_out", _vp), ("grad_residual_out_dtype", _i32),
     ]
 
 

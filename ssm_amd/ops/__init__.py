@@ -970,15 +970,22 @@ def _norm_forward(x, weight, bias, residual, is_rms, eps, prenorm, residual_in_f
 
 
 def _norm_backward(grad_out, x, weight, residual, mean, rstd, is_rms, prenorm, want_dbias, want_dres,
-                   out=None):
-    """``ssm_norm_bwd``.  With ``out = (dx, dres, dw, db)`` (preallocated, contiguous; ``None`` where a
+                   out=None, grad_residual_out=None):
+    """``ssm_norm_bwd``.  ``grad_residual_out`` is the gradient of ``residual_out = x (+ residual when prenorm)``; the
+    kernel adds it to ``dx`` (and ``dres``).  With ``out = (dx, dres, dw, db)`` (preallocated, contiguous; ``None`` where a
     gradient is not wanted) the call goes to ``ssm_norm_bwd_static`` instead and allocates nothing on
     the device: inputs must then already be contiguous and ``weight`` float32."""
     if K.f64_compute(x):
         if out is not None:
             raise ValueError("the allocation-free norm backward takes float32, bfloat16 or float16 tensors")
         from . import _f64
-        return _f64.norm_backward(grad_out, x, weight, residual, mean, rstd, is_rms, prenorm, want_dbias, want_dres)
+        dx, dres, dw, db = _f64.norm_backward(grad_out, x, weight, residual, mean, rstd, is_rms, prenorm, want_dbias,
+                                              want_dres)
+        if grad_residual_out is not None:
+            dx = dx + grad_residual_out.to(dx.dtype)
+            if dres is not None and prenorm:
+                dres = dres + grad_residual_out.to(dres.dtype)
+        return dx, dres, dw, db
     weight, residual = K.narrow(weight, residual)
     rows, hidden = K.check_norm(x, weight, None, residual)
     if out is not None:
@@ -1001,6 +1008,7 @@ def _norm_backward(grad_out, x, weight, residual, mean, rstd, is_rms, prenorm, w
     dev = K.require_gpu(x, weight, residual, grad_out)
     xc, gc = K.cast_c(x, x.dtype), K.cast_c(grad_out, x.dtype)
     rc = K.cast_c(residual, residual.dtype) if residual is not None else None
+    ro = K.cast_c(grad_residual_out, grad_residual_out.dtype) if grad_residual_out is not None else None
     wf = K.as_f32_vec(weight)
     dx = torch.empty_like(xc)
     dres = torch.empty_like(rc) if (want_dres and rc is not None) else None
@@ -1014,7 +1022,8 @@ def _norm_backward(grad_out, x, weight, residual, mean, rstd, is_rms, prenorm, w
         dbias=_lib.ptr(db), workspace=_lib.ptr(ws), workspace_bytes=nbytes, rows=rows, hidden=hidden,
         x_dtype=_lib.dtype_enum(xc.dtype),
         residual_dtype=_lib.dtype_enum(rc.dtype) if rc is not None else 0,
-        is_rms=int(bool(is_rms)), prenorm=int(bool(prenorm)))
+        is_rms=int(bool(is_rms)), prenorm=int(bool(prenorm)), grad_residual_out=_lib.ptr(ro),
+        grad_residual_out_dtype=_lib.dtype_enum(ro.dtype) if ro is not None else 0)
     _lib.call("ssm_norm_bwd", args, dev)
     return dx, dres, dw, db
 

@@ -62,6 +62,7 @@ class FusedNormFn(torch.autograd.Function):
             res_out = x.new_empty(0)
             ctx.mark_non_differentiable(res_out)
         ctx.has_res_out = want_res_out
+        ctx.set_materialize_grads(False)      # an output that nobody used costs no tensor of zeros
         return y, res_out
 
     @staticmethod
@@ -72,13 +73,12 @@ class FusedNormFn(torch.autograd.Function):
         is_rms, prenorm = ctx.cfg
         need = ctx.needs_input_grad
         want_dres = residual is not None and need[3]
+        if not ctx.has_res_out:
+            grad_res_out = None
+        if grad_y is None:
+            grad_y = torch.zeros_like(x)
         dx, dres, dw, db = _norm_backward(grad_y.contiguous(), x, weight, residual, mean, rstd, is_rms,
-                                          prenorm, bias is not None, want_dres)
-        if ctx.has_res_out and grad_res_out is not None and grad_res_out.numel() == x.numel():
-            # residual_out = x (+ residual when prenorm): its gradient flows straight through
-            dx = dx + grad_res_out.to(dx.dtype)
-            if dres is not None and prenorm:
-                dres = dres + grad_res_out.to(dres.dtype)
+                                          prenorm, bias is not None, want_dres, grad_residual_out=grad_res_out)
         return (_like(dx, x) if need[0] else None,
                 _like(dw, weight) if need[1] else None,
                 _like(db, bias) if (bias is not None and need[2]) else None,

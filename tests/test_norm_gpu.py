@@ -153,3 +153,29 @@ def test_postnorm_backward_with_a_residual_that_needs_no_gradient(is_rms):
     yr.backward(gy.float())
     torch.testing.assert_close(xg.grad.float().cpu(), xr.grad, rtol=2e-2, atol=2e-2)
     torch.testing.assert_close(wg.grad.cpu(), wr.grad, rtol=2e-2, atol=2e-2 * float(wr.grad.abs().max()))
+
+
+@pytest.mark.parametrize("dtype,res_dtype,hidden", [
+    (torch.bfloat16, torch.float32, 768), (torch.bfloat16, torch.bfloat16, 1028), (torch.float32, None, 100),
+    (torch.bfloat16, None, 256), (torch.float16, torch.bfloat16, 64), (torch.float32, torch.float32, 8200), (torch.bfloat16, torch.float32, 37)])
+@pytest.mark.parametrize("prenorm", [True, False])
+def test_gradient_through_residual_out_is_added_in_the_backward_kernel(dtype, res_dtype, hidden, prenorm):
+    """``residual_out = x (+ residual when prenorm)`` hands its gradient straight on: to ``dx``, and to the residual's
+    when it was added before the norm -- for typed kernels (one type for residual and that gradient), mixed types,
+    rows that are no multiple of four columns and rows beyond the register kernels."""
+    g = torch.Generator().manual_seed(hidden)
+    x, w = torch.randn(2, 5, hidden, generator=g).to(dtype), torch.randn(hidden, generator=g)
+    r = None if res_dtype is None else torch.randn(2, 5, hidden, generator=g).to(res_dtype)
+    gy, gr = torch.randn(2, 5, hidden, generator=g).to(dtype), torch.randn(2, 5, hidden, generator=g)
+    xg, rg = x.cuda().requires_grad_(), None if r is None else r.cuda().requires_grad_()
+    y, ro = _ops().fused_layer_norm_with_residual(xg, w.cuda(), None, residual=rg, is_rms=True, prenorm=prenorm)
+    got = torch.autograd.grad([y, ro], [xg] + ([] if r is None else [rg]), [gy.cuda(), gr.cuda()])
+    xd, rd = x.double().requires_grad_(), None if r is None else r.double().requires_grad_()
+    s = xd if r is None or not prenorm else xd + rd
+    out = s * torch.rsqrt((s * s).mean(-1, keepdim=True) + 1e-5) * w.double()
+    if r is not None and not prenorm:
+        out = out + rd
+    want = torch.autograd.grad([out, s], [xd] + ([] if r is None else [rd]), [gy.double(), gr.double()])
+    for a, b, t in zip(got, want, (x, r)):
+        tol = 1e-5 if t.dtype == torch.float32 else 2e-2
+        torch.testing.assert_close(a.double().cpu(), b, rtol=tol, atol=tol)
