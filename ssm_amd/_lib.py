@@ -8,6 +8,7 @@ or a call returns a non-zero status, an exception is raised.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import threading
 from pathlib import Path
 from typing import Optional
@@ -398,6 +399,32 @@ HOOKS_SYMBOLS = {
 }
 HOOKS_LIB_PATH = LIB_PATH.with_name("libssm_amd_testhooks.so")
 
+# The native host path of repeated calls (csrc/host/host.cpp), an extension module beside the library.
+HOST_PATH = Path(__file__).resolve().parent / "lib" / "_host.so"
+
+
+class _HostMissing:
+    """Stands in for the module where it cannot be loaded: every call says so."""
+
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise BackendUnavailable(f"{HOST_PATH.name}: {self._why}; build it with `python -m ssm_amd.build`")
+
+
+def _load_host():
+    try:
+        spec = importlib.util.spec_from_file_location("_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        return mod
+    except (ImportError, OSError) as exc:
+        return _HostMissing(exc)
+
+
+host = _load_host()
+
 _lock = threading.Lock()
 _libs: dict = {}                     # hooks? -> CDLL
 _load_errors: dict = {}              # hooks? -> Exception
@@ -433,7 +460,10 @@ def _load(hooks: bool) -> C.CDLL:
         if hooks in _load_errors:
             raise BackendUnavailable(str(_load_errors[hooks]))
         try:
-            _libs[hooks] = _bind(HOOKS_LIB_PATH if hooks else LIB_PATH, hooks)
+            lib = _bind(HOOKS_LIB_PATH if hooks else LIB_PATH, hooks)
+            if hooks == (_hooks_active > 0) and not isinstance(host, _HostMissing):
+                host.bind(lib._handle, KernelError)
+            _libs[hooks] = lib
         except Exception as exc:  # remembered: a broken install stays broken
             _load_errors[hooks] = exc
             raise BackendUnavailable(str(exc)) from exc
@@ -459,13 +489,15 @@ class test_hooks_build:
 
     def __enter__(self):
         global _hooks_active
-        load_test_hooks()
+        lib = load_test_hooks()
         _hooks_active += 1
-        return _libs[True]
+        host.bind(lib._handle, KernelError)
+        return lib
 
     def __exit__(self, *exc):
         global _hooks_active
         _hooks_active -= 1
+        host.bind(load()._handle, KernelError)
         return False
 
 

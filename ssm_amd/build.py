@@ -7,6 +7,9 @@ A second library, ``libssm_amd_testhooks.so``, is linked from the same objects
 except that the sources which pick between kernels are compiled once more with
 ``-DSSM_TEST_HOOKS`` (``include/ssm_amd_testing.h``): the test suite uses it to
 run a chosen kernel where the shipped library would pick another.
+
+A third, ``_host.so``, is a Python extension module (C++ against torch, no device code): the host path of repeated
+operator calls (``csrc/host/host.cpp``).  It calls the C ABI of whichever library ``ssm_amd._lib`` binds it to.
 """
 
 from __future__ import annotations
@@ -14,6 +17,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -22,6 +26,8 @@ CSRC = PKG / "csrc"
 OBJ = PKG / "lib" / "obj"
 LIB = PKG / "lib" / "libssm_amd.so"
 HOOKS_LIB = PKG / "lib" / "libssm_amd_testhooks.so"
+HOST_SRC = CSRC / "host" / "host.cpp"
+HOST_LIB = PKG / "lib" / "_host.so"
 # the sources that read a kernel selector (SSM_RESERVED) or record the kernel taken
 HOOKED = ("scan_fwd.hip", "scan_bwd.hip", "dscan_bwd.hip", "ssd.hip")
 
@@ -55,8 +61,24 @@ def _compile(src: Path, extra: list[str], suffix: str = "") -> Path:
     return obj
 
 
+def _build_host() -> None:
+    """The extension module of the host path; plain C++, so the host compiler builds it."""
+    from torch.utils import cpp_extension
+
+    rocm = Path(hipcc()).resolve().parent.parent
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"],
+           next(str(d) for d in (rocm / "include", Path("/opt/rocm/include")) if (d / "hip").is_dir())]
+    libs = cpp_extension.library_paths()
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", *(f"-I{d}" for d in inc), str(HOST_SRC), "-o", str(HOST_LIB), *(f"-L{d}" for d in libs),
+           "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", *(f"-Wl,-rpath,{d}" for d in libs)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on {HOST_SRC.name}:\n{proc.stderr}")
+
+
 def build(verbose: bool = True, extra: list[str] | None = None, jobs: int | None = None) -> Path:
-    """Compile every ``csrc/*.hip`` for gfx950 and link the shared library."""
+    """Compile every ``csrc/*.hip`` for gfx950, link the shared libraries, and build the host path's module."""
     OBJ.mkdir(parents=True, exist_ok=True)
     srcs = sources()
     if not srcs:
@@ -66,7 +88,9 @@ def build(verbose: bool = True, extra: list[str] | None = None, jobs: int | None
     hooked = [s for s in srcs if s.name in HOOKED]
     tasks = [(s, extra, "") for s in srcs] + [(s, [*extra, "-DSSM_TEST_HOOKS"], "_hooks") for s in hooked]
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_build_host)
         done = list(pool.map(lambda t: _compile(*t), tasks))
+        host.result()
     objs, hook_objs = done[:len(srcs)], dict(zip((s.name for s in hooked), done[len(srcs):]))
     for lib, parts in ((LIB, objs), (HOOKS_LIB, [hook_objs.get(s.name, o) for s, o in zip(srcs, objs)])):
         cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(lib), *map(str, parts)]
@@ -74,7 +98,7 @@ def build(verbose: bool = True, extra: list[str] | None = None, jobs: int | None
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
     if verbose:
-        print(f"built {LIB} and {HOOKS_LIB.name} from {len(srcs)} sources")
+        print(f"built {LIB}, {HOOKS_LIB.name} and {HOST_LIB.name} from {len(srcs) + 1} sources")
     return LIB
 
 

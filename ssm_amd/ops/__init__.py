@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
+from .._lib import host as _native
 from . import _contract as K
 from ._contract import DeviceError
 
@@ -97,70 +98,36 @@ class ScanPlan:
         _lib.call("ssm_scan_fwd", self.args, self.device)
         return self.out, self.last
 
+    def remember(self, *call):
+        """Let later calls of this form (the tensors the plan was made from, ``softplus``) skip the plan."""
+        _native.selective_scan(_SCAN_FORMS, bytes(self.args), *call, self.last is not None)
+
 
 # Argument structs of calls that were validated before, by everything the validation looks at: a repeated call of
-# the same form (a block calls with one form for its whole life) fills in its pointers and goes.
-_SCAN_FORMS = {}
-_F32 = torch.float32
+# the same form (a block calls with one form for its whole life) fills in its pointers and goes, in native code
+# (csrc/host/host.cpp; one dict per operator, which says what the form is known by).  Calls the native path does not
+# take -- a form not seen yet, tensors that need a cast or a copy first -- go the long way below, which also produces
+# the error messages.
+_SCAN_FORMS, _STEP_FORMS, _DECODE_FORMS, _MAMBA2_FORMS, _WINDOW_FORMS = {}, {}, {}, {}, {}
+_CONV_FORMS, _NORM_FORMS, _CHUNK_FORMS = {}, {}, {}
 
 
-def _scan_forward_again(u, delta, A, B, C, D, z, dt_bias, softplus, want_state):
-    """The call through a struct remembered from an earlier call of the same form, or ``None`` if this form is new
-    or any tensor needs a cast or a copy first (those go the long way, which also produces the error messages)."""
-    dt = u.dtype
-    if not (K.on_gpu(u) and delta.dtype == dt and A.dtype == _F32 and B.dtype == C.dtype and u.is_contiguous()
-            and delta.is_contiguous() and A.is_contiguous() and B.is_contiguous() and C.is_contiguous()):
-        return None
-    for t, want in ((D, _F32), (z, dt), (dt_bias, _F32)):
-        if t is not None and not (t.dtype == want and t.is_contiguous()):
-            return None
-    if (u.data_ptr() | delta.data_ptr() | B.data_ptr() | C.data_ptr() | (0 if z is None else z.data_ptr())) & 15:
-        return None                      # a view off the 16-byte grid: the long way copies it
-    dev = u.device
-    key = (u.shape, dt, delta.shape, A.shape, B.shape, B.dtype, C.shape, None if D is None else D.shape,
-           None if z is None else z.shape, None if dt_bias is None else dt_bias.shape, bool(softplus),
-           bool(want_state), dev.index)
-    form = _SCAN_FORMS.get(key)
-    if form is None:
-        return None
-    for t in (delta, A, B, C, D, z, dt_bias):
-        if t is not None and t.device != dev:
-            return None
-    args = _lib.ScanFwdArgs.from_buffer_copy(form)
-    out = torch.empty_like(u)
-    last = torch.empty((u.shape[0], u.shape[1], A.shape[1]), dtype=dt, device=dev) if want_state else None
-    args.u, args.delta, args.A, args.Bproj, args.Cproj, args.out = (u.data_ptr(), delta.data_ptr(), A.data_ptr(),
-                                                                    B.data_ptr(), C.data_ptr(), out.data_ptr())
-    args.Dskip = None if D is None else D.data_ptr()
-    args.z = None if z is None else z.data_ptr()
-    args.dt_bias = None if dt_bias is None else dt_bias.data_ptr()
-    args.last_state = None if last is None else last.data_ptr()
-    _lib.call("ssm_scan_fwd", args, dev)
-    return out, last, key
+def _needs_graph(*tensors):
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
 def _scan_forward(u, delta, A, B, C, D, z, dt_bias, softplus, want_state, tune_items=0):
     """Validate, normalise dtypes/layout, and run ``ssm_scan_fwd``."""
-    if not tune_items:
-        again = _scan_forward_again(u, delta, A, B, C, D, z, dt_bias, softplus, want_state)
-        if again is not None:
-            return again[0], again[1]
+    if not tune_items and not _needs_graph(u, delta, A, B, C, D, z, dt_bias):
+        got = _native.selective_scan(_SCAN_FORMS, None, u, delta, A, B, C, D, z, dt_bias, softplus, want_state)
+        if got is not None:
+            return got if want_state else (got, None)
     plan = ScanPlan(u, delta, A, B, C, D, z, dt_bias, softplus, want_state, tune_items)
     out, last = plan.run()
     if plan.f64 is not None:
         return out, last
-    if not tune_items and plan.chunk_states is None and len(_SCAN_FORMS) < 256:
-        # remembered under the key that _scan_forward_again forms from the caller's tensors: only a call whose
-        # tensors went in as they were (no cast, no copy) can be repeated through it
-        k = plan.keep
-        same = all(a is None or b is None or a.data_ptr() == b.data_ptr()
-                   for a, b in ((u, k["u"]), (delta, k["delta"]), (z, k["z"]), (B, k["B"]), (C, k["C"]), (A, k["A"]),
-                                (D, k["D"]), (dt_bias, k["bias"])))
-        if same and K.on_gpu(u):
-            key = (u.shape, u.dtype, delta.shape, A.shape, B.shape, B.dtype, C.shape, None if D is None else D.shape,
-                   None if z is None else z.shape, None if dt_bias is None else dt_bias.shape, bool(softplus),
-                   bool(want_state), u.device.index)
-            _SCAN_FORMS[key] = bytes(plan.args)
+    if not tune_items:
+        plan.remember(u, delta, A, B, C, D, z, dt_bias, softplus)
     if out.dtype != plan.result_dtype:
         out = out.to(plan.result_dtype)
         last = last.to(plan.result_dtype) if last is not None else None
@@ -301,8 +268,10 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, dt_bias=None, softplus=Fal
     Returns:
         ``(B, D, L)`` tensor in ``u.dtype``, or ``(output, last_state)``.
     """
-    tensors = (u, delta, A, B, C, D, z, dt_bias)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    got = _native.selective_scan(_SCAN_FORMS, None, u, delta, A, B, C, D, z, dt_bias, softplus, return_last_state)
+    if got is not None:
+        return got
+    if _needs_graph(u, delta, A, B, C, D, z, dt_bias):
         from ._autograd import SelectiveScanFn
         out, last = SelectiveScanFn.apply(u, delta, A, B, C, D, z, dt_bias, bool(softplus),
                                           bool(return_last_state))
@@ -418,45 +387,6 @@ def _state_step_backward(grad_out, grad_state, state, x, dt, A, B, C, D, z, dt_b
     return dstate, dx, ddt, dA, dB, dC, dD, dz, dbias
 
 
-# Argument structs of state steps that were validated before, keyed by everything the validation looks at (as
-# _SCAN_FORMS for the scan): a decoding loop calls with one form for its whole life, a new token's tensors each time.
-_STEP_FORMS = {}
-
-
-def _state_step_again(state, x, dt, A, B, C, D, z, dt_bias, softplus):
-    """The step through a struct remembered from an earlier call of the same form, or ``None`` if the form is new or
-    a tensor would need a cast, a copy or a batch stride first (those go the long way)."""
-    io = x.dtype
-    if not (K.on_gpu(state) and dt.dtype == io and A.dtype == _F32 and B.dtype == C.dtype and state.is_contiguous()
-            and x.is_contiguous() and dt.is_contiguous() and A.is_contiguous() and B.is_contiguous() and C.is_contiguous()):
-        return None
-    for t, want in ((D, _F32), (z, io), (dt_bias, _F32)):
-        if t is not None and not (t.dtype == want and t.is_contiguous()):
-            return None
-    if (state.data_ptr() | x.data_ptr() | dt.data_ptr() | A.data_ptr() | B.data_ptr() | C.data_ptr()
-            | (0 if z is None else z.data_ptr()) | (0 if D is None else D.data_ptr())
-            | (0 if dt_bias is None else dt_bias.data_ptr())) & 15:
-        return None
-    dev = state.device
-    key = (state.shape, state.dtype, x.shape, io, A.shape, B.shape, B.dtype, C.shape, D is None or D.shape,
-           z is None or z.shape, dt_bias is None or dt_bias.shape, bool(softplus), dev.index)
-    form = _STEP_FORMS.get(key)
-    if form is None:
-        return None
-    for t in (x, dt, A, B, C, D, z, dt_bias):
-        if t is not None and t.device != dev:
-            return None
-    args = _lib.StateStepArgs.from_buffer_copy(form)
-    out = torch.empty_like(x)
-    args.state, args.x, args.dt, args.A, args.Bproj, args.Cproj, args.out = (
-        state.data_ptr(), x.data_ptr(), dt.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr(), out.data_ptr())
-    args.z = None if z is None else z.data_ptr()
-    args.Dskip = None if D is None else D.data_ptr()
-    args.dt_bias = None if dt_bias is None else dt_bias.data_ptr()
-    _lib.call("ssm_state_step", args, dev)
-    return out
-
-
 def selective_state_step(state, x, dt, A, B, C, D=None, z=None, dt_bias=None, softplus=True):
     """Advance the selective state by one token on the GPU; ``state`` is updated in place.
 
@@ -475,28 +405,17 @@ def selective_state_step(state, x, dt, A, B, C, D=None, z=None, dt_bias=None, so
     Returns:
         Output ``(B, D)`` in ``x.dtype``.
     """
-    tensors = (state, x, dt, A, B, C, D, z, dt_bias)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    got = _native.state_step(_STEP_FORMS, None, state, x, dt, A, B, C, D, z, dt_bias, softplus)
+    if got is not None:
+        return got
+    if _needs_graph(state, x, dt, A, B, C, D, z, dt_bias):
         from ._autograd import state_step_with_grad
         return state_step_with_grad(state, x, dt, A, B, C, D, z, dt_bias, bool(softplus))
-    again = _state_step_again(state, x, dt, A, B, C, D, z, dt_bias, softplus)
-    if again is not None:
-        return again
     if state.is_contiguous():
         plan = StepPlan(state, x, dt, A, B, C, D, z, dt_bias, softplus)
         out = plan.run()
-        if plan.f64 is None and len(_STEP_FORMS) < 256 and out.dtype == x.dtype:
-            # remembered only when every tensor went in as it was (no cast, no copy, no batch stride): that is what
-            # _state_step_again can repeat
-            k, a = plan.keep, plan.args
-            same = all(p is None or q is None or p.data_ptr() == q.data_ptr()
-                       for p, q in ((x, k["x"]), (dt, k["dt"]), (z, k["z"]), (B, k["B"]), (C, k["C"]), (A, k["A"]),
-                                    (D, k["D"]), (dt_bias, k["bias"])))
-            if same and not (a.z_batch_stride or a.b_batch_stride or a.c_batch_stride) and K.on_gpu(state):
-                key = (state.shape, state.dtype, x.shape, x.dtype, A.shape, B.shape, B.dtype, C.shape,
-                       D is None or D.shape, z is None or z.shape, dt_bias is None or dt_bias.shape, bool(softplus),
-                       state.device.index)
-                _STEP_FORMS[key] = bytes(a)
+        if plan.f64 is None:
+            _native.state_step(_STEP_FORMS, bytes(plan.args), state, x, dt, A, B, C, D, z, dt_bias, softplus)
     else:
         work = state.contiguous()
         plan = StepPlan(work, x, dt, A, B, C, D, z, dt_bias, softplus)
@@ -565,11 +484,16 @@ def decode_step(conv_state, ssm_state, x, dt, A, B, C, conv_weight, conv_bias=No
     Returns:
         ``y (B, D)`` in ``x.dtype``, or ``(y, conv_out)``.
     """
-    plan = DecodePlan(conv_state, ssm_state, x, dt, A, B, C, conv_weight, conv_bias, D, z, dt_bias, softplus,
-                      activation, want_conv_out=return_conv_out)
+    call = (conv_state, ssm_state, x, dt, A, B, C, conv_weight, conv_bias, D, z, dt_bias, softplus, activation)
+    if not return_conv_out:
+        y = _native.decode_step(_DECODE_FORMS, None, *call)
+        if y is not None:
+            return y
+    plan = DecodePlan(*call, want_conv_out=return_conv_out)
     y = plan.run()
     if return_conv_out:
         return y, plan.conv_out
+    _native.decode_step(_DECODE_FORMS, bytes(plan.args), *call)
     return y
 
 
@@ -593,6 +517,11 @@ def mamba2_decode_step(zxbcdt, conv_state, ssm_state, conv_weight, conv_bias, A,
     Returns:
         ``y (B, d_inner)`` in ``zxbcdt.dtype``, or ``(y, conv_out)``.
     """
+    call = (zxbcdt, conv_state, ssm_state, conv_weight, conv_bias, A, D, dt_bias, ngroups, softplus, gate)
+    if not return_conv_out:
+        y = _native.mamba2_decode_step(_MAMBA2_FORMS, None, *call)
+        if y is not None:
+            return y
     if ssm_state.ndim != 4 or zxbcdt.ndim != 2 or conv_state.ndim != 3:
         raise ValueError("zxbcdt must be (B, proj), conv_state (B, C, K) and ssm_state (B, H, P, N).")
     batch, heads, hdim, nstate = (int(v) for v in ssm_state.shape)
@@ -621,7 +550,10 @@ def mamba2_decode_step(zxbcdt, conv_state, ssm_state, conv_weight, conv_bias, A,
         io_dtype=_lib.dtype_enum(row.dtype), d_per_p=int(D is not None and D.ndim == 2),
         dt_softplus=int(bool(softplus)), gate=int(bool(gate)))
     _lib.call("ssm_mamba2_decode_step", args, dev)
-    return (y, xbc) if return_conv_out else y
+    if return_conv_out:
+        return y, xbc
+    _native.mamba2_decode_step(_MAMBA2_FORMS, bytes(args), *call)
+    return y
 
 
 def conv_window_step(conv_state, x, weight, bias=None, activation="silu"):
@@ -641,6 +573,9 @@ def conv_window_step(conv_state, x, weight, bias=None, activation="silu"):
     Returns:
         ``(B, C)`` tensor in ``x.dtype``.
     """
+    out = _native.conv_window_step(_WINDOW_FORMS, None, conv_state, x, weight, bias, activation)
+    if out is not None:
+        return out
     if conv_state.ndim != 3 or x.ndim != 2 or tuple(conv_state.shape[:2]) != tuple(x.shape):
         raise ValueError("conv_state must have shape (B, C, K) and x (B, C).")
     batch, chans, width = (int(v) for v in conv_state.shape)
@@ -666,6 +601,7 @@ def conv_window_step(conv_state, x, weight, bias=None, activation="silu"):
         x_row_stride=int(xs.stride(0)), batch=batch, channels=chans, width=width,
         io_dtype=_lib.dtype_enum(x.dtype), activation=_lib.ACT_SILU if act in ("silu", "swish") else _lib.ACT_IDENTITY)
     _lib.call("ssm_conv1d_update", args, dev)
+    _native.conv_window_step(_WINDOW_FORMS, bytes(args), conv_state, x, weight, bias, activation)
     return out
 
 
@@ -683,6 +619,7 @@ def _dscan_forward(X, dt, A, B, C, chunk_size, D, z, lengths, initial_states, wa
         from . import _f64
         Y = _f64.dscan_forward(X, dt, A, B, C, chunk_size, D, z, lengths, initial_states)
         return (Y, None) if want_round_states else Y
+    call = (X, dt, A, B, C, int(chunk_size), D, z, lengths, initial_states)
     dt, A, B, C, D, z, initial_states = K.narrow(dt, A, B, C, D, z, initial_states)
     batch, seqlen, heads, proj, a_per_p, bk, ck, d_per_p, z_per_p = \
         K.check_chunk_scan(X, dt, A, B, C, chunk_size, D, z, initial_states)
@@ -710,6 +647,7 @@ def _dscan_forward(X, dt, A, B, C, chunk_size, D, z, lengths, initial_states, wa
         table = torch.empty(batch, (seqlen + 63) // 64, heads * proj, dtype=torch.float32, device=dev)
         args.round_states = _lib.ptr(table)
     _lib.call("ssm_dscan_fwd", args, dev)
+    _native.chunk_scan(_CHUNK_FORMS, bytes(args), *call)
     return (Y, table) if want_round_states else Y
 
 
@@ -793,11 +731,18 @@ def ssd_chunk_scan(X, dt, A, B, C, chunk_size, D=None, z=None, seq_meta=None, in
     Returns:
         Tensor ``(B, L, H, P)`` in ``X.dtype``.
     """
-    tensors = (X, dt, A, B, C, D, z, initial_states)
+    if not seq_meta:
+        Y = _native.chunk_scan(_CHUNK_FORMS, None, X, dt, A, B, C, chunk_size, D, z, None, initial_states)
+        if Y is not None:
+            return Y
     K.check_chunk_scan(X, dt, A, B, C, chunk_size, D, z, initial_states)
     dev = K.require_gpu(X, dt, A, B, C, D, z, initial_states)
     lengths = K.sequence_lengths(seq_meta, int(X.shape[0]), dev)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    if lengths is not None:
+        Y = _native.chunk_scan(_CHUNK_FORMS, None, X, dt, A, B, C, chunk_size, D, z, lengths, initial_states)
+        if Y is not None:
+            return Y
+    if _needs_graph(X, dt, A, B, C, D, z, initial_states):
         from ._autograd import DiagScanFn
         return DiagScanFn.apply(X, dt, A, B, C, int(chunk_size), D, z, lengths, initial_states)
     return _dscan_forward(X, dt, A, B, C, chunk_size, D, z, lengths, initial_states)
@@ -844,6 +789,7 @@ def _conv_forward(x, weight, bias, activation, channels_last=None):
     if K.f64_compute(x):
         from . import _f64
         return _f64.conv_forward(x, weight, bias, activation, channels_last)
+    call = (x, weight, bias, activation, channels_last)
     weight, bias = K.narrow(weight, bias)
     batch, chans, length, width, channels_first, silu = K.check_conv(x, weight, bias, activation, channels_last)
     dev = K.require_gpu(x, weight, bias)
@@ -863,6 +809,8 @@ def _conv_forward(x, weight, bias, activation, channels_last=None):
         layout=layout, activation=_lib.ACT_SILU if silu else _lib.ACT_IDENTITY,
         x_batch_stride=strides[0], x_row_stride=strides[1])
     _lib.call("ssm_conv1d_fwd", args, dev)
+    if rows is None:
+        _native.causal_conv(_CONV_FORMS, bytes(args), *call)
     return y
 
 
@@ -924,8 +872,10 @@ def dw_causal_conv_channels_last(x, weight, bias=None, activation="silu"):
 
 
 def _dw_causal_conv(x, weight, bias, activation, channels_last):
-    tensors = (x, weight, bias)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    y = _native.causal_conv(_CONV_FORMS, None, x, weight, bias, activation, channels_last)
+    if y is not None:
+        return y
+    if _needs_graph(x, weight, bias):
         from ._autograd import CausalConvFn
         return CausalConvFn.apply(x, weight, bias, activation, channels_last)
     return _conv_forward(x, weight, bias, activation, channels_last)
@@ -940,6 +890,7 @@ def _norm_forward(x, weight, bias, residual, is_rms, eps, prenorm, residual_in_f
     if K.f64_compute(x):
         from . import _f64
         return _f64.norm_forward(x, weight, bias, residual, is_rms, eps, prenorm, want_residual_out)
+    call = (x, weight, bias, residual, is_rms, eps, prenorm, residual_in_fp32, want_residual_out)
     weight, bias, residual = K.narrow(weight, bias, residual)
     rows, hidden = K.check_norm(x, weight, bias, residual)
     dev = K.require_gpu(x, weight, bias, residual)
@@ -966,6 +917,7 @@ def _norm_forward(x, weight, bias, residual, is_rms, eps, prenorm, residual_in_f
         residual_out_dtype=_lib.dtype_enum(res_out.dtype) if res_out is not None else 0,
         is_rms=int(bool(is_rms)), prenorm=int(bool(prenorm)), eps=float(eps))
     _lib.call("ssm_norm_fwd", args, dev)
+    _native.fused_norm(_NORM_FORMS, bytes(args), *call)
     return y, res_out, mean, rstd
 
 
@@ -1045,8 +997,10 @@ def fused_layer_norm(x, weight, bias, residual=None, is_rms=False, eps=1e-5, pre
     Returns:
         Normalised tensor with the shape and dtype of ``x``.
     """
-    tensors = (x, weight, bias, residual)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    y = _native.fused_norm(_NORM_FORMS, None, x, weight, bias, residual, is_rms, eps, prenorm, residual_in_fp32, False)
+    if y is not None:
+        return y
+    if _needs_graph(x, weight, bias, residual):
         from ._autograd import FusedNormFn
         return FusedNormFn.apply(x, weight, bias, residual, bool(is_rms), float(eps), bool(prenorm),
                                  bool(residual_in_fp32), False)[0]
@@ -1069,8 +1023,10 @@ def fused_layer_norm_with_residual(x, weight, bias, residual=None, is_rms=False,
         ``(y, residual_out)`` where ``residual_out = x (+ residual if prenorm)`` in
         float32 when ``residual_in_fp32`` else in the residual's (or ``x``'s) dtype.
     """
-    tensors = (x, weight, bias, residual)
-    if any(t is not None and t.requires_grad for t in tensors) and torch.is_grad_enabled():
+    got = _native.fused_norm(_NORM_FORMS, None, x, weight, bias, residual, is_rms, eps, prenorm, residual_in_fp32, True)
+    if got is not None:
+        return got
+    if _needs_graph(x, weight, bias, residual):
         from ._autograd import FusedNormFn
         return FusedNormFn.apply(x, weight, bias, residual, bool(is_rms), float(eps), bool(prenorm),
                                  bool(residual_in_fp32), True)

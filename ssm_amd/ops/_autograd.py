@@ -94,6 +94,8 @@ class SelectiveScanFn(torch.autograd.Function):
         keep_cs = A.shape[-1] <= _BWD_MAX_STATES
         plan = ScanPlan(u, delta, A, B, C, D, z, dt_bias, softplus, want_state, want_chunk_states=keep_cs)
         out, last = plan.run()
+        if plan.f64 is None:
+            plan.remember(u, delta, A, B, C, D, z, dt_bias, softplus)
         if out.dtype != u.dtype:
             out = out.to(u.dtype)
             last = last.to(u.dtype) if last is not None else None

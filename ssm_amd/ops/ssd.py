@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
+from .._lib import host as _native
 from . import _contract as K
 
 
@@ -389,6 +390,9 @@ def _rows_in_place(t):
     return (t, int(sl)) if ok and not t.is_contiguous() else (K.cast_c(t, t.dtype), 0)
 
 
+_FUSED_FORMS = {}      # argument structs of one-pass calls seen before (see the forms in ssm_amd/ops/__init__.py)
+
+
 def _ssd_fused(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt_limit, return_final_states, shape,
                seq_idx=None):
     batch, seqlen, heads, hdim, groups, nstate = shape
@@ -425,6 +429,9 @@ def _ssd_fused(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt
         dt_min=float(dt_limit[0]), dt_max=float(dt_limit[1]), seq_idx=_lib.ptr(si), b_row_stride=b_row,
         c_row_stride=c_row)
     _lib.call("ssm_ssd_combined_fwd", args, dev)
+    if seq_idx is None:
+        _native.ssd_combined(_FUSED_FORMS, bytes(args), x, dt, A, B, C, int(Q), D, z, dt_bias, initial_states, dt_softplus,
+                             dt_limit[0], dt_limit[1], return_final_states)
     if return_final_states:
         return y, final
     return y
@@ -476,6 +483,11 @@ def ssd_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initi
         ``return_varlen_states`` a tuple ``(y[, final_states (B, H, P, N)][, varlen_states])``.
     """
     Q = int(chunk_size)
+    if states_dtype is None and not force_generic and fused is not False and seq_idx is None and not return_varlen_states:
+        out = _native.ssd_combined(_FUSED_FORMS, None, x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus,
+                                   dt_limit[0], dt_limit[1], return_final_states)
+        if out is not None:
+            return out
     seqlen = int(x.shape[1]) if x.ndim == 4 else 0
     if (x.ndim == 4 and x.dtype in (torch.bfloat16, torch.float16) and Q > 0 and seqlen % Q != 0 and not force_generic
             and float(dt_limit[0]) <= 0.0 and dt.ndim == 3):
