@@ -382,6 +382,7 @@ PLAIN_SYMBOLS = {
     "ssm_scan_chunk_len": (C.c_int, []),
     "ssm_scan_bwd_workspace_bytes": (C.c_size_t, [C.c_int] * 8),
     "ssm_scan_bwd_per_row_workspace_bytes": (C.c_size_t, [C.POINTER(ScanBwdArgs)]),
+    "ssm_scan_bwd_full_workspace_bytes": (C.c_size_t, [C.POINTER(ScanBwdArgs)]),
     "ssm_state_step_bwd_workspace_bytes": (C.c_size_t, [C.c_int] * 3),
     "ssm_dscan_fwd_workspace_bytes": (C.c_size_t, [C.c_int] * 4),
     "ssm_dscan_bwd_workspace_bytes": (C.c_size_t, [C.c_int] * 4),

@@ -138,6 +138,64 @@ __device__ __forceinline__ void store_run(T *base, int t, int len, bool vec_ok, 
   }
 }
 
+// A wave-uniform base plus a 32-bit byte offset per lane: the form of address the memory instructions take as
+// it is (a base in scalar registers, an offset in one vector register), with no 64-bit arithmetic per access.
+template <typename T, typename B>
+__device__ __forceinline__ T *at_bytes(B *base, unsigned bytes) {
+  using C = typename std::conditional<std::is_const<B>::value, const char, char>::type;
+  return reinterpret_cast<T *>(reinterpret_cast<C *>(base) + bytes);
+}
+
+// A lane's run of K steps of a row of `len` steps.  RAGGED = false: rows start on 16-byte boundaries and are whole runs
+// long (and shorter than 2^29 steps), so a run is inside or outside as a whole (outside: some run of the row is read; the
+// caller masks its steps).
+// RAGGED = true: any length and any start (the memory takes vector accesses at any element boundary).  `tail`, the same
+// for the whole wave, says that the chunk at hand reaches past the end: what lies there then reads as zero.  A run
+// that crosses the end is still one vector access as long as it stays within the `room` elements from the row's start to
+// the end of the tensor, and goes element by element only there.
+template <bool RAGGED, typename T, int K>
+__device__ __forceinline__ Pack<T, K> load_steps(const T *row, int t, int len, bool tail, size_t room) {
+  if constexpr (!RAGGED) {
+    return *at_bytes<const Pack<T, K>>(row, (unsigned)(t < len ? t : 0) * (unsigned)sizeof(T));
+  } else {
+    struct __attribute__((packed)) Any { T v[K]; };
+    Pack<T, K> r;
+    if (!tail) {
+      const Any a = *reinterpret_cast<const Any *>(row + t);
+#pragma unroll
+      for (int i = 0; i < K; ++i) r.v[i] = a.v[i];
+    } else if ((size_t)t + K <= room) {
+      const Any a = *reinterpret_cast<const Any *>(row + t);
+#pragma unroll
+      for (int i = 0; i < K; ++i) r.v[i] = t + i < len ? a.v[i] : T{};
+    } else {
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        r.v[i] = T{};
+        if (t + i < len) r.v[i] = row[t + i];
+      }
+    }
+    return r;
+  }
+}
+
+template <bool RAGGED, typename T, int K>
+__device__ __forceinline__ void store_steps(T *row, int t, int len, const Pack<T, K> &v) {
+  if constexpr (!RAGGED) {
+    if (t < len) *at_bytes<Pack<T, K>>(row, (unsigned)t * (unsigned)sizeof(T)) = v;
+  } else if (t + K <= len) {
+    struct __attribute__((packed)) Any { T v[K]; };
+    Any a;
+#pragma unroll
+    for (int i = 0; i < K; ++i) a.v[i] = v.v[i];
+    *reinterpret_cast<Any *>(row + t) = a;
+  } else {
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+      if (t + i < len) row[t + i] = v.v[i];
+  }
+}
+
 // 2^x on the transcendental unit (v_exp_f32, 1 ulp; results below 2^-126 flush to 0).
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float log2_hw(float x) { return __builtin_amdgcn_logf(x); }
@@ -279,14 +337,6 @@ template <> __device__ __forceinline__ float Word<bf16_t>::elem(int v) const {
 }
 template <> __device__ __forceinline__ float Word<f16_t>::elem(int v) const {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(v ? (w >> 16) : (w & 0xffffu)));
-}
-
-// A wave-uniform base plus a 32-bit byte offset per lane: the form of address the memory instructions take as
-// it is (a base in scalar registers, an offset in one vector register), with no 64-bit arithmetic per access.
-template <typename T, typename B>
-__device__ __forceinline__ T *at_bytes(B *base, unsigned bytes) {
-  using C = typename std::conditional<std::is_const<B>::value, const char, char>::type;
-  return reinterpret_cast<T *>(reinterpret_cast<C *>(base) + bytes);
 }
 
 __device__ __forceinline__ int wave_id_uniform() {

@@ -38,7 +38,7 @@ using torch::autograd::variable_list;
 struct Abi {
 #define SSM_ENTRY(name) decltype(&::name) name = nullptr;
 #define SSM_ENTRIES(X)                                                                                             \
-  X(ssm_scan_fwd) X(ssm_scan_bwd) X(ssm_scan_bwd_workspace_bytes) X(ssm_scan_bwd_per_row_workspace_bytes)          \
+  X(ssm_scan_fwd) X(ssm_scan_bwd) X(ssm_scan_bwd_full_workspace_bytes)             \
   X(ssm_scan_chunk_len) X(ssm_state_step) X(ssm_decode_step) X(ssm_mamba2_decode_step) X(ssm_conv1d_update)        \
   X(ssm_conv1d_fwd) X(ssm_conv1d_bwd) X(ssm_conv1d_bwd_workspace_bytes) X(ssm_norm_fwd) X(ssm_norm_bwd)            \
   X(ssm_norm_bwd_workspace_bytes) X(ssm_dscan_fwd) X(ssm_dscan_bwd) X(ssm_dscan_fwd_workspace_bytes)               \
@@ -347,13 +347,11 @@ struct SelectiveScan : torch::autograd::Function<SelectiveScan> {
     a.batch = f.batch; a.dim = f.dim; a.seqlen = f.seqlen; a.nstate = f.nstate;
     a.io_dtype = f.io_dtype; a.bc_dtype = f.bc_dtype; a.b_kind = f.b_kind; a.c_kind = f.c_kind;
     a.b_groups = f.b_groups; a.c_groups = f.c_groups; a.delta_softplus = f.delta_softplus;
-    // projections of their own per channel: no partial sums of dB and dC, and their own type
-    size_t bytes = abi.ssm_scan_bwd_per_row_workspace_bytes(&a);
-    const at::ScalarType gt = bytes ? B.scalar_type() : at::kFloat;
+    const bool vary = f.b_kind == SSM_PROJ_BGNL && f.c_kind == SSM_PROJ_BGNL;
+    const at::ScalarType gt = vary ? B.scalar_type() : at::kFloat;
     Tensor dB = empty(B.sizes(), u, gt), dC = empty(C.sizes(), u, gt);
     a.dB = ptr<float>(dB); a.dC = ptr<float>(dC); a.dbc_dtype = dtype_enum(gt);
-    if (!bytes)
-      bytes = abi.ssm_scan_bwd_workspace_bytes(f.batch, f.dim, f.seqlen, f.nstate, f.b_kind, f.c_kind, f.b_groups, f.c_groups);
+    const size_t bytes = abi.ssm_scan_bwd_full_workspace_bytes(&a);
     Tensor ws = empty_bytes(bytes, u);
     a.workspace = ptr<void>(ws); a.workspace_bytes = bytes;
     SSM_ENQUEUE(ssm_scan_bwd, a, u.device().index());

@@ -48,6 +48,10 @@ struct ScanBwdParams {
   int rows_per_wg;       // channels walked by one workgroup (all in one B group and one C group)
   int nblk;              // workgroups per batch row = dim / rows_per_wg
   int bc_vec_ok;
+  int ragged;            // specialised kernels: rows are not whole aligned runs
+  const float2 *maps;    // specialised kernels: (B, D, ceil(L / 512), N) maps of the chunks (scan_bwd_maps.hpp), which then are
+                         // units of work of their own; the per-row sums above gain a leading axis of chunks.  NULL: a
+                         // unit walks all chunks of its rows
   int spin_limit;        // wave-per-row kernel: looks at a neighbour's slot count before a wave gives up (scan_bwd_fast.hpp)
 };
 
@@ -636,39 +640,70 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(const float *in, float *
   }
 }
 
-// Up to five such sums in one launch (dA, dD, the bias and, for projections constant in time, dB and dC: launches
-// of a few microseconds each, of which the gaps between them were as long as the work): workgroup ranges per job.
+// All sums that a backward call ends with, in one launch of workgroup ranges per job:
+//   out[o][i] = sum_{j < count} in[(o * count + j) * inner + i], added in order of j, written as `dtype`.
+// dA, dD, the bias and projections constant in time sum over the batch (and over chunks that ran side by side); dB and
+// dC of grouped projections over the workgroups of a group, straight into the projections' own type when asked.  As
+// launches of their own, with the casts behind them, they took 5 to 10 us each, of which the gaps were half.
 constexpr int FOLD_JOBS = 5;
 struct FoldJobs {
   const float *in[FOLD_JOBS];
-  float *out[FOLD_JOBS];
-  size_t inner[FOLD_JOBS];
-  int count[FOLD_JOBS];
+  void *out[FOLD_JOBS];
+  size_t outer[FOLD_JOBS], inner[FOLD_JOBS];
+  int count[FOLD_JOBS], dtype[FOLD_JOBS], width[FOLD_JOBS];     // width: outputs per thread, 1 or 4
   unsigned first_block[FOLD_JOBS + 1];
   int n;
 };
 
-__global__ __launch_bounds__(256) void fold_rows_multi_kernel(const FoldJobs jobs) {
+template <int W>
+__device__ __forceinline__ void fold_job(const float *in, void *out, size_t outer, size_t inner, int count, int dtype,
+                                         size_t first, size_t stride) {
+  const size_t per = inner / W;
+  for (size_t e = first; e < outer * per; e += stride) {
+    const size_t o = e / per, i = (e % per) * W;
+    const float *src = in + o * count * inner + i;
+    Pack<float, W> s;
+#pragma unroll
+    for (int w = 0; w < W; ++w) s.v[w] = 0.0f;
+    int j = 0;
+    for (; j + 8 <= count; j += 8) {                       // eight terms' reads in flight together
+      Pack<float, W> v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)(j + k) * inner);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int w = 0; w < W; ++w) s.v[w] += v[k].v[w];
+    }
+    for (; j < count; ++j) {
+      const Pack<float, W> v = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)j * inner);
+#pragma unroll
+      for (int w = 0; w < W; ++w) s.v[w] += v.v[w];
+    }
+    const size_t at = o * inner + i;
+    if (dtype == SSM_F32) {
+      *reinterpret_cast<Pack<float, W> *>(reinterpret_cast<float *>(out) + at) = s;
+    } else if (dtype == SSM_BF16) {
+      Pack<bf16_t, W> r;
+#pragma unroll
+      for (int w = 0; w < W; ++w) r.v[w] = from_f32<bf16_t>(s.v[w]);
+      *reinterpret_cast<Pack<bf16_t, W> *>(reinterpret_cast<bf16_t *>(out) + at) = r;
+    } else {
+      Pack<f16_t, W> r;
+#pragma unroll
+      for (int w = 0; w < W; ++w) r.v[w] = from_f32<f16_t>(s.v[w]);
+      *reinterpret_cast<Pack<f16_t, W> *>(reinterpret_cast<f16_t *>(out) + at) = r;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void fold_jobs_kernel(const FoldJobs jobs) {
   int j = 0;
   while (j + 1 < jobs.n && blockIdx.x >= jobs.first_block[j + 1]) ++j;
-  const float *in = jobs.in[j];
-  float *out = jobs.out[j];
-  const size_t inner = jobs.inner[j];
-  const int count = jobs.count[j];
-  const size_t blocks = jobs.first_block[j + 1] - jobs.first_block[j];
-  for (size_t i = (size_t)(blockIdx.x - jobs.first_block[j]) * blockDim.x + threadIdx.x; i < inner; i += blocks * blockDim.x) {
-    float s = 0.0f;
-    int k0 = 0;
-    for (; k0 + 8 <= count; k0 += 8) {
-      float v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = in[(size_t)(k0 + k) * inner + i];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) s += v[k];
-    }
-    for (; k0 < count; ++k0) s += in[(size_t)k0 * inner + i];
-    out[i] = s;
-  }
+  const size_t first = (size_t)(blockIdx.x - jobs.first_block[j]) * blockDim.x + threadIdx.x;
+  const size_t stride = (size_t)(jobs.first_block[j + 1] - jobs.first_block[j]) * blockDim.x;
+  if (jobs.width[j] == 4) fold_job<4>(jobs.in[j], jobs.out[j], jobs.outer[j], jobs.inner[j], jobs.count[j], jobs.dtype[j], first, stride);
+  else fold_job<1>(jobs.in[j], jobs.out[j], jobs.outer[j], jobs.inner[j], jobs.count[j], jobs.dtype[j], first, stride);
 }
 
 static unsigned fold_grid(size_t n) {
@@ -712,8 +747,10 @@ __global__ __launch_bounds__(256) void fold_sum_wide_kernel(const float *in, flo
   }
 }
 
+static bool fold_sum_is_wide(size_t outer, int count, size_t inner) { return outer * inner < 65536 && count >= 64; }
+
 void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_t inner, hipStream_t s) {
-  if (outer * inner < 65536 && count >= 64) {
+  if (fold_sum_is_wide(outer, count, inner)) {
     const int cols = inner >= 16 ? 16 : (inner >= 8 ? 8 : (inner >= 4 ? 4 : (inner >= 2 ? 2 : 1)));
     const int bpo = (int)((inner + cols - 1) / cols);
     hipLaunchKernelGGL(fold_sum_wide_kernel, dim3((unsigned)(outer * bpo)), dim3(256), 0, s, in, out, count, inner, cols,
@@ -727,13 +764,19 @@ void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_
   hipLaunchKernelGGL(fold_sum_kernel, dim3(fold_grid(outer * inner)), dim3(256), 0, s, in, out, outer, count, inner);
 }
 
+constexpr int BF_ROWS = 16;              // channels a workgroup of the wave-per-row kernel (scan_bwd_fast.hpp) takes at once
+
+// How a call is cut into work, from its sizes alone (the workspace is sized before the tensors are known).
 struct BwdPlan {
-  int rows_per_wg, nblk;
-  size_t off_dA, off_dD, off_dbias, off_dB, off_dC, total;   // byte offsets into the workspace
+  int rows_per_wg, nblk;                 // general kernel
+  enum { GENERAL, GROUPED, OWN, CONSTANT } route;   // the kernel for whose shape the call has, types permitting
+  int rpw, fast_nblk;                    // GROUPED: rows per wave in turn, workgroups per batch row
+  int nsplit;                            // chunks that may run side by side (1: a unit walks all of them)
+  size_t off_dA, off_dD, off_dbias, off_q, off_dB, off_dC, total;   // byte offsets into the workspace
 };
 
 static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int c_kind, int b_groups,
-                        int c_groups) {
+                        int c_groups, bool own_split = true) {
   const bool bv = b_kind == SSM_PROJ_BGNL, cv = c_kind == SSM_PROJ_BGNL;
   const int per_b = bv ? dim / b_groups : dim, per_c = cv ? dim / c_groups : dim;
   // Block of channels (<= 32) that stays inside one B group and one C group; among
@@ -743,16 +786,55 @@ static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int
     if (per_b % r == 0 && per_c % r == 0) { rows = r; break; }
   for (int r = 32; r >= 8; --r)
     if (per_b % r == 0 && per_c % r == 0 && ((size_t)batch * (dim / r)) % 256 == 0) { rows = r; break; }
-  BwdPlan pl;
+  BwdPlan pl{};
   pl.rows_per_wg = rows;
   pl.nblk = dim / rows;
+  pl.nsplit = 1;
+  const int nchunks = (len + BW_T - 1) / BW_T;
+  const double all = (double)batch * dim;
+  // Side by side, the chunks fill the chip better and cost a launch more (scan_bwd_maps.hpp), us.
+  const double maps = 12.0 + 0.5 * all * nchunks / 256;
+  if (bv && cv && b_groups == dim && c_groups == dim) {
+    pl.route = BwdPlan::OWN;
+    // bound by memory once the chip is busy, and the maps read C once more: 512 rows of 2048 steps 98 -> 78 us in float32,
+    // 1024 168 -> 152, 1536 223 -> 232
+    if (own_split && nchunks > 1 && all <= 1024) pl.nsplit = nchunks;
+  } else if (bv && cv && per_b % BF_ROWS == 0 && per_c % BF_ROWS == 0) {
+    pl.route = BwdPlan::GROUPED;
+    // us that a chunk takes with a workgroup of 16 x rpw rows on few of the CUs, and how much more on all of them
+    const double alone[3] = {29.0, 53.0, 77.0}, crowd[3] = {9.0, 11.6, 15.0};
+    auto time = [&](int rpw, double units) {
+      const double full = (double)(long)(units / 256), rest = units - full * 256;
+      return full * (alone[rpw - 1] + crowd[rpw - 1]) + (rest > 0.0 ? alone[rpw - 1] + crowd[rpw - 1] * rest / 256 : 0.0);
+    };
+    double best = 0.0;
+    for (int rpw = 3; rpw >= 1; --rpw) {               // fewer, larger workgroups leave fewer partial sums of dB and dC
+      if (per_b % (BF_ROWS * rpw) || per_c % (BF_ROWS * rpw)) continue;
+      const double units = all / (BF_ROWS * rpw);
+      for (int k = 0; k < (nchunks > 1 ? 2 : 1); ++k) {
+        const double cost = k ? time(rpw, units * nchunks) + maps : time(rpw, units) * nchunks;
+        if (pl.rpw && cost >= best) continue;
+        best = cost;
+        pl.rpw = rpw;
+        pl.nsplit = k ? nchunks : 1;
+      }
+    }
+    pl.fast_nblk = dim / (BF_ROWS * pl.rpw);
+  } else if (!bv && !cv) {
+    pl.route = BwdPlan::CONSTANT;
+    // (walks of 1024 steps are few at ordinary lengths: 512 rows of 8192 steps 133 -> 84 us, of 2048 no gain)
+    if (nchunks >= 8 && all <= 512) pl.nsplit = nchunks;
+  }
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) / 256 * 256; return o; };
-  pl.off_dA = take((size_t)batch * dim * nstate * 4);
-  pl.off_dD = take((size_t)batch * dim * 4);
-  pl.off_dbias = take((size_t)batch * dim * 4);
-  pl.off_dB = take(bv ? (size_t)batch * pl.nblk * nstate * len * 4 : (size_t)batch * dim * nstate * 4);
-  pl.off_dC = take(cv ? (size_t)batch * pl.nblk * nstate * len * 4 : (size_t)batch * dim * nstate * 4);
+  const size_t rows_all = (size_t)pl.nsplit * batch * dim;
+  const size_t blocks = pl.nblk > pl.fast_nblk ? pl.nblk : pl.fast_nblk;
+  pl.off_dA = take(rows_all * nstate * 4);
+  pl.off_dD = take(rows_all * 4);
+  pl.off_dbias = take(rows_all * 4);
+  pl.off_q = take(pl.nsplit > 1 ? (size_t)batch * dim * nchunks * nstate * sizeof(float2) : 0);
+  pl.off_dB = take(bv ? (size_t)batch * blocks * nstate * len * 4 : rows_all * nstate * 4);
+  pl.off_dC = take(cv ? (size_t)batch * blocks * nstate * len * 4 : rows_all * nstate * 4);
   pl.total = off;
   return pl;
 }
@@ -786,6 +868,7 @@ static int launch_bwd(const ScanBwdParams &p, hipStream_t s) {
 
 #include "scan_bwd_fast.hpp"
 #include "scan_bwd_rowbc.hpp"
+#include "scan_bwd_maps.hpp"
 
 extern "C" size_t ssm_scan_bwd_workspace_bytes(int batch, int dim, int seqlen, int nstate, int b_kind, int c_kind,
                                                int b_groups, int c_groups) {
@@ -796,35 +879,41 @@ extern "C" size_t ssm_scan_bwd_workspace_bytes(int batch, int dim, int seqlen, i
   return plan_bwd(batch, dim, seqlen, nstate, b_kind, c_kind, b_groups, c_groups).total;
 }
 
-// Whether a call takes the kernel for projections of their own per channel (scan_bwd_rowbc.hpp): B and C of shape
-// (B, D, N, L), activations in aligned rows of whole 8-step runs.  A selector of 1 (test-hooks build) keeps the
-// general kernel.
-static bool scan_bwd_is_per_row(const ssm_scan_bwd_args *a) {
-  using namespace ssm;
-  if (!a || SSM_RESERVED(a) == 1) return false;
-  if (a->b_kind != SSM_PROJ_BGNL || a->c_kind != SSM_PROJ_BGNL || a->b_groups != a->dim || a->c_groups != a->dim) return false;
-  if (a->seqlen <= 0 || a->seqlen % 8 != 0 || a->nstate <= 0 || a->nstate > BW_MAX_N) return false;
-  if (!valid_dtype(a->io_dtype) || !(a->bc_dtype == a->io_dtype || a->bc_dtype == SSM_F32)) return false;
-  const int bs = dtype_size(a->bc_dtype);
-  return aligned_to(a->u, 16) && aligned_to(a->delta, 16) && aligned_to(a->dout, 16) && aligned_to(a->du, 16) &&
-         aligned_to(a->ddelta, 16) && (!a->z || (aligned_to(a->z, 16) && aligned_to(a->dz, 16))) &&
-         aligned_to(a->Bproj, 8 * bs) && aligned_to(a->Cproj, 8 * bs) && aligned_to(a->dB, 16) && aligned_to(a->dC, 16);
+namespace ssm {
+template <typename io_t>
+static int launch_bwd_maps(const ScanBwdParams &p, int route, float2 *maps, hipStream_t s) {
+  if (route == BwdPlan::CONSTANT) return launch_scan_maps_as<io_t, float, false, true>(p, maps, s);
+  const bool bc32 = p.bc_dtype == SSM_F32;
+  if (route == BwdPlan::GROUPED)
+    return bc32 ? launch_scan_maps_as<io_t, float, true, false>(p, maps, s) : launch_scan_maps_as<io_t, io_t, true, false>(p, maps, s);
+  return bc32 ? launch_scan_maps_as<io_t, float, false, false>(p, maps, s) : launch_scan_maps_as<io_t, io_t, false, false>(p, maps, s);
 }
+}  // namespace ssm
 
-// Whether a call takes the wave-per-row kernel for projections that are constant in time, (D, N) or (B, D, N).
-static bool scan_bwd_is_const_row(const ssm_scan_bwd_args *a) {
+// The kernel a call takes: that of its plan when the element types allow it (projections of the activations' type or
+// float32; any for constant ones).  A selector of 1 (test-hooks build) keeps the general kernel.
+static int scan_bwd_route(const ssm_scan_bwd_args *a, const ssm::BwdPlan &pl) {
   using namespace ssm;
-  if (!a || SSM_RESERVED(a) == 1) return false;
-  if (a->b_kind == SSM_PROJ_BGNL || a->c_kind == SSM_PROJ_BGNL) return false;
-  if (a->seqlen <= 0 || a->seqlen % 8 != 0 || a->nstate <= 0 || a->nstate > BW_MAX_N) return false;
-  if (!valid_dtype(a->io_dtype) || !valid_dtype(a->bc_dtype)) return false;
-  return aligned_to(a->u, 16) && aligned_to(a->delta, 16) && aligned_to(a->dout, 16) && aligned_to(a->du, 16) &&
-         aligned_to(a->ddelta, 16) && (!a->z || (aligned_to(a->z, 16) && aligned_to(a->dz, 16)));
+  if (SSM_RESERVED(a) == 1 || !valid_dtype(a->io_dtype) || !valid_dtype(a->bc_dtype)) return BwdPlan::GENERAL;
+  if (pl.route != BwdPlan::CONSTANT && a->bc_dtype != a->io_dtype && a->bc_dtype != SSM_F32) return BwdPlan::GENERAL;
+  return pl.route;
 }
 
 extern "C" size_t ssm_scan_bwd_per_row_workspace_bytes(const ssm_scan_bwd_args *a) {
-  if (!scan_bwd_is_per_row(a)) return 0;
-  return ssm::plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind, a->b_groups, a->c_groups).off_dB;
+  using namespace ssm;
+  if (!a || a->seqlen <= 0 || a->batch <= 0 || a->dim <= 0 || a->nstate <= 0 || a->nstate > BW_MAX_N) return 0;
+  if (a->b_kind != SSM_PROJ_BGNL || a->c_kind != SSM_PROJ_BGNL || a->b_groups != a->dim || a->c_groups != a->dim) return 0;
+  const BwdPlan pl = plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind, a->b_groups, a->c_groups, false);
+  return scan_bwd_route(a, pl) == BwdPlan::OWN ? pl.off_dB : 0;
+}
+
+extern "C" size_t ssm_scan_bwd_full_workspace_bytes(const ssm_scan_bwd_args *a) {
+  using namespace ssm;
+  if (!a) return 0;
+  const size_t all = ssm_scan_bwd_workspace_bytes(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind, a->b_groups, a->c_groups);
+  if (!all || a->nstate > BW_MAX_N) return all;
+  const BwdPlan pl = plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind, a->b_groups, a->c_groups);
+  return scan_bwd_route(a, pl) == BwdPlan::OWN ? pl.off_dB : all;
 }
 
 extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
@@ -855,12 +944,15 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   SSM_REQUIRE((size_t)a->batch * a->dim < ((size_t)1 << 31) &&
                   (size_t)a->batch * a->dim * a->seqlen < ((size_t)1 << 40),
               SSM_ERR_TOO_LARGE, "ssm_scan_bwd: tensor too large");
-  const BwdPlan pl = plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind,
-                              bv ? a->b_groups : 1, cv ? a->c_groups : 1);
-  const bool per_row = scan_bwd_is_per_row(a);
-  SSM_REQUIRE(a->dbc_dtype == SSM_F32 || (per_row && a->dbc_dtype == a->bc_dtype), SSM_ERR_BAD_DTYPE,
-              "ssm_scan_bwd: dbc_dtype=%d: dB and dC are float32, or of the projections' type in a call for which "
-              "ssm_scan_bwd_per_row_workspace_bytes() is not 0", a->dbc_dtype);
+  BwdPlan pl = plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind,
+                        bv ? a->b_groups : 1, cv ? a->c_groups : 1);
+  const int route = scan_bwd_route(a, pl);
+  const bool per_row = route == BwdPlan::OWN;
+  if (per_row && a->workspace_bytes < pl.off_dB)           // room for the per-row sums only: chunks in turn
+    pl = plan_bwd(a->batch, a->dim, a->seqlen, a->nstate, a->b_kind, a->c_kind, a->b_groups, a->c_groups, false);
+  SSM_REQUIRE(a->dbc_dtype == SSM_F32 || (bv && cv && a->dbc_dtype == a->bc_dtype), SSM_ERR_BAD_DTYPE,
+              "ssm_scan_bwd: dbc_dtype=%d: dB and dC are float32, or of the projections' type where both vary in time",
+              a->dbc_dtype);
   const size_t ws_need = per_row ? pl.off_dB : pl.total;     // per row: no partial sums of dB and dC
   SSM_REQUIRE(a->workspace && a->workspace_bytes >= ws_need && aligned_to(a->workspace, 256), SSM_ERR_WORKSPACE,
               "ssm_scan_bwd: a 256-byte aligned workspace of %zu bytes is required", ws_need);
@@ -891,28 +983,33 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   // the wave-per-row kernel runs: every wave goes on at once and poisons dB and dC.
   p.spin_limit = SSM_RESERVED(a) == 2 ? 0 : (1 << 16);
 
+  auto whole = [&](const void *q, size_t n) { return !q || aligned_to(q, n); };
+  const bool rows_whole = a->seqlen % 8 == 0 && a->seqlen < (1 << 29) && whole(a->u, 16) && whole(a->delta, 16) && whole(a->dout, 16) && whole(a->du, 16) &&
+                          whole(a->ddelta, 16) && whole(a->z, 16) && whole(a->dz, 16);
+  p.ragged = !(rows_whole && (route == BwdPlan::CONSTANT || (whole(a->Bproj, (per_row ? 8 : 4) * bs) && whole(a->Cproj, (per_row ? 8 : 4) * bs))));
+
   hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
-  int rc;
-  // The specialised kernel: activations in aligned rows of whole 8-step runs, time-varying B and C of the
-  // activations' type or float32, groups that workgroups of 16, 32 or 48 channels tile, and no more partial
-  // sums than the workspace was sized for.  A selector of 1 keeps the general kernel.
-  int fast_rpw = 0;
-  if (bv && cv && SSM_RESERVED(a) != 1 && a->seqlen % 8 == 0 &&
-      (a->bc_dtype == a->io_dtype || a->bc_dtype == SSM_F32) && aligned_to(a->u, 16) && aligned_to(a->delta, 16) &&
-      aligned_to(a->dout, 16) && aligned_to(a->du, 16) && aligned_to(a->ddelta, 16) &&
-      (!a->z || (aligned_to(a->z, 16) && aligned_to(a->dz, 16))) && aligned_to(a->Bproj, 4 * bs) &&
-      aligned_to(a->Cproj, 4 * bs)) {
-    fast_rpw = scan_bwd_fast_rpw(a->batch, a->dim, a->dim / p.b_groups, a->dim / p.c_groups);
-    if (fast_rpw && a->dim / (BF_WAVES * fast_rpw) > pl.nblk) fast_rpw = 0;
+  int rc, copies = a->batch;               // per-row sums to add up for dA, dD and the bias
+  if (route != BwdPlan::GENERAL && pl.nsplit > 1) {
+    float2 *maps = reinterpret_cast<float2 *>(ws + pl.off_q);
+    switch (a->io_dtype) {
+      case SSM_F32: rc = launch_bwd_maps<float>(p, route, maps, s); break;
+      case SSM_BF16: rc = launch_bwd_maps<bf16_t>(p, route, maps, s); break;
+      default: rc = launch_bwd_maps<f16_t>(p, route, maps, s); break;
+    }
+    if (rc != SSM_OK) return rc;
+    p.maps = maps;
+    const int T = route == BwdPlan::CONSTANT && scan_bwd_const_long(a->seqlen, p.ragged) ? 2 * FAST_T : FAST_T;
+    copies = a->batch * ((a->seqlen + T - 1) / T);
   }
-  if (scan_bwd_is_const_row(a)) {
+  const bool bc32 = a->bc_dtype == SSM_F32, o32 = a->dbc_dtype == SSM_F32;
+  if (route == BwdPlan::CONSTANT) {
     switch (a->io_dtype) {
       case SSM_F32: rc = launch_bwd_row_const<float>(p, s); break;
       case SSM_BF16: rc = launch_bwd_row_const<bf16_t>(p, s); break;
       default: rc = launch_bwd_row_const<f16_t>(p, s); break;
     }
   } else if (per_row) {
-    const bool bc32 = a->bc_dtype == SSM_F32, o32 = a->dbc_dtype == SSM_F32;
     if (a->io_dtype == SSM_F32) rc = launch_bwd_rowbc<float, float, float>(p, a->dB, a->dC, s);
     else if (a->io_dtype == SSM_BF16)
       rc = bc32 ? launch_bwd_rowbc<bf16_t, float, float>(p, a->dB, a->dC, s)
@@ -920,13 +1017,12 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
     else
       rc = bc32 ? launch_bwd_rowbc<f16_t, float, float>(p, a->dB, a->dC, s)
                 : (o32 ? launch_bwd_rowbc<f16_t, f16_t, float>(p, a->dB, a->dC, s) : launch_bwd_rowbc<f16_t, f16_t, f16_t>(p, a->dB, a->dC, s));
-  } else if (fast_rpw) {
-    p.rows_per_wg = BF_WAVES * fast_rpw;
-    p.nblk = a->dim / p.rows_per_wg;
-    const bool bc32 = a->bc_dtype == SSM_F32;
-    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, fast_rpw, s);
-    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, fast_rpw, s) : launch_bwd_fast<bf16_t, bf16_t>(p, fast_rpw, s);
-    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, fast_rpw, s) : launch_bwd_fast<f16_t, f16_t>(p, fast_rpw, s);
+  } else if (route == BwdPlan::GROUPED) {
+    p.rows_per_wg = BF_WAVES * pl.rpw;
+    p.nblk = pl.fast_nblk;
+    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, pl.rpw, s);
+    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, pl.rpw, s) : launch_bwd_fast<bf16_t, bf16_t>(p, pl.rpw, s);
+    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, pl.rpw, s) : launch_bwd_fast<f16_t, f16_t>(p, pl.rpw, s);
   } else {
     switch (a->io_dtype) {
       case SSM_F32: rc = launch_bwd<float>(p, s); break;
@@ -937,33 +1033,37 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   if (rc != SSM_OK) return rc;
 
   const int Bn = a->batch, D = a->dim, N = a->nstate, L = a->seqlen;
-  // dA (D,N), dD (D,), dbias (D,): sums over the batch; dB / dC in the shape of the given projection.  The sums
-  // over rows share one launch.
+  // dA (D,N), dD (D,), dbias (D,): sums over the batch; dB / dC in the shape of the given projection
   FoldJobs jobs{};
-  auto add_job = [&](const float *in, float *out, int count, size_t inner) {
+  auto add_job = [&](const float *in, void *out, size_t outer, int count, size_t inner, int dtype) {
     const int j = jobs.n++;
-    jobs.in[j] = in; jobs.out[j] = out; jobs.count[j] = count; jobs.inner[j] = inner;
-    jobs.first_block[j + 1] = jobs.first_block[j] + fold_grid(inner);
+    jobs.in[j] = in; jobs.out[j] = out; jobs.outer[j] = outer; jobs.count[j] = count; jobs.inner[j] = inner; jobs.dtype[j] = dtype;
+    jobs.width[j] = inner % 4 == 0 && aligned_to(in, 16) && aligned_to(out, 16) ? 4 : 1;
+    jobs.first_block[j + 1] = jobs.first_block[j] + fold_grid(outer * inner / jobs.width[j]);
   };
-  add_job(p.dA_rows, a->dA, Bn, (size_t)D * N);
-  if (a->dD) add_job(p.dD_rows, a->dD, Bn, (size_t)D);
-  if (a->ddt_bias) add_job(p.dbias_rows, a->ddt_bias, Bn, (size_t)D);
-  auto fold_proj = [&](int kind, int groups, const float *partial, float *out) {
+  // (dB and dC, the longest sums, first)
+  auto fold_proj = [&](int kind, int groups, const float *partial, void *out) {
     if (kind == SSM_PROJ_BGNL) {
       // (B, G, nblk/G, N*L) -> (B, G, N*L)
       const int per_group = p.nblk / groups;
-      launch_fold_sum(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, s);
+      if (a->dbc_dtype == SSM_F32 && fold_sum_is_wide((size_t)Bn * groups, per_group, (size_t)N * L))
+        launch_fold_sum(partial, reinterpret_cast<float *>(out), (size_t)Bn * groups, per_group, (size_t)N * L, s);
+      else
+        add_job(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, a->dbc_dtype);
     } else if (kind == SSM_PROJ_BDN) {
-      add_job(partial, out, 1, (size_t)Bn * D * N);
+      add_job(partial, out, 1, copies / Bn, (size_t)Bn * D * N, SSM_F32);
     } else {
-      add_job(partial, out, Bn, (size_t)D * N);
+      add_job(partial, out, 1, copies, (size_t)D * N, SSM_F32);
     }
   };
   if (!per_row) {
-    fold_proj(a->b_kind, p.b_groups, p.dB_part, reinterpret_cast<float *>(a->dB));
-    fold_proj(a->c_kind, p.c_groups, p.dC_part, reinterpret_cast<float *>(a->dC));
+    fold_proj(a->b_kind, p.b_groups, p.dB_part, a->dB);
+    fold_proj(a->c_kind, p.c_groups, p.dC_part, a->dC);
   }
-  hipLaunchKernelGGL(fold_rows_multi_kernel, dim3(jobs.first_block[jobs.n]), dim3(256), 0, s, jobs);
+  add_job(p.dA_rows, a->dA, 1, copies, (size_t)D * N, SSM_F32);
+  if (a->dD) add_job(p.dD_rows, a->dD, 1, copies, (size_t)D, SSM_F32);
+  if (a->ddt_bias) add_job(p.dbias_rows, a->ddt_bias, 1, copies, (size_t)D, SSM_F32);
+  hipLaunchKernelGGL(fold_jobs_kernel, dim3(jobs.first_block[jobs.n]), dim3(256), 0, s, jobs);
   SSM_CHECK_LAUNCH("ssm_scan_bwd(fold)");
   return SSM_OK;
 }

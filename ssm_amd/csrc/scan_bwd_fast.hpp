@@ -1,5 +1,5 @@
 // Selective scan, backward: the kernel for the common call shape (time-varying grouped B and C,
-// at most 16 states, activations of any supported type in aligned rows of whole 8-step runs).  Included by
+// at most 16 states, activations of any supported type; rows of any length and start in its RAGGED form).  Included by
 // scan_bwd.hip after ScanBwdParams.
 //
 // A wavefront owns one row at a time and walks its states one after the other, lanes split
@@ -24,7 +24,7 @@
 
 namespace ssm {
 
-constexpr int BF_WAVES = 16;
+constexpr int BF_WAVES = BF_ROWS;
 constexpr int BF_THREADS = WAVE * BF_WAVES;
 constexpr int BF_K = 8;
 constexpr int BF_DEP = 1;             // wave w takes a state over from wave w + BF_DEP (-1 measured 2 % slower)
@@ -54,7 +54,9 @@ __device__ __forceinline__ bool wait_for_slots(lds_int *flag, int want, int spin
   return reached;
 }
 
-template <typename io_t, typename bc_t, int RPW, bool HAS_Z>
+// A workgroup walks all chunks of its rows, last to first, or (p.maps: the maps of the chunks are known) one of
+// them; blockIdx then counts chunks fastest, and the per-row sums are left per chunk.
+template <typename io_t, typename bc_t, int RPW, bool HAS_Z, bool RAGGED>
 __global__ __launch_bounds__(BF_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void scan_bwd_fast_kernel(const ScanBwdParams p) {
   constexpr int K = BF_K, T = FAST_T, NS = FAST_N;
@@ -71,14 +73,19 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
   const int wave = wave_id_uniform();
   const int lane = lane_id();
   const int tid = threadIdx.x;
-  const int b = (int)blockIdx.x / p.nblk;
-  const int blk = (int)blockIdx.x % p.nblk;
-  const int d_first = blk * rows;
   const int L = p.len, N = p.nstate;
   const int nchunks = (L + T - 1) / T;
+  const int side_by_side = p.maps ? nchunks : 1;
+  const int part = (int)blockIdx.x % side_by_side, unit = (int)blockIdx.x / side_by_side;
+  const int c_last = p.maps ? part : nchunks - 1, c_first = p.maps ? part : 0;
+  const int b = unit / p.nblk;
+  const int blk = unit % p.nblk;
+  const int d_first = blk * rows;
   const int rev_lane = WAVE - 1 - lane;
-  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + ((size_t)b * p.b_groups + d_first / (p.dim / p.b_groups)) * (size_t)N * L;
-  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + ((size_t)b * p.c_groups + d_first / (p.dim / p.c_groups)) * (size_t)N * L;
+  const size_t bg = (size_t)b * p.b_groups + d_first / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d_first / (p.dim / p.c_groups);
+  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + bg * N * L;
+  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + cg * N * L;
+  const size_t Broom = ((size_t)p.batch * p.b_groups - bg) * N * L, Croom = ((size_t)p.batch * p.c_groups - cg) * N * L;
   const io_t *U = reinterpret_cast<const io_t *>(p.u), *DT = reinterpret_cast<const io_t *>(p.delta);
   const io_t *GO = reinterpret_cast<const io_t *>(p.dout), *Z = reinterpret_cast<const io_t *>(HAS_Z ? p.z : p.u);
   io_t *DU = reinterpret_cast<io_t *>(p.du), *DDL = reinterpret_cast<io_t *>(p.ddelta), *DZ = reinterpret_cast<io_t *>(p.dz);
@@ -88,7 +95,11 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     const size_t row = (size_t)b * p.dim + d;
     if (lane < NS) {
       rowA2[r * NS + lane] = lane < N ? p.A[(size_t)d * N + lane] * LOG2E : 0.0f;
-      rowq[r * NS + lane] = (p.dlast && lane < N) ? p.dlast[row * N + lane] : 0.0f;      // adjoint from beyond the end
+      // adjoint from beyond the end, and from there through the chunks behind
+      float q0 = (p.dlast && lane < N) ? p.dlast[row * N + lane] : 0.0f;
+      if (p.maps && lane < N)
+        q0 = compose_maps(p.maps + (row * nchunks + nchunks - 1) * (size_t)N + lane, nchunks - 1 - c_last, -N, q0);
+      rowq[r * NS + lane] = q0;
       rowdA[r * NS + lane] = 0.0f;
     }
     if (lane == 0) rowdD[r] = rowdb[r] = 0.0f;
@@ -96,15 +107,14 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
   if (lane == 0) done[wave] = 0;
   int nslots = 0;                          // the same in every wave at the same point of the walk
 
-  for (int c = nchunks - 1; c >= 0; --c) {
+  for (int c = c_last; c >= c_first; --c) {
     const int t0 = c * T;
     const int t = t0 + lane * K;
-    const bool live = t < L;
-    const int tc = live ? t : 0;
+    const bool tail = t0 + T > L;
 
     __syncthreads();                       // the sums of the chunk before are in memory, its slabs are free
-    fast_stage<bc_t, WAVE>(Bs, Bg, L, t0, N, BF_THREADS);
-    fast_stage<bc_t, WAVE>(Cs, Cg, L, t0, N, BF_THREADS);
+    fast_stage<bc_t, WAVE, RAGGED>(Bs, Bg, L, t0, N, BF_THREADS, Broom);
+    fast_stage<bc_t, WAVE, RAGGED>(Cs, Cg, L, t0, N, BF_THREADS, Croom);
     for (int e = tid; e < 2 * NS * T / 4; e += BF_THREADS) reinterpret_cast<float4 *>(accB)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
 
@@ -112,16 +122,19 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     for (int rr = 0; rr < RPW; ++rr) {
       const int r = wave * RPW + rr, d = d_first + r;
       const size_t row = (size_t)b * p.dim + d;
-      const size_t at = row * L + tc;
+      const size_t at = row * L, room = ((size_t)p.batch * p.dim - row) * L;
       const float A2_lanes = rowA2[r * NS + (lane & (NS - 1))];
       float qcarry = rowq[r * NS + (lane & (NS - 1))], dA_lanes = 0.0f;
       const float Dk = p.Dk ? p.Dk[d] : 0.0f, bias = p.bias ? p.bias[d] : 0.0f;
       float dD_part = 0.0f, db_part = 0.0f;
-      const Pack<io_t, K> ur = *reinterpret_cast<const Pack<io_t, K> *>(U + at);
-      const Pack<io_t, K> dr = *reinterpret_cast<const Pack<io_t, K> *>(DT + at);
-      const Pack<io_t, K> gr = *reinterpret_cast<const Pack<io_t, K> *>(GO + at);
-      Pack<io_t, K> zr;
-      if (HAS_Z) zr = *reinterpret_cast<const Pack<io_t, K> *>(Z + at);
+      Pack<io_t, K> ur, dr, gr, zr;
+      auto fetch = [&]() {
+        ur = load_steps<RAGGED, io_t, K>(U + at, t, L, tail, room);
+        dr = load_steps<RAGGED, io_t, K>(DT + at, t, L, tail, room);
+        gr = load_steps<RAGGED, io_t, K>(GO + at, t, L, tail, room);
+        if (HAS_Z) zr = load_steps<RAGGED, io_t, K>(Z + at, t, L, tail, room);
+      };
+      fetch();
       const float Hin_lanes = lane < N ? p.chunk_states[(row * nchunks + c) * (size_t)N + lane] : 0.0f;
 
       float dl[K], du[K], g[K], ghB[K], At[K], pre[K];
@@ -130,6 +143,7 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
       for (int i = 0; i < K; ++i) {
         float x = to_f32(dr.v[i]) + bias;
         if (p.softplus) x = fast_softplus(x);
+        const bool live = t + (RAGGED ? i : 0) < L;
         dl[i] = live ? x : 0.0f;                       // steps past the end: identity maps, no contributions
         du[i] = dl[i] * to_f32(ur.v[i]);
         float gg = live ? to_f32(gr.v[i]) : 0.0f;
@@ -226,7 +240,10 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
         if (lane == 0) *(volatile lds_int *)(done + wave) = nslots;
       }
 
-      // ---- what the row's elements receive
+      // ---- what the row's elements receive; the inputs are read again (the caches hold them) rather than kept in
+      // registers over the walk of the states, where they would spill
+      __asm__ volatile("" ::: "memory");
+      fetch();
       float du_o[K], dd_o[K], dz_o[K];
 #pragma unroll
       for (int i = 0; i < K; ++i) {
@@ -237,7 +254,7 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
           const float e = exp2_hw(fminf(to_f32(dr.v[i]) + bias, 60.0f) * LOG2E);
           dd *= e * rcp_hw(1.0f + e);                  // softplus' = sigmoid
         }
-        dd = live ? dd : 0.0f;
+        dd = t + (RAGGED ? i : 0) < L ? dd : 0.0f;
         dd_o[i] = dd;
         db_part += dd;
         dD_part = __builtin_fmaf(g[i], uu, dD_part);
@@ -259,19 +276,17 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
           rowdb[r] += sb;
         }
       }
-      if (live) {
-        Pack<io_t, K> o;
+      Pack<io_t, K> o;
 #pragma unroll
-        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(du_o[i]);
-        *reinterpret_cast<Pack<io_t, K> *>(DU + at) = o;
+      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(du_o[i]);
+      store_steps<RAGGED, io_t, K>(DU + at, t, L, o);
 #pragma unroll
-        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dd_o[i]);
-        *reinterpret_cast<Pack<io_t, K> *>(DDL + at) = o;
-        if (HAS_Z) {
+      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dd_o[i]);
+      store_steps<RAGGED, io_t, K>(DDL + at, t, L, o);
+      if (HAS_Z) {
 #pragma unroll
-          for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dz_o[i]);
-          *reinterpret_cast<Pack<io_t, K> *>(DZ + at) = o;
-        }
+        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dz_o[i]);
+        store_steps<RAGGED, io_t, K>(DZ + at, t, L, o);
       }
     }
 
@@ -285,16 +300,15 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
         const float *src = (which ? accC : accB) + n * T + ln * 4;
         const float4 v0 = *reinterpret_cast<const float4 *>(src);
         const float4 v1 = *reinterpret_cast<const float4 *>(src + WAVE * 4);
-        float *dst = (which ? p.dC_part : p.dB_part) + (((size_t)b * p.nblk + blk) * N + n) * (size_t)L + tt;
-        *reinterpret_cast<float4 *>(dst) = v0;
-        *reinterpret_cast<float4 *>(dst + 4) = v1;
+        float *dst = (which ? p.dC_part : p.dB_part) + (((size_t)b * p.nblk + blk) * N + n) * (size_t)L;
+        store_steps<RAGGED, float, K>(dst, tt, L, Pack<float, K>{{v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w}});
       }
     }
   }
 
   for (int rr = 0; rr < RPW; ++rr) {
     const int r = wave * RPW + rr;
-    const size_t row = (size_t)b * p.dim + d_first + r;
+    const size_t row = ((size_t)(p.maps ? part : 0) * p.batch + b) * p.dim + d_first + r;
     if (lane < N) p.dA_rows[row * N + lane] = rowdA[r * NS + lane];
     if (lane == 0) {
       p.dD_rows[row] = rowdD[r];
@@ -303,26 +317,13 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
   }
 }
 
-// Rows per wave in turn for which the workgroups (16 waves) tile the groups, or 0.
-inline int scan_bwd_fast_rpw(int batch, int dim, int per_b, int per_c) {
-  const int cand[3] = {3, 2, 1};
-  int best = 0;
-  for (int i = 0; i < 3; ++i) {
-    const int r = BF_WAVES * cand[i];
-    if (per_b % r || per_c % r) continue;
-    if (!best) best = cand[i];
-    if ((size_t)batch * (dim / r) >= 256) return cand[i];       // the largest block that still gives every CU one
-  }
-  return best;
-}
-
 template <typename io_t, typename bc_t>
 static int launch_bwd_fast(const ScanBwdParams &p, int rpw, hipStream_t s) {
   const size_t ldsb = ((size_t)4 * FAST_N * FAST_T + (size_t)BF_WAVES * rpw * (3 * FAST_N + 2) + BF_WAVES) * sizeof(float);
-  const unsigned grid = (unsigned)((size_t)p.batch * p.nblk);
+  const unsigned grid = (unsigned)((size_t)p.batch * p.nblk * (p.maps ? (p.len + FAST_T - 1) / FAST_T : 1));
 #define SSM_BF_LAUNCH(R, HZ)                                                                   \
   {                                                                                            \
-    auto kernel = scan_bwd_fast_kernel<io_t, bc_t, R, HZ>;                                     \
+    auto kernel = p.ragged ? scan_bwd_fast_kernel<io_t, bc_t, R, HZ, true> : scan_bwd_fast_kernel<io_t, bc_t, R, HZ, false>; \
     if (allow_dynamic_lds(kernel, ldsb) != hipSuccess) {                                       \
       (void)hipGetLastError();                                                                 \
       set_error("ssm_scan_bwd: cannot reserve %zu bytes of LDS", ldsb);                        \

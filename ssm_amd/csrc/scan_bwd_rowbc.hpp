@@ -25,20 +25,27 @@ namespace ssm {
 
 constexpr int BR_WAVES = 4;
 
+// With p.maps (the maps of the 512-step chunks are known) a wave walks one chunk instead of all of its row's; waves
+// count chunks fastest, and the per-row sums are left per chunk.
 // K: steps per lane, 8 or 16 (a lane's run; 64 runs make a chunk of the walk).  The states that enter chunks come
 // from the forward in steps of FAST_T = 512, so a walk in chunks of 1024 takes every second one.
-template <typename io_t, typename bc_t, typename out_t, bool HAS_Z, bool CONST_BC = false, int K = BF_K, int OCC = (CONST_BC ? 4 : 2)>
+template <typename io_t, typename bc_t, typename out_t, bool HAS_Z, bool RAGGED, bool CONST_BC = false, int K = BF_K, int OCC = (CONST_BC ? 4 : 2)>
 __global__ __launch_bounds__(WAVE *BR_WAVES) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
   constexpr int T = WAVE * K;
   static_assert(T % FAST_T == 0, "chunks of the walk are whole chunks of the forward");
   const int wave = wave_id_uniform();
   const int lane = lane_id();
-  const size_t row = (size_t)blockIdx.x * BR_WAVES + wave;
-  if (row >= (size_t)p.batch * p.dim) return;                // no barrier below: a wave may leave alone
-  const int d = (int)(row % p.dim);
   const int L = p.len, N = p.nstate;
   const int nchunks = (L + T - 1) / T;
+  const int side_by_side = p.maps ? nchunks : 1;
+  const size_t unit = (size_t)blockIdx.x * BR_WAVES + wave;
+  const size_t row = unit / side_by_side;
+  const int part = (int)(unit % side_by_side);
+  if (row >= (size_t)p.batch * p.dim) return;                // no barrier below: a wave may leave alone
+  const int c_last = p.maps ? part : nchunks - 1, c_first = p.maps ? part : 0;
+  const int d = (int)(row % p.dim);
+  const size_t room = ((size_t)p.batch * p.dim - row) * L, proom = room * N;       // elements to the ends of the tensors
   const int fwd_chunks = (L + FAST_T - 1) / FAST_T;           // rows of chunk_states per (batch, channel)
   const int rev_lane = WAVE - 1 - lane;
   const size_t proj0 = CONST_BC ? 0 : row * (size_t)N * L;    // the row's own (N, L) block of B, C, dB and dC
@@ -57,25 +64,27 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
   // lane n holds what belongs to state n: A log2(e), the adjoint carried between chunks, the sum for dA
   const float A2_lanes = lane < N ? p.A[(size_t)d * N + lane] * LOG2E : 0.0f;
   float qcarry = (p.dlast && lane < N) ? p.dlast[row * N + lane] : 0.0f;
+  if (p.maps && lane < N)
+    qcarry = compose_maps(p.maps + (row * fwd_chunks + fwd_chunks - 1) * (size_t)N + lane,
+                          fwd_chunks - min((part + 1) * (T / FAST_T), fwd_chunks), -N, qcarry);
   float dA_lanes = 0.0f;
   const float Dk = p.Dk ? p.Dk[d] : 0.0f, bias = p.bias ? p.bias[d] : 0.0f;
   float dD_part = 0.0f, db_part = 0.0f;
 
-  for (int c = nchunks - 1; c >= 0; --c) {
+  for (int c = c_last; c >= c_first; --c) {
     const int t = c * T + lane * K;
-    const bool live = t < L;
-    const int tc = live ? t : 0;
-    const size_t at = row * L + tc;
+    const bool tail = (c + 1) * T > L;
+    const size_t at = row * L;
     Pack<bc_t, K> braw, craw;
     if (!CONST_BC) {
-      braw = *reinterpret_cast<const Pack<bc_t, K> *>(Bg + tc);
-      craw = *reinterpret_cast<const Pack<bc_t, K> *>(Cg + tc);
+      braw = load_steps<RAGGED, bc_t, K>(Bg, t, L, tail, proom);
+      craw = load_steps<RAGGED, bc_t, K>(Cg, t, L, tail, proom);
     }
-    const Pack<io_t, K> ur = *reinterpret_cast<const Pack<io_t, K> *>(U + at);
-    const Pack<io_t, K> dr = *reinterpret_cast<const Pack<io_t, K> *>(DT + at);
-    const Pack<io_t, K> gr = *reinterpret_cast<const Pack<io_t, K> *>(GO + at);
+    const Pack<io_t, K> ur = load_steps<RAGGED, io_t, K>(U + at, t, L, tail, room);
+    const Pack<io_t, K> dr = load_steps<RAGGED, io_t, K>(DT + at, t, L, tail, room);
+    const Pack<io_t, K> gr = load_steps<RAGGED, io_t, K>(GO + at, t, L, tail, room);
     Pack<io_t, K> zr;
-    if (HAS_Z) zr = *reinterpret_cast<const Pack<io_t, K> *>(Z + at);
+    if (HAS_Z) zr = load_steps<RAGGED, io_t, K>(Z + at, t, L, tail, room);
     const float Hin_lanes = lane < N ? p.chunk_states[(row * fwd_chunks + c * (T / FAST_T)) * (size_t)N + lane] : 0.0f;
 
     float dl[K], du[K], g[K], ghB[K], At[K], pre[K];
@@ -84,6 +93,7 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
     for (int i = 0; i < K; ++i) {
       float x = to_f32(dr.v[i]) + bias;
       if (p.softplus) x = fast_softplus(x);
+      const bool live = t + (RAGGED ? i : 0) < L;
       dl[i] = live ? x : 0.0f;                         // steps past the end: identity maps, no contributions
       du[i] = dl[i] * to_f32(ur.v[i]);
       float gg = live ? to_f32(gr.v[i]) : 0.0f;
@@ -102,8 +112,8 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
       Pack<bc_t, K> bnext, cnext;
       float bq[K], cq[K];
       if (!CONST_BC) {
-        bnext = *reinterpret_cast<const Pack<bc_t, K> *>(Bg + (size_t)nn * L + tc);
-        cnext = *reinterpret_cast<const Pack<bc_t, K> *>(Cg + (size_t)nn * L + tc);
+        bnext = load_steps<RAGGED, bc_t, K>(Bg + (size_t)nn * L, t, L, tail, proom - (size_t)nn * L);
+        cnext = load_steps<RAGGED, bc_t, K>(Cg + (size_t)nn * L, t, L, tail, proom - (size_t)nn * L);
 #pragma unroll
         for (int i = 0; i < K; ++i) {
           bq[i] = to_f32(braw.v[i]);
@@ -169,10 +179,8 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
       const float tot = wave_sum(sA);
       dA_lanes += lane == n ? tot : 0.0f;
       if (!CONST_BC) {
-        if (live) {
-          *reinterpret_cast<Pack<out_t, K> *>(dBg + (size_t)n * L + tc) = ob;
-          *reinterpret_cast<Pack<out_t, K> *>(dCg + (size_t)n * L + tc) = oc;
-        }
+        store_steps<RAGGED, out_t, K>(dBg + (size_t)n * L, t, L, ob);
+        store_steps<RAGGED, out_t, K>(dCg + (size_t)n * L, t, L, oc);
         braw = bnext;
         craw = cnext;
       } else {
@@ -193,7 +201,7 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
         const float e = exp2_hw(fminf(to_f32(dr.v[i]) + bias, 60.0f) * LOG2E);
         dd *= e * rcp_hw(1.0f + e);                    // softplus' = sigmoid
       }
-      dd = live ? dd : 0.0f;
+      dd = t + (RAGGED ? i : 0) < L ? dd : 0.0f;
       dd_o[i] = dd;
       db_part += dd;
       dD_part = __builtin_fmaf(g[i], uu, dD_part);
@@ -204,60 +212,80 @@ void scan_bwd_rowbc_kernel(const ScanBwdParams p, out_t *dBo, out_t *dCo) {
         dz_o[i] = to_f32(gr.v[i]) * full * s * __builtin_fmaf(zz, 1.0f - s, 1.0f);
       }
     }
-    if (live) {
-      Pack<io_t, K> o;
+    Pack<io_t, K> o;
 #pragma unroll
-      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(du_o[i]);
-      *reinterpret_cast<Pack<io_t, K> *>(DU + at) = o;
+    for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(du_o[i]);
+    store_steps<RAGGED, io_t, K>(DU + at, t, L, o);
 #pragma unroll
-      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dd_o[i]);
-      *reinterpret_cast<Pack<io_t, K> *>(DDL + at) = o;
-      if (HAS_Z) {
+    for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dd_o[i]);
+    store_steps<RAGGED, io_t, K>(DDL + at, t, L, o);
+    if (HAS_Z) {
 #pragma unroll
-        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dz_o[i]);
-        *reinterpret_cast<Pack<io_t, K> *>(DZ + at) = o;
-      }
+      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dz_o[i]);
+      store_steps<RAGGED, io_t, K>(DZ + at, t, L, o);
     }
   }
 
   const float sd = wave_sum(dD_part), sb = wave_sum(db_part);
-  if (lane < N) p.dA_rows[row * N + lane] = dA_lanes;
+  const size_t out = (size_t)(p.maps ? part : 0) * p.batch * p.dim + row;
+  if (lane < N) p.dA_rows[out * N + lane] = dA_lanes;
   if (CONST_BC && lane < N) {
-    p.dB_part[row * N + lane] = dB_lanes;
-    p.dC_part[row * N + lane] = dC_lanes;
+    p.dB_part[out * N + lane] = dB_lanes;
+    p.dC_part[out * N + lane] = dC_lanes;
   }
   if (lane == 0) {
-    p.dD_rows[row] = sd;
-    p.dbias_rows[row] = sb;
+    p.dD_rows[out] = sd;
+    p.dbias_rows[out] = sb;
   }
 }
+
+// Whether sequences of constant projections are walked in 16-step runs per lane, chunks of 1024 steps: half the lane
+// scans and wave sums per step, at 243 registers and two waves per SIMD (at three, 66 spill): 303 against 323 us at
+// 8 x 1536 x 2048.  For sequences that fill such chunks.
+static bool scan_bwd_const_long(int len, bool ragged) {
+  const int tail = len % (2 * FAST_T);
+  return (ragged || len % 16 == 0) && len >= 2 * FAST_T && (tail == 0 || tail > FAST_T);
+}
+
+#define SSM_BR_LAUNCH(...)                                                                                     \
+  do {                                                                                                         \
+    if (p.z && p.ragged) hipLaunchKernelGGL((SSM_BR_KERNEL(true, true)), grid, block, 0, s, __VA_ARGS__);      \
+    else if (p.z) hipLaunchKernelGGL((SSM_BR_KERNEL(true, false)), grid, block, 0, s, __VA_ARGS__);            \
+    else if (p.ragged) hipLaunchKernelGGL((SSM_BR_KERNEL(false, true)), grid, block, 0, s, __VA_ARGS__);       \
+    else hipLaunchKernelGGL((SSM_BR_KERNEL(false, false)), grid, block, 0, s, __VA_ARGS__);                    \
+  } while (0)
 
 // Projections constant in time: the partial sums per row go to p.dB_part / p.dC_part, (B, D, N) float32.
 template <typename io_t>
 static int launch_bwd_row_const(const ScanBwdParams &p, hipStream_t s) {
-  const size_t rows = (size_t)p.batch * p.dim;
-  const dim3 grid((unsigned)((rows + BR_WAVES - 1) / BR_WAVES)), block(WAVE * BR_WAVES);
-  // 16-step runs halve the lane scans and wave sums per step; their 243 registers leave two waves per SIMD (at three,
-  // 66 spill): 303 against 323 us at 8 x 1536 x 2048.  For sequences that fill chunks of 1024 steps.
-  const int tail = p.len % 1024;
-  if (p.len % 16 == 0 && p.len >= 1024 && (tail == 0 || tail > 512)) {
-    if (p.z) hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, float, float, true, true, 16, 2>), grid, block, 0, s, p, nullptr, nullptr);
-    else hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, float, float, false, true, 16, 2>), grid, block, 0, s, p, nullptr, nullptr);
-  } else if (p.z) hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, float, float, true, true>), grid, block, 0, s, p, nullptr, nullptr);
-  else hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, float, float, false, true>), grid, block, 0, s, p, nullptr, nullptr);
+  const bool longs = scan_bwd_const_long(p.len, p.ragged);
+  const int T = longs ? 2 * FAST_T : FAST_T;
+  const size_t units = (size_t)p.batch * p.dim * (p.maps ? (p.len + T - 1) / T : 1);
+  const dim3 grid((unsigned)((units + BR_WAVES - 1) / BR_WAVES)), block(WAVE * BR_WAVES);
+  if (longs) {
+#define SSM_BR_KERNEL(HZ, R) scan_bwd_rowbc_kernel<io_t, float, float, HZ, R, true, 16, 2>
+    SSM_BR_LAUNCH(p, nullptr, nullptr);
+#undef SSM_BR_KERNEL
+  } else {
+#define SSM_BR_KERNEL(HZ, R) scan_bwd_rowbc_kernel<io_t, float, float, HZ, R, true>
+    SSM_BR_LAUNCH(p, nullptr, nullptr);
+#undef SSM_BR_KERNEL
+  }
   SSM_CHECK_LAUNCH("ssm_scan_bwd");
   return SSM_OK;
 }
 
 template <typename io_t, typename bc_t, typename out_t>
 static int launch_bwd_rowbc(const ScanBwdParams &p, void *dB, void *dC, hipStream_t s) {
-  const size_t rows = (size_t)p.batch * p.dim;
-  const dim3 grid((unsigned)((rows + BR_WAVES - 1) / BR_WAVES)), block(WAVE * BR_WAVES);
+  const size_t units = (size_t)p.batch * p.dim * (p.maps ? (p.len + FAST_T - 1) / FAST_T : 1);
+  const dim3 grid((unsigned)((units + BR_WAVES - 1) / BR_WAVES)), block(WAVE * BR_WAVES);
   out_t *b = reinterpret_cast<out_t *>(dB), *c = reinterpret_cast<out_t *>(dC);
-  if (p.z) hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, bc_t, out_t, true>), grid, block, 0, s, p, b, c);
-  else hipLaunchKernelGGL((scan_bwd_rowbc_kernel<io_t, bc_t, out_t, false>), grid, block, 0, s, p, b, c);
+#define SSM_BR_KERNEL(HZ, R) scan_bwd_rowbc_kernel<io_t, bc_t, out_t, HZ, R>
+  SSM_BR_LAUNCH(p, b, c);
+#undef SSM_BR_KERNEL
   SSM_CHECK_LAUNCH("ssm_scan_bwd");
   return SSM_OK;
 }
+#undef SSM_BR_LAUNCH
 
 }  // namespace ssm

@@ -15,6 +15,19 @@ extern template int scan_fwd_fast_dispatch<bf16_t, float>(const ScanFwdParams &,
 extern template int scan_fwd_fast_dispatch<f16_t, f16_t>(const ScanFwdParams &, int, hipStream_t);
 extern template int scan_fwd_fast_dispatch<f16_t, float>(const ScanFwdParams &, int, hipStream_t);
 
+// Rows up to which the chunks of a row run side by side in one workgroup (scan_fwd_split.hpp) rather than in turn; us at
+// 16 states in turn / side by side:
+//   grouped, 512 x 2048 float32 31.7 / 15.0, 1024 x 2048 38.3 / 25.9, 1024 x 8192 144 / 130, 1536 x 4096 76.5 / 101;
+//   bf16 512 x 2048 32.2 / 13.8, 1536 x 2048 34.3 / 30.0, 1536 x 8192 145 / 128, 2048 x 8192 150 / 152.
+//   Every wave reads B and C itself there, and runs of odd rows at a lower rate: 1024 x 2047 39 / 47, 512 x 2047 33 / 23.
+//   A group per channel: 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
+//   Constant projections: 256 x 2048 18.4 / 10.2, 512 x 8192 68 / 43, 512 x 1024 10.6 / 10.9, 1024 x 4096 41 / 43.
+static bool scan_fwd_splits(size_t rows, int len, bool varying, bool half, bool ragged) {
+  if (len <= FAST_T) return false;
+  if (!varying) return rows <= (len > 2 * FAST_T ? 512 : 384);
+  return rows <= (ragged ? 512 : half ? 1536 : 1024);
+}
+
 static bool valid_kind(int k) { return k == SSM_PROJ_DN || k == SSM_PROJ_BDN || k == SSM_PROJ_BGNL; }
 
 }  // namespace ssm
@@ -77,11 +90,15 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   int tune = SSM_RESERVED(a);               // 0 = automatic
   hipStream_t stream = reinterpret_cast<hipStream_t>(hip_stream);
 
-  // The specialised kernel: time-varying B and C of one element type (that of the activations, or fp32), at most
-  // 16 states, aligned rows of whole 16-step runs.  A selector of 100000 + v asks for its variant v.
-  const bool fast_ok = bvary && cvary && a->nstate <= FAST_N && p.vec_ok && a->seqlen % 16 == 0 &&
-                       aligned_to(a->Bproj, 4 * bs) && aligned_to(a->Cproj, 4 * bs) &&
-                       (a->bc_dtype == a->io_dtype || a->bc_dtype == SSM_F32);
+  // The specialised kernels: time-varying B and C of one element type (that of the activations, or fp32), at most
+  // 16 states.  Rows that are not aligned whole 16-step runs take their RAGGED form.  A selector of 100000 + v asks for
+  // variant v.
+  const bool whole_rows = p.vec_ok && a->seqlen % 16 == 0 && a->seqlen < (1 << 29) && (!bvary || aligned_to(a->Bproj, 4 * bs)) &&
+                          (!cvary || aligned_to(a->Cproj, 4 * bs));
+  const bool fast_ok = bvary && cvary && a->nstate <= FAST_N && (a->bc_dtype == a->io_dtype || a->bc_dtype == SSM_F32);
+  const bool const_ok = !bvary && !cvary && a->nstate <= FAST_N;
+  p.ragged = const_ok ? !(p.vec_ok && a->seqlen % 8 == 0 && a->seqlen < (1 << 29)) : !whole_rows;
+  p.split = scan_fwd_splits(rows_total, a->seqlen, !const_ok, a->io_dtype != SSM_F32, p.ragged);
   if (tune == 0 && fast_ok && a->seqlen > 256) {
     // The variant whose workgroups (48, 24 or 8 channels of one group) still give every CU its share:
     // two rows per wave with 16-step runs and two slabs where 256 such workgroups exist, else 8-step runs at six waves
@@ -91,20 +108,21 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
     // headline shape, where twice the bytes per step leave more to wait for); 16-bit: the 16-step runs (120.5 / 133.3)
     const int pref16[3] = {22123, 12121, 11082}, pref32[3] = {12121, 22123, 11082};
     const int *pref = a->io_dtype == SSM_F32 ? pref32 : pref16;
-    int pick = 0;
+    int pick = p.split ? 31041 : 0;
     for (int i = 0; i < 3 && !pick; ++i) {
       const int per_wg = scan_fwd_fast_rows(pref[i]);
       if (per_b % per_wg == 0 && per_c % per_wg == 0 && (total / per_wg >= 256 || i == 2)) pick = pref[i];
     }
-    // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave
-    if (!pick && aligned_to(a->Bproj, 16) && aligned_to(a->Cproj, 16) && ((size_t)a->seqlen * bs) % 16 == 0) pick = 31041;
-    if (pick) tune = 100000 + pick;
+    // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave, which reads its runs of
+    // B and C as 16-byte vectors
+    if (!pick) pick = 31041;
+    if (pick == 31041 && !(aligned_to(a->Bproj, 16) && aligned_to(a->Cproj, 16) && ((size_t)a->seqlen * bs) % 16 == 0)) p.ragged = 1;
+    tune = 100000 + pick;
   }
   // Projections constant in time, (D, N) or (B, D, N): a row per wave with B and C in lanes (variant 31042).
-  const bool const_ok = !bvary && !cvary && a->nstate <= FAST_N && p.vec_ok && a->seqlen % 8 == 0;
   if ((tune == 0 && const_ok && a->seqlen > 256) || tune == 100000 + 31042) {
-    SSM_REQUIRE(const_ok, SSM_ERR_BAD_KIND, "ssm_scan_fwd: selector %d needs constant projections, at most %d states "
-                "and aligned rows of whole 8-step runs", tune, FAST_N);
+    SSM_REQUIRE(const_ok, SSM_ERR_BAD_KIND, "ssm_scan_fwd: selector %d needs constant projections and at most %d states",
+                tune, FAST_N);
     switch (a->io_dtype) {
       case SSM_F32: return scan_fwd_fast_dispatch<float, float>(p, 31042, stream);
       case SSM_BF16: return scan_fwd_fast_dispatch<bf16_t, float>(p, 31042, stream);
@@ -116,6 +134,8 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
     const int v = tune - 100000, per_wg = scan_fwd_fast_rows(v);
     SSM_REQUIRE(per_wg > 0 && per_b % per_wg == 0 && per_c % per_wg == 0, SSM_ERR_BAD_KIND,
                 "ssm_scan_fwd: variant %d takes %d channels per workgroup, which must divide a group", v, per_wg);
+    SSM_REQUIRE(!p.ragged || !SSM_RESERVED(a) || per_wg == 1, SSM_ERR_BAD_KIND,
+                "ssm_scan_fwd: selector %d is for aligned rows of whole 16-step runs", tune);
     const bool bc32 = a->bc_dtype == SSM_F32;
     switch (a->io_dtype) {
       case SSM_F32: return scan_fwd_fast_dispatch<float, float>(p, v, stream);

@@ -1,7 +1,7 @@
 // Selective scan, forward: the kernel for the common call shape.
 //
-//   time-varying grouped B and C (B, G, N, L), N <= 16, rows of u / delta / z / out
-//   aligned to 16 bytes, L a multiple of 16.
+//   time-varying grouped B and C (B, G, N, L), N <= 16; rows of u / delta / z / out aligned to
+//   16 bytes and L a multiple of 16, or (RAGGED) rows of any length and start.
 //
 // Same decomposition as scan_fwd_kernel.hpp (time in chunks of 512 steps, a lane
 // owns a run of consecutive steps, per state a fold / lane scan / replay),
@@ -23,16 +23,16 @@ constexpr int FAST_N = 16;     // states held by the slab
 
 // [n][T] slab of one projection into LDS as fp32; a lane's K steps end up as K/4 float4
 // at [n][q][lane of the row] so that the reads of a wave are conflict-free.
-template <typename bc_t, int LPR>
-__device__ __forceinline__ void fast_stage(float *dst, const bc_t *src, int len, int t0, int nn, int nthreads) {
+// `room`: elements from src to the end of the tensor.
+template <typename bc_t, int LPR, bool RAGGED = false>
+__device__ __forceinline__ void fast_stage(float *dst, const bc_t *src, int len, int t0, int nn, int nthreads, size_t room) {
   constexpr int K = FAST_T / LPR, QT = FAST_T / 4;
   for (int e = threadIdx.x; e < nn * QT; e += nthreads) {
     const int nl = e / QT;
     const int tl = (e % QT) * 4;
     const int t = t0 + tl;
-    const bool inside = t < len;                       // len % 4 == 0: a group of four is inside or outside as a whole
-    const bc_t *at = src + (size_t)nl * len + (inside ? t : 0);
-    const Pack<bc_t, 4> raw = *reinterpret_cast<const Pack<bc_t, 4> *>(at);
+    const bool inside = RAGGED || t < len;             // not ragged: a group of four is inside or outside as a whole
+    const Pack<bc_t, 4> raw = load_steps<RAGGED, bc_t, 4>(src + (size_t)nl * len, t, len, t0 + FAST_T > len, room - (size_t)nl * len);
     float4 v;
     v.x = inside ? to_f32(raw.v[0]) : 0.0f;
     v.y = inside ? to_f32(raw.v[1]) : 0.0f;
@@ -107,7 +107,7 @@ __device__ __forceinline__ float group_read_lane(float v, int src, int lane) {
 // DB: two slabs in LDS (for variants of which one workgroup fills a CU): the slab of the next chunk is staged by
 // each wave as soon as it is done with its rows of this one, while slower waves still work, and a chunk costs
 // one barrier instead of two.
-template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB>
+template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED>
 __global__ __launch_bounds__(WAVE *WAVES) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void scan_fwd_fast_kernel(const ScanFwdParams p) {
   constexpr int T = FAST_T, K = T / LPR, SUBS = WAVE / LPR;
@@ -123,8 +123,10 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   const int b = (int)blockIdx.x / blocks_per_batch;
   const int d0 = ((int)blockIdx.x % blocks_per_batch) * rows;
   const int L = p.len, N = p.nstate;
-  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + ((size_t)b * p.b_groups + d0 / (p.dim / p.b_groups)) * (size_t)N * L;
-  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + ((size_t)b * p.c_groups + d0 / (p.dim / p.c_groups)) * (size_t)N * L;
+  const size_t bg = (size_t)b * p.b_groups + d0 / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d0 / (p.dim / p.c_groups);
+  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + bg * N * L;
+  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + cg * N * L;
+  const size_t Broom = ((size_t)p.batch * p.b_groups - bg) * N * L, Croom = ((size_t)p.batch * p.c_groups - cg) * N * L;
   const io_t *U = reinterpret_cast<const io_t *>(p.u), *DT = reinterpret_cast<const io_t *>(p.delta);
   const io_t *Z = reinterpret_cast<const io_t *>(p.z);
   io_t *Y = reinterpret_cast<io_t *>(p.out);
@@ -144,21 +146,19 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   for (int c = 0; c < nchunks; ++c) {
     const int t0 = c * T;
     const int t = t0 + sl * K;
-    const bool live = t < L;                 // L % K == 0: a lane's run is inside or outside as a whole
-    const int tc = live ? t : 0;
 
     if constexpr (DB) {
       if (c == 0) {
-        fast_stage<bc_t, LPR>(Bs, Bg, L, 0, N, WAVE * WAVES);
-        fast_stage<bc_t, LPR>(Cs, Cg, L, 0, N, WAVE * WAVES);
+        fast_stage<bc_t, LPR, RAGGED>(Bs, Bg, L, 0, N, WAVE * WAVES, Broom);
+        fast_stage<bc_t, LPR, RAGGED>(Cs, Cg, L, 0, N, WAVE * WAVES, Croom);
       }
       __syncthreads();           // slab c is complete; every wave is done with slab c - 1 (staged over below)
       Bs = tiles + (c & 1) * 2 * FAST_N * T;
       Cs = Bs + FAST_N * T;
     } else {
       __syncthreads();
-      fast_stage<bc_t, LPR>(Bs, Bg, L, t0, N, WAVE * WAVES);
-      fast_stage<bc_t, LPR>(Cs, Cg, L, t0, N, WAVE * WAVES);
+      fast_stage<bc_t, LPR, RAGGED>(Bs, Bg, L, t0, N, WAVE * WAVES, Broom);
+      fast_stage<bc_t, LPR, RAGGED>(Cs, Cg, L, t0, N, WAVE * WAVES, Croom);
       __syncthreads();
     }
 
@@ -166,13 +166,13 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
     for (int rr = 0; rr < RPW; ++rr) {
       const int d = d0 + (wave * RPW + rr) * SUBS + sub;
       const size_t row = (size_t)b * p.dim + d;
-      const size_t at = row * L + tc;
       float dl[K], du[K], y[K];
       Pack<io_t, K> zr;
       {
-        const Pack<io_t, K> ur = *reinterpret_cast<const Pack<io_t, K> *>(U + at);
-        const Pack<io_t, K> dr = *reinterpret_cast<const Pack<io_t, K> *>(DT + at);
-        if (p.z) zr = *reinterpret_cast<const Pack<io_t, K> *>(Z + at);
+        const size_t room = ((size_t)p.batch * p.dim - row) * L;
+        const Pack<io_t, K> ur = load_steps<RAGGED, io_t, K>(U + row * L, t, L, t0 + T > L, room);
+        const Pack<io_t, K> dr = load_steps<RAGGED, io_t, K>(DT + row * L, t, L, t0 + T > L, room);
+        if (p.z) zr = load_steps<RAGGED, io_t, K>(Z + row * L, t, L, t0 + T > L, room);
         if (p.chunk_states && sl < N) p.chunk_states[(row * nchunks + c) * (size_t)N + sl] = carry_lanes[rr];
 #pragma unroll
         for (int i = 0; i < K; ++i) dl[i] = to_f32(dr.v[i]) + bias[rr];
@@ -182,7 +182,7 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
         }
         if (t0 + T > L) {                      // only the last chunk can have lanes past the end: the identity map there
 #pragma unroll
-          for (int i = 0; i < K; ++i) dl[i] = live ? dl[i] : 0.0f;
+          for (int i = 0; i < K; ++i) dl[i] = t + (RAGGED ? i : 0) < L ? dl[i] : 0.0f;
         }
 #pragma unroll
         for (int i = 0; i < K; ++i) {
@@ -298,18 +298,16 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
           y[i] *= zz * rcp_hw(1.0f + exp2_hw(-LOG2E * zz));
         }
       }
-      if (live) {
-        Pack<io_t, K> o;
+      Pack<io_t, K> o;
 #pragma unroll
-        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(y[i]);
-        *reinterpret_cast<Pack<io_t, K> *>(Y + at) = o;
-      }
+      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(y[i]);
+      store_steps<RAGGED, io_t, K>(Y + row * L, t, L, o);
     }
     if constexpr (DB) {
       if (c + 1 < nchunks) {
         float *nb = tiles + ((c + 1) & 1) * 2 * FAST_N * T;
-        fast_stage<bc_t, LPR>(nb, Bg, L, t0 + T, N, WAVE * WAVES);
-        fast_stage<bc_t, LPR>(nb + FAST_N * T, Cg, L, t0 + T, N, WAVE * WAVES);
+        fast_stage<bc_t, LPR, RAGGED>(nb, Bg, L, t0 + T, N, WAVE * WAVES, Broom);
+        fast_stage<bc_t, LPR, RAGGED>(nb + FAST_N * T, Cg, L, t0 + T, N, WAVE * WAVES, Croom);
       }
     }
   }
@@ -332,7 +330,7 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
 // of the projections is read inside the loop.
 // K: steps per lane, 8 or 16; with 16 a chunk of the walk is two chunks of FAST_T steps and the state that enters
 // the second one (what lane 32 starts from) is written to chunk_states as well.
-template <typename io_t, typename bc_t, int WAVES, int OCC, bool CONST_BC = false, int K = 8>
+template <typename io_t, typename bc_t, int WAVES, int OCC, bool RAGGED, bool CONST_BC = false, int K = 8>
 __global__ __launch_bounds__(WAVE *WAVES) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
   constexpr int T = WAVE * K;
@@ -344,6 +342,8 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
   const int b = (int)(row / p.dim), d = (int)(row % p.dim);
   const int L = p.len, N = p.nstate;
   const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp), *Cg = reinterpret_cast<const bc_t *>(p.Cp);
+  size_t Broom = 0, Croom = 0;                               // elements to the ends of the tensors
+  const size_t room = ((size_t)p.batch * p.dim - row) * L;
   float B_lanes = 0.0f, C_lanes = 0.0f;
   if constexpr (CONST_BC) {
     if (lane < N) {
@@ -351,8 +351,11 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
       C_lanes = load_as_f32(p.Cp, p.bc_dtype, (p.c_kind == SSM_PROJ_BDN ? row : (size_t)d) * N + lane);
     }
   } else {
-    Bg += ((size_t)b * p.b_groups + d / (p.dim / p.b_groups)) * (size_t)N * L;
-    Cg += ((size_t)b * p.c_groups + d / (p.dim / p.c_groups)) * (size_t)N * L;
+    const size_t bg = (size_t)b * p.b_groups + d / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d / (p.dim / p.c_groups);
+    Bg += bg * N * L;
+    Cg += cg * N * L;
+    Broom = ((size_t)p.batch * p.b_groups - bg) * N * L;
+    Croom = ((size_t)p.batch * p.c_groups - cg) * N * L;
   }
   const io_t *U = reinterpret_cast<const io_t *>(p.u), *DT = reinterpret_cast<const io_t *>(p.delta);
   const io_t *Z = reinterpret_cast<const io_t *>(p.z);
@@ -366,20 +369,18 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
   const int state_chunks = (L + FAST_T - 1) / FAST_T;         // rows of chunk_states per (batch, channel)
   for (int c = 0; c < nchunks; ++c) {
     const int t = c * T + lane * K;
-    const bool live = t < L;
-    const int tc = live ? t : 0;
-    const size_t at = row * L + tc;
+    const bool tail = (c + 1) * T > L;
     float dl[K], du[K], y[K];
     Pack<io_t, K> zr;
     Pack<bc_t, K> braw, craw;
     if constexpr (!CONST_BC) {
-      braw = *reinterpret_cast<const Pack<bc_t, K> *>(Bg + tc);
-      craw = *reinterpret_cast<const Pack<bc_t, K> *>(Cg + tc);
+      braw = load_steps<RAGGED, bc_t, K>(Bg, t, L, tail, Broom);
+      craw = load_steps<RAGGED, bc_t, K>(Cg, t, L, tail, Croom);
     }
     {
-      const Pack<io_t, K> ur = *reinterpret_cast<const Pack<io_t, K> *>(U + at);
-      const Pack<io_t, K> dr = *reinterpret_cast<const Pack<io_t, K> *>(DT + at);
-      if (p.z) zr = *reinterpret_cast<const Pack<io_t, K> *>(Z + at);
+      const Pack<io_t, K> ur = load_steps<RAGGED, io_t, K>(U + row * L, t, L, tail, room);
+      const Pack<io_t, K> dr = load_steps<RAGGED, io_t, K>(DT + row * L, t, L, tail, room);
+      if (p.z) zr = load_steps<RAGGED, io_t, K>(Z + row * L, t, L, tail, room);
       if (p.chunk_states && lane < N) p.chunk_states[(row * state_chunks + c * (T / FAST_T)) * (size_t)N + lane] = carry_lanes;
 #pragma unroll
       for (int i = 0; i < K; ++i) dl[i] = to_f32(dr.v[i]) + bias;
@@ -390,7 +391,7 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
 #pragma unroll
       for (int i = 0; i < K; ++i) {
         const float uu = to_f32(ur.v[i]);
-        dl[i] = live ? dl[i] : 0.0f;
+        dl[i] = t + (RAGGED ? i : 0) < L ? dl[i] : 0.0f;
         du[i] = dl[i] * uu;
         y[i] = Dk * uu;
       }
@@ -405,8 +406,8 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
       Pack<bc_t, K> bnext, cnext;
       float bq[K], cq[K];
       if constexpr (!CONST_BC) {
-        bnext = *reinterpret_cast<const Pack<bc_t, K> *>(Bg + (size_t)nn * L + tc);
-        cnext = *reinterpret_cast<const Pack<bc_t, K> *>(Cg + (size_t)nn * L + tc);
+        bnext = load_steps<RAGGED, bc_t, K>(Bg + (size_t)nn * L, t, L, tail, Broom - (size_t)nn * L);
+        cnext = load_steps<RAGGED, bc_t, K>(Cg + (size_t)nn * L, t, L, tail, Croom - (size_t)nn * L);
 #pragma unroll
         for (int i = 0; i < K; ++i) {
           bq[i] = to_f32(braw.v[i]);
@@ -460,30 +461,38 @@ void scan_fwd_rowbc_kernel(const ScanFwdParams p) {
         y[i] *= zz * rcp_hw(1.0f + exp2_hw(-LOG2E * zz));
       }
     }
-    if (live) {
-      Pack<io_t, K> o;
+    Pack<io_t, K> o;
 #pragma unroll
-      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(y[i]);
-      *reinterpret_cast<Pack<io_t, K> *>(Y + at) = o;
-    }
+    for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(y[i]);
+    store_steps<RAGGED, io_t, K>(Y + row * L, t, L, o);
   }
   if (p.last && lane < N) reinterpret_cast<io_t *>(p.last)[row * N + lane] = from_f32<io_t>(carry_lanes);
 }
+
+// Rows of any length and start take the RAGGED form of a kernel: the same walk, with the run that crosses the end of a
+// row read and written by element.
+#define SSM_RAGGED_LAUNCH(p, KERNEL, grid, block, lds, stream)                       \
+  do {                                                                                \
+    if ((p).ragged) hipLaunchKernelGGL((KERNEL(true)), grid, block, lds, stream, p);  \
+    else hipLaunchKernelGGL((KERNEL(false)), grid, block, lds, stream, p);            \
+  } while (0)
 
 template <typename io_t, typename bc_t>
 static int launch_scan_fwd_rowbc(const ScanFwdParams &p, hipStream_t stream) {
   constexpr int WAVES = 4;
   const size_t rows = (size_t)p.batch * p.dim;
-  hipLaunchKernelGGL((scan_fwd_rowbc_kernel<io_t, bc_t, WAVES, 6>), dim3((unsigned)((rows + WAVES - 1) / WAVES)),
-                     dim3(WAVE * WAVES), 0, stream, p);
+  const dim3 grid((unsigned)((rows + WAVES - 1) / WAVES)), block(WAVE * WAVES);
+#define SSM_K(R) scan_fwd_rowbc_kernel<io_t, bc_t, WAVES, 6, R>
+  SSM_RAGGED_LAUNCH(p, SSM_K, grid, block, 0, stream);
+#undef SSM_K
   SSM_CHECK_LAUNCH("ssm_scan_fwd");
   return SSM_OK;
 }
 
-template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB = false>
-static int launch_scan_fwd_fast(const ScanFwdParams &p, hipStream_t stream) {
+template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED>
+static int launch_scan_fwd_fast_as(const ScanFwdParams &p, hipStream_t stream) {
   const size_t lds = (size_t)(DB ? 4 : 2) * FAST_N * FAST_T * sizeof(float);
-  auto kernel = scan_fwd_fast_kernel<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB>;
+  auto kernel = scan_fwd_fast_kernel<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, RAGGED>;
   if (allow_dynamic_lds(kernel, lds) != hipSuccess) {
     (void)hipGetLastError();
     set_error("ssm_scan_fwd: cannot reserve %zu bytes of LDS", lds);
@@ -495,19 +504,35 @@ static int launch_scan_fwd_fast(const ScanFwdParams &p, hipStream_t stream) {
   return SSM_OK;
 }
 
+template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB = false>
+static int launch_scan_fwd_fast(const ScanFwdParams &p, hipStream_t stream) {
+  return p.ragged ? launch_scan_fwd_fast_as<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, true>(p, stream)
+                  : launch_scan_fwd_fast_as<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, false>(p, stream);
+}
+
 template <typename io_t>
 static int launch_scan_fwd_row_const(const ScanFwdParams &p, hipStream_t stream) {
   constexpr int WAVES = 4;
   const size_t rows = (size_t)p.batch * p.dim;
   const dim3 grid((unsigned)((rows + WAVES - 1) / WAVES)), block(WAVE * WAVES);
   const int tail = p.len % (2 * FAST_T);
-  if (p.len % 16 == 0 && p.len >= 2 * FAST_T && (tail == 0 || tail > FAST_T))
-    hipLaunchKernelGGL((scan_fwd_rowbc_kernel<io_t, float, WAVES, 4, true, 16>), grid, block, 0, stream, p);
+#define SSM_K16(R) scan_fwd_rowbc_kernel<io_t, float, WAVES, 4, R, true, 16>
+#define SSM_K8(R) scan_fwd_rowbc_kernel<io_t, float, WAVES, 6, R, true>
+  if ((p.ragged || p.len % 16 == 0) && p.len >= 2 * FAST_T && (tail == 0 || tail > FAST_T))
+    SSM_RAGGED_LAUNCH(p, SSM_K16, grid, block, 0, stream);
   else
-    hipLaunchKernelGGL((scan_fwd_rowbc_kernel<io_t, float, WAVES, 6, true>), grid, block, 0, stream, p);
+    SSM_RAGGED_LAUNCH(p, SSM_K8, grid, block, 0, stream);
+#undef SSM_K16
+#undef SSM_K8
   SSM_CHECK_LAUNCH("ssm_scan_fwd");
   return SSM_OK;
 }
+
+}  // namespace ssm
+
+#include "scan_fwd_split.hpp"
+
+namespace ssm {
 
 // Channels per workgroup of a variant; 0 for an unknown one.
 // variant = 10000 * (rows a wave walks at once) + 1000 * (rows a wave walks in turn) + 10 * waves + states in flight
@@ -526,14 +551,14 @@ inline int scan_fwd_fast_rows(int variant) {
 template <typename io_t, typename bc_t>
 int scan_fwd_fast_dispatch(const ScanFwdParams &p, int variant, hipStream_t s) {
   switch (variant) {
-    case 13082: return launch_scan_fwd_fast<io_t, bc_t, 64, 3, 8, 2, 4>(p, s);     // 4 waves per SIMD
+    case 13082: return launch_scan_fwd_fast_as<io_t, bc_t, 64, 3, 8, 2, 4, false, false>(p, s);     // 4 waves per SIMD
     case 12121: return launch_scan_fwd_fast<io_t, bc_t, 64, 2, 12, 1, 6>(p, s);    // 6 waves per SIMD
     case 11082: return launch_scan_fwd_fast<io_t, bc_t, 64, 1, 8, 2, 4>(p, s);
-    case 22121: return launch_scan_fwd_fast<io_t, bc_t, 32, 2, 12, 1, 3>(p, s);    // 3 waves per SIMD, 16-step runs
+    case 22121: return launch_scan_fwd_fast_as<io_t, bc_t, 32, 2, 12, 1, 3, false, false>(p, s);    // 3 waves per SIMD, 16-step runs
     case 22123: return launch_scan_fwd_fast<io_t, bc_t, 32, 2, 12, 1, 3, true>(p, s);   // the same with two slabs
-    case 21081: return launch_scan_fwd_fast<io_t, bc_t, 32, 1, 8, 1, 4>(p, s);
-    case 31041: return launch_scan_fwd_rowbc<io_t, bc_t>(p, s);
-    case 31042: return launch_scan_fwd_row_const<io_t>(p, s);
+    case 21081: return launch_scan_fwd_fast_as<io_t, bc_t, 32, 1, 8, 1, 4, false, false>(p, s);
+    case 31041: return p.split ? launch_scan_fwd_split<io_t, bc_t, false>(p, s) : launch_scan_fwd_rowbc<io_t, bc_t>(p, s);
+    case 31042: return p.split ? launch_scan_fwd_split<io_t, float, true>(p, s) : launch_scan_fwd_row_const<io_t>(p, s);
     default:
       set_error("ssm_scan_fwd: unknown variant %d of the specialised kernel", variant);
       return SSM_ERR_BAD_KIND;

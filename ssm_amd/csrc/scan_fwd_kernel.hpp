@@ -38,7 +38,23 @@ struct ScanFwdParams {
   int softplus;
   int vec_ok;     // rows of u/delta/z/out are 16-byte aligned
   int bc_vec_ok;  // rows of B/C allow 4-element vector loads
+  int ragged;     // specialised kernels: rows are not whole aligned runs
+  int split;      // row-per-wave kernels: the chunks of a row side by side (scan_fwd_split.hpp)
 };
+
+// `v` through the chunk maps (scan_bwd_maps.hpp) of `count` chunks, the first at `m`, `step` elements apart; eight are
+// requested together.
+__device__ __forceinline__ float compose_maps(const float2 *m, int count, ptrdiff_t step, float v) {
+  for (int k = 0; k < count; k += 8) {
+    float2 f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = m[(ptrdiff_t)min(k + j, count - 1) * step];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (k + j < count) v = __builtin_fmaf(f[j].x, v, f[j].y);
+  }
+  return v;
+}
 
 // Copy the [nn][T] slab of one time-varying projection into LDS as fp32.
 // src_off is the element offset of (b, g, nb, 0); rows are `len` apart.

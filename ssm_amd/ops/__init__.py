@@ -150,9 +150,9 @@ def _scan_backward(grad_out, grad_last, u, delta, A, B, C, D, z, dt_bias, softpl
     """Run ``ssm_scan_bwd``; returns fp32/io-dtype gradients in input order
     ``(du, ddelta, dA, dB, dC, dD, dz, ddt_bias)``.  State sizes above 16 are
     processed in blocks of 16 states (the recurrence is independent per state and
-    every gradient is additive over states).  With ``grads_in_input_dtype``, ``dB`` and ``dC`` of projections that
-    every channel has for itself, ``(B, D, N, L)``, come back in the projections' own type where the kernel for
-    that form writes them (no float32 tensors of that size, and no cast of them afterwards)."""
+    every gradient is additive over states).  With ``grads_in_input_dtype``, ``dB`` and ``dC`` of
+    projections that vary in time come back in the projections' own type (no float32 tensors of that size, and no
+    cast of them afterwards)."""
     if K.f64_compute(u, A):
         from . import _f64
         return _f64.scan_backward(grad_out, grad_last, u, delta, A, B, C, D, z, dt_bias, softplus)
@@ -208,9 +208,8 @@ def _scan_backward(grad_out, grad_last, u, delta, A, B, C, D, z, dt_bias, softpl
             batch=batch, dim=dim, seqlen=length, nstate=n_blk, io_dtype=_lib.dtype_enum(io),
             bc_dtype=_lib.dtype_enum(bc), b_kind=bkind, c_kind=ckind, b_groups=bgroups, c_groups=cgroups,
             delta_softplus=int(bool(softplus)), reserved=int(tune_items))
-        # projections of their own per channel: no partial sums of dB and dC, and their own type on request
-        nbytes = int((_lib.load_test_hooks() if tune_items else lib).ssm_scan_bwd_per_row_workspace_bytes(args))
-        g_dtype = bc if (nbytes and grads_in_input_dtype and single) else torch.float32
+        vary = bkind == ckind == _lib.PROJ_BGNL
+        g_dtype = bc if (vary and grads_in_input_dtype and single) else torch.float32
         dB_b, dC_b = (torch.empty(B_b.shape, dtype=g_dtype, device=dev), torch.empty(C_b.shape, dtype=g_dtype, device=dev))
         args.dB, args.dC, args.dbc_dtype = _lib.ptr(dB_b), _lib.ptr(dC_b), _lib.dtype_enum(g_dtype)
         if single:
@@ -218,8 +217,7 @@ def _scan_backward(grad_out, grad_last, u, delta, A, B, C, D, z, dt_bias, softpl
         elif dB is None:
             dB = torch.empty(B_c.shape, dtype=torch.float32, device=dev)
             dC = torch.empty(C_c.shape, dtype=torch.float32, device=dev)
-        if not nbytes:
-            nbytes = lib.ssm_scan_bwd_workspace_bytes(batch, dim, length, n_blk, bkind, ckind, bgroups, cgroups)
+        nbytes = int((_lib.load_test_hooks() if tune_items else lib).ssm_scan_bwd_full_workspace_bytes(args))
         ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=dev)
         args.workspace, args.workspace_bytes = (ws.data_ptr() + 255) // 256 * 256, nbytes
         _lib.call("ssm_scan_bwd", args, dev)

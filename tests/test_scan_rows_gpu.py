@@ -1,0 +1,83 @@
+"""Scan rows that are no whole aligned runs, and calls of few rows whose chunks run side by side: forward and backward
+against float64 autograd through the oracle, at the edges of runs (8 and 16 steps), chunks (512 steps), the walks of
+1024 steps and the eight chunks a workgroup takes at once; and the end of a tensor, which no read may pass."""
+
+import pytest
+import torch
+
+from oracle import ops_oracle as O
+from tests.test_scan_fwd_gpu import make_inputs
+
+pytestmark = pytest.mark.gpu
+NAMES = ("u", "delta", "A", "B", "C", "D", "z", "dt_bias")
+
+
+def _close(a, b, half, what, scale_tol):
+    a, b = a.detach().double().cpu(), b.detach().double()
+    scale = float(b.abs().max()) + 1e-30
+    tol = dict(rtol=2e-2, atol=4e-3 * scale) if half else dict(rtol=1e-3, atol=scale_tol * scale)
+    torch.testing.assert_close(a, b, **tol, msg=lambda m: f"{what}: {m}")
+
+
+@pytest.mark.parametrize("kind", ["grouped", "own", "dn"])
+@pytest.mark.parametrize("length,dim,dtype,use_z", [
+    (511, 16, torch.float32, True), (513, 48, torch.bfloat16, True), (519, 16, torch.float16, False),
+    (1021, 96, torch.bfloat16, True), (1025, 16, torch.float32, True), (1543, 24, torch.float32, True),
+    (4097, 16, torch.float32, False), (4608, 16, torch.bfloat16, True)])
+def test_rows_of_any_length(kind, length, dim, dtype, use_z):
+    from ssm_amd import ops
+    if kind == "own" and length > 2048:
+        length = length % 2048 + 520
+    kw = dict(groups=dim) if kind == "own" else dict(groups=1) if kind == "grouped" else dict(bkind="dn", ckind="dn")
+    inp = make_inputs(length, 2, dim, length, 16, dtype=dtype, bc_dtype=torch.float32 if kind == "dn" else dtype, use_z=use_z, **kw)
+    g = torch.Generator().manual_seed(1)
+    go, gl = torch.randn(2, dim, length, generator=g).to(dtype), torch.randn(2, dim, 16, generator=g).to(dtype)
+    got = {k: (None if v is None else v.cuda().requires_grad_(True)) for k, v in inp.items()}
+    want = {k: (None if v is None else v.double().requires_grad_(True)) for k, v in inp.items()}
+    y, h = ops.selective_scan(*(got[k] for k in NAMES[:5]), D=got["D"], z=got["z"], dt_bias=got["dt_bias"], softplus=True,
+                              return_last_state=True)
+    yr, hr = O.selective_scan(*(want[k] for k in NAMES[:5]), D=want["D"], z=want["z"], dt_bias=want["dt_bias"], softplus=True,
+                              return_last_state=True, acc=torch.float64)
+    half = dtype != torch.float32
+    _close(y, yr, half, "y", 1e-5)
+    _close(h, hr, half, "last state", 1e-5)
+    with torch.no_grad():
+        y0 = ops.selective_scan(*(got[k] for k in NAMES[:5]), D=got["D"], z=got["z"], dt_bias=got["dt_bias"], softplus=True)
+    assert torch.equal(y0, y)
+    torch.autograd.backward([y, h], [go.cuda(), gl.cuda()])
+    torch.autograd.backward([yr, hr], [go.double(), gl.double()])
+    for k in NAMES:
+        if want[k] is not None:
+            _close(got[k].grad, want[k].grad, half and got[k].dtype == dtype, f"grad {k}", 1e-4)
+
+
+def test_many_rows_of_odd_length_walk_their_chunks_in_turn():
+    """Enough rows that no chunk runs beside another (workgroups of 8 channels forward, of 16 backward): the same
+    numbers as the first rows computed alone, which take the other kernels."""
+    from ssm_amd import ops
+    inp = make_inputs(7, 4, 1040, 521, 16, dtype=torch.float32, groups=1)
+    go = torch.randn(4, 1040, 521, generator=torch.Generator().manual_seed(2)).cuda()
+
+    def run(batch):
+        t = {k: (v[:batch] if k in ("u", "delta", "z", "B", "C") else v).cuda().requires_grad_(True) for k, v in inp.items()}
+        y = ops.selective_scan(*(t[k] for k in NAMES[:5]), D=t["D"], z=t["z"], dt_bias=t["dt_bias"], softplus=True)
+        y.backward(go[:batch].contiguous())
+        return [y] + [t[k].grad for k in ("u", "delta", "z", "B", "C")]
+    for a, b, what in zip(run(4), run(1), ("y", "u", "delta", "z", "B", "C")):
+        scale = float(b.detach().abs().max())
+        torch.testing.assert_close(a[:1], b, rtol=1e-4, atol=2e-5 * scale, msg=lambda m: f"{what}: {m}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_what_lies_past_a_row_never_enters_it(dtype):
+    """The row after next holds infinities: steps past the end of a row are read with it and must count for nothing."""
+    from ssm_amd import ops
+    inp = make_inputs(3, 2, 16, 515, 16, dtype=dtype, groups=1)
+    t = {k: (None if v is None else v.cuda()) for k, v in inp.items()}
+    call = lambda: ops.selective_scan(*(t[k] for k in NAMES[:5]), D=t["D"], z=t["z"], dt_bias=t["dt_bias"], softplus=True,
+                                      return_last_state=True)
+    y, h = call()
+    for k in ("u", "delta", "z", "B", "C"):
+        t[k][1] = float("inf")
+    y2, h2 = call()
+    assert torch.equal(y2[0], y[0]) and torch.equal(h2[0], h[0])
