@@ -63,6 +63,21 @@ inline hipError_t allow_dynamic_lds(KernelT kernel, size_t bytes) {
 void launch_fold_rows(const float *in, float *out, int count, size_t inner, hipStream_t s);
 void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_t inner, hipStream_t s);
 
+// All sums that a backward call ends with, in one launch of workgroup ranges per job (scan_bwd.hip):
+//   out[o][i] = sum_{j < count} in[(o * count + j) * inner + i], added in order of j, written as `dtype`.
+// As launches of their own, with the casts behind them, they took 5 to 10 us each, of which the gaps were half.
+constexpr int FOLD_JOBS = 5;
+struct FoldJobs {
+  const float *in[FOLD_JOBS];
+  void *out[FOLD_JOBS];
+  size_t outer[FOLD_JOBS], inner[FOLD_JOBS];
+  int count[FOLD_JOBS], dtype[FOLD_JOBS], width[FOLD_JOBS];     // width: outputs per thread, 1 or 4
+  unsigned first_block[FOLD_JOBS + 1];
+  int n;
+  void add(const float *in, void *out, size_t outer, int count, size_t inner, int dtype);
+};
+void launch_fold_jobs(const FoldJobs &jobs, hipStream_t s);
+
 // -------------------------------------------------------------- device side
 
 constexpr int WAVE = 64;

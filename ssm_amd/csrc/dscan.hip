@@ -11,7 +11,7 @@
 //           the segments before it, then replays its steps and emits y
 // which costs one extra read of X/dt/B but fills the device even when B*H*P is
 // small.  dt is used as given (no bias, no softplus), as in the reference.
-#include "common.hpp"
+#include "dscan_maps.hpp"
 
 #include <type_traits>
 
@@ -34,6 +34,9 @@ struct DscanParams {
   int z_per_p;                  // 1 for z (B,L,H,P), 0 for z (B,L,H)
   int seg_len, nseg;
   float *round_states;          // (B, ceil(L/64), HP): the state entering every 64 steps, or null (one-pass kernel)
+  // one-pass kernel: rounds per segment, and the maps of the segments (null: one segment, all of time)
+  int seg_rounds;
+  const float2 *maps;
 };
 
 __device__ __forceinline__ void ds_store(void *p, int dtype, size_t i, float v) {
@@ -214,6 +217,17 @@ __global__ __launch_bounds__(WAVE *DO_WAVES) void dscan_onepass_kernel(const Dsc
   };
 
   const int rounds = (L + DO_ROUND - 1) / DO_ROUND;
+  const int seg = blockIdx.z, r_first = seg * p.seg_rounds, r_end = min(rounds, r_first + p.seg_rounds);
+  if (wave == DO_WAVES - 1) {
+    // the state entering the segment, where a round leaves its own for the next (visible after the round's barrier)
+    float first[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) {
+      first[v] = p.init ? load_as_f32(p.init, p.init_dtype, (size_t)b * HP + ch + v) : 0.0f;
+      if (p.maps) first[v] = dscan_compose(p.maps + (size_t)b * gridDim.z * HP + ch + v, seg, HP, first[v]);
+    }
+    right[(r_first & 1) ^ 1][lane] = make_float2(first[0], first[VEC - 1]);
+  }
   auto round_of = [&](DoRegs<io_t, VEC> &cur, int r) {
     const int q = r & 1;
     const int t0 = r * DO_ROUND + wave * DO_SEG;
@@ -250,14 +264,9 @@ __global__ __launch_bounds__(WAVE *DO_WAVES) void dscan_onepass_kernel(const Dsc
     __syncthreads();
     // the state entering this wave's steps: the folds of the waves before it, from the state entering the round
     float enter[VEC];
-    if (r == 0) {
-#pragma unroll
-      for (int v = 0; v < VEC; ++v) enter[v] = p.init ? load_as_f32(p.init, p.init_dtype, (size_t)b * HP + ch + v) : 0.0f;
-    } else {
-      const float2 c = right[q ^ 1][lane];
-      enter[0] = c.x;
-      enter[VEC - 1] = c.y;
-    }
+    const float2 c = right[q ^ 1][lane];
+    enter[0] = c.x;
+    enter[VEC - 1] = c.y;
     for (int w = 0; w < wave; ++w) {
       const float4 f = segs[q][w][lane];
 #pragma unroll
@@ -306,20 +315,42 @@ __global__ __launch_bounds__(WAVE *DO_WAVES) void dscan_onepass_kernel(const Dsc
 
   // two sets of registers take turns: one is worked on while the other's reads are in flight
   DoRegs<io_t, VEC> ra, rb;
-  request(ra, 0);
-  for (int r = 0; r < rounds; r += 2) {
-    if (r + 1 < rounds) request(rb, r + 1);
+  request(ra, r_first);
+  for (int r = r_first; r < r_end; r += 2) {
+    if (r + 1 < r_end) request(rb, r + 1);
     round_of(ra, r);
-    if (r + 1 < rounds) {
-      if (r + 2 < rounds) request(ra, r + 2);
+    if (r + 1 < r_end) {
+      if (r + 2 < r_end) request(ra, r + 2);
       round_of(rb, r + 1);
     }
   }
 }
 
+// Cut a one-pass walk into segments when few workgroups share it; p.fold has room for p.nseg maps per channel.
 template <typename io_t, int VEC>
-static void launch_onepass(const DscanParams &p, bool params, hipStream_t s) {
-  const dim3 grid((unsigned)((size_t)p.heads * p.proj / (WAVE * VEC)), (unsigned)p.batch);
+static dim3 onepass_grid(DscanParams &p, bool params, hipStream_t s) {
+  const unsigned blocks = (unsigned)((size_t)p.heads * p.proj / (WAVE * VEC));
+  const int rounds = (p.len + DO_ROUND - 1) / DO_ROUND;
+  // 1.7 us a round: 29 us for the 16 rounds of 2048 steps by 32 workgroups
+  p.seg_rounds = dscan_rounds_per_segment((size_t)blocks * p.batch, rounds, 1.7);
+  int nseg = (rounds + p.seg_rounds - 1) / p.seg_rounds;
+  if (nseg > p.nseg) p.seg_rounds = rounds, nseg = 1;
+  p.maps = nullptr;
+  if (nseg > 1) {
+    DscanMapParams m{};
+    m.drive = p.X; m.dt = p.dt; m.proj = p.Bp; m.A = p.A; m.lengths = p.lengths; m.maps = reinterpret_cast<float2 *>(p.fold);
+    m.batch = p.batch; m.len = p.len; m.heads = p.heads; m.width = p.proj;
+    m.proj_dtype = p.bc_dtype; m.a_stride_p = p.a_stride_p; m.proj_stride_b = p.b_stride_b;
+    m.seg_len = p.seg_rounds * DO_ROUND; m.nseg = nseg;
+    params ? launch_dscan_maps<io_t, VEC, false, true>(m, s) : launch_dscan_maps<io_t, VEC, false, false>(m, s);
+    p.maps = m.maps;
+  }
+  return dim3(blocks, (unsigned)p.batch, (unsigned)nseg);
+}
+
+template <typename io_t, int VEC>
+static void launch_onepass(DscanParams &p, bool params, hipStream_t s) {
+  const dim3 grid = onepass_grid<io_t, VEC>(p, params, s);
   const dim3 block(WAVE * DO_WAVES);
   if (params) {
     if (p.z) hipLaunchKernelGGL((dscan_onepass_kernel<io_t, VEC, true, false, true>), grid, block, 0, s, p);
@@ -331,20 +362,22 @@ static void launch_onepass(const DscanParams &p, bool params, hipStream_t s) {
 }
 
 // The table of round states alone, for a call shape the one-pass kernels cover (the caller has checked).
-// b_const: B is one value per channel, (H,P) (b_stride_b 0) or (B,H,P) (b_stride_b H*P), of type bc_dtype.
+// b_const: B is one value per channel, (H,P) (b_stride_b 0) or (B,H,P) (b_stride_b H*P), of type bc_dtype.  maps: room
+// for nseg of them per channel.
 void launch_dscan_round_states(const void *X, const void *dt, const void *Bproj, const float *A, const void *init,
                                int init_dtype, const int *lengths, float *round_states, int batch, int len, int heads,
                                int proj, int x_dtype, bool b_const, int bc_dtype, long long b_stride_b, bool a_per_p,
-                               hipStream_t s) {
+                               float2 *maps, int nseg, hipStream_t s) {
   DscanParams p{};
+  p.fold = reinterpret_cast<float *>(maps); p.nseg = nseg;
   p.X = X; p.dt = dt; p.Bp = Bproj; p.Cp = Bproj; p.A = A; p.init = init; p.init_dtype = init_dtype;
   p.lengths = lengths; p.round_states = round_states;
   p.batch = batch; p.len = len; p.heads = heads; p.proj = proj;
   p.bc_dtype = bc_dtype; p.b_stride_b = p.c_stride_b = b_stride_b; p.a_stride_p = a_per_p ? 1 : 0;
-  const int vec = x_dtype == SSM_F32 ? 1 : 2;
-  const dim3 grid((unsigned)((size_t)heads * proj / (WAVE * vec)), (unsigned)batch), block(WAVE * DO_WAVES);
+  const dim3 block(WAVE * DO_WAVES);
 #define SSM_STATES(T, V)                                                                                    \
   {                                                                                                         \
+    const dim3 grid = onepass_grid<T, V>(p, b_const, s);                                                    \
     if (b_const) hipLaunchKernelGGL((dscan_onepass_kernel<T, V, false, true, true>), grid, block, 0, s, p); \
     else hipLaunchKernelGGL((dscan_onepass_kernel<T, V, false, true, false>), grid, block, 0, s, p);        \
   }

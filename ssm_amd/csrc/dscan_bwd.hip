@@ -15,8 +15,9 @@
 // rebuilds what enters a segment from both sides out of those folds, sweeps forward storing the
 // states, then sweeps backward producing every gradient.  Sums over channels, batch, segments or time
 // beyond a thread's own loop are written as partials and folded in a fixed order.
-#include "common.hpp"
+#include "dscan_maps.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ssm {
@@ -29,7 +30,7 @@ int dscan_segments(int batch, int len, int hp);   // dscan.hip: the forward's ch
 void launch_dscan_round_states(const void *X, const void *dt, const void *Bproj, const float *A, const void *init,
                                int init_dtype, const int *lengths, float *round_states, int batch, int len, int heads,
                                int proj, int x_dtype, bool b_const, int bc_dtype, long long b_stride_b, bool a_per_p,
-                               hipStream_t s);
+                               float2 *maps, int nseg, hipStream_t s);
 
 struct DscanBwdParams {
   const void *gy, *X, *dt, *Bp, *Cp, *z, *init;
@@ -53,6 +54,8 @@ struct DscanBwdParams {
   long long b_stride_b, b_stride_t, c_stride_b, c_stride_t;
   int z_per_p;
   int seg_len, nseg;
+  int seg_rounds;                 // one-pass kernel: rounds per segment, and the maps of the segments (null: one)
+  const float2 *maps;
 };
 
 __device__ __forceinline__ void db_store(void *p, int dtype, size_t i, float v) {
@@ -372,34 +375,41 @@ extern "C" int ssm_dscan_bwd(const ssm_dscan_bwd_args *a, void *hip_stream) {
     p.round_states = a->round_states ? const_cast<float *>(a->round_states) : ws;
     // per-channel sums of a batch row, (B, HP) each; those that are the caller's gradient already go there
     float *sums = ws + (size_t)Bn * rounds * HP;
+    // 2.3 us a round: 75 us for the 32 rounds of 2048 steps by 32 workgroups
+    p.seg_rounds = dscan_rounds_per_segment((size_t)Bn * (HP / (WAVE * vec)), rounds, 2.3);
+    const int segs = (rounds + p.seg_rounds - 1) / p.seg_rounds, copies = segs * Bn;
+    const size_t each = (size_t)copies * HP;
+    SSM_REQUIRE((size_t)Bn * rounds * HP + 4 * each + 2 * bhp * std::max(segs, nseg) + 1 <= a->workspace_bytes / 4, SSM_ERR_WORKSPACE, "ssm_dscan_bwd: workspace too small");
     p.pA = sums;
-    p.pD = sums + bhp;
-    p.pB = (constant && a->b_kind == SSM_CHUNK_BHP) ? reinterpret_cast<float *>(a->dB) : sums + 2 * bhp;
-    p.pC = (constant && a->c_kind == SSM_CHUNK_BHP) ? reinterpret_cast<float *>(a->dC) : sums + 3 * bhp;
-    float *head_tmp = sums + 4 * bhp;                      // (HP) on the way to a per-head sum
+    p.pD = sums + each;
+    const bool b_direct = constant && a->b_kind == SSM_CHUNK_BHP && segs == 1, c_direct = constant && a->c_kind == SSM_CHUNK_BHP && segs == 1;
+    p.pB = b_direct ? reinterpret_cast<float *>(a->dB) : sums + 2 * each;
+    p.pC = c_direct ? reinterpret_cast<float *>(a->dC) : sums + 3 * each;
+    float *after = sums + 4 * each;
+    float2 *maps = reinterpret_cast<float2 *>(after + (aligned_to(after, 8) ? 0 : 1));
     p.ddt_direct = a->ddt;
     if (a->round_states == nullptr)                      // no table from the forward: make it
       launch_dscan_round_states(a->X, a->dt, a->Bproj, a->A, a->initial_states, a->init_dtype, a->seq_lens, ws, Bn, L, H,
-                                P, a->x_dtype, constant, a->bc_dtype, p.b_stride_b, a->a_per_p != 0, s);
-    if (a->x_dtype == SSM_BF16) launch_bwd_onepass<bf16_t, 2>(p, grads_io, constant, s);
-    else if (a->x_dtype == SSM_F16) launch_bwd_onepass<f16_t, 2>(p, grads_io, constant, s);
-    else launch_bwd_onepass<float, 1>(p, grads_io, constant, s);
+                                P, a->x_dtype, constant, a->bc_dtype, p.b_stride_b, a->a_per_p != 0, maps, nseg, s);
+    if (a->x_dtype == SSM_BF16) launch_bwd_onepass<bf16_t, 2>(p, grads_io, constant, maps, s);
+    else if (a->x_dtype == SSM_F16) launch_bwd_onepass<f16_t, 2>(p, grads_io, constant, maps, s);
+    else launch_bwd_onepass<float, 1>(p, grads_io, constant, maps, s);
     SSM_CHECK_LAUNCH("ssm_dscan_bwd");
-    if (!a->a_per_p && !a->d_per_p) {
-      hipLaunchKernelGGL(dscan_bwd_head_sums_kernel, dim3(H), dim3(WAVE), 0, s, p.pA, p.pD, a->dA, a->dD, Bn, H, P);
-    } else {
-      auto param_sum = [&](const float *partial, float *out, bool per_p) {
-        if (per_p) launch_fold_rows(partial, out, Bn, (size_t)HP, s);
-        else {
-          launch_fold_rows(partial, head_tmp, Bn, (size_t)HP, s);
-          launch_fold_sum(head_tmp, out, (size_t)H, P, 1, s);
-        }
-      };
-      param_sum(p.pA, a->dA, a->a_per_p != 0);
-      if (a->dD) param_sum(p.pD, a->dD, a->d_per_p != 0);
+    float *head_A = a->a_per_p ? nullptr : a->dA, *head_D = a->d_per_p ? nullptr : a->dD;
+    if (head_A || head_D)
+      hipLaunchKernelGGL(dscan_bwd_head_sums_kernel, dim3(H), dim3(WAVE), 0, s, p.pA, p.pD, head_A, head_D, copies, H, P);
+    FoldJobs jobs{};
+    if (a->a_per_p) jobs.add(p.pA, a->dA, 1, copies, (size_t)HP, SSM_F32);
+    if (a->dD && a->d_per_p) jobs.add(p.pD, a->dD, 1, copies, (size_t)HP, SSM_F32);
+    auto proj_sum = [&](int kind, bool direct, const float *partial, void *out) {
+      if (kind == SSM_CHUNK_HP) jobs.add(partial, out, 1, copies, (size_t)HP, SSM_F32);
+      else if (!direct) jobs.add(partial, out, 1, segs, bhp, SSM_F32);
+    };
+    if (constant) {
+      proj_sum(a->b_kind, b_direct, p.pB, a->dB);
+      proj_sum(a->c_kind, c_direct, p.pC, a->dC);
     }
-    if (constant && a->b_kind == SSM_CHUNK_HP) launch_fold_rows(p.pB, reinterpret_cast<float *>(a->dB), Bn, (size_t)HP, s);
-    if (constant && a->c_kind == SSM_CHUNK_HP) launch_fold_rows(p.pC, reinterpret_cast<float *>(a->dC), Bn, (size_t)HP, s);
+    launch_fold_jobs(jobs, s);
     SSM_CHECK_LAUNCH("ssm_dscan_bwd(sums)");
     return SSM_OK;
   } else {

@@ -15,6 +15,7 @@
 // round's left edge: it leaves the adjoint there in LDS for everyone's next round.  The state entering a round
 // comes from a table written beforehand: by the forward's one-pass kernel, or by that kernel's walk reduced to
 // X, B and dt (launch_dscan_round_states).  The reads of the next round are requested before the arithmetic of this one.
+// A call of few channels is cut into segments of time that run side by side (dscan_maps.hpp; blockIdx.z counts them).
 #pragma once
 
 namespace ssm {
@@ -71,6 +72,16 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
   float *DDT = p.ddt_direct + row0 * p.heads;
   const int rounds = (L + DBO_ROUND - 1) / DBO_ROUND;
   const float *table = p.round_states + (size_t)b * rounds * HP;
+  const int seg = blockIdx.z, r_first = seg * p.seg_rounds, r_last = min(rounds, r_first + p.seg_rounds) - 1;
+  if (wave == 0) {
+    // the adjoint entering the segment from the right, where a round leaves its own for the next
+    float mu0[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v)
+      mu0[v] = p.maps ? dscan_compose(p.maps + ((size_t)b * gridDim.z + gridDim.z - 1) * HP + ch + v, (int)gridDim.z - 1 - seg, -(ptrdiff_t)HP, 0.0f)
+                      : 0.0f;
+    left[(r_last & 1) ^ 1][lane] = make_float2(mu0[0], mu0[VEC - 1]);
+  }
 
   auto request = [&](DboRegs<io_t, VEC, HAS_Z> &r, int round) {
     const int t0 = round * DBO_ROUND + wave * DBO_SEG;
@@ -157,11 +168,9 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
     }
     // the adjoint entering them: the folds of the waves after it, from the adjoint that left the round before
     float mu[VEC];
-    if (r < rounds - 1) {
-      const float2 c = left[q ^ 1][lane];
-      mu_left[0] = c.x;
-      mu_left[VEC - 1] = c.y;
-    }
+    const float2 c = left[q ^ 1][lane];
+    mu_left[0] = c.x;
+    mu_left[VEC - 1] = c.y;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) mu[v] = mu_left[v];
     for (int w = DBO_WAVES - 1; w > wave; --w) {
@@ -243,12 +252,12 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
 
   // two sets of registers take turns: one is worked on while the other's reads are in flight
   DboRegs<io_t, VEC, HAS_Z> ra, rb;
-  request(ra, rounds - 1);
-  for (int r = rounds - 1; r >= 0; r -= 2) {
-    if (r > 0) request(rb, r - 1);
+  request(ra, r_last);
+  for (int r = r_last; r >= r_first; r -= 2) {
+    if (r > r_first) request(rb, r - 1);
     round_of(ra, r);
-    if (r > 0) {
-      if (r > 1) request(ra, r - 2);
+    if (r > r_first) {
+      if (r > r_first + 1) request(ra, r - 2);
       round_of(rb, r - 1);
     }
   }
@@ -272,36 +281,46 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
       float sum = 0.0f;
 #pragma unroll
       for (int w = 0; w < DBO_WAVES; ++w) sum += red[((SUMS * v + wave) * DBO_WAVES + w) * WAVE + lane];
-      out[wave][(size_t)b * HP + ch + v] = sum;
-      if (wave == 0 && p.dinit) p.dinit[(size_t)b * HP + ch + v] = mu_left[v];     // lambda_0 a_0
+      out[wave][((size_t)seg * gridDim.y + b) * HP + ch + v] = sum;
+      if (wave == 0 && p.dinit && seg == 0) p.dinit[(size_t)b * HP + ch + v] = mu_left[v];     // lambda_0 a_0
     }
   }
 }
 
-// dA and dD per head: the workgroups' per-channel sums added over batch rows and the head's channels, one wave
-// per head, in a fixed order.
+// dA and dD (each or one of them) per head: the workgroups' per-channel sums added over their rows -- batch rows, and
+// segments -- and the head's channels, one wave per head, in a fixed order.
 __global__ __launch_bounds__(WAVE) void dscan_bwd_head_sums_kernel(const float *pA, const float *pD, float *dA, float *dD,
-                                                                   int batch, int heads, int proj) {
+                                                                   int rows, int heads, int proj) {
   const int h = blockIdx.x, lane = lane_id();
   float sa = 0.0f, sd = 0.0f;
-  for (int b = 0; b < batch; ++b) {
-    for (int pp = lane; pp < proj; pp += WAVE) {
-      const size_t at = ((size_t)b * heads + h) * proj + pp;
-      sa += pA[at];
-      sd += pD[at];
+  for (int pp = lane; pp < proj; pp += WAVE) {
+    for (int r = 0; r < rows; r += 8) {                          // eight rows' reads in flight together
+      float va[8], vd[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const size_t at = ((size_t)min(r + k, rows - 1) * heads + h) * proj + pp;
+        va[k] = dA ? pA[at] : 0.0f;
+        vd[k] = dD ? pD[at] : 0.0f;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        sa += r + k < rows ? va[k] : 0.0f;
+        sd += r + k < rows ? vd[k] : 0.0f;
+      }
     }
   }
   sa = wave_sum(sa);
   sd = wave_sum(sd);
   if (lane == 0) {
-    dA[h] = sa;
+    if (dA) dA[h] = sa;
     if (dD) dD[h] = sd;
   }
 }
 
 template <typename io_t, typename g_t, int VEC, bool HAS_Z, bool PARAMS>
 static void launch_dbo_lph(const DscanBwdParams &p, int lph, hipStream_t s) {
-  const dim3 grid((unsigned)((size_t)p.heads * p.proj / (WAVE * VEC)), (unsigned)p.batch);
+  const int rounds = (p.len + DBO_ROUND - 1) / DBO_ROUND;
+  const dim3 grid((unsigned)((size_t)p.heads * p.proj / (WAVE * VEC)), (unsigned)p.batch, (unsigned)((rounds + p.seg_rounds - 1) / p.seg_rounds));
   const dim3 block(WAVE * DBO_WAVES);
   if (lph == 16) hipLaunchKernelGGL((dscan_bwd_onepass_kernel<io_t, g_t, VEC, HAS_Z, 16, PARAMS>), grid, block, 0, s, p);
   else if (lph == 32) hipLaunchKernelGGL((dscan_bwd_onepass_kernel<io_t, g_t, VEC, HAS_Z, 32, PARAMS>), grid, block, 0, s, p);
@@ -311,8 +330,18 @@ static void launch_dbo_lph(const DscanBwdParams &p, int lph, hipStream_t s) {
 // The one-pass backward for one element type.  params: B and C are per-channel constants (their gradients and dz
 // then are the only ones whose type grads_io chooses, and without a gate none is).
 template <typename io_t, int VEC>
-static void launch_bwd_onepass(const DscanBwdParams &p, bool grads_io, bool params, hipStream_t s) {
+static void launch_bwd_onepass(DscanBwdParams &p, bool grads_io, bool params, float2 *maps, hipStream_t s) {
   const int lph = p.proj / VEC;
+  const int nseg = ((p.len + DBO_ROUND - 1) / DBO_ROUND + p.seg_rounds - 1) / p.seg_rounds;
+  if (nseg > 1) {
+    DscanMapParams m{};
+    m.drive = p.gy; m.dt = p.dt; m.proj = p.Cp; m.z = p.z; m.A = p.A; m.lengths = p.lengths; m.maps = maps;
+    m.batch = p.batch; m.len = p.len; m.heads = p.heads; m.width = p.proj;
+    m.proj_dtype = p.bc_dtype; m.a_stride_p = p.a_stride_p; m.proj_stride_b = p.c_stride_b;
+    m.seg_len = p.seg_rounds * DBO_ROUND; m.nseg = nseg;
+    params ? launch_dscan_maps<io_t, VEC, true, true>(m, s) : launch_dscan_maps<io_t, VEC, true, false>(m, s);
+    p.maps = maps;
+  }
   if (params) {
     if (!p.z) launch_dbo_lph<io_t, io_t, VEC, false, true>(p, lph, s);
     else if (grads_io) launch_dbo_lph<io_t, io_t, VEC, true, true>(p, lph, s);

@@ -640,21 +640,9 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(const float *in, float *
   }
 }
 
-// All sums that a backward call ends with, in one launch of workgroup ranges per job:
-//   out[o][i] = sum_{j < count} in[(o * count + j) * inner + i], added in order of j, written as `dtype`.
-// dA, dD, the bias and projections constant in time sum over the batch (and over chunks that ran side by side); dB and
-// dC of grouped projections over the workgroups of a group, straight into the projections' own type when asked.  As
-// launches of their own, with the casts behind them, they took 5 to 10 us each, of which the gaps were half.
-constexpr int FOLD_JOBS = 5;
-struct FoldJobs {
-  const float *in[FOLD_JOBS];
-  void *out[FOLD_JOBS];
-  size_t outer[FOLD_JOBS], inner[FOLD_JOBS];
-  int count[FOLD_JOBS], dtype[FOLD_JOBS], width[FOLD_JOBS];     // width: outputs per thread, 1 or 4
-  unsigned first_block[FOLD_JOBS + 1];
-  int n;
-};
-
+// The sums of FoldJobs: dA, dD, the bias and projections constant in time over the batch (and over chunks that ran side
+// by side); dB and dC of grouped projections over the workgroups of a group, straight into the projections' own type
+// when asked.
 template <int W>
 __device__ __forceinline__ void fold_job(const float *in, void *out, size_t outer, size_t inner, int count, int dtype,
                                          size_t first, size_t stride) {
@@ -709,6 +697,17 @@ __global__ __launch_bounds__(256) void fold_jobs_kernel(const FoldJobs jobs) {
 static unsigned fold_grid(size_t n) {
   const size_t g = (n + 255) / 256;
   return (unsigned)(g < 1 ? 1 : (g > 65535 ? 65535 : g));
+}
+
+void FoldJobs::add(const float *src, void *dst, size_t outer_, int count_, size_t inner_, int dtype_) {
+  const int j = n++;
+  in[j] = src; out[j] = dst; outer[j] = outer_; count[j] = count_; inner[j] = inner_; dtype[j] = dtype_;
+  width[j] = inner_ % 4 == 0 && aligned_to(src, 16) && aligned_to(dst, 16) ? 4 : 1;
+  first_block[j + 1] = first_block[j] + fold_grid(outer_ * inner_ / width[j]);
+}
+
+void launch_fold_jobs(const FoldJobs &jobs, hipStream_t s) {
+  if (jobs.n) hipLaunchKernelGGL(fold_jobs_kernel, dim3(jobs.first_block[jobs.n]), dim3(256), 0, s, jobs);
 }
 
 void launch_fold_rows(const float *in, float *out, int count, size_t inner, hipStream_t s) {
@@ -1035,12 +1034,6 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   const int Bn = a->batch, D = a->dim, N = a->nstate, L = a->seqlen;
   // dA (D,N), dD (D,), dbias (D,): sums over the batch; dB / dC in the shape of the given projection
   FoldJobs jobs{};
-  auto add_job = [&](const float *in, void *out, size_t outer, int count, size_t inner, int dtype) {
-    const int j = jobs.n++;
-    jobs.in[j] = in; jobs.out[j] = out; jobs.outer[j] = outer; jobs.count[j] = count; jobs.inner[j] = inner; jobs.dtype[j] = dtype;
-    jobs.width[j] = inner % 4 == 0 && aligned_to(in, 16) && aligned_to(out, 16) ? 4 : 1;
-    jobs.first_block[j + 1] = jobs.first_block[j] + fold_grid(outer * inner / jobs.width[j]);
-  };
   // (dB and dC, the longest sums, first)
   auto fold_proj = [&](int kind, int groups, const float *partial, void *out) {
     if (kind == SSM_PROJ_BGNL) {
@@ -1049,21 +1042,21 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
       if (a->dbc_dtype == SSM_F32 && fold_sum_is_wide((size_t)Bn * groups, per_group, (size_t)N * L))
         launch_fold_sum(partial, reinterpret_cast<float *>(out), (size_t)Bn * groups, per_group, (size_t)N * L, s);
       else
-        add_job(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, a->dbc_dtype);
+        jobs.add(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, a->dbc_dtype);
     } else if (kind == SSM_PROJ_BDN) {
-      add_job(partial, out, 1, copies / Bn, (size_t)Bn * D * N, SSM_F32);
+      jobs.add(partial, out, 1, copies / Bn, (size_t)Bn * D * N, SSM_F32);
     } else {
-      add_job(partial, out, 1, copies, (size_t)D * N, SSM_F32);
+      jobs.add(partial, out, 1, copies, (size_t)D * N, SSM_F32);
     }
   };
   if (!per_row) {
     fold_proj(a->b_kind, p.b_groups, p.dB_part, a->dB);
     fold_proj(a->c_kind, p.c_groups, p.dC_part, a->dC);
   }
-  add_job(p.dA_rows, a->dA, 1, copies, (size_t)D * N, SSM_F32);
-  if (a->dD) add_job(p.dD_rows, a->dD, 1, copies, (size_t)D, SSM_F32);
-  if (a->ddt_bias) add_job(p.dbias_rows, a->ddt_bias, 1, copies, (size_t)D, SSM_F32);
-  hipLaunchKernelGGL(fold_jobs_kernel, dim3(jobs.first_block[jobs.n]), dim3(256), 0, s, jobs);
+  jobs.add(p.dA_rows, a->dA, 1, copies, (size_t)D * N, SSM_F32);
+  if (a->dD) jobs.add(p.dD_rows, a->dD, 1, copies, (size_t)D, SSM_F32);
+  if (a->ddt_bias) jobs.add(p.dbias_rows, a->ddt_bias, 1, copies, (size_t)D, SSM_F32);
+  launch_fold_jobs(jobs, s);
   SSM_CHECK_LAUNCH("ssm_scan_bwd(fold)");
   return SSM_OK;
 }

@@ -422,3 +422,29 @@ def test_one_pass_with_parameter_projections(dtype, hp, kinds, length, a_vec, z_
         assert auto[k].dtype == inp[k].dtype and auto[k].shape == inp[k].shape, k
         torch.testing.assert_close(auto[k].float(), g1.to(inp[k].dtype).float().reshape(inp[k].shape), rtol=1e-6, atol=0,
                                    msg=lambda m, n=k: f"grad {n} through autograd: {m}")
+
+
+# ------------------------------------------------------------------ few channels: segments of time side by side
+
+@pytest.mark.parametrize("dtype,kind", [(torch.float32, 4), (torch.float32, 2), (torch.bfloat16, 4), (torch.float16, 3)],
+                         ids=lambda v: str(v).replace("torch.", ""))
+@pytest.mark.parametrize("b,length,z_mode,init,lens", [(1, 129, 4, True, None), (2, 2048, 0, False, None),
+                                                       (3, 1025, 4, True, [1025, 640, 0]), (1, 4500, 4, False, [4353])])
+def test_time_in_segments(dtype, kind, b, length, z_mode, init, lens):
+    """64 or 128 channels: both directions cut time into segments of whole rounds (128 steps forward, 64 backward), the
+    last one short, with sequences that end inside a segment, at its edge or before it, up to the most segments there are."""
+    heads = 1 if dtype == torch.float32 else 2
+    inp = make(length + kind, b, length, heads, 64, dtype=dtype, bkind=kind, ckind=kind, a_vec=True, z_mode=z_mode, init=init)
+    inp["dt"] = inp["dt"].float() * 0.2                 # decays slow enough to reach over several segments
+    meta = {"seq_lens": lens} if lens else None
+    y, yr = both(inp, meta=meta)
+    torch.testing.assert_close(y.float(), yr.float(), **(FP32_TOL if dtype == torch.float32 else HALF_TOL))
+    gy = torch.randn(yr.shape, generator=torch.Generator().manual_seed(length)).to(dtype)
+    want = _grads_oracle({k: (v.float() if v is not None else None) for k, v in inp.items()}, meta, gy.float())
+    got = _grads_gpu(inp, meta, gy)
+    for k in GRAD_NAMES:
+        if want[k] is None:
+            continue
+        scale = float(want[k].abs().max()) + 1e-6
+        tol = dict(rtol=3e-2, atol=3e-2 * scale) if dtype != torch.float32 else dict(rtol=2e-4, atol=2e-5 * max(scale, 1.0))
+        torch.testing.assert_close(got[k].float().cpu().double(), want[k], msg=lambda m, n=k: f"grad {n}: {m}", **tol)
