@@ -474,11 +474,11 @@ int ssm_ssd_chunk_state_varlen(const ssm_ssd_chunk_state_varlen_args *args, void
 
 /* The whole forward (chunk_cumsum, bmm_chunk, chunk_state, state_passing,
  * chunk_scan; combined call recorded at scripts/refresh_mamba_goldens.py:591-604)
- * as one pass over the sequence that keeps the running state on chip: the
- * per-chunk states never reach device memory.  Covers bf16 and fp16 tensors with
- * headdim 64, chunk in {64, 128, 256}, nstate in {64, 128} and
- * seqlen % chunk == 0; ssm_ssd_combined_supported() tells, other shapes go
- * through the five calls above.  A head with A > 0 is treated as those calls
+ * in one call, for any sequence length: as one pass over the sequence that keeps
+ * the running state on chip, or chunk by chunk side by side where there are too
+ * few heads to fill the chip that way.  Covers bf16 and fp16 tensors with
+ * headdim 64, chunk in {64, 128, 256} and nstate in {64, 128};
+ * ssm_ssd_combined_supported() tells, other shapes go through the five calls above.  A head with A > 0 is treated as those calls
  * treat it (decays inside a chunk bounded by 1, the carried state growing). */
 typedef struct ssm_ssd_combined_args {
   const void *x;              /* (B,L,H,P) io dtype */
@@ -502,10 +502,32 @@ typedef struct ssm_ssd_combined_args {
   int64_t b_row_stride, c_row_stride;  /* elements from one step's (G, N) block of Bm / Cm to the next step's; 0: dense
                                  (G * N).  Lets B and C be the two halves of one projected row, read in place; rows
                                  stay 16-byte aligned (a multiple of 8 elements) */
+  int32_t keep_for_backward;  /* nonzero: workspace of ssm_ssd_combined_keep_bytes() bytes, which holds afterwards what
+                                 ssm_ssd_combined_bwd reads */
 } ssm_ssd_combined_args;
 int ssm_ssd_combined_supported(const ssm_ssd_dims *dims, int io_dtype);   /* 1 / 0 */
 size_t ssm_ssd_combined_workspace_bytes(const ssm_ssd_dims *dims);
 int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *args, void *hip_stream);
+size_t ssm_ssd_combined_keep_bytes(const ssm_ssd_dims *dims);
+
+/* Gradients of ssm_ssd_combined_fwd for bfloat16 calls without seq_idx and with at most a per-head Dskip
+ * (ssm_ssd_combined_bwd_supported: of the rest, ssm_ssd_combined_supported); sums over batch and time in float32, in
+ * one order.  The reference holds no code for them (see the fixture named at ssm_ssd_bwd_gate_args). */
+typedef struct ssm_ssd_combined_bwd_args {
+  ssm_ssd_combined_args fwd;  /* the forward's own, run with keep_for_backward, its workspace as the forward left it */
+  const void *dout;           /* (B,L,H,P) io dtype */
+  const float *dfinal;        /* (B,H,P,N) or NULL */
+  void *dx, *dz;              /* (B,L,H,P) io dtype; dz NULL exactly when z is */
+  void *dB, *dC;              /* (B,L,G,N) io dtype, dense */
+  void *ddt;                  /* (B,L,H) dt dtype */
+  float *dA, *dD, *ddt_bias;  /* (H,); dD and ddt_bias or NULL */
+  float *dinitial_states;     /* (B,H,P,N) or NULL */
+  void *workspace;            /* ssm_ssd_combined_bwd_workspace_bytes() bytes, 256-byte aligned */
+  size_t workspace_bytes;
+} ssm_ssd_combined_bwd_args;
+int ssm_ssd_combined_bwd_supported(const ssm_ssd_dims *dims, int io_dtype);   /* 1 / 0 */
+size_t ssm_ssd_combined_bwd_workspace_bytes(const ssm_ssd_dims *dims);
+int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *args, void *hip_stream);
 
 /* Element-wise stages of the gradient of the combined forward.  The reference holds no code for them: its
  * fixture `ssd_combined.combined_full.gradients` (tests/mamba_reference_cases.json, written by

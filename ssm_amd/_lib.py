@@ -181,7 +181,13 @@ class SsdCombinedArgs(C.Structure):
                 ("z", _vp), ("initial_states", _vp), ("y", _vp), ("final_states", _vp), ("workspace", _vp),
                 ("workspace_bytes", C.c_size_t), ("dims", SsdDims), ("io_dtype", _i32), ("dt_dtype", _i32),
                 ("dt_softplus", _i32), ("d_per_p", _i32), ("dt_min", C.c_float), ("dt_max", C.c_float),
-                ("seq_idx", _vp), ("b_row_stride", _i64), ("c_row_stride", _i64)]
+                ("seq_idx", _vp), ("b_row_stride", _i64), ("c_row_stride", _i64), ("keep_for_backward", _i32)]
+
+
+class SsdCombinedBwdArgs(C.Structure):
+    _fields_ = [("fwd", SsdCombinedArgs), ("dout", _vp), ("dfinal", _vp), ("dx", _vp), ("dz", _vp), ("dB", _vp), ("dC", _vp),
+                ("ddt", _vp), ("dA", _vp), ("dD", _vp), ("ddt_bias", _vp), ("dinitial_states", _vp), ("workspace", _vp),
+                ("workspace_bytes", C.c_size_t)]
 
 
 class SsdBwdGateArgs(C.Structure):
@@ -390,6 +396,10 @@ PLAIN_SYMBOLS = {
     "ssm_ssd_chunk_state_workspace_bytes": (C.c_size_t, [C.POINTER(SsdDims)]),
     "ssm_ssd_combined_supported": (C.c_int, [C.POINTER(SsdDims), C.c_int]),
     "ssm_ssd_combined_workspace_bytes": (C.c_size_t, [C.POINTER(SsdDims)]),
+    "ssm_ssd_combined_keep_bytes": (C.c_size_t, [C.POINTER(SsdDims)]),
+    "ssm_ssd_combined_bwd": (C.c_int, [C.POINTER(SsdCombinedBwdArgs), C.c_void_p]),
+    "ssm_ssd_combined_bwd_supported": (C.c_int, [C.POINTER(SsdDims), C.c_int]),
+    "ssm_ssd_combined_bwd_workspace_bytes": (C.c_size_t, [C.POINTER(SsdDims)]),
     "ssm_conv1d_bwd_workspace_bytes": (C.c_size_t, [C.c_int, C.c_int, C.c_int]),
     "ssm_norm_bwd_workspace_bytes": (C.c_size_t, [C.c_int, C.c_int]),
 }

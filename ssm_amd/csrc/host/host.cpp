@@ -43,7 +43,8 @@ struct Abi {
   X(ssm_conv1d_fwd) X(ssm_conv1d_bwd) X(ssm_conv1d_bwd_workspace_bytes) X(ssm_norm_fwd) X(ssm_norm_bwd)            \
   X(ssm_norm_bwd_workspace_bytes) X(ssm_dscan_fwd) X(ssm_dscan_bwd) X(ssm_dscan_fwd_workspace_bytes)               \
   X(ssm_dscan_bwd_workspace_bytes) X(ssm_dscan_fwd_one_pass) X(ssm_ssd_combined_fwd)                               \
-  X(ssm_ssd_combined_workspace_bytes) X(ssm_amd_last_error) X(ssm_amd_status_string)
+  X(ssm_ssd_combined_workspace_bytes) X(ssm_ssd_combined_keep_bytes) X(ssm_ssd_combined_bwd)                        \
+  X(ssm_ssd_combined_bwd_supported) X(ssm_ssd_combined_bwd_workspace_bytes) X(ssm_amd_last_error) X(ssm_amd_status_string)
   SSM_ENTRIES(SSM_ENTRY)
 #undef SSM_ENTRY
 };
@@ -741,7 +742,7 @@ PyObject *chunk_scan(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   END_HANDLE_TH_ERRORS
 }
 
-// ---------------------------------------------------------------- SSD, one-pass forward
+// ---------------------------------------------------------------- SSD
 
 // A (B, L, G, N) operand read where it lies: its (G, N) blocks dense, at one stride through batch and time.
 bool rows_in_place(const Tensor &t) {
@@ -751,6 +752,65 @@ bool rows_in_place(const Tensor &t) {
   return s[3] == 1 && (n[2] == 1 || s[2] == n[3]) && s[1] >= n[2] * n[3] && s[1] % 8 == 0 &&
          (n[0] == 1 || s[0] == n[1] * s[1]) && !(reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15);
 }
+
+// -> y, the final states when asked for, and the workspace.
+std::tuple<Tensor, Tensor, Tensor> ssd_fwd(ssm_ssd_combined_args &a, const Tensor &x, const Tensor &dt, const Tensor &A,
+                                           const Tensor &B, const Tensor &C, const Tensor &D, const Tensor &z,
+                                           const Tensor &bias, const Tensor &init, bool want_final, bool keep) {
+  Tensor y = empty_as(x), final;
+  if (want_final) final = empty({a.dims.batch, a.dims.heads, a.dims.headdim, a.dims.nstate}, x, at::kFloat);
+  a.keep_for_backward = keep;
+  if (keep) a.workspace_bytes = abi.ssm_ssd_combined_keep_bytes(&a.dims);
+  Tensor ws = empty_bytes(a.workspace_bytes, x);         // (torch's allocations start on 512-byte boundaries)
+  a.x = ptr(x); a.dt = ptr(dt); a.A = ptr<const float>(A); a.dt_bias = ptr<const float>(bias); a.Bm = ptr(B); a.Cm = ptr(C);
+  a.Dskip = ptr<const float>(D); a.z = ptr(z); a.initial_states = ptr<const float>(init); a.y = ptr<void>(y);
+  a.final_states = ptr<float>(final); a.workspace = ptr<void>(ws);
+  SSM_ENQUEUE(ssm_ssd_combined_fwd, a, x.device().index());
+  return {y, final, ws};
+}
+
+// The forward's workspace (steps, running sums, operand fragments, the states entering the chunks) is kept for the backward.
+struct SsdCombined : torch::autograd::Function<SsdCombined> {
+  static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &dt, const Tensor &A, const Tensor &B,
+                               const Tensor &C, const Maybe &D_, const Maybe &z_, const Maybe &bias_, const Maybe &init_,
+                               const ssm_ssd_combined_args *form, bool want_final, int64_t wanted) {
+    ssm_ssd_combined_args a = *form;
+    const Tensor D = get(D_), z = get(z_), bias = get(bias_), init = get(init_);
+    auto [y, final, ws] = ssd_fwd(a, x, dt, A, B, C, D, z, bias, init, want_final, true);
+    ctx->save_for_backward({x, dt, A, B, C, D, z, bias, init, ws});
+    ctx->saved_data["form"] = pack(a);
+    ctx->saved_data["wanted"] = wanted;
+    ctx->set_materialize_grads(false);
+    if (want_final) return {y, final};
+    return {y};
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &dt = s[1], &A = s[2], &B = s[3], &C = s[4], &D = s[5], &z = s[6], &bias = s[7], &init = s[8], &ws = s[9];
+    ssm_ssd_combined_bwd_args a{};
+    a.fwd = unpack<ssm_ssd_combined_args>(ctx->saved_data["form"]);
+    // (saved tensors may have been moved and brought back)
+    a.fwd.x = ptr(x); a.fwd.dt = ptr(dt); a.fwd.A = ptr<const float>(A); a.fwd.Dskip = ptr<const float>(D); a.fwd.z = ptr(z);
+    a.fwd.dt_bias = ptr<const float>(bias); a.fwd.initial_states = ptr<const float>(init); a.fwd.workspace = ptr<void>(ws);
+    const Tensor go = grads[0].defined() ? as_input(grads[0], x.scalar_type()) : at::zeros_like(x);
+    const Tensor gfinal = grads.size() > 1 ? as_f32(grads[1]) : Tensor();
+    Tensor dx = empty_as(x), ddt = empty_as(dt), dz = z.defined() ? empty_as(z) : Tensor();
+    Tensor dB = empty(B.sizes(), B, B.scalar_type()), dC = empty(C.sizes(), C, C.scalar_type());
+    Tensor dA = empty(A.sizes(), x, at::kFloat), dD = D.defined() ? empty(D.sizes(), x, at::kFloat) : Tensor();
+    Tensor dbias = bias.defined() ? empty(bias.sizes(), x, at::kFloat) : Tensor();
+    Tensor dinit = init.defined() ? empty(init.sizes(), x, at::kFloat) : Tensor();
+    const size_t bytes = abi.ssm_ssd_combined_bwd_workspace_bytes(&a.fwd.dims);
+    Tensor scratch = empty_bytes(bytes, x);
+    a.dout = ptr(go); a.dfinal = ptr<const float>(gfinal); a.dx = ptr<void>(dx); a.dz = ptr<void>(dz); a.dB = ptr<void>(dB);
+    a.dC = ptr<void>(dC); a.ddt = ptr<void>(ddt); a.dA = ptr<float>(dA); a.dD = ptr<float>(dD); a.ddt_bias = ptr<float>(dbias);
+    a.dinitial_states = ptr<float>(dinit); a.workspace = ptr<void>(scratch); a.workspace_bytes = bytes;
+    SSM_ENQUEUE(ssm_ssd_combined_bwd, a, x.device().index());
+    const Wanted pick(ctx);
+    return {pick(0, dx, x), pick(1, ddt, dt), pick(2, dA, A), pick(3, dB, B), pick(4, dC, C), pick(5, dD, D), pick(6, dz, z),
+            pick(7, dbias, bias), pick(8, dinit, init), Tensor(), Tensor(), Tensor()};
+  }
+};
 
 PyObject *ssd_combined(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   HANDLE_TH_ERRORS
@@ -763,7 +823,6 @@ PyObject *ssd_combined(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
   const double lo = r.real(), hi = r.real();
   const bool want_final = r.flag();
   if (!r.ok || !x.defined() || !dt.defined() || !A.defined() || !B.defined() || !C.defined()) Py_RETURN_NONE;
-  if (wants_grad({&x, &dt, &A, &B, &C, &D, &z, &bias, &init})) Py_RETURN_NONE;
   Key k;
   const auto xt = x.scalar_type();
   k.need((xt == at::kBFloat16 || xt == at::kHalf) && B.scalar_type() == xt && C.scalar_type() == xt && absent_or(z, xt) &&
@@ -776,15 +835,16 @@ PyObject *ssd_combined(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     k.put(C.stride(1));
   }
   k.put(Q); k.put(softplus); k.put(lo); k.put(hi); k.put(want_final);
+  const bool train = wants_grad({&x, &dt, &A, &B, &C, &D, &z, &bias, &init});
   ssm_ssd_combined_args a;
   if (!recall(forms, remember, k, &a)) Py_RETURN_NONE;
-  Tensor y = empty_as(x), final;
-  if (want_final) final = empty({a.dims.batch, a.dims.heads, a.dims.headdim, a.dims.nstate}, x, at::kFloat);
-  Tensor ws = empty_bytes(a.workspace_bytes, x);         // (torch's allocations start on 512-byte boundaries)
-  a.x = ptr(x); a.dt = ptr(dt); a.A = ptr<const float>(A); a.dt_bias = ptr<const float>(bias); a.Bm = ptr(B); a.Cm = ptr(C);
-  a.Dskip = ptr<const float>(D); a.z = ptr(z); a.initial_states = ptr<const float>(init); a.y = ptr<void>(y);
-  a.final_states = ptr<float>(final); a.workspace = ptr<void>(ws);
-  SSM_ENQUEUE(ssm_ssd_combined_fwd, a, k.device);
+  if (train) {
+    if (a.d_per_p || !abi.ssm_ssd_combined_bwd_supported(&a.dims, a.io_dtype)) Py_RETURN_NONE;
+    auto out = SsdCombined::apply(x, dt, A, B, C, maybe(D), maybe(z), maybe(bias), maybe(init), &a, want_final,
+                                  grad_bits({&x, &dt, &A, &B, &C, &D, &z, &bias, &init}));
+    return want_final ? wrap_pair(out[0], out[1]) : wrap(out[0]);
+  }
+  auto [y, final, ws] = ssd_fwd(a, x, dt, A, B, C, D, z, bias, init, want_final, false);
   return want_final ? wrap_pair(y, final) : wrap(y);
   END_HANDLE_TH_ERRORS
 }

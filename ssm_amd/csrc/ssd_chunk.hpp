@@ -1,0 +1,590 @@
+// The SSD of 16-bit calls with the chunks side by side, forward and backward: one workgroup per (batch, chunk, head).
+//
+//   states: what a chunk adds to the state,             S_c = sum_s exp(cs_Q - cs_s) dt_s x_s (x) B_s
+//   pass:   the state entering each chunk,              H_{c+1} = exp(cs_Q) H_c + S_c        (in place)
+//   scan:   y_l = exp(cs_l) C_l.H_c + sum_{s<=l} (C_l.B_s) exp(cs_l - cs_s) dt_s x_s
+//
+// and, for the gradients, the same three with the adjoint in the place of x: dS_c = sum_l exp(cs_l) dy_l (x) C_l, passed
+// from the last chunk to the first, and u_s = exp(cs_Q - cs_s) B_s.G_c + sum_{l>=s} (C_l.B_s) exp(cs_l - cs_s) dy_l
+// with dx_s = dt_s u_s + D dy_s.
+//
+// States travel in float32 and in fragment order: [p / 32][n / 16][lane][8], lane = p % 32 + 32 (n % 16 / 8), the order
+// in which a wave holds 32 x 16 of them as a matrix operand.  A wave's accumulators of S^T are written as whole KiB that
+// way, the pass is element by element in any order, and the scan reads operands without a transposition.
+//
+// The 64 channels of a chunk's rows are staged once, transposed, in LDS ([p][s], 16-byte pieces XOR-swizzled by p: no
+// bank conflicts on either side); the fragments of B, C and C.B come from L2, shared by the heads of a group, whose
+// workgroups are numbered onto one XCD.  What bounds these kernels is the traffic of x, z, y and the states: the matrix
+// products take about 1 us of a CU per workgroup, a decay factor per element of C.B another.
+//
+// A growing head (A > 0): decays between steps of a chunk are bounded by 1, the factors on carried states are not (as in
+// ssd_fused.hip); the gradients are those of that function.
+#pragma once
+#include "ssd_common.hpp"
+
+namespace ssm {
+
+// Workgroups go to the 8 XCDs round-robin: consecutive results of this go to one XCD.
+__device__ __forceinline__ unsigned xcd_order(unsigned id, unsigned n) {
+  const unsigned q = n >> 3, r = n & 7, x = id & 7;
+  return x * q + min(x, r) + (id >> 3);
+}
+
+template <typename E, int C> struct Row { static_assert(sizeof(E) == 2); E v[C]; } __attribute__((aligned(2 * C)));
+
+// (batch, chunk, head) of a workgroup and what follows from it.
+struct ChunkUnit {
+  int b, c, h, g, rows;          // rows: steps of this chunk
+  size_t row0, step0, unit, state;
+  __device__ __forceinline__ ChunkUnit(int len, int heads, int groups, int nchunks, int Q, int N) {
+    const unsigned vid = xcd_order(blockIdx.x, gridDim.x);
+    h = (int)(vid % heads);
+    const unsigned bc = vid / heads;
+    c = (int)(bc % nchunks);
+    b = (int)(bc / nchunks);
+    g = h / (heads / groups);
+    rows = min(Q, len - c * Q);
+    row0 = (size_t)b * len + (size_t)c * Q;                       // of (B, L, ...)
+    step0 = (((size_t)b * heads + h) * nchunks + c) * Q;          // of (B, H, nc, Q)
+    unit = (size_t)bc * groups + g;                               // of the fragments
+    state = (size_t)vid * (SSD_P * N);                            // of (B, nc, H, 64 N)
+  }
+};
+
+// Eight rows x Q / 32 channels per thread of the 256: channel group tid % TPR, rows 8 (tid / TPR) ...
+template <int Q> struct Staging {
+  static constexpr int CPT = Q / 32, TPR = 64 / CPT, QMASK = Q >= 128 ? 15 : Q / 8 - 1;
+};
+
+template <typename E, int Q>
+__device__ __forceinline__ void stage_transposed(E *xT, int tid, const V8<E> (&col)[Q / 32]) {
+  using S = Staging<Q>;
+  const int cg = tid % S::TPR, rg = tid / S::TPR;
+#pragma unroll
+  for (int i = 0; i < S::CPT; ++i) {
+    const int p = cg * S::CPT + i;
+    *reinterpret_cast<V8<E> *>(xT + p * Q + ((rg ^ (p & S::QMASK)) << 3)) = col[i];
+  }
+}
+// Operand fragment of channels 32 pt .. and steps 16 ks ..
+template <typename E, int Q>
+__device__ __forceinline__ V8<E> staged_frag(const E *xT, int pt, int ks, int m, int g2) {
+  return load_frag_e<E>(xT + (32 * pt + m) * Q + (((2 * ks + g2) ^ (m & Staging<Q>::QMASK)) << 3));
+}
+
+__device__ __forceinline__ void load8(const float *p, float (&v)[8]) {
+  const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+// ---------------------------------------------------------------------- states
+
+struct SsdStatesParams {
+  const void *x;                 // forward: x;  backward: dout
+  const void *z;                 // backward: the gate, or null
+  void *dy;                      // backward: dout silu(z) in the element type
+  const void *frag;              // forward: Btblk;  backward: Ctblk
+  const float *dA2, *dtv;
+  float *states;
+  int len, heads, groups, nchunks;
+};
+
+// 8 x2 float32 tiles per workgroup, 16 steps of two products per wave; 33 KB of LDS.
+template <typename E, int Q, int N, bool BWD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_states_kernel(const SsdStatesParams p) {
+  __shared__ __align__(16) E xT[SSD_P * Q];
+  using S = Staging<Q>;
+  constexpr int KS = Q >> 4, KN = N >> 4, NT = N >> 5, PW = NT >= 4 ? 2 : 1, AHEAD = BWD || KS < 8 ? 4 : 8;
+  const ChunkUnit u(p.len, p.heads, p.groups, p.nchunks, Q, N);
+  const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
+  const int m = lane & 31, g2 = lane >> 5;
+  const int nt = PW == 2 ? wave : wave & 1, pt0 = PW == 2 ? 0 : wave >> 1;
+  const int cg = tid % S::TPR, rg = tid / S::TPR;
+  const unsigned pitch = (unsigned)p.heads * SSD_P * 2;                // bytes between rows
+  const size_t at = (u.row0 * p.heads + u.h) * SSD_P;
+  unsigned off[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) off[r] = (unsigned)min(8 * rg + r, u.rows - 1) * pitch + cg * S::CPT * 2;
+  typedef Row<E, S::CPT> row_t;
+  row_t raw[8], gate[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) raw[r] = *at_bytes<const row_t>(reinterpret_cast<const E *>(p.x) + at, off[r]);
+  if (BWD && p.z) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) gate[r] = *at_bytes<const row_t>(reinterpret_cast<const E *>(p.z) + at, off[r]);
+  }
+  float w[8];
+  load8(p.dA2 + u.step0 + 8 * rg, w);
+  if (BWD) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) w[r] = 8 * rg + r < u.rows ? exp2_hw(w[r]) : 0.0f;
+  } else {
+    float dt[8];
+    load8(p.dtv + u.step0 + 8 * rg, dt);
+    const float end = p.dA2[u.step0 + Q - 1];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) w[r] = dt[r] * exp2_hw(fminf(end - w[r], 0.0f));
+  }
+  if (BWD && p.z) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+#pragma unroll
+      for (int i = 0; i < S::CPT; ++i) raw[r].v[i] = (E)((float)raw[r].v[i] * silu_f32((float)gate[r].v[i]));
+    }
+  }
+  if (BWD && p.dy) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (8 * rg + r < u.rows) *at_bytes<row_t>(reinterpret_cast<E *>(p.dy) + at, off[r]) = raw[r];
+  }
+  const E *frag = reinterpret_cast<const E *>(p.frag) + (u.unit * KS * NT + nt) * SSD_FRAG + lane * 8;
+  V8<E> f[AHEAD];
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) f[k] = load_frag_e<E>(frag + k * NT * SSD_FRAG);
+  V8<E> col[S::CPT];
+#pragma unroll
+  for (int i = 0; i < S::CPT; ++i) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) col[i][r] = (E)((float)raw[r].v[i] * w[r]);
+  }
+  stage_transposed<E, Q>(xT, tid, col);
+  __syncthreads();
+  f32x16_t acc[PW];
+#pragma unroll
+  for (int pt = 0; pt < PW; ++pt) acc[pt] = (f32x16_t){0};
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+    for (int pt = 0; pt < PW; ++pt) acc[pt] = mma(f[ks % AHEAD], staged_frag<E, Q>(xT, pt0 + pt, ks, m, g2), acc[pt]);
+    if (ks + AHEAD < KS) f[ks % AHEAD] = load_frag_e<E>(frag + (ks + AHEAD) * NT * SSD_FRAG);
+  }
+  float *out = p.states + u.state;
+#pragma unroll
+  for (int pt = 0; pt < PW; ++pt) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<float4 *>(out + ((pt0 + pt) * KN + 2 * nt + (q >> 1)) * SSD_FRAG + (m + 32 * (q & 1)) * 8 + 4 * g2) =
+          make_float4(acc[pt][4 * q], acc[pt][4 * q + 1], acc[pt][4 * q + 2], acc[pt][4 * q + 3]);
+  }
+}
+
+// ---------------------------------------------------------------------- pass
+
+struct SsdCarryParams {
+  float *states;                 // (B, nc, H, dim) in fragment order, rewritten
+  void *states16;                // where the entering states go instead, in the element type, or null
+  const float *dA2;              // (B, H, nc, Q)
+  const float *first;            // (B, H, P, N): the state before the first chunk (after the last one), or null
+  float *last;                   // (B, H, P, N) or null
+  const float *entering;         // backward: the forward's states, for <G, H> at the chunk boundaries
+  float *anchor;                 // backward: (B, H, nc, dim / 256) partial sums of it
+  int heads, nchunks, chunk, nstate;
+};
+
+// Four elements per thread over all chunks, eight chunks' reads in flight; 64 N / 1024 workgroups per (batch, head).
+template <typename E, bool REV>
+__global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) {
+  const int N = p.nstate, dim = SSD_P * N, per = dim >> 10;
+  const unsigned vid = blockIdx.x;
+  const int part = (int)(vid % per);
+  const size_t bh = vid / per;
+  const int h = (int)(bh % p.heads);
+  const size_t b = bh / p.heads;
+  const int e = (part * 256 + (int)threadIdx.x) * 4;
+  const int frag = e >> 9, fl = (e >> 3) & 63, kn = N >> 4;
+  const size_t user = (bh * SSD_P + 32 * (frag / kn) + (fl & 31)) * N + 16 * (frag % kn) + 8 * (fl >> 5) + (e & 7);
+  const size_t pitch = (size_t)p.heads * dim;
+  const size_t at = (b * p.nchunks * p.heads + h) * dim + e;
+  float *st = p.states + at;
+  const float *ent = p.entering + at;
+  const float *end = p.dA2 + bh * p.nchunks * p.chunk + p.chunk - 1;
+  float4 run = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (p.first) run = make_float4(p.first[user], p.first[user + 1], p.first[user + 2], p.first[user + 3]);
+  constexpr int AHEAD = REV ? 4 : 8;
+  for (int i0 = 0; i0 < p.nchunks; i0 += AHEAD) {
+    float4 v[AHEAD], hin[AHEAD];
+    float a[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      const int i = min(i0 + k, p.nchunks - 1), c = REV ? p.nchunks - 1 - i : i;
+      v[k] = *reinterpret_cast<const float4 *>(st + c * pitch);
+      if (REV) hin[k] = *reinterpret_cast<const float4 *>(ent + c * pitch);
+      a[k] = end[(size_t)c * p.chunk];
+    }
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      const int i = i0 + k, c = REV ? p.nchunks - 1 - i : i;
+      if (i < p.nchunks) {
+        if (!REV && p.states16) {
+          const float r4[4] = {run.x, run.y, run.z, run.w};
+          store4_e<E>(reinterpret_cast<E *>(p.states16) + at + c * pitch, r4);
+        } else {
+          *reinterpret_cast<float4 *>(st + c * pitch) = run;
+        }
+        const float f = exp2_hw(a[k]);
+        run.x = __builtin_fmaf(run.x, f, v[k].x);
+        run.y = __builtin_fmaf(run.y, f, v[k].y);
+        run.z = __builtin_fmaf(run.z, f, v[k].z);
+        run.w = __builtin_fmaf(run.w, f, v[k].w);
+        if (REV) {                    // run is now the adjoint of the state that entered chunk c
+          const float s = wave_sum(run.x * hin[k].x + run.y * hin[k].y + run.z * hin[k].z + run.w * hin[k].w);
+          if (lane_id() == 0) p.anchor[(bh * p.nchunks + c) * (dim >> 8) + part * 4 + (threadIdx.x >> 6)] = s;
+        }
+      }
+    }
+  }
+  if (p.last) *reinterpret_cast<float4 *>(p.last + user) = run;
+}
+
+// ---------------------------------------------------------------------- scan
+
+enum { SCAN_Y, SCAN_DZ, SCAN_DX };
+
+struct SsdChunkScanParams {
+  const void *op;                // rows of the in-chunk product: x, or dy for SCAN_DX
+  const void *blk;               // fragments of C.B (transposed for SCAN_DX)
+  const void *carry;             // fragments of C (of B for SCAN_DX)
+  const void *states;            // H entering the chunks (G leaving them for SCAN_DX), fragment order
+  const float *dA2, *dtv, *Dk;
+  const void *x, *dy, *z, *dout; // (B, L, H, 64) rows the last step reads
+  void *out;                     // y, dz (or null) or dx
+  float *sum0, *sum1;            // (B, H, nc, Q): SCAN_DZ <dy, y before skip>;  SCAN_DX <x, u> and <round(dt x), u>
+  float *dD;                     // SCAN_DZ: (B, nc, H) sums of dy x, or null
+  int len, heads, groups, nchunks, d_per_p;
+  int has_first;                 // a state enters the first chunk (leaves the last)
+  int states16;                  // states are of the element type (else float32)
+};
+
+// Row blocks of 32 steps: a wave takes blocks NLB - 1 - i and i (NLB + 1 of the blocks on and below the diagonal
+// whatever i is), both halves of the channels where there are four such pairs, else one half.  The decays multiply the
+// elements of C.B in registers, in front of their product: on the diagonal one exp2 per element, below it
+//   exp(cs_l - cs_s) = exp(cs_l - cs[end of the block before l's]) exp(.. - cs[end of s's block]) exp(.. - cs_s),
+// a factor of each side from a table and a scalar per block (every factor at most 1).  With an exp2 per element
+// everywhere the vector ALU was the bound .  The accumulators (lane = step, registers = channels)
+// go through LDS to whole rows for the last step: skip and gate, or dz and the row sums, or dx and its sums.
+// SCAN_Y takes the step into that factor, so that x itself is the operand and each product is rounded once.
+// SCAN_DZ and SCAN_DX take it into the staged x, and form the same rounded numbers C.B x decay: what the difference of their row sums needs (see
+// ssd_bwd_dt_kernel) is that both multiply the same block.
+template <typename E, int Q, int N, int MODE, bool HAS_Z>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_chunk_scan_kernel(const SsdChunkScanParams p) {
+  using S = Staging<Q>;
+  constexpr int NLB = Q >> 5, KS = Q >> 4, KN = N >> 4, NPAIR = NLB / 2, PW = NPAIR >= 4 ? 2 : 1;
+  __shared__ __align__(16) E xT[SSD_P * Q];
+  __shared__ __align__(16) E hs[SSD_P * N];
+  __shared__ __align__(16) float dAs[Q];
+  __shared__ __align__(16) float Ps[Q], Rs[Q];                           // decay from the block before to a step, from a step to the end of its block
+  __shared__ __align__(16) float l2s[MODE == SCAN_Y ? Q : 4];            // log2 dt
+  __shared__ float halves[PW == 1 && MODE != SCAN_Y ? 4 * Q : 4];       // row sums of half rows; or one sum per wave
+  const ChunkUnit u(p.len, p.heads, p.groups, p.nchunks, Q, N);
+  const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
+  const int m = lane & 31, g2 = lane >> 5;
+  const int pair = PW == 2 ? wave : wave >> 1, pt0 = PW == 2 ? 0 : wave & 1;
+  const bool active = pair < NPAIR;
+  const int rbs[2] = {NLB - 1 - pair, pair};
+  const bool carried = MODE == SCAN_DX ? (u.c < p.nchunks - 1 || p.has_first) : (u.c > 0 || p.has_first);
+  const int cg = tid % S::TPR, rg = tid / S::TPR;
+  const unsigned pitch = (unsigned)p.heads * SSD_P * 2;                // bytes between rows
+  const size_t at = (u.row0 * p.heads + u.h) * SSD_P;
+
+  // ---- stage the rows and the carried state
+  typedef Row<E, S::CPT> row_t;
+  row_t raw[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+    raw[r] = *at_bytes<const row_t>(reinterpret_cast<const E *>(p.op) + at, (unsigned)min(8 * rg + r, u.rows - 1) * pitch + cg * S::CPT * 2);
+  float w[8];
+  if (MODE == SCAN_DZ) load8(p.dtv + u.step0 + 8 * rg, w);      // zero past the end
+  // The blocks of this wave in the order of use: those below the diagonal of the first row block (nA of them), of the
+  // second, then the two on the diagonal, second row block first: NLB + 1 steps whatever the wave, unrolled, so that
+  // fragments can be requested AHEAD steps before their use without a register ever being copied.
+  constexpr int AHEAD = MODE == SCAN_Y ? 4 : 2;
+  const int nA = MODE == SCAN_DX ? NLB - 1 - rbs[0] : rbs[0];
+  const E *bf = reinterpret_cast<const E *>(p.blk) + u.unit * NLB * KS * SSD_FRAG + lane * 8;
+  V8<E> ring[AHEAD][2];
+  const auto row_of = [&](int t) { return t < nA || t == NLB ? rbs[0] : rbs[1]; };
+  const auto other_of = [&](int t) {
+    return t >= NLB - 1 ? row_of(t) : (MODE == SCAN_DX ? row_of(t) + 1 : 0) + (t < nA ? t : t - nA);
+  };
+  const auto request = [&](int t) {
+    const E *f = bf + (row_of(t) * KS + 2 * other_of(t)) * SSD_FRAG;
+    ring[t % AHEAD][0] = load_frag_e<E>(f);
+    ring[t % AHEAD][1] = load_frag_e<E>(f + SSD_FRAG);
+  };
+  V8<E> fc[2][KN];
+  if (active && carried) {
+    const E *cf = reinterpret_cast<const E *>(p.carry) + u.unit * NLB * KN * SSD_FRAG + lane * 8;
+#pragma unroll
+    for (int k = 0; k < KN; ++k) {
+      fc[0][k] = load_frag_e<E>(cf + (rbs[0] * KN + k) * SSD_FRAG);
+      fc[1][k] = load_frag_e<E>(cf + (rbs[1] * KN + k) * SSD_FRAG);
+    }
+  }
+  if (tid < Q) {
+    const float cs = p.dA2[u.step0 + tid];
+    dAs[tid] = cs;
+    const float before = tid < 32 ? 0.0f : p.dA2[u.step0 + (tid & ~31) - 1];
+    Ps[tid] = exp2_hw(fminf(cs - before, 0.0f));
+    float r = exp2_hw(fminf(__shfl(cs, lane | 31, WAVE) - cs, 0.0f));
+    if (MODE == SCAN_Y) {
+      const float dt = p.dtv[u.step0 + tid];
+      r *= dt;
+      l2s[tid] = log2_hw(dt);                                   // dt = 0: -inf, a weight of zero
+    }
+    Rs[tid] = r;
+  }
+  if (carried) {
+    if (MODE == SCAN_Y && p.states16) {
+      const E *st = reinterpret_cast<const E *>(p.states) + u.state;
+#pragma unroll
+      for (int i = 0; i < SSD_P * N / 2048; ++i)
+        *reinterpret_cast<V8<E> *>(hs + (i * 256 + tid) * 8) = load_frag_e<E>(st + (i * 256 + tid) * 8);
+    } else {
+      const float *st = reinterpret_cast<const float *>(p.states) + u.state;
+#pragma unroll
+      for (int i = 0; i < SSD_P * N / 2048; ++i) {
+        float v[8];
+        load8(st + (i * 256 + tid) * 8, v);
+        *reinterpret_cast<V8<E> *>(hs + (i * 256 + tid) * 8) = pack8_e<E>(v);
+      }
+    }
+  }
+  V8<E> col[S::CPT];
+#pragma unroll
+  for (int i = 0; i < S::CPT; ++i) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      col[i][r] = MODE == SCAN_DZ ? (E)((float)raw[r].v[i] * w[r])
+                                  : MODE == SCAN_Y || 8 * rg + r < u.rows ? raw[r].v[i] : (E)0.0f;
+  }
+  stage_transposed<E, Q>(xT, tid, col);
+  __syncthreads();
+
+  const float head_D = p.Dk && !p.d_per_p ? p.Dk[u.h] : 0.0f;
+  f32x16_t acc[2][PW];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int pt = 0; pt < PW; ++pt) acc[i][pt] = (f32x16_t){0};
+  }
+  if (active) {
+#pragma unroll
+    for (int t = 0; t < AHEAD && t <= NLB; ++t) request(t);
+    // ---- the carried state
+    if (carried) {
+#pragma unroll
+      for (int k = 0; k < KN; ++k) {
+#pragma unroll
+        for (int pt = 0; pt < PW; ++pt) {
+          const V8<E> h = load_frag_e<E>(hs + ((pt0 + pt) * KN + k) * SSD_FRAG + lane * 8);
+          acc[0][pt] = mma(h, fc[0][k], acc[0][pt]);
+          acc[1][pt] = mma(h, fc[1][k], acc[1][pt]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float own = dAs[32 * rbs[i] + m];
+        const float f = exp2_hw(MODE == SCAN_DX ? fminf(dAs[Q - 1] - own, 0.0f) : own);
+#pragma unroll
+        for (int pt = 0; pt < PW; ++pt) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][pt][r] *= f;
+        }
+      }
+    }
+    // ---- the chunk's own steps
+    const auto step = [&](int t, f32x16_t (&to)[PW], auto diagonal) {
+      const int rb = row_of(t), ob = other_of(t);
+      const int lb = MODE == SCAN_DX ? ob : rb, sb = MODE == SCAN_DX ? rb : ob;
+      const float own = dAs[32 * rb + m];
+      float lane_f = 0.0f;
+      if (!diagonal.value)
+        lane_f = (MODE == SCAN_DX ? Rs : Ps)[32 * rb + m] * exp2_hw(fminf(dAs[32 * lb - 1] - dAs[32 * sb + 31], 0.0f));
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        float d[8], v[8];
+        const V8<E> f = ring[t % AHEAD][kk];
+        const int o = 32 * ob + 16 * kk + 8 * g2;
+        if constexpr (diagonal.value) {
+          load8(dAs + o, d);
+          if constexpr (MODE == SCAN_Y) {
+            // dt_s exp(min(cs_l - cs_s, 0)) as one exponential: min(a, 0) + b = min(a + b, b)
+            float l2[8];
+            load8(l2s + o, l2);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              // a skip factor per head joins the diagonal: CB dt + D at s = l, rounded as one number
+              const float skip = 16 * kk + 8 * g2 + j == m ? head_D : 0.0f;
+              v[j] = __builtin_fmaf((float)f[j], exp2_hw(fminf(own + (l2[j] - d[j]), l2[j])), skip);
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (float)f[j] * exp2_hw(fminf(MODE == SCAN_DX ? d[j] - own : own - d[j], 0.0f));
+          }
+        } else {
+          load8((MODE == SCAN_DX ? Ps : Rs) + o, d);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = (float)f[j] * d[j] * lane_f;
+        }
+        const V8<E> wv = pack8_e<E>(v);
+#pragma unroll
+        for (int pt = 0; pt < PW; ++pt) to[pt] = mma(staged_frag<E, Q>(xT, pt0 + pt, 2 * ob + kk, m, g2), wv, to[pt]);
+      }
+      if (t + AHEAD <= NLB) request(t + AHEAD);
+    };
+    const auto swap = [&]() {
+#pragma unroll
+      for (int pt = 0; pt < PW; ++pt) {
+        const f32x16_t v = acc[0][pt];
+        acc[0][pt] = acc[1][pt];
+        acc[1][pt] = v;
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < NLB - 1; ++t) {
+      if (t == nA) swap();
+      step(t, acc[0], std::false_type{});
+    }
+    if (nA == NLB - 1) swap();             // acc[0] now belongs to the second row block
+    step(NLB - 1, acc[0], std::true_type{});
+    step(NLB, acc[1], std::true_type{});
+  }
+  __syncthreads();                       // the staged rows are through: their place turns accumulators into rows
+
+  // ---- whole rows: a lane holds 8 channels of a row.  What a row block reads from memory is requested in front of the
+  // work on the block before it.
+  constexpr int LPR = 4 * PW, RPP = 64 / LPR, PASSES = 32 / RPP, SMASK = 8 * PW - 1;      // lanes per row, rows per pass
+  constexpr bool Z = HAS_Z && MODE != SCAN_DX;
+  float *stg = reinterpret_cast<float *>(xT) + wave * (32 * 32 * PW);
+  const int c8 = lane % LPR, ch = 32 * pt0 + 8 * c8;
+  const bool skip_rows = MODE == SCAN_Y && p.Dk && p.d_per_p;
+  float D8[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) D8[j] = MODE != SCAN_Y ? head_D : skip_rows ? p.Dk[u.h * SSD_P + ch + j] : 0.0f;
+  constexpr int AT_ONCE = MODE == SCAN_Y ? PASSES : PASSES / 2, GROUPS = PASSES / AT_ONCE;      // what the registers hold
+  V8<E> rx[AT_ONCE], rdy[AT_ONCE], rz[AT_ONCE], rgo[AT_ONCE];
+  float rdt[AT_ONCE];
+  const auto request_rows = [&](int rb, int first) {
+#pragma unroll
+    for (int pass = 0; pass < AT_ONCE; ++pass) {
+      const int l = 32 * rb + (first + pass) * RPP + lane / LPR;
+      const unsigned ra = (unsigned)min(l, u.rows - 1) * pitch + ch * 2;
+      if (MODE != SCAN_Y || skip_rows) rx[pass] = *at_bytes<const V8<E>>(reinterpret_cast<const E *>(p.x) + at, ra);
+      if (MODE != SCAN_Y) rdy[pass] = *at_bytes<const V8<E>>(reinterpret_cast<const E *>(p.dy) + at, ra);
+      if (Z) rz[pass] = *at_bytes<const V8<E>>(reinterpret_cast<const E *>(p.z) + at, ra);
+      if (Z && MODE == SCAN_DZ) rgo[pass] = *at_bytes<const V8<E>>(reinterpret_cast<const E *>(p.dout) + at, ra);
+      if (MODE == SCAN_DX) rdt[pass] = p.dtv[u.step0 + l];
+    }
+  };
+  float dyx = 0.0f;
+  if (active) {
+    request_rows(rbs[1], 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int pt = 0; pt < PW; ++pt) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4 *>(stg + m * 32 * PW + (((8 * pt + 2 * q + g2) ^ (m & SMASK)) << 2)) =
+              make_float4(acc[i][pt][4 * q], acc[i][pt][4 * q + 1], acc[i][pt][4 * q + 2], acc[i][pt][4 * q + 3]);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int grp = 0; grp < GROUPS; ++grp) {
+        V8<E> res[AT_ONCE];
+        float s0[AT_ONCE], s1[AT_ONCE];
+#pragma unroll
+        for (int pass = 0; pass < AT_ONCE; ++pass) {
+          const int lr = (grp * AT_ONCE + pass) * RPP + lane / LPR;
+          const bool live = 32 * rbs[1 - i] + lr < u.rows;
+          const float4 a0 = *reinterpret_cast<const float4 *>(stg + lr * 32 * PW + (((2 * c8) ^ (lr & SMASK)) << 2));
+          const float4 a1 = *reinterpret_cast<const float4 *>(stg + lr * 32 * PW + (((2 * c8 + 1) ^ (lr & SMASK)) << 2));
+          float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+          const V8<E> x = rx[pass], dy = rdy[pass], z = rz[pass], go = rgo[pass];
+          s0[pass] = 0.0f;
+          s1[pass] = 0.0f;
+          if (MODE == SCAN_Y) {
+            if (skip_rows) {
+#pragma unroll
+              for (int j = 0; j < 8; ++j) v[j] = __builtin_fmaf(D8[j], (float)x[j], v[j]);
+            }
+            if (Z) {
+#pragma unroll
+              for (int j = 0; j < 8; ++j) v[j] *= silu_f32((float)z[j]);
+            }
+          } else if (MODE == SCAN_DZ) {
+            float dyx_row = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float xf = (float)x[j];
+              s0[pass] = __builtin_fmaf((float)dy[j], v[j], s0[pass]);
+              if (Z) {
+                const float zf = (float)z[j], sg = sigmoid_f32(zf), gf = (float)go[j];
+                dyx_row = __builtin_fmaf(gf * zf * sg, xf, dyx_row);            // dy before its rounding
+                v[j] = gf * __builtin_fmaf(D8[j], xf, v[j]) * (sg * __builtin_fmaf(zf, 1.0f - sg, 1.0f));
+              } else {
+                dyx_row = __builtin_fmaf((float)dy[j], xf, dyx_row);
+              }
+            }
+            dyx += live ? dyx_row : 0.0f;
+            asm volatile("" : "+v"(dyx));        // formed here: left to the compiler, all its terms wait for the end of the kernel
+          } else {
+            const float dt = rdt[pass];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float xf = (float)x[j];
+              s0[pass] = __builtin_fmaf(xf, v[j], s0[pass]);
+              s1[pass] = __builtin_fmaf((float)(E)(xf * dt), v[j], s1[pass]);
+              v[j] = __builtin_fmaf(dt, v[j], D8[j] * (float)dy[j]);
+            }
+          }
+          res[pass] = pack8_e<E>(v);
+          s0[pass] = live ? s0[pass] : 0.0f;
+          s1[pass] = live ? s1[pass] : 0.0f;
+        }
+        if (grp + 1 < GROUPS) request_rows(rbs[1 - i], (grp + 1) * AT_ONCE);
+        else if (i == 0) request_rows(rbs[0], 0);
+#pragma unroll
+        for (int pass = 0; pass < AT_ONCE; ++pass) {
+          const int l = 32 * rbs[1 - i] + (grp * AT_ONCE + pass) * RPP + lane / LPR;
+          if ((MODE != SCAN_DZ || Z) && l < u.rows)
+            *at_bytes<V8<E>>(reinterpret_cast<E *>(p.out) + at, (unsigned)l * pitch + ch * 2) = res[pass];
+          if (MODE == SCAN_Y) continue;
+          if (PW == 2) {
+            const float t0 = lane_run_sum_last<8>(s0[pass]), t1 = MODE == SCAN_DX ? lane_run_sum_last<8>(s1[pass]) : 0.0f;
+            if (c8 == 7) {
+              p.sum0[u.step0 + l] = t0;
+              if (MODE == SCAN_DX) p.sum1[u.step0 + l] = t1;
+            }
+          } else {
+            float t0 = s0[pass], t1 = s1[pass];
+            t0 += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, t0);
+            t0 += dpp_move<DPP_ROW_SHR2, 0xf>(0.0f, t0);
+            t1 += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, t1);
+            t1 += dpp_move<DPP_ROW_SHR2, 0xf>(0.0f, t1);
+            if (c8 == 3) {
+              halves[pt0 * Q + l] = t0;
+              if (MODE == SCAN_DX) halves[(2 + pt0) * Q + l] = t1;
+            }
+          }
+        }
+      }
+    }
+  }
+  if (MODE == SCAN_Y) return;
+  if (PW == 1) {
+    __syncthreads();
+    if (tid < Q) {
+      p.sum0[u.step0 + tid] = halves[tid] + halves[Q + tid];
+      if (MODE == SCAN_DX) p.sum1[u.step0 + tid] = halves[2 * Q + tid] + halves[3 * Q + tid];
+    }
+  }
+  if (MODE == SCAN_DZ && p.dD) {
+    const float t = wave_sum(dyx);
+    __syncthreads();
+    if (lane == 0) halves[wave] = t;
+    __syncthreads();
+    if (tid == 0) p.dD[(size_t)(u.b * p.nchunks + u.c) * p.heads + u.h] = (halves[0] + halves[1]) + (halves[2] + halves[3]);
+  }
+}
+
+}  // namespace ssm

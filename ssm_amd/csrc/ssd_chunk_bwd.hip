@@ -1,0 +1,425 @@
+// Backward of the side-by-side SSD (ssd_chunk.hpp) for bfloat16 calls:
+//
+//   states  dy = dout silu(z), rounded and kept; what each chunk adds to the adjoint state
+//   carry   the adjoint state leaving each chunk, last to first, and <G, H> at the chunk boundaries
+//   scan    y again for dz and its row sums;  u for dx and its row sums
+//   dbc     dB and dC, every head of a group in one workgroup
+//   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one launch adds those up
+//
+// What the forward prepared (steps, running sums, operand fragments, the states entering the chunks) is read, not formed again.
+#include "ssd_chunk.hpp"
+
+namespace ssm {
+
+typedef __bf16 elem_t;
+
+// ---------------------------------------------------------------------- dB, dC
+
+// Inside a chunk dB and dC follow from one matrix, summed over the heads h of the group,
+//   M[l,s] = sum_h dt_s exp(cs_l - cs_s) <dy_l, x_s>   (s <= l),      dC_l = sum_s M[l,s] B_s,   dB_s = sum_l M[l,s] C_l,
+// and across chunk boundaries dC_l += sum_h exp(cs_l) dy_l.H_c,   dB_s += sum_h dt_s exp(cs_Q - cs_s) x_s.G_c.
+struct SsdDbcParams {
+  const elem_t *x, *dy;          // (B, L, H, 64)
+  const float *H, *G;            // states entering / adjoint states leaving the chunks, fragment order
+  const float *dA2, *dtv;
+  const void *Btblk, *Ctblk;
+  elem_t *dB, *dC;               // (B, L, G, N)
+  int len, heads, groups, nchunks, units;      // units = batch * nchunks * groups
+};
+
+// A workgroup of 8 waves takes 64 rows of dC (or of dB) of one (batch, chunk, group) and walks the heads: the 64 own rows,
+// all rows they meet (s <= l, or l >= s) and the state of the next head are on their way from L2 to registers while those
+// of this head, in LDS, are multiplied (one barrier per head).  Wave w has the own tile w & 1 and every fourth of the
+// tiles it meets; M stays in its accumulators, in float32, over all heads and is rounded once, for the product with B or C.
+// Rows are read whole (128 bytes a row) and turned into fragments by LDS, 16-byte pieces XOR-swizzled by row.
+// The 64-row cut keeps the reads at 2.5 times the tensors (32 rows: 4.5 times) with 8 such workgroups per chunk.
+template <int Q, int N>
+__global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
+  typedef V8<elem_t> v8;
+  constexpr int KS = Q >> 4, KN = N >> 4, NT = N >> 5, NR = Q >> 6, QMASK = Staging<Q>::QMASK;
+  constexpr int TILE = 64 * 64, BUF = (1 + NR) * TILE + N * 64;        // own rows, met rows, state
+  extern __shared__ __align__(16) unsigned char smem[];
+  elem_t *bufs = reinterpret_cast<elem_t *>(smem);                     // [2][BUF]
+  float *steps = reinterpret_cast<float *>(smem + 2 * BUF * sizeof(elem_t));     // [2][4][Q]: running sum, log2 dt, P, R
+  const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
+  const int m = lane & 31, g2 = lane >> 5, ot = wave & 1, k4 = wave >> 1;
+  // the workgroups that meet the most rows start first
+  const unsigned rank = blockIdx.x / (2u * p.units), rest = blockIdx.x % (2u * p.units);
+  const bool for_b = rest & 1;
+  const unsigned unit = rest >> 1;
+  const int r = for_b ? (int)rank : NR - 1 - (int)rank;
+  const int meets = (int)(NR - rank);                                  // blocks of 64 rows
+  const int g = (int)(unit % p.groups), bc = (int)(unit / p.groups), c = bc % p.nchunks, b = bc / p.nchunks;
+  const int per = p.heads / p.groups, h0 = g * per;
+  const int rows = min(Q, p.len - c * Q);
+  if (64 * r >= rows) return;
+  const size_t pitch = (size_t)p.heads * SSD_P;
+  const size_t row0 = ((size_t)b * p.len + (size_t)c * Q) * pitch + h0 * SSD_P;
+  const elem_t *own_src = (for_b ? p.x : p.dy) + row0, *met_src = (for_b ? p.dy : p.x) + row0;
+  const float *st_src = (for_b ? p.G : p.H) + ((size_t)bc * p.heads + h0) * (SSD_P * N);
+  const size_t step0 = (((size_t)b * p.heads + h0) * p.nchunks + c) * Q, step_pitch = (size_t)p.nchunks * Q;
+  const int met0 = for_b ? 64 * r : 0;                                 // first met row
+
+  // ---- one head's operands, global -> registers -> LDS
+  const int lr = tid >> 3, piece = tid & 7;                            // row of a 64-row block, 16-byte piece
+  const unsigned own_at = (unsigned)min(64 * r + lr, rows - 1) * (unsigned)pitch + piece * 8;
+  unsigned met_at[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) met_at[k] = (unsigned)min(met0 + 64 * k + lr, rows - 1) * (unsigned)pitch + piece * 8;
+  // 4 channels x 4 states of the state per thread: in fragment order states run along memory, so the transposition to
+  // [n][p] is one of 4 x 4 registers
+  const bool st_mine = tid < N * 4;
+  const int st_pq = tid & 7, st_j = (tid >> 3 & 1) * 4, st_up = tid >> 4 & 1, st_frag = tid >> 5;
+  v8 own_r, met_r[NR];
+  float4 st_r[4];
+  float cs_r = 0.0f, dt_r = 0.0f, cs_b = 0.0f;
+  const auto fetch = [&](int h) {
+    own_r = *reinterpret_cast<const v8 *>(own_src + h * SSD_P + own_at);
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (k < meets) met_r[k] = *reinterpret_cast<const v8 *>(met_src + h * SSD_P + met_at[k]);
+    if (st_mine) {
+      const float *s = st_src + (size_t)h * (SSD_P * N) + st_frag * SSD_FRAG + (32 * st_up + 4 * st_pq) * 8 + st_j;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) st_r[i] = *reinterpret_cast<const float4 *>(s + i * 8);
+    }
+    if (tid < Q) {
+      cs_r = p.dA2[step0 + h * step_pitch + tid];
+      dt_r = p.dtv[step0 + h * step_pitch + tid];
+      if (wave) cs_b = p.dA2[step0 + h * step_pitch + 64 * wave - 1];
+    }
+  };
+  const auto put = [&](int at) {
+    elem_t *own = bufs + at * BUF, *met = own + TILE, *st = met + NR * TILE;
+    *reinterpret_cast<v8 *>(own + lr * 64 + ((piece ^ (lr & 7)) << 3)) = own_r;
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (k < meets) *reinterpret_cast<v8 *>(met + (64 * k + lr) * 64 + ((piece ^ (lr & 7)) << 3)) = met_r[k];
+    if (st_mine) {
+      const int n0 = 16 * (st_frag % KN) + 8 * st_up + st_j, p0 = 32 * (st_frag / KN) + 4 * st_pq;
+      const float t[4][4] = {{st_r[0].x, st_r[1].x, st_r[2].x, st_r[3].x}, {st_r[0].y, st_r[1].y, st_r[2].y, st_r[3].y},
+                             {st_r[0].z, st_r[1].z, st_r[2].z, st_r[3].z}, {st_r[0].w, st_r[1].w, st_r[2].w, st_r[3].w}};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) store4_e<elem_t>(st + (n0 + j) * 64 + (((p0 >> 3) ^ ((n0 + j) & 7)) << 3) + (p0 & 7), t[j]);
+    }
+    if (tid < Q) {
+      // decays from the block of 32 before to a step, and (times dt) from a step to the end of its block
+      float *t = steps + 4 * at * Q + tid;
+      const float before = __shfl(cs_r, 31, WAVE);
+      t[0] = cs_r;
+      t[Q] = log2_hw(dt_r);                                            // dt = 0: -inf, a weight of zero
+      t[2 * Q] = exp2_hw(fminf(cs_r - (lane & 32 ? before : cs_b), 0.0f));
+      t[3 * Q] = dt_r * exp2_hw(fminf(__shfl(cs_r, lane | 31, WAVE) - cs_r, 0.0f));
+    }
+  };
+  const auto frag = [&](const elem_t *tile, int row, int kp) {
+    return load_frag_e<elem_t>(tile + row * 64 + (((2 * kp + g2) ^ (row & 7)) << 3));
+  };
+
+  f32x16_t M[NR / 2 ? NR / 2 : 1], out = {0};
+#pragma unroll
+  for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) M[i] = (f32x16_t){0};
+  const int own_row = 64 * r + 32 * ot + m;                            // of the chunk
+  fetch(0);
+  put(0);
+  __syncthreads();
+  for (int h = 0; h < per; ++h) {
+    const int at = h & 1;
+    if (h + 1 < per) fetch(h + 1);
+    const elem_t *own = bufs + at * BUF, *met = own + TILE, *st = met + NR * TILE;
+    const float *cs = steps + 4 * at * Q, *l2 = cs + Q, *P = l2 + Q, *R = P + Q;
+    const float cs_own = cs[own_row], l2_own = l2[own_row];
+    v8 of[4];
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp) of[kp] = frag(own, 32 * ot + m, kp);
+#pragma unroll
+    for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) {
+      const int t = k4 + 4 * i, tile = (met0 >> 5) + t, mine = 2 * r + ot;
+      if (t < 2 * meets && (for_b ? tile >= mine : tile <= mine)) {
+        f32x16_t d = {0};
+#pragma unroll
+        for (int kp = 0; kp < 4; ++kp) d = mma(frag(met, 32 * t + m, kp), of[kp], d);
+        if (tile == mine) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int row = 32 * tile + 8 * q + 4 * g2;
+            const float4 c4 = *reinterpret_cast<const float4 *>(cs + row), l4 = *reinterpret_cast<const float4 *>(l2 + row);
+            const float cm[4] = {c4.x, c4.y, c4.z, c4.w}, lm[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              // dt_s exp(min(cs_l - cs_s, 0)) as one exponential
+              const float w = for_b ? exp2_hw(fminf(cm[j] - cs_own, 0.0f) + l2_own) : exp2_hw(fminf(cs_own - cm[j], 0.0f) + lm[j]);
+              const bool in = for_b ? row + j >= own_row : row + j <= own_row;
+              M[i][4 * q + j] = __builtin_fmaf(in ? w : 0.0f, d[4 * q + j], M[i][4 * q + j]);
+            }
+          }
+        } else {
+          // off the diagonal a factor per own row, a scalar per pair of blocks and a factor per met row (ssd_chunk.hpp)
+          const int lb = for_b ? tile : mine, sb = for_b ? mine : tile;
+          const float f = (for_b ? R : P)[own_row] * exp2_hw(fminf(cs[32 * lb - 1] - cs[32 * sb + 31], 0.0f));
+          const float *T = (for_b ? P : R) + 32 * tile + 4 * g2;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float4 t = *reinterpret_cast<const float4 *>(T + 8 * q);
+            M[i][4 * q] = __builtin_fmaf(t.x * f, d[4 * q], M[i][4 * q]);
+            M[i][4 * q + 1] = __builtin_fmaf(t.y * f, d[4 * q + 1], M[i][4 * q + 1]);
+            M[i][4 * q + 2] = __builtin_fmaf(t.z * f, d[4 * q + 2], M[i][4 * q + 2]);
+            M[i][4 * q + 3] = __builtin_fmaf(t.w * f, d[4 * q + 3], M[i][4 * q + 3]);
+          }
+        }
+      }
+    }
+    if (k4 < NT) {
+      f32x16_t d = {0};
+#pragma unroll
+      for (int kp = 0; kp < 4; ++kp) d = mma(frag(st, 32 * k4 + m, kp), of[kp], d);
+      const float w = for_b ? exp2_hw(fminf(cs[Q - 1] - cs_own, 0.0f) + l2_own) : exp2_hw(cs_own);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) out[j] = __builtin_fmaf(w, d[j], out[j]);
+    }
+    if (h + 1 < per) put(at ^ 1);
+    __syncthreads();
+  }
+  // ---- M, rounded, as an operand (rows = own, columns = met), times the columns of B (of C)
+  elem_t *Ms = bufs;                                                   // [64][Q]
+#pragma unroll
+  for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) {
+    const int t = k4 + 4 * i, row = 32 * ot + m;
+    if (t < 2 * meets) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v[4] = {M[i][4 * q], M[i][4 * q + 1], M[i][4 * q + 2], M[i][4 * q + 3]};
+        store4_e<elem_t>(Ms + row * Q + (((4 * t + q) ^ (row & QMASK)) << 3) + 4 * g2, v);
+      }
+    }
+  }
+  __syncthreads();
+  if (k4 >= NT) return;
+  const elem_t *bt = reinterpret_cast<const elem_t *>(for_b ? p.Ctblk : p.Btblk) + (((size_t)unit * KS + (met0 >> 4)) * NT + k4) * SSD_FRAG + lane * 8;
+  for (int ks = 0; ks < 4 * meets; ++ks) {
+    const int row = 32 * ot + m;
+    out = mma(load_frag_e<elem_t>(bt + ks * NT * SSD_FRAG),
+              load_frag_e<elem_t>(Ms + row * Q + (((2 * ks + g2) ^ (row & QMASK)) << 3)), out);
+  }
+  if (own_row < rows) {
+    elem_t *dst = (for_b ? p.dB : p.dC) + (((size_t)b * p.len + (size_t)c * Q + own_row) * p.groups + g) * N + 32 * k4 + 4 * g2;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v[4] = {out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
+      store4_e<elem_t>(dst + 8 * q, v);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------- dt
+
+// With q_t = a_t <G_t, H_{t-1}>:  ddt_t = A q_t + <x_t, u_t>,  dA = sum dt_t q_t.  Inside a chunk q follows from row sums of the
+// two scans, q_{t+1} = q_t + <dt_t x_t, u_t> - <dy_t, y_t>, starting at each chunk's first step from <G, H> at the boundary
+// (float32 states): what the two scans round differently adds up over one chunk only.
+struct SsdDtParams {
+  const float *s2, *xu, *s1;     // (B, H, nc, Q)
+  const float *dtv;
+  const float *anchor;           // (B, H, nc, anchors) partial sums
+  const void *dt_raw;            // (B, L, H)
+  const float *A, *bias;
+  void *ddt;                     // (B, L, H)
+  float *dA, *dbias;             // (B, nc, H) partial sums
+  int len, heads, nchunks, anchors, dt_dtype, softplus;
+  float dt_min, dt_max;
+};
+
+// A workgroup takes a chunk of 4 heads, a wave one of them, each lane Q / 64 neighbouring steps.  (16 heads per workgroup, a
+// row's 32 bytes together: 64 workgroups and 16 us at batch 4, 2048 steps, 24 heads.)
+constexpr int DT_HEADS = 4;
+template <int Q>
+__global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
+  constexpr int PER = Q / 64;
+  __shared__ float tile[DT_HEADS][Q + 1];
+  const int hgroups = (p.heads + DT_HEADS - 1) / DT_HEADS;
+  const int hg = (int)(blockIdx.x % hgroups), bc = (int)(blockIdx.x / hgroups), c = bc % p.nchunks, b = bc / p.nchunks;
+  const int h0 = hg * DT_HEADS, rows = min(Q, p.len - c * Q);
+  const size_t base = ((size_t)b * p.len + (size_t)c * Q) * p.heads + h0;
+  const int hh = (int)threadIdx.x % DT_HEADS, l0 = (int)threadIdx.x / DT_HEADS;
+  for (int l = l0; l < Q; l += 256 / DT_HEADS)
+    tile[hh][l] = h0 + hh < p.heads && l < rows ? load_as_f32(p.dt_raw, p.dt_dtype, base + (size_t)l * p.heads + hh) : 0.0f;
+  __syncthreads();
+  const int wave = wave_id_uniform(), lane = lane_id();
+  for (int k = wave; k < DT_HEADS; k += 4) {
+    const int h = h0 + k;
+    if (h >= p.heads) break;
+    const size_t unit = ((size_t)b * p.heads + h) * p.nchunks + c, at = unit * Q + lane * PER;
+    float s1[PER], s2[PER], xu[PER], dt[PER], d[PER], tot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      s1[i] = p.s1[at + i];
+      s2[i] = p.s2[at + i];
+      xu[i] = p.xu[at + i];
+      dt[i] = p.dtv[at + i];
+    }
+    const float a0 = wave_sum(lane < p.anchors ? p.anchor[unit * p.anchors + lane] : 0.0f);
+    const float A = p.A[h], bias = p.bias ? p.bias[h] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      d[i] = tot;
+      tot += s1[i] - s2[i];
+    }
+    const float before = a0 + wave_prev(wave_inclusive_sum(tot), 0.0f);
+    float dA = 0.0f, db = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int l = lane * PER + i;
+      const float q = before + d[i];
+      const float raw = tile[k][l] + bias;
+      const float v = p.softplus ? softplus_f32(raw) : raw;
+      const float chain = v >= p.dt_min && v <= p.dt_max ? (p.softplus ? sigmoid_f32(raw) : 1.0f) : 0.0f;
+      const float g = l < rows ? __builtin_fmaf(A, q, xu[i]) * chain : 0.0f;
+      dA = l < rows ? __builtin_fmaf(dt[i], q, dA) : dA;
+      db += g;
+      tile[k][l] = g;
+    }
+    dA = wave_sum(dA);
+    db = wave_sum(db);
+    if (lane == 0) {
+      p.dA[(size_t)bc * p.heads + h] = dA;
+      p.dbias[(size_t)bc * p.heads + h] = db;
+    }
+  }
+  __syncthreads();
+  if (h0 + hh < p.heads)
+    for (int l = l0; l < rows; l += 256 / DT_HEADS) store_any(p.ddt, p.dt_dtype, base + (size_t)l * p.heads + hh, tile[hh][l]);
+}
+
+// ---------------------------------------------------------------------- host
+
+struct BwdLayout {
+  size_t dy, states, s2, xu, s1, anchor, dA, dbias, dD, total;
+};
+
+static BwdLayout bwd_layout(const SsdDims &d) {
+  BwdLayout f;
+  const size_t units = (size_t)d.batch * d.nchunks * d.heads;
+  size_t at = 0;
+  const auto take = [&](size_t bytes) { const size_t v = at; at += ssd_align_up(bytes); return v; };
+  f.dy = take((size_t)d.batch * d.len * d.heads * SSD_P * 2);
+  f.states = take(units * SSD_P * d.nstate * 4);
+  f.s2 = take(units * d.chunk * 4);
+  f.xu = take(units * d.chunk * 4);
+  f.s1 = take(units * d.chunk * 4);
+  f.anchor = take(units * (SSD_P * d.nstate / 256) * 4);
+  f.dA = take(units * 4);
+  f.dbias = take(units * 4);
+  f.dD = take(units * 4);
+  f.total = at;
+  return f;
+}
+
+static SsdDims plain_dims(const ssm_ssd_dims &s) {
+  SsdDims d;
+  d.batch = s.batch; d.len = s.seqlen; d.heads = s.heads; d.hdim = s.headdim; d.groups = s.groups;
+  d.nstate = s.nstate; d.chunk = s.chunk; d.nchunks = (s.seqlen + s.chunk - 1) / s.chunk;
+  return d;
+}
+
+static bool bwd_shape_ok(const ssm_ssd_dims *s, int io_dtype) {
+  if (!s || io_dtype != SSM_BF16 || !ssm_ssd_combined_supported(s, io_dtype)) return false;
+  const SsdDims d = plain_dims(*s);
+  // a chunk's rows are addressed by 32-bit offsets
+  return (size_t)d.batch * d.nchunks * d.heads < ((size_t)1 << 26) && (size_t)d.chunk * d.heads * SSD_P < ((size_t)1 << 31);
+}
+
+template <int Q, int N>
+static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca, const SsdChunkScanParams &dz,
+                             const SsdChunkScanParams &dx, const SsdDbcParams &bc, const SsdDtParams &dt, const SsdDims &d,
+                             hipStream_t s) {
+  const dim3 units((unsigned)(d.batch * d.nchunks * d.heads)), block(256);
+  constexpr size_t dbc_lds = 2 * ((1 + Q / 64) * 64 * 64 + N * 64) * sizeof(elem_t) + 8 * Q * sizeof(float);
+  if (allow_dynamic_lds(ssd_dbc_kernel<Q, N>, dbc_lds) != hipSuccess) {
+    set_error("ssm_ssd_combined_bwd: cannot reserve %zu bytes of LDS", dbc_lds);
+    return SSM_ERR_LAUNCH;
+  }
+  hipLaunchKernelGGL((ssd_states_kernel<elem_t, Q, N, true>), units, block, 0, s, st);
+  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true>), dim3((unsigned)(d.batch * d.heads) * (SSD_P * N / 1024)), block, 0, s, ca);
+  if (dz.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, true>), units, block, 0, s, dz);
+  else hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, false>), units, block, 0, s, dz);
+  hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DX, false>), units, block, 0, s, dx);
+  hipLaunchKernelGGL((ssd_dbc_kernel<Q, N>), dim3(2u * bc.units * (Q / 64)), dim3(512), dbc_lds, s, bc);
+  hipLaunchKernelGGL((ssd_dt_kernel<Q>), dim3((unsigned)(d.batch * d.nchunks * ((d.heads + DT_HEADS - 1) / DT_HEADS))), block, 0, s, dt);
+  return SSM_OK;
+}
+
+}  // namespace ssm
+
+extern "C" int ssm_ssd_combined_bwd_supported(const ssm_ssd_dims *dims, int io_dtype) { return ssm::bwd_shape_ok(dims, io_dtype) ? 1 : 0; }
+
+extern "C" size_t ssm_ssd_combined_bwd_workspace_bytes(const ssm_ssd_dims *dims) {
+  return ssm::bwd_shape_ok(dims, SSM_BF16) ? ssm::bwd_layout(ssm::plain_dims(*dims)).total : 0;
+}
+
+extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hip_stream) {
+  using namespace ssm;
+  SSM_REQUIRE(a && a->fwd.x && a->fwd.dt && a->fwd.A && a->fwd.workspace && a->dout && a->dx && a->dB && a->dC && a->ddt && a->dA,
+              SSM_ERR_NULL_POINTER, "ssm_ssd_combined_bwd: x, dt, A, the forward's workspace, dout, dx, dB, dC, ddt and dA are required");
+  const ssm_ssd_combined_args &f = a->fwd;
+  SSM_REQUIRE(bwd_shape_ok(&f.dims, f.io_dtype) && !f.seq_idx && !f.d_per_p && f.keep_for_backward, SSM_ERR_BAD_SHAPE,
+              "ssm_ssd_combined_bwd: needs a bf16 forward run with keep_for_backward, a shape ssm_ssd_combined_bwd_supported accepts, "
+              "no seq_idx and no per-channel Dskip");
+  SSM_REQUIRE(valid_dtype(f.dt_dtype), SSM_ERR_BAD_DTYPE, "ssm_ssd_combined_bwd: dt_dtype=%d", f.dt_dtype);
+  const SsdDims d = plain_dims(f.dims);
+  const SsdWorkLayout kept = ssd_work_layout(d, true);
+  const BwdLayout lay = bwd_layout(d);
+  SSM_REQUIRE(f.workspace_bytes >= kept.total && a->workspace && a->workspace_bytes >= lay.total, SSM_ERR_WORKSPACE,
+              "ssm_ssd_combined_bwd: workspaces of %zu (kept) and %zu bytes required", kept.total, lay.total);
+  SSM_REQUIRE((f.z != nullptr) == (a->dz != nullptr), SSM_ERR_NULL_POINTER, "ssm_ssd_combined_bwd: dz is given exactly with z");
+  SSM_REQUIRE(aligned_to(f.x, 16) && aligned_to(a->dout, 16) && (!f.z || aligned_to(f.z, 16)) && aligned_to(a->dx, 16) &&
+                  (!a->dz || aligned_to(a->dz, 16)) && aligned_to(a->dB, 8) && aligned_to(a->dC, 8) && aligned_to(f.workspace, 256) &&
+                  aligned_to(a->workspace, 256) && (!a->dinitial_states || aligned_to(a->dinitial_states, 16)),
+              SSM_ERR_ALIGNMENT, "ssm_ssd_combined_bwd: tensors must be 16-byte aligned (workspaces 256)");
+  hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
+  const unsigned char *kw = reinterpret_cast<const unsigned char *>(f.workspace);
+  unsigned char *ws = reinterpret_cast<unsigned char *>(a->workspace);
+  const float *dA2 = reinterpret_cast<const float *>(kw + kept.dA2), *dtv = reinterpret_cast<const float *>(kw + kept.dt_out);
+  const float *H = reinterpret_cast<const float *>(kw + kept.states);
+  float *G = reinterpret_cast<float *>(ws + lay.states);
+  const auto f32 = [&](size_t off) { return reinterpret_cast<float *>(ws + off); };
+
+  SsdStatesParams st{};
+  st.x = a->dout; st.z = f.z; st.dy = ws + lay.dy; st.frag = kw + kept.Ctblk; st.dA2 = dA2; st.dtv = dtv; st.states = G;
+  st.len = d.len; st.heads = d.heads; st.groups = d.groups; st.nchunks = d.nchunks;
+  SsdCarryParams ca{};
+  ca.states = G; ca.dA2 = dA2; ca.first = a->dfinal; ca.last = a->dinitial_states; ca.entering = H; ca.anchor = f32(lay.anchor);
+  ca.heads = d.heads; ca.nchunks = d.nchunks; ca.chunk = d.chunk; ca.nstate = d.nstate;
+  SsdChunkScanParams dz{};
+  dz.op = f.x; dz.blk = kw + kept.CBblk; dz.carry = kw + kept.Cblk; dz.states = H; dz.dA2 = dA2; dz.dtv = dtv; dz.Dk = f.Dskip;
+  dz.x = f.x; dz.dy = ws + lay.dy; dz.z = f.z; dz.dout = a->dout; dz.out = a->dz; dz.sum0 = f32(lay.s2);
+  dz.dD = f.Dskip ? f32(lay.dD) : nullptr; dz.len = d.len; dz.heads = d.heads; dz.groups = d.groups; dz.nchunks = d.nchunks;
+  dz.has_first = f.initial_states != nullptr;
+  SsdChunkScanParams dx = dz;
+  dx.op = ws + lay.dy; dx.blk = kw + kept.CBtblk; dx.carry = kw + kept.Bblk; dx.states = G; dx.z = nullptr; dx.out = a->dx;
+  dx.sum0 = f32(lay.xu); dx.sum1 = f32(lay.s1); dx.dD = nullptr; dx.has_first = a->dfinal != nullptr;
+  SsdDbcParams bc{};
+  bc.x = reinterpret_cast<const elem_t *>(f.x); bc.dy = reinterpret_cast<const elem_t *>(ws + lay.dy); bc.H = H; bc.G = G;
+  bc.dA2 = dA2; bc.dtv = dtv; bc.Btblk = kw + kept.Btblk; bc.Ctblk = kw + kept.Ctblk;
+  bc.dB = reinterpret_cast<elem_t *>(a->dB); bc.dC = reinterpret_cast<elem_t *>(a->dC);
+  bc.len = d.len; bc.heads = d.heads; bc.groups = d.groups; bc.nchunks = d.nchunks; bc.units = d.batch * d.nchunks * d.groups;
+  SsdDtParams dt{};
+  dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.anchor = f32(lay.anchor); dt.dt_raw = f.dt;
+  dt.A = f.A; dt.bias = f.dt_bias; dt.ddt = a->ddt; dt.dA = f32(lay.dA); dt.dbias = f32(lay.dbias);
+  dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.anchors = SSD_P * d.nstate / 256; dt.dt_dtype = f.dt_dtype;
+  dt.softplus = f.dt_softplus ? 1 : 0; dt.dt_min = f.dt_min; dt.dt_max = f.dt_max;
+
+  int rc = SSM_OK;
+#define SSM_CHUNK_BACKWARD(QQ, NN) \
+  if (d.chunk == QQ && d.nstate == NN) rc = backward_launches<QQ, NN>(st, ca, dz, dx, bc, dt, d, s);
+  SSM_CHUNK_BACKWARD(256, 128) SSM_CHUNK_BACKWARD(128, 128) SSM_CHUNK_BACKWARD(64, 128)
+  SSM_CHUNK_BACKWARD(256, 64) SSM_CHUNK_BACKWARD(128, 64) SSM_CHUNK_BACKWARD(64, 64)
+#undef SSM_CHUNK_BACKWARD
+  if (rc != SSM_OK) return rc;
+  FoldJobs jobs{};
+  const int parts = d.batch * d.nchunks;
+  jobs.add(f32(lay.dA), a->dA, 1, parts, (size_t)d.heads, SSM_F32);
+  if (a->ddt_bias) jobs.add(f32(lay.dbias), a->ddt_bias, 1, parts, (size_t)d.heads, SSM_F32);
+  if (a->dD && f.Dskip) jobs.add(f32(lay.dD), a->dD, 1, parts, (size_t)d.heads, SSM_F32);
+  launch_fold_jobs(jobs, s);
+  SSM_CHECK_LAUNCH("ssm_ssd_combined_bwd");
+  return SSM_OK;
+}

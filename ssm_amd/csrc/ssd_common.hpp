@@ -85,6 +85,53 @@ struct SsdScanParams {
   int x_reversed;             // as in SsdStateParams
 };
 
+// ---- the matrix-core forward and backward of 16-bit calls (ssd_fused.hip, ssd_chunk*.hip): heads of 64 channels, chunks of
+// 64, 128 or 256 steps, 64 or 128 states; nc = ceil(L / Q) chunks, the last one of any length.
+constexpr int SSD_P = 64;
+constexpr int SSD_FRAG = 512;           // elements per operand fragment: 64 lanes x 8
+
+// What one preparation launch leaves for them: byte offsets into the workspace of a call.
+struct SsdWorkLayout {
+  size_t dt_out, dA2;                   // (B, H, nc, Q) float32: the step, and its running sum times A log2(e)
+  size_t Cblk, Btblk, CBblk;            // operand fragments (prep in ssd_fused.hip)
+  size_t Bblk, Ctblk, CBtblk;           // ... that only the backward reads; empty without `keep`
+  size_t states, states16;              // (B, nc, H, 64 N) in fragment order, float32 and 16 bits (without `keep`); empty on
+                                        // the one-pass route
+  size_t total;
+};
+
+inline size_t ssd_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// Whether the forward takes the chunks side by side (ssd_chunk.hip) rather than one after the other (ssd_fused.hip).
+bool ssd_side_by_side(const SsdDims &d);
+
+inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep) {
+  SsdWorkLayout f;
+  const size_t steps = (size_t)d.nchunks * d.chunk;
+  const size_t per_step = ssd_align_up((size_t)d.batch * d.heads * steps * sizeof(float));
+  const size_t bc = ssd_align_up((size_t)d.batch * steps * d.groups * d.nstate * 2);
+  const size_t cb = ssd_align_up((size_t)d.batch * steps * d.groups * d.chunk * 2);
+  size_t at = 0;
+  f.dt_out = at; at += per_step;
+  f.dA2 = at; at += per_step;
+  f.Cblk = at; at += bc;
+  f.Btblk = at; at += bc;
+  f.CBblk = at; at += cb;
+  f.Bblk = at; at += keep ? bc : 0;
+  f.Ctblk = at; at += keep ? bc : 0;
+  f.CBtblk = at; at += keep ? cb : 0;
+  f.states = at;
+  const size_t states = (size_t)d.batch * d.nchunks * d.heads * SSD_P * d.nstate;
+  if (keep || ssd_side_by_side(d)) at += ssd_align_up(states * sizeof(float));
+  f.states16 = at;
+  if (!keep && ssd_side_by_side(d)) at += ssd_align_up(states * 2);
+  f.total = at;
+  return f;
+}
+
+// x -> y, final states; the states entering the chunks stay in the workspace.
+int ssd_chunk_forward(const ssm_ssd_combined_args &a, const SsdDims &d, const SsdWorkLayout &lay, hipStream_t s);
+
 __device__ __forceinline__ void store_any(void *p, int dtype, size_t i, float v) {
   if (dtype == SSM_F32) reinterpret_cast<float *>(p)[i] = v;
   else if (dtype == SSM_BF16) reinterpret_cast<bf16_t *>(p)[i] = from_f32<bf16_t>(v);

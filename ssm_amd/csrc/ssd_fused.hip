@@ -22,7 +22,7 @@
 // B, C and CB are re-laid once per call so that every MFMA operand fragment is
 // one contiguous KiB (64 lanes x 8 bf16).
 //
-// Requires bf16 or fp16 tensors (the kernels are compiled per element type), P = 64, Q in {64, 128, 256}, N in {64, 128} and L % Q == 0.
+// Requires bf16 or fp16 tensors (the kernels are compiled per element type), P = 64, Q in {64, 128, 256}, N in {64, 128}.
 //
 // A head with A > 0 (a growing state): the published kernels evaluate the decays inside a chunk as
 // exp(min(x, 0)) - chunk_state's weights and chunk_scan's in-chunk factors - and leave the two factors on the
@@ -35,8 +35,8 @@
 
 namespace ssm {
 
-constexpr int FU_P = 64;
-constexpr int FRAG = 512;                                  // bf16 elements per operand fragment
+constexpr int FU_P = SSD_P;
+constexpr int FRAG = SSD_FRAG;
 
 struct SsdFusedParams {                 // x, z, y and the fragment copies hold the call's 16-bit element type
   const void *x, *z;
@@ -68,16 +68,21 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 //        32 x 16 block: row 32 rb + lane % 32, column 16 kb + 8 (lane / 32) + j.
 //          Cblk [(b,c,g)][lb][kn]  from C  (rows = time, columns = state)
 //          Btblk[(b,c,g)][ks][nt]  from B  (rows = state, columns = time)
+//        and, where a backward will follow, Bblk and Ctblk with B and C in each other's place.
 //  CB:   one wave per 32 x 32 block on or below the diagonal of C B^T of a chunk:
 //        MFMA over the state dimension, then through a wave-private LDS tile into
 //          CBblk[(b,c,g)][lb][ks]  (rows = l, columns = s),
-//        with zeros above the diagonal inside the diagonal blocks.
+//        with zeros above the diagonal inside the diagonal blocks; for a backward also its transpose,
+//          CBtblk[(b,c,g)][sb][kl]  (rows = s, columns = l).
+// Steps past the end of a last chunk that is no whole one: size zero, rows of B and C zero.
 constexpr int PD_HEADS = 4;
 struct SsdPrepParams {
   SsdCumsumParams cs;
   float *dA2;
   const void *Cm, *Bm;                   // element type of the call
   void *Cblk, *Btblk, *CBblk;
+  void *Bblk, *Ctblk, *CBtblk;           // what the backward reads besides (n_kinds = 4), or null
+  unsigned n_kinds;
   unsigned n_dt, n_pack;                 // workgroups of the first two roles
   const int *seq_idx;                    // (B, L) sequence ids of a packed batch, or null
   size_t b_row, c_row;                   // elements between the (G, N) blocks of consecutive steps in Bm / Cm
@@ -102,12 +107,14 @@ __device__ __forceinline__ void prep_dt_role(const SsdCumsumParams &p, float *dA
   for (int e = threadIdx.x; e < Q * PD_HEADS; e += 256) {
     const int l = e / PD_HEADS, hh = e % PD_HEADS;
     float v = 0.0f;
-    if (h0 + hh < d.heads) v = load_as_f32(p.dt, p.dt_dtype, ((size_t)b * d.len + (size_t)c * Q + l) * d.heads + h0 + hh);
+    if (h0 + hh < d.heads && c * Q + l < d.len)
+      v = load_as_f32(p.dt, p.dt_dtype, ((size_t)b * d.len + (size_t)c * Q + l) * d.heads + h0 + hh);
     tile[hh][l] = v;
   }
   __syncthreads();
   const int wave = wave_id_uniform(), lane = lane_id();
   const int per = (Q + 63) >> 6;
+  const int rows = min(Q, d.len - c * Q);          // steps past the end have size zero
   for (int hh = wave; hh < PD_HEADS; hh += 4) {
     const int h = h0 + hh;
     if (h >= d.heads) break;
@@ -119,13 +126,13 @@ __device__ __forceinline__ void prep_dt_role(const SsdCumsumParams &p, float *dA
     for (int i = 0; i < 4; ++i) {
       const int l = lane * per + i;
       v[i] = 0.0f;
-      if (i < per && l < Q) {
+      if (i < per && l < rows) {
         float x = tile[hh][l] + bias;
         if (p.softplus) x = softplus_f32(x);
         v[i] = fminf(fmaxf(x, p.dt_min), p.dt_max);
       }
       tot = __builtin_fmaf(v[i], A, tot);
-      if (seq_idx && i < per && l < Q) {
+      if (seq_idx && i < per && l < rows) {
         const size_t t = (size_t)c * Q + l;
         const int *sid = seq_idx + (size_t)b * d.len;
         if (t == 0 ? sid[0] != 0 : sid[t] != sid[t - 1]) tot += SEQ_JUMP_LN;
@@ -153,35 +160,43 @@ __device__ __forceinline__ void prep_dt_role(const SsdCumsumParams &p, float *dA
 
 template <typename E>
 __device__ __forceinline__ void prep_pack_role(const SsdPrepParams &pp, unsigned wg) {
-  const E *Cm = reinterpret_cast<const E *>(pp.Cm), *Bm = reinterpret_cast<const E *>(pp.Bm);
   const SsdDims &d = pp.cs.d;
   const int wave = wave_id_uniform(), lane = lane_id();
   const int Q = d.chunk, N = d.nstate, nc = d.nchunks, groups = d.groups, len = d.len;
-  const int NLB = Q >> 5, KS = Q >> 4, KN = N >> 4, NT = N >> 5;
-  const size_t units = (size_t)d.batch * nc * groups;
-  const size_t nC = units * NLB * KN, nB = units * KS * NT;
+  const int KN = N >> 4, NT = N >> 5;
+  const int per_unit = (Q >> 5) * KN;                     // = (Q / 16) * NT
+  const size_t each = (size_t)d.batch * nc * groups * per_unit;
   size_t f = (size_t)wg * 4 + wave;
-  if (f >= nC + nB) return;
-  const bool is_c = f < nC;
-  if (!is_c) f -= nC;
-  const int per_unit = is_c ? NLB * KN : KS * NT;
+  if (f >= each * pp.n_kinds) return;
+  const int kind = (int)(f / each);                       // rows of C, columns of B, rows of B, columns of C
+  f -= kind * each;
+  const bool rows = kind == 0 || kind == 2, from_c = kind == 0 || kind == 3;
+  const E *src = reinterpret_cast<const E *>(from_c ? pp.Cm : pp.Bm);
+  const size_t stride = from_c ? pp.c_row : pp.b_row;
+  void *dst = kind == 0 ? pp.Cblk : kind == 1 ? pp.Btblk : kind == 2 ? pp.Bblk : pp.Ctblk;
   const int inner = (int)(f % per_unit);
   const size_t unit = f / per_unit;
   const int g = (int)(unit % groups);
   const int c = (int)((unit / groups) % nc);
   const int b = (int)(unit / ((size_t)groups * nc));
   const int m = lane & 31, g2 = lane >> 5;
+  src += (size_t)b * len * stride + (size_t)g * N;
   V8<E> v;
-  if (is_c) {
+  if (rows) {
     const int lb = inner / KN, kn = inner % KN;
-    v = load_frag_e<E>(Cm + ((size_t)b * len + (size_t)c * Q + 32 * lb + m) * pp.c_row + (size_t)g * N + 16 * kn + 8 * g2);
+    const int t = c * Q + 32 * lb + m;
+    v = load_frag_e<E>(src + (size_t)min(t, len - 1) * stride + 16 * kn + 8 * g2);
+    if (t >= len) v = V8<E>{};
   } else {
     const int ks = inner / NT, nt = inner % NT;
-    const E *col = Bm + ((size_t)b * len + (size_t)c * Q + 16 * ks + 8 * g2) * pp.b_row + (size_t)g * N + 32 * nt + m;
+    const int t = c * Q + 16 * ks + 8 * g2;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = col[(size_t)j * pp.b_row];
+    for (int j = 0; j < 8; ++j) v[j] = src[(size_t)min(t + j, len - 1) * stride + 32 * nt + m];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (t + j >= len) v[j] = (E)0.0f;
   }
-  *reinterpret_cast<V8<E> *>(reinterpret_cast<E *>(is_c ? pp.Cblk : pp.Btblk) + f * FRAG + lane * 8) = v;
+  *reinterpret_cast<V8<E> *>(reinterpret_cast<E *>(dst) + f * FRAG + lane * 8) = v;
 }
 
 template <typename E>
@@ -200,10 +215,11 @@ __device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned w
   while ((lb + 1) * (lb + 2) / 2 <= idx) ++lb;
   const int sb = idx - lb * (lb + 1) / 2;
   const int g = (int)(unit % groups);
-  const size_t bc = unit / groups;                        // b * nchunks + c: the chunk's first row is bc * Q
+  const int c = (int)((unit / groups) % d.nchunks);
+  const size_t row0 = unit / groups / d.nchunks * d.len;  // rows past the end stand for the last one: they meet only zeros
   const int m = lane & 31, g2 = lane >> 5;
-  const E *crow_p = reinterpret_cast<const E *>(pp.Cm) + (bc * Q + 32 * lb + m) * pp.c_row + (size_t)g * N + 8 * g2;
-  const E *brow_p = reinterpret_cast<const E *>(pp.Bm) + (bc * Q + 32 * sb + m) * pp.b_row + (size_t)g * N + 8 * g2;
+  const E *crow_p = reinterpret_cast<const E *>(pp.Cm) + (row0 + min(c * Q + 32 * lb + m, d.len - 1)) * pp.c_row + (size_t)g * N + 8 * g2;
+  const E *brow_p = reinterpret_cast<const E *>(pp.Bm) + (row0 + min(c * Q + 32 * sb + m, d.len - 1)) * pp.b_row + (size_t)g * N + 8 * g2;
   f32x16_t acc = {0};
   for (int k0 = 0; k0 < N; k0 += 16) acc = mma(load_frag_e<E>(crow_p + k0), load_frag_e<E>(brow_p + k0), acc);
   float (*tile)[33] = reinterpret_cast<float (*)[33]>(lds + wave * 32 * 33);
@@ -220,6 +236,18 @@ __device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned w
       v[j] = (sb < lb || sl <= m) ? tile[m][sl] : 0.0f;
     }
     *reinterpret_cast<V8<E> *>(out + kk * FRAG) = pack8_e<E>(v);
+  }
+  if (!pp.CBtblk) return;
+  E *out_t = reinterpret_cast<E *>(pp.CBtblk) + ((unit * NLB + sb) * KS + 2 * lb) * FRAG + lane * 8;
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int ll = 16 * kk + 8 * g2 + j;
+      v[j] = (sb < lb || m <= ll) ? tile[ll][m] : 0.0f;
+    }
+    *reinterpret_cast<V8<E> *>(out_t + kk * FRAG) = pack8_e<E>(v);
   }
 }
 
@@ -433,8 +461,7 @@ void ssd_fused_half_kernel(const SsdFusedParams p) {
   const int t_dA = (int)((const char *)p.dA2 - (const char *)p.dtv);
   const rsrc_t rf = make_rsrc(p.Cblk);
   const int f_cb = (int)((const char *)p.CBblk - (const char *)p.Cblk), f_bt = (int)((const char *)p.Btblk - (const char *)p.Cblk);
-  const int srow = min(tid >> 3, (Q >> 3) - 1) * 8, spb = tid & 7;
-  const int v_raw = srow * xrow_b + spb * 8;                       // x for staging: rows srow.., 4 channels
+  const int srow = min(tid >> 3, (Q >> 3) - 1) * 8, spb = tid & 7;   // x for staging: rows srow.., 4 channels
   const int v_row = (lane >> 2) * xrow_b + (lane & 3) * 16;        // row-major passes: row lane / 4, 8 channels
   const int v_t = min(tid, Q - 1) * 4;
   HalfStream st;
@@ -459,7 +486,10 @@ void ssd_fused_half_kernel(const SsdFusedParams p) {
 #define FH_REQUEST_CHUNK(CC)                                                                              \
   {                                                                                                       \
     const int xo_ = (CC) * Q * xrow_b, to_ = (CC) * Q * 4;                                                \
-    _Pragma("unroll") for (int r = 0; r < 8; ++r) raw[r] = buf_load8<E>(rx, v_raw, xo_ + r * xrow_b);        \
+    /* rows past the end read the last one: their step is zero */                                         \
+    const int last_ = min(Q, p.len - (CC) * Q) - 1;                                                       \
+    _Pragma("unroll") for (int r = 0; r < 8; ++r)                                                         \
+      raw[r] = buf_load8<E>(rx, min(srow + r, last_) * xrow_b + spb * 8, xo_);                            \
     dA_t = buf_load_f1(rt, v_t, t_dA + to_);                                                              \
     dt_t = buf_load_f1(rt, v_t, to_);                                                                     \
   }
@@ -622,8 +652,9 @@ void ssd_fused_half_kernel(const SsdFusedParams p) {
       {                                                                                         \
         if (yact && HAS_Z) {                                                                    \
           _Pragma("unroll") for (int pass = 0; pass < 2; ++pass) {                              \
-            zF[pass] = buf_load16<E>(rz, v_row, row_o + (32 * lbF + 16 * pass) * xrow_b);          \
-            zS[pass] = buf_load16<E>(rz, v_row, row_o + (32 * lbS + 16 * pass) * xrow_b);          \
+            const int l_ = (lane >> 2) + 16 * pass, last_ = min(Q, p.len - c * Q) - 1, at_ = (lane & 3) * 16; \
+            zF[pass] = buf_load16<E>(rz, min(32 * lbF + l_, last_) * xrow_b + at_, row_o);          \
+            zS[pass] = buf_load16<E>(rz, min(32 * lbS + l_, last_) * xrow_b + at_, row_o);          \
           }                                                                                     \
         }                                                                                       \
         FH_REQUEST_CHUNK(cn)                                                                    \
@@ -699,7 +730,8 @@ void ssd_fused_half_kernel(const SsdFusedParams p) {
           // read under load (wrong dwords in the last quarter of each 16 lanes).  So the data stays live, and
           // idle slots follow the store.
           const u32x4_t packed = __builtin_bit_cast(u32x4_t, pack8_e<E>(v));
-          __builtin_amdgcn_raw_buffer_store_b128(packed, ry, v_row, row_o + (32 * lb + 16 * pass) * xrow_b, 0);
+          if (c * Q + 32 * lb + l < p.len)
+            __builtin_amdgcn_raw_buffer_store_b128(packed, ry, v_row, row_o + (32 * lb + 16 * pass) * xrow_b, 0);
           asm volatile("s_nop 3" : : "v"(packed) : "memory");
         }
         wave_lds_sync();
@@ -717,36 +749,16 @@ void ssd_fused_half_kernel(const SsdFusedParams p) {
   }
 }
 
-static size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
-
-struct FusedLayout {
-  size_t dt_out, dA2, Cblk, Btblk, CBblk, total;
-};
-
-static FusedLayout fused_layout(const SsdDims &d) {
-  FusedLayout f;
-  const size_t per_step = align_up((size_t)d.batch * d.heads * d.len * sizeof(float));
-  const size_t bc = align_up((size_t)d.batch * d.len * d.groups * d.nstate * 2);
-  const size_t cb = align_up((size_t)d.batch * d.nchunks * d.groups * d.chunk * d.chunk * 2);
-  size_t at = 0;
-  f.dt_out = at; at += per_step;
-  f.dA2 = at; at += per_step;
-  f.Cblk = at; at += bc;
-  f.Btblk = at; at += bc;
-  f.CBblk = at; at += cb;
-  f.total = at;
-  return f;
-}
-
 static bool fused_shape_ok(const SsdDims &d) {
   const bool q_ok = d.chunk == 64 || d.chunk == 128 || d.chunk == 256;
   const bool n_ok = d.nstate == 64 || d.nstate == 128;
-  if (!(q_ok && n_ok && d.hdim == FU_P && d.len % d.chunk == 0 && d.heads % d.groups == 0)) return false;
+  if (!(q_ok && n_ok && d.hdim == FU_P && d.heads % d.groups == 0)) return false;
   // the kernel addresses with 32-bit byte offsets: inside one batch row of x, z and y, inside the
   // per-step arrays and inside the fragment copies
   const size_t lim = (size_t)1 << 31;
-  const FusedLayout f = fused_layout(d);
-  return (size_t)d.len * d.heads * FU_P * 2 < lim && f.Cblk - f.dt_out + (size_t)d.len * 4 < lim && f.total - f.Cblk < lim;
+  const SsdWorkLayout f = ssd_work_layout(d, false);
+  return (size_t)d.nchunks * d.chunk * d.heads * FU_P * 2 < lim && f.Cblk - f.dt_out + (size_t)d.nchunks * d.chunk * 4 < lim &&
+         f.Bblk - f.Cblk < lim;
 }
 
 }  // namespace ssm
@@ -775,7 +787,13 @@ extern "C" int ssm_ssd_combined_supported(const ssm_ssd_dims *dims, int io_dtype
 extern "C" size_t ssm_ssd_combined_workspace_bytes(const ssm_ssd_dims *dims) {
   ssm::SsdDims d;
   if (fused_dims("ssm_ssd_combined_workspace_bytes", dims, d) != SSM_OK) return 0;
-  return ssm::fused_layout(d).total;
+  return ssm::ssd_work_layout(d, false).total;
+}
+
+extern "C" size_t ssm_ssd_combined_keep_bytes(const ssm_ssd_dims *dims) {
+  ssm::SsdDims d;
+  if (fused_dims("ssm_ssd_combined_keep_bytes", dims, d) != SSM_OK) return 0;
+  return ssm::ssd_work_layout(d, true).total;
 }
 
 extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_stream) {
@@ -789,10 +807,11 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
               "ssm_ssd_combined_fwd: x, z, y, Bm and Cm must be bf16 or fp16 (one type for all)");
   SSM_REQUIRE(valid_dtype(a->dt_dtype), SSM_ERR_BAD_DTYPE, "ssm_ssd_combined_fwd: dt_dtype=%d", a->dt_dtype);
   SSM_REQUIRE(fused_shape_ok(d), SSM_ERR_BAD_SHAPE,
-              "ssm_ssd_combined_fwd: needs headdim 64, chunk in {64,128,256}, nstate in {64,128} and "
-              "seqlen %% chunk == 0 (got headdim=%d chunk=%d nstate=%d seqlen=%d)",
-              d.hdim, d.chunk, d.nstate, d.len);
-  const FusedLayout lay = fused_layout(d);
+              "ssm_ssd_combined_fwd: needs headdim 64, chunk in {64,128,256} and nstate in {64,128} "
+              "(got headdim=%d chunk=%d nstate=%d)",
+              d.hdim, d.chunk, d.nstate);
+  const bool keep = a->keep_for_backward != 0;
+  const SsdWorkLayout lay = ssd_work_layout(d, keep);
   SSM_REQUIRE(a->workspace && a->workspace_bytes >= lay.total, SSM_ERR_WORKSPACE,
               "ssm_ssd_combined_fwd: workspace of %zu bytes required", lay.total);
   SSM_REQUIRE(aligned_to(a->x, 16) && aligned_to(a->y, 16) && (!a->z || aligned_to(a->z, 16)) && aligned_to(a->Bm, 16) &&
@@ -804,7 +823,7 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   unsigned char *ws = reinterpret_cast<unsigned char *>(a->workspace);
 
   const size_t bcg = (size_t)d.batch * d.nchunks * d.groups;
-  const int NLB = d.chunk >> 5, KS = d.chunk >> 4, KN = d.nstate >> 4, NT = d.nstate >> 5;
+  const int NLB = d.chunk >> 5, KN = d.nstate >> 4;
   SsdPrepParams pp{};
   SsdCumsumParams &cp = pp.cs;
   cp.dt = a->dt; cp.A = a->A; cp.bias = a->dt_bias;
@@ -822,8 +841,10 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   pp.c_row = a->c_row_stride ? (size_t)a->c_row_stride : dense_row;
   void *Cblk = ws + lay.Cblk, *Btblk = ws + lay.Btblk;
   pp.Cblk = Cblk; pp.Btblk = Btblk; pp.CBblk = ws + lay.CBblk;
+  pp.n_kinds = keep ? 4 : 2;
+  if (keep) { pp.Bblk = ws + lay.Bblk; pp.Ctblk = ws + lay.Ctblk; pp.CBtblk = ws + lay.CBtblk; }
   const size_t n_dt = (size_t)d.batch * d.nchunks * ((d.heads + PD_HEADS - 1) / PD_HEADS);
-  const size_t n_pack = (bcg * NLB * KN + bcg * KS * NT + 3) / 4;
+  const size_t n_pack = (bcg * NLB * KN * pp.n_kinds + 3) / 4;
   const size_t n_cb = (bcg * (NLB * (NLB + 1) / 2) + 3) / 4;
   SSM_REQUIRE(n_dt + n_pack + n_cb < ((size_t)1 << 31), SSM_ERR_TOO_LARGE, "ssm_ssd_combined_fwd: too many workgroups");
   pp.n_dt = (unsigned)n_dt; pp.n_pack = (unsigned)n_pack;
@@ -832,6 +853,8 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   if (f16) hipLaunchKernelGGL(ssd_fused_prep_kernel<_Float16>, dim3((unsigned)(n_dt + n_pack + n_cb)), dim3(256), 0, s, pp);
   else hipLaunchKernelGGL(ssd_fused_prep_kernel<__bf16>, dim3((unsigned)(n_dt + n_pack + n_cb)), dim3(256), 0, s, pp);
   SSM_CHECK_LAUNCH("ssm_ssd_combined_fwd(prep)");
+  note_mfma_launch(8);
+  if (keep || ssd_side_by_side(d)) return ssd_chunk_forward(*a, d, lay, s);
 
   SsdFusedParams fp{};
   fp.x = a->x; fp.z = a->z;
@@ -876,6 +899,5 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
 #undef SSM_LAUNCH_FUSED_DZ
 #undef SSM_LAUNCH_FUSED
   SSM_CHECK_LAUNCH("ssm_ssd_combined_fwd");
-  note_mfma_launch(8);
   return SSM_OK;
 }

@@ -367,16 +367,26 @@ def chunk_state_varlen(B, x, dt, dA_cumsum, cu_seqlens, chunk_states):
     return out
 
 
-def _fused_ok(x, dt, B, C, z, D, batch, seqlen, heads, hdim, groups, nstate, Q):
-    """Whether the one-pass kernel covers this call (bf16 or fp16 tensors of one type on the GPU and a
-    shape ``ssm_ssd_combined_supported`` accepts)."""
-    if Q <= 0 or seqlen % Q != 0:
+def _fused_ok(x, B, C, z, Q, heads, hdim):
+    """Whether ``ssm_ssd_combined_fwd`` covers this call (bf16 or fp16 tensors of one type on the GPU and a shape
+    ``ssm_ssd_combined_supported`` accepts), with ``heads`` heads of ``hdim`` channels."""
+    if Q <= 0:
         return False
     tensors = [x, B, C] + ([z] if z is not None else [])
     if x.dtype not in (torch.bfloat16, torch.float16) or any(t.dtype != x.dtype for t in tensors) or not x.is_cuda:
         return False
-    dims = _dims(batch, seqlen, heads, hdim, groups, nstate, Q)
+    dims = _dims(int(x.shape[0]), int(x.shape[1]), heads, hdim, int(B.shape[2]), int(B.shape[3]), Q)
     return bool(_lib.load().ssm_ssd_combined_supported(dims, _lib.dtype_enum(x.dtype)))
+
+
+def _fused_ok_wide(x, B, C, z, Q):
+    """:func:`_fused_ok` of a call as it will be made: a head of 64k channels as k heads of 64."""
+    if x.ndim != 4 or B.ndim != 4 or B.shape != C.shape or B.shape[:2] != x.shape[:2]:
+        return False
+    heads, hdim, groups = int(x.shape[2]), int(x.shape[3]), int(B.shape[2])
+    if hdim <= 0 or hdim % 64 or groups <= 0 or heads % groups:
+        return False
+    return _fused_ok(x, B, C, z, Q, heads * (hdim // 64), 64)
 
 
 def _rows_in_place(t):
@@ -393,17 +403,47 @@ def _rows_in_place(t):
 _FUSED_FORMS = {}      # argument structs of one-pass calls seen before (see the forms in ssm_amd/ops/__init__.py)
 
 
+def _fused_args(x, dt, B, b_row, c_row, Q, d_per_p, dt_softplus, dt_limit):
+    """The part of a call's argument struct that its form fixes."""
+    (batch, seqlen, heads, hdim), (groups, nstate) = x.shape, B.shape[2:]
+    dims = _dims(batch, seqlen, heads, hdim, groups, nstate, Q)
+    return _lib.SsdCombinedArgs(
+        workspace_bytes=int(_lib.load().ssm_ssd_combined_workspace_bytes(dims)), dims=dims, io_dtype=_lib.dtype_enum(x.dtype),
+        dt_dtype=_lib.dtype_enum(dt.dtype), dt_softplus=int(bool(dt_softplus)), d_per_p=int(d_per_p),
+        dt_min=float(dt_limit[0]), dt_max=float(dt_limit[1]), b_row_stride=b_row, c_row_stride=c_row)
+
+
+def _ssd_train(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt_limit, return_final_states):
+    """The call with its own backward (``ssm_ssd_combined_bwd``; bf16, heads of 64 channels, at most a skip factor per head),
+    or ``None`` where that does not cover it."""
+    heads, hdim = int(x.shape[2]), int(x.shape[3])
+    if (x.dtype != torch.bfloat16 or hdim != 64 or not _fused_ok(x, B, C, z, Q, heads, hdim)
+            or (D is not None and D.ndim != 1) or not dt.is_floating_point() or dt.dtype == torch.float64):
+        return None
+
+    def dense(t):
+        t = t.contiguous()
+        return t.clone() if t.data_ptr() % 16 else t
+
+    x, dt, z, initial_states = (None if t is None else dense(t) for t in (x, dt, z, initial_states))
+    A, D, dt_bias, initial_states = (None if t is None else dense(t.to(torch.float32)) for t in (A, D, dt_bias, initial_states))
+    (_, b_row), (_, c_row) = _rows_in_place(B.detach()), _rows_in_place(C.detach())
+    B, C = B if b_row else dense(B), C if c_row else dense(C)
+    K.require_gpu(x, dt, A, B, C, D, z, dt_bias, initial_states)
+    call = lambda remember: _native.ssd_combined(_FUSED_FORMS, remember, x, dt, A, B, C, int(Q), D, z, dt_bias, initial_states,
+                                                 dt_softplus, float(dt_limit[0]), float(dt_limit[1]), return_final_states)
+    out = call(None)
+    if out is None:
+        call(bytes(_fused_args(x, dt, B, b_row, c_row, Q, False, dt_softplus, dt_limit)))
+        out = call(None)
+    return out
+
+
 def _ssd_fused(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt_limit, return_final_states, shape,
                seq_idx=None):
     batch, seqlen, heads, hdim, groups, nstate = shape
     si = _seq_idx_i32(seq_idx, batch, seqlen)
-    d_per_p = False
-    if D is not None:
-        _need(tuple(D.shape) in ((heads,), (heads, hdim)), "D must have shape (H,) or (H, P).")
-        d_per_p = D.ndim == 2
-    _need(z is None or z.shape == x.shape, "z must have the shape of x.")
-    _need(tuple(A.shape) == (heads,), "A must have shape (H,).")
-    _need(dt_bias is None or tuple(dt_bias.shape) == (heads,), "dt_bias must have shape (H,).")
+    d_per_p = D is not None and D.ndim == 2
     dev = K.require_gpu(x, dt, A, B, C, D, z, dt_bias, initial_states)
     xc = K.cast_c(x, x.dtype)
     # B and C cut out of wider rows (the two halves of one projection) are read where they are
@@ -414,20 +454,15 @@ def _ssd_fused(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt
     Af, Df, bf, init = K.as_f32_vec(A), K.as_f32_vec(D), K.as_f32_vec(dt_bias), K.as_f32_vec(initial_states)
     if d_per_p and Df.data_ptr() % 16:          # a view into a larger buffer: the kernel reads (H, P) factors as 16-byte vectors
         Df = Df.clone()
-    dims = _dims(batch, seqlen, heads, hdim, groups, nstate, Q)
-    nbytes = int(_lib.load().ssm_ssd_combined_workspace_bytes(dims))
-    work = torch.empty(nbytes + 256, dtype=torch.uint8, device=dev)
+    args = _fused_args(xc, dtc, Bc, b_row, c_row, Q, d_per_p, dt_softplus, dt_limit)
+    work = torch.empty(args.workspace_bytes + 256, dtype=torch.uint8, device=dev)
     off = (-work.data_ptr()) % 256
     y = torch.empty_like(xc)
     final = torch.empty(batch, heads, hdim, nstate, dtype=torch.float32, device=dev) if return_final_states else None
-    args = _lib.SsdCombinedArgs(
-        x=_lib.ptr(xc), dt=_lib.ptr(dtc), A=_lib.ptr(Af), dt_bias=_lib.ptr(bf), Bm=_lib.ptr(Bc), Cm=_lib.ptr(Cc),
-        Dskip=_lib.ptr(Df), z=_lib.ptr(zc), initial_states=_lib.ptr(init), y=_lib.ptr(y),
-        final_states=_lib.ptr(final), workspace=work.data_ptr() + off, workspace_bytes=nbytes, dims=dims,
-        io_dtype=_lib.dtype_enum(xc.dtype), dt_dtype=_lib.dtype_enum(dtc.dtype),
-        dt_softplus=int(bool(dt_softplus)), d_per_p=int(d_per_p),
-        dt_min=float(dt_limit[0]), dt_max=float(dt_limit[1]), seq_idx=_lib.ptr(si), b_row_stride=b_row,
-        c_row_stride=c_row)
+    for name, t in (("x", xc), ("dt", dtc), ("A", Af), ("dt_bias", bf), ("Bm", Bc), ("Cm", Cc), ("Dskip", Df), ("z", zc),
+                    ("initial_states", init), ("y", y), ("final_states", final), ("seq_idx", si)):
+        setattr(args, name, _lib.ptr(t))
+    args.workspace = work.data_ptr() + off
     _lib.call("ssm_ssd_combined_fwd", args, dev)
     if seq_idx is None:
         _native.ssd_combined(_FUSED_FORMS, bytes(args), x, dt, A, B, C, int(Q), D, z, dt_bias, initial_states, dt_softplus,
@@ -488,11 +523,20 @@ def ssd_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initi
                                    dt_limit[0], dt_limit[1], return_final_states)
         if out is not None:
             return out
+    tensors = (x, dt, A, B, C, D, z, dt_bias, initial_states)
+    wants_grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
     seqlen = int(x.shape[1]) if x.ndim == 4 else 0
+    one_call = fused is not False and not force_generic and not return_varlen_states and _fused_ok_wide(x, B, C, z, Q)
+    if wants_grad and one_call and seq_idx is None and states_dtype is None:
+        _check_combined(x, dt, A, B, C, D, z, dt_bias, initial_states)
+        out = _ssd_train(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt_limit, return_final_states)
+        if out is not None:
+            return out
+    one_call = one_call and not wants_grad
     if (x.ndim == 4 and x.dtype in (torch.bfloat16, torch.float16) and Q > 0 and seqlen % Q != 0 and not force_generic
-            and float(dt_limit[0]) <= 0.0 and dt.ndim == 3):
-        # The matrix-core kernels take whole chunks.  Steps of size zero neither decay the state nor add to
-        # it, so a ragged end is filled up with them (zeros for x, B, C, z) and the extra rows of y dropped;
+            and not one_call and float(dt_limit[0]) <= 0.0 and dt.ndim == 3):
+        # The five matrix-core kernels and the passes of the backward take whole chunks.  Steps of size zero neither
+        # decay the state nor add to it, so a ragged end is filled up with them (zeros for x, B, C, z) and the extra rows of y dropped;
         # gradients flow through the padding and the slice.
         pad = (Q - seqlen % Q) % Q
         tpad = lambda t: None if t is None else torch.nn.functional.pad(t, (0, 0) * (t.ndim - 2) + (0, pad))
@@ -516,8 +560,7 @@ def ssd_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initi
         if isinstance(out, tuple):
             return (out[0][:, :seqlen],) + tuple(out[1:])
         return out[:, :seqlen]
-    tensors = (x, dt, A, B, C, D, z, dt_bias, initial_states)
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
+    if wants_grad:
         from ._autograd import SsdCombinedFn, SsdVarlenStatesFn
         _need(not return_varlen_states or cu_seqlens is not None, "return_varlen_states needs cu_seqlens.")
         si = None if seq_idx is None else _seq_idx_i32(seq_idx, int(x.shape[0]), int(x.shape[1]))
@@ -538,16 +581,26 @@ def ssd_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initi
                                  return_varlen_states=return_varlen_states)
 
 
+def _check_combined(x, dt, A, B, C, D, z, dt_bias, initial_states):
+    """Shapes of a combined call; returns its sizes."""
+    batch, seqlen, heads, hdim, groups, nstate = sizes = _ssd_shapes(x, B)
+    _need(C.shape == B.shape, "B and C must have the same shape.")
+    _need(tuple(dt.shape) == (batch, seqlen, heads), "dt must have shape (B, L, H).")
+    _need(initial_states is None or tuple(initial_states.shape) == (batch, heads, hdim, nstate),
+          "initial_states must have shape (B, H, P, N).")
+    _need(D is None or tuple(D.shape) in ((heads,), (heads, hdim)), "D must have shape (H,) or (H, P).")
+    _need(z is None or z.shape == x.shape, "z must have the shape of x.")
+    _need(tuple(A.shape) == (heads,), "A must have shape (H,).")
+    _need(dt_bias is None or tuple(dt_bias.shape) == (heads,), "dt_bias must have shape (H,).")
+    return sizes
+
+
 def _ssd_combined_forward(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initial_states=None,
                           dt_softplus=False, dt_limit=(0.0, float("inf")), return_final_states=False,
                           states_dtype=None, force_generic=False, fused=None, seq_idx=None, cu_seqlens=None,
                           return_varlen_states=False):
     """The forward of :func:`ssd_combined` (same arguments); runs no autograd bookkeeping."""
-    batch, seqlen, heads, hdim, groups, nstate = _ssd_shapes(x, B)
-    _need(C.shape == B.shape, "B and C must have the same shape.")
-    _need(tuple(dt.shape) == (batch, seqlen, heads), "dt must have shape (B, L, H).")
-    _need(initial_states is None or tuple(initial_states.shape) == (batch, heads, hdim, nstate),
-          "initial_states must have shape (B, H, P, N).")
+    batch, seqlen, heads, hdim, groups, nstate = _check_combined(x, dt, A, B, C, D, z, dt_bias, initial_states)
     Q = int(chunk_size)
     _need(not return_varlen_states or cu_seqlens is not None, "return_varlen_states needs cu_seqlens.")
     _need(cu_seqlens is None or batch == 1, "cu_seqlens describes one packed batch row: batch size must be 1.")
@@ -571,9 +624,9 @@ def _ssd_combined_forward(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=No
             outs[i] = outs[i].reshape(outs[i].shape[0], heads, hdim, nstate)
         return outs[0] if len(outs) == 1 else tuple(outs)
     can_fuse = not force_generic and fused is not False and not return_varlen_states and \
-        _fused_ok(x, dt, B, C, z, D, batch, seqlen, heads, hdim, groups, nstate, Q)
+        _fused_ok(x, B, C, z, Q, heads, hdim)
     _need(can_fuse or not fused, "fused=True, but the one-pass kernel needs bf16 or fp16 x/B/C/z, headdim 64, "
-          "chunk in {64,128,256}, nstate in {64,128} and seqlen % chunk == 0.")
+          "chunk in {64,128,256} and nstate in {64,128}.")
     if can_fuse:
         return _ssd_fused(x, dt, A, B, C, Q, D, z, dt_bias, initial_states, dt_softplus, dt_limit,
                           return_final_states, (batch, seqlen, heads, hdim, groups, nstate), seq_idx=seq_idx)
