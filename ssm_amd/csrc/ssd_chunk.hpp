@@ -176,8 +176,8 @@ struct SsdCarryParams {
   const float *dA2;              // (B, H, nc, Q)
   const float *first;            // (B, H, P, N): the state before the first chunk (after the last one), or null
   float *last;                   // (B, H, P, N) or null
-  const float *entering;         // backward: the forward's states, for <G, H> at the chunk boundaries
-  float *anchor;                 // backward: (B, H, nc, dim / 256) partial sums of it
+  const float *entering;         // backward: the forward's states H
+  float *anchor;                 // backward: (B, H, nc, dim / 256) partial sums of exp(cs_Q) <G, H>
   int heads, nchunks, chunk, nstate;
 };
 
@@ -222,12 +222,13 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) 
           *reinterpret_cast<float4 *>(st + c * pitch) = run;
         }
         const float f = exp2_hw(a[k]);
+        const float through = REV ? f * (run.x * hin[k].x + run.y * hin[k].y + run.z * hin[k].z + run.w * hin[k].w) : 0.0f;
         run.x = __builtin_fmaf(run.x, f, v[k].x);
         run.y = __builtin_fmaf(run.y, f, v[k].y);
         run.z = __builtin_fmaf(run.z, f, v[k].z);
         run.w = __builtin_fmaf(run.w, f, v[k].w);
-        if (REV) {                    // run is now the adjoint of the state that entered chunk c
-          const float s = wave_sum(run.x * hin[k].x + run.y * hin[k].y + run.z * hin[k].z + run.w * hin[k].w);
+        if (REV) {                    // through the whole chunk
+          const float s = wave_sum(through);
           if (lane_id() == 0) p.anchor[(bh * p.nchunks + c) * (dim >> 8) + part * 4 + (threadIdx.x >> 6)] = s;
         }
       }
@@ -250,6 +251,7 @@ struct SsdChunkScanParams {
   void *out;                     // y, dz (or null) or dx
   float *sum0, *sum1;            // (B, H, nc, Q): SCAN_DZ <dy, y before skip>;  SCAN_DX <x, u> and <round(dt x), u>
   float *dD;                     // SCAN_DZ: (B, nc, H) sums of dy x, or null
+  float *carried;                // SCAN_DZ: (B, H, nc) sums of <dy, what the state entering the chunk adds to y>
   int len, heads, groups, nchunks, d_per_p;
   int has_first;                 // a state enters the first chunk (leaves the last)
   int states16;                  // states are of the element type (else float32)
@@ -269,12 +271,14 @@ template <typename E, int Q, int N, int MODE, bool HAS_Z>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_chunk_scan_kernel(const SsdChunkScanParams p) {
   using S = Staging<Q>;
   constexpr int NLB = Q >> 5, KS = Q >> 4, KN = N >> 4, NPAIR = NLB / 2, PW = NPAIR >= 4 ? 2 : 1;
-  __shared__ __align__(16) E xT[SSD_P * Q];
-  __shared__ __align__(16) E hs[SSD_P * N];
+  // the carried state is through before the staged rows take its place
+  constexpr int TILE = SSD_P * (Q > N ? Q : N);
+  __shared__ __align__(16) E tile[TILE];
+  E *xT = tile, *hs = tile;
   __shared__ __align__(16) float dAs[Q];
   __shared__ __align__(16) float Ps[Q], Rs[Q];                           // decay from the block before to a step, from a step to the end of its block
   __shared__ __align__(16) float l2s[MODE == SCAN_Y ? Q : 4];            // log2 dt
-  __shared__ float halves[PW == 1 && MODE != SCAN_Y ? 4 * Q : 4];       // row sums of half rows; or one sum per wave
+  __shared__ float halves[PW == 1 && MODE != SCAN_Y ? 4 * Q : 8];       // row sums of half rows; or sums per wave
   const ChunkUnit u(p.len, p.heads, p.groups, p.nchunks, Q, N);
   const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
   const int m = lane & 31, g2 = lane >> 5;
@@ -310,14 +314,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
     ring[t % AHEAD][0] = load_frag_e<E>(f);
     ring[t % AHEAD][1] = load_frag_e<E>(f + SSD_FRAG);
   };
-  V8<E> fc[2][KN];
+  // fragments of the carried product, CAHEAD of its KN steps ahead
+  constexpr int CAHEAD = MODE == SCAN_Y ? (KN < 8 ? KN : 8) : 4;
+  V8<E> fc[2][CAHEAD];
+  const E *cf = reinterpret_cast<const E *>(p.carry) + u.unit * NLB * KN * SSD_FRAG + lane * 8;
+  const auto request_carry = [&](int k) {
+    fc[0][k % CAHEAD] = load_frag_e<E>(cf + (rbs[0] * KN + k) * SSD_FRAG);
+    fc[1][k % CAHEAD] = load_frag_e<E>(cf + (rbs[1] * KN + k) * SSD_FRAG);
+  };
   if (active && carried) {
-    const E *cf = reinterpret_cast<const E *>(p.carry) + u.unit * NLB * KN * SSD_FRAG + lane * 8;
 #pragma unroll
-    for (int k = 0; k < KN; ++k) {
-      fc[0][k] = load_frag_e<E>(cf + (rbs[0] * KN + k) * SSD_FRAG);
-      fc[1][k] = load_frag_e<E>(cf + (rbs[1] * KN + k) * SSD_FRAG);
-    }
+    for (int k = 0; k < CAHEAD; ++k) request_carry(k);
   }
   if (tid < Q) {
     const float cs = p.dA2[u.step0 + tid];
@@ -348,6 +355,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
       }
     }
   }
+  __syncthreads();
+
+  // ---- the carried state
+  float carried_dy = 0.0f;
+  f32x16_t acc[2][PW];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int pt = 0; pt < PW; ++pt) acc[i][pt] = (f32x16_t){0};
+  }
+  if (active && carried) {
+#pragma unroll
+    for (int k = 0; k < KN; ++k) {
+#pragma unroll
+      for (int pt = 0; pt < PW; ++pt) {
+        const V8<E> h = load_frag_e<E>(hs + ((pt0 + pt) * KN + k) * SSD_FRAG + lane * 8);
+        acc[0][pt] = mma(h, fc[0][k % CAHEAD], acc[0][pt]);
+        acc[1][pt] = mma(h, fc[1][k % CAHEAD], acc[1][pt]);
+      }
+      if (k + CAHEAD < KN) request_carry(k + CAHEAD);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float own = dAs[32 * rbs[i] + m];
+      const float f = exp2_hw(MODE == SCAN_DX ? fminf(dAs[Q - 1] - own, 0.0f) : own);
+#pragma unroll
+      for (int pt = 0; pt < PW; ++pt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][pt][r] *= f;
+        if (MODE == SCAN_DZ) {
+          const unsigned row = (unsigned)min(32 * rbs[i] + m, u.rows - 1) * pitch + (32 * (pt0 + pt) + 4 * g2) * 2;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float d[4];
+            load4_e<E>(at_bytes<const E>(reinterpret_cast<const E *>(p.dy) + at, row + 16 * q), d);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) carried_dy = __builtin_fmaf(d[j], acc[i][pt][4 * q + j], carried_dy);
+          }
+        }
+      }
+    }
+    if (MODE == SCAN_DZ) asm volatile("" : "+v"(carried_dy));
+  }
+  if (active) {
+#pragma unroll
+    for (int t = 0; t < AHEAD && t <= NLB; ++t) request(t);
+  }
+  if (carried) __syncthreads();
   V8<E> col[S::CPT];
 #pragma unroll
   for (int i = 0; i < S::CPT; ++i) {
@@ -360,37 +415,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   __syncthreads();
 
   const float head_D = p.Dk && !p.d_per_p ? p.Dk[u.h] : 0.0f;
-  f32x16_t acc[2][PW];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int pt = 0; pt < PW; ++pt) acc[i][pt] = (f32x16_t){0};
-  }
   if (active) {
-#pragma unroll
-    for (int t = 0; t < AHEAD && t <= NLB; ++t) request(t);
-    // ---- the carried state
-    if (carried) {
-#pragma unroll
-      for (int k = 0; k < KN; ++k) {
-#pragma unroll
-        for (int pt = 0; pt < PW; ++pt) {
-          const V8<E> h = load_frag_e<E>(hs + ((pt0 + pt) * KN + k) * SSD_FRAG + lane * 8);
-          acc[0][pt] = mma(h, fc[0][k], acc[0][pt]);
-          acc[1][pt] = mma(h, fc[1][k], acc[1][pt]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float own = dAs[32 * rbs[i] + m];
-        const float f = exp2_hw(MODE == SCAN_DX ? fminf(dAs[Q - 1] - own, 0.0f) : own);
-#pragma unroll
-        for (int pt = 0; pt < PW; ++pt) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][pt][r] *= f;
-        }
-      }
-    }
     // ---- the chunk's own steps
     const auto step = [&](int t, f32x16_t (&to)[PW], auto diagonal) {
       const int rb = row_of(t), ob = other_of(t);
@@ -454,7 +479,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   // work on the block before it.
   constexpr int LPR = 4 * PW, RPP = 64 / LPR, PASSES = 32 / RPP, SMASK = 8 * PW - 1;      // lanes per row, rows per pass
   constexpr bool Z = HAS_Z && MODE != SCAN_DX;
-  float *stg = reinterpret_cast<float *>(xT) + wave * (32 * 32 * PW);
+  float *stg = reinterpret_cast<float *>(tile) + wave * (32 * 32 * PW);
   const int c8 = lane % LPR, ch = 32 * pt0 + 8 * c8;
   const bool skip_rows = MODE == SCAN_Y && p.Dk && p.d_per_p;
   float D8[8];
@@ -578,12 +603,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
       if (MODE == SCAN_DX) p.sum1[u.step0 + tid] = halves[2 * Q + tid] + halves[3 * Q + tid];
     }
   }
-  if (MODE == SCAN_DZ && p.dD) {
-    const float t = wave_sum(dyx);
+  if (MODE == SCAN_DZ) {
+    const float t0 = wave_sum(dyx), t1 = wave_sum(carried_dy);
     __syncthreads();
-    if (lane == 0) halves[wave] = t;
+    if (lane == 0) {
+      halves[wave] = t0;
+      halves[4 + wave] = t1;
+    }
     __syncthreads();
-    if (tid == 0) p.dD[(size_t)(u.b * p.nchunks + u.c) * p.heads + u.h] = (halves[0] + halves[1]) + (halves[2] + halves[3]);
+    if (tid == 0 && p.dD) p.dD[(size_t)(u.b * p.nchunks + u.c) * p.heads + u.h] = (halves[0] + halves[1]) + (halves[2] + halves[3]);
+    if (tid == 0) p.carried[u.step0 / Q] = (halves[4] + halves[5]) + (halves[6] + halves[7]);
   }
 }
 

@@ -1,7 +1,7 @@
 // Backward of the side-by-side SSD (ssd_chunk.hpp) for bfloat16 calls:
 //
 //   states  dy = dout silu(z), rounded and kept; what each chunk adds to the adjoint state
-//   carry   the adjoint state leaving each chunk, last to first, and <G, H> at the chunk boundaries
+//   carry   the adjoint state leaving each chunk, last to first, and what of <G, H> goes through each chunk
 //   scan    y again for dz and its row sums;  u for dx and its row sums
 //   dbc     dB and dC, every head of a group in one workgroup
 //   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one launch adds those up
@@ -214,12 +214,16 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
 // ---------------------------------------------------------------------- dt
 
 // With q_t = a_t <G_t, H_{t-1}>:  ddt_t = A q_t + <x_t, u_t>,  dA = sum dt_t q_t.  Inside a chunk q follows from row sums of the
-// two scans, q_{t+1} = q_t + <dt_t x_t, u_t> - <dy_t, y_t>, starting at each chunk's first step from <G, H> at the boundary
-// (float32 states): what the two scans round differently adds up over one chunk only.
+// two scans, q_{t+1} = q_t + <dt_t x_t, u_t> - <dy_t, y_t>.  At a chunk's first step it is
+//   exp(cs_Q) <G_c, H_c> + sum_l <dy_l, exp(cs_l) C_l.H_c>,
+// the sum taken over the very terms that <dy_l, y_l> holds: what their 16-bit operands are off by leaves q again with each
+// row it came from.  (From <G, H> at the boundary in float32 instead, the difference stayed in q over the whole chunk, long
+// after the state had forgotten it, and was most of the error of dA and of the bias: 1 to 4 % against 0.1 to 0.5 %.)
 struct SsdDtParams {
   const float *s2, *xu, *s1;     // (B, H, nc, Q)
   const float *dtv;
-  const float *anchor;           // (B, H, nc, anchors) partial sums
+  const float *anchor;           // (B, H, nc, anchors) partial sums of exp(cs_Q) <G, H>
+  const float *carried;          // (B, H, nc)
   const void *dt_raw;            // (B, L, H)
   const float *A, *bias;
   void *ddt;                     // (B, L, H)
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
       xu[i] = p.xu[at + i];
       dt[i] = p.dtv[at + i];
     }
-    const float a0 = wave_sum(lane < p.anchors ? p.anchor[unit * p.anchors + lane] : 0.0f);
+    const float a0 = p.carried[unit] + wave_sum(lane < p.anchors ? p.anchor[unit * p.anchors + lane] : 0.0f);
     const float A = p.A[h], bias = p.bias ? p.bias[h] : 0.0f;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -292,7 +296,7 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
 // ---------------------------------------------------------------------- host
 
 struct BwdLayout {
-  size_t dy, states, s2, xu, s1, anchor, dA, dbias, dD, total;
+  size_t dy, states, s2, xu, s1, anchor, carried, dA, dbias, dD, total;
 };
 
 static BwdLayout bwd_layout(const SsdDims &d) {
@@ -306,6 +310,7 @@ static BwdLayout bwd_layout(const SsdDims &d) {
   f.xu = take(units * d.chunk * 4);
   f.s1 = take(units * d.chunk * 4);
   f.anchor = take(units * (SSD_P * d.nstate / 256) * 4);
+  f.carried = take(units * 4);
   f.dA = take(units * 4);
   f.dbias = take(units * 4);
   f.dD = take(units * 4);
@@ -391,7 +396,7 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   SsdChunkScanParams dz{};
   dz.op = f.x; dz.blk = kw + kept.CBblk; dz.carry = kw + kept.Cblk; dz.states = H; dz.dA2 = dA2; dz.dtv = dtv; dz.Dk = f.Dskip;
   dz.x = f.x; dz.dy = ws + lay.dy; dz.z = f.z; dz.dout = a->dout; dz.out = a->dz; dz.sum0 = f32(lay.s2);
-  dz.dD = f.Dskip ? f32(lay.dD) : nullptr; dz.len = d.len; dz.heads = d.heads; dz.groups = d.groups; dz.nchunks = d.nchunks;
+  dz.carried = f32(lay.carried); dz.dD = f.Dskip ? f32(lay.dD) : nullptr; dz.len = d.len; dz.heads = d.heads; dz.groups = d.groups; dz.nchunks = d.nchunks;
   dz.has_first = f.initial_states != nullptr;
   SsdChunkScanParams dx = dz;
   dx.op = ws + lay.dy; dx.blk = kw + kept.CBtblk; dx.carry = kw + kept.Bblk; dx.states = G; dx.z = nullptr; dx.out = a->dx;
@@ -402,7 +407,7 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   bc.dB = reinterpret_cast<elem_t *>(a->dB); bc.dC = reinterpret_cast<elem_t *>(a->dC);
   bc.len = d.len; bc.heads = d.heads; bc.groups = d.groups; bc.nchunks = d.nchunks; bc.units = d.batch * d.nchunks * d.groups;
   SsdDtParams dt{};
-  dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.anchor = f32(lay.anchor); dt.dt_raw = f.dt;
+  dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.anchor = f32(lay.anchor); dt.carried = f32(lay.carried); dt.dt_raw = f.dt;
   dt.A = f.A; dt.bias = f.dt_bias; dt.ddt = a->ddt; dt.dA = f32(lay.dA); dt.dbias = f32(lay.dbias);
   dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.anchors = SSD_P * d.nstate / 256; dt.dt_dtype = f.dt_dtype;
   dt.softplus = f.dt_softplus ? 1 : 0; dt.dt_min = f.dt_min; dt.dt_max = f.dt_max;
