@@ -466,11 +466,10 @@ __host__ __device__ inline int conv_cl_seg_len(int len) {
   return per < 16 ? 16 : per;
 }
 
-// AL: rows (channel vectors) start on 16-byte boundaries and the row length (channel count) is a whole
-// number of vectors; otherwise the same kernel reads and writes element by element.
+// The kernel for rows that do not start on 16-byte boundaries or hold no whole number of 16-byte vectors.
 constexpr int CONV_CL_BWD_BYTES = 4;   // bytes of channels per thread: the walk keeps ~20 values per channel in registers
-template <typename T, bool AL, int TAPS>
-__global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvParams p) {
+template <typename T, int TAPS>
+__global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_walk_kernel(const ConvParams p) {
   constexpr int VEC = CONV_CL_BWD_BYTES / sizeof(T);
   constexpr int HIST = TAPS - 1;
   const int cvecs = (p.chans + VEC - 1) / VEC;
@@ -486,13 +485,10 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
   const int cw = min(VEC, p.chans - c0);          // channels of this vector that exist
   const int K = p.K;
   float wrev[VEC][TAPS], bias[VEC], dwr[VEC][TAPS], db[VEC];
-  if constexpr (AL) load_taps_of<VEC, TAPS>(p.w, p.bias, c0, K, p.wide_taps, wrev, bias);
-  else {
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      bias[i] = (p.bias && i < cw) ? p.bias[c0 + i] : 0.0f;
-      load_taps(p.w, i < cw ? c0 + i : c0, K, wrev[i]);
-    }
+  for (int i = 0; i < VEC; ++i) {
+    bias[i] = (p.bias && i < cw) ? p.bias[c0 + i] : 0.0f;
+    load_taps(p.w, i < cw ? c0 + i : c0, K, wrev[i]);
   }
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
@@ -511,7 +507,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
   for (int j = 0; j < HIST; ++j) {
     const int ts = t_begin - 1 - j;
     float v[VEC];
-    if (ts >= 0) load_run<T, VEC>(xb + (size_t)ts * p.chans, 0, cw, AL, v);
+    if (ts >= 0) load_run<T, VEC>(xb + (size_t)ts * p.chans, 0, cw, false, v);
     else {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) v[i] = 0.0f;
@@ -578,44 +574,19 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
         for (int j = 0; j < TAPS; ++j) acc = __builtin_fmaf(gh[HIST - j][i], wrev[i][j], acc);
         out[i] = acc;
       }
-      store_run<T, VEC>(dxb + (size_t)td * p.chans, 0, cw, AL, out);
+      store_run<T, VEC>(dxb + (size_t)td * p.chans, 0, cw, false, out);
     }
   };
-  if constexpr (AL) {
-    // rows of a group of steps are requested together, unconditionally (row index clamped into the sequence)
-    constexpr int GROUP = 8;
-    for (int tg = t_begin; tg < t_last; tg += GROUP) {
-      Pack<T, VEC> rx[GROUP], rg[GROUP];
+  for (int t = t_begin; t < t_last; ++t) {
+    float cur[VEC], go[VEC];
+    if (t < p.len) {
+      load_run<T, VEC>(xb + (size_t)t * p.chans, 0, cw, false, cur);
+      load_run<T, VEC>(gb + (size_t)t * p.chans, 0, cw, false, go);
+    } else {
 #pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        const size_t at = (size_t)min(tg + j, p.len - 1) * p.chans;
-        rx[j] = *reinterpret_cast<const Pack<T, VEC> *>(xb + at);
-        rg[j] = *reinterpret_cast<const Pack<T, VEC> *>(gb + at);
-      }
-#pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        if (tg + j >= t_last) break;
-        float cur[VEC], go[VEC];
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-          cur[i] = to_f32(rx[j].v[i]);
-          go[i] = to_f32(rg[j].v[i]);
-        }
-        step(tg + j, cur, go);
-      }
+      for (int i = 0; i < VEC; ++i) cur[i] = go[i] = 0.0f;
     }
-  } else {
-    for (int t = t_begin; t < t_last; ++t) {
-      float cur[VEC], go[VEC];
-      if (t < p.len) {
-        load_run<T, VEC>(xb + (size_t)t * p.chans, 0, cw, AL, cur);
-        load_run<T, VEC>(gb + (size_t)t * p.chans, 0, cw, AL, go);
-      } else {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) cur[i] = go[i] = 0.0f;
-      }
-      step(t, cur, go);
-    }
+    step(t, cur, go);
   }
   // partial[(b * nseg + seg)][c][K + 1]: taps in the order of w, then the bias sum
 #pragma unroll
@@ -626,6 +597,106 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
     for (int m = 0; m < TAPS; ++m)
       if (m < K) part[K - 1 - m] = dwr[i][m];
     part[K] = db[i];
+  }
+}
+
+// Dense aligned rows: a workgroup takes 4 bytes of channels per lane (a wave's row access is 256 contiguous bytes) and 64
+// steps, 16 per wave.  A thread requests all the rows its strip needs at once - its 16 and the neighbours that its first
+// pre-activations and its last dx read - so that it meets memory latency once; a walk of 64 steps in groups of eight met it
+// nine times, and that was the time of every shape: 62 us for the 1536 and the 256 channels of a 4 x 2048 mixer together,
+// 31 here.  The sums for dw and dbias meet in LDS, one partial per (batch, segment of at least 64 steps).
+constexpr int CONV_CL_STEPS = 16, CONV_CL_WAVES = CONV_THREADS / WAVE, CONV_CL_TILE = CONV_CL_STEPS * CONV_CL_WAVES;
+
+__host__ __device__ inline int conv_cl_tiles_per_seg(int len) {
+  const int tiles = (len + CONV_CL_TILE - 1) / CONV_CL_TILE;
+  return (tiles + CONV_CL_SEGS - 1) / CONV_CL_SEGS;
+}
+
+template <typename T, int TAPS>
+__global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvParams p) {
+  constexpr int VEC = CONV_CL_BWD_BYTES / sizeof(T), HIST = TAPS - 1, SL = CONV_CL_STEPS, SUMS = TAPS + 1;
+  __shared__ float part[CONV_CL_WAVES][SUMS * VEC][WAVE];
+  const int wave = wave_id_uniform(), lane = lane_id();
+  const int cblocks = (p.chans + WAVE * VEC - 1) / (WAVE * VEC);
+  const int seg_len = conv_cl_tiles_per_seg(p.len) * CONV_CL_TILE, nseg = (p.len + seg_len - 1) / seg_len;
+  const int cb = (int)(blockIdx.x % cblocks), seg = (int)((blockIdx.x / cblocks) % nseg), b = (int)(blockIdx.x / ((unsigned)cblocks * nseg));
+  const int c0 = (cb * WAVE + lane) * VEC;
+  const bool live = c0 < p.chans;
+  const unsigned row = (unsigned)p.chans * sizeof(T), at = (unsigned)(live ? c0 : 0) * sizeof(T);
+  float wrev[VEC][TAPS], bias[VEC], sums[SUMS][VEC];
+  load_taps_of<VEC, TAPS>(p.w, p.bias, live ? c0 : 0, p.K, p.wide_taps, wrev, bias);
+#pragma unroll
+  for (int m = 0; m < SUMS; ++m)
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) sums[m][i] = 0.0f;
+  typedef Pack<T, VEC> vec_t;
+  const size_t base = (size_t)b * p.len * p.chans;
+  const int end = min(p.len, (seg + 1) * seg_len);
+  for (int t0 = seg * seg_len + wave * SL; t0 < end; t0 += CONV_CL_TILE) {
+    // (a row index is clamped into the sequence; what lies outside is made zero below)
+    const T *xt = reinterpret_cast<const T *>(p.x) + base, *gt = reinterpret_cast<const T *>(p.dout) + base;
+    vec_t rx[SL + 2 * HIST], rg[SL + HIST];
+#pragma unroll
+    for (int j = 0; j < SL + 2 * HIST; ++j)
+      rx[j] = *at_bytes<const vec_t>(xt + (size_t)min(max(t0 + j - HIST, 0), p.len - 1) * p.chans, at);
+#pragma unroll
+    for (int j = 0; j < SL + HIST; ++j) rg[j] = *at_bytes<const vec_t>(gt + (size_t)min(t0 + j, p.len - 1) * p.chans, at);
+    T *dxt = reinterpret_cast<T *>(p.y) + base + (size_t)t0 * p.chans;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      // a sliding window: x of this step and the HIST before it, the gradients at the pre-activations of the last TAPS steps
+      float xh[TAPS], gh[TAPS];
+#pragma unroll
+      for (int m = 0; m < TAPS; ++m) gh[m] = 0.0f;
+#pragma unroll
+      for (int m = 0; m < HIST; ++m) xh[m] = t0 + m - HIST >= 0 ? to_f32(rx[m].v[i]) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < SL + HIST; ++j) {
+        const int t = t0 + j;
+        // xh[(j + HIST) % TAPS] is x_t
+        xh[(j + HIST) % TAPS] = to_f32(rx[j + HIST].v[i]);
+        float g = to_f32(rg[j].v[i]);
+        if (p.silu) {
+          float pre = bias[i];
+#pragma unroll
+          for (int m = 0; m < TAPS; ++m) pre = __builtin_fmaf(wrev[i][m], xh[(j + HIST - m + TAPS) % TAPS], pre);
+          g *= silu_grad(pre);
+        }
+        g = t < p.len ? g : 0.0f;
+        gh[j % TAPS] = g;
+        if (j < SL) {                      // own step (past the end: g is zero)
+          sums[TAPS][i] += g;
+#pragma unroll
+          for (int m = 0; m < TAPS; ++m) sums[m][i] = __builtin_fmaf(g, xh[(j + HIST - m + TAPS) % TAPS], sums[m][i]);
+        }
+        if (j >= HIST) {                   // dx of the step HIST back: sum_m g_{t'+m} wrev[m]
+          float acc = 0.0f;
+#pragma unroll
+          for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(gh[(j - HIST + m) % TAPS], wrev[i][m], acc);
+          rx[j - HIST].v[i] = from_f32<T>(acc);        // (the register of a row that is through)
+        }
+      }
+    }
+    if (live) {
+#pragma unroll
+      for (int j = 0; j < SL; ++j)
+        if (t0 + j < end) *at_bytes<vec_t>(dxt, (unsigned)j * row + at) = rx[j];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < SUMS; ++m)
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) part[wave][m * VEC + i][lane] = sums[m][i];
+  __syncthreads();
+  // partial[(b * nseg + seg)][c][K + 1]: taps in the order of w, then the bias sum
+  const int K = p.K;
+  for (int e = wave; e < SUMS * VEC; e += CONV_CL_WAVES) {
+    const int m = e / VEC, c = c0 + e % VEC;
+    float t = 0.0f;
+#pragma unroll
+    for (int w = 0; w < CONV_CL_WAVES; ++w) t += part[w][e][lane];
+    if (live && (m < K || m == TAPS))
+      p.partial[(((size_t)b * nseg + seg) * p.chans + c) * (K + 1) + (m == TAPS ? K : K - 1 - m)] = t;
   }
 }
 
@@ -999,13 +1070,15 @@ static int conv_bwd_typed(const ConvParams &p, int layout, bool vec_ok, float *d
       return SSM_OK;
     }
   } else if (p.K <= CONV_TAPS && channels_last) {
-    const int seg_len = conv_cl_seg_len(p.len);
-    const int nseg = (p.len + seg_len - 1) / seg_len;
     constexpr int VECB = CONV_CL_BWD_BYTES / sizeof(T);
-    const size_t threads = (size_t)p.batch * nseg * ((p.chans + VECB - 1) / VECB);
-    const dim3 grid((unsigned)((threads + CONV_THREADS - 1) / CONV_THREADS));
-    if (vec_ok && p.chans % VEC == 0) CONV_LAUNCH(conv_bwd_cl_kernel, CONV_T_AL(true), grid, dim3(CONV_THREADS));
-    else CONV_LAUNCH(conv_bwd_cl_kernel, CONV_T_AL(false), grid, dim3(CONV_THREADS));
+    // (a strip's rows are addressed by 32-bit offsets)
+    const bool dense = vec_ok && p.chans % VEC == 0 && (size_t)p.chans * sizeof(T) * CONV_CL_STEPS < ((size_t)1 << 31);
+    const int seg_len = dense ? conv_cl_tiles_per_seg(p.len) * CONV_CL_TILE : conv_cl_seg_len(p.len);
+    const int nseg = (p.len + seg_len - 1) / seg_len;
+    const size_t vecs = (p.chans + VECB - 1) / VECB, walkers = (size_t)p.batch * nseg * vecs;
+    const size_t blocks = dense ? (size_t)p.batch * nseg * ((vecs + WAVE - 1) / WAVE) : (walkers + CONV_THREADS - 1) / CONV_THREADS;
+    if (dense) CONV_LAUNCH(conv_bwd_cl_kernel, T, dim3((unsigned)blocks), dim3(CONV_THREADS));
+    else CONV_LAUNCH(conv_bwd_cl_walk_kernel, T, dim3((unsigned)blocks), dim3(CONV_THREADS));
     fold_count = p.batch * nseg;
   } else {
     const int rows = p.batch * p.chans;
