@@ -25,7 +25,9 @@ static void forward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
                              hipStream_t s) {
   const dim3 units((unsigned)(d.batch * d.nchunks * d.heads)), block(256);
   hipLaunchKernelGGL((ssd_states_kernel<E, Q, N, false>), units, block, 0, s, st);
-  hipLaunchKernelGGL((ssd_carry_kernel<E, false>), dim3((unsigned)(d.batch * d.heads) * (SSD_P * N / 1024)), block, 0, s, ca);
+  const unsigned carriers = (unsigned)(d.batch * d.heads) * (SSD_P * N / 1024);
+  if (ca.turned) hipLaunchKernelGGL((ssd_carry_kernel<E, false, true>), dim3(carriers / 4), block, 0, s, ca);
+  else hipLaunchKernelGGL((ssd_carry_kernel<E, false, false>), dim3(carriers), block, 0, s, ca);
   if (sc.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, SCAN_Y, true>), units, block, 0, s, sc);
   else hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, SCAN_Y, false>), units, block, 0, s, sc);
 }
@@ -33,17 +35,17 @@ static void forward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
 int ssd_chunk_forward(const ssm_ssd_combined_args &a, const SsdDims &d, const SsdWorkLayout &lay, hipStream_t s) {
   SSM_REQUIRE((size_t)d.batch * d.nchunks * d.heads < ((size_t)1 << 26), SSM_ERR_TOO_LARGE, "ssm_ssd_combined_fwd: too many workgroups");
   unsigned char *ws = reinterpret_cast<unsigned char *>(a.workspace);
-  float *states = reinterpret_cast<float *>(ws + lay.states);
+  float *added = reinterpret_cast<float *>(ws + lay.added);
   const float *dA2 = reinterpret_cast<const float *>(ws + lay.dA2), *dtv = reinterpret_cast<const float *>(ws + lay.dt_out);
   SsdStatesParams st{};
-  st.x = a.x; st.frag = ws + lay.Btblk; st.dA2 = dA2; st.dtv = dtv; st.states = states;
+  st.x = a.x; st.frag = ws + lay.Btblk; st.dA2 = dA2; st.dtv = dtv; st.states = added;
   st.len = d.len; st.heads = d.heads; st.groups = d.groups; st.nchunks = d.nchunks;
   SsdCarryParams ca{};
-  if (!a.keep_for_backward) ca.states16 = ws + lay.states16;
-  ca.states = states; ca.dA2 = dA2; ca.first = a.initial_states; ca.last = a.final_states;
+  if (a.keep_for_backward) ca.turned = ws + lay.turned;
+  ca.added = added; ca.states = ws + lay.states; ca.dA2 = dA2; ca.first = a.initial_states; ca.last = a.final_states;
   ca.heads = d.heads; ca.nchunks = d.nchunks; ca.chunk = d.chunk; ca.nstate = d.nstate;
   SsdChunkScanParams sc{};
-  sc.op = a.x; sc.blk = ws + lay.CBblk; sc.carry = ws + lay.Cblk; sc.states = ca.states16 ? ca.states16 : states; sc.states16 = ca.states16 != nullptr; sc.dA2 = dA2; sc.dtv = dtv;
+  sc.op = a.x; sc.blk = ws + lay.CBblk; sc.carry = ws + lay.Cblk; sc.states = ws + lay.states; sc.dA2 = dA2; sc.dtv = dtv;
   sc.Dk = a.Dskip; sc.x = a.x; sc.z = a.z; sc.out = a.y; sc.len = d.len; sc.heads = d.heads; sc.groups = d.groups;
   sc.nchunks = d.nchunks; sc.d_per_p = a.d_per_p ? 1 : 0; sc.has_first = a.initial_states != nullptr;
 #define SSM_CHUNK_FORWARD(E, QQ, NN) \

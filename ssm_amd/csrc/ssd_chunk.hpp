@@ -1,14 +1,15 @@
 // The SSD of 16-bit calls with the chunks side by side, forward and backward: one workgroup per (batch, chunk, head).
 //
 //   states: what a chunk adds to the state,             S_c = sum_s exp(cs_Q - cs_s) dt_s x_s (x) B_s
-//   pass:   the state entering each chunk,              H_{c+1} = exp(cs_Q) H_c + S_c        (in place)
+//   carry:  the state entering each chunk,              H_{c+1} = exp(cs_Q) H_c + S_c
 //   scan:   y_l = exp(cs_l) C_l.H_c + sum_{s<=l} (C_l.B_s) exp(cs_l - cs_s) dt_s x_s
 //
 // and, for the gradients, the same three with the adjoint in the place of x: dS_c = sum_l exp(cs_l) dy_l (x) C_l, passed
 // from the last chunk to the first, and u_s = exp(cs_Q - cs_s) B_s.G_c + sum_{l>=s} (C_l.B_s) exp(cs_l - cs_s) dy_l
 // with dx_s = dt_s u_s + D dy_s.
 //
-// States travel in float32 and in fragment order: [p / 32][n / 16][lane][8], lane = p % 32 + 32 (n % 16 / 8), the order
+// What chunks add travels in float32, the states entering them in the element type (they are operands only; the recurrence
+// is in float32), both in fragment order: [p / 32][n / 16][lane][8], lane = p % 32 + 32 (n % 16 / 8), the order
 // in which a wave holds 32 x 16 of them as a matrix operand.  A wave's accumulators of S^T are written as whole KiB that
 // way, the pass is element by element in any order, and the scan reads operands without a transposition.
 //
@@ -168,73 +169,96 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   }
 }
 
-// ---------------------------------------------------------------------- pass
+// ---------------------------------------------------------------------- carry
 
 struct SsdCarryParams {
-  float *states;                 // (B, nc, H, dim) in fragment order, rewritten
-  void *states16;                // where the entering states go instead, in the element type, or null
+  const float *added;            // (B, nc, H, dim) in fragment order: what each chunk adds
+  void *states;                  // (B, nc, H, dim): the state entering each chunk, element type, fragment order
+  void *turned;                  // the same as rows of 64 channels, (B, nc, H, N, 64): what ssd_dbc_kernel reads (TURN)
   const float *dA2;              // (B, H, nc, Q)
   const float *first;            // (B, H, P, N): the state before the first chunk (after the last one), or null
   float *last;                   // (B, H, P, N) or null
-  const float *entering;         // backward: the forward's states H
-  float *anchor;                 // backward: (B, H, nc, dim / 256) partial sums of exp(cs_Q) <G, H>
+  const void *entering;          // REV: the forward's states H
+  float *through;                // REV: (B, H, nc, dim / 1024) partial sums of exp(cs_Q) <G, H>
   int heads, nchunks, chunk, nstate;
 };
 
-// Four elements per thread over all chunks, eight chunks' reads in flight; 64 N / 1024 workgroups per (batch, head).
-template <typename E, bool REV>
+// A thread carries 4 states of one channel over all chunks, or with TURN of four neighbouring channels, whose 4 x 4 it
+// also stores with channels innermost.  The reads of several chunks are in flight: with no more than one workgroup on
+// most CUs, it is latency that this launch consists of.
+template <typename E, bool REV, bool TURN>
 __global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) {
-  const int N = p.nstate, dim = SSD_P * N, per = dim >> 10;
+  constexpr int C = TURN ? 4 : 1, AHEAD = TURN ? 4 : 8;
+  const int N = p.nstate, dim = SSD_P * N, per = dim / (1024 * C), kn = N >> 4;
   const unsigned vid = blockIdx.x;
-  const int part = (int)(vid % per);
+  const int part = (int)(vid % per), tid = part * 256 + (int)threadIdx.x;
   const size_t bh = vid / per;
   const int h = (int)(bh % p.heads);
   const size_t b = bh / p.heads;
-  const int e = (part * 256 + (int)threadIdx.x) * 4;
-  const int frag = e >> 9, fl = (e >> 3) & 63, kn = N >> 4;
-  const size_t user = (bh * SSD_P + 32 * (frag / kn) + (fl & 31)) * N + 16 * (frag % kn) + 8 * (fl >> 5) + (e & 7);
-  const size_t pitch = (size_t)p.heads * dim;
-  const size_t at = (b * p.nchunks * p.heads + h) * dim + e;
-  float *st = p.states + at;
-  const float *ent = p.entering + at;
+  // element 4 (tid % 2) of lane fl of fragment frag; with TURN of the lanes fl .. fl + 3
+  const int frag = TURN ? tid >> 5 : tid >> 7, j = (TURN ? tid >> 3 & 1 : tid & 1) * 4;
+  const int fl = TURN ? (tid >> 4 & 1) * 32 + (tid & 7) * 4 : tid >> 1 & 63;
+  const int e = frag * SSD_FRAG + fl * 8 + j, ch = 32 * (frag / kn) + (fl & 31), n = 16 * (frag % kn) + 8 * (fl >> 5) + j;
+  const size_t user = (bh * SSD_P + ch) * N + n;
+  const size_t pitch = (size_t)p.heads * dim, at = (b * p.nchunks * p.heads + h) * dim;
   const float *end = p.dA2 + bh * p.nchunks * p.chunk + p.chunk - 1;
-  float4 run = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (p.first) run = make_float4(p.first[user], p.first[user + 1], p.first[user + 2], p.first[user + 3]);
-  constexpr int AHEAD = REV ? 4 : 8;
+  float run[C][4];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) run[i][k] = p.first ? p.first[user + (size_t)i * N + k] : 0.0f;
+  }
   for (int i0 = 0; i0 < p.nchunks; i0 += AHEAD) {
-    float4 v[AHEAD], hin[AHEAD];
-    float a[AHEAD];
+    float4 v[AHEAD][C];
+    float hin[AHEAD][C][4], a[AHEAD];
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) {
       const int i = min(i0 + k, p.nchunks - 1), c = REV ? p.nchunks - 1 - i : i;
-      v[k] = *reinterpret_cast<const float4 *>(st + c * pitch);
-      if (REV) hin[k] = *reinterpret_cast<const float4 *>(ent + c * pitch);
+      const size_t o = at + c * pitch + e;
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        v[k][q] = *reinterpret_cast<const float4 *>(p.added + o + q * 8);
+        if (REV) load4_e<E>(reinterpret_cast<const E *>(p.entering) + o + q * 8, hin[k][q]);
+      }
       a[k] = end[(size_t)c * p.chunk];
     }
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) {
       const int i = i0 + k, c = REV ? p.nchunks - 1 - i : i;
       if (i < p.nchunks) {
-        if (!REV && p.states16) {
-          const float r4[4] = {run.x, run.y, run.z, run.w};
-          store4_e<E>(reinterpret_cast<E *>(p.states16) + at + c * pitch, r4);
-        } else {
-          *reinterpret_cast<float4 *>(st + c * pitch) = run;
-        }
+        const size_t o = at + c * pitch;
         const float f = exp2_hw(a[k]);
-        const float through = REV ? f * (run.x * hin[k].x + run.y * hin[k].y + run.z * hin[k].z + run.w * hin[k].w) : 0.0f;
-        run.x = __builtin_fmaf(run.x, f, v[k].x);
-        run.y = __builtin_fmaf(run.y, f, v[k].y);
-        run.z = __builtin_fmaf(run.z, f, v[k].z);
-        run.w = __builtin_fmaf(run.w, f, v[k].w);
-        if (REV) {                    // through the whole chunk
-          const float s = wave_sum(through);
-          if (lane_id() == 0) p.anchor[(bh * p.nchunks + c) * (dim >> 8) + part * 4 + (threadIdx.x >> 6)] = s;
+        float through = 0.0f;
+#pragma unroll
+        for (int q = 0; q < C; ++q) store4_e<E>(reinterpret_cast<E *>(p.states) + o + e + q * 8, run[q]);
+        if constexpr (TURN) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const float t[4] = {run[0][s], run[1][s], run[2][s], run[3][s]};
+            store4_e<E>(reinterpret_cast<E *>(p.turned) + o + (n + s) * SSD_P + ch, t);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+          const float add[4] = {v[k][q].x, v[k][q].y, v[k][q].z, v[k][q].w};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            if (REV) through = __builtin_fmaf(run[q][s], hin[k][q][s], through);
+            run[q][s] = __builtin_fmaf(run[q][s], f, add[s]);
+          }
+        }
+        if (REV) {
+          through = wave_sum(through) * f;
+          if (lane_id() == 0) p.through[(bh * p.nchunks + c) * (dim >> 10) + part * 4 + (threadIdx.x >> 6)] = through;
         }
       }
     }
   }
-  if (p.last) *reinterpret_cast<float4 *>(p.last + user) = run;
+  if (p.last) {
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+      *reinterpret_cast<float4 *>(p.last + user + (size_t)i * N) = make_float4(run[i][0], run[i][1], run[i][2], run[i][3]);
+  }
 }
 
 // ---------------------------------------------------------------------- scan
@@ -245,7 +269,7 @@ struct SsdChunkScanParams {
   const void *op;                // rows of the in-chunk product: x, or dy for SCAN_DX
   const void *blk;               // fragments of C.B (transposed for SCAN_DX)
   const void *carry;             // fragments of C (of B for SCAN_DX)
-  const void *states;            // H entering the chunks (G leaving them for SCAN_DX), fragment order
+  const void *states;            // H entering the chunks (G leaving them for SCAN_DX), element type, fragment order
   const float *dA2, *dtv, *Dk;
   const void *x, *dy, *z, *dout; // (B, L, H, 64) rows the last step reads
   void *out;                     // y, dz (or null) or dx
@@ -254,7 +278,6 @@ struct SsdChunkScanParams {
   float *carried;                // SCAN_DZ: (B, H, nc) sums of <dy, what the state entering the chunk adds to y>
   int len, heads, groups, nchunks, d_per_p;
   int has_first;                 // a state enters the first chunk (leaves the last)
-  int states16;                  // states are of the element type (else float32)
 };
 
 // Row blocks of 32 steps: a wave takes blocks NLB - 1 - i and i (NLB + 1 of the blocks on and below the diagonal
@@ -340,20 +363,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
     Rs[tid] = r;
   }
   if (carried) {
-    if (MODE == SCAN_Y && p.states16) {
-      const E *st = reinterpret_cast<const E *>(p.states) + u.state;
+    const E *st = reinterpret_cast<const E *>(p.states) + u.state;
 #pragma unroll
-      for (int i = 0; i < SSD_P * N / 2048; ++i)
-        *reinterpret_cast<V8<E> *>(hs + (i * 256 + tid) * 8) = load_frag_e<E>(st + (i * 256 + tid) * 8);
-    } else {
-      const float *st = reinterpret_cast<const float *>(p.states) + u.state;
-#pragma unroll
-      for (int i = 0; i < SSD_P * N / 2048; ++i) {
-        float v[8];
-        load8(st + (i * 256 + tid) * 8, v);
-        *reinterpret_cast<V8<E> *>(hs + (i * 256 + tid) * 8) = pack8_e<E>(v);
-      }
-    }
+    for (int i = 0; i < SSD_P * N / 2048; ++i)
+      *reinterpret_cast<V8<E> *>(hs + (i * 256 + tid) * 8) = load_frag_e<E>(st + (i * 256 + tid) * 8);
   }
   __syncthreads();
 
@@ -485,7 +498,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   float D8[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) D8[j] = MODE != SCAN_Y ? head_D : skip_rows ? p.Dk[u.h * SSD_P + ch + j] : 0.0f;
-  constexpr int AT_ONCE = MODE == SCAN_Y ? PASSES : PASSES / 2, GROUPS = PASSES / AT_ONCE;      // what the registers hold
+  constexpr int AT_ONCE = MODE == SCAN_Y ? PASSES : MODE == SCAN_DZ ? (PASSES + 3) / 4 : PASSES / 2, GROUPS = PASSES / AT_ONCE;      // what the registers hold
   V8<E> rx[AT_ONCE], rdy[AT_ONCE], rz[AT_ONCE], rgo[AT_ONCE];
   float rdt[AT_ONCE];
   const auto request_rows = [&](int rb, int first) {

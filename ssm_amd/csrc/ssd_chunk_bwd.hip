@@ -20,7 +20,7 @@ typedef __bf16 elem_t;
 // and across chunk boundaries dC_l += sum_h exp(cs_l) dy_l.H_c,   dB_s += sum_h dt_s exp(cs_Q - cs_s) x_s.G_c.
 struct SsdDbcParams {
   const elem_t *x, *dy;          // (B, L, H, 64)
-  const float *H, *G;            // states entering / adjoint states leaving the chunks, fragment order
+  const elem_t *H, *G;           // states entering / adjoint states leaving the chunks, (B, nc, H, N, 64)
   const float *dA2, *dtv;
   const void *Btblk, *Ctblk;
   elem_t *dB, *dC;               // (B, L, G, N)
@@ -36,7 +36,7 @@ struct SsdDbcParams {
 template <int Q, int N>
 __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
   typedef V8<elem_t> v8;
-  constexpr int KS = Q >> 4, KN = N >> 4, NT = N >> 5, NR = Q >> 6, QMASK = Staging<Q>::QMASK;
+  constexpr int KS = Q >> 4, NT = N >> 5, NR = Q >> 6, QMASK = Staging<Q>::QMASK;
   constexpr int TILE = 64 * 64, BUF = (1 + NR) * TILE + N * 64;        // own rows, met rows, state
   extern __shared__ __align__(16) unsigned char smem[];
   elem_t *bufs = reinterpret_cast<elem_t *>(smem);                     // [2][BUF]
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
   const size_t pitch = (size_t)p.heads * SSD_P;
   const size_t row0 = ((size_t)b * p.len + (size_t)c * Q) * pitch + h0 * SSD_P;
   const elem_t *own_src = (for_b ? p.x : p.dy) + row0, *met_src = (for_b ? p.dy : p.x) + row0;
-  const float *st_src = (for_b ? p.G : p.H) + ((size_t)bc * p.heads + h0) * (SSD_P * N);
+  const elem_t *st_src = (for_b ? p.G : p.H) + ((size_t)bc * p.heads + h0) * (SSD_P * N);
   const size_t step0 = (((size_t)b * p.heads + h0) * p.nchunks + c) * Q, step_pitch = (size_t)p.nchunks * Q;
   const int met0 = for_b ? 64 * r : 0;                                 // first met row
 
@@ -66,23 +66,17 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
   unsigned met_at[NR];
 #pragma unroll
   for (int k = 0; k < NR; ++k) met_at[k] = (unsigned)min(met0 + 64 * k + lr, rows - 1) * (unsigned)pitch + piece * 8;
-  // 4 channels x 4 states of the state per thread: in fragment order states run along memory, so the transposition to
-  // [n][p] is one of 4 x 4 registers
-  const bool st_mine = tid < N * 4;
-  const int st_pq = tid & 7, st_j = (tid >> 3 & 1) * 4, st_up = tid >> 4 & 1, st_frag = tid >> 5;
   v8 own_r, met_r[NR];
-  float4 st_r[4];
+  v8 st_r[N / 64];
   float cs_r = 0.0f, dt_r = 0.0f, cs_b = 0.0f;
   const auto fetch = [&](int h) {
     own_r = *reinterpret_cast<const v8 *>(own_src + h * SSD_P + own_at);
 #pragma unroll
     for (int k = 0; k < NR; ++k)
       if (k < meets) met_r[k] = *reinterpret_cast<const v8 *>(met_src + h * SSD_P + met_at[k]);
-    if (st_mine) {
-      const float *s = st_src + (size_t)h * (SSD_P * N) + st_frag * SSD_FRAG + (32 * st_up + 4 * st_pq) * 8 + st_j;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) st_r[i] = *reinterpret_cast<const float4 *>(s + i * 8);
-    }
+    for (int k = 0; k < N / 64; ++k)
+      st_r[k] = *reinterpret_cast<const v8 *>(st_src + (size_t)h * (SSD_P * N) + (64 * k + lr) * 64 + piece * 8);
     if (tid < Q) {
       cs_r = p.dA2[step0 + h * step_pitch + tid];
       dt_r = p.dtv[step0 + h * step_pitch + tid];
@@ -95,13 +89,9 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
 #pragma unroll
     for (int k = 0; k < NR; ++k)
       if (k < meets) *reinterpret_cast<v8 *>(met + (64 * k + lr) * 64 + ((piece ^ (lr & 7)) << 3)) = met_r[k];
-    if (st_mine) {
-      const int n0 = 16 * (st_frag % KN) + 8 * st_up + st_j, p0 = 32 * (st_frag / KN) + 4 * st_pq;
-      const float t[4][4] = {{st_r[0].x, st_r[1].x, st_r[2].x, st_r[3].x}, {st_r[0].y, st_r[1].y, st_r[2].y, st_r[3].y},
-                             {st_r[0].z, st_r[1].z, st_r[2].z, st_r[3].z}, {st_r[0].w, st_r[1].w, st_r[2].w, st_r[3].w}};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) store4_e<elem_t>(st + (n0 + j) * 64 + (((p0 >> 3) ^ ((n0 + j) & 7)) << 3) + (p0 & 7), t[j]);
-    }
+    for (int k = 0; k < N / 64; ++k)
+      *reinterpret_cast<v8 *>(st + (64 * k + lr) * 64 + ((piece ^ (lr & 7)) << 3)) = st_r[k];
     if (tid < Q) {
       // decays from the block of 32 before to a step, and (times dt) from a step to the end of its block
       float *t = steps + 4 * at * Q + tid;
@@ -222,13 +212,13 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
 struct SsdDtParams {
   const float *s2, *xu, *s1;     // (B, H, nc, Q)
   const float *dtv;
-  const float *anchor;           // (B, H, nc, anchors) partial sums of exp(cs_Q) <G, H>
+  const float *through;          // (B, H, nc, parts) partial sums of exp(cs_Q) <G, H>
   const float *carried;          // (B, H, nc)
   const void *dt_raw;            // (B, L, H)
   const float *A, *bias;
   void *ddt;                     // (B, L, H)
   float *dA, *dbias;             // (B, nc, H) partial sums
-  int len, heads, nchunks, anchors, dt_dtype, softplus;
+  int len, heads, nchunks, parts, dt_dtype, softplus;
   float dt_min, dt_max;
 };
 
@@ -260,7 +250,7 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
       xu[i] = p.xu[at + i];
       dt[i] = p.dtv[at + i];
     }
-    const float a0 = p.carried[unit] + wave_sum(lane < p.anchors ? p.anchor[unit * p.anchors + lane] : 0.0f);
+    const float a0 = p.carried[unit] + wave_sum(lane < p.parts ? p.through[unit * p.parts + lane] : 0.0f);
     const float A = p.A[h], bias = p.bias ? p.bias[h] : 0.0f;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -296,7 +286,7 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
 // ---------------------------------------------------------------------- host
 
 struct BwdLayout {
-  size_t dy, states, s2, xu, s1, anchor, carried, dA, dbias, dD, total;
+  size_t dy, added, states, turned, s2, xu, s1, through, carried, dA, dbias, dD, total;
 };
 
 static BwdLayout bwd_layout(const SsdDims &d) {
@@ -305,11 +295,13 @@ static BwdLayout bwd_layout(const SsdDims &d) {
   size_t at = 0;
   const auto take = [&](size_t bytes) { const size_t v = at; at += ssd_align_up(bytes); return v; };
   f.dy = take((size_t)d.batch * d.len * d.heads * SSD_P * 2);
-  f.states = take(units * SSD_P * d.nstate * 4);
+  f.added = take(units * SSD_P * d.nstate * 4);
+  f.states = take(units * SSD_P * d.nstate * 2);
+  f.turned = take(units * SSD_P * d.nstate * 2);
   f.s2 = take(units * d.chunk * 4);
   f.xu = take(units * d.chunk * 4);
   f.s1 = take(units * d.chunk * 4);
-  f.anchor = take(units * (SSD_P * d.nstate / 256) * 4);
+  f.through = take(units * (SSD_P * d.nstate / 1024) * 4);
   f.carried = take(units * 4);
   f.dA = take(units * 4);
   f.dbias = take(units * 4);
@@ -343,7 +335,7 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
     return SSM_ERR_LAUNCH;
   }
   hipLaunchKernelGGL((ssd_states_kernel<elem_t, Q, N, true>), units, block, 0, s, st);
-  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true>), dim3((unsigned)(d.batch * d.heads) * (SSD_P * N / 1024)), block, 0, s, ca);
+  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(d.batch * d.heads) * (SSD_P * N / 4096)), block, 0, s, ca);
   if (dz.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, true>), units, block, 0, s, dz);
   else hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, false>), units, block, 0, s, dz);
   hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DX, false>), units, block, 0, s, dx);
@@ -383,33 +375,31 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   const unsigned char *kw = reinterpret_cast<const unsigned char *>(f.workspace);
   unsigned char *ws = reinterpret_cast<unsigned char *>(a->workspace);
   const float *dA2 = reinterpret_cast<const float *>(kw + kept.dA2), *dtv = reinterpret_cast<const float *>(kw + kept.dt_out);
-  const float *H = reinterpret_cast<const float *>(kw + kept.states);
-  float *G = reinterpret_cast<float *>(ws + lay.states);
   const auto f32 = [&](size_t off) { return reinterpret_cast<float *>(ws + off); };
 
   SsdStatesParams st{};
-  st.x = a->dout; st.z = f.z; st.dy = ws + lay.dy; st.frag = kw + kept.Ctblk; st.dA2 = dA2; st.dtv = dtv; st.states = G;
+  st.x = a->dout; st.z = f.z; st.dy = ws + lay.dy; st.frag = kw + kept.Ctblk; st.dA2 = dA2; st.dtv = dtv; st.states = f32(lay.added);
   st.len = d.len; st.heads = d.heads; st.groups = d.groups; st.nchunks = d.nchunks;
   SsdCarryParams ca{};
-  ca.states = G; ca.dA2 = dA2; ca.first = a->dfinal; ca.last = a->dinitial_states; ca.entering = H; ca.anchor = f32(lay.anchor);
+  ca.added = f32(lay.added); ca.states = ws + lay.states; ca.turned = ws + lay.turned; ca.dA2 = dA2; ca.first = a->dfinal; ca.last = a->dinitial_states; ca.entering = kw + kept.states; ca.through = f32(lay.through);
   ca.heads = d.heads; ca.nchunks = d.nchunks; ca.chunk = d.chunk; ca.nstate = d.nstate;
   SsdChunkScanParams dz{};
-  dz.op = f.x; dz.blk = kw + kept.CBblk; dz.carry = kw + kept.Cblk; dz.states = H; dz.dA2 = dA2; dz.dtv = dtv; dz.Dk = f.Dskip;
+  dz.op = f.x; dz.blk = kw + kept.CBblk; dz.carry = kw + kept.Cblk; dz.states = kw + kept.states; dz.dA2 = dA2; dz.dtv = dtv; dz.Dk = f.Dskip;
   dz.x = f.x; dz.dy = ws + lay.dy; dz.z = f.z; dz.dout = a->dout; dz.out = a->dz; dz.sum0 = f32(lay.s2);
   dz.carried = f32(lay.carried); dz.dD = f.Dskip ? f32(lay.dD) : nullptr; dz.len = d.len; dz.heads = d.heads; dz.groups = d.groups; dz.nchunks = d.nchunks;
   dz.has_first = f.initial_states != nullptr;
   SsdChunkScanParams dx = dz;
-  dx.op = ws + lay.dy; dx.blk = kw + kept.CBtblk; dx.carry = kw + kept.Bblk; dx.states = G; dx.z = nullptr; dx.out = a->dx;
+  dx.op = ws + lay.dy; dx.blk = kw + kept.CBtblk; dx.carry = kw + kept.Bblk; dx.states = ws + lay.states; dx.z = nullptr; dx.out = a->dx;
   dx.sum0 = f32(lay.xu); dx.sum1 = f32(lay.s1); dx.dD = nullptr; dx.has_first = a->dfinal != nullptr;
   SsdDbcParams bc{};
-  bc.x = reinterpret_cast<const elem_t *>(f.x); bc.dy = reinterpret_cast<const elem_t *>(ws + lay.dy); bc.H = H; bc.G = G;
+  bc.x = reinterpret_cast<const elem_t *>(f.x); bc.dy = reinterpret_cast<const elem_t *>(ws + lay.dy); bc.H = reinterpret_cast<const elem_t *>(kw + kept.turned); bc.G = reinterpret_cast<const elem_t *>(ws + lay.turned);
   bc.dA2 = dA2; bc.dtv = dtv; bc.Btblk = kw + kept.Btblk; bc.Ctblk = kw + kept.Ctblk;
   bc.dB = reinterpret_cast<elem_t *>(a->dB); bc.dC = reinterpret_cast<elem_t *>(a->dC);
   bc.len = d.len; bc.heads = d.heads; bc.groups = d.groups; bc.nchunks = d.nchunks; bc.units = d.batch * d.nchunks * d.groups;
   SsdDtParams dt{};
-  dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.anchor = f32(lay.anchor); dt.carried = f32(lay.carried); dt.dt_raw = f.dt;
+  dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.through = f32(lay.through); dt.carried = f32(lay.carried); dt.dt_raw = f.dt;
   dt.A = f.A; dt.bias = f.dt_bias; dt.ddt = a->ddt; dt.dA = f32(lay.dA); dt.dbias = f32(lay.dbias);
-  dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.anchors = SSD_P * d.nstate / 256; dt.dt_dtype = f.dt_dtype;
+  dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.parts = SSD_P * d.nstate / 1024; dt.dt_dtype = f.dt_dtype;
   dt.softplus = f.dt_softplus ? 1 : 0; dt.dt_min = f.dt_min; dt.dt_max = f.dt_max;
 
   int rc = SSM_OK;

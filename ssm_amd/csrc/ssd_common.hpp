@@ -95,8 +95,8 @@ struct SsdWorkLayout {
   size_t dt_out, dA2;                   // (B, H, nc, Q) float32: the step, and its running sum times A log2(e)
   size_t Cblk, Btblk, CBblk;            // operand fragments (prep in ssd_fused.hip)
   size_t Bblk, Ctblk, CBtblk;           // ... that only the backward reads; empty without `keep`
-  size_t states, states16;              // (B, nc, H, 64 N) in fragment order, float32 and 16 bits (without `keep`); empty on
-                                        // the one-pass route
+  size_t states, turned;                // (B, nc, H, 64 N) entering the chunks, and (with `keep`) with channels innermost
+  size_t added;                         // (B, nc, H, 64 N) float32: what each chunk adds; these three empty on the one-pass route
   size_t total;
 };
 
@@ -120,11 +120,10 @@ inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep) {
   f.Bblk = at; at += keep ? bc : 0;
   f.Ctblk = at; at += keep ? bc : 0;
   f.CBtblk = at; at += keep ? cb : 0;
-  f.states = at;
-  const size_t states = (size_t)d.batch * d.nchunks * d.heads * SSD_P * d.nstate;
-  if (keep || ssd_side_by_side(d)) at += ssd_align_up(states * sizeof(float));
-  f.states16 = at;
-  if (!keep && ssd_side_by_side(d)) at += ssd_align_up(states * 2);
+  const size_t states = keep || ssd_side_by_side(d) ? (size_t)d.batch * d.nchunks * d.heads * SSD_P * d.nstate : 0;
+  f.states = at; at += ssd_align_up(states * 2);
+  f.turned = at; at += keep ? ssd_align_up(states * 2) : 0;
+  f.added = at; at += ssd_align_up(states * sizeof(float));
   f.total = at;
   return f;
 }
