@@ -178,7 +178,8 @@ __global__ __launch_bounds__(WAVE *DO_WAVES) void dscan_onepass_kernel(const Dsc
   __shared__ float2 right[2][WAVE];
   const int wave = wave_id_uniform(), lane = lane_id();
   const int HP = p.heads * p.proj;
-  const unsigned ch = ((unsigned)blockIdx.x * WAVE + lane) * VEC;
+  // (channels past the last one of a last workgroup that is not full stand for it: the same values to the same places)
+  const unsigned ch = min(((unsigned)blockIdx.x * WAVE + lane) * VEC, (unsigned)HP - VEC);
   const int b = blockIdx.y;
   const int h = (int)ch / p.proj;
   const int L = p.len;
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(WAVE *DO_WAVES) void dscan_onepass_kernel(const Dsc
 // Cut a one-pass walk into segments when few workgroups share it; p.fold has room for p.nseg maps per channel.
 template <typename io_t, int VEC>
 static dim3 onepass_grid(DscanParams &p, bool params, hipStream_t s) {
-  const unsigned blocks = (unsigned)((size_t)p.heads * p.proj / (WAVE * VEC));
+  const unsigned blocks = (unsigned)(((size_t)p.heads * p.proj + WAVE * VEC - 1) / (WAVE * VEC));
   const int rounds = (p.len + DO_ROUND - 1) / DO_ROUND;
   // 1.7 us a round: 29 us for the 16 rounds of 2048 steps by 32 workgroups
   p.seg_rounds = dscan_rounds_per_segment((size_t)blocks * p.batch, rounds, 1.7);
@@ -405,7 +406,7 @@ extern "C" size_t ssm_dscan_fwd_workspace_bytes(int batch, int seqlen, int heads
   return (size_t)batch * nseg * heads * proj * 2 * sizeof(float);
 }
 
-// One pass: float32 dt, a gate of X's shape and type or none, channels in whole waves, vectors aligned, and either
+// One pass: float32 dt, a gate of X's shape and type or none, a head's channels in whole vectors, vectors aligned, and either
 // per-token B and C of X's type with per-head A and D (*params = false), or B and C one value per channel -- (H,P)
 // or (B,H,P), any type -- with A and D per head or per channel (*params = true).
 static bool dscan_fwd_takes_one_pass(const ssm_dscan_fwd_args *a, bool *params = nullptr) {
@@ -421,7 +422,7 @@ static bool dscan_fwd_takes_one_pass(const ssm_dscan_fwd_args *a, bool *params =
                         aligned_to(a->Bproj, dtype_size(a->bc_dtype)) && aligned_to(a->Cproj, dtype_size(a->bc_dtype));
   if (params) *params = constant;
   return (streamed || constant) && a->dt_dtype == SSM_F32 && (!a->z || (a->z_dtype == a->x_dtype && a->z_per_p)) &&
-         HP % (WAVE * vec) == 0 && a->proj % vec == 0 && (long long)a->seqlen * HP < (1ll << 30) &&
+         a->proj % vec == 0 && (long long)a->seqlen * HP < (1ll << 30) &&
          aligned_to(a->X, bytes) && aligned_to(a->Y, bytes) && (!a->z || aligned_to(a->z, bytes)) && a->batch < 65536;
 }
 

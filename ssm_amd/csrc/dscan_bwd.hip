@@ -367,7 +367,7 @@ extern "C" int ssm_dscan_bwd(const ssm_dscan_bwd_args *a, void *hip_stream) {
                         aligned_to(a->dB, 4) && aligned_to(a->dC, 4);
   const bool onepass = SSM_RESERVED(a) == 0 && a->batch < 65536 && (streamed || constant) && a->dt_dtype == SSM_F32 &&
                        (!a->z || (a->z_dtype == a->x_dtype && a->z_per_p)) && (lph == 16 || lph == 32 || lph == 64) &&
-                       HP % (WAVE * vec) == 0 && (size_t)L * HP < ((size_t)1 << 30) && aligned_to(a->X, vbytes) &&
+                       (size_t)L * HP < ((size_t)1 << 30) && aligned_to(a->X, vbytes) &&
                        aligned_to(a->grad_y, vbytes) && aligned_to(a->dX, vbytes) &&
                        (!a->z || (aligned_to(a->z, vbytes) && aligned_to(a->dz, gbytes)));
   if (onepass) {
@@ -376,7 +376,7 @@ extern "C" int ssm_dscan_bwd(const ssm_dscan_bwd_args *a, void *hip_stream) {
     // per-channel sums of a batch row, (B, HP) each; those that are the caller's gradient already go there
     float *sums = ws + (size_t)Bn * rounds * HP;
     // 2.3 us a round: 75 us for the 32 rounds of 2048 steps by 32 workgroups
-    p.seg_rounds = dscan_rounds_per_segment((size_t)Bn * (HP / (WAVE * vec)), rounds, 2.3);
+    p.seg_rounds = dscan_rounds_per_segment((size_t)Bn * ((HP + WAVE * vec - 1) / (WAVE * vec)), rounds, 2.3);
     const int segs = (rounds + p.seg_rounds - 1) / p.seg_rounds, copies = segs * Bn;
     const size_t each = (size_t)copies * HP;
     SSM_REQUIRE((size_t)Bn * rounds * HP + 4 * each + 2 * bhp * std::max(segs, nseg) + 1 <= a->workspace_bytes / 4, SSM_ERR_WORKSPACE, "ssm_dscan_bwd: workspace too small");

@@ -42,7 +42,9 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
   __shared__ float2 left[2][WAVE];               // the adjoint leaving the round, from wave 0 to everyone's next round
   const int wave = wave_id_uniform(), lane = lane_id();
   const int HP = p.heads * p.proj;
-  const unsigned ch = ((unsigned)blockIdx.x * WAVE + lane) * VEC;
+  // (channels past the last one of a last workgroup that is not full stand for it: the same values to the same places)
+  const unsigned ch = min(((unsigned)blockIdx.x * WAVE + lane) * VEC, (unsigned)HP - VEC);
+  const bool head_lane = (lane & (LPH - 1)) == LPH - 1 && ((unsigned)blockIdx.x * WAVE + lane) * VEC < (unsigned)HP;
   const int b = blockIdx.y;
   const int h = (int)ch / p.proj;
   const int L = p.len;
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(WAVE *DBO_WAVES) void dscan_bwd_onepass_kernel(cons
         if (!PARAMS) *at_bytes<Pack<g_t, VEC>>(dB, at * (unsigned)sizeof(g_t)) = ob;
         if (!PARAMS) *at_bytes<Pack<g_t, VEC>>(dC, at * (unsigned)sizeof(g_t)) = oc;
         if (HAS_Z) *at_bytes<Pack<g_t, VEC>>(dZ, at * (unsigned)sizeof(g_t)) = oz;
-        if ((lane & (LPH - 1)) == LPH - 1) *at_bytes<float>(DDT, ((unsigned)t * (unsigned)p.heads + (unsigned)h) * 4u) = head;
+        if (head_lane) *at_bytes<float>(DDT, ((unsigned)t * (unsigned)p.heads + (unsigned)h) * 4u) = head;
       }
     }
   };
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(WAVE) void dscan_bwd_head_sums_kernel(const float *
 template <typename io_t, typename g_t, int VEC, bool HAS_Z, bool PARAMS>
 static void launch_dbo_lph(const DscanBwdParams &p, int lph, hipStream_t s) {
   const int rounds = (p.len + DBO_ROUND - 1) / DBO_ROUND;
-  const dim3 grid((unsigned)((size_t)p.heads * p.proj / (WAVE * VEC)), (unsigned)p.batch, (unsigned)((rounds + p.seg_rounds - 1) / p.seg_rounds));
+  const dim3 grid((unsigned)(((size_t)p.heads * p.proj + WAVE * VEC - 1) / (WAVE * VEC)), (unsigned)p.batch, (unsigned)((rounds + p.seg_rounds - 1) / p.seg_rounds));
   const dim3 block(WAVE * DBO_WAVES);
   if (lph == 16) hipLaunchKernelGGL((dscan_bwd_onepass_kernel<io_t, g_t, VEC, HAS_Z, 16, PARAMS>), grid, block, 0, s, p);
   else if (lph == 32) hipLaunchKernelGGL((dscan_bwd_onepass_kernel<io_t, g_t, VEC, HAS_Z, 32, PARAMS>), grid, block, 0, s, p);

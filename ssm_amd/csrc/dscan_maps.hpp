@@ -32,7 +32,8 @@ __global__ __launch_bounds__(WAVE *DM_WAVES) void dscan_maps_kernel(const DscanM
   __shared__ float2 folds[DM_WAVES][VEC][WAVE];
   const int wave = wave_id_uniform(), lane = lane_id();
   const int HP = p.heads * p.width;
-  const unsigned ch = ((unsigned)blockIdx.x * WAVE + lane) * VEC;
+  // (channels past the last one of a last workgroup that is not full stand for it: the same values to the same places)
+  const unsigned ch = min(((unsigned)blockIdx.x * WAVE + lane) * VEC, (unsigned)HP - VEC);
   const int b = blockIdx.y, seg = blockIdx.z;
   const int h = (int)ch / p.width;
   const int L = p.len;
@@ -123,7 +124,7 @@ __device__ __forceinline__ float dscan_compose(const float2 *m, int count, ptrdi
 
 template <typename io_t, int VEC, bool BWD, bool PARAMS>
 static void launch_dscan_maps(const DscanMapParams &p, hipStream_t s) {
-  const dim3 grid((unsigned)((size_t)p.heads * p.width / (WAVE * VEC)), (unsigned)p.batch, (unsigned)p.nseg), block(WAVE * DM_WAVES);
+  const dim3 grid((unsigned)(((size_t)p.heads * p.width + WAVE * VEC - 1) / (WAVE * VEC)), (unsigned)p.batch, (unsigned)p.nseg), block(WAVE * DM_WAVES);
   if constexpr (BWD) {
     if (p.z) {
       hipLaunchKernelGGL((dscan_maps_kernel<io_t, VEC, true, true, PARAMS>), grid, block, 0, s, p);

@@ -448,3 +448,13 @@ def test_time_in_segments(dtype, kind, b, length, z_mode, init, lens):
         scale = float(want[k].abs().max()) + 1e-6
         tol = dict(rtol=3e-2, atol=3e-2 * scale) if dtype != torch.float32 else dict(rtol=2e-4, atol=2e-5 * max(scale, 1.0))
         torch.testing.assert_close(got[k].float().cpu().double(), want[k], msg=lambda m, n=k: f"grad {n}: {m}", **tol)
+
+
+@pytest.mark.parametrize("dtype,hp", [(torch.bfloat16, (1, 64)), (torch.float16, (5, 64)), (torch.bfloat16, (3, 32)), (torch.float32, (5, 32))],
+                         ids=lambda v: str(v).replace("torch.", "").replace(" ", ""))
+def test_last_workgroup_of_the_one_pass_kernels_not_full(dtype, hp):
+    """Channels that fill no whole number of waves: the lanes past the last channel stand for it."""
+    for length in (63, 700):
+        test_one_pass_call_shape(dtype, hp, length, 4, "vec", True, False)
+        test_one_pass_backward_call_shape(dtype, hp, length, 4, "vec", True, False)
+        test_one_pass_with_parameter_projections(dtype, hp, (2, 3), length, True, 4, "mat", True, True)
