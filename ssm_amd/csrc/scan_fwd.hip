@@ -99,7 +99,9 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   const bool const_ok = !bvary && !cvary && a->nstate <= FAST_N;
   p.ragged = const_ok ? !(p.vec_ok && a->seqlen % 8 == 0 && a->seqlen < (1 << 29)) : !whole_rows;
   p.split = scan_fwd_splits(rows_total, a->seqlen, !const_ok, a->io_dtype != SSM_F32, p.ragged);
-  if (tune == 0 && fast_ok && a->seqlen > 256) {
+  // Rows of at most 256 steps fill half a chunk there; the general kernel, which has chunks of 256, keeps them (6720 rows of
+  // 256 bf16 20 us against 33) unless every channel has its own projections: 58 against 26 us, of 195 119 against 63.
+  if (tune == 0 && fast_ok && (a->seqlen > 256 || (per_b == 1 && per_c == 1))) {
     // The variant whose workgroups (48, 24 or 8 channels of one group) still give every CU its share:
     // two rows per wave with 16-step runs and two slabs where 256 such workgroups exist, else 8-step runs at six waves
     // per SIMD, else the smallest workgroup.

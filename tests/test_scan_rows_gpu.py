@@ -81,3 +81,9 @@ def test_what_lies_past_a_row_never_enters_it(dtype):
         t[k][1] = float("inf")
     y2, h2 = call()
     assert torch.equal(y2[0], y[0]) and torch.equal(h2[0], h[0])
+
+
+@pytest.mark.parametrize("length,dtype", [(1, torch.float32), (15, torch.bfloat16), (64, torch.float32), (195, torch.bfloat16),
+                                          (256, torch.float16)])
+def test_short_rows_with_projections_per_channel(length, dtype):
+    test_rows_of_any_length("own", length, 16, dtype, True)
