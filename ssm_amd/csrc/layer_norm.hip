@@ -549,47 +549,53 @@ __global__ __launch_bounds__(LN_THREADS) void norm_bwd_long_kernel(const NormPar
   }
 }
 
-// dw[c] = sum_w partial[w][0][c], db[c] = sum_w partial[w][1][c].  A workgroup takes 16 columns; its 256
-// threads are 16 columns x 16 slices of the partials, summed in a fixed order (slice by slice, then over slices).
-constexpr int FOLD_COLS = 16, FOLD_SLICES = LN_THREADS / FOLD_COLS;
-__global__ __launch_bounds__(LN_THREADS) void norm_bwd_fold_kernel(const float *partial, float *dw, float *db,
-                                                                    int nparts, int hidden) {
-  __shared__ float sw_s[FOLD_SLICES][FOLD_COLS], sb_s[FOLD_SLICES][FOLD_COLS];
+// dw[c] = sum_w partial[w][0][c], db[c] = sum_w partial[w][1][c].  A workgroup takes 16 columns; its 1024
+// threads are 16 columns x 64 slices of the partials, summed in a fixed order (slice by slice, then over slices).
+// Bound by latency: few workgroups (hidden / 16) that each walk up to 1024 partials, so the walk is cut to at most
+// two rounds of reads, and the second half of a partial is left alone where there is no bias.
+// 1024 partials of 768 columns 6.5 -> 4.8 us, of 1536 6.8 -> 4.3 us (before: 256 threads, 16 slices, both halves read).
+constexpr int FOLD_COLS = 16, FOLD_THREADS = 1024, FOLD_SLICES = FOLD_THREADS / FOLD_COLS;
+
+template <bool BIAS>
+__global__ __launch_bounds__(FOLD_THREADS) void norm_bwd_fold_kernel(const float *partial, float *dw, float *db,
+                                                                     int nparts, int hidden) {
+  constexpr int SUMS = BIAS ? 2 : 1;
+  __shared__ float part[SUMS][FOLD_SLICES][FOLD_COLS];
   const int cl = threadIdx.x % FOLD_COLS, sl = threadIdx.x / FOLD_COLS;
   const int c = blockIdx.x * FOLD_COLS + cl;
-  float sw = 0.0f, sb = 0.0f;
+  float sum[SUMS] = {};
   if (c < hidden) {
     // eight partials at a time: their reads are in flight together, the additions keep their order
     int w = sl;
     for (; w + 7 * FOLD_SLICES < nparts; w += 8 * FOLD_SLICES) {
-      float a[8], b[8];
+      float v[SUMS][8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        a[k] = partial[(size_t)(w + k * FOLD_SLICES) * 2 * hidden + c];
-        b[k] = partial[(size_t)(w + k * FOLD_SLICES) * 2 * hidden + hidden + c];
-      }
+      for (int k = 0; k < 8; ++k)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        sw += a[k];
-        sb += b[k];
-      }
+        for (int q = 0; q < SUMS; ++q) v[q][k] = partial[((size_t)(w + k * FOLD_SLICES) * 2 + q) * hidden + c];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int q = 0; q < SUMS; ++q) sum[q] += v[q][k];
     }
-    for (; w < nparts; w += FOLD_SLICES) {
-      sw += partial[(size_t)w * 2 * hidden + c];
-      sb += partial[(size_t)w * 2 * hidden + hidden + c];
-    }
+    for (; w < nparts; w += FOLD_SLICES)
+#pragma unroll
+      for (int q = 0; q < SUMS; ++q) sum[q] += partial[((size_t)w * 2 + q) * hidden + c];
   }
-  sw_s[sl][cl] = sw;
-  sb_s[sl][cl] = sb;
+#pragma unroll
+  for (int q = 0; q < SUMS; ++q) part[q][sl][cl] = sum[q];
   __syncthreads();
-  if (sl == 0 && c < hidden) {
-    float a = 0.0f, b = 0.0f;
-    for (int j = 0; j < FOLD_SLICES; ++j) {
-      a += sw_s[j][cl];
-      b += sb_s[j][cl];
+  // the first wave: four lanes a column, a quarter of the slices each
+  if (threadIdx.x < WAVE) {
+#pragma unroll
+    for (int q = 0; q < SUMS; ++q) {
+      float t = 0.0f;
+#pragma unroll
+      for (int j = 0; j < FOLD_SLICES / 4; ++j) t += part[q][4 * j + sl][cl];
+      t += __shfl_xor(t, FOLD_COLS, WAVE);
+      t += __shfl_xor(t, 2 * FOLD_COLS, WAVE);
+      if (sl == 0 && c < hidden) (q ? db : dw)[c] = t;
     }
-    dw[c] = a;
-    if (db) db[c] = b;
   }
 }
 
@@ -735,8 +741,9 @@ static int norm_bwd_launch(const ssm_norm_bwd_args *a, float *partial, void *hip
   else hipLaunchKernelGGL(norm_bwd_long_kernel, dim3(grid), dim3(LN_THREADS), 0, s, p);
   SSM_CHECK_LAUNCH("ssm_norm_bwd");
   const int nparts = a->hidden <= 8192 ? grid : grid * LN_WAVES;   // the long-row kernel writes one per wave
-  hipLaunchKernelGGL(norm_bwd_fold_kernel, dim3((a->hidden + FOLD_COLS - 1) / FOLD_COLS), dim3(LN_THREADS), 0, s,
-                     p.partial, a->dweight, a->dbias, nparts, a->hidden);
+  const dim3 fold((a->hidden + FOLD_COLS - 1) / FOLD_COLS);
+  if (a->dbias) hipLaunchKernelGGL(norm_bwd_fold_kernel<true>, fold, dim3(FOLD_THREADS), 0, s, p.partial, a->dweight, a->dbias, nparts, a->hidden);
+  else hipLaunchKernelGGL(norm_bwd_fold_kernel<false>, fold, dim3(FOLD_THREADS), 0, s, p.partial, a->dweight, nullptr, nparts, a->hidden);
   SSM_CHECK_LAUNCH("ssm_norm_bwd(fold)");
   return SSM_OK;
 }
