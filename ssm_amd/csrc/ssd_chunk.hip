@@ -3,29 +3,27 @@
 
 namespace ssm {
 
-// Chunks one after the other (the state never leaves the chip; 32 channels per workgroup, so few heads leave CUs idle) or
-// side by side (states through memory, twice x)?  Both times in us, heads counted over the batch.  A round of the walk,
-// up to 768 workgroups, takes per chunk a fixed time and more for each workgroup beyond the first hundred or so; the
-// workgroups of the other way (one per chunk and head) a fixed share of the chip each, on top of two more launches.
-// Fitted to both routes at 660 sizes (24 to 1536 heads, 2 to 32 chunks, each chunk length and state size, inputs that
-// change from call to call); the route taken is the faster one or within 5 % of it at all but 16, on average 0.3 % off.
-//   heads, 16 chunks (256 steps, 128 states):   24         160         240         320         400         640
-//   walk / side by side:                     139 / 48   196 / 154   189 / 223   273 / 284   372 / 353   458 / 547
-//   128 steps, 128 states:                   101 / 31   122 / 106   122 / 152   151 / 201   226 / 248   260 / 390
-//   64 steps, 64 states:                      75 / 21    91 / 58     92 / 79    102 / 103   164 / 123   182 / 197
-// Two chunks never gain (24 heads: 22 / 26).
+// One walk over the sequence (the state never leaves the chip; a workgroup per head, or per two, so few heads leave CUs idle)
+// or the chunks side by side (states through memory, twice x)?  Both times in us, heads counted over the batch.  The walk
+// takes a time per block of 32 steps that grows with the heads that share memory, and above 256 heads, two to a workgroup,
+// faster; 512 fill the chip.  The workgroups of the other way (one per chunk and head) take a fixed share of the chip each.
+// Fitted to both routes at 210 sizes (24 to 640 heads, 256 to 8192 steps, each chunk length and state size):
+//   heads, 4096 steps, 128 states:       24         64         96         128        160        256        320        400
+//   walk / side by side, chunks of 256: 109 / 41   110 / 67   114 / 97   118 / 125  120 / 152  146 / 244  192 / 289  211 / 356
+// Up to two chunks the walk is always the faster one (24 heads, 512 steps: 21 / 24).
 bool ssd_side_by_side(const SsdDims &d) {
-  struct Fit {
-    double chunk_us, group_us, unit_us;
+  // the walk's offsets from the start of a head have 32 bits, some blocks past its end included
+  if ((size_t)(d.len + 512) * d.heads * SSD_P * 2 >= (size_t)1 << 31) return true;
+  static const double unit_us[3][2] = {{0.0167, 0.0264}, {0.0262, 0.0355}, {0.0421, 0.0536}};   // chunks of 64, 128, 256 steps; 64, 128 states
+  const bool large = d.nstate > 64;
+  const auto block_us = [&](int64_t n) {
+    if (n == 0) return 0.0;
+    if (n <= 256) return large ? 0.77 + 0.0012 * (double)n : 0.62 + 0.0010 * (double)n;
+    return large ? 0.68 + 0.0024 * (double)n : 0.55 + 0.0020 * (double)n;
   };
-  static const Fit fits[3][2] = {{{3.8, 0.0032, 0.0167}, {4.5, 0.0026, 0.0264}},       // chunks of 64 steps: 64, 128 states
-                                 {{4.1, 0.0060, 0.0262}, {5.2, 0.0059, 0.0355}},
-                                 {{6.5, 0.0124, 0.0421}, {7.0, 0.0139, 0.0536}}};
-  const Fit &f = fits[d.chunk > 128 ? 2 : d.chunk > 64][d.nstate > 64];
-  const int64_t groups = 2 * (int64_t)d.batch * d.heads;
-  const auto chunk = [&](int64_t n) { return n ? f.chunk_us + f.group_us * (double)(n > 100 ? n - 100 : 0) : 0.0; };
-  const double walk = 9.0 + d.nchunks * ((double)(groups / 768) * chunk(768) + chunk(groups % 768));
-  return d.nchunks > 2 && walk > 16.0 + f.unit_us * 0.5 * (double)groups * d.nchunks;
+  const int64_t heads = (int64_t)d.batch * d.heads;
+  const double walk = 7.5 + ssd_walk_turns(ssd_walk_blocks(d.len)) * ((double)(heads / 512) * block_us(512) + block_us(heads % 512));
+  return d.nchunks > 2 && walk > 16.0 + unit_us[d.chunk > 128 ? 2 : d.chunk > 64][large] * (double)heads * d.nchunks;
 }
 
 template <typename E, int Q, int N>

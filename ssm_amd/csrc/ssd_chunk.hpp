@@ -19,7 +19,7 @@
 // products take about 1 us of a CU per workgroup, a decay factor per element of C.B another.
 //
 // A growing head (A > 0): decays between steps of a chunk are bounded by 1, the factors on carried states are not (as in
-// ssd_fused.hip); the gradients are those of that function.
+// ssd_walk.hip); the gradients are those of that function.
 #pragma once
 #include "ssd_common.hpp"
 

@@ -89,14 +89,20 @@ struct SsdScanParams {
 // 64, 128 or 256 steps, 64 or 128 states; nc = ceil(L / Q) chunks, the last one of any length.
 constexpr int SSD_P = 64;
 constexpr int SSD_FRAG = 512;           // elements per operand fragment: 64 lanes x 8
+constexpr int SSD_WALK_BLOCK = 32;      // steps that the one-pass route takes at a time
+
+inline int ssd_walk_blocks(int len) { return (len + SSD_WALK_BLOCK - 1) / SSD_WALK_BLOCK; }
+__host__ __device__ inline int ssd_walk_turns(int nblocks) { return (nblocks + 3) & ~3; }
 
 // What one preparation launch leaves for them: byte offsets into the workspace of a call.
 struct SsdWorkLayout {
   size_t dt_out, dA2;                   // (B, H, nc, Q) float32: the step, and its running sum times A log2(e)
+  size_t steps, ends;                   // in their place on the one-pass route: the same of its blocks (SsdWalkParams)
   size_t Cblk, Btblk, CBblk;            // operand fragments (prep in ssd_fused.hip)
   size_t Bblk, Ctblk, CBtblk;           // ... that only the backward reads; empty without `keep`
   size_t states, states_low;            // (B, nc, H, 64 N) entering the chunks, and (with `keep`) the rest of their float32
   size_t added;                         // (B, nc, H, 64 N) float32: what each chunk adds; these three empty on the one-pass route
+  size_t grown;                         // one-pass route: SsdWalkParams::grown
   size_t total;                         // (without `added` where `keep`: it lies in the call's scratch, ssd_added_bytes)
 };
 
@@ -111,13 +117,17 @@ inline size_t ssd_added_bytes(const SsdDims &d) {
 
 inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep, bool side_by_side) {
   SsdWorkLayout f;
-  const size_t steps = (size_t)d.nchunks * d.chunk;
+  const bool walk = !keep && !side_by_side;
+  const size_t steps = walk ? (size_t)ssd_walk_blocks(d.len) * SSD_WALK_BLOCK : (size_t)d.nchunks * d.chunk;
   const size_t per_step = ssd_align_up((size_t)d.batch * d.heads * steps * sizeof(float));
   const size_t bc = ssd_align_up((size_t)d.batch * steps * d.groups * d.nstate * 2);
-  const size_t cb = ssd_align_up((size_t)d.batch * steps * d.groups * d.chunk * 2);
+  const size_t cb = ssd_align_up((size_t)d.batch * steps * d.groups * (walk ? SSD_WALK_BLOCK : d.chunk) * 2);
   size_t at = 0;
-  f.dt_out = at; at += per_step;
-  f.dA2 = at; at += per_step;
+  const size_t turns = walk ? (size_t)d.batch * d.heads * ssd_walk_turns(ssd_walk_blocks(d.len)) : 0;
+  f.steps = at; at += turns * 2 * SSD_WALK_BLOCK * sizeof(float);
+  f.ends = at; at += ssd_align_up(turns * sizeof(float));
+  f.dt_out = at; at += walk ? 0 : per_step;
+  f.dA2 = at; at += walk ? 0 : per_step;
   f.Cblk = at; at += bc;
   f.Btblk = at; at += bc;
   f.CBblk = at; at += cb;
@@ -128,6 +138,7 @@ inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep, bool side_by_s
   f.states = at; at += ssd_align_up(states * 2);
   f.states_low = at; at += keep ? ssd_align_up(states * 2) : 0;
   f.added = at; at += states && !keep ? ssd_added_bytes(d) : 0;
+  f.grown = at; at += walk ? ssd_align_up((size_t)d.batch * d.heads * SSD_P * d.nstate * sizeof(float)) : 0;
   f.total = at;
   return f;
 }

@@ -1,0 +1,648 @@
+// Mamba-2 SSD forward of 16-bit calls as one pass over the sequence: a workgroup owns the 64 channels of one (batch, head),
+// or of two neighbouring heads, and walks their steps in blocks of 32 with the running state in matrix-core accumulators,
+// so that x, z and y are all that travels between HBM and the chip.  Per block, with cs the running sum of dt A since the
+// block's first step:
+//
+//   y_l = exp(cs_l) C_l.S + sum_{s<=l} (C_l.B_s) exp(cs_l - cs_s) dt_s x_s  (+ D x_l, gate)
+//   S  <- exp(cs_31) S + sum_s exp(cs_31 - cs_s) dt_s x_s (x) B_s
+//
+// Four waves multiply: wave (pt, nh) holds the states of 32 channels and half of the state dimension, S^T as tiles [n][p].
+// A tile is the left operand of C.S as it stands - lane = channel, registers = states - once the fragments of C hold the
+// states in the order of the accumulators' rows (prep_pack_role), so the state is rounded to 16 bits in registers and never
+// goes through LDS.  Four more waves per head do what is element by element: they weight x for the block after the one being
+// multiplied, add what the two halves of the state gave to the block before it, gate that and store it as whole rows.
+// One barrier per block.  x is read from LDS with transposing reads (ds_read_b64_tr_b16); 16-byte pieces of a row are
+// XOR-swizzled by the row.
+//
+// Decays.  Where a block decays by no more than 2^-160, they factor at its middle, r = cs_31 / 2: with x~_s = exp(r - cs_s)
+// dt_s x_s and the state held at the middle of its block, S~ = exp(r) S,
+//   y_l = exp(cs_l - r) (C_l.S~ + sum_{s<=l} (C_l.B_s) x~_s),      S~ <- exp(..) (S~ + sum_s x~_s (x) B_s),
+// no element of C.B needs a factor, and C.B goes from memory to the matrix cores as it is.  What rounding to bfloat16 takes
+// from x~ joins the products inside the block as an operand of its own, so that these lose nothing beyond the rounding of
+// C.B.  Heads with a block beyond that range, growing heads (A > 0) and float16 calls (whose exponents hold no such x~)
+// form exp(cs_l - cs_s) dt_s (C_l.B_s) per element instead, x weighted towards the block's end for the state.
+//
+// What bounds it: a CU takes in x and z at no more than about 20 (one head's rows of 128 bytes) to 27 (two heads') bytes per
+// ns whatever is in flight - a kernel that only streams them this way takes 88 us for 256 heads x 4096 steps on 256 CUs, 148
+// us for 320 heads, as a CU with two workgroups takes twice as long, and 114 us for these as 160 pairs - and the vector ALU
+// issues behind the matrix cores, not beside them.  So: a head per workgroup while every workgroup has a CU of its own,
+// two neighbours beyond; and the fragments of B and C into LDS once per workgroup.  4 x 4096 steps, 128 states, 64 / 80 heads:
+// 137 / 195 us a call.  Before (half a head per workgroup, 64-byte rows, chunks of 256 steps): 200 / 279.
+// With fragments loaded by each wave 135 / 200.
+//
+// A growing head: decays between steps of one of the call's chunks are bounded by 1, the factors on the state entering the
+// chunk are not (the published kernels evaluate exp(min(x, 0)) and exp(x) there).  Such a head keeps that state apart from
+// what the chunk has added so far; the sign of A is read per head, on the device.
+#include "ssd_common.hpp"
+#include "ssd_walk.hpp"
+
+namespace ssm {
+
+constexpr int WK = SSD_WALK_BLOCK, WK_TILE = WK * SSD_P * 2;             // steps of a block; bytes of its 64 channels
+constexpr float WALK_RANGE = 160.0f;                                     // powers of two: far from the end of float32 on either side
+constexpr int WALK_SINGLES = 256;                                        // heads that get a workgroup each: the CUs
+
+// Byte offsets into LDS.  Twice each: 32 rows of x per head, weighted (X ..), and what their rounding lost, or x itself
+// (NH tiles on); part sums [head][nh][pt][step][32 channels] of float32.
+template <int NH> struct WalkLds {
+  static constexpr int X = 2 * NH * WK_TILE, PARTS = NH * 4 * 4096, PART = 2 * X, END = PART + 2 * PARTS;
+};
+// Heads that factor: fragments of three blocks.
+template <int NH, int N> struct FactoredLds {
+  static constexpr int KN = N / 16, C = WalkLds<NH>::END, B = C + 3 * KN * 1024, CB = B + 3 * KN * 1024, BYTES = CB + 3 * 2048;
+};
+// Others, one at a time: decayed C.B of two blocks; cs, log2 dt - cs and log2 dt (cs less half of the block's) of four.
+struct PlainLds {
+  static constexpr int W = WalkLds<1>::END, STEPS = W + 2 * 2048, STEP_BYTES = 3 * WK * 4, BYTES = STEPS + 4 * STEP_BYTES;
+};
+static_assert(FactoredLds<2, 128>::BYTES <= 160 * 1024 && 2 * PlainLds::BYTES <= 160 * 1024, "one pair per CU, or two plain heads");
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
+typedef const __attribute__((address_space(4))) float *scalar_floats;
+
+// The barrier without the wait for accesses to memory that a fence would bring.
+__device__ __forceinline__ void walk_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// 16 bytes per lane from memory to LDS, lane i to byte `at` + 16 i.  Written out, because the compiler would make every
+// later read of LDS wait for it; the waits are factored_products'.
+__device__ __forceinline__ void to_lds16(const void *base, unsigned off, unsigned at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base) : "memory");
+}
+
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
+// Operand fragment from rows in LDS: lane (m, g2) gets steps 8 g2 .. + 7 of its channel; `a0` and `a1` are the lane's byte
+// addresses for the first and the last four of them.
+template <typename E>
+__device__ __forceinline__ V8<E> transposed_frag(const unsigned char *lds, int a0, int a1) {
+  typedef __attribute__((address_space(3))) i16x4_t *ptr;
+  struct { i16x4_t a, b; } r = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(lds + a0)), __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(lds + a1))};
+  return __builtin_bit_cast(V8<E>, r);
+}
+
+template <typename E>
+__device__ __forceinline__ V8<E> state_frag(const f32x16_t &s, int t) {
+  V8<E> r;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) r[j] = (E)s[8 * t + j];
+  return r;
+}
+
+// One head, or two neighbouring heads of a group (the last of an odd number alone: it is computed twice and written once).
+template <int NH>
+struct WalkHeads {
+  int b, g, h0, h1;
+  bool two;
+  __device__ __forceinline__ WalkHeads(const SsdWalkParams &p, int id) {
+    const int per_group = p.heads / p.groups, sets = (per_group + NH - 1) / NH;
+    const int i = id % sets;
+    g = id / sets % p.groups;
+    b = id / sets / p.groups;
+    h0 = g * per_group + NH * i;
+    two = NH == 2 && 2 * i + 1 < per_group;
+    h1 = two ? h0 + 1 : h0;
+  }
+  __device__ __forceinline__ WalkHeads(const SsdWalkParams &p, int b_, int h) : b(b_), g(h / (p.heads / p.groups)), h0(h), h1(h), two(false) {}
+  // Running sums at the ends of a head's blocks, read through the scalar cache.
+  __device__ __forceinline__ scalar_floats ends(const SsdWalkParams &p, int second) const {
+    return (scalar_floats)(size_t)(p.ends + ((size_t)b * p.heads + (second ? h1 : h0)) * p.turns);
+  }
+  // The pair's stretch of x, z or y as a buffer: reads past the last row give zero, stores there are dropped.
+  __device__ __forceinline__ rsrc_t rsrc(const void *base, const SsdWalkParams &p) const {
+    const unsigned pitch = (unsigned)p.heads * SSD_P * 2;
+    const unsigned char *at = reinterpret_cast<const unsigned char *>(base) + ((size_t)b * p.len * p.heads + h0) * SSD_P * 2;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char *>(at), 0, (int)((unsigned)(p.len - 1) * pitch + (two ? 2 : 1) * SSD_P * 2), 0x00020000);
+  }
+};
+
+// The waves of rows.  Turn c: gate and store block c - 1, stage block c + 1.  Each thread has eight channels of one row of
+// every block; what it takes from memory of them is requested four turns ahead.
+template <typename E, int NH, int DMODE, bool HAS_Z, bool FACTOR>
+__device__ __forceinline__ void walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
+  static_assert(FACTOR || NH == 1);
+  using L = WalkLds<NH>;
+  const int wave = wave_id_uniform() - 4, lane = lane_id(), tid = wave * WAVE + lane;
+  const int row = tid / (8 * NH), second = NH == 2 ? tid >> 3 & 1 : 0, piece = tid & 7;
+  const unsigned pitch = (unsigned)p.heads * SSD_P * 2, block = WK * pitch;
+  const rsrc_t rx = hp.rsrc(p.x, p), rz = hp.rsrc(HAS_Z ? p.z : p.x, p), ry = hp.rsrc(p.y, p);
+  const unsigned mine = (unsigned)row * pitch + (hp.two ? second : 0) * (SSD_P * 2) + piece * 16;
+  const bool drop = second && !hp.two;
+  const float2 *steps = reinterpret_cast<const float2 *>(p.steps) + ((size_t)hp.b * p.heads + hp.h0) * p.turns * WK;
+  const unsigned step_at = ((hp.two ? second : 0) * (unsigned)p.turns * WK + row) * 8;
+  const int h = second ? hp.h1 : hp.h0;
+  float D8[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) D8[j] = DMODE == 0 ? 0.0f : p.Dk[DMODE == 2 ? h * SSD_P + 8 * piece + j : h];
+  // !FACTOR: the four places of a block's C.B that this thread decays: row m, steps w_s ..
+  typedef __attribute__((__vector_size__(4 * sizeof(E)))) E vec4_t;
+  const int m = lane & 31, w_s = 16 * (wave >> 1) + 8 * (lane >> 5) + 4 * (wave & 1), w_at = (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8;
+  const unsigned char *pcb = reinterpret_cast<const unsigned char *>(p.CBblk) + ((size_t)hp.b * p.nblocks * p.groups + hp.g) * 2048;
+
+  V8<E> x[4], z[4];
+  float2 step[4];
+  vec4_t cb[4];
+  float skip[2][8], grow[2];
+  // A ring's place is loaded again once `after` is there: a load in front of the last use of what the place held would take
+  // another register, and the copy back at the end of the loop would wait for it.
+  const auto load_rows = [&](rsrc_t r, int c, const V8<E> &after) {
+    unsigned off = mine + (unsigned)c * block;
+    asm volatile("" : "+v"(off) : "v"(after));
+    return __builtin_bit_cast(V8<E>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  };
+  const auto load_step = [&](int c, const V8<E> &after) {
+    unsigned off = step_at;
+    asm volatile("" : "+v"(off) : "v"(after));
+    return *at_bytes<const float2>(steps + (size_t)min(c, p.turns - 1) * WK, off);
+  };
+  const auto load_cb = [&](int c, const vec4_t &after) {
+    unsigned off = (unsigned)w_at;
+    asm volatile("" : "+v"(off) : "v"(after));
+    return *at_bytes<const vec4_t>(pcb + (size_t)min(c, p.nblocks - 1) * p.groups * 2048, off);
+  };
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    x[u] = load_rows(rx, u, V8<E>{});
+    if (HAS_Z) z[u] = load_rows(rz, u, V8<E>{});
+    step[u] = load_step(u, V8<E>{});
+    if (!FACTOR) cb[u] = load_cb(u, vec4_t{});
+  }
+  const int at16 = second * WK_TILE + row * 128 + ((piece ^ (row & 7)) << 4);
+  const int half_at = L::PART + second * 16384 + (piece >> 2) * 4096 + row * 128;
+  const int q0 = half_at + (((2 * (piece & 3)) ^ (row & 7)) << 4), q1 = half_at + (((2 * (piece & 3) + 1) ^ (row & 7)) << 4);
+
+  const auto publish = [&](int u) __attribute__((always_inline)) {       // !FACTOR: what the block's steps mean to others
+    asm volatile("" : "+v"(step[u].x), "+v"(step[u].y));
+    float *st = reinterpret_cast<float *>(lds + PlainLds::STEPS + u * PlainLds::STEP_BYTES);
+    const float l2 = log2_hw(step[u].y);                   // dt = 0: -inf, a weight of zero
+    if (piece == 0) {
+      st[row] = step[u].x;
+      st[WK + row] = l2 - step[u].x;
+      st[2 * WK + row] = l2;
+    }
+  };
+  const auto stage = [&](int c, int u) __attribute__((always_inline)) {
+    // first looked at here: the scheduler would start on blocks ahead, and wait for reads that are still on their way
+    asm volatile("" : "+v"(x[u]), "+v"(step[u].x), "+v"(step[u].y));
+    float v[8];
+    unpack8(x[u], v);
+    if (DMODE != 0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) skip[u & 1][j] = D8[j] * v[j];
+    }
+    unsigned char *to = lds + (u & 1) * L::X + at16;
+    if constexpr (FACTOR) {
+      const float w = step[u].y * exp2_hw(-step[u].x);
+      grow[u & 1] = exp2_hw(step[u].x);
+      float lost[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] *= w;
+      const V8<E> rounded = pack8_e<E>(v);
+      unpack8(rounded, lost);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) lost[j] = v[j] - lost[j];
+      const V8<E> rest = pack8_e<E>(lost);
+      *reinterpret_cast<V8<E> *>(to) = rounded;
+      *reinterpret_cast<V8<E> *>(to + NH * WK_TILE) = rest;
+      x[u] = load_rows(rx, c + 4, rest);
+      step[u] = load_step(c + 4, rest);
+    } else {
+      const float *st = reinterpret_cast<const float *>(lds + PlainLds::STEPS + u * PlainLds::STEP_BYTES);
+      const float w = step[u].y * exp2_hw(fminf(st[31] - step[u].x, 0.0f)), own = st[m];
+      const float4 e4 = *reinterpret_cast<const float4 *>(st + WK + w_s), l4 = *reinterpret_cast<const float4 *>(st + 2 * WK + w_s);
+      *reinterpret_cast<V8<E> *>(to + WK_TILE) = x[u];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] *= w;
+      const V8<E> rounded = pack8_e<E>(v);
+      *reinterpret_cast<V8<E> *>(to) = rounded;
+      x[u] = load_rows(rx, c + 4, rounded);
+      step[u] = load_step(c + 4, rounded);
+      const float e[4] = {e4.x, e4.y, e4.z, e4.w}, l2[4] = {l4.x, l4.y, l4.z, l4.w};
+      asm volatile("" : "+v"(cb[u]));
+      vec4_t d;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        // dt_s exp(min(cs_l - cs_s, 0)) as one exponential: min(a, 0) + b = min(a + b, b) with b = log2 dt_s.  The bound is
+        // inactive on and below the diagonal of a decaying head, is the clamp of a growing one, and keeps the places above
+        // the diagonal (zeros of C.B) finite.
+        d[j] = (E)((float)cb[u][j] * exp2_hw(fminf(own + e[j], l2[j])));
+      }
+      *reinterpret_cast<vec4_t *>(lds + PlainLds::W + (u & 1) * 2048 + w_at) = d;
+      cb[u] = load_cb(c + 4, d);
+    }
+  };
+  struct Parts { float4 a0, a1, b0, b1; };
+  const auto read_parts = [&](int u) __attribute__((always_inline)) {
+    const unsigned char *half = lds + (u & 1) * L::PARTS;
+    return Parts{*reinterpret_cast<const float4 *>(half + q0), *reinterpret_cast<const float4 *>(half + q1),
+                 *reinterpret_cast<const float4 *>(half + 8192 + q0), *reinterpret_cast<const float4 *>(half + 8192 + q1)};
+  };
+  const auto gate = [&](int c, int u, const Parts &r, float up, const float (&dx)[8]) __attribute__((always_inline)) {
+    float v[8] = {r.a0.x + r.b0.x, r.a0.y + r.b0.y, r.a0.z + r.b0.z, r.a0.w + r.b0.w, r.a1.x + r.b1.x, r.a1.y + r.b1.y, r.a1.z + r.b1.z, r.a1.w + r.b1.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (FACTOR) v[j] = DMODE == 0 ? v[j] * up : __builtin_fmaf(v[j], up, dx[j]);
+      else if (DMODE != 0) v[j] += dx[j];
+    }
+    if (HAS_Z) {
+      float zf[8];
+      asm volatile("" : "+v"(z[u]));
+      unpack8(z[u], zf);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] *= silu_f32(zf[j]);
+    }
+    const V8<E> out = pack8_e<E>(v);
+    if (HAS_Z) z[u] = load_rows(rz, c + 4, out);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
+  };
+  if (!FACTOR) {
+    publish(0);
+    publish(1);
+  }
+  walk_barrier();                                          // (the products' first fragments; the first steps)
+  stage(0, 0);
+  walk_barrier();
+  for (int c0 = 0; c0 < p.turns; c0 += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = c0 + u, before = (u + 3) & 3;
+      const Parts parts = read_parts(before);              // of block c - 1 (before the first: values whose store is dropped)
+      const float up = grow[before & 1];
+      float dx[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dx[j] = skip[before & 1][j];
+      if (!FACTOR) publish((u + 2) & 3);
+      stage(c + 1, (u + 1) & 3);                           // of the block after the last: values that nothing reads
+      gate(c - 1, before, parts, up, dx);
+      walk_barrier();
+    }
+  }
+  gate(p.turns - 1, 3, read_parts(3), grow[1], skip[1]);
+}
+
+// The four waves of products of a head that does not factor.  Turn c: block c.
+template <typename E, int N, bool GROW>
+__device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned char *lds, int b, int h) {
+  using L = WalkLds<1>;
+  constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16;
+  const int wave = wave_id_uniform(), lane = lane_id();
+  const int m = lane & 31, g2 = lane >> 5, pt = wave & 1, nh = wave >> 1;
+
+  // a lane's addresses for transposing reads (transposed_frag), and of its row m among the part sums
+  const int k = lane & 15, tr_row = 8 * g2 + (k >> 2), tr_piece = 4 * pt + 2 * (lane >> 4 & 1) + ((k & 3) >> 1);
+  const int tr0 = tr_row * 128 + ((tr_piece ^ (k >> 2)) << 4) + (k & 1) * 8, tr1 = (tr0 + 512) ^ 64;
+  unsigned char *const part = lds + L::PART + (2 * nh + pt) * 4096 + m * 128;
+
+  // fragments of block c, this wave's part
+  const size_t unit0 = (size_t)b * p.nblocks * p.groups + h / (p.heads / p.groups);
+  const E *pc = reinterpret_cast<const E *>(p.Cblk) + (unit0 * KN + 2 * nh * TPW) * SSD_FRAG;
+  const E *pb = reinterpret_cast<const E *>(p.Btblk) + (unit0 * 2 * NT + nh * TPW) * SSD_FRAG;
+  const unsigned lane16 = (unsigned)lane * 16;
+  const auto c_frag = [&](int c, int i, int t) { return *at_bytes<const V8<E>>(pc + (size_t)(c * p.groups) * (KN * SSD_FRAG) + (2 * i + t) * SSD_FRAG, lane16); };
+  const auto b_frag = [&](int c, int i, int ks) { return *at_bytes<const V8<E>>(pb + (size_t)(c * p.groups) * (KN * SSD_FRAG) + (ks * NT + i) * SSD_FRAG, lane16); };
+
+  f32x16_t S[TPW];
+  V8<E> hf[GROW ? TPW : 1][2];                             // growing: the state entering the chunk, as operands; its float32 is in memory
+  float4 *const grown = reinterpret_cast<float4 *>(p.grown + ((size_t)b * p.heads + h) * SSD_P * N) + (wave * TPW * 4) * WAVE + lane;
+  const size_t state0 = (((size_t)b * p.heads + h) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    S[i] = (f32x16_t){0};
+    if (p.init) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[i][r] = p.init[state0 + 32 * i + crow(r, g2)];
+    }
+  }
+  V8<E> cf[TPW][2], bf[TPW][2];
+  // requested a block ahead (those of B in the same turn by a growing head, which keeps twice the state)
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      // without a state to start from the first block's product with it is zero whatever C holds
+      cf[i][t] = V8<E>{};
+      if (p.init) cf[i][t] = c_frag(0, i, t);
+      if (!GROW) bf[i][t] = b_frag(0, i, t);
+    }
+  }
+  float base = 0.0f;                                       // growing: running sum up to the block, from its chunk's first step
+
+  walk_barrier();
+  for (int c = 0; c < p.turns; ++c) {                      // turns past the last block: steps of size zero
+    const float *st = reinterpret_cast<const float *>(lds + PlainLds::STEPS + (c & 3) * PlainLds::STEP_BYTES);
+    const unsigned char *xwt = lds + (c & 1) * L::X, *xt = xwt + WK_TILE;
+    const int next = min(c + 1, p.nblocks - 1);
+    walk_barrier();
+    const float own = st[m] + st[31], end = 2.0f * st[31];
+    if (GROW && c % p.chunk_blocks == 0) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) grown[(4 * i + q) * WAVE] = make_float4(S[i][4 * q], S[i][4 * q + 1], S[i][4 * q + 2], S[i][4 * q + 3]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) hf[i][t] = state_frag<E>(S[i], t);
+        S[i] = (f32x16_t){0};
+      }
+      base = 0.0f;
+    }
+    f32x16_t acc = {0};
+    f32x16_t acc_h = {0};
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        acc = mma(state_frag<E>(S[i], t), cf[i][t], acc);
+        if (GROW) {
+          acc_h = mma(hf[i][t], cf[i][t], acc_h);
+          bf[i][t] = b_frag(min(c, p.nblocks - 1), i, t);
+        }
+        cf[i][t] = c_frag(next, i, t);
+      }
+    }
+    const float f = exp2_hw(GROW ? fminf(own, 0.0f) : own);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] *= f;
+    if (GROW) {
+      const float fh = fminf(exp2_hw(base + own), 3.0e38f);      // (finite: what is zero stays zero)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(acc_h[r], fh, acc[r]);
+    }
+    const float gs = exp2_hw(GROW ? fminf(end, 0.0f) : end);
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[i][r] *= gs;
+    }
+    acc = mma(transposed_frag<E>(xt, tr0 + nh * 2048, tr1 + nh * 2048),
+              load_frag_e<E>(lds + PlainLds::W + (c & 1) * 2048 + nh * 1024 + lane * 16), acc);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const V8<E> xf = transposed_frag<E>(xwt, tr0 + ks * 2048, tr1 + ks * 2048);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        S[i] = mma(bf[i][ks], xf, S[i]);
+        if (!GROW) bf[i][ks] = b_frag(next, i, ks);
+      }
+    }
+    if (GROW) {
+      base += end;
+      if ((c + 1) % p.chunk_blocks == 0 || c + 1 == p.turns) {
+        const float gh = fminf(exp2_hw(base), 3.0e38f);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float4 v = grown[(4 * i + q) * WAVE];
+            S[i][4 * q] = __builtin_fmaf(v.x, gh, S[i][4 * q]);
+            S[i][4 * q + 1] = __builtin_fmaf(v.y, gh, S[i][4 * q + 1]);
+            S[i][4 * q + 2] = __builtin_fmaf(v.z, gh, S[i][4 * q + 2]);
+            S[i][4 * q + 3] = __builtin_fmaf(v.w, gh, S[i][4 * q + 3]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      *reinterpret_cast<float4 *>(part + (c & 1) * L::PARTS + (((2 * q + g2) ^ (m & 7)) << 4)) =
+          make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    }
+  }
+  walk_barrier();
+
+  if (p.final_states) {
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4 *>(p.final_states + state0 + 32 * i + 8 * q + 4 * g2) =
+            make_float4(S[i][4 * q], S[i][4 * q + 1], S[i][4 * q + 2], S[i][4 * q + 3]);
+    }
+  }
+}
+
+// The four waves of products of heads that factor.  Turn c: block c.
+template <typename E, int NH, int N>
+__device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
+  using F = WalkLds<NH>;
+  using L = FactoredLds<NH, N>;
+  constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16, SHARE = KN / 4;
+  const int wave = wave_id_uniform(), lane = lane_id();
+  const int m = lane & 31, g2 = lane >> 5, pt = wave & 1, nh = wave >> 1;
+  const int k = lane & 15, tr_row = 8 * g2 + (k >> 2), tr_piece = 4 * pt + 2 * (lane >> 4 & 1) + ((k & 3) >> 1);
+  const int tr0 = tr_row * 128 + ((tr_piece ^ (k >> 2)) << 4) + (k & 1) * 8, tr1 = (tr0 + 512) ^ 64;
+  unsigned char *const part = lds + F::PART + (2 * nh + pt) * 4096 + m * 128;
+  const scalar_floats ends[2] = {hp.ends(p, 0), hp.ends(p, NH - 1)};
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds;
+  const unsigned lane16 = (unsigned)lane * 16;
+
+  // Fragments go from memory into LDS, a quarter by each wave, so that a workgroup reads each once: those of C three blocks
+  // ahead, of B and C.B two.
+  const size_t unit0 = (size_t)hp.b * p.nblocks * p.groups + hp.g;
+  const auto unit = [&](int c) { return unit0 + (size_t)min(c, p.nblocks - 1) * p.groups; };
+  const auto request_c = [&](int c, int slot) {
+    const E *from = reinterpret_cast<const E *>(p.Cblk) + (unit(c) * KN + SHARE * wave) * SSD_FRAG;
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) to_lds16(from + i * SSD_FRAG, lane16, lds0 + L::C + (slot * KN + SHARE * wave + i) * 1024);
+  };
+  const auto request_b = [&](int c, int slot) {
+    const E *from = reinterpret_cast<const E *>(p.Btblk) + (unit(c) * KN + SHARE * wave) * SSD_FRAG;
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) to_lds16(from + i * SSD_FRAG, lane16, lds0 + L::B + (slot * KN + SHARE * wave + i) * 1024);
+    if (wave < 2) to_lds16(reinterpret_cast<const E *>(p.CBblk) + (unit(c) * 2 + wave) * SSD_FRAG, lane16, lds0 + L::CB + slot * 2048 + wave * 1024);
+  };
+  const auto frag = [&](int at) { return load_frag_e<E>(lds + at + lane16); };
+
+  f32x16_t S[NH][TPW];
+  size_t state0[NH];
+#pragma unroll
+  for (int hd = 0; hd < NH; ++hd) {
+    state0[hd] = (((size_t)hp.b * p.heads + (hd ? hp.h1 : hp.h0)) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      S[hd][i] = (f32x16_t){0};
+      if (p.init) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[hd][i][r] = p.init[state0[hd] + 32 * i + crow(r, g2)];
+      }
+    }
+  }
+  request_c(1, 1);
+  request_c(2, 2);
+  request_b(0, 0);
+  request_b(1, 1);
+  if (p.init) {
+    request_c(0, 0);
+  } else {
+    // without a state to start from the first block's product with it is zero whatever C holds
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) *reinterpret_cast<V8<E> *>(lds + L::C + (SHARE * wave + i) * 1024 + lane16) = V8<E>{};
+  }
+  wait_memory<0>();
+  walk_barrier();
+  __builtin_amdgcn_s_setprio(1);
+  float end[NH] = {};
+  for (int c = 0, t3 = 0; c < p.turns; ++c) {              // turns past the last block: steps of size zero
+    const int last3 = t3 == 0 ? 2 : t3 - 1;
+    // in the turn of the block before, c - 1: the state, brought from the middle of that block to the middle of this one
+    f32x16_t acc[NH];
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) {
+      const float e = ends[hd][c];
+      float to_here = 0.5f * (end[hd] + e);
+      if (to_here < -120.0f) {                             // a factor that float32 does not hold, in two that it does
+        const float g = exp2_hw(0.5f * end[hd]);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+        }
+        to_here = 0.5f * e;
+      }
+      const float g = exp2_hw(to_here);
+      end[hd] = e;
+      acc[hd] = (f32x16_t){0};
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[hd] = mma(state_frag<E>(S[hd][i], t), frag(L::C + (t3 * KN + 2 * (nh * TPW + i) + t) * 1024), acc[hd]);
+      }
+    }
+    if (wave < 2) wait_memory<2 * SHARE + 1>();            // what turn c - 1 requested may be under way, no more
+    else wait_memory<2 * SHARE>();
+    walk_barrier();
+    request_c(c + 3, t3);
+    request_b(c + 2, last3);
+    const V8<E> cb = frag(L::CB + t3 * 2048 + nh * 1024);
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) {
+      const unsigned char *xt = lds + (c & 1) * F::X + hd * WK_TILE;
+      const V8<E> xf[2] = {transposed_frag<E>(xt, tr0, tr1), transposed_frag<E>(xt, tr0 + 2048, tr1 + 2048)};
+      acc[hd] = mma(nh ? xf[1] : xf[0], cb, acc[hd]);
+      acc[hd] = mma(transposed_frag<E>(xt + NH * WK_TILE, tr0 + 2048 * nh, tr1 + 2048 * nh), cb, acc[hd]);
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) S[hd][i] = mma(frag(L::B + (t3 * KN + ks * NT + nh * TPW + i) * 1024), xf[ks], S[hd][i]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4 *>(part + (c & 1) * F::PARTS + hd * 16384 + (((2 * q + g2) ^ (m & 7)) << 4)) =
+            make_float4(acc[hd][4 * q], acc[hd][4 * q + 1], acc[hd][4 * q + 2], acc[hd][4 * q + 3]);
+    }
+    t3 = t3 == 2 ? 0 : t3 + 1;
+  }
+  walk_barrier();
+  if (p.final_states) {
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) {
+      const float g = exp2_hw(0.5f * end[hd]);
+      if (hd && !hp.two) break;
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<float4 *>(p.final_states + state0[hd] + 32 * i + 8 * q + 4 * g2) =
+              make_float4(S[hd][i][4 * q] * g, S[hd][i][4 * q + 1] * g, S[hd][i][4 * q + 2] * g, S[hd][i][4 * q + 3] * g);
+      }
+    }
+  }
+  wait_memory<0>();                                        // nothing may land in LDS that is another workgroup's by then
+}
+
+// Whether all of the heads' blocks decay by at most WALK_RANGE (in powers of two), and none grows.
+template <int NH>
+__device__ __forceinline__ bool decays_factor(const SsdWalkParams &p, const WalkHeads<NH> &hp) {
+  const float *e0 = p.ends + ((size_t)hp.b * p.heads + hp.h0) * p.turns, *e1 = p.ends + ((size_t)hp.b * p.heads + hp.h1) * p.turns;
+  bool ok = p.A[hp.h0] <= 0.0f && p.A[hp.h1] <= 0.0f;
+  for (int c = lane_id(); c < p.turns; c += WAVE) ok = ok && e0[c] >= -WALK_RANGE && e0[c] <= 0.0f && e1[c] >= -WALK_RANGE && e1[c] <= 0.0f;
+  return __all(ok);
+}
+
+// Workgroups go to the 8 XCDs round-robin by their index: neighbouring heads of a batch row, which read the same fragments,
+// are numbered onto one.
+__device__ __forceinline__ int walk_order(unsigned id, unsigned n) {
+  const unsigned q = n >> 3, r = n & 7, x = id & 7;
+  return (int)(x * q + min(x, r) + (id >> 3));
+}
+
+constexpr int PLAIN_THREADS = 512;
+template <typename E, int N, int DMODE, bool HAS_Z>
+__device__ __forceinline__ void plain_head(const SsdWalkParams &p, unsigned char *lds, int b, int h) {
+  if (wave_id_uniform() >= 4) walk_rows<E, 1, DMODE, HAS_Z, false>(p, lds, WalkHeads<1>(p, b, h));
+  else if (p.A[h] > 0.0f) plain_products<E, N, true>(p, lds, b, h);
+  else plain_products<E, N, false>(p, lds, b, h);
+}
+
+constexpr int walk_threads(int nh) { return nh == 2 ? 768 : PLAIN_THREADS; }
+
+// NH = 0: no head factors, one per workgroup.  Else those that do, NH of them per workgroup, and behind them a workgroup for
+// each head again, which most of the time finds nothing to do.
+template <typename E, int NH, int N, int DMODE, bool HAS_Z>
+__global__ __launch_bounds__(walk_threads(NH)) __attribute__((amdgpu_waves_per_eu(NH == 0 ? 4 : NH + 1)))
+void ssd_walk_kernel(const SsdWalkParams p) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  if constexpr (NH == 0) {
+    const int vid = walk_order(blockIdx.x, gridDim.x);
+    plain_head<E, N, DMODE, HAS_Z>(p, lds, vid / p.heads, vid % p.heads);
+  } else if (blockIdx.x < (unsigned)p.sets) {
+    const WalkHeads<NH> hp(p, walk_order(blockIdx.x, p.sets));
+    if (!decays_factor(p, hp)) return;
+    if (wave_id_uniform() >= 4) walk_rows<E, NH, DMODE, HAS_Z, true>(p, lds, hp);
+    else factored_products<E, NH, N>(p, lds, hp);
+  } else {
+    const unsigned id = blockIdx.x - p.sets, second = NH == 2 ? id & 1 : 0;
+    const WalkHeads<NH> hp(p, walk_order(id / NH, p.sets));
+    if (wave_id_uniform() >= PLAIN_THREADS / WAVE || (second && !hp.two) || decays_factor(p, hp)) return;
+    plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, second ? hp.h1 : hp.h0);
+  }
+}
+
+template <typename E, int NH, int N>
+static int launch_walk(const SsdWalkParams &p, int dmode, hipStream_t s) {
+  constexpr int LDS = NH && FactoredLds<NH ? NH : 1, N>::BYTES > PlainLds::BYTES ? FactoredLds<NH ? NH : 1, N>::BYTES : PlainLds::BYTES;
+  const unsigned grid = (unsigned)(NH == 0 ? p.batch * p.heads : p.sets * (1 + NH));
+#define SSM_WALK(DM, HZ)                                                                              \
+  {                                                                                                   \
+    const auto kernel = ssd_walk_kernel<E, NH, N, DM, HZ>;                                            \
+    if (allow_dynamic_lds(kernel, LDS) != hipSuccess) {                                               \
+      set_error("ssm_ssd_combined_fwd: cannot reserve %d bytes of LDS", LDS);                         \
+      return SSM_ERR_LAUNCH;                                                                          \
+    }                                                                                                 \
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(walk_threads(NH)), LDS, s, p);                        \
+  }
+  if (p.z) {
+    if (dmode == 0) SSM_WALK(0, true)
+    else if (dmode == 1) SSM_WALK(1, true)
+    else SSM_WALK(2, true)
+  } else {
+    if (dmode == 0) SSM_WALK(0, false)
+    else if (dmode == 1) SSM_WALK(1, false)
+    else SSM_WALK(2, false)
+  }
+#undef SSM_WALK
+  SSM_CHECK_LAUNCH("ssm_ssd_combined_fwd");
+  return SSM_OK;
+}
+
+int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s) {
+  const int per_group = p.heads / p.groups;
+  // one head per workgroup while every workgroup has a CU of its own
+  const int nh = f16 ? 0 : p.batch * p.heads <= WALK_SINGLES ? 1 : 2;
+  p.sets = nh ? p.batch * p.groups * ((per_group + nh - 1) / nh) : 0;
+#define SSM_WALK_N(NN)                                                        \
+  return nh == 0   ? launch_walk<_Float16, 0, NN>(p, dmode, s)                \
+         : nh == 1 ? launch_walk<__bf16, 1, NN>(p, dmode, s)                  \
+                   : launch_walk<__bf16, 2, NN>(p, dmode, s);
+  if (nstate == 128) SSM_WALK_N(128)
+  SSM_WALK_N(64)
+#undef SSM_WALK_N
+}
+
+}  // namespace ssm

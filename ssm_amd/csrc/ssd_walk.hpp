@@ -1,0 +1,24 @@
+// What the one-pass SSD forward (ssd_walk.hip) is called with.
+#pragma once
+#include "ssd_common.hpp"
+
+namespace ssm {
+
+struct SsdWalkParams {                  // x, z, y and the fragment copies hold the call's 16-bit element type
+  const void *x, *z;
+  void *y;
+  const float *steps;                   // (B, H, turns, 32, 2): cs (running sum of dt A log2(e) since the block's first step) less half of the block's, and dt
+  const float *ends;                    // (B, H, turns): cs at the block's last step
+  const void *Cblk, *Btblk, *CBblk;     // fragments of blocks of 32 steps
+  const float *Dk, *init, *A;
+  float *final_states;
+  float *grown;                         // (B, H, 64 N): where a growing head keeps the state entering a chunk
+  int batch, len, heads, groups, nblocks;
+  int sets;                             // workgroups of one or two heads (set by ssd_walk_forward)
+  int turns;                            // nblocks in whole turns through a ring of four
+  int chunk_blocks;                     // blocks in a chunk of the call (what a growing head's factors go by)
+};
+
+int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s);
+
+}  // namespace ssm
