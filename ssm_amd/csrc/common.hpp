@@ -319,6 +319,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
 }
 
+// Running sum over each half of the lanes.
+__device__ __forceinline__ float half_wave_inclusive_sum(float v) {
+  v += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR2, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR4, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR8, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_BCAST15, 0xa>(0.0f, v);
+  return v;
+}
+
 // Running sum over the lanes: lane l ends with the sum of lanes 0..l (the same steps as wave_sum).
 __device__ __forceinline__ float wave_inclusive_sum(float v) {
   v += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, v);

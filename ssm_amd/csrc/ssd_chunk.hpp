@@ -25,12 +25,6 @@
 
 namespace ssm {
 
-// Workgroups go to the 8 XCDs round-robin: consecutive results of this go to one XCD.
-__device__ __forceinline__ unsigned xcd_order(unsigned id, unsigned n) {
-  const unsigned q = n >> 3, r = n & 7, x = id & 7;
-  return x * q + min(x, r) + (id >> 3);
-}
-
 template <typename E, int C> struct Row { static_assert(sizeof(E) == 2); E v[C]; } __attribute__((aligned(2 * C)));
 
 // (batch, chunk, head) of a workgroup and what follows from it.

@@ -108,7 +108,7 @@ struct SsdWorkLayout {
 
 inline size_t ssd_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// Whether the forward takes the chunks side by side (ssd_chunk.hip) rather than one after the other (ssd_fused.hip).
+// Whether the forward takes the chunks side by side (ssd_chunk.hip) rather than one after the other (ssd_walk.hip).
 bool ssd_side_by_side(const SsdDims &d);
 
 inline size_t ssd_added_bytes(const SsdDims &d) {
@@ -145,6 +145,12 @@ inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep, bool side_by_s
 
 // x -> y, final states; the states entering the chunks stay in the workspace.
 int ssd_chunk_forward(const ssm_ssd_combined_args &a, const SsdDims &d, const SsdWorkLayout &lay, hipStream_t s);
+
+// Workgroups go to the 8 XCDs round-robin: consecutive results of this go to one XCD.
+__device__ __forceinline__ unsigned xcd_order(unsigned id, unsigned n) {
+  const unsigned q = n >> 3, r = n & 7, x = id & 7;
+  return x * q + min(x, r) + (id >> 3);
+}
 
 __device__ __forceinline__ void store_any(void *p, int dtype, size_t i, float v) {
   if (dtype == SSM_F32) reinterpret_cast<float *>(p)[i] = v;

@@ -24,8 +24,7 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 //        row (16 contiguous bytes per step) into LDS transposed to [head][step];
 //        then one wave per head forms dt' = clamp(softplus(dt + bias)) and the
 //        running sum of dt' A (stored scaled by log2 e, the unit of the kernels'
-//        exponentials).  For the walk the sums start anew every 32 steps, and what it takes from a
-//        step is written as it uses it (SsdWalkParams::steps).
+//        exponentials).  For the walk the sums start anew every 32 steps (prep_walk_dt_role).
 //  pack: one wave per operand fragment of C and B^T.  Fragment (lane, j) of a
 //        32 x 16 block: row 32 rb + lane % 32, column 16 kb + 8 (lane / 32) + j.
 //          Cblk [(b,c,g)][lb][kn]  from C  (rows = time, columns = state)
@@ -37,9 +36,12 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 //        with zeros above the diagonal inside the diagonal blocks; for a backward also its transpose,
 //          CBtblk[(b,c,g)][sb][kl]  (rows = s, columns = l).
 // Steps past the end of a last chunk that is no whole one: size zero, rows of B and C zero.
+// What bounds it is the lines of B, C and dt that each workgroup touches: 4 x 2048 steps, 24 heads, everything a backward
+// needs, 14.5 us (17.3 with 64-bit divisions per wave and neighbours on different XCDs); 4 x 4096 steps, 80 heads, for the
+// walk, 15.2 (16.0).
 // The walk takes the last two roles with chunks of 32 steps, and a fragment of C with its states in the order in which
 // an accumulator's registers hold rows: (lane, j) = state 16 kn + 4 (lane / 32) + j, 8 further for j >= 4.
-constexpr int PD_HEADS = 4;
+constexpr int PD_HEADS = 4, PW_HEADS = 32;     // heads of a workgroup of either dt role
 struct SsdPrepParams {
   SsdCumsumParams cs;
   float *dA2;
@@ -60,18 +62,27 @@ struct SsdPrepParams {
 // reaches 2^14, where float32 still resolves 1e-3 of the exponent.
 constexpr float SEQ_JUMP_LN = -64.0f * 0.69314718056f;
 
-template <bool WALK>
-__device__ __forceinline__ void prep_dt_role(const SsdPrepParams &pp, int wg, float *lds) {
+// dt' = clamp(softplus(dt + bias)), and what a step adds to the running sum of dt' A beyond its product: the jump into a
+// sequence at step t of batch row b.
+__device__ __forceinline__ float prep_step(const SsdCumsumParams &p, float x) {
+  if (p.softplus) x = softplus_f32(x);
+  return fminf(fmaxf(x, p.dt_min), p.dt_max);
+}
+__device__ __forceinline__ float sequence_jump(const SsdPrepParams &pp, int b, size_t t) {
+  const int *sid = pp.seq_idx + (size_t)b * pp.cs.d.len;
+  return (t == 0 ? sid[0] != 0 : sid[t] != sid[t - 1]) ? SEQ_JUMP_LN : 0.0f;
+}
+
+__device__ __forceinline__ void prep_dt_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
   float (*tile)[256 + 1] = reinterpret_cast<float (*)[256 + 1]>(lds);
   const SsdCumsumParams &p = pp.cs;
   const SsdDims &d = p.d;
-  const int Q = WALK ? 256 : d.chunk;              // steps of this workgroup
-  const int nunits = WALK ? (d.len + 255) >> 8 : d.nchunks;
-  const int hgroups = (d.heads + PD_HEADS - 1) / PD_HEADS;
-  const int hg = wg % hgroups;
-  const int c = (wg / hgroups) % nunits;
-  const int b = wg / (hgroups * nunits);
-  const int h0 = hg * PD_HEADS;
+  const int Q = d.chunk;
+  const unsigned hgroups = (unsigned)(d.heads + PD_HEADS - 1) / PD_HEADS, rest = wg / hgroups;
+  const int h0 = (int)(wg - rest * hgroups) * PD_HEADS, b = (int)(rest / (unsigned)d.nchunks), c = (int)rest - b * d.nchunks;
+  const int wave = wave_id_uniform(), lane = lane_id(), h = h0 + wave;        // a wave a head
+  const float A = p.A[min(h, d.heads - 1)], bias = p.bias ? p.bias[min(h, d.heads - 1)] : 0.0f;
+#pragma unroll 4
   for (int e = threadIdx.x; e < Q * PD_HEADS; e += 256) {
     const int l = e / PD_HEADS, hh = e % PD_HEADS;
     float v = 0.0f;
@@ -80,88 +91,82 @@ __device__ __forceinline__ void prep_dt_role(const SsdPrepParams &pp, int wg, fl
     tile[hh][l] = v;
   }
   __syncthreads();
-  const int wave = wave_id_uniform(), lane = lane_id();
+  if (h >= d.heads) return;
   const int per = (Q + 63) >> 6;
-  constexpr int SPAN = WALK ? SSD_WALK_BLOCK / 4 : WAVE;      // lanes that a running sum goes over
   const int rows = min(Q, d.len - c * Q);          // steps past the end have size zero
-  for (int hh = wave; hh < PD_HEADS; hh += 4) {
-    const int h = h0 + hh;
-    if (h >= d.heads) break;
-    const float A = p.A[h];
-    const float bias = p.bias ? p.bias[h] : 0.0f;
-    float v[4], run[4];
-    float tot = 0.0f;
+  float v[4], run[4];
+  float tot = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int l = lane * per + i;
-      v[i] = 0.0f;
-      if (i < per && l < rows) {
-        float x = tile[hh][l] + bias;
-        if (p.softplus) x = softplus_f32(x);
-        v[i] = fminf(fmaxf(x, p.dt_min), p.dt_max);
-      }
-      tot = __builtin_fmaf(v[i], A, tot);
-      if (pp.seq_idx && i < per && l < rows) {
-        const size_t t = (size_t)c * Q + l;
-        const int *sid = pp.seq_idx + (size_t)b * d.len;
-        if (t == 0 ? sid[0] != 0 : sid[t] != sid[t - 1]) tot += SEQ_JUMP_LN;
-      }
-      run[i] = tot;
-    }
-    float incl = tot;
+  for (int i = 0; i < 4; ++i) {
+    const int l = lane * per + i;
+    const bool live = i < per && l < rows;
+    v[i] = live ? prep_step(p, tile[wave][l] + bias) : 0.0f;
+    tot = __builtin_fmaf(v[i], A, tot);
+    if (pp.seq_idx && live) tot += sequence_jump(pp, b, (size_t)c * Q + l);
+    run[i] = tot;
+  }
+  const float excl = wave_inclusive_sum(tot) - tot;
+  const size_t out = (((size_t)b * d.heads + h) * d.nchunks + c) * (size_t)Q;
 #pragma unroll
-    for (int off = 1; off < SPAN; off <<= 1) {
-      const float t = __shfl_up(incl, off, SPAN);
-      if (lane % SPAN >= off) incl += t;
-    }
-    const float excl = incl - tot;
-    if constexpr (WALK) {
-      const float end = __shfl(incl, SPAN - 1, SPAN) * LOG2E;
-      const int blk = c * 8 + lane / SPAN, turns = ssd_walk_turns(d.nchunks);
-      if (blk >= turns) continue;
-      const size_t at = ((size_t)b * d.heads + h) * turns + blk;
-      float cs[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) cs[i] = (excl + run[i]) * LOG2E - 0.5f * end;
-      float *out = pp.steps + at * (2 * SSD_WALK_BLOCK) + lane % SPAN * 8;
-      *reinterpret_cast<float4 *>(out) = make_float4(cs[0], v[0], cs[1], v[1]);
-      *reinterpret_cast<float4 *>(out + 4) = make_float4(cs[2], v[2], cs[3], v[3]);
-      if (lane % SPAN == SPAN - 1) pp.ends[at] = end;
-    } else {
-      const size_t out = (((size_t)b * d.heads + h) * d.nchunks + c) * (size_t)Q;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int l = lane * per + i;
-        if (i < per && l < Q) {
-          p.dt_out[out + l] = v[i];
-          pp.dA2[out + l] = (excl + run[i]) * LOG2E;
-        }
-      }
+  for (int i = 0; i < 4; ++i) {
+    const int l = lane * per + i;
+    if (i < per && l < Q) {
+      p.dt_out[out + l] = v[i];
+      pp.dA2[out + l] = (excl + run[i]) * LOG2E;
     }
   }
 }
 
-template <typename E>
+// For the walk: two blocks of 32 heads, whose 64 bytes of a row are read together.
+__device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
+  float (*tile)[64 + 1] = reinterpret_cast<float (*)[64 + 1]>(lds);
+  const SsdCumsumParams &p = pp.cs;
+  const SsdDims &d = p.d;
+  const unsigned turns = (unsigned)ssd_walk_turns(d.nchunks), hgroups = (unsigned)(d.heads + PW_HEADS - 1) / PW_HEADS, rest = wg / hgroups;
+  const int h0 = (int)(wg - rest * hgroups) * PW_HEADS, b = (int)(rest / (turns >> 1)), unit = (int)(rest - b * (turns >> 1));
+  const int l0 = 64 * unit;
+#pragma unroll
+  for (int e = (int)threadIdx.x; e < 64 * PW_HEADS; e += 256) {
+    const int l = e / PW_HEADS, hh = e % PW_HEADS;
+    float v = 0.0f;
+    if (h0 + hh < d.heads && l0 + l < d.len) v = load_as_f32(p.dt, p.dt_dtype, ((size_t)b * d.len + l0 + l) * d.heads + h0 + hh);
+    tile[hh][l] = v;
+  }
+  __syncthreads();
+  const int wave = wave_id_uniform(), lane = lane_id();
+  const bool live = l0 + lane < d.len;               // steps past the end have size zero
+  const float jump = pp.seq_idx && live ? sequence_jump(pp, b, (size_t)l0 + lane) : 0.0f;
+#pragma unroll 2
+  for (int k = 0; k < PW_HEADS / 4; ++k) {
+    const int hh = wave * (PW_HEADS / 4) + k, h = h0 + hh;
+    if (h >= d.heads) return;
+    const float v = live ? prep_step(p, tile[hh][lane] + (p.bias ? p.bias[h] : 0.0f)) : 0.0f;
+    const float cs = half_wave_inclusive_sum(__builtin_fmaf(v, p.A[h], jump)) * LOG2E;
+    const float end = lane < SSD_WALK_BLOCK ? wave_read_lane(cs, SSD_WALK_BLOCK - 1) : wave_read_lane(cs, 2 * SSD_WALK_BLOCK - 1);
+    const size_t at = ((size_t)b * d.heads + h) * turns + 2 * unit;           // block
+    reinterpret_cast<float2 *>(pp.steps)[at * SSD_WALK_BLOCK + lane] = make_float2(cs - 0.5f * end, v);
+    if (lane % SSD_WALK_BLOCK == SSD_WALK_BLOCK - 1) pp.ends[at + lane / SSD_WALK_BLOCK] = end;
+  }
+}
+
+template <typename E, int KN>
 __device__ __forceinline__ void prep_pack_role(const SsdPrepParams &pp, unsigned wg) {
   const SsdDims &d = pp.cs.d;
   const int wave = wave_id_uniform(), lane = lane_id();
-  const int Q = d.chunk, N = d.nstate, nc = d.nchunks, groups = d.groups, len = d.len;
-  const int KN = N >> 4, NT = N >> 5;
-  const int per_unit = (Q >> 5) * KN;                     // = (Q / 16) * NT
-  const size_t each = (size_t)d.batch * nc * groups * per_unit;
-  size_t f = (size_t)wg * 4 + wave;
-  if (f >= each * pp.n_kinds) return;
-  const int kind = (int)(f / each);                       // rows of C, columns of B, rows of B, columns of C
-  f -= kind * each;
+  constexpr int N = 16 * KN, NT = N >> 5;
+  const int Q = d.chunk, nc = d.nchunks, groups = d.groups, len = d.len;
+  const unsigned per_unit = (unsigned)(Q >> 5) * KN;      // = (Q / 16) * NT fragments, whole workgroups of four
+  const unsigned each = (unsigned)d.batch * nc * groups * (per_unit >> 2);
+  const int kind = (int)(wg / each);                      // rows of C, columns of B, rows of B, columns of C
+  wg -= kind * each;
   const bool rows = kind == 0 || kind == 2, from_c = kind == 0 || kind == 3;
   const E *src = reinterpret_cast<const E *>(from_c ? pp.Cm : pp.Bm);
   const size_t stride = from_c ? pp.c_row : pp.b_row;
   void *dst = kind == 0 ? pp.Cblk : kind == 1 ? pp.Btblk : kind == 2 ? pp.Bblk : pp.Ctblk;
-  const int inner = (int)(f % per_unit);
-  const size_t unit = f / per_unit;
-  const int g = (int)(unit % groups);
-  const int c = (int)((unit / groups) % nc);
-  const int b = (int)(unit / ((size_t)groups * nc));
+  const unsigned unit = wg / (per_unit >> 2), bc = unit / (unsigned)groups;
+  const int inner = (int)((wg - unit * (per_unit >> 2)) * 4) + wave;
+  const size_t f = (size_t)unit * per_unit + inner;
+  const int g = (int)(unit - bc * groups), b = (int)(bc / (unsigned)nc), c = (int)bc - b * nc;
   const int m = lane & 31, g2 = lane >> 5;
   src += (size_t)b * len * stride + (size_t)g * N;
   V8<E> v;
@@ -189,29 +194,37 @@ __device__ __forceinline__ void prep_pack_role(const SsdPrepParams &pp, unsigned
   *reinterpret_cast<V8<E> *>(reinterpret_cast<E *>(dst) + f * FRAG + lane * 8) = v;
 }
 
-template <typename E>
+template <typename E, int KN>
 __device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
   const SsdDims &d = pp.cs.d;
   const int wave = wave_id_uniform(), lane = lane_id();
-  const int Q = d.chunk, N = d.nstate, groups = d.groups;
+  constexpr int N = 16 * KN;
+  const int Q = d.chunk, groups = d.groups;
   const int NLB = Q >> 5, KS = Q >> 4;
-  const int per_unit = NLB * (NLB + 1) / 2;
-  const size_t units = (size_t)d.batch * d.nchunks * groups;
-  const size_t blk = (size_t)wg * 4 + wave;
-  if (blk >= units * per_unit) return;
-  const size_t unit = blk / per_unit;
-  const int idx = (int)(blk % per_unit);
+  const unsigned per_unit = (unsigned)NLB * (NLB + 1) / 2;
+  const unsigned units = (unsigned)d.batch * d.nchunks * groups;
+  const unsigned blk = wg * 4 + wave, unit32 = blk / per_unit;
+  if (unit32 >= units) return;
+  const size_t unit = unit32;
+  const int idx = (int)(blk - unit32 * per_unit);
   int lb = 0;
   while ((lb + 1) * (lb + 2) / 2 <= idx) ++lb;
   const int sb = idx - lb * (lb + 1) / 2;
-  const int g = (int)(unit % groups);
-  const int c = (int)((unit / groups) % d.nchunks);
-  const size_t row0 = unit / groups / d.nchunks * d.len;  // rows past the end stand for the last one: they meet only zeros
+  const unsigned bc = unit32 / (unsigned)groups, b = bc / (unsigned)d.nchunks;
+  const int g = (int)(unit32 - bc * groups), c = (int)(bc - b * d.nchunks);
+  const size_t row0 = (size_t)b * d.len;                  // rows past the end stand for the last one: they meet only zeros
   const int m = lane & 31, g2 = lane >> 5;
   const E *crow_p = reinterpret_cast<const E *>(pp.Cm) + (row0 + min(c * Q + 32 * lb + m, d.len - 1)) * pp.c_row + (size_t)g * N + 8 * g2;
   const E *brow_p = reinterpret_cast<const E *>(pp.Bm) + (row0 + min(c * Q + 32 * sb + m, d.len - 1)) * pp.b_row + (size_t)g * N + 8 * g2;
   f32x16_t acc = {0};
-  for (int k0 = 0; k0 < N; k0 += 16) acc = mma(load_frag_e<E>(crow_p + k0), load_frag_e<E>(brow_p + k0), acc);
+  V8<E> cf[KN], bf[KN];
+#pragma unroll
+  for (int i = 0; i < KN; ++i) {
+    cf[i] = load_frag_e<E>(crow_p + 16 * i);
+    bf[i] = load_frag_e<E>(brow_p + 16 * i);
+  }
+#pragma unroll
+  for (int i = 0; i < KN; ++i) acc = mma(cf[i], bf[i], acc);
   float (*tile)[33] = reinterpret_cast<float (*)[33]>(lds + wave * 32 * 33);
 #pragma unroll
   for (int r = 0; r < 16; ++r) tile[crow(r, g2)][m] = acc[r];
@@ -241,13 +254,19 @@ __device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned w
   }
 }
 
-template <typename E>
+template <typename E, int KN>
 __global__ __launch_bounds__(256) void ssd_fused_prep_kernel(const SsdPrepParams pp) {
   __shared__ float lds[4 * 32 * 33];
   const unsigned wg = blockIdx.x;
-  if (wg < pp.n_dt) pp.steps ? prep_dt_role<true>(pp, (int)wg, lds) : prep_dt_role<false>(pp, (int)wg, lds);
-  else if (wg < pp.n_dt + pp.n_pack) prep_pack_role<E>(pp, wg - pp.n_dt);
-  else prep_cb_role<E>(pp, wg - pp.n_dt - pp.n_pack, lds);
+  // neighbours in a role, which read the same lines, on one XCD
+  if (wg < pp.n_dt) {
+    if (pp.steps) prep_walk_dt_role(pp, xcd_order(wg, pp.n_dt), lds);
+    else prep_dt_role(pp, xcd_order(wg, pp.n_dt), lds);
+  } else if (wg < pp.n_dt + pp.n_pack) {
+    prep_pack_role<E, KN>(pp, xcd_order(wg - pp.n_dt, pp.n_pack));
+  } else {
+    prep_cb_role<E, KN>(pp, xcd_order(wg - pp.n_dt - pp.n_pack, gridDim.x - pp.n_dt - pp.n_pack), lds);
+  }
 }
 
 static bool fused_shape_ok(const SsdDims &d) {
@@ -368,15 +387,22 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   pp.Cblk = Cblk; pp.Btblk = Btblk; pp.CBblk = ws + lay.CBblk;
   pp.n_kinds = keep ? 4 : 2;
   if (keep) { pp.Bblk = ws + lay.Bblk; pp.Ctblk = ws + lay.Ctblk; pp.CBtblk = ws + lay.CBtblk; }
-  const size_t n_dt = (size_t)d.batch * (side_by_side ? (size_t)d.nchunks : ((size_t)d.len + 255) / 256) * ((d.heads + PD_HEADS - 1) / PD_HEADS);
-  const size_t n_pack = (bcg * NLB * KN * pp.n_kinds + 3) / 4;
+  const size_t n_dt = side_by_side ? (size_t)d.batch * d.nchunks * ((d.heads + PD_HEADS - 1) / PD_HEADS)
+                                   : (size_t)d.batch * (ssd_walk_turns(units.nchunks) / 2) * ((d.heads + PW_HEADS - 1) / PW_HEADS);
+  const size_t n_pack = bcg * NLB * KN * pp.n_kinds / 4;
   const size_t n_cb = (bcg * (NLB * (NLB + 1) / 2) + 3) / 4;
-  SSM_REQUIRE(n_dt + n_pack + n_cb < ((size_t)1 << 31), SSM_ERR_TOO_LARGE, "ssm_ssd_combined_fwd: too many workgroups");
+  SSM_REQUIRE(n_dt + n_pack + n_cb < ((size_t)1 << 29), SSM_ERR_TOO_LARGE, "ssm_ssd_combined_fwd: too many workgroups");
   pp.n_dt = (unsigned)n_dt; pp.n_pack = (unsigned)n_pack;
   pp.seq_idx = a->seq_idx;
   const bool f16 = a->io_dtype == SSM_F16;
-  if (f16) hipLaunchKernelGGL(ssd_fused_prep_kernel<_Float16>, dim3((unsigned)(n_dt + n_pack + n_cb)), dim3(256), 0, s, pp);
-  else hipLaunchKernelGGL(ssd_fused_prep_kernel<__bf16>, dim3((unsigned)(n_dt + n_pack + n_cb)), dim3(256), 0, s, pp);
+  const dim3 prep_grid((unsigned)(n_dt + n_pack + n_cb)), prep_block(256);
+  if (d.nstate == 128) {
+    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 8>), prep_grid, prep_block, 0, s, pp);
+    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 8>), prep_grid, prep_block, 0, s, pp);
+  } else {
+    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 4>), prep_grid, prep_block, 0, s, pp);
+    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 4>), prep_grid, prep_block, 0, s, pp);
+  }
   SSM_CHECK_LAUNCH("ssm_ssd_combined_fwd(prep)");
   note_mfma_launch(side_by_side ? 16 : 8);
   if (side_by_side) return ssd_chunk_forward(*a, d, lay, s);

@@ -565,13 +565,6 @@ __device__ __forceinline__ bool decays_factor(const SsdWalkParams &p, const Walk
   return __all(ok);
 }
 
-// Workgroups go to the 8 XCDs round-robin by their index: neighbouring heads of a batch row, which read the same fragments,
-// are numbered onto one.
-__device__ __forceinline__ int walk_order(unsigned id, unsigned n) {
-  const unsigned q = n >> 3, r = n & 7, x = id & 7;
-  return (int)(x * q + min(x, r) + (id >> 3));
-}
-
 constexpr int PLAIN_THREADS = 512;
 template <typename E, int N, int DMODE, bool HAS_Z>
 __device__ __forceinline__ void plain_head(const SsdWalkParams &p, unsigned char *lds, int b, int h) {
@@ -582,6 +575,7 @@ __device__ __forceinline__ void plain_head(const SsdWalkParams &p, unsigned char
 
 constexpr int walk_threads(int nh) { return nh == 2 ? 768 : PLAIN_THREADS; }
 
+// (xcd_order: neighbouring heads of a batch row, which read the same fragments, go to one XCD.)
 // NH = 0: no head factors, one per workgroup.  Else those that do, NH of them per workgroup, and behind them a workgroup for
 // each head again, which most of the time finds nothing to do.
 template <typename E, int NH, int N, int DMODE, bool HAS_Z>
@@ -589,16 +583,16 @@ __global__ __launch_bounds__(walk_threads(NH)) __attribute__((amdgpu_waves_per_e
 void ssd_walk_kernel(const SsdWalkParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
   if constexpr (NH == 0) {
-    const int vid = walk_order(blockIdx.x, gridDim.x);
+    const int vid = (int)xcd_order(blockIdx.x, gridDim.x);
     plain_head<E, N, DMODE, HAS_Z>(p, lds, vid / p.heads, vid % p.heads);
   } else if (blockIdx.x < (unsigned)p.sets) {
-    const WalkHeads<NH> hp(p, walk_order(blockIdx.x, p.sets));
+    const WalkHeads<NH> hp(p, (int)xcd_order(blockIdx.x, p.sets));
     if (!decays_factor(p, hp)) return;
     if (wave_id_uniform() >= 4) walk_rows<E, NH, DMODE, HAS_Z, true>(p, lds, hp);
     else factored_products<E, NH, N>(p, lds, hp);
   } else {
     const unsigned id = blockIdx.x - p.sets, second = NH == 2 ? id & 1 : 0;
-    const WalkHeads<NH> hp(p, walk_order(id / NH, p.sets));
+    const WalkHeads<NH> hp(p, (int)xcd_order(id / NH, p.sets));
     if (wave_id_uniform() >= PLAIN_THREADS / WAVE || (second && !hp.two) || decays_factor(p, hp)) return;
     plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, second ? hp.h1 : hp.h0);
   }
