@@ -27,25 +27,36 @@ struct SsdDbcParams {
   int len, heads, groups, nchunks, units;      // units = batch * nchunks * groups
 };
 
-// A workgroup of 8 waves takes 64 rows of dC (or of dB) of one (batch, chunk, group) and walks the heads: the 64 own rows,
-// all rows they meet (s <= l, or l >= s) and the state of the next head are on their way from L2 to registers while those
-// of this head, in LDS, are multiplied (one barrier per head).  Wave w has the own tile w & 1 and every fourth of the
-// tiles it meets; M stays in its accumulators, in float32, over all heads and is rounded once, for the product with B or C.
-// Rows are read whole (128 bytes a row) and turned into fragments by LDS, 16-byte pieces XOR-swizzled by row.
+// A workgroup takes 64 rows of dC (or of dB) of one (batch, chunk, group) and walks the heads: the 64 own rows, all rows they
+// meet (s <= l, or l >= s) and the state of the next head are on their way from L2 to registers while those of this head, in
+// LDS, are multiplied (one barrier per head).  Wave w has the own tile w & 1 and, of the tiles it meets, every eighth (every
+// fourth in shorter chunks); M stays in its accumulators, in float32, over all heads and is rounded once, for the product
+// with B or C.  Rows are read whole (128 bytes a row) and turned into fragments by LDS, 16-byte pieces XOR-swizzled by pairs
+// of rows: two rows are all banks.
 // The 64-row cut keeps the reads at 2.5 times the tensors (32 rows: 4.5 times) with 8 such workgroups per chunk.
-template <int Q, int N>
-__global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
+// Bound: the chain from one barrier to the next, one workgroup to a CU: fragments, four dependent products, weights, rows
+// to LDS.  At 4 x 2048 steps, 24 heads, 128 states, chunks of 256 it takes 48.5 us; its loads without the arithmetic take
+// 36, the arithmetic without the loads 43.  Before, 58.6: 8 waves hid less of the chain (57 with everything else as it is
+// now), a swizzle by single rows left every read two to a bank (50.3), and 64-bit addresses, masks in scalars and both sides
+// in one body took the registers that 16 waves do not have.  Tiles of a chunk's two ends paired, so that every workgroup
+// meets as many: 48.7 here, 1.5 % more of a training step at three times the batch.
+template <int Q> constexpr int DBC_WAVES = Q >= 256 ? 16 : 8;
+template <int Q, int N, bool for_b>
+__device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned char *smem) {
   typedef V8<elem_t> v8;
+  typedef const __attribute__((address_space(1))) char *global_bytes;
+  typedef const __attribute__((address_space(1))) v8 *global_v8;
+  typedef const __attribute__((address_space(1))) float *global_f32;
   constexpr int KS = Q >> 4, NT = N >> 5, NR = Q >> 6, QMASK = Staging<Q>::QMASK;
   constexpr int TILE = 64 * 64, BUF = (1 + NR) * TILE + N * 64;        // own rows, met rows, state
-  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int MW = DBC_WAVES<Q> / 2, MT = (2 * NR + MW - 1) / MW;      // waves an own tile has, tiles it meets in each
+  constexpr int RPP = 8 * DBC_WAVES<Q>, MET = (64 * NR + RPP - 1) / RPP, ST = (N + RPP - 1) / RPP;     // rows read at a time
   elem_t *bufs = reinterpret_cast<elem_t *>(smem);                     // [2][BUF]
   float *steps = reinterpret_cast<float *>(smem + 2 * BUF * sizeof(elem_t));     // [2][4][Q]: running sum, log2 dt, P, R
   const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
-  const int m = lane & 31, g2 = lane >> 5, ot = wave & 1, k4 = wave >> 1;
+  const int m = lane & 31, g2 = lane >> 5, ot = wave & 1, mw = wave >> 1;
   // the workgroups that meet the most rows start first
   const unsigned rank = blockIdx.x / (2u * p.units), rest = blockIdx.x % (2u * p.units);
-  const bool for_b = rest & 1;
   const unsigned unit = rest >> 1;
   const int r = for_b ? (int)rank : NR - 1 - (int)rank;
   const int meets = (int)(NR - rank);                                  // blocks of 64 rows
@@ -61,37 +72,41 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
   const int met0 = for_b ? 64 * r : 0;                                 // first met row
 
   // ---- one head's operands, global -> registers -> LDS
-  const int lr = tid >> 3, piece = tid & 7;                            // row of a 64-row block, 16-byte piece
-  const unsigned own_at = (unsigned)min(64 * r + lr, rows - 1) * (unsigned)pitch + piece * 8;
-  unsigned met_at[NR];
+  const int lr = tid >> 3, piece = tid & 7;                            // row of those read at a time, 16-byte piece
+  const unsigned own_at = ((unsigned)min(64 * r + lr, rows - 1) * (unsigned)pitch + piece * 8) * 2;      // bytes
+  unsigned met_at[MET];
 #pragma unroll
-  for (int k = 0; k < NR; ++k) met_at[k] = (unsigned)min(met0 + 64 * k + lr, rows - 1) * (unsigned)pitch + piece * 8;
-  v8 own_r, met_r[NR];
-  v8 st_r[N / 64];
+  for (int k = 0; k < MET; ++k) met_at[k] = ((unsigned)min(met0 + RPP * k + lr, rows - 1) * (unsigned)pitch + piece * 8) * 2;
+  v8 own_r, met_r[MET], st_r[ST];
   float cs_r = 0.0f, dt_r = 0.0f, cs_b = 0.0f;
   const auto fetch = [&](int h) {
-    own_r = *reinterpret_cast<const v8 *>(own_src + h * SSD_P + own_at);
+    // scalar bases, formed anew for each head: a lane keeps 32-bit offsets alone
+    global_bytes own_h = (global_bytes)(own_src + h * SSD_P), met_h = (global_bytes)(met_src + h * SSD_P);
+    global_bytes st_h = (global_bytes)(st_src + (size_t)h * (SSD_P * N));
+    global_bytes cs_h = (global_bytes)(p.dA2 + step0 + h * step_pitch), dt_h = (global_bytes)(p.dtv + step0 + h * step_pitch);
+    asm volatile("" : "+s"(own_h), "+s"(met_h), "+s"(st_h), "+s"(cs_h), "+s"(dt_h));
+    if (lr < 64) own_r = *(global_v8)(own_h + own_at);
 #pragma unroll
-    for (int k = 0; k < NR; ++k)
-      if (k < meets) met_r[k] = *reinterpret_cast<const v8 *>(met_src + h * SSD_P + met_at[k]);
+    for (int k = 0; k < MET; ++k)
+      if (RPP * k + lr < 64 * meets) met_r[k] = *(global_v8)(met_h + met_at[k]);
 #pragma unroll
-    for (int k = 0; k < N / 64; ++k)
-      st_r[k] = *reinterpret_cast<const v8 *>(st_src + (size_t)h * (SSD_P * N) + (64 * k + lr) * 64 + piece * 8);
+    for (int k = 0; k < ST; ++k)
+      if (RPP * k + lr < N) st_r[k] = *(global_v8)(st_h + (RPP * k * 128 + (unsigned)tid * 16));
     if (tid < Q) {
-      cs_r = p.dA2[step0 + h * step_pitch + tid];
-      dt_r = p.dtv[step0 + h * step_pitch + tid];
-      if (wave) cs_b = p.dA2[step0 + h * step_pitch + 64 * wave - 1];
+      cs_r = *(global_f32)(cs_h + (unsigned)tid * 4);
+      dt_r = *(global_f32)(dt_h + (unsigned)tid * 4);
+      if (wave) cs_b = *(global_f32)(cs_h + (256 * wave - 4));
     }
   };
   const auto put = [&](int at) {
     elem_t *own = bufs + at * BUF, *met = own + TILE, *st = met + NR * TILE;
-    *reinterpret_cast<v8 *>(own + lr * 64 + ((piece ^ (lr & 7)) << 3)) = own_r;
+    if (lr < 64) *reinterpret_cast<v8 *>(own + lr * 64 + ((piece ^ (lr >> 1 & 7)) << 3)) = own_r;
 #pragma unroll
-    for (int k = 0; k < NR; ++k)
-      if (k < meets) *reinterpret_cast<v8 *>(met + (64 * k + lr) * 64 + ((piece ^ (lr & 7)) << 3)) = met_r[k];
+    for (int k = 0; k < MET; ++k)
+      if (RPP * k + lr < 64 * meets) *reinterpret_cast<v8 *>(met + (RPP * k + lr) * 64 + ((piece ^ (lr >> 1 & 7)) << 3)) = met_r[k];
 #pragma unroll
-    for (int k = 0; k < N / 64; ++k)
-      *reinterpret_cast<v8 *>(st + (64 * k + lr) * 64 + ((piece ^ (lr & 7)) << 3)) = st_r[k];
+    for (int k = 0; k < ST; ++k)
+      if (RPP * k + lr < N) *reinterpret_cast<v8 *>(st + (RPP * k + lr) * 64 + ((piece ^ (lr >> 1 & 7)) << 3)) = st_r[k];
     if (tid < Q) {
       // decays from the block of 32 before to a step, and (times dt) from a step to the end of its block
       float *t = steps + 4 * at * Q + tid;
@@ -102,13 +117,15 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
       t[3 * Q] = dt_r * exp2_hw(fminf(__shfl(cs_r, lane | 31, WAVE) - cs_r, 0.0f));
     }
   };
-  const auto frag = [&](const elem_t *tile, int row, int kp) {
-    return load_frag_e<elem_t>(tile + row * 64 + (((2 * kp + g2) ^ (row & 7)) << 3));
-  };
+  const auto frag = [&](const elem_t *tile, int kp) { return load_frag_e<elem_t>(tile + (m * 64 + (((2 * kp + g2) ^ (m >> 1 & 7)) << 3))); };
 
-  f32x16_t M[NR / 2 ? NR / 2 : 1], out = {0};
+  const auto load4 = [](const float *from, float (&v)[4]) {
+    const float4 t = *reinterpret_cast<const float4 *>(from);
+    v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+  };
+  f32x16_t M[MT], out = {0};
 #pragma unroll
-  for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) M[i] = (f32x16_t){0};
+  for (int i = 0; i < MT; ++i) M[i] = (f32x16_t){0};
   const int own_row = 64 * r + 32 * ot + m;                            // of the chunk
   fetch(0);
   put(0);
@@ -119,50 +136,50 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
     const elem_t *own = bufs + at * BUF, *met = own + TILE, *st = met + NR * TILE;
     const float *cs = steps + 4 * at * Q, *l2 = cs + Q, *P = l2 + Q, *R = P + Q;
     const float cs_own = cs[own_row], l2_own = l2[own_row];
-    v8 of[4];
 #pragma unroll
-    for (int kp = 0; kp < 4; ++kp) of[kp] = frag(own, 32 * ot + m, kp);
-#pragma unroll
-    for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) {
-      const int t = k4 + 4 * i, tile = (met0 >> 5) + t, mine = 2 * r + ot;
+    for (int i = 0; i < MT; ++i) {
+      const int t = mw + MW * i, tile = (met0 >> 5) + t, mine = 2 * r + ot;
       if (t < 2 * meets && (for_b ? tile >= mine : tile <= mine)) {
         f32x16_t d = {0};
 #pragma unroll
-        for (int kp = 0; kp < 4; ++kp) d = mma(frag(met, 32 * t + m, kp), of[kp], d);
-        if (tile == mine) {
+        for (int kp = 0; kp < 4; ++kp) d = mma(frag(met + 32 * t * 64, kp), frag(own + 32 * ot * 64, kp), d);
+        // off the diagonal a factor per own row, a scalar per pair of blocks and a factor per met row (ssd_chunk.hpp)
+        const int lb = for_b ? tile : mine, sb = for_b ? mine : tile;
+        float f = 0.0f;
+        int own_lane = m;
+        asm volatile("" : "+v"(own_lane));                               // its 16 comparisons stay here: the scalars are few
+        if (tile != mine) f = (for_b ? R : P)[own_row] * exp2_hw(fminf(cs[32 * lb - 1] - cs[32 * sb + 31], 0.0f));
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int row = 32 * tile + 8 * q + 4 * g2;
-            const float4 c4 = *reinterpret_cast<const float4 *>(cs + row), l4 = *reinterpret_cast<const float4 *>(l2 + row);
-            const float cm[4] = {c4.x, c4.y, c4.z, c4.w}, lm[4] = {l4.x, l4.y, l4.z, l4.w};
+        for (int q = 0; q < 4; ++q) {
+          const int row = 32 * tile + 8 * q + 4 * g2;
+          float w[4];
+          if (tile == mine) {
+            load4(cs + row, w);
+            float l[4];
+            if (!for_b) load4(l2 + row, l);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               // dt_s exp(min(cs_l - cs_s, 0)) as one exponential
-              const float w = for_b ? exp2_hw(fminf(cm[j] - cs_own, 0.0f) + l2_own) : exp2_hw(fminf(cs_own - cm[j], 0.0f) + lm[j]);
-              const bool in = for_b ? row + j >= own_row : row + j <= own_row;
-              M[i][4 * q + j] = __builtin_fmaf(in ? w : 0.0f, d[4 * q + j], M[i][4 * q + j]);
+              w[j] = for_b ? exp2_hw(fminf(w[j] - cs_own, 0.0f) + l2_own) : exp2_hw(fminf(cs_own - w[j], 0.0f) + l[j]);
+              const int at = 8 * q + 4 * g2 + j;
+              w[j] = (for_b ? at >= own_lane : at <= own_lane) ? w[j] : 0.0f;
             }
-          }
-        } else {
-          // off the diagonal a factor per own row, a scalar per pair of blocks and a factor per met row (ssd_chunk.hpp)
-          const int lb = for_b ? tile : mine, sb = for_b ? mine : tile;
-          const float f = (for_b ? R : P)[own_row] * exp2_hw(fminf(cs[32 * lb - 1] - cs[32 * sb + 31], 0.0f));
-          const float *T = (for_b ? P : R) + 32 * tile + 4 * g2;
+          } else {
+            load4((for_b ? P : R) + row, w);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float4 t = *reinterpret_cast<const float4 *>(T + 8 * q);
-            M[i][4 * q] = __builtin_fmaf(t.x * f, d[4 * q], M[i][4 * q]);
-            M[i][4 * q + 1] = __builtin_fmaf(t.y * f, d[4 * q + 1], M[i][4 * q + 1]);
-            M[i][4 * q + 2] = __builtin_fmaf(t.z * f, d[4 * q + 2], M[i][4 * q + 2]);
-            M[i][4 * q + 3] = __builtin_fmaf(t.w * f, d[4 * q + 3], M[i][4 * q + 3]);
+            for (int j = 0; j < 4; ++j) w[j] *= f;
           }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) M[i][4 * q + j] = __builtin_fmaf(w[j], d[4 * q + j], M[i][4 * q + j]);
         }
       }
     }
-    if (k4 < NT) {
+    if (mw < NT) {
       f32x16_t d = {0};
+      int again = 32 * ot * 64;
+      asm volatile("" : "+s"(again));                                    // read a second time, not kept in registers
 #pragma unroll
-      for (int kp = 0; kp < 4; ++kp) d = mma(frag(st, 32 * k4 + m, kp), of[kp], d);
+      for (int kp = 0; kp < 4; ++kp) d = mma(frag(st + 32 * mw * 64, kp), frag(own + again, kp), d);
       const float w = for_b ? exp2_hw(fminf(cs[Q - 1] - cs_own, 0.0f) + l2_own) : exp2_hw(cs_own);
 #pragma unroll
       for (int j = 0; j < 16; ++j) out[j] = __builtin_fmaf(w, d[j], out[j]);
@@ -173,8 +190,8 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
   // ---- M, rounded, as an operand (rows = own, columns = met), times the columns of B (of C)
   elem_t *Ms = bufs;                                                   // [64][Q]
 #pragma unroll
-  for (int i = 0; i < (NR / 2 ? NR / 2 : 1); ++i) {
-    const int t = k4 + 4 * i, row = 32 * ot + m;
+  for (int i = 0; i < MT; ++i) {
+    const int t = mw + MW * i, row = 32 * ot + m;
     if (t < 2 * meets) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -184,21 +201,28 @@ __global__ __launch_bounds__(512) void ssd_dbc_kernel(const SsdDbcParams p) {
     }
   }
   __syncthreads();
-  if (k4 >= NT) return;
-  const elem_t *bt = reinterpret_cast<const elem_t *>(for_b ? p.Ctblk : p.Btblk) + (((size_t)unit * KS + (met0 >> 4)) * NT + k4) * SSD_FRAG + lane * 8;
+  if (mw >= NT) return;
+  const elem_t *bt = reinterpret_cast<const elem_t *>(for_b ? p.Ctblk : p.Btblk) + (((size_t)unit * KS + (met0 >> 4)) * NT + mw) * SSD_FRAG + lane * 8;
   for (int ks = 0; ks < 4 * meets; ++ks) {
     const int row = 32 * ot + m;
     out = mma(load_frag_e<elem_t>(bt + ks * NT * SSD_FRAG),
               load_frag_e<elem_t>(Ms + row * Q + (((2 * ks + g2) ^ (row & QMASK)) << 3)), out);
   }
   if (own_row < rows) {
-    elem_t *dst = (for_b ? p.dB : p.dC) + (((size_t)b * p.len + (size_t)c * Q + own_row) * p.groups + g) * N + 32 * k4 + 4 * g2;
+    elem_t *dst = (for_b ? p.dB : p.dC) + (((size_t)b * p.len + (size_t)c * Q + own_row) * p.groups + g) * N + 32 * mw + 4 * g2;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float v[4] = {out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
       store4_e<elem_t>(dst + 8 * q, v);
     }
   }
+}
+
+template <int Q, int N>
+__global__ __launch_bounds__(64 * DBC_WAVES<Q>) void ssd_dbc_kernel(const SsdDbcParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x & 1) dbc_rows<Q, N, true>(p, smem);
+  else dbc_rows<Q, N, false>(p, smem);
 }
 
 // ---------------------------------------------------------------------- dt
@@ -342,7 +366,7 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
   if (dz.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, true>), units, block, 0, s, dz);
   else hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, false>), units, block, 0, s, dz);
   hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DX, false>), units, block, 0, s, dx);
-  hipLaunchKernelGGL((ssd_dbc_kernel<Q, N>), dim3(2u * bc.units * (Q / 64)), dim3(512), dbc_lds, s, bc);
+  hipLaunchKernelGGL((ssd_dbc_kernel<Q, N>), dim3(2u * bc.units * (Q / 64)), dim3(64 * DBC_WAVES<Q>), dbc_lds, s, bc);
   hipLaunchKernelGGL((ssd_dt_kernel<Q>), dim3((unsigned)(d.batch * d.nchunks * ((d.heads + DT_HEADS - 1) / DT_HEADS))), block, 0, s, dt);
   return SSM_OK;
 }
