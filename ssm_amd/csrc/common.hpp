@@ -161,6 +161,21 @@ __device__ __forceinline__ T *at_bytes(B *base, unsigned bytes) {
   return reinterpret_cast<T *>(reinterpret_cast<C *>(base) + bytes);
 }
 
+// A read of memory that nobody is going to read again soon: it takes no place in the caches from what is written, or waits
+// to be read, beside it.
+template <typename P>
+__device__ __forceinline__ P load_once(const P *p) {
+  constexpr int BYTES = sizeof(P) > 16 ? 16 : sizeof(P);
+  static_assert(BYTES % 4 == 0 && sizeof(P) % BYTES == 0);
+  typedef unsigned words __attribute__((ext_vector_type(BYTES / 4)));
+  words w[sizeof(P) / BYTES];
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(P) / BYTES; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const words *>(p) + i);
+  P v;
+  __builtin_memcpy(&v, w, sizeof(P));
+  return v;
+}
+
 // A lane's run of K steps of a row of `len` steps.  RAGGED = false: rows start on 16-byte boundaries and are whole runs
 // long (and shorter than 2^29 steps), so a run is inside or outside as a whole (outside: some run of the row is read; the
 // caller masks its steps).

@@ -34,8 +34,16 @@ struct NormParams {
   int rows, hidden;
   int x_dtype, res_dtype, res_out_dtype, gro_dtype;
   int is_rms, prenorm;
+  int past_caches;                  // typed kernels: how to read what is not read again (NORM_CACHED)
   float eps;
 };
+
+// Elements up to which a call's tensors are left to the caches.  Larger calls read what is not read again past them (the
+// forward its residual, the backward all it reads): the space is better spent on what is written, for those who read that.
+// Forward and backward, bf16 with a float32 residual and gradient through it, us without / with: 2048 x 768 16.6 / 17.4,
+// 2048 x 2560 36 / 40, 4 x 2048 x 768 43.2 / 42.1, 8 x 2048 x 768 75.5 / 70.1, 16 x 2048 x 768 149 / 136 (the
+// forward's x past the caches too: 137; what is written past them: slower).
+constexpr size_t NORM_CACHED = (size_t)5632 << 10;
 
 __device__ __forceinline__ void store_f32_as(void *p, int dtype, size_t i, float v) {
   if (dtype == SSM_F32) reinterpret_cast<float *>(p)[i] = v;
@@ -183,6 +191,7 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_kernel(const NormParams p
 // unconditional - column indices are clamped into the row, an absent residual or bias reads a stand-in of
 // the same type whose value is dropped - so a wavefront's reads are in flight together instead of one
 // behind the other, which is what a call on a handful of rows (a decoding step) waits for.
+// Past NORM_CACHED the residual is read past the caches: what a backward reads again is x.
 template <typename T, int VEC>
 __device__ __forceinline__ void ld_pack(const void *p, size_t i, float (&v)[VEC]) {
   const Pack<T, VEC> raw = *reinterpret_cast<const Pack<T, VEC> *>(reinterpret_cast<const T *>(p) + i);
@@ -197,6 +206,12 @@ __device__ __forceinline__ void st_pack(void *p, size_t i, const float (&v)[VEC]
   *reinterpret_cast<Pack<T, VEC> *>(reinterpret_cast<T *>(p) + i) = raw;
 }
 
+template <typename T, int VEC>
+__device__ __forceinline__ void ld_once(const void *p, size_t i, float (&v)[VEC]) {
+  const Pack<T, VEC> raw = load_once(reinterpret_cast<const Pack<T, VEC> *>(reinterpret_cast<const T *>(p) + i));
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) v[j] = to_f32(raw.v[j]);
+}
 template <int TRIPS, bool WG, typename XT, typename RT>
 __global__ __launch_bounds__(LN_THREADS) void norm_fwd_typed_kernel(const NormParams p) {
   constexpr int VEC = 4;
@@ -218,7 +233,10 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_typed_kernel(const NormPa
     const int colc = min((k * OWNERS + lane) * VEC, H - VEC);
     ld_pack<XT, VEC>(p.x, base + colc, v[k]);
   }
-  if (has_res) {                 // one test in front of all of a row's residual reads, none between them
+  if (has_res && p.past_caches) {                 // one test in front of all of a row's residual reads, none between them
+#pragma unroll
+    for (int k = 0; k < TRIPS; ++k) ld_once<RT, VEC>(resp, base + min((k * OWNERS + lane) * VEC, H - VEC), r[k]);
+  } else if (has_res) {
 #pragma unroll
     for (int k = 0; k < TRIPS; ++k) ld_pack<RT, VEC>(resp, base + min((k * OWNERS + lane) * VEC, H - VEC), r[k]);
   } else {
@@ -355,6 +373,17 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_long_kernel(const NormPar
 
 // ----------------------------------------------------------------- backward
 
+// The words of a pack as they stand here: what is made of them further on is made there, not kept from before.
+template <typename T, int VEC>
+__device__ __forceinline__ void pin_pack(Pack<T, VEC> &v) {
+  static_assert(sizeof(v) % 4 == 0);
+  unsigned w[sizeof(v) / 4];
+  __builtin_memcpy(w, &v, sizeof(v));
+#pragma unroll
+  for (unsigned &x : w) asm volatile("" : "+v"(x));
+  __builtin_memcpy(&v, w, sizeof(v));
+}
+
 // Each wave handles rows wave_global, wave_global + nwaves, ...; columns are
 // owned by (lane, trip) exactly as in the forward kernel.
 // XT = void: element types looked up at run time.  Otherwise x, dy, dx have type XT, residual and dresidual
@@ -364,15 +393,26 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_long_kernel(const NormPar
 // GRO (typed form): the gradient that arrives through residual_out = x (+ residual), of type RT, is added to dx and
 // dresidual while they are in registers.  The pass is bound by memory; added in launches of its own, that gradient
 // cost a (16 x 2048 x 768) bf16 step with a float32 residual 106 us beside the 66 of this kernel.
+//
+// Bound by memory: 16 x 2048 x 768, bf16 with a float32 residual and gradient through it, 400 MB, 74 us.  Before, 98 with
+// 50 for the forward's 300 MB, now 63: what the backward no longer leaves in the caches the forward has to write out itself;
+// together they are at the rate of a large copy.
+// The grid is held to the workgroups that the registers let onto the chip at once (with four to a CU for any width, the
+// fourth of three ran alone), and the registers are few: words as they came, 32-bit offsets from a scalar row, no value kept
+// that can be formed again.  Forward and backward, 4096 rows of 4096 columns 107 -> 95 us, of 8192 223 -> 197.
+constexpr int norm_bwd_resident(int trips, bool gro) {                   // workgroups to a CU of a typed kernel
+  return trips <= 2 ? 4 : trips == 3 ? (gro ? 3 : 4) : trips == 4 ? (gro ? 2 : 3) : trips == 5 ? 2 : trips == 6 ? (gro ? 1 : 2) : 1;
+}
 template <int TRIPS, bool WG, typename XT = void, typename RT = void, bool GRO = false>
-__global__ __launch_bounds__(LN_THREADS) void norm_bwd_kernel(const NormParams p, int vec_ok) {
+__global__ __launch_bounds__(LN_THREADS) __attribute__((amdgpu_waves_per_eu(std::is_void<XT>::value ? 1 : norm_bwd_resident(TRIPS, GRO))))
+void norm_bwd_kernel(const NormParams p, int vec_ok) {
   constexpr int VEC = 4;
   constexpr bool TYPED = !std::is_void<XT>::value;
   using xt = typename std::conditional<TYPED, XT, float>::type;
   using rt = typename std::conditional<TYPED, RT, float>::type;
   constexpr int OWNERS = WG ? LN_THREADS : WAVE;       // threads that share a row
   __shared__ float red[LN_WAVES];
-  const int wave = threadIdx.x >> 6, lane = WG ? (int)threadIdx.x : (int)(threadIdx.x & 63);
+  const int wave = wave_id_uniform(), lane = WG ? (int)threadIdx.x : (int)(threadIdx.x & 63);
   const int nwaves = WG ? (int)gridDim.x : (int)(gridDim.x * LN_WAVES);      // row owners in the grid
   const int gw = WG ? (int)blockIdx.x : (int)(blockIdx.x * LN_WAVES + wave);
   const int H = p.hidden;
@@ -397,18 +437,27 @@ __global__ __launch_bounds__(LN_THREADS) void norm_bwd_kernel(const NormParams p
     float mean = meanp[row];
     if (p.is_rms) mean = 0.0f;
     const float rstd = p.rstd[row];
-    float xh[TRIPS][VEC], g[TRIPS][VEC], dyv[TRIPS][VEC];
+    float xh[TRIPS][VEC], g[TRIPS][VEC], dyv[TRIPS][VEC], gin[TRIPS][VEC];
     float s1 = 0.0f, s2 = 0.0f;     // sum g*xhat, sum g
-    float vin[TRIPS][VEC], rin[TRIPS][VEC], gin[TRIPS][VEC];
+    Pack<xt, VEC> xr[TRIPS], dyr[TRIPS];
+    Pack<rt, VEC> rr[TRIPS], gr[TRIPS];
     if constexpr (TYPED) {
+      const auto read = [&](auto past) {
+        const auto get = [&](const auto *q) {
+          if constexpr (past.value) return load_once(q);
+          else return *q;
+        };
 #pragma unroll
-      for (int k = 0; k < TRIPS; ++k) {
-        const int colc = min((k * OWNERS + lane) * VEC, H - VEC);
-        ld_pack<xt, VEC>(p.x, base + colc, vin[k]);
-        ld_pack<rt, VEC>(resp, base + colc, rin[k]);
-        ld_pack<xt, VEC>(p.dy, base + colc, dyv[k]);
-        if constexpr (GRO) ld_pack<rt, VEC>(p.gro, base + colc, gin[k]);
-      }
+        for (int k = 0; k < TRIPS; ++k) {
+          const unsigned colc = (unsigned)min((k * OWNERS + lane) * VEC, H - VEC);
+          xr[k] = get(at_bytes<const Pack<xt, VEC>>(reinterpret_cast<const xt *>(p.x) + base, colc * (unsigned)sizeof(xt)));
+          rr[k] = get(at_bytes<const Pack<rt, VEC>>(reinterpret_cast<const rt *>(resp) + base, colc * (unsigned)sizeof(rt)));
+          dyr[k] = get(at_bytes<const Pack<xt, VEC>>(reinterpret_cast<const xt *>(p.dy) + base, colc * (unsigned)sizeof(xt)));
+          if constexpr (GRO) gr[k] = get(at_bytes<const Pack<rt, VEC>>(reinterpret_cast<const rt *>(p.gro) + base, colc * (unsigned)sizeof(rt)));
+        }
+      };
+      if (p.past_caches) read(std::true_type{});
+      else read(std::false_type{});
     }
 #pragma unroll
     for (int k = 0; k < TRIPS; ++k) {
@@ -416,7 +465,11 @@ __global__ __launch_bounds__(LN_THREADS) void norm_bwd_kernel(const NormParams p
       float v[VEC];
       if constexpr (TYPED) {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) v[i] = has_add ? vin[k][i] + rin[k][i] : vin[k][i];
+        for (int i = 0; i < VEC; ++i) {
+          v[i] = to_f32(xr[k].v[i]);
+          if (has_add) v[i] += to_f32(rr[k].v[i]);
+          dyv[k][i] = to_f32(dyr[k].v[i]);
+        }
       } else {
         load_cols<VEC>(p.x, p.x_dtype, base, col, H, vok, v);
         if (has_add) {
@@ -445,6 +498,15 @@ __global__ __launch_bounds__(LN_THREADS) void norm_bwd_kernel(const NormParams p
       const int col = (k * OWNERS + lane) * VEC;
       if (col >= H) continue;
       float dxv[VEC];
+      if constexpr (TYPED) {
+        pin_pack(dyr[k]);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+          dyv[k][i] = to_f32(dyr[k].v[i]);
+          g[k][i] = dyv[k][i] * wv[k][i];
+          if constexpr (GRO) gin[k][i] = to_f32(gr[k].v[i]);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < VEC; ++i) dxv[i] = (g[k][i] - c2 - xh[k][i] * c1) * rstd;
       if constexpr (!TYPED) {
@@ -455,8 +517,8 @@ __global__ __launch_bounds__(LN_THREADS) void norm_bwd_kernel(const NormParams p
         for (int i = 0; i < VEC; ++i) dxv[i] += gin[k][i];
       }
       if constexpr (TYPED) {
-        st_pack<xt, VEC>(p.dx, base + col, dxv);
-        if (p.dres) st_pack<rt, VEC>(p.dres, base + col, p.prenorm ? dxv : dyv[k]);
+        st_pack<xt, VEC>(reinterpret_cast<xt *>(p.dx) + base, (unsigned)col, dxv);
+        if (p.dres) st_pack<rt, VEC>(reinterpret_cast<rt *>(p.dres) + base, (unsigned)col, p.prenorm ? dxv : dyv[k]);
       } else {
         store_cols<VEC>(p.dx, p.x_dtype, base, col, H, vok, dxv);
         if (p.dres) store_cols<VEC>(p.dres, p.res_dtype, base, col, H, vok, p.prenorm ? dxv : dyv[k]);
@@ -631,6 +693,7 @@ extern "C" int ssm_norm_fwd(const ssm_norm_fwd_args *a, void *hip_stream) {
   p.mean = a->mean; p.rstd = a->rstd;
   p.rows = a->rows; p.hidden = a->hidden;
   p.x_dtype = a->x_dtype; p.res_dtype = a->residual_dtype; p.res_out_dtype = a->residual_out_dtype;
+  p.past_caches = (size_t)a->rows * a->hidden > NORM_CACHED;
   p.is_rms = a->is_rms ? 1 : 0; p.prenorm = a->prenorm ? 1 : 0; p.eps = a->eps;
   const int vec_ok = a->hidden % 4 == 0 && aligned_to(a->x, 16) && aligned_to(a->y, 16) &&
                      aligned_to(a->weight, 16) && (!a->bias || aligned_to(a->bias, 16)) &&
@@ -657,26 +720,32 @@ extern "C" int ssm_norm_fwd(const ssm_norm_fwd_args *a, void *hip_stream) {
 }
 
 namespace ssm {
+// The typed kernels; the workgroups launched, at most `grid`.
+template <int TRIPS, bool WG, typename XT, typename RT, bool GRO>
+static int launch_norm_bwd_trips(const NormParams &p, int grid, hipStream_t s) {
+  const int resident = 256 * norm_bwd_resident(TRIPS, GRO), g = grid < resident ? grid : resident;
+  hipLaunchKernelGGL((norm_bwd_kernel<TRIPS, WG, XT, RT, GRO>), dim3(g), dim3(LN_THREADS), 0, s, p, 1);
+  return g;
+}
 template <typename XT, typename RT, bool GRO>
-static void launch_norm_bwd_gro(const NormParams &p, int hidden, int grid, hipStream_t s) {
+static int launch_norm_bwd_gro(const NormParams &p, int hidden, int grid, hipStream_t s) {
   const int per_lane = (hidden + WAVE - 1) / WAVE;
-  const dim3 g(grid), b(LN_THREADS);
-  if (per_lane <= 4) hipLaunchKernelGGL((norm_bwd_kernel<1, false, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (per_lane <= 8) hipLaunchKernelGGL((norm_bwd_kernel<2, false, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (per_lane <= 12) hipLaunchKernelGGL((norm_bwd_kernel<3, false, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (hidden <= 1024) hipLaunchKernelGGL((norm_bwd_kernel<1, true, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (hidden <= 2048) hipLaunchKernelGGL((norm_bwd_kernel<2, true, XT, RT, GRO>), g, b, 0, s, p, 1);
+  if (per_lane <= 4) return launch_norm_bwd_trips<1, false, XT, RT, GRO>(p, grid, s);
+  if (per_lane <= 8) return launch_norm_bwd_trips<2, false, XT, RT, GRO>(p, grid, s);
+  if (per_lane <= 12) return launch_norm_bwd_trips<3, false, XT, RT, GRO>(p, grid, s);
+  if (hidden <= 1024) return launch_norm_bwd_trips<1, true, XT, RT, GRO>(p, grid, s);
+  if (hidden <= 2048) return launch_norm_bwd_trips<2, true, XT, RT, GRO>(p, grid, s);
   // a thread's registers grow with the trips it is compiled for: the widths of common models (2560, 5120) get
   // their own count rather than the next power of two
-  else if (hidden <= 3072) hipLaunchKernelGGL((norm_bwd_kernel<3, true, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (hidden <= 4096) hipLaunchKernelGGL((norm_bwd_kernel<4, true, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (hidden <= 5120) hipLaunchKernelGGL((norm_bwd_kernel<5, true, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else if (hidden <= 6144) hipLaunchKernelGGL((norm_bwd_kernel<6, true, XT, RT, GRO>), g, b, 0, s, p, 1);
-  else hipLaunchKernelGGL((norm_bwd_kernel<8, true, XT, RT, GRO>), g, b, 0, s, p, 1);
+  if (hidden <= 3072) return launch_norm_bwd_trips<3, true, XT, RT, GRO>(p, grid, s);
+  if (hidden <= 4096) return launch_norm_bwd_trips<4, true, XT, RT, GRO>(p, grid, s);
+  if (hidden <= 5120) return launch_norm_bwd_trips<5, true, XT, RT, GRO>(p, grid, s);
+  if (hidden <= 6144) return launch_norm_bwd_trips<6, true, XT, RT, GRO>(p, grid, s);
+  return launch_norm_bwd_trips<8, true, XT, RT, GRO>(p, grid, s);
 }
 template <typename XT, typename RT>
-static void launch_norm_bwd_typed(const NormParams &p, int hidden, int grid, hipStream_t s) {
-  p.gro ? launch_norm_bwd_gro<XT, RT, true>(p, hidden, grid, s) : launch_norm_bwd_gro<XT, RT, false>(p, hidden, grid, s);
+static int launch_norm_bwd_typed(const NormParams &p, int hidden, int grid, hipStream_t s) {
+  return p.gro ? launch_norm_bwd_gro<XT, RT, true>(p, hidden, grid, s) : launch_norm_bwd_gro<XT, RT, false>(p, hidden, grid, s);
 }
 }  // namespace ssm
 
@@ -715,21 +784,22 @@ static int norm_bwd_launch(const ssm_norm_bwd_args *a, float *partial, void *hip
   p.rows = a->rows; p.hidden = a->hidden;
   p.x_dtype = a->x_dtype; p.res_dtype = a->residual_dtype;
   p.gro = a->grad_residual_out; p.gro_dtype = a->grad_residual_out_dtype;
+  p.past_caches = (size_t)a->rows * a->hidden > NORM_CACHED;
   p.is_rms = a->is_rms ? 1 : 0; p.prenorm = a->prenorm ? 1 : 0;
   const int vec_ok = a->hidden % 4 == 0 && aligned_to(a->x, 16) && aligned_to(a->dy, 16) && aligned_to(a->dx, 16) &&
                      aligned_to(a->weight, 16) && (!a->residual || aligned_to(a->residual, 16)) &&
                      (!a->dresidual || aligned_to(a->dresidual, 16)) &&
                      (!a->grad_residual_out || aligned_to(a->grad_residual_out, 16));
   hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
-  const int grid = norm_bwd_grid(a->rows);
+  int grid = norm_bwd_grid(a->rows);
   const int per_lane = (a->hidden + WAVE - 1) / WAVE;
   // typed kernels: one element type RT (float32 or that of x) for residual, dresidual and grad_residual_out
   const int rt = (a->residual || a->dresidual) ? a->residual_dtype : p.gro ? p.gro_dtype : a->x_dtype;
   if (vec_ok && a->hidden >= 4 && a->hidden <= 8192 && (rt == SSM_F32 || rt == a->x_dtype) && (!p.gro || p.gro_dtype == rt)) {
     const bool rf = rt == SSM_F32;
-    if (a->x_dtype == SSM_BF16) rf ? launch_norm_bwd_typed<bf16_t, float>(p, a->hidden, grid, s) : launch_norm_bwd_typed<bf16_t, bf16_t>(p, a->hidden, grid, s);
-    else if (a->x_dtype == SSM_F16) rf ? launch_norm_bwd_typed<f16_t, float>(p, a->hidden, grid, s) : launch_norm_bwd_typed<f16_t, f16_t>(p, a->hidden, grid, s);
-    else launch_norm_bwd_typed<float, float>(p, a->hidden, grid, s);
+    if (a->x_dtype == SSM_BF16) grid = rf ? launch_norm_bwd_typed<bf16_t, float>(p, a->hidden, grid, s) : launch_norm_bwd_typed<bf16_t, bf16_t>(p, a->hidden, grid, s);
+    else if (a->x_dtype == SSM_F16) grid = rf ? launch_norm_bwd_typed<f16_t, float>(p, a->hidden, grid, s) : launch_norm_bwd_typed<f16_t, f16_t>(p, a->hidden, grid, s);
+    else grid = launch_norm_bwd_typed<float, float>(p, a->hidden, grid, s);
   }
   else if (per_lane <= 4) hipLaunchKernelGGL((norm_bwd_kernel<1, false>), dim3(grid), dim3(LN_THREADS), 0, s, p, vec_ok);
   else if (per_lane <= 8) hipLaunchKernelGGL((norm_bwd_kernel<2, false>), dim3(grid), dim3(LN_THREADS), 0, s, p, vec_ok);

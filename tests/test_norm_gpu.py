@@ -179,3 +179,30 @@ def test_gradient_through_residual_out_is_added_in_the_backward_kernel(dtype, re
     for a, b, t in zip(got, want, (x, r)):
         tol = 1e-5 if t.dtype == torch.float32 else 2e-2
         torch.testing.assert_close(a.double().cpu(), b, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("dtype,res_dtype,hidden", [
+    (torch.bfloat16, torch.float32, 768), (torch.float16, torch.float16, 2560), (torch.float32, torch.float32, 5120),
+    (torch.bfloat16, torch.float32, 6148)])
+def test_rows_of_a_large_call_are_those_of_its_halves(dtype, res_dtype, hidden):
+    """Large calls read past the caches; a row does not depend on the others, so its results are the same to the bit."""
+    rows = (3 << 20) // hidden                               # twice that: more elements than the caches are left, once: fewer
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, r, w = rand(2, rows, hidden).to(dtype), rand(2, rows, hidden).to(res_dtype), rand(hidden)
+    go, gr = rand(2, rows, hidden).to(dtype), rand(2, rows, hidden).to(res_dtype)
+
+    def run(part):
+        leaves = [x[part].clone().requires_grad_(), r[part].clone().requires_grad_(), w.clone().requires_grad_()]
+        y, out = _ops().fused_layer_norm_with_residual(leaves[0], leaves[2], None, residual=leaves[1], is_rms=True, eps=1e-5,
+                                                       prenorm=True, residual_in_fp32=res_dtype == torch.float32)
+        torch.autograd.backward([y, out], [go[part], gr[part]])
+        return [y.detach(), out.detach()] + [t.grad for t in leaves]
+
+    whole, halves = run(slice(None)), [run(slice(0, 1)), run(slice(1, 2))]
+    for i in range(4):
+        torch.testing.assert_close(whole[i], torch.cat([h[i] for h in halves]), rtol=0, atol=0)
+    # the weight's gradient: sums of 2 `rows` products, any order off by at most 2 rows 2^-24 of the sum of their sizes
+    v = x.double() + r.double()
+    bound = 2 * rows * 2.0 ** -23 * (go.double() * v * (v * v).mean(-1, keepdim=True).add(1e-5).rsqrt()).abs().sum((0, 1))
+    assert ((whole[4] - halves[0][4] - halves[1][4]).abs().double() <= bound).all()
