@@ -38,7 +38,7 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 // Steps past the end of a last chunk that is no whole one: size zero, rows of B and C zero.
 // What bounds it is the lines of B, C and dt that each workgroup touches: 4 x 2048 steps, 24 heads, everything a backward
 // needs, 14.5 us (17.3 with 64-bit divisions per wave and neighbours on different XCDs); 4 x 4096 steps, 80 heads, for the
-// walk, 15.2 (16.0).
+// walk, 14.7 (16.0).
 // The walk takes the last two roles with chunks of 32 steps, and a fragment of C with its states in the order in which
 // an accumulator's registers hold rows: (lane, j) = state 16 kn + 4 (lane / 32) + j, 8 further for j >= 4.
 constexpr int PD_HEADS = 4, PW_HEADS = 32;     // heads of a workgroup of either dt role
@@ -117,7 +117,22 @@ __device__ __forceinline__ void prep_dt_role(const SsdPrepParams &pp, unsigned w
   }
 }
 
+// 64 steps of 32 heads of dt, from (row, h0) on, into LDS as [head][65]; past the last step or head some other value.  A
+// thread's reads are in flight together: the type is looked up once, not in front of each of them.
+template <typename T>
+__device__ __forceinline__ void stage_walk_dt(const void *dt, size_t row, int steps, int h0, int heads, float *tile) {
+  T raw[PW_HEADS / 4];
+  const int hh = (int)threadIdx.x % PW_HEADS, l0 = (int)threadIdx.x / PW_HEADS;
+  const T *from = reinterpret_cast<const T *>(dt) + row * heads + min(h0 + hh, heads - 1);
+#pragma unroll
+  for (int i = 0; i < PW_HEADS / 4; ++i) raw[i] = from[(size_t)min(l0 + 8 * i, steps - 1) * heads];
+#pragma unroll
+  for (int i = 0; i < PW_HEADS / 4; ++i) tile[hh * 65 + l0 + 8 * i] = to_f32(raw[i]);
+}
+
 // For the walk: two blocks of 32 heads, whose 64 bytes of a row are read together.
+// Bound by latency: 80 heads of 512 steps 4.8 us for the launch, 24 heads of 256 5.3 (8.5 and 6.8 with the reads of dt, A and
+// bias one behind the other).
 __device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
   float (*tile)[64 + 1] = reinterpret_cast<float (*)[64 + 1]>(lds);
   const SsdCumsumParams &p = pp.cs;
@@ -125,23 +140,25 @@ __device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsig
   const unsigned turns = (unsigned)ssd_walk_turns(d.nchunks), hgroups = (unsigned)(d.heads + PW_HEADS - 1) / PW_HEADS, rest = wg / hgroups;
   const int h0 = (int)(wg - rest * hgroups) * PW_HEADS, b = (int)(rest / (turns >> 1)), unit = (int)(rest - b * (turns >> 1));
   const int l0 = 64 * unit;
-#pragma unroll
-  for (int e = (int)threadIdx.x; e < 64 * PW_HEADS; e += 256) {
-    const int l = e / PW_HEADS, hh = e % PW_HEADS;
-    float v = 0.0f;
-    if (h0 + hh < d.heads && l0 + l < d.len) v = load_as_f32(p.dt, p.dt_dtype, ((size_t)b * d.len + l0 + l) * d.heads + h0 + hh);
-    tile[hh][l] = v;
+  const int wave = wave_id_uniform(), lane = lane_id();
+  // lane k: what this wave's k-th head multiplies and adds
+  const int lane_h = min(h0 + 4 * (lane % (PW_HEADS / 4)) + wave, d.heads - 1);
+  const float A_lanes = p.A[lane_h], bias_lanes = p.bias ? p.bias[lane_h] : 0.0f;
+  if (l0 < d.len) {
+    const size_t row = (size_t)b * d.len + l0;
+    if (p.dt_dtype == SSM_F32) stage_walk_dt<float>(p.dt, row, d.len - l0, h0, d.heads, lds);
+    else if (p.dt_dtype == SSM_BF16) stage_walk_dt<bf16_t>(p.dt, row, d.len - l0, h0, d.heads, lds);
+    else stage_walk_dt<f16_t>(p.dt, row, d.len - l0, h0, d.heads, lds);
   }
   __syncthreads();
-  const int wave = wave_id_uniform(), lane = lane_id();
   const bool live = l0 + lane < d.len;               // steps past the end have size zero
   const float jump = pp.seq_idx && live ? sequence_jump(pp, b, (size_t)l0 + lane) : 0.0f;
 #pragma unroll 2
   for (int k = 0; k < PW_HEADS / 4; ++k) {
-    const int hh = wave * (PW_HEADS / 4) + k, h = h0 + hh;
+    const int hh = 4 * k + wave, h = h0 + hh;
     if (h >= d.heads) return;
-    const float v = live ? prep_step(p, tile[hh][lane] + (p.bias ? p.bias[h] : 0.0f)) : 0.0f;
-    const float cs = half_wave_inclusive_sum(__builtin_fmaf(v, p.A[h], jump)) * LOG2E;
+    const float v = live ? prep_step(p, tile[hh][lane] + wave_read_lane(bias_lanes, k)) : 0.0f;
+    const float cs = half_wave_inclusive_sum(__builtin_fmaf(v, wave_read_lane(A_lanes, k), jump)) * LOG2E;
     const float end = lane < SSD_WALK_BLOCK ? wave_read_lane(cs, SSD_WALK_BLOCK - 1) : wave_read_lane(cs, 2 * SSD_WALK_BLOCK - 1);
     const size_t at = ((size_t)b * d.heads + h) * turns + 2 * unit;           // block
     reinterpret_cast<float2 *>(pp.steps)[at * SSD_WALK_BLOCK + lane] = make_float2(cs - 0.5f * end, v);
