@@ -1,29 +1,37 @@
 // Forward launches of the side-by-side SSD (ssd_chunk.hpp).
 #include "ssd_chunk.hpp"
+#include <algorithm>
 
 namespace ssm {
 
 // One walk over the sequence (the state never leaves the chip; a workgroup per head, or per two, so few heads leave CUs idle)
 // or the chunks side by side (states through memory, twice x)?  Both times in us, heads counted over the batch.  The walk
 // takes a time per block of 32 steps that grows with the heads that share memory, and above 256 heads, two to a workgroup,
-// faster; 512 fill the chip.  The workgroups of the other way (one per chunk and head) take a fixed share of the chip each.
-// Fitted to both routes at 210 sizes (24 to 640 heads, 256 to 8192 steps, each chunk length and state size):
-//   heads, 4096 steps, 128 states:       24         64         96         128        160        256        320        400
-//   walk / side by side, chunks of 256: 109 / 41   110 / 67   114 / 97   118 / 125  120 / 152  146 / 244  192 / 289  211 / 356
-// Up to two chunks the walk is always the faster one (24 heads, 512 steps: 21 / 24).
+// faster; 512 fill the chip.  The workgroups of the other way (one per chunk and head) share it, a little better while they
+// all fit.  Fitted to both routes, replayed as graphs, at 350 sizes (8 to 400 heads, 256 to 4096 steps):
+//   heads, 4096 steps, 128 states:       24         48         80         112        128        160        256        400
+//   walk / side by side, chunks of 256: 109 / 38   110 / 53   113 / 83   115 / 109  122 / 128  119 / 151  139 / 243  192 / 352
+// Up to two chunks the walk is always the faster one (24 heads, 512 steps: 20.8 / 23.7).
 bool ssd_side_by_side(const SsdDims &d) {
   // the walk's offsets from the start of a head have 32 bits, some blocks past its end included
   if ((size_t)(d.len + 512) * d.heads * SSD_P * 2 >= (size_t)1 << 31) return true;
-  static const double unit_us[3][2] = {{0.0167, 0.0264}, {0.0262, 0.0355}, {0.0421, 0.0536}};   // chunks of 64, 128, 256 steps; 64, 128 states
+  struct Chunks { double start, each, more, from; };         // `more` for each workgroup after the first `from`
+  static const Chunks chunks[3][2] = {{{16.0, 0.0135, 0.0060, 2300.0}, {20.0, 0.0175, 0.0116, 1600.0}},      // of 64 steps; 64, 128 states
+                                      {{16.0, 0.0195, 0.0075, 1280.0}, {18.0, 0.0255, 0.0120, 1280.0}},
+                                      {{20.5, 0.0295, 0.0145, 640.0}, {22.5, 0.0385, 0.0150, 640.0}}};
   const bool large = d.nstate > 64;
   const auto block_us = [&](int64_t n) {
     if (n == 0) return 0.0;
-    if (n <= 256) return large ? 0.77 + 0.0012 * (double)n : 0.62 + 0.0010 * (double)n;
-    return large ? 0.68 + 0.0024 * (double)n : 0.55 + 0.0020 * (double)n;
+    const double share = std::max(0.0, (double)n - 192.0);
+    if (n <= 256) return large ? 0.775 + 0.0005 * (double)n + 0.0018 * share : 0.62 + 0.0005 * (double)n + 0.0012 * share;
+    return large ? 0.77 + 0.0016 * (double)n : 0.72 + 0.0012 * (double)n;
   };
   const int64_t heads = (int64_t)d.batch * d.heads;
-  const double walk = 7.5 + ssd_walk_turns(ssd_walk_blocks(d.len)) * ((double)(heads / 512) * block_us(512) + block_us(heads % 512));
-  return d.nchunks > 2 && walk > 16.0 + unit_us[d.chunk > 128 ? 2 : d.chunk > 64][large] * (double)heads * d.nchunks;
+  const double start = heads > 256 ? (large ? 12.7 : 10.0) : large ? 8.7 : 7.7;
+  const double walk = start + ssd_walk_turns(ssd_walk_blocks(d.len)) * ((double)(heads / 512) * block_us(512) + block_us(heads % 512));
+  const Chunks &c = chunks[d.chunk > 128 ? 2 : d.chunk > 64][large];
+  const double units = (double)heads * d.nchunks;
+  return d.nchunks > 2 && walk > c.start + c.each * units + c.more * std::max(0.0, units - c.from);
 }
 
 template <typename E, int Q, int N>
