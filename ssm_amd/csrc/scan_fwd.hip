@@ -17,15 +17,22 @@ extern template int scan_fwd_fast_dispatch<f16_t, float>(const ScanFwdParams &, 
 
 // Rows up to which the chunks of a row run side by side in one workgroup (scan_fwd_split.hpp) rather than in turn; us at
 // 16 states in turn / side by side:
-//   grouped, 512 x 2048 float32 31.7 / 15.0, 1024 x 2048 38.3 / 25.9, 1024 x 8192 144 / 130, 1536 x 4096 76.5 / 101;
-//   bf16 512 x 2048 32.2 / 13.8, 1536 x 2048 34.3 / 30.0, 1536 x 8192 145 / 128, 2048 x 8192 150 / 152.
-//   Every wave reads B and C itself there, and runs of odd rows at a lower rate: 1024 x 2047 39 / 47, 512 x 2047 33 / 23.
-//   A group per channel: 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
+//   grouped, float32, 512 x 2048 31.7 / 15.0, 768 x 8192 109 / 93, 1024 x 2048 30.7 / 25.7, 1024 x 4096 58 / 67,
+//   1280 x 2048 32 / 29.9, 1536 x 1024 18.1 / 16.7, 1536 x 2048 32.8 / 33.7;
+//   bf16 512 x 2048 32.2 / 13.8, 1280 x 1024 16.6 / 14.3, 1280 x 8192 104 / 93.5, 1536 x 1024 16.6 / 17.2,
+//   1536 x 2048 29.0 / 27.7, 1536 x 4096 56 / 59.
+//   Every wave reads B and C itself there, and runs of odd rows at a lower rate: float32 512 x 2047 33 / 23, 768 x 2047
+//   33 / 42, bf16 768 x 2047 32 / 27, 768 x 1021 18.6 / 19.5, 768 x 3000 48 / 67.
+//   Few channels to a group (a row per wave in turn): 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
 //   Constant projections: 256 x 2048 18.4 / 10.2, 512 x 8192 68 / 43, 512 x 1024 10.6 / 10.9, 1024 x 4096 41 / 43.
-static bool scan_fwd_splits(size_t rows, int len, bool varying, bool half, bool ragged) {
+static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged) {
   if (len <= FAST_T) return false;
   if (!varying) return rows <= (len > 2 * FAST_T ? 512 : 384);
-  return rows <= (ragged ? 512 : half ? 1536 : 1024);
+  const bool to_four = len > 2 * FAST_T && len <= 4 * FAST_T;       // chunks
+  if (ragged) return rows <= (grouped && half && to_four ? 768 : 512);
+  if (!grouped) return rows <= (half ? 1536 : 1024);
+  if (half) return rows <= (to_four ? 1536 : 1280);
+  return rows <= (len <= 2 * FAST_T ? 1536 : len <= 4 * FAST_T ? 1280 : 768);
 }
 
 static bool valid_kind(int k) { return k == SSM_PROJ_DN || k == SSM_PROJ_BDN || k == SSM_PROJ_BGNL; }
@@ -100,7 +107,7 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   p.ragged = const_ok ? !(p.vec_ok && a->seqlen % 8 == 0 && a->seqlen < (1 << 29)) : !whole_rows;
   const bool in_turn = tune >= 200000;      // a selector of 200000 + v: variant v, a row's chunks in turn however few the rows are
   if (in_turn) tune -= 100000;
-  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, a->io_dtype != SSM_F32, p.ragged);
+  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, per_b % 8 == 0 && per_c % 8 == 0, a->io_dtype != SSM_F32, p.ragged);
   // Rows of at most 256 steps fill half a chunk there; the general kernel, which has chunks of 256, keeps them (6720 rows of
   // 256 bf16 20 us against 33) unless every channel has its own projections: 58 against 26 us, of 195 119 against 63.
   if (tune == 0 && fast_ok && (a->seqlen > 256 || (per_b == 1 && per_c == 1))) {
@@ -117,6 +124,9 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
       const int per_wg = scan_fwd_fast_rows(pref[i]);
       if (per_b % per_wg == 0 && per_c % per_wg == 0 && (total / per_wg >= 256 || i == 2)) pick = pref[i];
     }
+    // its rows by two waves each where that leaves a CU no more than one such workgroup and there are chunks to walk: 1920
+    // rows, us with one / two, 1024 steps 19.1 / 18.8, 2048 40.4 / 33.6, 8192 139 / 112, bf16 17.0 / 16.8, 32.1 / 29.3, 129 / 106
+    if (pick == 11082 && total <= 2048 && a->seqlen > 2 * FAST_T) pick = 11162;
     // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave, which reads its runs of
     // B and C as 16-byte vectors
     if (!pick) pick = 31041;

@@ -68,6 +68,30 @@ def test_many_rows_of_odd_length_walk_their_chunks_in_turn():
         torch.testing.assert_close(a[:1], b, rtol=1e-4, atol=2e-5 * scale, msg=lambda m: f"{what}: {m}")
 
 
+@pytest.mark.parametrize("batch,dim,length,nstate,dtype", [
+    (3, 344, 1543, 16, torch.float32), (2, 648, 4112, 16, torch.float32), (2, 1016, 1040, 5, torch.float32),
+    (2, 800, 2064, 16, torch.bfloat16), (2, 496, 1537, 9, torch.float16), (2, 1024, 2063, 16, torch.bfloat16)])
+def test_rows_shared_by_two_waves(batch, dim, length, nstate, dtype):
+    """Rows so few that two waves take each, with half of the states: the numbers of the first batch row alone, whose chunks
+    run side by side in another kernel."""
+    from ssm_amd import ops
+    inp = make_inputs(length, batch, dim, length, nstate, dtype=dtype, bc_dtype=dtype, groups=1)
+    g = torch.Generator().manual_seed(2)
+    go, gl = torch.randn(batch, dim, length, generator=g).to(dtype).cuda(), torch.randn(batch, dim, nstate, generator=g).to(dtype).cuda()
+
+    def run(rows):
+        t = {k: (v[:rows] if k in ("u", "delta", "z", "B", "C") else v).cuda().requires_grad_(True) for k, v in inp.items()}
+        y, h = ops.selective_scan(*(t[k] for k in NAMES[:5]), D=t["D"], z=t["z"], dt_bias=t["dt_bias"], softplus=True,
+                                  return_last_state=True)
+        torch.autograd.backward([y, h], [go[:rows].contiguous(), gl[:rows].contiguous()])
+        return [y, h] + [t[k].grad for k in ("u", "delta", "z", "B", "C")]
+    for a, b, what in zip(run(batch), run(1), ("y", "last state", "u", "delta", "z", "B", "C")):
+        a, b = a.detach()[:1].float(), b.detach().float()
+        # both sum in float32; a 16-bit result may be rounded to either neighbour
+        tol = dict(rtol=1e-4, atol=2e-5) if dtype == torch.float32 else dict(rtol=2.0 ** -7, atol=1e-4)
+        torch.testing.assert_close(a, b, rtol=tol["rtol"], atol=tol["atol"] * float(b.abs().max()), msg=lambda m: f"{what}: {m}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_what_lies_past_a_row_never_enters_it(dtype):
     """The row after next holds infinities: steps past the end of a row are read with it and must count for nothing."""
