@@ -34,6 +34,22 @@ bool ssd_side_by_side(const SsdDims &d) {
   return d.nchunks > 2 && walk > c.start + c.each * units + c.more * std::max(0.0, units - c.from);
 }
 
+// Callers size workspaces ahead of a call and keep them, so a shape goes on asking for what it did when the line between the
+// routes lay elsewhere: room for the states up to more heads, steps and running sums of whole chunks otherwise.
+size_t ssd_settled_workspace_bytes(const SsdDims &d) {
+  struct Chunks { double chunk, group, unit; };
+  static const Chunks chunks[3][2] = {{{3.8, 0.0032, 0.0167}, {4.5, 0.0026, 0.0264}},
+                                      {{4.1, 0.0060, 0.0262}, {5.2, 0.0059, 0.0355}},
+                                      {{6.5, 0.0124, 0.0421}, {7.0, 0.0139, 0.0536}}};
+  const Chunks &f = chunks[d.chunk > 128 ? 2 : d.chunk > 64][d.nstate > 64];
+  const int64_t halves = 2 * (int64_t)d.batch * d.heads;
+  const auto chunk = [&](int64_t n) { return n ? f.chunk + f.group * std::max(0.0, (double)n - 100.0) : 0.0; };
+  const double walk = 9.0 + d.nchunks * ((double)(halves / 768) * chunk(768) + chunk(halves % 768));
+  if (d.nchunks > 2 && walk > 16.0 + f.unit * 0.5 * (double)halves * d.nchunks) return ssd_work_layout(d, false, true).total;
+  const size_t steps = (size_t)d.nchunks * d.chunk, rows = (size_t)d.batch * steps * d.groups * 2;
+  return 2 * ssd_align_up((size_t)d.batch * d.heads * steps * sizeof(float)) + 2 * ssd_align_up(rows * d.nstate) + ssd_align_up(rows * d.chunk);
+}
+
 template <typename E, int Q, int N>
 static void forward_launches(const SsdStatesParams &st, const SsdCarryParams &ca, const SsdChunkScanParams &sc, const SsdDims &d,
                              hipStream_t s) {

@@ -102,7 +102,6 @@ struct SsdWorkLayout {
   size_t Bblk, Ctblk, CBtblk;           // ... that only the backward reads; empty without `keep`
   size_t states, states_low;            // (B, nc, H, 64 N) entering the chunks, and (with `keep`) the rest of their float32
   size_t added;                         // (B, nc, H, 64 N) float32: what each chunk adds; these three empty on the one-pass route
-  size_t grown;                         // one-pass route: SsdWalkParams::grown
   size_t total;                         // (without `added` where `keep`: it lies in the call's scratch, ssd_added_bytes)
 };
 
@@ -110,6 +109,8 @@ inline size_t ssd_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Whether the forward takes the chunks side by side (ssd_chunk.hip) rather than one after the other (ssd_walk.hip).
 bool ssd_side_by_side(const SsdDims &d);
+// Bytes a forward's workspace has had for a shape since before the walk: what the query never goes below.
+size_t ssd_settled_workspace_bytes(const SsdDims &d);
 
 inline size_t ssd_added_bytes(const SsdDims &d) {
   return ssd_align_up((size_t)d.batch * d.nchunks * d.heads * SSD_P * d.nstate * sizeof(float));
@@ -138,7 +139,6 @@ inline SsdWorkLayout ssd_work_layout(const SsdDims &d, bool keep, bool side_by_s
   f.states = at; at += ssd_align_up(states * 2);
   f.states_low = at; at += keep ? ssd_align_up(states * 2) : 0;
   f.added = at; at += states && !keep ? ssd_added_bytes(d) : 0;
-  f.grown = at; at += walk ? ssd_align_up((size_t)d.batch * d.heads * SSD_P * d.nstate * sizeof(float)) : 0;
   f.total = at;
   return f;
 }

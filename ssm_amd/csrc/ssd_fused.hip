@@ -326,7 +326,7 @@ extern "C" size_t ssm_ssd_combined_workspace_bytes(const ssm_ssd_dims *dims) {
 #ifdef SSM_TEST_HOOKS
   return std::max(ssm::ssd_work_layout(d, false, true).total, ssm::ssd_work_layout(d, false, false).total);
 #else
-  return ssm::ssd_work_layout(d, false, ssm::ssd_side_by_side(d)).total;
+  return std::max(ssm::ssd_work_layout(d, false, ssm::ssd_side_by_side(d)).total, ssm::ssd_settled_workspace_bytes(d));
 #endif
 }
 
@@ -428,7 +428,6 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   wp.x = a->x; wp.z = a->z; wp.y = a->y;
   wp.steps = pp.steps; wp.ends = pp.ends; wp.Cblk = Cblk; wp.CBblk = ws + lay.CBblk; wp.Btblk = Btblk;
   wp.Dk = a->Dskip; wp.init = a->initial_states; wp.A = a->A; wp.final_states = a->final_states;
-  wp.grown = reinterpret_cast<float *>(ws + lay.grown);
   wp.batch = d.batch; wp.len = d.len; wp.heads = d.heads; wp.groups = d.groups;
   wp.nblocks = units.nchunks; wp.turns = ssd_walk_turns(units.nchunks); wp.chunk_blocks = d.chunk / SSD_WALK_BLOCK;
   return ssd_walk_forward(wp, !a->Dskip ? 0 : (a->d_per_p ? 2 : 1), f16, d.nstate, s);

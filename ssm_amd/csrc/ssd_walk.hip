@@ -307,8 +307,7 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
   const auto b_frag = [&](int c, int i, int ks) { return *at_bytes<const V8<E>>(pb + (size_t)(c * p.groups) * (KN * SSD_FRAG) + (ks * NT + i) * SSD_FRAG, lane16); };
 
   f32x16_t S[TPW];
-  V8<E> hf[GROW ? TPW : 1][2];                             // growing: the state entering the chunk, as operands; its float32 is in memory
-  float4 *const grown = reinterpret_cast<float4 *>(p.grown + ((size_t)b * p.heads + h) * SSD_P * N) + (wave * TPW * 4) * WAVE + lane;
+  f32x16_t entered[GROW ? TPW : 1];                        // growing: the state entering the chunk
   const size_t state0 = (((size_t)b * p.heads + h) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
@@ -319,14 +318,14 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
     }
   }
   V8<E> cf[TPW][2], bf[TPW][2];
-  // requested a block ahead (those of B in the same turn by a growing head, which keeps twice the state)
+  // requested a block ahead (by a growing head, which keeps twice the state, where they are used)
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       // without a state to start from the first block's product with it is zero whatever C holds
       cf[i][t] = V8<E>{};
-      if (p.init) cf[i][t] = c_frag(0, i, t);
+      if (!GROW && p.init) cf[i][t] = c_frag(0, i, t);
       if (!GROW) bf[i][t] = b_frag(0, i, t);
     }
   }
@@ -342,10 +341,7 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
     if (GROW && c % p.chunk_blocks == 0) {
 #pragma unroll
       for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) grown[(4 * i + q) * WAVE] = make_float4(S[i][4 * q], S[i][4 * q + 1], S[i][4 * q + 2], S[i][4 * q + 3]);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) hf[i][t] = state_frag<E>(S[i], t);
+        entered[i] = S[i];
         S[i] = (f32x16_t){0};
       }
       base = 0.0f;
@@ -356,12 +352,15 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
     for (int i = 0; i < TPW; ++i) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        acc = mma(state_frag<E>(S[i], t), cf[i][t], acc);
         if (GROW) {
-          acc_h = mma(hf[i][t], cf[i][t], acc_h);
-          bf[i][t] = b_frag(min(c, p.nblocks - 1), i, t);
+          V8<E> cg{};
+          if (c || p.init) cg = c_frag(min(c, p.nblocks - 1), i, t);
+          acc = mma(state_frag<E>(S[i], t), cg, acc);
+          acc_h = mma(state_frag<E>(entered[i], t), cg, acc_h);
+        } else {
+          acc = mma(state_frag<E>(S[i], t), cf[i][t], acc);
+          cf[i][t] = c_frag(next, i, t);
         }
-        cf[i][t] = c_frag(next, i, t);
       }
     }
     const float f = exp2_hw(GROW ? fminf(own, 0.0f) : own);
@@ -385,8 +384,12 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
       const V8<E> xf = transposed_frag<E>(xwt, tr0 + ks * 2048, tr1 + ks * 2048);
 #pragma unroll
       for (int i = 0; i < TPW; ++i) {
-        S[i] = mma(bf[i][ks], xf, S[i]);
-        if (!GROW) bf[i][ks] = b_frag(next, i, ks);
+        if (GROW) {
+          S[i] = mma(b_frag(min(c, p.nblocks - 1), i, ks), xf, S[i]);
+        } else {
+          S[i] = mma(bf[i][ks], xf, S[i]);
+          bf[i][ks] = b_frag(next, i, ks);
+        }
       }
     }
     if (GROW) {
@@ -396,13 +399,7 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float4 v = grown[(4 * i + q) * WAVE];
-            S[i][4 * q] = __builtin_fmaf(v.x, gh, S[i][4 * q]);
-            S[i][4 * q + 1] = __builtin_fmaf(v.y, gh, S[i][4 * q + 1]);
-            S[i][4 * q + 2] = __builtin_fmaf(v.z, gh, S[i][4 * q + 2]);
-            S[i][4 * q + 3] = __builtin_fmaf(v.w, gh, S[i][4 * q + 3]);
-          }
+          for (int r = 0; r < 16; ++r) S[i][r] = __builtin_fmaf(entered[i][r], gh, S[i][r]);
         }
       }
     }

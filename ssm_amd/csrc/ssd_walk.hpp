@@ -12,7 +12,6 @@ struct SsdWalkParams {                  // x, z, y and the fragment copies hold 
   const void *Cblk, *Btblk, *CBblk;     // fragments of blocks of 32 steps
   const float *Dk, *init, *A;
   float *final_states;
-  float *grown;                         // (B, H, 64 N): where a growing head keeps the state entering a chunk
   int batch, len, heads, groups, nblocks;
   int sets;                             // workgroups of one or two heads (set by ssd_walk_forward)
   int turns;                            // nblocks in whole turns through a ring of four
