@@ -38,12 +38,14 @@ struct NormParams {
   float eps;
 };
 
-// Elements up to which a call's tensors are left to the caches.  Larger calls read what is not read again past them (the
-// forward its residual, the backward all it reads): the space is better spent on what is written, for those who read that.
-// Forward and backward, bf16 with a float32 residual and gradient through it, us without / with: 2048 x 768 16.6 / 17.4,
-// 2048 x 2560 36 / 40, 4 x 2048 x 768 43.2 / 42.1, 8 x 2048 x 768 75.5 / 70.1, 16 x 2048 x 768 149 / 136 (the
-// forward's x past the caches too: 137; what is written past them: slower).
-constexpr size_t NORM_CACHED = (size_t)5632 << 10;
+// Calls up to these sizes leave what they read to the caches; larger ones read past them what is not read again (a backward
+// everything, a forward its residual: x is what a backward reads again): the space is better spent on what is written, for
+// those who read that.  Forward and backward (the forward keeps rstd), by elements, bf16 with a float32 residual and gradient
+// through it, us without / with: 2048 x 768 16.6 / 17.4, 2048 x 2560 36 / 40, 4 x 2048 x 768 43.2 / 42.1, 8 x 2048 x 768
+// 75.5 / 70.1, 16 x 2048 x 768 149 / 136 (the forward's x past the caches too 137; what is written past them: slower).  A
+// forward alone, by bytes, where they are more than the last-level cache holds: 75 MB 13.5 / 15.5, 252 MB 44.0 / 44.8, 302 MB
+// 49.1 / 48.2, float32 403 MB 71.8 / 63.1.
+constexpr size_t NORM_CACHED = (size_t)5632 << 10, NORM_CACHED_BYTES = (size_t)268 << 20;
 
 __device__ __forceinline__ void store_f32_as(void *p, int dtype, size_t i, float v) {
   if (dtype == SSM_F32) reinterpret_cast<float *>(p)[i] = v;
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_kernel(const NormParams p
 // unconditional - column indices are clamped into the row, an absent residual or bias reads a stand-in of
 // the same type whose value is dropped - so a wavefront's reads are in flight together instead of one
 // behind the other, which is what a call on a handful of rows (a decoding step) waits for.
-// Past NORM_CACHED the residual is read past the caches: what a backward reads again is x.
+// Large calls (NORM_CACHED) read the residual past the caches.
 template <typename T, int VEC>
 __device__ __forceinline__ void ld_pack(const void *p, size_t i, float (&v)[VEC]) {
   const Pack<T, VEC> raw = *reinterpret_cast<const Pack<T, VEC> *>(reinterpret_cast<const T *>(p) + i);
@@ -212,7 +214,7 @@ __device__ __forceinline__ void ld_once(const void *p, size_t i, float (&v)[VEC]
 #pragma unroll
   for (int j = 0; j < VEC; ++j) v[j] = to_f32(raw.v[j]);
 }
-template <int TRIPS, bool WG, typename XT, typename RT>
+template <int TRIPS, bool WG, typename XT, typename RT, bool PAST>
 __global__ __launch_bounds__(LN_THREADS) void norm_fwd_typed_kernel(const NormParams p) {
   constexpr int VEC = 4;
   constexpr int OWNERS = WG ? LN_THREADS : WAVE;       // threads that share a row
@@ -233,12 +235,13 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_typed_kernel(const NormPa
     const int colc = min((k * OWNERS + lane) * VEC, H - VEC);
     ld_pack<XT, VEC>(p.x, base + colc, v[k]);
   }
-  if (has_res && p.past_caches) {                 // one test in front of all of a row's residual reads, none between them
+  if (has_res) {                 // one test in front of all of a row's residual reads, none between them
 #pragma unroll
-    for (int k = 0; k < TRIPS; ++k) ld_once<RT, VEC>(resp, base + min((k * OWNERS + lane) * VEC, H - VEC), r[k]);
-  } else if (has_res) {
-#pragma unroll
-    for (int k = 0; k < TRIPS; ++k) ld_pack<RT, VEC>(resp, base + min((k * OWNERS + lane) * VEC, H - VEC), r[k]);
+    for (int k = 0; k < TRIPS; ++k) {
+      const int colc = min((k * OWNERS + lane) * VEC, H - VEC);
+      if constexpr (PAST) ld_once<RT, VEC>(resp, base + colc, r[k]);
+      else ld_pack<RT, VEC>(resp, base + colc, r[k]);
+    }
   } else {
 #pragma unroll
     for (int k = 0; k < TRIPS; ++k)
@@ -297,23 +300,28 @@ __global__ __launch_bounds__(LN_THREADS) void norm_fwd_typed_kernel(const NormPa
   }
 }
 
+template <typename XT, typename RT, bool PAST>
+static void launch_norm_fwd_typed_as(const NormParams &p, int per_lane, unsigned grid, hipStream_t s) {
+  const dim3 b(LN_THREADS);
+  if (per_lane <= 4) hipLaunchKernelGGL((norm_fwd_typed_kernel<1, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 8) hipLaunchKernelGGL((norm_fwd_typed_kernel<2, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 12) hipLaunchKernelGGL((norm_fwd_typed_kernel<3, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 16) hipLaunchKernelGGL((norm_fwd_typed_kernel<4, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  // (a trip that holds no column still reads one: rows of 1280, 1536 and 1792 columns get trip counts of their own)
+  else if (per_lane <= 20) hipLaunchKernelGGL((norm_fwd_typed_kernel<5, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 24) hipLaunchKernelGGL((norm_fwd_typed_kernel<6, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 28) hipLaunchKernelGGL((norm_fwd_typed_kernel<7, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (per_lane <= 32) hipLaunchKernelGGL((norm_fwd_typed_kernel<8, false, XT, RT, PAST>), dim3(grid), b, 0, s, p);
+  else if (p.hidden <= 4096) hipLaunchKernelGGL((norm_fwd_typed_kernel<4, true, XT, RT, PAST>), dim3(p.rows), b, 0, s, p);
+  else if (p.hidden <= 5120) hipLaunchKernelGGL((norm_fwd_typed_kernel<5, true, XT, RT, PAST>), dim3(p.rows), b, 0, s, p);
+  else if (p.hidden <= 6144) hipLaunchKernelGGL((norm_fwd_typed_kernel<6, true, XT, RT, PAST>), dim3(p.rows), b, 0, s, p);
+  else if (p.hidden <= 8192) hipLaunchKernelGGL((norm_fwd_typed_kernel<8, true, XT, RT, PAST>), dim3(p.rows), b, 0, s, p);
+  else hipLaunchKernelGGL((norm_fwd_typed_kernel<16, true, XT, RT, PAST>), dim3(p.rows), b, 0, s, p);
+}
 template <typename XT, typename RT>
 static void launch_norm_fwd_typed(const NormParams &p, int per_lane, unsigned grid, hipStream_t s) {
-  const dim3 b(LN_THREADS);
-  if (per_lane <= 4) hipLaunchKernelGGL((norm_fwd_typed_kernel<1, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 8) hipLaunchKernelGGL((norm_fwd_typed_kernel<2, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 12) hipLaunchKernelGGL((norm_fwd_typed_kernel<3, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 16) hipLaunchKernelGGL((norm_fwd_typed_kernel<4, false, XT, RT>), dim3(grid), b, 0, s, p);
-  // (a trip that holds no column still reads one: rows of 1280, 1536 and 1792 columns get trip counts of their own)
-  else if (per_lane <= 20) hipLaunchKernelGGL((norm_fwd_typed_kernel<5, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 24) hipLaunchKernelGGL((norm_fwd_typed_kernel<6, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 28) hipLaunchKernelGGL((norm_fwd_typed_kernel<7, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (per_lane <= 32) hipLaunchKernelGGL((norm_fwd_typed_kernel<8, false, XT, RT>), dim3(grid), b, 0, s, p);
-  else if (p.hidden <= 4096) hipLaunchKernelGGL((norm_fwd_typed_kernel<4, true, XT, RT>), dim3(p.rows), b, 0, s, p);
-  else if (p.hidden <= 5120) hipLaunchKernelGGL((norm_fwd_typed_kernel<5, true, XT, RT>), dim3(p.rows), b, 0, s, p);
-  else if (p.hidden <= 6144) hipLaunchKernelGGL((norm_fwd_typed_kernel<6, true, XT, RT>), dim3(p.rows), b, 0, s, p);
-  else if (p.hidden <= 8192) hipLaunchKernelGGL((norm_fwd_typed_kernel<8, true, XT, RT>), dim3(p.rows), b, 0, s, p);
-  else hipLaunchKernelGGL((norm_fwd_typed_kernel<16, true, XT, RT>), dim3(p.rows), b, 0, s, p);
+  if (p.past_caches && p.res) launch_norm_fwd_typed_as<XT, RT, true>(p, per_lane, grid, s);
+  else launch_norm_fwd_typed_as<XT, RT, false>(p, per_lane, grid, s);
 }
 
 // True when the call was taken by a typed kernel.
@@ -693,7 +701,9 @@ extern "C" int ssm_norm_fwd(const ssm_norm_fwd_args *a, void *hip_stream) {
   p.mean = a->mean; p.rstd = a->rstd;
   p.rows = a->rows; p.hidden = a->hidden;
   p.x_dtype = a->x_dtype; p.res_dtype = a->residual_dtype; p.res_out_dtype = a->residual_out_dtype;
-  p.past_caches = (size_t)a->rows * a->hidden > NORM_CACHED;
+  const size_t each = 2 * (a->x_dtype == SSM_F32 ? 4 : 2) + (a->residual ? (a->residual_dtype == SSM_F32 ? 4 : 2) : 0) +
+                      (a->residual_out ? (a->residual_out_dtype == SSM_F32 ? 4 : 2) : 0);        // bytes moved
+  p.past_caches = a->rstd ? (size_t)a->rows * a->hidden > NORM_CACHED : (size_t)a->rows * a->hidden * each > NORM_CACHED_BYTES;
   p.is_rms = a->is_rms ? 1 : 0; p.prenorm = a->prenorm ? 1 : 0; p.eps = a->eps;
   const int vec_ok = a->hidden % 4 == 0 && aligned_to(a->x, 16) && aligned_to(a->y, 16) &&
                      aligned_to(a->weight, 16) && (!a->bias || aligned_to(a->bias, 16)) &&
