@@ -21,6 +21,8 @@
 // from x~ joins the products inside the block as an operand of its own, so that these lose nothing beyond the rounding of
 // C.B.  Heads with a block beyond that range, growing heads (A > 0) and float16 calls (whose exponents hold no such x~)
 // form exp(cs_l - cs_s) dt_s (C_l.B_s) per element instead, x weighted towards the block's end for the state.
+// The factors r - cs_s reach 2^80: where dt x is so large that x~, or what it is summed into, leaves bfloat16, a y or a state
+// comes out infinite or not a number, and the workgroup does its heads again per element, whose factors are at most 1.
 //
 // What bounds it: a CU takes in x and z at no more than about 20 (one head's rows of 128 bytes) to 27 (two heads') bytes per
 // ns whatever is in flight - a kernel that only streams them this way takes 88 us for 256 heads x 4096 steps on 256 CUs, 148
@@ -49,7 +51,8 @@ template <int NH> struct WalkLds {
 };
 // Heads that factor: fragments of three blocks.
 template <int NH, int N> struct FactoredLds {
-  static constexpr int KN = N / 16, C = WalkLds<NH>::END, B = C + 3 * KN * 1024, CB = B + 3 * KN * 1024, BYTES = CB + 3 * 2048;
+  static constexpr int KN = N / 16, C = WalkLds<NH>::END, B = C + 3 * KN * 1024, CB = B + 3 * KN * 1024, AGAIN = CB + 3 * 2048;
+  static constexpr int BYTES = AGAIN + 16;                               // (a word: whether something left the range)
 };
 // Others, one at a time: decayed C.B of two blocks; cs, log2 dt - cs and log2 dt (cs less half of the block's) of four.
 struct PlainLds {
@@ -94,6 +97,15 @@ __device__ __forceinline__ V8<E> state_frag(const f32x16_t &s, int t) {
   return r;
 }
 
+// Keeps in `seen` that one of eight values stored as bfloat16 was infinite or no number: read as float16 these bits are no
+// number, nor are those from 2^121 on, and a maximum that passes on what is no number costs half an instruction a word.
+__device__ __forceinline__ void note_overflow(unsigned &seen, const V8<__bf16> &v) {
+  const u32x4_t w = __builtin_bit_cast(u32x4_t, v);
+  asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(seen) : "v"(w[0]), "v"(w[1]));
+  asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(seen) : "v"(w[2]), "v"(w[3]));
+}
+__device__ __forceinline__ bool noted_overflow(unsigned seen) { return (seen & 0x7fffu) > 0x7c00u || (seen >> 16 & 0x7fffu) > 0x7c00u; }
+
 // One head, or two neighbouring heads of a group (the last of an odd number alone: it is computed twice and written once).
 template <int NH>
 struct WalkHeads {
@@ -122,9 +134,9 @@ struct WalkHeads {
 };
 
 // The waves of rows.  Turn c: gate and store block c - 1, stage block c + 1.  Each thread has eight channels of one row of
-// every block; what it takes from memory of them is requested four turns ahead.
+// every block; what it takes from memory of them is requested four turns ahead.  FACTOR: whether a y left the range.
 template <typename E, int NH, int DMODE, bool HAS_Z, bool FACTOR>
-__device__ __forceinline__ void walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
+__device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
   static_assert(FACTOR || NH == 1);
   using L = WalkLds<NH>;
   const int wave = wave_id_uniform() - 4, lane = lane_id(), tid = wave * WAVE + lane;
@@ -148,6 +160,7 @@ __device__ __forceinline__ void walk_rows(const SsdWalkParams &p, unsigned char 
   float2 step[4];
   vec4_t cb[4];
   float skip[2][8], grow[2];
+  unsigned seen = 0;
   // A ring's place is loaded again once `after` is there: a load in front of the last use of what the place held would take
   // another register, and the copy back at the end of the loop would wait for it.
   const auto load_rows = [&](rsrc_t r, int c, const V8<E> &after) {
@@ -257,6 +270,9 @@ __device__ __forceinline__ void walk_rows(const SsdWalkParams &p, unsigned char 
       for (int j = 0; j < 8; ++j) v[j] *= silu_f32(zf[j]);
     }
     const V8<E> out = pack8_e<E>(v);
+    if constexpr (FACTOR) {
+      if (c >= 0) note_overflow(seen, out);
+    }
     if (HAS_Z) z[u] = load_rows(rz, c + 4, out);
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
   };
@@ -283,6 +299,7 @@ __device__ __forceinline__ void walk_rows(const SsdWalkParams &p, unsigned char 
     }
   }
   gate(p.turns - 1, 3, read_parts(3), grow[1], skip[1]);
+  return __any(noted_overflow(seen));
 }
 
 // The four waves of products of a head that does not factor.  Turn c: block c.
@@ -422,9 +439,10 @@ __device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned 
   }
 }
 
-// The four waves of products of heads that factor.  Turn c: block c.
-template <typename E, int NH, int N>
-__device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
+// The four waves of products of heads that factor.  Turn c: block c.  Final states are written once `settled` (asked when this
+// wave's share of the heads is done, with whether it left the range) has said that they stand.
+template <typename E, int NH, int N, typename Settled>
+__device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const Settled &settled) {
   using F = WalkLds<NH>;
   using L = FactoredLds<NH, N>;
   constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16, SHARE = KN / 4;
@@ -536,7 +554,17 @@ __device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsign
     t3 = t3 == 2 ? 0 : t3 + 1;
   }
   walk_barrier();
-  if (p.final_states) {
+  wait_memory<0>();                                        // nothing may land in LDS that is others' by then
+  float zero = 0.0f;                                       // no number once a state is infinite or none
+#pragma unroll
+  for (int hd = 0; hd < NH; ++hd) {
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) zero = __builtin_fmaf(S[hd][i][r], 0.0f, zero);
+    }
+  }
+  if (settled(__any(zero != 0.0f)) && p.final_states) {
 #pragma unroll
     for (int hd = 0; hd < NH; ++hd) {
       const float g = exp2_hw(0.5f * end[hd]);
@@ -550,7 +578,6 @@ __device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsign
       }
     }
   }
-  wait_memory<0>();                                        // nothing may land in LDS that is another workgroup's by then
 }
 
 // Whether all of the heads' blocks decay by at most WALK_RANGE (in powers of two), and none grows.
@@ -585,8 +612,24 @@ void ssd_walk_kernel(const SsdWalkParams p) {
   } else if (blockIdx.x < (unsigned)p.sets) {
     const WalkHeads<NH> hp(p, (int)xcd_order(blockIdx.x, p.sets));
     if (!decays_factor(p, hp)) return;
-    if (wave_id_uniform() >= 4) walk_rows<E, NH, DMODE, HAS_Z, true>(p, lds, hp);
-    else factored_products<E, NH, N>(p, lds, hp);
+    int *again = reinterpret_cast<int *>(lds + FactoredLds<NH, N>::AGAIN);
+    if (threadIdx.x == 0) *again = 0;
+    const auto settled = [&](bool left_range) {
+      if (left_range) *again = 1;
+      walk_barrier();
+      const int v = __builtin_amdgcn_readfirstlane(*again);
+      walk_barrier();                                      // LDS is others' to write
+      return v == 0;
+    };
+    bool done = true;
+    if (wave_id_uniform() >= 4) done = settled(walk_rows<E, NH, DMODE, HAS_Z, true>(p, lds, hp));
+    else factored_products<E, NH, N>(p, lds, hp, [&](bool left_range) { return done = settled(left_range); });
+    if (done || wave_id_uniform() >= PLAIN_THREADS / WAVE) return;
+    plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, hp.h0);
+    if (hp.two) {
+      walk_barrier();
+      plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, hp.h1);
+    }
   } else {
     const unsigned id = blockIdx.x - p.sets, second = NH == 2 ? id & 1 : 0;
     const WalkHeads<NH> hp(p, (int)xcd_order(id / NH, p.sets));
