@@ -6,6 +6,7 @@
 #include "ssd_common.hpp"
 #include "ssd_walk.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace ssm {
 
@@ -133,6 +134,7 @@ __device__ __forceinline__ void stage_walk_dt(const void *dt, size_t row, int st
 // For the walk: two blocks of 32 heads, whose 64 bytes of a row are read together.
 // Bound by latency: 80 heads of 512 steps 4.8 us for the launch, 24 heads of 256 5.3 (8.5 and 6.8 with the reads of dt, A and
 // bias one behind the other).
+template <bool FACTORS>
 __device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
   float (*tile)[64 + 1] = reinterpret_cast<float (*)[64 + 1]>(lds);
   const SsdCumsumParams &p = pp.cs;
@@ -161,7 +163,7 @@ __device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsig
     const float cs = half_wave_inclusive_sum(__builtin_fmaf(v, wave_read_lane(A_lanes, k), jump)) * LOG2E;
     const float end = lane < SSD_WALK_BLOCK ? wave_read_lane(cs, SSD_WALK_BLOCK - 1) : wave_read_lane(cs, 2 * SSD_WALK_BLOCK - 1);
     const size_t at = ((size_t)b * d.heads + h) * turns + 2 * unit;           // block
-    reinterpret_cast<float2 *>(pp.steps)[at * SSD_WALK_BLOCK + lane] = make_float2(cs - 0.5f * end, v);
+    reinterpret_cast<float2 *>(pp.steps)[at * SSD_WALK_BLOCK + lane] = make_float2(FACTORS && walk_factors(end) ? cs - 0.5f * end : cs, v);
     if (lane % SSD_WALK_BLOCK == SSD_WALK_BLOCK - 1) pp.ends[at + lane / SSD_WALK_BLOCK] = end;
   }
 }
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(256) void ssd_fused_prep_kernel(const SsdPrepParams
   const unsigned wg = blockIdx.x;
   // neighbours in a role, which read the same lines, on one XCD
   if (wg < pp.n_dt) {
-    if (pp.steps) prep_walk_dt_role(pp, xcd_order(wg, pp.n_dt), lds);
+    if (pp.steps) prep_walk_dt_role<std::is_same<E, __bf16>::value>(pp, xcd_order(wg, pp.n_dt), lds);
     else prep_dt_role(pp, xcd_order(wg, pp.n_dt), lds);
   } else if (wg < pp.n_dt + pp.n_pack) {
     prep_pack_role<E, KN>(pp, xcd_order(wg - pp.n_dt, pp.n_pack));

@@ -19,46 +19,51 @@
 //   y_l = exp(cs_l - r) (C_l.S~ + sum_{s<=l} (C_l.B_s) x~_s),      S~ <- exp(..) (S~ + sum_s x~_s (x) B_s),
 // no element of C.B needs a factor, and C.B goes from memory to the matrix cores as it is.  What rounding to bfloat16 takes
 // from x~ joins the products inside the block as an operand of its own, so that these lose nothing beyond the rounding of
-// C.B.  Heads with a block beyond that range, growing heads (A > 0) and float16 calls (whose exponents hold no such x~)
-// form exp(cs_l - cs_s) dt_s (C_l.B_s) per element instead, x weighted towards the block's end for the state.
+// C.B.  Heads of which a block goes beyond that range, and float16 calls (whose exponents hold no such x~), form
+// exp(cs_l - cs_s) dt_s (C_l.B_s) per element instead, x weighted towards the block's end for the state.
 // The factors r - cs_s reach 2^80: where dt x is so large that x~, or what it is summed into, leaves bfloat16, a y or a state
 // comes out infinite or not a number, and the workgroup does its heads again per element, whose factors are at most 1.
+//
+// A growing head (A > 0): decays between steps of one of the call's chunks are bounded by 1, the factors on the state entering
+// the chunk are not (the published kernels evaluate exp(min(x, 0)) and exp(x) there).  Such a head goes per element and keeps
+// that state apart from what the chunk has added so far.
+//
+// Which of the three ways a workgroup goes is told from A and the blocks' sums on the device; each has a loop of its own.
+// Choosing block by block inside one loop cost every call 0.05 to 0.1 us a block.  4 x 80 heads of 4096 steps, 128 states, us
+// a call with all heads factoring, one in eight not, none, all growing: 174, 187, 186, 309; 4 x 64 heads 139, 143, 139, 168; 24
+// heads of 512 steps 21.0, 22.4, 22.7, 25.8.  (With workgroups of their own for the heads that do not factor, behind the others:
+// 180, 250, 250, 671; 182, 229, 142, 330; 21.4, 21.3, 21.6, 43.  Before this walk: 274; 203; 21.9, whatever the decays.)
 //
 // What bounds it: a CU takes in x and z at no more than about 20 (one head's rows of 128 bytes) to 27 (two heads') bytes per
 // ns whatever is in flight - a kernel that only streams them this way takes 88 us for 256 heads x 4096 steps on 256 CUs, 148
 // us for 320 heads, as a CU with two workgroups takes twice as long, and 114 us for these as 160 pairs - and the vector ALU
 // issues behind the matrix cores, not beside them.  So: a head per workgroup while every workgroup has a CU of its own,
 // two neighbours beyond; and the fragments of B and C into LDS once per workgroup.  4 x 4096 steps, 128 states, 64 / 80 heads:
-// 137 / 195 us a call.  Before (half a head per workgroup, 64-byte rows, chunks of 256 steps): 200 / 279.
-// With fragments loaded by each wave 135 / 200.
-//
-// A growing head: decays between steps of one of the call's chunks are bounded by 1, the factors on the state entering the
-// chunk are not (the published kernels evaluate exp(min(x, 0)) and exp(x) there).  Such a head keeps that state apart from
-// what the chunk has added so far; the sign of A is read per head, on the device.
+// 139 / 174 us a call.  Before (half a head per workgroup, 64-byte rows, chunks of 256 steps): 203 / 274.
+// With fragments loaded by each wave it was 135 / 200 when this was 137 / 195.
 #include "ssd_common.hpp"
 #include "ssd_walk.hpp"
+#include <type_traits>
 
 namespace ssm {
 
 constexpr int WK = SSD_WALK_BLOCK, WK_TILE = WK * SSD_P * 2;             // steps of a block; bytes of its 64 channels
-constexpr float WALK_RANGE = 160.0f;                                     // powers of two: far from the end of float32 on either side
 constexpr int WALK_SINGLES = 256;                                        // heads that get a workgroup each: the CUs
 
+// FACTORS: heads whose decays factor; ELEMENTS: element by element; GROWS: the same, and the state that enters a chunk of the
+// call apart.
+enum WalkMode { FACTORS, ELEMENTS, GROWS };
+template <WalkMode M> using walk_mode = std::integral_constant<WalkMode, M>;
+
 // Byte offsets into LDS.  Twice each: 32 rows of x per head, weighted (X ..), and what their rounding lost, or x itself
-// (NH tiles on); part sums [head][nh][pt][step][32 channels] of float32.
-template <int NH> struct WalkLds {
-  static constexpr int X = 2 * NH * WK_TILE, PARTS = NH * 4 * 4096, PART = 2 * X, END = PART + 2 * PARTS;
+// (NH tiles on); part sums [head][nh][pt][step][32 channels] of float32; per head cs, log2 dt - cs and log2 dt of a block taken
+// element by element.  Fragments of three blocks.  A word: whether something left the range.
+template <int NH, int N> struct WalkLds {
+  static constexpr int KN = N / 16, X = 2 * NH * WK_TILE, PARTS = NH * 4 * 4096, STEPS = 3 * WK * 4;
+  static constexpr int PART = 2 * X, C = PART + 2 * PARTS, B = C + 3 * KN * 1024, CB = B + 3 * KN * 1024, STEP = CB + 3 * 2048;
+  static constexpr int AGAIN = STEP + 2 * NH * STEPS, BYTES = AGAIN + 16;
 };
-// Heads that factor: fragments of three blocks.
-template <int NH, int N> struct FactoredLds {
-  static constexpr int KN = N / 16, C = WalkLds<NH>::END, B = C + 3 * KN * 1024, CB = B + 3 * KN * 1024, AGAIN = CB + 3 * 2048;
-  static constexpr int BYTES = AGAIN + 16;                               // (a word: whether something left the range)
-};
-// Others, one at a time: decayed C.B of two blocks; cs, log2 dt - cs and log2 dt (cs less half of the block's) of four.
-struct PlainLds {
-  static constexpr int W = WalkLds<1>::END, STEPS = W + 2 * 2048, STEP_BYTES = 3 * WK * 4, BYTES = STEPS + 4 * STEP_BYTES;
-};
-static_assert(FactoredLds<2, 128>::BYTES <= 160 * 1024 && 2 * PlainLds::BYTES <= 160 * 1024, "one pair per CU, or two plain heads");
+static_assert(WalkLds<2, 128>::BYTES <= 160 * 1024, "one pair per CU");
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4_t;
@@ -97,6 +102,10 @@ __device__ __forceinline__ V8<E> state_frag(const f32x16_t &s, int t) {
   return r;
 }
 
+// What the running sums of a block that factors are relative to: the sum at its middle.
+template <typename E>
+__device__ __forceinline__ float walk_middle(float end) { return std::is_same<E, __bf16>::value && walk_factors(end) ? 0.5f * end : 0.0f; }
+
 // Keeps in `seen` that one of eight values stored as bfloat16 was infinite or no number: read as float16 these bits are no
 // number, nor are those from 2^121 on, and a maximum that passes on what is no number costs half an instruction a word.
 __device__ __forceinline__ void note_overflow(unsigned &seen, const V8<__bf16> &v) {
@@ -120,7 +129,7 @@ struct WalkHeads {
     two = NH == 2 && 2 * i + 1 < per_group;
     h1 = two ? h0 + 1 : h0;
   }
-  __device__ __forceinline__ WalkHeads(const SsdWalkParams &p, int b_, int h) : b(b_), g(h / (p.heads / p.groups)), h0(h), h1(h), two(false) {}
+  __device__ __forceinline__ WalkHeads(int b_, int g_, int h) : b(b_), g(g_), h0(h), h1(h), two(false) {}
   // Running sums at the ends of a head's blocks, read through the scalar cache.
   __device__ __forceinline__ scalar_floats ends(const SsdWalkParams &p, int second) const {
     return (scalar_floats)(size_t)(p.ends + ((size_t)b * p.heads + (second ? h1 : h0)) * p.turns);
@@ -133,12 +142,24 @@ struct WalkHeads {
   }
 };
 
+// Whether all of the heads' blocks factor.
+template <int NH>
+__device__ __forceinline__ bool heads_factor(const SsdWalkParams &p, const WalkHeads<NH> &hp) {
+  const float *e0 = p.ends + ((size_t)hp.b * p.heads + hp.h0) * p.turns, *e1 = p.ends + ((size_t)hp.b * p.heads + hp.h1) * p.turns;
+  bool ok = true;
+  for (int c0 = 0; c0 < p.turns; c0 += WAVE) {
+    const int c = min(c0 + lane_id(), p.turns - 1);
+    const float a = e0[c], b = NH == 2 ? e1[c] : a;
+    ok = ok && walk_factors(a) && walk_factors(b);
+  }
+  return __all(ok);
+}
+
 // The waves of rows.  Turn c: gate and store block c - 1, stage block c + 1.  Each thread has eight channels of one row of
-// every block; what it takes from memory of them is requested four turns ahead.  FACTOR: whether a y left the range.
-template <typename E, int NH, int DMODE, bool HAS_Z, bool FACTOR>
-__device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp) {
-  static_assert(FACTOR || NH == 1);
-  using L = WalkLds<NH>;
+// every block; what it takes from memory of them is requested four turns ahead.  Whether a y left the range.
+template <typename E, int NH, int N, int DMODE, bool HAS_Z, typename InMode>
+__device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const InMode &in_mode) {
+  using L = WalkLds<NH, N>;
   const int wave = wave_id_uniform() - 4, lane = lane_id(), tid = wave * WAVE + lane;
   const int row = tid / (8 * NH), second = NH == 2 ? tid >> 3 & 1 : 0, piece = tid & 7;
   const unsigned pitch = (unsigned)p.heads * SSD_P * 2, block = WK * pitch;
@@ -151,306 +172,145 @@ __device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char 
   float D8[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) D8[j] = DMODE == 0 ? 0.0f : p.Dk[DMODE == 2 ? h * SSD_P + 8 * piece + j : h];
-  // !FACTOR: the four places of a block's C.B that this thread decays: row m, steps w_s ..
-  typedef __attribute__((__vector_size__(4 * sizeof(E)))) E vec4_t;
-  const int m = lane & 31, w_s = 16 * (wave >> 1) + 8 * (lane >> 5) + 4 * (wave & 1), w_at = (wave >> 1) * 1024 + lane * 16 + (wave & 1) * 8;
-  const unsigned char *pcb = reinterpret_cast<const unsigned char *>(p.CBblk) + ((size_t)hp.b * p.nblocks * p.groups + hp.g) * 2048;
+  const scalar_floats ends[2] = {hp.ends(p, 0), hp.ends(p, NH - 1)};
 
-  V8<E> x[4], z[4];
-  float2 step[4];
-  vec4_t cb[4];
-  float skip[2][8], grow[2];
   unsigned seen = 0;
-  // A ring's place is loaded again once `after` is there: a load in front of the last use of what the place held would take
-  // another register, and the copy back at the end of the loop would wait for it.
-  const auto load_rows = [&](rsrc_t r, int c, const V8<E> &after) {
-    unsigned off = mine + (unsigned)c * block;
-    asm volatile("" : "+v"(off) : "v"(after));
-    return __builtin_bit_cast(V8<E>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-  };
-  const auto load_step = [&](int c, const V8<E> &after) {
-    unsigned off = step_at;
-    asm volatile("" : "+v"(off) : "v"(after));
-    return *at_bytes<const float2>(steps + (size_t)min(c, p.turns - 1) * WK, off);
-  };
-  const auto load_cb = [&](int c, const vec4_t &after) {
-    unsigned off = (unsigned)w_at;
-    asm volatile("" : "+v"(off) : "v"(after));
-    return *at_bytes<const vec4_t>(pcb + (size_t)min(c, p.nblocks - 1) * p.groups * 2048, off);
-  };
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    x[u] = load_rows(rx, u, V8<E>{});
-    if (HAS_Z) z[u] = load_rows(rz, u, V8<E>{});
-    step[u] = load_step(u, V8<E>{});
-    if (!FACTOR) cb[u] = load_cb(u, vec4_t{});
-  }
   const int at16 = second * WK_TILE + row * 128 + ((piece ^ (row & 7)) << 4);
   const int half_at = L::PART + second * 16384 + (piece >> 2) * 4096 + row * 128;
   const int q0 = half_at + (((2 * (piece & 3)) ^ (row & 7)) << 4), q1 = half_at + (((2 * (piece & 3) + 1) ^ (row & 7)) << 4);
 
-  const auto publish = [&](int u) __attribute__((always_inline)) {       // !FACTOR: what the block's steps mean to others
-    asm volatile("" : "+v"(step[u].x), "+v"(step[u].y));
-    float *st = reinterpret_cast<float *>(lds + PlainLds::STEPS + u * PlainLds::STEP_BYTES);
-    const float l2 = log2_hw(step[u].y);                   // dt = 0: -inf, a weight of zero
-    if (piece == 0) {
-      st[row] = step[u].x;
-      st[WK + row] = l2 - step[u].x;
-      st[2 * WK + row] = l2;
-    }
-  };
-  const auto stage = [&](int c, int u) __attribute__((always_inline)) {
-    // first looked at here: the scheduler would start on blocks ahead, and wait for reads that are still on their way
-    asm volatile("" : "+v"(x[u]), "+v"(step[u].x), "+v"(step[u].y));
-    float v[8];
-    unpack8(x[u], v);
-    if (DMODE != 0) {
+  const auto rows = [&](auto mode) __attribute__((always_inline)) {
+    constexpr WalkMode MODE = decltype(mode)::value;
+    V8<E> x[4], z[4];
+    float2 step[4];
+    float skip[2][8], grow[2];
+    // A ring's place is loaded again once `after` is there: a load in front of the last use of what the place held would take
+    // another register, and the copy back at the end of the loop would wait for it.
+    const auto load_rows = [&](rsrc_t r, int c, const V8<E> &after) {
+      unsigned off = mine + (unsigned)c * block;
+      asm volatile("" : "+v"(off) : "v"(after));
+      return __builtin_bit_cast(V8<E>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    };
+    const auto load_step = [&](int c, const V8<E> &after) {
+      unsigned off = step_at;
+      asm volatile("" : "+v"(off) : "v"(after));
+      return *at_bytes<const float2>(steps + (size_t)min(c, p.turns - 1) * WK, off);
+    };
 #pragma unroll
-      for (int j = 0; j < 8; ++j) skip[u & 1][j] = D8[j] * v[j];
+    for (int u = 0; u < 4; ++u) {
+      x[u] = load_rows(rx, u, V8<E>{});
+      if (HAS_Z) z[u] = load_rows(rz, u, V8<E>{});
+      step[u] = load_step(u, V8<E>{});
     }
-    unsigned char *to = lds + (u & 1) * L::X + at16;
-    if constexpr (FACTOR) {
-      const float w = step[u].y * exp2_hw(-step[u].x);
-      grow[u & 1] = exp2_hw(step[u].x);
-      float lost[8];
+    const auto stage = [&](int c, int u, const float (&end)[2]) __attribute__((always_inline)) {
+      // first looked at here: the scheduler would start on blocks ahead, and wait for reads that are still on their way
+      asm volatile("" : "+v"(x[u]), "+v"(step[u].x), "+v"(step[u].y));
+      float v[8], lost[8];
+      unpack8(x[u], v);
+      if (DMODE != 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) skip[u & 1][j] = D8[j] * v[j];
+      }
+      V8<E> rounded, rest;
+      const float to_end = NH == 2 && second ? end[1] : end[0], cs = step[u].x + (MODE == FACTORS ? 0.0f : walk_middle<E>(to_end));
+      const float w = step[u].y * exp2_hw(MODE == FACTORS ? -cs : fminf(to_end - cs, 0.0f));
+      rest = x[u];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] *= w;
-      const V8<E> rounded = pack8_e<E>(v);
-      unpack8(rounded, lost);
+      rounded = pack8_e<E>(v);
+      if constexpr (MODE == FACTORS) {
+        grow[u & 1] = exp2_hw(cs);
+        unpack8(rounded, lost);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) lost[j] = v[j] - lost[j];
-      const V8<E> rest = pack8_e<E>(lost);
+        for (int j = 0; j < 8; ++j) lost[j] = v[j] - lost[j];
+        rest = pack8_e<E>(lost);
+      } else if (piece == 0) {
+        float *st = reinterpret_cast<float *>(lds + L::STEP + ((u & 1) * NH + second) * L::STEPS);
+        const float l2 = log2_hw(step[u].y);                 // dt = 0: -inf, a weight of zero
+        st[row] = cs;
+        st[WK + row] = l2 - cs;
+        st[2 * WK + row] = l2;
+      }
+      unsigned char *to = lds + (u & 1) * L::X + at16;
       *reinterpret_cast<V8<E> *>(to) = rounded;
       *reinterpret_cast<V8<E> *>(to + NH * WK_TILE) = rest;
       x[u] = load_rows(rx, c + 4, rest);
       step[u] = load_step(c + 4, rest);
-    } else {
-      const float *st = reinterpret_cast<const float *>(lds + PlainLds::STEPS + u * PlainLds::STEP_BYTES);
-      const float w = step[u].y * exp2_hw(fminf(st[31] - step[u].x, 0.0f)), own = st[m];
-      const float4 e4 = *reinterpret_cast<const float4 *>(st + WK + w_s), l4 = *reinterpret_cast<const float4 *>(st + 2 * WK + w_s);
-      *reinterpret_cast<V8<E> *>(to + WK_TILE) = x[u];
+    };
+    struct Parts { float4 a0, a1, b0, b1; };
+    const auto read_parts = [&](int u) __attribute__((always_inline)) {
+      const unsigned char *half = lds + (u & 1) * L::PARTS;
+      return Parts{*reinterpret_cast<const float4 *>(half + q0), *reinterpret_cast<const float4 *>(half + q1),
+                   *reinterpret_cast<const float4 *>(half + 8192 + q0), *reinterpret_cast<const float4 *>(half + 8192 + q1)};
+    };
+    const auto gate = [&](int c, int u, const Parts &r, float up, const float (&dx)[8]) __attribute__((always_inline)) {
+      float v[8] = {r.a0.x + r.b0.x, r.a0.y + r.b0.y, r.a0.z + r.b0.z, r.a0.w + r.b0.w, r.a1.x + r.b1.x, r.a1.y + r.b1.y, r.a1.z + r.b1.z, r.a1.w + r.b1.w};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] *= w;
-      const V8<E> rounded = pack8_e<E>(v);
-      *reinterpret_cast<V8<E> *>(to) = rounded;
-      x[u] = load_rows(rx, c + 4, rounded);
-      step[u] = load_step(c + 4, rounded);
-      const float e[4] = {e4.x, e4.y, e4.z, e4.w}, l2[4] = {l4.x, l4.y, l4.z, l4.w};
-      asm volatile("" : "+v"(cb[u]));
-      vec4_t d;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // dt_s exp(min(cs_l - cs_s, 0)) as one exponential: min(a, 0) + b = min(a + b, b) with b = log2 dt_s.  The bound is
-        // inactive on and below the diagonal of a decaying head, is the clamp of a growing one, and keeps the places above
-        // the diagonal (zeros of C.B) finite.
-        d[j] = (E)((float)cb[u][j] * exp2_hw(fminf(own + e[j], l2[j])));
+      for (int j = 0; j < 8; ++j) {
+        if (MODE == FACTORS) v[j] = DMODE == 0 ? v[j] * up : __builtin_fmaf(v[j], up, dx[j]);
+        else if (DMODE != 0) v[j] += dx[j];
       }
-      *reinterpret_cast<vec4_t *>(lds + PlainLds::W + (u & 1) * 2048 + w_at) = d;
-      cb[u] = load_cb(c + 4, d);
+      if (HAS_Z) {
+        float zf[8];
+        asm volatile("" : "+v"(z[u]));
+        unpack8(z[u], zf);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] *= silu_f32(zf[j]);
+      }
+      const V8<E> out = pack8_e<E>(v);
+      if constexpr (MODE == FACTORS) {
+        if (c >= 0) note_overflow(seen, out);
+      }
+      if (HAS_Z) z[u] = load_rows(rz, c + 4, out);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
+    };
+    // Ends of blocks are asked for a turn before they are looked at, and not looked at behind reads of LDS.
+    float end[2] = {};
+    const auto next_ends = [&](int c) __attribute__((always_inline)) {
+      if (MODE == FACTORS) return;
+      asm volatile("" ::: "memory");
+      end[0] = ends[0][min(c, p.turns - 1)];
+      end[1] = NH == 2 ? ends[1][min(c, p.turns - 1)] : end[0];
+    };
+    next_ends(0);
+    walk_barrier();                                          // (the products' first fragments)
+    stage(0, 0, end);
+    next_ends(1);
+    walk_barrier();
+    for (int c0 = 0; c0 < p.turns; c0 += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int c = c0 + u, before = (u + 3) & 3;
+        const float to[2] = {end[0], end[1]};
+        if (MODE != FACTORS) asm volatile("" ::"s"(to[0]), "s"(to[1]) : "memory");
+        next_ends(c + 2);
+        const Parts parts = read_parts(before);              // of block c - 1 (before the first: values whose store is dropped)
+        const float up = grow[before & 1];
+        float dx[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dx[j] = skip[before & 1][j];
+        stage(c + 1, (u + 1) & 3, to);                       // of the block after the last: values that nothing reads
+        gate(c - 1, before, parts, up, dx);
+        walk_barrier();
+      }
     }
+    gate(p.turns - 1, 3, read_parts(3), grow[1], skip[1]);
   };
-  struct Parts { float4 a0, a1, b0, b1; };
-  const auto read_parts = [&](int u) __attribute__((always_inline)) {
-    const unsigned char *half = lds + (u & 1) * L::PARTS;
-    return Parts{*reinterpret_cast<const float4 *>(half + q0), *reinterpret_cast<const float4 *>(half + q1),
-                 *reinterpret_cast<const float4 *>(half + 8192 + q0), *reinterpret_cast<const float4 *>(half + 8192 + q1)};
-  };
-  const auto gate = [&](int c, int u, const Parts &r, float up, const float (&dx)[8]) __attribute__((always_inline)) {
-    float v[8] = {r.a0.x + r.b0.x, r.a0.y + r.b0.y, r.a0.z + r.b0.z, r.a0.w + r.b0.w, r.a1.x + r.b1.x, r.a1.y + r.b1.y, r.a1.z + r.b1.z, r.a1.w + r.b1.w};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (FACTOR) v[j] = DMODE == 0 ? v[j] * up : __builtin_fmaf(v[j], up, dx[j]);
-      else if (DMODE != 0) v[j] += dx[j];
-    }
-    if (HAS_Z) {
-      float zf[8];
-      asm volatile("" : "+v"(z[u]));
-      unpack8(z[u], zf);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] *= silu_f32(zf[j]);
-    }
-    const V8<E> out = pack8_e<E>(v);
-    if constexpr (FACTOR) {
-      if (c >= 0) note_overflow(seen, out);
-    }
-    if (HAS_Z) z[u] = load_rows(rz, c + 4, out);
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
-  };
-  if (!FACTOR) {
-    publish(0);
-    publish(1);
-  }
-  walk_barrier();                                          // (the products' first fragments; the first steps)
-  stage(0, 0);
-  walk_barrier();
-  for (int c0 = 0; c0 < p.turns; c0 += 4) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = c0 + u, before = (u + 3) & 3;
-      const Parts parts = read_parts(before);              // of block c - 1 (before the first: values whose store is dropped)
-      const float up = grow[before & 1];
-      float dx[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dx[j] = skip[before & 1][j];
-      if (!FACTOR) publish((u + 2) & 3);
-      stage(c + 1, (u + 1) & 3);                           // of the block after the last: values that nothing reads
-      gate(c - 1, before, parts, up, dx);
-      walk_barrier();
-    }
-  }
-  gate(p.turns - 1, 3, read_parts(3), grow[1], skip[1]);
+  in_mode(rows);
   return __any(noted_overflow(seen));
 }
 
-// The four waves of products of a head that does not factor.  Turn c: block c.
-template <typename E, int N, bool GROW>
-__device__ __forceinline__ void plain_products(const SsdWalkParams &p, unsigned char *lds, int b, int h) {
-  using L = WalkLds<1>;
-  constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16;
-  const int wave = wave_id_uniform(), lane = lane_id();
-  const int m = lane & 31, g2 = lane >> 5, pt = wave & 1, nh = wave >> 1;
-
-  // a lane's addresses for transposing reads (transposed_frag), and of its row m among the part sums
-  const int k = lane & 15, tr_row = 8 * g2 + (k >> 2), tr_piece = 4 * pt + 2 * (lane >> 4 & 1) + ((k & 3) >> 1);
-  const int tr0 = tr_row * 128 + ((tr_piece ^ (k >> 2)) << 4) + (k & 1) * 8, tr1 = (tr0 + 512) ^ 64;
-  unsigned char *const part = lds + L::PART + (2 * nh + pt) * 4096 + m * 128;
-
-  // fragments of block c, this wave's part
-  const size_t unit0 = (size_t)b * p.nblocks * p.groups + h / (p.heads / p.groups);
-  const E *pc = reinterpret_cast<const E *>(p.Cblk) + (unit0 * KN + 2 * nh * TPW) * SSD_FRAG;
-  const E *pb = reinterpret_cast<const E *>(p.Btblk) + (unit0 * 2 * NT + nh * TPW) * SSD_FRAG;
-  const unsigned lane16 = (unsigned)lane * 16;
-  const auto c_frag = [&](int c, int i, int t) { return *at_bytes<const V8<E>>(pc + (size_t)(c * p.groups) * (KN * SSD_FRAG) + (2 * i + t) * SSD_FRAG, lane16); };
-  const auto b_frag = [&](int c, int i, int ks) { return *at_bytes<const V8<E>>(pb + (size_t)(c * p.groups) * (KN * SSD_FRAG) + (ks * NT + i) * SSD_FRAG, lane16); };
-
-  f32x16_t S[TPW];
-  f32x16_t entered[GROW ? TPW : 1];                        // growing: the state entering the chunk
-  const size_t state0 = (((size_t)b * p.heads + h) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    S[i] = (f32x16_t){0};
-    if (p.init) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) S[i][r] = p.init[state0 + 32 * i + crow(r, g2)];
-    }
-  }
-  V8<E> cf[TPW][2], bf[TPW][2];
-  // requested a block ahead (by a growing head, which keeps twice the state, where they are used)
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      // without a state to start from the first block's product with it is zero whatever C holds
-      cf[i][t] = V8<E>{};
-      if (!GROW && p.init) cf[i][t] = c_frag(0, i, t);
-      if (!GROW) bf[i][t] = b_frag(0, i, t);
-    }
-  }
-  float base = 0.0f;                                       // growing: running sum up to the block, from its chunk's first step
-
-  walk_barrier();
-  for (int c = 0; c < p.turns; ++c) {                      // turns past the last block: steps of size zero
-    const float *st = reinterpret_cast<const float *>(lds + PlainLds::STEPS + (c & 3) * PlainLds::STEP_BYTES);
-    const unsigned char *xwt = lds + (c & 1) * L::X, *xt = xwt + WK_TILE;
-    const int next = min(c + 1, p.nblocks - 1);
-    walk_barrier();
-    const float own = st[m] + st[31], end = 2.0f * st[31];
-    if (GROW && c % p.chunk_blocks == 0) {
-#pragma unroll
-      for (int i = 0; i < TPW; ++i) {
-        entered[i] = S[i];
-        S[i] = (f32x16_t){0};
-      }
-      base = 0.0f;
-    }
-    f32x16_t acc = {0};
-    f32x16_t acc_h = {0};
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (GROW) {
-          V8<E> cg{};
-          if (c || p.init) cg = c_frag(min(c, p.nblocks - 1), i, t);
-          acc = mma(state_frag<E>(S[i], t), cg, acc);
-          acc_h = mma(state_frag<E>(entered[i], t), cg, acc_h);
-        } else {
-          acc = mma(state_frag<E>(S[i], t), cf[i][t], acc);
-          cf[i][t] = c_frag(next, i, t);
-        }
-      }
-    }
-    const float f = exp2_hw(GROW ? fminf(own, 0.0f) : own);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] *= f;
-    if (GROW) {
-      const float fh = fminf(exp2_hw(base + own), 3.0e38f);      // (finite: what is zero stays zero)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(acc_h[r], fh, acc[r]);
-    }
-    const float gs = exp2_hw(GROW ? fminf(end, 0.0f) : end);
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) S[i][r] *= gs;
-    }
-    acc = mma(transposed_frag<E>(xt, tr0 + nh * 2048, tr1 + nh * 2048),
-              load_frag_e<E>(lds + PlainLds::W + (c & 1) * 2048 + nh * 1024 + lane * 16), acc);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const V8<E> xf = transposed_frag<E>(xwt, tr0 + ks * 2048, tr1 + ks * 2048);
-#pragma unroll
-      for (int i = 0; i < TPW; ++i) {
-        if (GROW) {
-          S[i] = mma(b_frag(min(c, p.nblocks - 1), i, ks), xf, S[i]);
-        } else {
-          S[i] = mma(bf[i][ks], xf, S[i]);
-          bf[i][ks] = b_frag(next, i, ks);
-        }
-      }
-    }
-    if (GROW) {
-      base += end;
-      if ((c + 1) % p.chunk_blocks == 0 || c + 1 == p.turns) {
-        const float gh = fminf(exp2_hw(base), 3.0e38f);
-#pragma unroll
-        for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) S[i][r] = __builtin_fmaf(entered[i][r], gh, S[i][r]);
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      *reinterpret_cast<float4 *>(part + (c & 1) * L::PARTS + (((2 * q + g2) ^ (m & 7)) << 4)) =
-          make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-    }
-  }
-  walk_barrier();
-
-  if (p.final_states) {
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4 *>(p.final_states + state0 + 32 * i + 8 * q + 4 * g2) =
-            make_float4(S[i][4 * q], S[i][4 * q + 1], S[i][4 * q + 2], S[i][4 * q + 3]);
-    }
-  }
-}
-
-// The four waves of products of heads that factor.  Turn c: block c.  Final states are written once `settled` (asked when this
-// wave's share of the heads is done, with whether it left the range) has said that they stand.
-template <typename E, int NH, int N, typename Settled>
-__device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const Settled &settled) {
-  using F = WalkLds<NH>;
-  using L = FactoredLds<NH, N>;
+// The four waves of products.  Turn c: block c.  Final states are written once `settled` (asked when this wave's share of the
+// heads is done, with whether it left the range) has said that they stand.
+template <typename E, int NH, int N, typename InMode, typename Settled>
+__device__ __forceinline__ void walk_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const InMode &in_mode, const Settled &settled) {
+  using L = WalkLds<NH, N>;
   constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16, SHARE = KN / 4;
   const int wave = wave_id_uniform(), lane = lane_id();
   const int m = lane & 31, g2 = lane >> 5, pt = wave & 1, nh = wave >> 1;
   const int k = lane & 15, tr_row = 8 * g2 + (k >> 2), tr_piece = 4 * pt + 2 * (lane >> 4 & 1) + ((k & 3) >> 1);
   const int tr0 = tr_row * 128 + ((tr_piece ^ (k >> 2)) << 4) + (k & 1) * 8, tr1 = (tr0 + 512) ^ 64;
-  unsigned char *const part = lds + F::PART + (2 * nh + pt) * 4096 + m * 128;
+  unsigned char *const part = lds + L::PART + (2 * nh + pt) * 4096 + m * 128;
   const scalar_floats ends[2] = {hp.ends(p, 0), hp.ends(p, NH - 1)};
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds;
   const unsigned lane16 = (unsigned)lane * 16;
@@ -472,20 +332,6 @@ __device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsign
   };
   const auto frag = [&](int at) { return load_frag_e<E>(lds + at + lane16); };
 
-  f32x16_t S[NH][TPW];
-  size_t state0[NH];
-#pragma unroll
-  for (int hd = 0; hd < NH; ++hd) {
-    state0[hd] = (((size_t)hp.b * p.heads + (hd ? hp.h1 : hp.h0)) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      S[hd][i] = (f32x16_t){0};
-      if (p.init) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) S[hd][i][r] = p.init[state0[hd] + 32 * i + crow(r, g2)];
-      }
-    }
-  }
   request_c(1, 1);
   request_c(2, 2);
   request_b(0, 0);
@@ -497,151 +343,261 @@ __device__ __forceinline__ void factored_products(const SsdWalkParams &p, unsign
 #pragma unroll
     for (int i = 0; i < SHARE; ++i) *reinterpret_cast<V8<E> *>(lds + L::C + (SHARE * wave + i) * 1024 + lane16) = V8<E>{};
   }
-  wait_memory<0>();
-  walk_barrier();
-  __builtin_amdgcn_s_setprio(1);
-  float end[NH] = {};
-  for (int c = 0, t3 = 0; c < p.turns; ++c) {              // turns past the last block: steps of size zero
-    const int last3 = t3 == 0 ? 2 : t3 - 1;
-    // in the turn of the block before, c - 1: the state, brought from the middle of that block to the middle of this one
-    f32x16_t acc[NH];
+  const auto products = [&](auto mode) __attribute__((always_inline)) {
+    constexpr WalkMode MODE = decltype(mode)::value;
+    static_assert(MODE != GROWS || NH == 1 || N == 64);      // (registers)
+    f32x16_t S[NH][TPW];
+    size_t state0[NH];
 #pragma unroll
     for (int hd = 0; hd < NH; ++hd) {
-      const float e = ends[hd][c];
-      float to_here = 0.5f * (end[hd] + e);
-      if (to_here < -120.0f) {                             // a factor that float32 does not hold, in two that it does
-        const float g = exp2_hw(0.5f * end[hd]);
+      state0[hd] = (((size_t)hp.b * p.heads + (hd ? hp.h1 : hp.h0)) * SSD_P + 32 * pt + m) * N + 32 * nh * TPW;
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        S[hd][i] = (f32x16_t){0};
+        if (p.init) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[hd][i][r] = p.init[state0[hd] + 32 * i + crow(r, g2)];
+        }
+      }
+    }
+    wait_memory<0>();
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) {                        // (said to the compiler too: it would wait inside the loop)
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) asm volatile("" : "+v"(S[hd][i]));
+    }
+    walk_barrier();
+    __builtin_amdgcn_s_setprio(1);
+    f32x16_t entered[MODE == GROWS ? NH : 1][TPW];           // the state entering the chunk,
+    float base[NH] = {};                                     // and the running sum up to the block, from the chunk's first step
+    float held[NH] = {}, next[NH];                           // from the block's middle, where the state is held, to its end
+#pragma unroll
+    for (int hd = 0; hd < NH; ++hd) next[hd] = ends[hd][0];
+    for (int c = 0, t3 = 0; c < p.turns; ++c) {              // turns past the last block: steps of size zero
+      const int last3 = t3 == 0 ? 2 : t3 - 1;
+      float end[NH];
+#pragma unroll
+      for (int hd = 0; hd < NH; ++hd) end[hd] = next[hd];
+      // in the turn of the block before, c - 1: the state, brought from the middle of that block to the middle of this one
+      f32x16_t acc[NH], acc_entered[MODE == GROWS ? NH : 1];
+      const bool any_entered = c >= p.chunk_blocks || p.init;
+      if (MODE == GROWS && c % p.chunk_blocks == 0) {
+#pragma unroll
+        for (int hd = 0; hd < NH; ++hd) {
+#pragma unroll
+          for (int i = 0; i < TPW; ++i) {
+            entered[hd][i] = S[hd][i];
+            S[hd][i] = (f32x16_t){0};
+          }
+          base[hd] = 0.0f;
+        }
+      }
+#pragma unroll
+      for (int hd = 0; hd < NH; ++hd) {
+        if (MODE == FACTORS) {
+          const float here = 0.5f * end[hd];
+          float to_here = held[hd] + here;
+          if (to_here < -120.0f) {                           // a factor that float32 does not hold, in two that it does
+            const float g = exp2_hw(held[hd]);
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+              for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+            }
+            to_here = here;
+          }
+          const float g = exp2_hw(to_here);
+          held[hd] = here;
+#pragma unroll
+          for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+          }
+        }
+        acc[hd] = (f32x16_t){0};
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+          for (int t = 0; t < 2; ++t) acc[hd] = mma(state_frag<E>(S[hd][i], t), frag(L::C + (t3 * KN + 2 * (nh * TPW + i) + t) * 1024), acc[hd]);
         }
-        to_here = 0.5f * e;
+        if (MODE == GROWS) {
+          acc_entered[hd] = (f32x16_t){0};
+          if (N == 64 || any_entered) {
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+              for (int t = 0; t < 2; ++t)
+                acc_entered[hd] = mma(state_frag<E>(entered[hd][i], t), frag(L::C + (t3 * KN + 2 * (nh * TPW + i) + t) * 1024), acc_entered[hd]);
+            }
+          }
+        }
       }
-      const float g = exp2_hw(to_here);
-      end[hd] = e;
-      acc[hd] = (f32x16_t){0};
+      if (wave < 2) wait_memory<2 * SHARE + 1>();            // what turn c - 1 requested may be under way, no more
+      else wait_memory<2 * SHARE>();
+      walk_barrier();
+      request_c(c + 3, t3);
+      request_b(c + 2, last3);
 #pragma unroll
-      for (int i = 0; i < TPW; ++i) {
+      for (int hd = 0; hd < NH; ++hd) next[hd] = ends[hd][min(c + 1, p.turns - 1)];
+      const V8<E> cb = frag(L::CB + t3 * 2048 + nh * 1024);
+      V8<E> w[NH];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
+      for (int hd = 0; hd < NH; ++hd) {
+        w[hd] = cb;
+        if (MODE == FACTORS) continue;
+        const float *st = reinterpret_cast<const float *>(lds + L::STEP + ((c & 1) * NH + hd) * L::STEPS), own = st[m];
+        const float f = exp2_hw(MODE == GROWS ? fminf(own, 0.0f) : own);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[hd] = mma(state_frag<E>(S[hd][i], t), frag(L::C + (t3 * KN + 2 * (nh * TPW + i) + t) * 1024), acc[hd]);
+        for (int r = 0; r < 16; ++r) acc[hd][r] *= f;
+        if (MODE == GROWS) {
+          const float fh = fminf(exp2_hw(base[hd] + own), 3.0e38f);    // (finite: what is zero stays zero)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[hd][r] = __builtin_fmaf(acc_entered[hd][r], fh, acc[hd][r]);
+        }
+        // dt_s exp(min(cs_l - cs_s, 0)) as one exponential: min(a, 0) + b = min(a + b, b) with b = log2 dt_s.  The bound is
+        // inactive on and below the diagonal of a decaying head, is the clamp of a growing one, and keeps the places above
+        // the diagonal (zeros of C.B) finite.
+#pragma unroll
+        for (int k4 = 0; k4 < 2; ++k4) {
+          const float4 e4 = *reinterpret_cast<const float4 *>(st + WK + 16 * nh + 8 * g2 + 4 * k4);
+          const float4 l4 = *reinterpret_cast<const float4 *>(st + 2 * WK + 16 * nh + 8 * g2 + 4 * k4);
+          const float e[4] = {e4.x, e4.y, e4.z, e4.w}, l2[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[hd][4 * k4 + j] = (E)((float)cb[4 * k4 + j] * exp2_hw(fminf(own + e[j], l2[j])));
+        }
+        const float gs = exp2_hw(MODE == GROWS ? fminf(end[hd], 0.0f) : end[hd]);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[hd][i][r] *= gs;
+        }
       }
-    }
-    if (wave < 2) wait_memory<2 * SHARE + 1>();            // what turn c - 1 requested may be under way, no more
-    else wait_memory<2 * SHARE>();
-    walk_barrier();
-    request_c(c + 3, t3);
-    request_b(c + 2, last3);
-    const V8<E> cb = frag(L::CB + t3 * 2048 + nh * 1024);
 #pragma unroll
-    for (int hd = 0; hd < NH; ++hd) {
-      const unsigned char *xt = lds + (c & 1) * F::X + hd * WK_TILE;
-      const V8<E> xf[2] = {transposed_frag<E>(xt, tr0, tr1), transposed_frag<E>(xt, tr0 + 2048, tr1 + 2048)};
-      acc[hd] = mma(nh ? xf[1] : xf[0], cb, acc[hd]);
-      acc[hd] = mma(transposed_frag<E>(xt + NH * WK_TILE, tr0 + 2048 * nh, tr1 + 2048 * nh), cb, acc[hd]);
+      for (int hd = 0; hd < NH; ++hd) {
+        const unsigned char *xt = lds + (c & 1) * L::X + hd * WK_TILE;
+        const V8<E> xf[2] = {transposed_frag<E>(xt, tr0, tr1), transposed_frag<E>(xt, tr0 + 2048, tr1 + 2048)};
+        if (MODE == FACTORS) acc[hd] = mma(nh ? xf[1] : xf[0], cb, acc[hd]);
+        acc[hd] = mma(transposed_frag<E>(xt + NH * WK_TILE, tr0 + 2048 * nh, tr1 + 2048 * nh), w[hd], acc[hd]);
 #pragma unroll
-      for (int i = 0; i < TPW; ++i) {
+        for (int i = 0; i < TPW; ++i) {
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) S[hd][i] = mma(frag(L::B + (t3 * KN + ks * NT + nh * TPW + i) * 1024), xf[ks], S[hd][i]);
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4 *>(part + (c & 1) * F::PARTS + hd * 16384 + (((2 * q + g2) ^ (m & 7)) << 4)) =
-            make_float4(acc[hd][4 * q], acc[hd][4 * q + 1], acc[hd][4 * q + 2], acc[hd][4 * q + 3]);
-    }
-    t3 = t3 == 2 ? 0 : t3 + 1;
-  }
-  walk_barrier();
-  wait_memory<0>();                                        // nothing may land in LDS that is others' by then
-  float zero = 0.0f;                                       // no number once a state is infinite or none
-#pragma unroll
-  for (int hd = 0; hd < NH; ++hd) {
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) zero = __builtin_fmaf(S[hd][i][r], 0.0f, zero);
-    }
-  }
-  if (settled(__any(zero != 0.0f)) && p.final_states) {
-#pragma unroll
-    for (int hd = 0; hd < NH; ++hd) {
-      const float g = exp2_hw(0.5f * end[hd]);
-      if (hd && !hp.two) break;
-#pragma unroll
-      for (int i = 0; i < TPW; ++i) {
+          for (int ks = 0; ks < 2; ++ks) S[hd][i] = mma(frag(L::B + (t3 * KN + ks * NT + nh * TPW + i) * 1024), xf[ks], S[hd][i]);
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<float4 *>(p.final_states + state0[hd] + 32 * i + 8 * q + 4 * g2) =
-              make_float4(S[hd][i][4 * q] * g, S[hd][i][4 * q + 1] * g, S[hd][i][4 * q + 2] * g, S[hd][i][4 * q + 3] * g);
+          *reinterpret_cast<float4 *>(part + (c & 1) * L::PARTS + hd * 16384 + (((2 * q + g2) ^ (m & 7)) << 4)) =
+              make_float4(acc[hd][4 * q], acc[hd][4 * q + 1], acc[hd][4 * q + 2], acc[hd][4 * q + 3]);
       }
+      if (MODE == GROWS) {
+        const bool last = (c + 1) % p.chunk_blocks == 0 || c + 1 == p.turns;
+#pragma unroll
+        for (int hd = 0; hd < NH; ++hd) {
+          base[hd] += end[hd];
+          if (last) {
+            const float gh = fminf(exp2_hw(base[hd]), 3.0e38f);
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+              for (int r = 0; r < 16; ++r) S[hd][i][r] = __builtin_fmaf(entered[hd][i][r], gh, S[hd][i][r]);
+            }
+          }
+        }
+      }
+      t3 = t3 == 2 ? 0 : t3 + 1;
     }
-  }
+    walk_barrier();
+    wait_memory<0>();                                        // nothing may land in LDS that is others' by then
+    // (a walk after this one writes what was not good once more, and may take the state it starts from out of the same place)
+    const auto write_states = [&] {
+#pragma unroll
+      for (int hd = 0; hd < NH; ++hd) {
+        const float g = MODE == FACTORS ? exp2_hw(held[hd]) : 1.0f;
+        if (hd && !hp.two) break;
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4 *>(p.final_states + state0[hd] + 32 * i + 8 * q + 4 * g2) =
+                make_float4(S[hd][i][4 * q] * g, S[hd][i][4 * q + 1] * g, S[hd][i][4 * q + 2] * g, S[hd][i][4 * q + 3] * g);
+        }
+      }
+    };
+    const bool in_place = p.final_states == p.init;          // (or neither)
+    if (!in_place && p.final_states) write_states();
+    bool left = false;
+    if (MODE == FACTORS && p.final_states) {                 // (a state that no y has seen)
+      float most[2] = {};                                    // passes on what is no number
+#pragma unroll
+      for (int hd = 0; hd < NH; ++hd) {
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(most[r >> 1 & 1]) : "v"(S[hd][i][r]), "v"(S[hd][i][r + 1]));
+        }
+      }
+      left = !__all(most[0] < __builtin_inff() && most[1] < __builtin_inff());
+    }
+    if (settled(left) && in_place && p.final_states) write_states();
+  };
+  in_mode(products);
 }
 
-// Whether all of the heads' blocks decay by at most WALK_RANGE (in powers of two), and none grows.
-template <int NH>
-__device__ __forceinline__ bool decays_factor(const SsdWalkParams &p, const WalkHeads<NH> &hp) {
-  const float *e0 = p.ends + ((size_t)hp.b * p.heads + hp.h0) * p.turns, *e1 = p.ends + ((size_t)hp.b * p.heads + hp.h1) * p.turns;
-  bool ok = p.A[hp.h0] <= 0.0f && p.A[hp.h1] <= 0.0f;
-  for (int c = lane_id(); c < p.turns; c += WAVE) ok = ok && e0[c] >= -WALK_RANGE && e0[c] <= 0.0f && e1[c] >= -WALK_RANGE && e1[c] <= 0.0f;
-  return __all(ok);
+// One walk over the heads; whether what it wrote stands.
+template <typename E, int NH, int N, int DMODE, bool HAS_Z, bool KEEP_ENTERED>
+__device__ __forceinline__ bool walk(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, bool factor = false) {
+  int *again = reinterpret_cast<int *>(lds + WalkLds<NH, N>::AGAIN);
+  if (threadIdx.x == 0) *again = 0;
+  bool stands;
+  const auto settled = [&](bool left_range) {
+    if (left_range) *again = 1;
+    walk_barrier();
+    stands = __builtin_amdgcn_readfirstlane(*again) == 0;
+    walk_barrier();                                        // LDS is others' to write
+    return stands;
+  };
+  const auto in_mode = [&](const auto &part) __attribute__((always_inline)) {
+    if constexpr (KEEP_ENTERED) part(walk_mode<GROWS>{});
+    else if constexpr (std::is_same<E, _Float16>::value) part(walk_mode<ELEMENTS>{});
+    else if (factor) part(walk_mode<FACTORS>{});
+    else part(walk_mode<ELEMENTS>{});
+  };
+  if (wave_id_uniform() >= 4) settled(walk_rows<E, NH, N, DMODE, HAS_Z>(p, lds, hp, in_mode));
+  else walk_products<E, NH, N>(p, lds, hp, in_mode, settled);
+  return stands;
 }
 
-constexpr int PLAIN_THREADS = 512;
-template <typename E, int N, int DMODE, bool HAS_Z>
-__device__ __forceinline__ void plain_head(const SsdWalkParams &p, unsigned char *lds, int b, int h) {
-  if (wave_id_uniform() >= 4) walk_rows<E, 1, DMODE, HAS_Z, false>(p, lds, WalkHeads<1>(p, b, h));
-  else if (p.A[h] > 0.0f) plain_products<E, N, true>(p, lds, b, h);
-  else plain_products<E, N, false>(p, lds, b, h);
-}
-
-constexpr int walk_threads(int nh) { return nh == 2 ? 768 : PLAIN_THREADS; }
+constexpr int walk_threads(int nh) { return nh == 2 ? 768 : 512; }
 
 // (xcd_order: neighbouring heads of a batch row, which read the same fragments, go to one XCD.)
-// NH = 0: no head factors, one per workgroup.  Else those that do, NH of them per workgroup, and behind them a workgroup for
-// each head again, which most of the time finds nothing to do.
 template <typename E, int NH, int N, int DMODE, bool HAS_Z>
-__global__ __launch_bounds__(walk_threads(NH)) __attribute__((amdgpu_waves_per_eu(NH == 0 ? 4 : NH + 1)))
+__global__ __launch_bounds__(walk_threads(NH)) __attribute__((amdgpu_waves_per_eu(NH + 1)))
 void ssd_walk_kernel(const SsdWalkParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
-  if constexpr (NH == 0) {
-    const int vid = (int)xcd_order(blockIdx.x, gridDim.x);
-    plain_head<E, N, DMODE, HAS_Z>(p, lds, vid / p.heads, vid % p.heads);
-  } else if (blockIdx.x < (unsigned)p.sets) {
-    const WalkHeads<NH> hp(p, (int)xcd_order(blockIdx.x, p.sets));
-    if (!decays_factor(p, hp)) return;
-    int *again = reinterpret_cast<int *>(lds + FactoredLds<NH, N>::AGAIN);
-    if (threadIdx.x == 0) *again = 0;
-    const auto settled = [&](bool left_range) {
-      if (left_range) *again = 1;
-      walk_barrier();
-      const int v = __builtin_amdgcn_readfirstlane(*again);
-      walk_barrier();                                      // LDS is others' to write
-      return v == 0;
-    };
-    bool done = true;
-    if (wave_id_uniform() >= 4) done = settled(walk_rows<E, NH, DMODE, HAS_Z, true>(p, lds, hp));
-    else factored_products<E, NH, N>(p, lds, hp, [&](bool left_range) { return done = settled(left_range); });
-    if (done || wave_id_uniform() >= PLAIN_THREADS / WAVE) return;
-    plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, hp.h0);
-    if (hp.two) {
-      walk_barrier();
-      plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, hp.h1);
-    }
+  const WalkHeads<NH> all(p, (int)xcd_order(blockIdx.x, p.sets));
+  const float A0 = p.A[all.h0], A1 = p.A[all.h1];          // (asked for together with what heads_factor reads)
+  const bool factor = std::is_same<E, __bf16>::value && heads_factor(p, all);
+  const bool grows0 = A0 > 0.0f, grows1 = A1 > 0.0f;
+  const WalkHeads<NH> one(all.b, all.g, grows0 ? all.h1 : all.h0);
+  bool stands = true;
+  if (!grows0 || !grows1) stands = walk<E, NH, N, DMODE, HAS_Z, false>(p, lds, grows0 == grows1 ? all : one, factor);
+  // those that grow, or left the range
+  if (stands && !grows0 && !grows1) return;
+  wait_memory<0>();                                        // what is written again is written after this
+  walk_barrier();
+  if constexpr (NH == 1 || N == 64) {
+    walk<E, NH, N, DMODE, HAS_Z, true>(p, lds, !stands || grows0 == grows1 ? all : WalkHeads<NH>(all.b, all.g, grows0 ? all.h0 : all.h1));
   } else {
-    const unsigned id = blockIdx.x - p.sets, second = NH == 2 ? id & 1 : 0;
-    const WalkHeads<NH> hp(p, (int)xcd_order(id / NH, p.sets));
-    if (wave_id_uniform() >= PLAIN_THREADS / WAVE || (second && !hp.two) || decays_factor(p, hp)) return;
-    plain_head<E, N, DMODE, HAS_Z>(p, lds, hp.b, second ? hp.h1 : hp.h0);
+    if (wave_id_uniform() >= walk_threads(1) / WAVE) return;
+#pragma nounroll
+    for (int second = 0; second < (all.two ? 2 : 1); ++second)
+      if (!stands || (second ? grows1 : grows0)) walk<E, 1, N, DMODE, HAS_Z, true>(p, lds, WalkHeads<1>(all.b, all.g, second ? all.h1 : all.h0));
   }
 }
 
 template <typename E, int NH, int N>
 static int launch_walk(const SsdWalkParams &p, int dmode, hipStream_t s) {
-  constexpr int LDS = NH && FactoredLds<NH ? NH : 1, N>::BYTES > PlainLds::BYTES ? FactoredLds<NH ? NH : 1, N>::BYTES : PlainLds::BYTES;
-  const unsigned grid = (unsigned)(NH == 0 ? p.batch * p.heads : p.sets * (1 + NH));
+  constexpr int LDS = WalkLds<NH, N>::BYTES;
+  const unsigned grid = (unsigned)p.sets;
 #define SSM_WALK(DM, HZ)                                                                              \
   {                                                                                                   \
     const auto kernel = ssd_walk_kernel<E, NH, N, DM, HZ>;                                            \
@@ -668,14 +624,15 @@ static int launch_walk(const SsdWalkParams &p, int dmode, hipStream_t s) {
 int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s) {
   const int per_group = p.heads / p.groups;
   // one head per workgroup while every workgroup has a CU of its own
-  const int nh = f16 ? 0 : p.batch * p.heads <= WALK_SINGLES ? 1 : 2;
-  p.sets = nh ? p.batch * p.groups * ((per_group + nh - 1) / nh) : 0;
-#define SSM_WALK_N(NN)                                                        \
-  return nh == 0   ? launch_walk<_Float16, 0, NN>(p, dmode, s)                \
-         : nh == 1 ? launch_walk<__bf16, 1, NN>(p, dmode, s)                  \
-                   : launch_walk<__bf16, 2, NN>(p, dmode, s);
-  if (nstate == 128) SSM_WALK_N(128)
-  SSM_WALK_N(64)
+  const int nh = p.batch * p.heads <= WALK_SINGLES ? 1 : 2;
+  p.sets = p.batch * p.groups * ((per_group + nh - 1) / nh);
+#define SSM_WALK_N(E, NN) return nh == 1 ? launch_walk<E, 1, NN>(p, dmode, s) : launch_walk<E, 2, NN>(p, dmode, s);
+  if (f16) {
+    if (nstate == 128) SSM_WALK_N(_Float16, 128)
+    SSM_WALK_N(_Float16, 64)
+  }
+  if (nstate == 128) SSM_WALK_N(__bf16, 128)
+  SSM_WALK_N(__bf16, 64)
 #undef SSM_WALK_N
 }
 
