@@ -23,6 +23,7 @@
 // exp(cs_l - cs_s) dt_s (C_l.B_s) per element instead, x weighted towards the block's end for the state.
 // The factors r - cs_s reach 2^80: where dt x is so large that x~, or what it is summed into, leaves bfloat16, a y or a state
 // comes out infinite or not a number, and the workgroup does its heads again per element, whose factors are at most 1.
+// In float16 the same is done where a state goes beyond 65504: the second time it is rounded to float16 scaled by a power of two.
 //
 // A growing head (A > 0): decays between steps of one of the call's chunks are bounded by 1, the factors on the state entering
 // the chunk are not (the published kernels evaluate exp(min(x, 0)) and exp(x) there).  Such a head goes per element and keeps
@@ -102,16 +103,24 @@ __device__ __forceinline__ V8<E> state_frag(const f32x16_t &s, int t) {
   return r;
 }
 
+// The larger of `most` and the sizes of two values, no number if one of them is none.
+__device__ __forceinline__ void note_size(float &most, float a, float b) { asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(a), "v"(b)); }
+
 // What the running sums of a block that factors are relative to: the sum at its middle.
 template <typename E>
 __device__ __forceinline__ float walk_middle(float end) { return std::is_same<E, __bf16>::value && walk_factors(end) ? 0.5f * end : 0.0f; }
 
-// Keeps in `seen` that one of eight values stored as bfloat16 was infinite or no number: read as float16 these bits are no
+// Keeps in `seen` that one of eight values stored was infinite or no number.  bfloat16: read as float16 these bits are no
 // number, nor are those from 2^121 on, and a maximum that passes on what is no number costs half an instruction a word.
 __device__ __forceinline__ void note_overflow(unsigned &seen, const V8<__bf16> &v) {
   const u32x4_t w = __builtin_bit_cast(u32x4_t, v);
   asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(seen) : "v"(w[0]), "v"(w[1]));
   asm("v_pk_maximum3_f16 %0, %1, %2, %0" : "+v"(seen) : "v"(w[2]), "v"(w[3]));
+}
+__device__ __forceinline__ void note_overflow(unsigned &seen, const V8<_Float16> &v) {
+  const u32x4_t w = __builtin_bit_cast(u32x4_t, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm("v_pk_fma_f16 %0, %1, 0, %0" : "+v"(seen) : "v"(w[i]));
 }
 __device__ __forceinline__ bool noted_overflow(unsigned seen) { return (seen & 0x7fffu) > 0x7c00u || (seen >> 16 & 0x7fffu) > 0x7c00u; }
 
@@ -160,6 +169,7 @@ __device__ __forceinline__ bool heads_factor(const SsdWalkParams &p, const WalkH
 template <typename E, int NH, int N, int DMODE, bool HAS_Z, typename InMode>
 __device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const InMode &in_mode) {
   using L = WalkLds<NH, N>;
+  constexpr bool F16 = std::is_same<E, _Float16>::value;
   const int wave = wave_id_uniform() - 4, lane = lane_id(), tid = wave * WAVE + lane;
   const int row = tid / (8 * NH), second = NH == 2 ? tid >> 3 & 1 : 0, piece = tid & 7;
   const unsigned pitch = (unsigned)p.heads * SSD_P * 2, block = WK * pitch;
@@ -258,9 +268,8 @@ __device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char 
         for (int j = 0; j < 8; ++j) v[j] *= silu_f32(zf[j]);
       }
       const V8<E> out = pack8_e<E>(v);
-      if constexpr (MODE == FACTORS) {
+      if (MODE == FACTORS || (F16 && MODE == ELEMENTS))
         if (c >= 0) note_overflow(seen, out);
-      }
       if (HAS_Z) z[u] = load_rows(rz, c + 4, out);
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
     };
@@ -305,6 +314,7 @@ __device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char 
 template <typename E, int NH, int N, typename InMode, typename Settled>
 __device__ __forceinline__ void walk_products(const SsdWalkParams &p, unsigned char *lds, const WalkHeads<NH> &hp, const InMode &in_mode, const Settled &settled) {
   using L = WalkLds<NH, N>;
+  constexpr bool F16 = std::is_same<E, _Float16>::value;
   constexpr int NT = N / 32, TPW = NT / 2, KN = N / 16, SHARE = KN / 4;
   const int wave = wave_id_uniform(), lane = lane_id();
   const int m = lane & 31, g2 = lane >> 5, pt = wave & 1, nh = wave >> 1;
@@ -414,6 +424,33 @@ __device__ __forceinline__ void walk_products(const SsdWalkParams &p, unsigned c
             for (int r = 0; r < 16; ++r) S[hd][i][r] *= g;
           }
         }
+        float up = 1.0f;
+        const auto scale_states = [&](float by) __attribute__((always_inline)) {
+#pragma unroll
+          for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              S[hd][i][r] *= by;
+              if (MODE == GROWS) entered[hd][i][r] *= by;
+            }
+          }
+        };
+        if (F16 && MODE == GROWS) {                          // a state that float16 does not hold
+          float most2[2] = {};
+#pragma unroll
+          for (int i = 0; i < TPW; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) note_size(most2[r & 1], S[hd][i][r], entered[hd][i][r]);
+          }
+          float most = fmaxf(most2[0], most2[1]);
+          if (__any(most >= 32768.0f)) {
+#pragma unroll
+            for (int other = 1; other < WAVE; other <<= 1) most = fmaxf(most, __shfl_xor(most, other, WAVE));
+            const int above = (int)(__float_as_uint(most) >> 23) - (127 + 14);
+            up = exp2_hw((float)above);
+            scale_states(exp2_hw((float)-above));
+          }
+        }
         acc[hd] = (f32x16_t){0};
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
@@ -422,12 +459,20 @@ __device__ __forceinline__ void walk_products(const SsdWalkParams &p, unsigned c
         }
         if (MODE == GROWS) {
           acc_entered[hd] = (f32x16_t){0};
-          if (N == 64 || any_entered) {
+          if ((N == 64 && NH == 1) || any_entered) {
 #pragma unroll
             for (int i = 0; i < TPW; ++i) {
 #pragma unroll
               for (int t = 0; t < 2; ++t)
                 acc_entered[hd] = mma(state_frag<E>(entered[hd][i], t), frag(L::C + (t3 * KN + 2 * (nh * TPW + i) + t) * 1024), acc_entered[hd]);
+            }
+          }
+          if (F16 && up != 1.0f) {
+            scale_states(up);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              acc[hd][r] *= up;
+              acc_entered[hd][r] *= up;
             }
           }
         }
@@ -526,13 +571,13 @@ __device__ __forceinline__ void walk_products(const SsdWalkParams &p, unsigned c
     if (!in_place && p.final_states) write_states();
     bool left = false;
     if (MODE == FACTORS && p.final_states) {                 // (a state that no y has seen)
-      float most[2] = {};                                    // passes on what is no number
+      float most[2] = {};
 #pragma unroll
       for (int hd = 0; hd < NH; ++hd) {
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
 #pragma unroll
-          for (int r = 0; r < 16; r += 2) asm("v_maximum3_f32 %0, |%1|, |%2|, %0" : "+v"(most[r >> 1 & 1]) : "v"(S[hd][i][r]), "v"(S[hd][i][r + 1]));
+          for (int r = 0; r < 16; r += 2) note_size(most[r >> 1 & 1], S[hd][i][r], S[hd][i][r + 1]);
         }
       }
       left = !__all(most[0] < __builtin_inff() && most[1] < __builtin_inff());
