@@ -80,9 +80,9 @@ template <int N>
 __device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 // 16 bytes per lane from memory to LDS, lane i to byte `at` + 16 i.  Written out, because the compiler would make every
-// later read of LDS wait for it; the waits are factored_products'.
+// later read of LDS wait for it; the waits are walk_products'.  `at` is asked for in m0, so that the compiler knows who has it.
 __device__ __forceinline__ void to_lds16(const void *base, unsigned off, unsigned at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(base) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(at), "v"(off), "s"(base) : "memory");
 }
 
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
