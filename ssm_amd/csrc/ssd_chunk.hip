@@ -8,9 +8,12 @@ namespace ssm {
 // or the chunks side by side (states through memory, twice x)?  Both times in us, heads counted over the batch.  The walk
 // takes a time per block of 32 steps that grows with the heads that share memory, and above 256 heads, two to a workgroup,
 // faster; 512 fill the chip.  The workgroups of the other way (one per chunk and head) share it, a little better while they
-// all fit.  Fitted to both routes, replayed as graphs, at 350 sizes (8 to 400 heads, 256 to 4096 steps):
+// all fit.  Fitted to both routes, replayed as graphs, at 350 sizes (8 to 400 heads, 256 to 4096 steps), and looked at again at
+// 390 (16 to 400 heads, 768 to 4096 steps, every chunk and state size) in either element type, one line for both: the route
+// taken is the faster one or within 5 % of it but at three of them in bfloat16 (11, 10 and 7 %), on average 0.1 % off.
 //   heads, 4096 steps, 128 states:       24         48         80         112        128        160        256        400
-//   walk / side by side, chunks of 256: 109 / 38   110 / 53   113 / 83   115 / 109  122 / 128  119 / 151  139 / 243  192 / 352
+//   walk / side by side, chunks of 256: 107 / 38   106 / 53   105 / 85   109 / 110  110 / 130  117 / 150  138 / 241  197 / 341
+//   float16                             113 / 39   113 / 55   116 / 87   118 / 112  123 / 131  124 / 151  146 / 243  215 / 357
 // Up to two chunks the walk is always the faster one (24 heads, 512 steps: 20.8 / 23.7).
 bool ssd_side_by_side(const SsdDims &d) {
   // the walk's offsets from the start of a head have 32 bits, some blocks past its end included
@@ -32,22 +35,6 @@ bool ssd_side_by_side(const SsdDims &d) {
   const Chunks &c = chunks[d.chunk > 128 ? 2 : d.chunk > 64][large];
   const double units = (double)heads * d.nchunks;
   return d.nchunks > 2 && walk > c.start + c.each * units + c.more * std::max(0.0, units - c.from);
-}
-
-// Callers size workspaces ahead of a call and keep them, so a shape goes on asking for what it did when the line between the
-// routes lay elsewhere: room for the states up to more heads, steps and running sums of whole chunks otherwise.
-size_t ssd_settled_workspace_bytes(const SsdDims &d) {
-  struct Chunks { double chunk, group, unit; };
-  static const Chunks chunks[3][2] = {{{3.8, 0.0032, 0.0167}, {4.5, 0.0026, 0.0264}},
-                                      {{4.1, 0.0060, 0.0262}, {5.2, 0.0059, 0.0355}},
-                                      {{6.5, 0.0124, 0.0421}, {7.0, 0.0139, 0.0536}}};
-  const Chunks &f = chunks[d.chunk > 128 ? 2 : d.chunk > 64][d.nstate > 64];
-  const int64_t halves = 2 * (int64_t)d.batch * d.heads;
-  const auto chunk = [&](int64_t n) { return n ? f.chunk + f.group * std::max(0.0, (double)n - 100.0) : 0.0; };
-  const double walk = 9.0 + d.nchunks * ((double)(halves / 768) * chunk(768) + chunk(halves % 768));
-  if (d.nchunks > 2 && walk > 16.0 + f.unit * 0.5 * (double)halves * d.nchunks) return ssd_work_layout(d, false, true).total;
-  const size_t steps = (size_t)d.nchunks * d.chunk, rows = (size_t)d.batch * steps * d.groups * 2;
-  return 2 * ssd_align_up((size_t)d.batch * d.heads * steps * sizeof(float)) + 2 * ssd_align_up(rows * d.nstate) + ssd_align_up(rows * d.chunk);
 }
 
 template <typename E, int Q, int N>

@@ -109,8 +109,6 @@ inline size_t ssd_align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Whether the forward takes the chunks side by side (ssd_chunk.hip) rather than one after the other (ssd_walk.hip).
 bool ssd_side_by_side(const SsdDims &d);
-// Bytes a forward's workspace has had for a shape since before the walk: what the query never goes below.
-size_t ssd_settled_workspace_bytes(const SsdDims &d);
 
 inline size_t ssd_added_bytes(const SsdDims &d) {
   return ssd_align_up((size_t)d.batch * d.nchunks * d.heads * SSD_P * d.nstate * sizeof(float));

@@ -328,7 +328,7 @@ extern "C" size_t ssm_ssd_combined_workspace_bytes(const ssm_ssd_dims *dims) {
 #ifdef SSM_TEST_HOOKS
   return std::max(ssm::ssd_work_layout(d, false, true).total, ssm::ssd_work_layout(d, false, false).total);
 #else
-  return std::max(ssm::ssd_work_layout(d, false, ssm::ssd_side_by_side(d)).total, ssm::ssd_settled_workspace_bytes(d));
+  return ssm::ssd_work_layout(d, false, ssm::ssd_side_by_side(d)).total;
 #endif
 }
 

@@ -189,19 +189,23 @@ def test_ssd_training_keeps_only_what_its_backward_reads():
 
 
 @pytest.mark.parametrize("chunk,nstate,heads,nchunks,side_by_side", [
-    (256, 128, 24, 16, True), (256, 128, 160, 16, True), (256, 128, 240, 8, False), (256, 128, 240, 32, False),
-    (256, 128, 320, 16, False), (256, 128, 400, 16, True), (256, 128, 512, 4, False), (256, 128, 820, 8, False),
-    (256, 64, 400, 16, True), (256, 64, 900, 4, False), (128, 128, 120, 8, True), (128, 128, 360, 16, False),
-    (64, 128, 120, 16, True), (64, 128, 240, 16, False), (64, 64, 24, 8, True), (64, 64, 700, 8, False),
-    (256, 128, 24, 2, False), (64, 64, 24, 2, False)])
+    (256, 128, 24, 16, True), (256, 128, 80, 8, True), (256, 128, 128, 16, False), (256, 128, 160, 16, False),
+    (256, 128, 400, 16, False), (256, 64, 80, 16, True), (256, 64, 128, 16, False), (256, 64, 160, 8, False),
+    (128, 128, 24, 8, True), (128, 128, 80, 16, True), (128, 128, 112, 16, False), (128, 64, 48, 16, True),
+    (128, 64, 112, 16, False), (64, 128, 24, 16, True), (64, 128, 80, 16, False), (64, 64, 24, 32, True),
+    (64, 64, 112, 32, False), (256, 128, 24, 2, False), (64, 64, 24, 2, False)])
 def test_the_faster_route_of_the_combined_ssd_is_taken(chunk, nstate, heads, nchunks, side_by_side):
-    """Sizes at which both routes were timed (csrc/ssd_chunk.hip) and are more than 3 % apart.  The chunks side by side
-    need room for the states; one pass over the sequence does not, and its workspace is what is left of a call's."""
+    """Sizes on both sides of the line (csrc/ssd_chunk.hip) at which both routes were timed, in bfloat16 and float16, and are
+    more than 3 % apart.  A forward needs the workspace of the route it takes: the chunks side by side room for the states, one
+    pass over the sequence none, but steps and fragments alone."""
     L = _lib()
-    d = L.SsdDims(batch=2, seqlen=nchunks * chunk - 3, heads=heads // 2, headdim=64, groups=1, nstate=nstate, chunk=chunk)
-    steps = 2 * nchunks * chunk
-    one_pass = steps * heads // 2 * 8 + 2 * steps * nstate * 2 + steps * chunk * 2 + 8 * 256
-    assert (L.load().ssm_ssd_combined_workspace_bytes(ctypes.byref(d)) > one_pass) == side_by_side
+    length = nchunks * chunk - 3
+    d = L.SsdDims(batch=2, seqlen=length, heads=heads // 2, headdim=64, groups=1, nstate=nstate, chunk=chunk)
+    steps, blocks = 2 * 128 * (-(-length // 128)), 2 * 32 * (-(-length // 32))
+    one_pass = steps * heads // 2 * (8 + 4 / 32) + blocks * (2 * nstate + 32) * 2
+    states = nchunks * heads * 64 * nstate * 2
+    got = L.load().ssm_ssd_combined_workspace_bytes(ctypes.byref(d))
+    assert got >= states + one_pass / 2 if side_by_side else one_pass <= got <= one_pass + 8 * 256
 
 
 def test_shipped_library_has_no_test_hooks_and_the_hooks_build_does():
