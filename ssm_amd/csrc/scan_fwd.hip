@@ -19,20 +19,21 @@ extern template int scan_fwd_fast_dispatch<f16_t, float>(const ScanFwdParams &, 
 // 16 states in turn / side by side:
 //   grouped, float32, 512 x 2048 31.7 / 15.0, 768 x 8192 109 / 93, 1024 x 2048 30.7 / 25.7, 1024 x 4096 58 / 67,
 //   1280 x 2048 32 / 29.9, 1536 x 1024 18.1 / 16.7, 1536 x 2048 32.8 / 33.7;
-//   bf16 512 x 2048 32.2 / 13.8, 1280 x 1024 16.6 / 14.3, 1280 x 8192 104 / 93.5, 1536 x 1024 16.6 / 17.2,
-//   1536 x 2048 29.0 / 27.7, 1536 x 4096 56 / 59.
+//   bf16 512 x 2048 32.2 / 13.8, 1280 x 1024 16.6 / 14.3, 1280 x 8192 104 / 93.5, 3 x 512 x 1024 21.2 / 19.6, x 2048 29.0 /
+//   27.7, x 4096 63.0 / 61.8, x 8192 118 / 117; with 4 states x 4096 31.5 / 27.0, x 8192 56 / 49.
+//   float32 of few states, whose rows two waves do not share (below): 1024 x 4096, 1 state 25.5 / 23.0.
 //   Every wave reads B and C itself there, and runs of odd rows at a lower rate: float32 512 x 2047 33 / 23, 768 x 2047
 //   33 / 42, bf16 768 x 2047 32 / 27, 768 x 1021 18.6 / 19.5, 768 x 3000 48 / 67.
 //   Few channels to a group (a row per wave in turn): 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
 //   Constant projections: 256 x 2048 18.4 / 10.2, 512 x 8192 68 / 43, 512 x 1024 10.6 / 10.9, 1024 x 4096 41 / 43.
-static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged) {
+static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged, bool few) {
   if (len <= FAST_T) return false;
   if (!varying) return rows <= (len > 2 * FAST_T ? 512 : 384);
   const bool to_four = len > 2 * FAST_T && len <= 4 * FAST_T;       // chunks
   if (ragged) return rows <= (grouped && half && to_four ? 768 : 512);
   if (!grouped) return rows <= (half ? 1536 : 1024);
-  if (half) return rows <= (to_four ? 1536 : 1280);
-  return rows <= (len <= 2 * FAST_T ? 1536 : len <= 4 * FAST_T ? 1280 : 768);
+  if (half) return rows <= 1536;
+  return rows <= (len <= 2 * FAST_T ? 1536 : len <= 4 * FAST_T ? 1280 : few ? 1024 : 768);
 }
 
 static bool valid_kind(int k) { return k == SSM_PROJ_DN || k == SSM_PROJ_BDN || k == SSM_PROJ_BGNL; }
@@ -107,7 +108,8 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   p.ragged = const_ok ? !(p.vec_ok && a->seqlen % 8 == 0 && a->seqlen < (1 << 29)) : !whole_rows;
   const bool in_turn = tune >= 200000;      // a selector of 200000 + v: variant v, a row's chunks in turn however few the rows are
   if (in_turn) tune -= 100000;
-  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, per_b % 8 == 0 && per_c % 8 == 0, a->io_dtype != SSM_F32, p.ragged);
+  const bool half = a->io_dtype != SSM_F32, few = a->nstate <= 4;
+  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, per_b % 8 == 0 && per_c % 8 == 0, half, p.ragged, few);
   // Rows of at most 256 steps fill half a chunk there; the general kernel, which has chunks of 256, keeps them (6720 rows of
   // 256 bf16 20 us against 33) unless every channel has its own projections: 58 against 26 us, of 195 119 against 63.
   if (tune == 0 && fast_ok && (a->seqlen > 256 || (per_b == 1 && per_c == 1))) {
@@ -124,9 +126,13 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
       const int per_wg = scan_fwd_fast_rows(pref[i]);
       if (per_b % per_wg == 0 && per_c % per_wg == 0 && (total / per_wg >= 256 || i == 2)) pick = pref[i];
     }
-    // its rows by two waves each where that leaves a CU no more than one such workgroup and there are chunks to walk: 1920
-    // rows, us with one / two, 1024 steps 19.1 / 18.8, 2048 40.4 / 33.6, 8192 139 / 112, bf16 17.0 / 16.8, 32.1 / 29.3, 129 / 106
-    if (pick == 11082 && total <= 2048 && a->seqlen > 2 * FAST_T) pick = 11162;
+    // its rows by two waves each where that leaves a CU no more than one such workgroup, there are chunks to walk (1920 rows of
+    // 16 states, us with one / two, 1024 steps 19.1 / 18.8, 2048 40.4 / 33.6, 8192 139 / 112, bf16 17.0 / 16.8, 32.1 / 29.3,
+    // 129 / 106) and states enough that halving them is worth forming a row's steps twice: 2 x 640 x 1030 float32 with 1, 4, 8,
+    // 16 states 13.4 / 14.7, 16.1 / 17.3, 21.5 / 21.3, 32.1 / 29.5, bf16 (runs of any start) 12.2 / 14.9, 14.9 / 17.4, 20.0 /
+    // 21.4, 29.9 / 29.2; 4 states, aligned, 2 x 640 x 4096 31.8 / 32.8, 3 x 512 x 4096 34.8 / 33.6, 2 x 640 x 8192 68.9 / 63.5
+    const bool halves = p.ragged ? a->nstate > (half ? 8 : 4) : a->nstate > 4 || (a->nstate > 2 && total * a->seqlen >= (size_t)6 << 20);
+    if (pick == 11082 && total <= 2048 && a->seqlen > 2 * FAST_T && halves) pick = 11162;
     // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave, which reads its runs of
     // B and C as 16-byte vectors
     if (!pick) pick = 31041;
