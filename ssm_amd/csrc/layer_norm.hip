@@ -41,10 +41,10 @@ struct NormParams {
 // Calls up to these sizes leave what they read to the caches; larger ones read past them what is not read again (a backward
 // everything, a forward its residual: x is what a backward reads again): the space is better spent on what is written, for
 // those who read that.  Forward and backward (the forward keeps rstd), by elements, bf16 with a float32 residual and gradient
-// through it, us without / with: 2048 x 768 16.6 / 17.4, 2048 x 2560 36 / 40, 4 x 2048 x 768 43.2 / 42.1, 8 x 2048 x 768
-// 75.5 / 70.1, 16 x 2048 x 768 149 / 136 (the forward's x past the caches too 137; what is written past them: slower).  A
-// forward alone, by bytes, where they are more than the last-level cache holds: 75 MB 13.5 / 15.5, 252 MB 44.0 / 44.8, 302 MB
-// 49.1 / 48.2, float32 403 MB 71.8 / 63.1.
+// through it, us without / with (replayed as graphs): 2048 x 768 16.8 / 17.4, 2048 x 2560 38.1 / 38.7, 4 x 2048 x 768 42.7 /
+// 42.0, 8 x 2048 x 768 72.8 / 73.4 (72.0 / 69.4 one behind the other), 16 x 2048 x 768 149 / 145.5 (147 / 139); what is written
+// past them: slower.  A forward alone, by bytes, where they are more than the last-level cache holds: 75 MB 13.8 / 15.9, 252 MB
+// 44.0 / 44.8, 302 MB 54.6 / 53.7, float32 403 MB 71.8 / 63.1.
 constexpr size_t NORM_CACHED = (size_t)5632 << 10, NORM_CACHED_BYTES = (size_t)268 << 20;
 
 __device__ __forceinline__ void store_f32_as(void *p, int dtype, size_t i, float v) {

@@ -18,7 +18,7 @@ template <typename E> using V4 = __attribute__((__vector_size__(4 * sizeof(E))))
 __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // ---------------------------------------------------------------------- prep
-// One launch prepares everything the fused kernel reads besides x and z; the
+// One launch prepares everything that the walk, or the kernels of the chunks side by side, read besides x and z; the
 // workgroups (256 threads) take one of three roles by their index:
 //
 //  dt:   one workgroup per (b, c, 4 heads).  The (Q x 4) slab of dt is read row by
@@ -59,8 +59,9 @@ struct SsdPrepParams {
 // Packed sequences: the first step of a sequence gets an extra decay of 2^-64 (a jump in the running sum),
 // so that nothing of the sequences before it - state or in-chunk terms - reaches it or the steps after it:
 // exp2(cs_l - cs_s) then carries that factor whenever a boundary lies in (s, l].  The steps of one sequence
-// see the same jumps on both sides of the difference; with every step of a 256-step chunk a boundary the sum
-// reaches 2^14, where float32 still resolves 1e-3 of the exponent.
+// see the same jumps on both sides of the difference; with every step a boundary the sum reaches 2^14 in a chunk of 256,
+// where float32 still resolves 1e-3 of the exponent, and 2^11 in a block of the walk.  (Three boundaries in a block are more
+// than the decays of one that factors: heads of such calls go element by element.)
 constexpr float SEQ_JUMP_LN = -64.0f * 0.69314718056f;
 
 // dt' = clamp(softplus(dt + bias)), and what a step adds to the running sum of dt' A beyond its product: the jump into a
