@@ -274,7 +274,7 @@ __device__ __forceinline__ bool walk_rows(const SsdWalkParams &p, unsigned char 
       // The scalar offset stays the constant 0: a 16-byte store reads its data some cycles after it issues, and only for that
       // form does the compiler keep what rewrites those registers away from it.  With the offset in a scalar register wrong
       // words have been seen under load.
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? ~0u : mine + (unsigned)c * block, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, out), ry, drop ? 1u << 31 : mine + (unsigned)c * block, 0, 0);
     };
     // Ends of blocks are asked for a turn before they are looked at, and not looked at behind reads of LDS.
     float end[2] = {};
