@@ -489,8 +489,8 @@ typedef struct ssm_ssd_combined_args {
   const float *Dskip;         /* (H,P) if d_per_p else (H,), or NULL */
   const void *z;              /* (B,L,H,P) io dtype or NULL */
   const float *initial_states;/* (B,H,P,N) fp32 or NULL */
-  void *y;                    /* (B,L,H,P) io dtype */
-  float *final_states;        /* (B,H,P,N) fp32 or NULL */
+  void *y;                    /* (B,L,H,P) io dtype; may be x or z itself where no backward follows */
+  float *final_states;        /* (B,H,P,N) fp32 or NULL; may be initial_states itself */
   void *workspace;            /* ssm_ssd_combined_workspace_bytes() bytes, 256-byte aligned */
   size_t workspace_bytes;
   ssm_ssd_dims dims;

@@ -24,6 +24,7 @@
 // The factors r - cs_s reach 2^80: where dt x is so large that x~, or what it is summed into, leaves bfloat16, a y or a state
 // comes out infinite or not a number, and the workgroup does its heads again per element, whose factors are at most 1.
 // In float16 the same is done where a state goes beyond 65504: the second time it is rounded to float16 scaled by a power of two.
+// Calls that write y over x or z, which are not there a second time, go that way at once.
 //
 // A growing head (A > 0): decays between steps of one of the call's chunks are bounded by 1, the factors on the state entering
 // the chunk are not (the published kernels evaluate exp(min(x, 0)) and exp(x) there).  Such a head goes per element and keeps
@@ -623,11 +624,12 @@ void ssd_walk_kernel(const SsdWalkParams p) {
   extern __shared__ __align__(16) unsigned char lds[];
   const WalkHeads<NH> all(p, (int)xcd_order(blockIdx.x, p.sets));
   const float A0 = p.A[all.h0], A1 = p.A[all.h1];          // (asked for together with what heads_factor reads)
-  const bool factor = std::is_same<E, __bf16>::value && heads_factor(p, all);
+  constexpr bool F16 = std::is_same<E, _Float16>::value;
+  const bool factor = !F16 && !p.in_place && heads_factor(p, all);
   const bool grows0 = A0 > 0.0f, grows1 = A1 > 0.0f;
   const WalkHeads<NH> one(all.b, all.g, grows0 ? all.h1 : all.h0);
-  bool stands = true;
-  if (!grows0 || !grows1) stands = walk<E, NH, N, DMODE, HAS_Z, false>(p, lds, grows0 == grows1 ? all : one, factor);
+  bool stands = !(F16 && p.in_place);
+  if (stands && (!grows0 || !grows1)) stands = walk<E, NH, N, DMODE, HAS_Z, false>(p, lds, grows0 == grows1 ? all : one, factor);
   // those that grow, or left the range
   if (stands && !grows0 && !grows1) return;
   wait_memory<0>();                                        // what is written again is written after this
@@ -670,6 +672,7 @@ static int launch_walk(const SsdWalkParams &p, int dmode, hipStream_t s) {
 }
 
 int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s) {
+  p.in_place = p.y == p.x || p.y == p.z;
   const int per_group = p.heads / p.groups;
   // one head per workgroup while every workgroup has a CU of its own
   const int nh = p.batch * p.heads <= WALK_SINGLES ? 1 : 2;

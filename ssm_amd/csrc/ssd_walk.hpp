@@ -20,6 +20,7 @@ struct SsdWalkParams {                  // x, z, y and the fragment copies hold 
   int sets;                             // workgroups of one or two heads (set by ssd_walk_forward)
   int turns;                            // nblocks in whole turns through a ring of four
   int chunk_blocks;                     // blocks in a chunk of the call (what a growing head's factors go by)
+  bool in_place;                        // y over x or z (set by ssd_walk_forward)
 };
 
 int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s);
