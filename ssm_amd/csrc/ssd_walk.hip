@@ -674,8 +674,12 @@ static int launch_walk(const SsdWalkParams &p, int dmode, hipStream_t s) {
 int ssd_walk_forward(SsdWalkParams p, int dmode, bool f16, int nstate, hipStream_t s) {
   p.in_place = p.y == p.x || p.y == p.z;
   const int per_group = p.heads / p.groups;
-  // one head per workgroup while every workgroup has a CU of its own
-  const int nh = p.batch * p.heads <= WALK_SINGLES ? 1 : 2;
+  // One head per workgroup while every workgroup has a CU of its own, or where heads share nothing: a group of one head is no
+  // pair, and 320 or 384 such heads take, two by two (each twice) / one by one, 4 x 4096 steps, 128 states 795 / 753 us, 64
+  // states 535 / 510, 4 x 512 101 / 89, chunks of 64 and 64 states 73 / 58, float16 108 / 89 (the preparation of B and C per
+  // head with it).  Groups of three, whose third head is done twice: 324 heads x 4096 357 / 369, x 512 49 / 55, 516 x 2048
+  // 322 / 304, 768 x 2048 386 / 382.
+  const int nh = p.batch * p.heads <= WALK_SINGLES || per_group == 1 ? 1 : 2;
   p.sets = p.batch * p.groups * ((per_group + nh - 1) / nh);
 #define SSM_WALK_N(E, NN) return nh == 1 ? launch_walk<E, 1, NN>(p, dmode, s) : launch_walk<E, 2, NN>(p, dmode, s);
   if (f16) {
