@@ -15,13 +15,17 @@ namespace ssm {
 //   walk / side by side, chunks of 256: 107 / 38   106 / 53   105 / 85   109 / 110  110 / 130  117 / 150  138 / 241  197 / 341
 //   float16                             113 / 39   113 / 55   116 / 87   118 / 112  123 / 131  124 / 151  146 / 243  215 / 357
 // Up to two chunks the walk is always the faster one (24 heads, 512 steps: 20.8 / 23.7).
+// Side by side a group beyond the first has C.B of its own for whole chunks, the walk for blocks of 32 steps: `group` is what
+// that costs more for each block of each group, fitted at 420 sizes of 1 to 128 groups, 600 to 4096 steps, and looked at again
+// at 700 others: within 5 % of the faster route at all but seven, the worst 11 % off.  Without it 52 %: 4096 steps, 128 states,
+// chunks of 256, 100 groups of one head 256 / 401, 48 of one 162 / 170, 24 of one 136 / 92, 8 of ten 117 / 98.
 bool ssd_side_by_side(const SsdDims &d) {
   // the walk's offsets from the start of a head have 32 bits, some blocks past its end included
   if ((size_t)(d.len + 512) * d.heads * SSD_P * 2 >= (size_t)1 << 31) return true;
-  struct Chunks { double start, each, more, from; };         // `more` for each workgroup after the first `from`
-  static const Chunks chunks[3][2] = {{{16.0, 0.0135, 0.0060, 2300.0}, {20.0, 0.0175, 0.0116, 1600.0}},      // of 64 steps; 64, 128 states
-                                      {{16.0, 0.0195, 0.0075, 1280.0}, {18.0, 0.0255, 0.0120, 1280.0}},
-                                      {{20.5, 0.0295, 0.0145, 640.0}, {22.5, 0.0385, 0.0150, 640.0}}};
+  struct Chunks { double start, each, more, from, group; };  // `more` for each workgroup after the first `from`
+  static const Chunks chunks[3][2] = {{{16.0, 0.0135, 0.0060, 2300.0, 0.0003}, {20.0, 0.0175, 0.0116, 1600.0, 0.0018}},      // of 64 steps; 64, 128 states
+                                      {{16.0, 0.0195, 0.0075, 1280.0, 0.0020}, {18.0, 0.0255, 0.0120, 1280.0, 0.0060}},
+                                      {{20.5, 0.0295, 0.0145, 640.0, 0.0060}, {22.5, 0.0385, 0.0150, 640.0, 0.0098}}};
   const bool large = d.nstate > 64;
   const auto block_us = [&](int64_t n) {
     if (n == 0) return 0.0;
@@ -33,8 +37,8 @@ bool ssd_side_by_side(const SsdDims &d) {
   const double start = heads > 256 ? (large ? 12.7 : 10.0) : large ? 8.7 : 7.7;
   const double walk = start + ssd_walk_turns(ssd_walk_blocks(d.len)) * ((double)(heads / 512) * block_us(512) + block_us(heads % 512));
   const Chunks &c = chunks[d.chunk > 128 ? 2 : d.chunk > 64][large];
-  const double units = (double)heads * d.nchunks;
-  return d.nchunks > 2 && walk > c.start + c.each * units + c.more * std::max(0.0, units - c.from);
+  const double units = (double)heads * d.nchunks, group_blocks = (double)d.batch * (d.groups - 1) * ssd_walk_blocks(d.len);
+  return d.nchunks > 2 && walk > c.start + c.each * units + c.more * std::max(0.0, units - c.from) + c.group * group_blocks;
 }
 
 template <typename E, int Q, int N>

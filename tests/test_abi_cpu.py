@@ -208,6 +208,20 @@ def test_the_faster_route_of_the_combined_ssd_is_taken(chunk, nstate, heads, nch
     assert got >= states + one_pass / 2 if side_by_side else one_pass <= got <= one_pass + 8 * 256
 
 
+@pytest.mark.parametrize("batch,length,heads,groups,nstate,chunk,side_by_side", [
+    (1, 3000, 100, 100, 128, 256, False), (1, 3000, 64, 64, 128, 256, False), (2, 4096, 48, 48, 64, 256, False),
+    (1, 1500, 48, 48, 128, 256, False), (3, 1024, 24, 24, 128, 128, False), (1, 4096, 24, 24, 128, 256, True),
+    (1, 4096, 80, 8, 128, 256, True), (1, 4096, 96, 8, 128, 256, True), (2, 4096, 24, 4, 128, 64, True)])
+def test_the_faster_route_of_the_combined_ssd_with_groups_is_taken(batch, length, heads, groups, nstate, chunk, side_by_side):
+    """As the test above, with groups: each has fragments of B, C and C.B of its own, of whole chunks side by side."""
+    L = _lib()
+    d = L.SsdDims(batch=batch, seqlen=length, heads=heads, headdim=64, groups=groups, nstate=nstate, chunk=chunk)
+    steps, blocks = 128 * (-(-length // 128)), 32 * (-(-length // 32))
+    one_pass = batch * (steps * heads * (8 + 4 / 32) + blocks * groups * (2 * nstate + 32) * 2)
+    got = L.load().ssm_ssd_combined_workspace_bytes(ctypes.byref(d))
+    assert (got > one_pass + 8 * 256) if side_by_side else one_pass <= got <= one_pass + 8 * 256
+
+
 def test_shipped_library_has_no_test_hooks_and_the_hooks_build_does():
     """Kernel selectors and the record of kernels taken exist in the -DSSM_TEST_HOOKS build only
     (include/ssm_amd_testing.h): the shipped library rejects a non-zero ``reserved`` field and does not export
