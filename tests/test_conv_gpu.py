@@ -118,6 +118,28 @@ def test_no_bias_and_layout_detection_prefers_channels_first():
     check(run_pair(x, w, None, "silu"), FP32_TOL, dict(rtol=1e-4, atol=1e-4))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("length", [1, 3, 7, 9, 511, 517, 2047, 2050])
+def test_rows_of_any_length_keep_to_themselves(dtype, length):
+    """Rows whose runs cross their end: every second channel is NaN and must not reach its neighbours.  One rounding to the
+    type of float32 sums of 4 terms; the sums over 2 x length steps for the weights' gradients take rounding errors of
+    float32 terms of size about 1."""
+    g = torch.Generator().manual_seed(length)
+    x, go = (torch.randn(2, 5, length, generator=g).to(dtype) for _ in range(2))
+    x[:, 1::2], go[:, 1::2] = float("nan"), float("nan")
+    w, b = torch.rand(5, 4, generator=g) - 0.5, torch.randn(5, generator=g) * 0.02
+    xg, wg, bg = (t.cuda().requires_grad_() for t in (x, w, b))
+    y = _ops().dw_causal_conv(xg, wg, bg, activation="silu")
+    got = [t[:, ::2] for t in (y, *torch.autograd.grad(y, [xg], go.cuda(), retain_graph=True))]
+    got += [t[::2] for t in torch.autograd.grad(y, [wg, bg], go.cuda())]
+    xr, wr, br = (t.double().requires_grad_() for t in (x[:, ::2], w[::2], b[::2]))
+    yr = torch.nn.functional.silu(torch.nn.functional.conv1d(torch.nn.functional.pad(xr, (3, 0)), wr[:, None], br, groups=3))
+    want = [yr, *torch.autograd.grad(yr, [xr, wr, br], go[:, ::2].double())]
+    eps = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for a, r, tol in zip(got, want, (eps, eps, 1e-5, 1e-5)):
+        torch.testing.assert_close(a.double().cpu(), r, rtol=tol, atol=4e-6 * length ** 0.5)
+
+
 def test_config1_shape_bf16():
     """B=8, C=1536, L=2048, K=4, bf16, SiLU: forward + backward at full size against
     the oracle on a channel slice (channels are independent)."""
