@@ -226,6 +226,48 @@ __device__ __forceinline__ void store_steps(T *row, int t, int len, const Pack<T
   }
 }
 
+// N elements of a row of `len` (at least N) from step t on, in one access at the elements' own address; what would cross the
+// row's end is read as the row's last N and left to be put right (row_end).
+template <typename T, int N>
+__device__ __forceinline__ Pack<T, N> row_run(const T *row, int t, int len) {
+  struct __attribute__((packed)) Any { T v[N]; };
+  const Any a = *at_bytes<const Any>(row, (unsigned)min(t, len - N) * (unsigned)sizeof(T));
+  Pack<T, N> r;
+#pragma unroll
+  for (int i = 0; i < N; ++i) r.v[i] = a.v[i];
+  return r;
+}
+// What row_run left: the run that crosses the row's end moves down by the steps it was read too early (the same for every
+// row, since runs start at multiples of N), zeros are past the end.  All in registers: reading the crossing run again element
+// by element, or even asking whether there is one, made the wave wait for all it had under way.
+template <typename T, int N>
+__device__ __forceinline__ void row_end(int t, int len, Pack<T, N> &r) {
+  constexpr int W = N * (int)sizeof(T) / 4, PER = 4 / (int)sizeof(T);      // 32-bit words, elements in one
+  unsigned w[W];
+  __builtin_memcpy(w, &r, sizeof(w));
+  const int early = (N - len % N) % N;
+  const bool inside = t < len, crosses = inside && t + N > len;
+  if (PER == 2 && (early & 1)) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const unsigned moved = __builtin_amdgcn_alignbit(i + 1 < W ? w[i + 1 < W ? i + 1 : 0] : 0u, w[i], 16);
+      w[i] = crosses ? moved : w[i];
+    }
+  }
+#pragma unroll
+  for (int by = 1; by < W; by *= 2)
+    if (early / PER & by) {
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const unsigned moved = i + by < W ? w[i + by < W ? i + by : 0] : 0u;
+        w[i] = crosses ? moved : w[i];
+      }
+    }
+#pragma unroll
+  for (int i = 0; i < W; ++i) w[i] = inside ? w[i] : 0u;
+  __builtin_memcpy(&r, w, sizeof(w));
+}
+
 // 2^x on the transcendental unit (v_exp_f32, 1 ulp; results below 2^-126 flush to 0).
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float log2_hw(float x) { return __builtin_amdgcn_logf(x); }

@@ -15,25 +15,52 @@ extern template int scan_fwd_fast_dispatch<bf16_t, float>(const ScanFwdParams &,
 extern template int scan_fwd_fast_dispatch<f16_t, f16_t>(const ScanFwdParams &, int, hipStream_t);
 extern template int scan_fwd_fast_dispatch<f16_t, float>(const ScanFwdParams &, int, hipStream_t);
 
-// Rows up to which the chunks of a row run side by side in one workgroup (scan_fwd_split.hpp) rather than in turn; us at
-// 16 states in turn / side by side:
-//   grouped, float32, 512 x 2048 31.7 / 15.0, 768 x 8192 109 / 93, 1024 x 2048 30.7 / 25.7, 1024 x 4096 58 / 67,
-//   1280 x 2048 32 / 29.9, 1536 x 1024 18.1 / 16.7, 1536 x 2048 32.8 / 33.7;
-//   bf16 512 x 2048 32.2 / 13.8, 1280 x 1024 16.6 / 14.3, 1280 x 8192 104 / 93.5, 3 x 512 x 1024 21.2 / 19.6, x 2048 29.0 /
-//   27.7, x 4096 63.0 / 61.8, x 8192 118 / 117; with 4 states x 4096 31.5 / 27.0, x 8192 56 / 49.
-//   float32 of few states, whose rows two waves do not share (below): 1024 x 4096, 1 state 25.5 / 23.0.
-//   Every wave reads B and C itself there, and runs of odd rows at a lower rate: float32 512 x 2047 33 / 23, 768 x 2047
-//   33 / 42, bf16 768 x 2047 32 / 27, 768 x 1021 18.6 / 19.5, 768 x 3000 48 / 67.
+// Rows up to which the chunks of a row run side by side in one workgroup (scan_fwd_split.hpp) rather than in turn, us at
+// 16 states, side by side / in turn (grouped: scan_fwd_rows.hpp):
+//   grouped, runs aligned, bf16: 1024 x 504 8.8 / 11.0, 2048 x 504 11.0 / 12.2, 1280 x 1024 15.5 / 17.6, 1536 x 1024 18.5 / 17.5,
+//   1536 x 2048 27.6 / 29.6, 1280 x 4096 50.5 / 53.9, 1280 x 8192 95 / 102, 1536 x 8192 112 / 103; six chunks, whose waves share a
+//   CU badly, 768 x 3072 29.4 / 35.7, 1024 x 3072 47 / 37.
+//   float32: 1536 x 504 11.0 / 11.3, 2048 x 504 11.8 / 11.5, 1536 x 1024 16.2 / 17.1, 2048 x 1024 23.4 / 17.7, 1024 x 2048 25.3 / 25.3,
+//   512 x 4096 34.7 / 43.9, 768 x 4096 51 / 44, 512 x 8192 67 / 83, 768 x 8192 99 / 83.
+//   Every wave reads B and C itself there, and runs of odd rows at a lower rate: bf16 768 x 1021 14.2 / 16.1, 1280 x 1021 20.9 /
+//   18.3, 1024 x 2045 26.3 / 27.5, 768 x 8111 80 / 90, 1024 x 8111 99 / 91; float32 1024 x 1021 16.0 / 16.0, 768 x 2045 21.3 / 25.3,
+//   1024 x 2045 31.1 / 26.6, 512 x 8111 71 / 84, 768 x 8111 104 / 85.
 //   Few channels to a group (a row per wave in turn): 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
 //   Constant projections: 256 x 2048 18.4 / 10.2, 512 x 8192 68 / 43, 512 x 1024 10.6 / 10.9, 1024 x 4096 41 / 43.
-static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged, bool few) {
-  if (len <= FAST_T) return false;
-  if (!varying) return rows <= (len > 2 * FAST_T ? 512 : 384);
-  const bool to_four = len > 2 * FAST_T && len <= 4 * FAST_T;       // chunks
-  if (ragged) return rows <= (grouped && half && to_four ? 768 : 512);
-  if (!grouped) return rows <= (half ? 1536 : 1024);
-  if (half) return rows <= 1536;
-  return rows <= (len <= 2 * FAST_T ? 1536 : len <= 4 * FAST_T ? 1280 : few ? 1024 : 768);
+static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged) {
+  const int chunks = (len + FAST_T - 1) / FAST_T;
+  if (!varying) return chunks > 1 && rows <= (chunks > 2 ? 512 : 384);
+  if (!grouped) return chunks > 1 && rows <= (ragged ? 512 : half ? 1536 : 1024);
+  if (len <= FAST_T / 2 || (ragged && chunks == 1)) return false;      // ragged: 864 x 403 f16 13.4 / 11.1
+  if (ragged) return rows <= (chunks <= 2 ? 896 : half ? (chunks <= 4 ? 1024 : 768) : (chunks <= 4 ? 832 : 512));
+  if (chunks == 1) return rows <= (half ? 2048 : 1536);
+  if (!half) return rows <= (chunks <= 2 ? 1536 : chunks <= 4 ? 1280 : 576);
+  const int turns = (chunks + SPLIT_MAX_WAVES - 1) / SPLIT_MAX_WAVES, waves = (chunks + turns - 1) / turns;
+  return rows <= (chunks <= 2 ? 1440 : chunks <= 4 ? 1536 : waves > 4 && waves < 8 ? 896 : 1280);
+}
+
+// Channels to a workgroup of scan_fwd_rows.hpp: those of the cheapest number of rounds of 256 workgroups.  A chunk costs a
+// workgroup 6.2 us for every twelve rows, 4.0, 5.0 or 6.2 for the last four, eight or twelve, and 0.9 (4 chunks of bf16 with 4, 8,
+// 12, 16, 24, 36, 48 rows on every CU: 27, 31, 36, 53, 61, 86, 111 us); the start of a workgroup another 3.
+static int scan_fwd_rows_per_wg(int batch, int spans, int span, int chunks) {
+  const size_t units = (size_t)batch * spans;
+  const size_t least = (units * ((span + ROWS_MAX - 1) / ROWS_MAX) + 255) / 256;
+  const double part[4] = {0.0, 4.0, 5.0, 6.2};
+  double best = 0.0;
+  int pick = 0;
+  for (size_t k = least; k < least + 4; ++k) {
+    const size_t blocks = k * 256 / units;                   // workgroups that a span may have
+    const int rows = blocks <= 1 ? span : (int)((span + blocks - 1) / blocks);
+    if (rows > ROWS_MAX) continue;
+    const size_t rounds = (units * ((span + rows - 1) / rows) + 255) / 256;
+    const double cost = (double)rounds * (3.0 + chunks * (0.9 + 6.2 * (rows / 12) + part[(rows % 12 + 3) / 4]));
+    if (!pick || cost < best) {
+      best = cost;
+      pick = rows;
+    }
+    if (rows <= 4) break;
+  }
+  return pick ? pick : ROWS_MAX;
 }
 
 static bool valid_kind(int k) { return k == SSM_PROJ_DN || k == SSM_PROJ_BDN || k == SSM_PROJ_BGNL; }
@@ -99,45 +126,55 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   hipStream_t stream = reinterpret_cast<hipStream_t>(hip_stream);
 
   // The specialised kernels: time-varying B and C of one element type (that of the activations, or fp32), at most
-  // 16 states.  Rows that are not aligned whole 16-step runs take their RAGGED form.  A selector of 100000 + v asks for
-  // variant v.
-  const bool whole_rows = p.vec_ok && a->seqlen % 16 == 0 && a->seqlen < (1 << 29) && (!bvary || aligned_to(a->Bproj, 4 * bs)) &&
-                          (!cvary || aligned_to(a->Cproj, 4 * bs));
+  // 16 states.  A selector of 100000 + v asks for variant v.
+  const bool aligned = p.vec_ok && a->seqlen < (1 << 29) && (!bvary || aligned_to(a->Bproj, 4 * bs)) && (!cvary || aligned_to(a->Cproj, 4 * bs));
   const bool fast_ok = bvary && cvary && a->nstate <= FAST_N && (a->bc_dtype == a->io_dtype || a->bc_dtype == SSM_F32);
   const bool const_ok = !bvary && !cvary && a->nstate <= FAST_N;
-  p.ragged = const_ok ? !(p.vec_ok && a->seqlen % 8 == 0 && a->seqlen < (1 << 29)) : !whole_rows;
+  const bool whole8 = (const_ok ? p.vec_ok && a->seqlen < (1 << 29) : aligned) && a->seqlen % 8 == 0;    // runs of 8 steps
+  const bool whole16 = aligned && a->seqlen % 16 == 0;
+  p.ragged = !whole8;
   const bool in_turn = tune >= 200000;      // a selector of 200000 + v: variant v, a row's chunks in turn however few the rows are
   if (in_turn) tune -= 100000;
-  const bool half = a->io_dtype != SSM_F32, few = a->nstate <= 4;
-  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, per_b % 8 == 0 && per_c % 8 == 0, half, p.ragged, few);
-  // Rows of at most 256 steps fill half a chunk there; the general kernel, which has chunks of 256, keeps them (6720 rows of
-  // 256 bf16 20 us against 33) unless every channel has its own projections: 58 against 26 us, of 195 119 against 63.
-  if (tune == 0 && fast_ok && (a->seqlen > 256 || (per_b == 1 && per_c == 1))) {
-    // The variant whose workgroups (48, 24 or 8 channels of one group) still give every CU its share:
-    // two rows per wave with 16-step runs and two slabs where 256 such workgroups exist, else 8-step runs at six waves
-    // per SIMD, else the smallest workgroup.
-    const size_t total = (size_t)a->batch * a->dim;
-    // float32 activations: the 8-step runs at six waves per SIMD come out ahead (142.9 against 149.6 us at the
-    // headline shape, where twice the bytes per step leave more to wait for); 16-bit: the 16-step runs (120.5 / 133.3)
-    const int pref16[3] = {22123, 12121, 11082}, pref32[3] = {12121, 22123, 11082};
-    const int *pref = a->io_dtype == SSM_F32 ? pref32 : pref16;
-    int pick = p.split ? 31041 : 0;
-    for (int i = 0; i < 3 && !pick; ++i) {
-      const int per_wg = scan_fwd_fast_rows(pref[i]);
-      if (per_b % per_wg == 0 && per_c % per_wg == 0 && (total / per_wg >= 256 || i == 2)) pick = pref[i];
+  const bool half = a->io_dtype != SSM_F32;
+  p.span = per_b;
+  for (int r = per_c; r;) {                 // channels that share a group of B and one of C
+    const int q = p.span % r;
+    p.span = r;
+    r = q;
+  }
+  const int spans = a->dim / p.span, nchunks = (a->seqlen + FAST_T - 1) / FAST_T;
+  p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, p.span >= ROWS_MIN, half, p.ragged);
+  if (tune == 0 && fast_ok) {
+    int pick = 0;
+    // (rows of at most 256 steps and few states: the general kernel, 3 x 1024 x 64 bf16 with 5 states 7.2 us against 8.5)
+    if (p.span >= ROWS_MIN && a->seqlen >= 4 && a->seqlen < (1 << 28) && (a->seqlen > FAST_T / 2 || a->nstate > 8)) {
+      // Any number of channels to a workgroup, but where two rows to a wave at once come out even (aligned 16-bit rows, 48 channels
+      // to a workgroup on every CU in every round: 109.6 us against 111.0 at the headline shape), or where so few states leave
+      // little but the reads, for which more waves do better (aligned, 8 x 1536 x 2048, at most 8 states: bf16 42 to 75 us
+      // against 49 to 77, float32 with 24 channels 88 to 103 against 102 to 109).
+      pick = p.split ? 31041 : ROWS_VARIANT;
+      const int even = half ? 48 : 24;
+      const size_t wgs = rows_total / even;
+      if (!p.split && whole16 && a->seqlen > FAST_T / 2 && p.span % even == 0 && wgs >= 256 &&
+          (a->nstate <= 8 || (half && wgs % 256 == 0))) pick = half ? 22123 : 12121;
+      // workgroups of 8 channels, two to a CU: for so few states (5 x 320 x 2304 f16, one state, 13.8 us against 17.5; 1648 x 1408
+      // bf16, two, 9.7 / 12.4; 3 x 1072 x 640 float32, one, 9.6 / 12.4), and where a single chunk would take a second turn for its last rows, or has no more than 8 on a
+      // CU (aligned, one chunk: 2 x 1984 x 448 f16 16.3 / 19.0, 8 x 384 x 448 bf16, 12 on a CU, 15.4 / 13.9, 8 x 256 x 448 10.4 / 12.2)
+      else if (!p.split && whole16 && a->seqlen > FAST_T / 2 && p.span % 8 == 0 &&
+               ((a->nstate <= 2 && (half || nchunks <= 4)) || (nchunks == 1 && rows_total <= 4096 && (rows_total <= 2048 || rows_total > 3072)))) pick = 11082;
+    } else if (per_b % 8 == 0 && per_c % 8 == 0 && a->seqlen > 256) {
+      pick = p.split ? 31041 : 11082;
+    } else if (a->seqlen > 256 || (per_b == 1 && per_c == 1)) {
+      // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave, which reads its runs of
+      // B and C as 16-byte vectors.  (Rows of at most 256 steps fill half a chunk there: the general kernel, which has chunks of
+      // 256, keeps them unless every channel has its own projections: 58 against 26 us, of 195 steps 119 against 63.)
+      pick = 31041;
     }
-    // its rows by two waves each where that leaves a CU no more than one such workgroup, there are chunks to walk (1920 rows of
-    // 16 states, us with one / two, 1024 steps 19.1 / 18.8, 2048 40.4 / 33.6, 8192 139 / 112, bf16 17.0 / 16.8, 32.1 / 29.3,
-    // 129 / 106) and states enough that halving them is worth forming a row's steps twice: 2 x 640 x 1030 float32 with 1, 4, 8,
-    // 16 states 13.4 / 14.7, 16.1 / 17.3, 21.5 / 21.3, 32.1 / 29.5, bf16 (runs of any start) 12.2 / 14.9, 14.9 / 17.4, 20.0 /
-    // 21.4, 29.9 / 29.2; 4 states, aligned, 2 x 640 x 4096 31.8 / 32.8, 3 x 512 x 4096 34.8 / 33.6, 2 x 640 x 8192 68.9 / 63.5
-    const bool halves = p.ragged ? a->nstate > (half ? 8 : 4) : a->nstate > 4 || (a->nstate > 2 && total * a->seqlen >= (size_t)6 << 20);
-    if (pick == 11082 && total <= 2048 && a->seqlen > 2 * FAST_T && halves) pick = 11162;
-    // groups of fewer than 8 channels (down to one per channel): nothing to share, a row per wave, which reads its runs of
-    // B and C as 16-byte vectors
-    if (!pick) pick = 31041;
-    if (pick == 31041 && !(aligned_to(a->Bproj, 16) && aligned_to(a->Cproj, 16) && ((size_t)a->seqlen * bs) % 16 == 0)) p.ragged = 1;
-    tune = 100000 + pick;
+    if (nchunks == 1) p.split = 0;          // nothing is beside a row's one chunk: 2 x 777 x 320 f16 10.0 us without what they exchange, 11.2 with
+    if (pick == 31041) p.ragged = !(whole8 && aligned_to(a->Bproj, 16) && aligned_to(a->Cproj, 16));
+    else if (pick != ROWS_VARIANT) p.ragged = !whole16;
+    p.rows_per_wg = pick == ROWS_VARIANT ? scan_fwd_rows_per_wg(a->batch, spans, p.span, nchunks) : 0;
+    if (pick) tune = 100000 + pick;
   }
   // Projections constant in time, (D, N) or (B, D, N): a row per wave with B and C in lanes (variant 31042).
   if ((tune == 0 && const_ok && a->seqlen > 256) || tune == 100000 + 31042) {
@@ -154,8 +191,10 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
     const int v = tune - 100000, per_wg = scan_fwd_fast_rows(v);
     SSM_REQUIRE(per_wg > 0 && per_b % per_wg == 0 && per_c % per_wg == 0, SSM_ERR_BAD_KIND,
                 "ssm_scan_fwd: variant %d takes %d channels per workgroup, which must divide a group", v, per_wg);
-    SSM_REQUIRE(!p.ragged || !SSM_RESERVED(a) || per_wg == 1, SSM_ERR_BAD_KIND,
-                "ssm_scan_fwd: selector %d is for aligned rows of whole 16-step runs", tune);
+    if (SSM_RESERVED(a)) {
+      SSM_REQUIRE(per_wg == 1 || whole16, SSM_ERR_BAD_KIND, "ssm_scan_fwd: selector %d is for aligned rows of whole 16-step runs", tune);
+      p.rows_per_wg = per_wg;
+    }
     const bool bc32 = a->bc_dtype == SSM_F32;
     switch (a->io_dtype) {
       case SSM_F32: return scan_fwd_fast_dispatch<float, float>(p, v, stream);

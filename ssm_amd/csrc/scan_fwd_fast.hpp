@@ -107,23 +107,15 @@ __device__ __forceinline__ float group_read_lane(float v, int src, int lane) {
 // DB: two slabs in LDS (for variants of which one workgroup fills a CU): the slab of the next chunk is staged by
 // each wave as soon as it is done with its rows of this one, while slower waves still work, and a chunk costs
 // one barrier instead of two.
-// NS = 2: two waves to a row, each with half of its states; the second hands its sums for y to the first through LDS.  For
-// calls of so few rows that their waves come to two a SIMD: those are bound by latency, and an instruction takes a SIMD 4
-// cycles with two waves to pick from, 2.5 with four.  With no more than those to hide it, a chunk's rows are requested while
-// the chunk before is worked on (16-bit runs of any start cost more registers than that is worth): 1920 rows of 8192
-// steps float32 139 us with a wave to a row, 122 with two, 112 with this; bfloat16, two slabs, 129, 111, 106.
-template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED, int NS = 1>
+template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED>
 __global__ __launch_bounds__(WAVE *WAVES) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void scan_fwd_fast_kernel(const ScanFwdParams p) {
   constexpr int T = FAST_T, K = T / LPR, SUBS = WAVE / LPR;
   extern __shared__ __align__(16) float tiles[];           // B [16][T] then C [16][T] (twice with DB)
   float *Bs = tiles, *Cs = tiles + FAST_N * T;
 
-  static_assert(NS == 1 || (RPW == 1 && LPR == WAVE));
-  constexpr bool AHEAD = NS == 2 && (sizeof(io_t) == 4 || !RAGGED);
-  constexpr int rows = WAVES / NS * RPW * SUBS;
+  constexpr int rows = WAVES * RPW * SUBS;
   const int wave = wave_id_uniform();
-  const int part = NS == 1 ? 0 : wave / (WAVES / NS), row_wave = NS == 1 ? wave : wave % (WAVES / NS);
   const int lane = lane_id();
   const int sl = lane & (LPR - 1);            // lane within the row
   const int sub = lane / LPR;                 // which of the wave's rows
@@ -131,7 +123,6 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   const int b = (int)blockIdx.x / blocks_per_batch;
   const int d0 = ((int)blockIdx.x % blocks_per_batch) * rows;
   const int L = p.len, N = p.nstate;
-  const int n_first = part ? min(N, (N + 3) / 4 * 2) : 0, n_end = NS == 2 && !part ? min(N, (N + 3) / 4 * 2) : N;      // this wave's states
   const size_t bg = (size_t)b * p.b_groups + d0 / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d0 / (p.dim / p.c_groups);
   const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + bg * N * L;
   const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + cg * N * L;
@@ -144,7 +135,7 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   float A2_lanes[RPW], carry_lanes[RPW], Dk[RPW], bias[RPW];
 #pragma unroll
   for (int rr = 0; rr < RPW; ++rr) {
-    const int d = d0 + (row_wave * RPW + rr) * SUBS + sub;
+    const int d = d0 + (wave * RPW + rr) * SUBS + sub;
     A2_lanes[rr] = sl < N ? p.A[(size_t)d * N + sl] * LOG2E : 0.0f;
     carry_lanes[rr] = 0.0f;
     Dk[rr] = p.Dk ? p.Dk[d] : 0.0f;
@@ -152,13 +143,6 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   }
 
   const int nchunks = (L + T - 1) / T;
-  Pack<io_t, K> ur, dr;
-  const auto request_rows = [&](size_t row, int c) {
-    const size_t room = ((size_t)p.batch * p.dim - row) * L;
-    ur = load_steps<RAGGED, io_t, K>(U + row * L, c * T + sl * K, L, c * T + T > L, room);
-    dr = load_steps<RAGGED, io_t, K>(DT + row * L, c * T + sl * K, L, c * T + T > L, room);
-  };
-  if constexpr (AHEAD) request_rows((size_t)b * p.dim + d0 + row_wave, 0);
   for (int c = 0; c < nchunks; ++c) {
     const int t0 = c * T;
     const int t = t0 + sl * K;
@@ -180,14 +164,16 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
 
 #pragma unroll
     for (int rr = 0; rr < RPW; ++rr) {
-      const int d = d0 + (row_wave * RPW + rr) * SUBS + sub;
+      const int d = d0 + (wave * RPW + rr) * SUBS + sub;
       const size_t row = (size_t)b * p.dim + d;
       float dl[K], du[K], y[K];
       Pack<io_t, K> zr;
       {
-        if constexpr (!AHEAD) request_rows(row, c);
-        if (p.z && !part) zr = load_steps<RAGGED, io_t, K>(Z + row * L, t, L, t0 + T > L, ((size_t)p.batch * p.dim - row) * L);
-        if (p.chunk_states && sl >= n_first && sl < n_end) p.chunk_states[(row * nchunks + c) * (size_t)N + sl] = carry_lanes[rr];
+        const size_t room = ((size_t)p.batch * p.dim - row) * L;
+        const Pack<io_t, K> ur = load_steps<RAGGED, io_t, K>(U + row * L, t, L, t0 + T > L, room);
+        const Pack<io_t, K> dr = load_steps<RAGGED, io_t, K>(DT + row * L, t, L, t0 + T > L, room);
+        if (p.z) zr = load_steps<RAGGED, io_t, K>(Z + row * L, t, L, t0 + T > L, room);
+        if (p.chunk_states && sl < N) p.chunk_states[(row * nchunks + c) * (size_t)N + sl] = carry_lanes[rr];
 #pragma unroll
         for (int i = 0; i < K; ++i) dl[i] = to_f32(dr.v[i]) + bias[rr];
         if (p.softplus) {
@@ -202,15 +188,12 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
         for (int i = 0; i < K; ++i) {
           const float uu = to_f32(ur.v[i]);
           du[i] = dl[i] * uu;
-          y[i] = part ? 0.0f : Dk[rr] * uu;
+          y[i] = Dk[rr] * uu;
         }
       }
       float dsum = 0.0f;
 #pragma unroll
       for (int i = 0; i < K; ++i) dsum += dl[i];
-      if constexpr (AHEAD) {
-        if (c + 1 < nchunks) request_rows(row, c + 1);
-      }
 
       auto process = [&](auto width_tag, int n0) {
         constexpr int WW = decltype(width_tag)::value;
@@ -297,31 +280,17 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
           else __builtin_amdgcn_s_setprio(3);
         }
       };
-      int n0 = n_first;
+      int n0 = 0;
       if constexpr (W == 2)
-        for (; n0 + 2 <= n_end; n0 += 2) {
+        for (; n0 + 2 <= N; n0 += 2) {
           turn(n0 >> 1);
           process(std::integral_constant<int, 2>{}, n0);
         }
-      for (; n0 < n_end; ++n0) {
+      for (; n0 < N; ++n0) {
         turn(n0);
         process(std::integral_constant<int, 1>{}, n0);
       }
 
-      if constexpr (NS == 2) {
-        float *sums = tiles + (DB ? 4 : 2) * FAST_N * T + row_wave * T + lane * 4;
-        if (part) {
-#pragma unroll
-          for (int q = 0; q < K / 4; ++q) *reinterpret_cast<float4 *>(sums + q * (LPR * 4)) = make_float4(y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
-        }
-        __syncthreads();
-        if (part) continue;
-#pragma unroll
-        for (int q = 0; q < K / 4; ++q) {
-          const float4 v = *reinterpret_cast<const float4 *>(sums + q * (LPR * 4));
-          y[4 * q] += v.x; y[4 * q + 1] += v.y; y[4 * q + 2] += v.z; y[4 * q + 3] += v.w;
-        }
-      }
       if (p.z) {
 #pragma unroll
         for (int i = 0; i < K; ++i) {
@@ -346,8 +315,8 @@ void scan_fwd_fast_kernel(const ScanFwdParams p) {
   if (p.last) {
 #pragma unroll
     for (int rr = 0; rr < RPW; ++rr) {
-      const size_t row = (size_t)b * p.dim + d0 + (row_wave * RPW + rr) * SUBS + sub;
-      if (sl >= n_first && sl < n_end) reinterpret_cast<io_t *>(p.last)[row * N + sl] = from_f32<io_t>(carry_lanes[rr]);
+      const size_t row = (size_t)b * p.dim + d0 + (wave * RPW + rr) * SUBS + sub;
+      if (sl < N) reinterpret_cast<io_t *>(p.last)[row * N + sl] = from_f32<io_t>(carry_lanes[rr]);
     }
   }
 }
@@ -520,25 +489,19 @@ static int launch_scan_fwd_rowbc(const ScanFwdParams &p, hipStream_t stream) {
   return SSM_OK;
 }
 
-template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED, int NS = 1>
+template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB, bool RAGGED>
 static int launch_scan_fwd_fast_as(const ScanFwdParams &p, hipStream_t stream) {
-  const size_t lds = ((size_t)(DB ? 4 : 2) * FAST_N + (NS == 2 ? WAVES / 2 : 0)) * FAST_T * sizeof(float);
-  auto kernel = scan_fwd_fast_kernel<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, RAGGED, NS>;
+  const size_t lds = (size_t)(DB ? 4 : 2) * FAST_N * FAST_T * sizeof(float);
+  auto kernel = scan_fwd_fast_kernel<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, RAGGED>;
   if (allow_dynamic_lds(kernel, lds) != hipSuccess) {
     (void)hipGetLastError();
     set_error("ssm_scan_fwd: cannot reserve %zu bytes of LDS", lds);
     return SSM_ERR_LAUNCH;
   }
-  const unsigned grid = (unsigned)((size_t)p.batch * (p.dim / (WAVES / NS * RPW * (WAVE / LPR))));
+  const unsigned grid = (unsigned)((size_t)p.batch * (p.dim / (WAVES * RPW * (WAVE / LPR))));
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(WAVE * WAVES), lds, stream, p);
   SSM_CHECK_LAUNCH("ssm_scan_fwd");
   return SSM_OK;
-}
-
-template <typename io_t, typename bc_t, int LPR, int RPW, int WAVES, int W, int OCC, bool DB = false, int NS = 1>
-static int launch_scan_fwd_fast(const ScanFwdParams &p, hipStream_t stream) {
-  return p.ragged ? launch_scan_fwd_fast_as<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, true, NS>(p, stream)
-                  : launch_scan_fwd_fast_as<io_t, bc_t, LPR, RPW, WAVES, W, OCC, DB, false, NS>(p, stream);
 }
 
 template <typename io_t>
@@ -562,19 +525,24 @@ static int launch_scan_fwd_row_const(const ScanFwdParams &p, hipStream_t stream)
 }  // namespace ssm
 
 #include "scan_fwd_split.hpp"
+#include "scan_fwd_rows.hpp"
 
 namespace ssm {
 
-// Channels per workgroup of a variant; 0 for an unknown one.
+// Channels per workgroup of a variant (1: any number); 0 for an unknown one.
 // variant = 10000 * (rows a wave walks at once) + 1000 * (rows a wave walks in turn) + 10 * waves + states in flight
 inline int scan_fwd_fast_rows(int variant) {
   switch (variant) {
-    case 13082: case 12121: return 24;
-    case 11082: case 11162: return 8;       // 11162: two waves to a row, half of its states each
-    case 22121: case 22123: return 48;
-    case 21081: return 16;
+    case 12121: return 24;
+    case 11082: return 8;
+    case 22123: return 48;
     case 31041: return 1;       // a row per wave, projections read straight from memory
     case 31042: return 1;       // a row per wave, projections constant in time
+    case ROWS_VARIANT: return 1;
+    case 13082: return 24;      // by selector: ROWS_VARIANT with so many channels to a workgroup
+    case 11162: return 8;
+    case 22121: return 48;
+    case 21081: return 16;
     default: return 0;
   }
 }
@@ -582,18 +550,13 @@ inline int scan_fwd_fast_rows(int variant) {
 template <typename io_t, typename bc_t>
 int scan_fwd_fast_dispatch(const ScanFwdParams &p, int variant, hipStream_t s) {
   switch (variant) {
-    case 13082: return launch_scan_fwd_fast_as<io_t, bc_t, 64, 3, 8, 2, 4, false, false>(p, s);     // 4 waves per SIMD
-    case 12121: return launch_scan_fwd_fast<io_t, bc_t, 64, 2, 12, 1, 6>(p, s);    // 6 waves per SIMD
-    case 11082: return launch_scan_fwd_fast<io_t, bc_t, 64, 1, 8, 2, 4>(p, s);
-    case 11162:
-      if constexpr (sizeof(io_t) == 4) return launch_scan_fwd_fast<io_t, bc_t, 64, 1, 16, 2, 4, false, 2>(p, s);
-      else return p.ragged ? launch_scan_fwd_fast_as<io_t, bc_t, 64, 1, 16, 2, 4, false, true, 2>(p, s)
-                           : launch_scan_fwd_fast_as<io_t, bc_t, 64, 1, 16, 2, 4, true, false, 2>(p, s);
-    case 22121: return launch_scan_fwd_fast_as<io_t, bc_t, 32, 2, 12, 1, 3, false, false>(p, s);    // 3 waves per SIMD, 16-step runs
-    case 22123: return launch_scan_fwd_fast<io_t, bc_t, 32, 2, 12, 1, 3, true>(p, s);   // the same with two slabs
-    case 21081: return launch_scan_fwd_fast_as<io_t, bc_t, 32, 1, 8, 1, 4, false, false>(p, s);
+    case 12121: return launch_scan_fwd_fast_as<io_t, bc_t, 64, 2, 12, 1, 6, false, false>(p, s);    // 6 waves per SIMD
+    case 11082: return p.ragged ? launch_scan_fwd_fast_as<io_t, bc_t, 64, 1, 8, 2, 4, false, true>(p, s)
+                                : launch_scan_fwd_fast_as<io_t, bc_t, 64, 1, 8, 2, 4, false, false>(p, s);
+    case 22123: return launch_scan_fwd_fast_as<io_t, bc_t, 32, 2, 12, 1, 3, true, false>(p, s);     // 3 waves per SIMD, 16-step runs, two slabs
     case 31041: return p.split ? launch_scan_fwd_split<io_t, bc_t, false>(p, s) : launch_scan_fwd_rowbc<io_t, bc_t>(p, s);
     case 31042: return p.split ? launch_scan_fwd_split<io_t, float, true>(p, s) : launch_scan_fwd_row_const<io_t>(p, s);
+    case ROWS_VARIANT: case 13082: case 11162: case 22121: case 21081: return launch_scan_fwd_rows<io_t, bc_t>(p, s);
     default:
       set_error("ssm_scan_fwd: unknown variant %d of the specialised kernel", variant);
       return SSM_ERR_BAD_KIND;

@@ -40,6 +40,7 @@ struct ScanFwdParams {
   int bc_vec_ok;  // rows of B/C allow 4-element vector loads
   int ragged;     // specialised kernels: rows are not whole aligned runs
   int split;      // row-per-wave kernels: the chunks of a row side by side (scan_fwd_split.hpp)
+  int span, rows_per_wg;    // scan_fwd_rows.hpp: channels that share a group of B and one of C, those of them to a workgroup
 };
 
 // `v` through the chunk maps (scan_bwd_maps.hpp) of `count` chunks, the first at `m`, `step` elements apart; eight are

@@ -18,6 +18,13 @@ namespace ssm {
 
 constexpr int SPLIT_MAX_WAVES = 8;
 
+// A lane's run: aligned whole runs by load_steps, runs of any start by row_run (and row_end where a row ends).
+template <bool RAGGED, typename T, int K>
+__device__ __forceinline__ Pack<T, K> lane_run(const T *row, int t, int len) {
+  if constexpr (RAGGED) return row_run<T, K>(row, t, len);
+  else return load_steps<false, T, K>(row, t, len, false, 0);
+}
+
 template <typename io_t, typename bc_t, bool CONST_BC, bool RAGGED>
 __global__ __launch_bounds__(WAVE *SPLIT_MAX_WAVES)
 void scan_fwd_split_kernel(const ScanFwdParams p) {
@@ -31,8 +38,6 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
   const int b = (int)(row / p.dim), d = (int)(row % p.dim);
   const int L = p.len, N = p.nstate;
   const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp), *Cg = reinterpret_cast<const bc_t *>(p.Cp);
-  size_t Broom = 0, Croom = 0;                              // elements to the ends of the tensors
-  const size_t room = ((size_t)p.batch * p.dim - row) * L;
   float B_lanes = 0.0f, C_lanes = 0.0f;
   if constexpr (CONST_BC) {
     if (lane < N) {
@@ -43,8 +48,6 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
     const size_t bg = (size_t)b * p.b_groups + d / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d / (p.dim / p.c_groups);
     Bg += bg * N * L;
     Cg += cg * N * L;
-    Broom = ((size_t)p.batch * p.b_groups - bg) * N * L;
-    Croom = ((size_t)p.batch * p.c_groups - cg) * N * L;
   }
   const io_t *U = reinterpret_cast<const io_t *>(p.u) + row * L, *DT = reinterpret_cast<const io_t *>(p.delta) + row * L;
   const io_t *Z = reinterpret_cast<const io_t *>(p.z) + row * L;
@@ -63,15 +66,17 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
         const size_t at = (size_t)min(n + w, N - 1) * L;
-        braw[w] = load_steps<RAGGED, bc_t, K>(Bg + at, t, L, tail, Broom - at);
-        craw[w] = load_steps<RAGGED, bc_t, K>(Cg + at, t, L, tail, Croom - at);
+        braw[w] = lane_run<RAGGED, bc_t, K>(Bg + at, t, L);
+        craw[w] = lane_run<RAGGED, bc_t, K>(Cg + at, t, L);
       }
     };
     if constexpr (!CONST_BC) fetch(0);
-    const Pack<io_t, K> ur = load_steps<RAGGED, io_t, K>(U, t, L, tail, room);
-    const Pack<io_t, K> dr = load_steps<RAGGED, io_t, K>(DT, t, L, tail, room);
-    Pack<io_t, K> zr;
-    if (p.z) zr = load_steps<RAGGED, io_t, K>(Z, t, L, tail, room);
+    Pack<io_t, K> ur = lane_run<RAGGED, io_t, K>(U, t, L), dr = lane_run<RAGGED, io_t, K>(DT, t, L), zr;
+    if (p.z) zr = lane_run<RAGGED, io_t, K>(Z, t, L);
+    if (RAGGED && tail) {
+      row_end(t, L, ur);
+      row_end(t, L, dr);
+    }
     float dl[K], du[K], y[K], dsum = 0.0f;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
@@ -98,6 +103,10 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
 #pragma unroll
           for (int i = 0; i < K; ++i) { bq[i] = bn; cq[w][i] = cn; }
         } else {
+          if (RAGGED && tail) {
+            row_end(t, L, braw[w]);
+            row_end(t, L, craw[w]);
+          }
 #pragma unroll
           for (int i = 0; i < K; ++i) { bq[i] = to_f32(braw[w].v[i]); cq[w][i] = to_f32(craw[w].v[i]); }
         }
@@ -139,6 +148,7 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
 
     if (p.chunk_states && c < nchunks && lane < N) p.chunk_states[(row * nchunks + c) * (size_t)N + lane] = Hin_lanes;
     if (p.z) {
+      if (RAGGED && tail) row_end(t, L, zr);
 #pragma unroll
       for (int i = 0; i < K; ++i) {
         const float zz = to_f32(zr.v[i]);

@@ -111,3 +111,38 @@ def test_what_lies_past_a_row_never_enters_it(dtype):
                                           (256, torch.float16)])
 def test_short_rows_with_projections_per_channel(length, dtype):
     test_rows_of_any_length("own", length, 16, dtype, True)
+
+
+@pytest.mark.parametrize("batch,dim,length,nstate,dtype,bc_dtype,groups", [
+    (3, 688, 1031, 16, torch.float32, torch.float32, (1, 1)),      # 2064 rows: nine to a workgroup, the last of a batch has fewer
+    (8, 400, 1544, 15, torch.bfloat16, torch.bfloat16, (1, 1)),    # thirteen: a second turn of one row; odd number of states
+    (4, 1616, 521, 16, torch.float16, torch.float16, (1, 1)),      # 26: three turns, a last chunk of nine steps
+    (6, 576, 1027, 9, torch.bfloat16, torch.float32, (4, 6)),      # runs of 48 channels share B and C
+    (9, 2720, 264, 16, torch.float32, torch.float32, (2, 1)),      # 24480 rows: one round of 96
+    (5, 304, 256, 16, torch.bfloat16, torch.bfloat16, (1, 1)), (5, 304, 251, 11, torch.float32, torch.float32, (1, 4)),
+    (2, 24, 4, 16, torch.float16, torch.float16, (1, 1)), (2, 12, 7, 16, torch.bfloat16, torch.float32, (1, 1))])
+def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype, bc_dtype, groups):
+    """The channels at a batch row's and a group's edges against float64, and the state after each chunk through the
+    gradients' entry; what lies in other rows (infinities beyond the compared ones) stays there."""
+    from ssm_amd import ops
+    inp = make_inputs(length, batch, dim, length, nstate, dtype=dtype, bc_dtype=bc_dtype, groups=1)
+    g = torch.Generator().manual_seed(1)
+    inp["B"], inp["C"] = (torch.randn(batch, n, nstate, length, generator=g).to(bc_dtype) for n in groups)
+    pick = sorted({0, 1, 11, 12 % dim, dim // 2, dim - 2, dim - 1})
+    for k in ("u", "delta"):
+        inp[k][:, [d for d in range(dim) if d not in pick and d % 5 == 0], -1] = float("inf")
+    t = {k: v.cuda() for k, v in inp.items()}
+    y, h = ops.selective_scan(*(t[k] for k in NAMES[:5]), D=t["D"], z=t["z"], dt_bias=t["dt_bias"], softplus=True,
+                              return_last_state=True)
+    part = {k: v[:, pick] for k, v in inp.items() if k in ("u", "delta", "z")}
+    part.update({k: inp[k][pick] for k in ("A", "D", "dt_bias")})
+    for k, n in zip("BC", groups):
+        part[k] = inp[k][:, [d // (dim // n) for d in pick]]
+    yr, hr = O.selective_scan(*(part[k].double() for k in NAMES[:5]), D=part["D"].double(), z=part["z"].double(),
+                              dt_bias=part["dt_bias"].double(), softplus=True, return_last_state=True, acc=torch.float64)
+    half = dtype != torch.float32
+    # one rounding of the float32 result to 16 bits (or of sums over the states to float32)
+    tol = dict(rtol=2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -10, atol=1e-4) if half else dict(rtol=1e-5, atol=1e-5)
+    for a, b, what in ((y[:, pick], yr, "y"), (h[:, pick], hr, "last state")):
+        scale = float(b.abs().max())
+        torch.testing.assert_close(a.double().cpu(), b, rtol=tol["rtol"], atol=tol["atol"] * scale, msg=lambda m: f"{what}: {m}")
