@@ -64,7 +64,7 @@ void launch_fold_rows(const float *in, float *out, int count, size_t inner, hipS
 void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_t inner, hipStream_t s);
 
 // All sums that a backward call ends with, in one launch of workgroup ranges per job (scan_bwd.hip):
-//   out[o][i] = sum_{j < count} in[(o * count + j) * inner + i], added in order of j, written as `dtype`.
+//   out[o][i] = sum_{j < count} in[(o * count + j) * inner + i], added in a fixed order, written as `dtype`.
 // As launches of their own, with the casts behind them, they took 5 to 10 us each, of which the gaps were half.
 constexpr int FOLD_JOBS = 5;
 struct FoldJobs {
@@ -72,6 +72,7 @@ struct FoldJobs {
   void *out[FOLD_JOBS];
   size_t outer[FOLD_JOBS], inner[FOLD_JOBS];
   int count[FOLD_JOBS], dtype[FOLD_JOBS], width[FOLD_JOBS];     // width: outputs per thread, 1 or 4
+  int sliced[FOLD_JOBS];                                        // few outputs of many terms: the terms in sixteen slices
   unsigned first_block[FOLD_JOBS + 1];
   int n;
   void add(const float *in, void *out, size_t outer, int count, size_t inner, int dtype);
@@ -365,14 +366,18 @@ __device__ __forceinline__ float wave_read_lane(float v, int lane) {
 
 // Sum over the 64 lanes, result valid in every lane (uniform).  Six DPP additions (a running
 // sum inside each row of 16, then the row totals passed on: lane 63 ends with everything) and
-// one read of lane 63: no trip through the LDS crossbar as with shuffles.
+// one read of lane 63: no trip through the LDS crossbar as with shuffles.  Written out: lanes whose source does not exist,
+// or whose row is masked off, keep their value, where the compiler moves a zero in first (ten instructions).
 __device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, v);
-  v += dpp_move<DPP_ROW_SHR2, 0xf>(0.0f, v);
-  v += dpp_move<DPP_ROW_SHR4, 0xf>(0.0f, v);
-  v += dpp_move<DPP_ROW_SHR8, 0xf>(0.0f, v);
-  v += dpp_move<DPP_ROW_BCAST15, 0xa>(0.0f, v);
-  v += dpp_move<DPP_ROW_BCAST31, 0xc>(0.0f, v);
+  asm volatile(
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+v"(v));
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
 }
 

@@ -46,7 +46,8 @@ struct ScanBwdParams {
   int b_kind, c_kind, b_groups, c_groups;
   int softplus;
   int rows_per_wg;       // channels walked by one workgroup (all in one B group and one C group)
-  int nblk;              // workgroups per batch row = dim / rows_per_wg
+  int span;              // channels that share a B group and a C group
+  int nblk;              // workgroups per batch row
   int bc_vec_ok;
   int ragged;            // specialised kernels: rows are not whole aligned runs
   const float2 *maps;    // specialised kernels: (B, D, ceil(L / 512), N) maps of the chunks (scan_bwd_maps.hpp), which then are
@@ -643,51 +644,89 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(const float *in, float *
 // The sums of FoldJobs: dA, dD, the bias and projections constant in time over the batch (and over chunks that ran side
 // by side); dB and dC of grouped projections over the workgroups of a group, straight into the projections' own type
 // when asked.
+// W neighbouring results as the output's type.
+template <int W>
+__device__ __forceinline__ void fold_write(void *out, size_t at, int dtype, const Pack<float, W> &s) {
+  if (dtype == SSM_F32) {
+    *reinterpret_cast<Pack<float, W> *>(reinterpret_cast<float *>(out) + at) = s;
+  } else if (dtype == SSM_BF16) {
+    Pack<bf16_t, W> r;
+#pragma unroll
+    for (int w = 0; w < W; ++w) r.v[w] = from_f32<bf16_t>(s.v[w]);
+    *reinterpret_cast<Pack<bf16_t, W> *>(reinterpret_cast<bf16_t *>(out) + at) = r;
+  } else {
+    Pack<f16_t, W> r;
+#pragma unroll
+    for (int w = 0; w < W; ++w) r.v[w] = from_f32<f16_t>(s.v[w]);
+    *reinterpret_cast<Pack<f16_t, W> *>(reinterpret_cast<f16_t *>(out) + at) = r;
+  }
+}
+
+// Terms first, first + step, ... of `count`, `inner` apart; eight terms' reads in flight together.
+template <int W>
+__device__ __forceinline__ Pack<float, W> fold_terms(const float *src, int first, int count, int step, size_t inner) {
+  Pack<float, W> s;
+#pragma unroll
+  for (int w = 0; w < W; ++w) s.v[w] = 0.0f;
+  int j = first;
+  for (; j + 7 * step < count; j += 8 * step) {
+    Pack<float, W> v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)(j + k * step) * inner);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int w = 0; w < W; ++w) s.v[w] += v[k].v[w];
+  }
+  for (; j < count; j += step) {
+    const Pack<float, W> v = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)j * inner);
+#pragma unroll
+    for (int w = 0; w < W; ++w) s.v[w] += v.v[w];
+  }
+  return s;
+}
+
 template <int W>
 __device__ __forceinline__ void fold_job(const float *in, void *out, size_t outer, size_t inner, int count, int dtype,
                                          size_t first, size_t stride) {
   const size_t per = inner / W;
   for (size_t e = first; e < outer * per; e += stride) {
     const size_t o = e / per, i = (e % per) * W;
-    const float *src = in + o * count * inner + i;
-    Pack<float, W> s;
+    fold_write<W>(out, o * inner + i, dtype, fold_terms<W>(in + o * count * inner + i, 0, count, 1, inner));
+  }
+}
+
+// Few outputs of many terms: a workgroup takes sixteen neighbouring vectors of outputs, its threads are those x sixteen
+// slices of the terms, which meet in LDS in order.  3 x 16336 sums of 80 terms: 21 us as a sum per thread of sixteen
+// neighbouring outputs to a workgroup, 8 so.
+template <int W>
+__device__ __forceinline__ void fold_job_sliced(const float *in, void *out, size_t outer, size_t inner, int count, int dtype, size_t block) {
+  __shared__ Pack<float, W> part[256];
+  const size_t per = inner / W, e = block * 16 + threadIdx.x % 16;
+  const bool mine = e < outer * per;
+  const size_t o = mine ? e / per : 0, i = mine ? (e % per) * W : 0;
+  const int slice = threadIdx.x / 16;
+  Pack<float, W> s{};
+  if (mine) s = fold_terms<W>(in + o * count * inner + i, slice, count, 16, inner);
+  part[threadIdx.x] = s;
+  __syncthreads();
+  if (slice == 0 && mine) {
+    for (int k = 1; k < 16; ++k)
 #pragma unroll
-    for (int w = 0; w < W; ++w) s.v[w] = 0.0f;
-    int j = 0;
-    for (; j + 8 <= count; j += 8) {                       // eight terms' reads in flight together
-      Pack<float, W> v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)(j + k) * inner);
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-#pragma unroll
-        for (int w = 0; w < W; ++w) s.v[w] += v[k].v[w];
-    }
-    for (; j < count; ++j) {
-      const Pack<float, W> v = *reinterpret_cast<const Pack<float, W> *>(src + (size_t)j * inner);
-#pragma unroll
-      for (int w = 0; w < W; ++w) s.v[w] += v.v[w];
-    }
-    const size_t at = o * inner + i;
-    if (dtype == SSM_F32) {
-      *reinterpret_cast<Pack<float, W> *>(reinterpret_cast<float *>(out) + at) = s;
-    } else if (dtype == SSM_BF16) {
-      Pack<bf16_t, W> r;
-#pragma unroll
-      for (int w = 0; w < W; ++w) r.v[w] = from_f32<bf16_t>(s.v[w]);
-      *reinterpret_cast<Pack<bf16_t, W> *>(reinterpret_cast<bf16_t *>(out) + at) = r;
-    } else {
-      Pack<f16_t, W> r;
-#pragma unroll
-      for (int w = 0; w < W; ++w) r.v[w] = from_f32<f16_t>(s.v[w]);
-      *reinterpret_cast<Pack<f16_t, W> *>(reinterpret_cast<f16_t *>(out) + at) = r;
-    }
+      for (int w = 0; w < W; ++w) s.v[w] += part[k * 16 + threadIdx.x].v[w];
+    fold_write<W>(out, o * inner + i, dtype, s);
   }
 }
 
 __global__ __launch_bounds__(256) void fold_jobs_kernel(const FoldJobs jobs) {
   int j = 0;
   while (j + 1 < jobs.n && blockIdx.x >= jobs.first_block[j + 1]) ++j;
+  if (jobs.sliced[j]) {
+    const size_t block = blockIdx.x - jobs.first_block[j];
+    if (jobs.width[j] == 4) fold_job_sliced<4>(jobs.in[j], jobs.out[j], jobs.outer[j], jobs.inner[j], jobs.count[j], jobs.dtype[j], block);
+    else fold_job_sliced<1>(jobs.in[j], jobs.out[j], jobs.outer[j], jobs.inner[j], jobs.count[j], jobs.dtype[j], block);
+    return;
+  }
   const size_t first = (size_t)(blockIdx.x - jobs.first_block[j]) * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)(jobs.first_block[j + 1] - jobs.first_block[j]) * blockDim.x;
   if (jobs.width[j] == 4) fold_job<4>(jobs.in[j], jobs.out[j], jobs.outer[j], jobs.inner[j], jobs.count[j], jobs.dtype[j], first, stride);
@@ -703,7 +742,9 @@ void FoldJobs::add(const float *src, void *dst, size_t outer_, int count_, size_
   const int j = n++;
   in[j] = src; out[j] = dst; outer[j] = outer_; count[j] = count_; inner[j] = inner_; dtype[j] = dtype_;
   width[j] = inner_ % 4 == 0 && aligned_to(src, 16) && aligned_to(dst, 16) ? 4 : 1;
-  first_block[j + 1] = first_block[j] + fold_grid(outer_ * inner_ / width[j]);
+  const size_t vectors = outer_ * inner_ / width[j];
+  sliced[j] = count_ >= 24 && vectors <= 65536;
+  first_block[j + 1] = first_block[j] + (sliced[j] ? (unsigned)((vectors + 15) / 16) : fold_grid(vectors));
 }
 
 void launch_fold_jobs(const FoldJobs &jobs, hipStream_t s) {
@@ -763,13 +804,13 @@ void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_
   hipLaunchKernelGGL(fold_sum_kernel, dim3(fold_grid(outer * inner)), dim3(256), 0, s, in, out, outer, count, inner);
 }
 
-constexpr int BF_ROWS = 16;              // channels a workgroup of the wave-per-row kernel (scan_bwd_fast.hpp) takes at once
+constexpr int BF_MAX_ROWS = 96;          // channels a workgroup of the wave-per-row kernel (scan_bwd_fast.hpp) takes at most
 
 // How a call is cut into work, from its sizes alone (the workspace is sized before the tensors are known).
 struct BwdPlan {
   int rows_per_wg, nblk;                 // general kernel
   enum { GENERAL, GROUPED, OWN, CONSTANT } route;   // the kernel for whose shape the call has, types permitting
-  int rpw, fast_nblk;                    // GROUPED: rows per wave in turn, workgroups per batch row
+  int span, fast_rows, fast_nblk;        // GROUPED: channels that share B and C, those of them to a workgroup, workgroups per batch row
   int nsplit;                            // chunks that may run side by side (1: a unit walks all of them)
   size_t off_dA, off_dD, off_dbias, off_q, off_dB, off_dC, total;   // byte offsets into the workspace
 };
@@ -792,34 +833,52 @@ static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int
   const int nchunks = (len + BW_T - 1) / BW_T;
   const bool may_split = nchunks > 1 && !in_turn;
   const double all = (double)batch * dim;
+  int span = per_b;                      // channels that share a B group and a C group
+  for (int r = per_c; r;) {
+    const int q = span % r;
+    span = r;
+    r = q;
+  }
+  pl.span = span;
   // Side by side, the chunks fill the chip better and cost a launch more (scan_bwd_maps.hpp), us.
-  const double maps = 12.0 + 0.5 * all * nchunks / 256;
+  const double maps = 7.0 + 0.5 * all * nchunks / 256;
   if (bv && cv && b_groups == dim && c_groups == dim) {
     pl.route = BwdPlan::OWN;
     // bound by memory once the chip is busy, and the maps read C once more: 512 rows of 2048 steps 98 -> 78 us in float32,
     // 1024 168 -> 152, 1536 223 -> 232
     if (own_split && may_split && all <= 1024) pl.nsplit = nchunks;
-  } else if (bv && cv && per_b % BF_ROWS == 0 && per_c % BF_ROWS == 0) {
+  } else if (bv && cv && span >= 8 && len >= 8 && len < (1 << 28)) {
     pl.route = BwdPlan::GROUPED;
-    // us that a chunk takes with a workgroup of 16 x rpw rows on few of the CUs, and how much more on all of them
-    const double alone[3] = {29.0, 53.0, 77.0}, crowd[3] = {9.0, 11.6, 15.0};
-    auto time = [&](int rpw, double units) {
-      const double full = (double)(long)(units / 256), rest = units - full * 256;
-      return full * (alone[rpw - 1] + crowd[rpw - 1]) + (rest > 0.0 ? alone[rpw - 1] + crowd[rpw - 1] * rest / 256 : 0.0);
-    };
+    // A chunk takes a workgroup 8 us, 25.5 for every sixteen rows and 12, 17, 21 or 25.5 for the last four, eight, twelve or
+    // sixteen; its start 5 (bf16, us a chunk measured / so: 9 rows 26 / 29, 14 30.5 / 33.5, 16 32.5 / 33.5, 18 44 / 45.5, 48 87 / 84.5,
+    // 64 rows a chunk each 118 / 115).  Every workgroup leaves a partial sum of dB and dC, which the fold reads.
+    const int units = batch * (dim / span);
+    const double part[5] = {0.0, 12.0, 17.0, 21.0, 25.5};
     double best = 0.0;
-    for (int rpw = 3; rpw >= 1; --rpw) {               // fewer, larger workgroups leave fewer partial sums of dB and dC
-      if (per_b % (BF_ROWS * rpw) || per_c % (BF_ROWS * rpw)) continue;
-      const double units = all / (BF_ROWS * rpw);
-      for (int k = 0; k < (may_split ? 2 : 1); ++k) {
-        const double cost = k ? time(rpw, units * nchunks) + maps : time(rpw, units) * nchunks;
-        if (pl.rpw && cost >= best) continue;
-        best = cost;
-        pl.rpw = rpw;
-        pl.nsplit = k ? nchunks : 1;
+    for (int side = 0; side < (may_split ? 2 : 1); ++side) {
+      const size_t pieces = side ? (size_t)units * nchunks : units;          // workgroups if a span were one
+      const size_t least = (pieces * ((span + BF_MAX_ROWS - 1) / BF_MAX_ROWS) + 255) / 256;
+      for (size_t k = least; k < least + 4; ++k) {
+        const size_t blocks = k * 256 / pieces;
+        int rows = blocks <= 1 ? span : (int)((span + blocks - 1) / blocks);
+        rows = rows < 8 ? 8 : (rows + 3) / 4 * 4;          // rows that cost nothing
+        if (rows > span) rows = span;
+        if (rows > BF_MAX_ROWS) continue;
+        const size_t count = (span + rows - 1) / rows;
+        const double chunk = 8.0 + 25.5 * (rows / 16) + part[(rows % 16 + 3) / 4];
+        const double rounds = (double)((pieces * count + 255) / 256);
+        double cost = rounds * (5.0 + (side ? chunk : chunk * nchunks)) + (side ? maps : 0.0) + 8.0 * units * count * nstate * len / 4.5e6;
+        if (side) cost *= 1.06;            // (where both come out alike: in turn)
+        if (!pl.fast_rows || cost < best) {
+          best = cost;
+          pl.fast_rows = rows;
+          pl.nsplit = side ? nchunks : 1;
+        }
+        if (rows <= 8) break;
       }
     }
-    pl.fast_nblk = dim / (BF_ROWS * pl.rpw);
+    if (!pl.fast_rows) pl.fast_rows = span < BF_MAX_ROWS ? span : BF_MAX_ROWS;
+    pl.fast_nblk = dim / span * ((span + pl.fast_rows - 1) / pl.fast_rows);
   } else if (!bv && !cv) {
     pl.route = BwdPlan::CONSTANT;
     // (walks of 1024 steps are few at ordinary lengths: 512 rows of 8192 steps 133 -> 84 us, of 2048 no gain)
@@ -884,7 +943,7 @@ template <typename io_t>
 static int launch_bwd_maps(const ScanBwdParams &p, int route, float2 *maps, hipStream_t s) {
   if (route == BwdPlan::CONSTANT) return launch_scan_maps_as<io_t, float, false, true>(p, maps, s);
   const bool bc32 = p.bc_dtype == SSM_F32;
-  if (route == BwdPlan::GROUPED)
+  if (route == BwdPlan::GROUPED && p.span % MAPS_WAVES == 0)     // (eight rows then share their slab of C)
     return bc32 ? launch_scan_maps_as<io_t, float, true, false>(p, maps, s) : launch_scan_maps_as<io_t, io_t, true, false>(p, maps, s);
   return bc32 ? launch_scan_maps_as<io_t, float, false, false>(p, maps, s) : launch_scan_maps_as<io_t, io_t, false, false>(p, maps, s);
 }
@@ -984,7 +1043,7 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   p.bc_dtype = a->bc_dtype; p.b_kind = a->b_kind; p.c_kind = a->c_kind;
   p.b_groups = bv ? a->b_groups : 1; p.c_groups = cv ? a->c_groups : 1;
   p.softplus = a->delta_softplus ? 1 : 0;
-  p.rows_per_wg = pl.rows_per_wg; p.nblk = pl.nblk;
+  p.rows_per_wg = pl.rows_per_wg; p.nblk = pl.nblk; p.span = pl.span;
   p.bc_vec_ok = a->seqlen % 4 == 0 && aligned_to(a->Bproj, 4 * bs) && aligned_to(a->Cproj, 4 * bs);
   // A selector of 2 (test-hooks build) lets no wave wait for its neighbour at all, so that the give-up path of
   // the wave-per-row kernel runs: every wave goes on at once and poisons dB and dC.
@@ -1025,11 +1084,11 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
       rc = bc32 ? launch_bwd_rowbc<f16_t, float, float>(p, a->dB, a->dC, s)
                 : (o32 ? launch_bwd_rowbc<f16_t, f16_t, float>(p, a->dB, a->dC, s) : launch_bwd_rowbc<f16_t, f16_t, f16_t>(p, a->dB, a->dC, s));
   } else if (route == BwdPlan::GROUPED) {
-    p.rows_per_wg = BF_WAVES * pl.rpw;
+    p.rows_per_wg = pl.fast_rows;
     p.nblk = pl.fast_nblk;
-    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, pl.rpw, s);
-    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, pl.rpw, s) : launch_bwd_fast<bf16_t, bf16_t>(p, pl.rpw, s);
-    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, pl.rpw, s) : launch_bwd_fast<f16_t, f16_t>(p, pl.rpw, s);
+    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, s);
+    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, s) : launch_bwd_fast<bf16_t, bf16_t>(p, s);
+    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, s) : launch_bwd_fast<f16_t, f16_t>(p, s);
   } else {
     switch (a->io_dtype) {
       case SSM_F32: rc = launch_bwd<float>(p, s); break;
@@ -1047,10 +1106,7 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
     if (kind == SSM_PROJ_BGNL) {
       // (B, G, nblk/G, N*L) -> (B, G, N*L)
       const int per_group = p.nblk / groups;
-      if (a->dbc_dtype == SSM_F32 && fold_sum_is_wide((size_t)Bn * groups, per_group, (size_t)N * L))
-        launch_fold_sum(partial, reinterpret_cast<float *>(out), (size_t)Bn * groups, per_group, (size_t)N * L, s);
-      else
-        jobs.add(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, a->dbc_dtype);
+      jobs.add(partial, out, (size_t)Bn * groups, per_group, (size_t)N * L, a->dbc_dtype);
     } else if (kind == SSM_PROJ_BDN) {
       jobs.add(partial, out, 1, copies / Bn, (size_t)Bn * D * N, SSM_F32);
     } else {

@@ -24,7 +24,7 @@
 
 namespace ssm {
 
-constexpr int BF_WAVES = BF_ROWS;
+constexpr int BF_WAVES = 16;
 constexpr int BF_THREADS = WAVE * BF_WAVES;
 constexpr int BF_K = 8;
 constexpr int BF_DEP = 1;             // wave w takes a state over from wave w + BF_DEP (-1 measured 2 % slower)
@@ -54,22 +54,29 @@ __device__ __forceinline__ bool wait_for_slots(lds_int *flag, int want, int spin
   return reached;
 }
 
+// Call the lines of a row's chunk into the L2 without waiting for them: a lane reads 4 bytes of a line each, to a place in
+// LDS that nobody looks at.
+__device__ __forceinline__ void touch_lines(const void *at, unsigned lds_at) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, off" ::"{m0}"(lds_at), "v"((uintptr_t)at & ~(uintptr_t)3) : "memory");
+}
+
 // A workgroup walks all chunks of its rows, last to first, or (p.maps: the maps of the chunks are known) one of
 // them; blockIdx then counts chunks fastest, and the per-row sums are left per chunk.
-template <typename io_t, typename bc_t, int RPW, bool HAS_Z, bool RAGGED>
+template <typename io_t, typename bc_t, bool HAS_Z>
 __global__ __launch_bounds__(BF_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void scan_bwd_fast_kernel(const ScanBwdParams p) {
   constexpr int K = BF_K, T = FAST_T, NS = FAST_N;
   extern __shared__ __align__(16) float lds[];
+  const int R = p.rows_per_wg;
   float *Bs = lds, *Cs = Bs + NS * T;            // projections of the chunk, [n][q][lane][4]
   float *accB = Cs + NS * T, *accC = accB + NS * T;   // sums over the workgroup's rows, same layout
+  float *dump = accC + NS * T;                   // touch_lines
   // per row, touched by the wave that owns the row only: A log2(e), the adjoint carried between chunks and the
   // sum for dA per state; the sums for dD and the bias
-  float *rowA2 = accC + NS * T, *rowq = rowA2 + BF_WAVES * RPW * NS, *rowdA = rowq + BF_WAVES * RPW * NS;
-  float *rowdD = rowdA + BF_WAVES * RPW * NS, *rowdb = rowdD + BF_WAVES * RPW;
-  lds_int *done = (lds_int *)reinterpret_cast<int *>(rowdb + BF_WAVES * RPW);     // per wave: slots finished since the kernel began
+  float *rowA2 = dump + BF_THREADS, *rowq = rowA2 + R * NS, *rowdA = rowq + R * NS;
+  float *rowdD = rowdA + R * NS, *rowdb = rowdD + R;
+  lds_int *done = (lds_int *)reinterpret_cast<int *>(rowdb + R);     // per wave: slots finished since the kernel began
 
-  constexpr int rows = BF_WAVES * RPW;
   const int wave = wave_id_uniform();
   const int lane = lane_id();
   const int tid = threadIdx.x;
@@ -78,20 +85,36 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
   const int side_by_side = p.maps ? nchunks : 1;
   const int part = (int)blockIdx.x % side_by_side, unit = (int)blockIdx.x / side_by_side;
   const int c_last = p.maps ? part : nchunks - 1, c_first = p.maps ? part : 0;
-  const int b = unit / p.nblk;
-  const int blk = unit % p.nblk;
-  const int d_first = blk * rows;
+  const int b = unit / p.nblk, blk = unit % p.nblk;
+  const int per_span = (p.span + R - 1) / R, in_span = blk % per_span * R;
+  const int d_first = blk / per_span * p.span + in_span, count = min(R, p.span - in_span);
+  const int turns = (count + BF_WAVES - 1) / BF_WAVES;
   const int rev_lane = WAVE - 1 - lane;
-  const size_t bg = (size_t)b * p.b_groups + d_first / (p.dim / p.b_groups), cg = (size_t)b * p.c_groups + d_first / (p.dim / p.c_groups);
-  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + bg * N * L;
-  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + cg * N * L;
-  const size_t Broom = ((size_t)p.batch * p.b_groups - bg) * N * L, Croom = ((size_t)p.batch * p.c_groups - cg) * N * L;
+  const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + ((size_t)b * p.b_groups + d_first / (p.dim / p.b_groups)) * N * L;
+  const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + ((size_t)b * p.c_groups + d_first / (p.dim / p.c_groups)) * N * L;
   const io_t *U = reinterpret_cast<const io_t *>(p.u), *DT = reinterpret_cast<const io_t *>(p.delta);
   const io_t *GO = reinterpret_cast<const io_t *>(p.dout), *Z = reinterpret_cast<const io_t *>(HAS_Z ? p.z : p.u);
   io_t *DU = reinterpret_cast<io_t *>(p.du), *DDL = reinterpret_cast<io_t *>(p.ddelta), *DZ = reinterpret_cast<io_t *>(p.dz);
 
-  for (int rr = 0; rr < RPW; ++rr) {
-    const int r = wave * RPW + rr, d = d_first + r;
+  Pack<io_t, K> ur, dr, gr, zr;
+  auto fetch = [&](int r, int c) {
+    const size_t at = ((size_t)b * p.dim + d_first + r) * L;
+    const int t = c * T + lane * K;
+    ur = row_run<io_t, K>(U + at, t, L);
+    dr = row_run<io_t, K>(DT + at, t, L);
+    gr = row_run<io_t, K>(GO + at, t, L);
+    if (HAS_Z) zr = row_run<io_t, K>(Z + at, t, L);
+  };
+  auto fetched = [&](int c) {                    // what crosses the rows' end put right, zeros past it
+    const int t = c * T + lane * K;
+    row_end(t, L, ur);
+    row_end(t, L, dr);
+    row_end(t, L, gr);
+    if (HAS_Z) row_end(t, L, zr);
+  };
+  if (wave < count) fetch(wave, c_last);
+  for (int r = wave; r < count; r += BF_WAVES) {
+    const int d = d_first + r;
     const size_t row = (size_t)b * p.dim + d;
     if (lane < NS) {
       rowA2[r * NS + lane] = lane < N ? p.A[(size_t)d * N + lane] * LOG2E : 0.0f;
@@ -112,52 +135,88 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     const int t = t0 + lane * K;
     const bool tail = t0 + T > L;
 
-    __syncthreads();                       // the sums of the chunk before are in memory, its slabs are free
-    fast_stage<bc_t, WAVE, RAGGED>(Bs, Bg, L, t0, N, BF_THREADS, Broom);
-    fast_stage<bc_t, WAVE, RAGGED>(Cs, Cg, L, t0, N, BF_THREADS, Croom);
+    __syncthreads();                       // the sums of the chunk before have been read, its slabs are free
+    if (wave < N) {                        // a lane's run of states `wave` of B and of C
+      Pack<bc_t, K> bslab = row_run<bc_t, K>(Bg + (size_t)wave * L, t, L), cslab = row_run<bc_t, K>(Cg + (size_t)wave * L, t, L);
+      if (tail) {
+        row_end(t, L, bslab);
+        row_end(t, L, cslab);
+      }
+#pragma unroll
+      for (int q = 0; q < K / 4; ++q) {
+        *reinterpret_cast<float4 *>(Bs + wave * T + q * (WAVE * 4) + lane * 4) =
+            make_float4(to_f32(bslab.v[4 * q]), to_f32(bslab.v[4 * q + 1]), to_f32(bslab.v[4 * q + 2]), to_f32(bslab.v[4 * q + 3]));
+        *reinterpret_cast<float4 *>(Cs + wave * T + q * (WAVE * 4) + lane * 4) =
+            make_float4(to_f32(cslab.v[4 * q]), to_f32(cslab.v[4 * q + 1]), to_f32(cslab.v[4 * q + 2]), to_f32(cslab.v[4 * q + 3]));
+      }
+    }
     for (int e = tid; e < 2 * NS * T / 4; e += BF_THREADS) reinterpret_cast<float4 *>(accB)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
 
 #pragma nounroll
-    for (int rr = 0; rr < RPW; ++rr) {
-      const int r = wave * RPW + rr, d = d_first + r;
+    for (int turn = 0; turn < turns; ++turn) {
+      const int r = turn * BF_WAVES + wave, d = d_first + r;
+      if (r >= count) {                    // no row: pass the states on
+        for (int slot = 0; slot < NS; ++slot) {
+          if (!wait_for_slots(done + ((wave + BF_DEP) & (BF_WAVES - 1)), nslots, p.spin_limit)) {
+            const int n = (BF_DEP * wave + slot) & (NS - 1);
+            accB[n * T + lane * 4] = accC[n * T + lane * 4] = __builtin_nanf("");
+          }
+          ++nslots;
+          __asm__ volatile("" ::: "memory");
+          if (lane == 0) *(volatile lds_int *)(done + wave) = nslots;
+        }
+        continue;
+      }
       const size_t row = (size_t)b * p.dim + d;
-      const size_t at = row * L, room = ((size_t)p.batch * p.dim - row) * L;
+      const size_t at = row * L;
+      const bool again = r + BF_WAVES < count;
+      const int r_next = again ? r + BF_WAVES : wave, c_next = again ? c : c - 1;       // the wave's next row and chunk
       const float A2_lanes = rowA2[r * NS + (lane & (NS - 1))];
       float qcarry = rowq[r * NS + (lane & (NS - 1))], dA_lanes = 0.0f;
       const float Dk = p.Dk ? p.Dk[d] : 0.0f, bias = p.bias ? p.bias[d] : 0.0f;
       float dD_part = 0.0f, db_part = 0.0f;
-      Pack<io_t, K> ur, dr, gr, zr;
-      auto fetch = [&]() {
-        ur = load_steps<RAGGED, io_t, K>(U + at, t, L, tail, room);
-        dr = load_steps<RAGGED, io_t, K>(DT + at, t, L, tail, room);
-        gr = load_steps<RAGGED, io_t, K>(GO + at, t, L, tail, room);
-        if (HAS_Z) zr = load_steps<RAGGED, io_t, K>(Z + at, t, L, tail, room);
-      };
-      fetch();
       const float Hin_lanes = lane < N ? p.chunk_states[(row * nchunks + c) * (size_t)N + lane] : 0.0f;
 
       float dl[K], du[K], g[K], ghB[K], At[K], pre[K];
       float dsum = 0.0f;
+      if (tail) fetched(c);
 #pragma unroll
       for (int i = 0; i < K; ++i) {
         float x = to_f32(dr.v[i]) + bias;
         if (p.softplus) x = fast_softplus(x);
-        const bool live = t + (RAGGED ? i : 0) < L;
-        dl[i] = live ? x : 0.0f;                       // steps past the end: identity maps, no contributions
-        du[i] = dl[i] * to_f32(ur.v[i]);
-        float gg = live ? to_f32(gr.v[i]) : 0.0f;
+        dl[i] = x;
+        float gg = to_f32(gr.v[i]);
         if (HAS_Z) {
           const float zz = to_f32(zr.v[i]);
           gg *= zz * rcp_hw(1.0f + exp2_hw(-LOG2E * zz));
         }
         g[i] = gg;
+      }
+      if (tail) {                          // steps past the end: identity maps, no contributions
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          dl[i] = t + i < L ? dl[i] : 0.0f;
+          g[i] = t + i < L ? g[i] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        du[i] = dl[i] * to_f32(ur.v[i]);
         ghB[i] = At[i] = pre[i] = 0.0f;
         dsum += dl[i];
       }
-
       for (int slot = 0; slot < NS; ++slot) {
         const int n = (BF_DEP * wave + slot) & (NS - 1);
+        if (sizeof(io_t) == 2 && slot == 1 && c_next >= c_first) {
+          // (not ahead of the first slot, whose wait for the entering states would wait for these too; float32 rows are twice
+          // as many lines, which the L2 does not hold for all CUs: 397 us without, 405 with)
+          constexpr int LINES = T * (int)sizeof(io_t) / 128;           // of 128 bytes, a lane each; 8 to a tensor's row
+          const size_t next = ((size_t)b * p.dim + d_first + r_next) * L + min(c_next * T + lane % LINES * (128 / (int)sizeof(io_t)), L - 1);
+          const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float *)dump + (unsigned)wave * (WAVE * 4u);
+          const int which = lane / LINES;
+          touch_lines((which == 0 ? U : which == 1 ? DT : which == 2 || !HAS_Z ? GO : Z) + next, to);
+        }
         // the SIMD serves its oldest wave first; turn the order round slot by slot so that its four waves keep pace
         {
           const int pr = (slot + (wave >> 2)) & 3;
@@ -243,26 +302,27 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
       // ---- what the row's elements receive; the inputs are read again (the caches hold them) rather than kept in
       // registers over the walk of the states, where they would spill
       __asm__ volatile("" ::: "memory");
-      fetch();
-      float du_o[K], dd_o[K], dz_o[K];
+      fetch(r, c);
+      if (tail) fetched(c);
+      Pack<io_t, K> du_o, dd_o, dz_o;
 #pragma unroll
       for (int i = 0; i < K; ++i) {
         const float uu = to_f32(ur.v[i]);
-        du_o[i] = __builtin_fmaf(dl[i], ghB[i], g[i] * Dk);
+        du_o.v[i] = from_f32<io_t>(__builtin_fmaf(dl[i], ghB[i], g[i] * Dk));
         float dd = __builtin_fmaf(uu, ghB[i], At[i] * LN2);
         if (p.softplus) {
           const float e = exp2_hw(fminf(to_f32(dr.v[i]) + bias, 60.0f) * LOG2E);
           dd *= e * rcp_hw(1.0f + e);                  // softplus' = sigmoid
         }
-        dd = t + (RAGGED ? i : 0) < L ? dd : 0.0f;
-        dd_o[i] = dd;
+        if (tail) dd = t + i < L ? dd : 0.0f;
+        dd_o.v[i] = from_f32<io_t>(dd);
         db_part += dd;
         dD_part = __builtin_fmaf(g[i], uu, dD_part);
         if (HAS_Z) {
           const float zz = to_f32(zr.v[i]);
           const float s = rcp_hw(1.0f + exp2_hw(-LOG2E * zz));
           const float full = __builtin_fmaf(Dk, uu, pre[i]);
-          dz_o[i] = to_f32(gr.v[i]) * full * s * __builtin_fmaf(zz, 1.0f - s, 1.0f);
+          dz_o.v[i] = from_f32<io_t>(to_f32(gr.v[i]) * full * s * __builtin_fmaf(zz, 1.0f - s, 1.0f));
         }
       }
       {
@@ -276,18 +336,10 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
           rowdb[r] += sb;
         }
       }
-      Pack<io_t, K> o;
-#pragma unroll
-      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(du_o[i]);
-      store_steps<RAGGED, io_t, K>(DU + at, t, L, o);
-#pragma unroll
-      for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dd_o[i]);
-      store_steps<RAGGED, io_t, K>(DDL + at, t, L, o);
-      if (HAS_Z) {
-#pragma unroll
-        for (int i = 0; i < K; ++i) o.v[i] = from_f32<io_t>(dz_o[i]);
-        store_steps<RAGGED, io_t, K>(DZ + at, t, L, o);
-      }
+      if (c_next >= c_first) fetch(r_next, c_next);
+      store_steps<true, io_t, K>(DU + at, t, L, du_o);
+      store_steps<true, io_t, K>(DDL + at, t, L, dd_o);
+      if (HAS_Z) store_steps<true, io_t, K>(DZ + at, t, L, dz_o);
     }
 
     __syncthreads();
@@ -301,13 +353,12 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
         const float4 v0 = *reinterpret_cast<const float4 *>(src);
         const float4 v1 = *reinterpret_cast<const float4 *>(src + WAVE * 4);
         float *dst = (which ? p.dC_part : p.dB_part) + (((size_t)b * p.nblk + blk) * N + n) * (size_t)L;
-        store_steps<RAGGED, float, K>(dst, tt, L, Pack<float, K>{{v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w}});
+        store_steps<true, float, K>(dst, tt, L, Pack<float, K>{{v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w}});
       }
     }
   }
 
-  for (int rr = 0; rr < RPW; ++rr) {
-    const int r = wave * RPW + rr;
+  for (int r = wave; r < count; r += BF_WAVES) {
     const size_t row = ((size_t)(p.maps ? part : 0) * p.batch + b) * p.dim + d_first + r;
     if (lane < N) p.dA_rows[row * N + lane] = rowdA[r * NS + lane];
     if (lane == 0) {
@@ -318,25 +369,16 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
 }
 
 template <typename io_t, typename bc_t>
-static int launch_bwd_fast(const ScanBwdParams &p, int rpw, hipStream_t s) {
-  const size_t ldsb = ((size_t)4 * FAST_N * FAST_T + (size_t)BF_WAVES * rpw * (3 * FAST_N + 2) + BF_WAVES) * sizeof(float);
+static int launch_bwd_fast(const ScanBwdParams &p, hipStream_t s) {
+  const size_t ldsb = ((size_t)4 * FAST_N * FAST_T + BF_THREADS + (size_t)p.rows_per_wg * (3 * FAST_N + 2) + BF_WAVES) * sizeof(float);
   const unsigned grid = (unsigned)((size_t)p.batch * p.nblk * (p.maps ? (p.len + FAST_T - 1) / FAST_T : 1));
-#define SSM_BF_LAUNCH(R, HZ)                                                                   \
-  {                                                                                            \
-    auto kernel = p.ragged ? scan_bwd_fast_kernel<io_t, bc_t, R, HZ, true> : scan_bwd_fast_kernel<io_t, bc_t, R, HZ, false>; \
-    if (allow_dynamic_lds(kernel, ldsb) != hipSuccess) {                                       \
-      (void)hipGetLastError();                                                                 \
-      set_error("ssm_scan_bwd: cannot reserve %zu bytes of LDS", ldsb);                        \
-      return SSM_ERR_LAUNCH;                                                                   \
-    }                                                                                          \
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(BF_THREADS), ldsb, s, p);                      \
+  auto kernel = p.z ? scan_bwd_fast_kernel<io_t, bc_t, true> : scan_bwd_fast_kernel<io_t, bc_t, false>;
+  if (allow_dynamic_lds(kernel, ldsb) != hipSuccess) {
+    (void)hipGetLastError();
+    set_error("ssm_scan_bwd: cannot reserve %zu bytes of LDS", ldsb);
+    return SSM_ERR_LAUNCH;
   }
-  if (p.z) {
-    if (rpw == 3) SSM_BF_LAUNCH(3, true) else if (rpw == 2) SSM_BF_LAUNCH(2, true) else SSM_BF_LAUNCH(1, true)
-  } else {
-    if (rpw == 3) SSM_BF_LAUNCH(3, false) else if (rpw == 2) SSM_BF_LAUNCH(2, false) else SSM_BF_LAUNCH(1, false)
-  }
-#undef SSM_BF_LAUNCH
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(BF_THREADS), ldsb, s, p);
   SSM_CHECK_LAUNCH("ssm_scan_bwd");
   return SSM_OK;
 }

@@ -6,7 +6,7 @@
 // the steps is the same for all states, and no scan over the lanes is left, only a wave sum per state.  The kernels
 // that walk the chunks compose the maps between the row's end and their chunk themselves (compose_maps).
 // A sixth of the backward's arithmetic per step.  A workgroup takes one chunk of eight rows, which share the slab of C in
-// LDS: with a row's chunks in one workgroup instead, every wave reading C from memory, that traffic bound the kernel.
+// LDS (where groups are whole blocks of eight channels; otherwise every wave reads its own): with a row's chunks in one workgroup instead, every wave reading C from memory, that traffic bound the kernel.
 #pragma once
 #include "scan_bwd_fast.hpp"
 

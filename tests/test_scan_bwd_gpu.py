@@ -380,6 +380,30 @@ def test_specialised_backward_is_bit_reproducible():
             assert (a is None and b is None) or torch.equal(a, b)
 
 
+@pytest.mark.parametrize("batch,dim,length,nstate,dtype,bc_dtype,groups", [
+    (8, 616, 131, 16, torch.float32, torch.float32, (1, 1)),        # 20 to a workgroup: a second turn of four rows
+    (6, 777, 520, 9, torch.bfloat16, torch.bfloat16, (1, 1)),       # a group's last workgroup has fewer; eight steps in the second chunk
+    (9, 2720, 40, 16, torch.float16, torch.float16, (1, 1)),        # 96: six turns
+    (1, 100, 1543, 16, torch.bfloat16, torch.float32, (1, 1)),      # chunks side by side, blocks of eight rows that straddle nothing
+    (2, 60, 2065, 16, torch.float32, torch.float32, (5, 3)),        # runs of four channels share B and C: the general kernel
+    (2, 48, 1031, 16, torch.bfloat16, torch.bfloat16, (2, 3)),      # runs of eight
+    (1, 8, 9, 5, torch.float32, torch.float32, (1, 1))])
+def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype, bc_dtype, groups):
+    """The wave-per-row kernel with channels left over in a workgroup, and with waves that have no row, against the general kernel on
+    the same inputs: both sum in float32."""
+    inp = make_inputs(length, batch, dim, length, nstate, dtype=dtype, bc_dtype=bc_dtype, groups=1)
+    g = torch.Generator().manual_seed(5)
+    inp["B"], inp["C"] = (torch.randn(batch, n, nstate, length, generator=g).to(bc_dtype) for n in groups)
+    go, gl = torch.randn(batch, dim, length, generator=g).to(dtype), torch.randn(batch, dim, nstate, generator=g)
+    fast, general = _bwd_direct(inp, go, gl, 0), _bwd_direct(inp, go, gl, 1)
+    for k, f, r in zip(("u", "delta", "A", "B", "C", "D", "z", "dt_bias"), fast, general):
+        f, r = f.float().cpu(), r.float().cpu()
+        scale = float(r.abs().max()) + 1e-30
+        # a rounding to 16 bits may go either way; sums over channels and steps in another order
+        tol = dict(rtol=2.0 ** -7, atol=1e-3 * scale) if k in ("u", "delta", "z") and dtype != torch.float32 else dict(rtol=2e-4, atol=2e-5 * scale)
+        torch.testing.assert_close(f, r, **tol, msg=lambda m, k=k: f"grad {k}: {m}")
+
+
 def test_a_wave_that_gives_up_its_wait_poisons_dB_and_dC():
     """The wave-per-row kernel bounds its wait for the neighbouring wave's slot count; a wave that gives up
     writes NaN into its sums so that the caller cannot take them for gradients.  The test-hooks build cuts the
