@@ -186,10 +186,9 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_generic_kernel(const Co
 
 constexpr int CONV_CL_STRIP = 16;   // time steps per thread
 
-// AL: rows (channel vectors) start on 16-byte boundaries and the row length (channel count) is a whole
-// number of vectors; otherwise the same kernel reads and writes element by element.
+// Rows that do not start on 16-byte boundaries or are no whole number of 16-byte vectors: read and written element by element.
 constexpr int CONV_CL_FWD_BYTES = 8;   // bytes of channels per thread
-template <typename T, bool AL, int TAPS>
+template <typename T, int TAPS>
 __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvParams p) {
   constexpr int VEC = CONV_CL_FWD_BYTES / sizeof(T);
   const int cvecs = (p.chans + VEC - 1) / VEC;
@@ -205,56 +204,22 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvPar
   const int K = p.K;
   constexpr int HIST = TAPS - 1;
   float wrev[VEC][TAPS], bias[VEC];
-  if constexpr (AL) load_taps_of<VEC, TAPS>(p.w, p.bias, c0, K, p.wide_taps, wrev, bias);
-  else {
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      bias[i] = (p.bias && i < cw) ? p.bias[c0 + i] : 0.0f;
-      load_taps(p.w, i < cw ? c0 + i : c0, K, wrev[i]);
-    }
+  for (int i = 0; i < VEC; ++i) {
+    bias[i] = (p.bias && i < cw) ? p.bias[c0 + i] : 0.0f;
+    load_taps(p.w, i < cw ? c0 + i : c0, K, wrev[i]);
   }
   const T *xb = reinterpret_cast<const T *>(p.x) + (size_t)b * p.len * p.chans + c0;
   T *yb = reinterpret_cast<T *>(p.y) + (size_t)b * p.len * p.chans + c0;
   const int t_begin = strip * CONV_CL_STRIP;
   const int t_end = min(p.len, t_begin + CONV_CL_STRIP);
-  if constexpr (AL) {
-    // all rows of the strip and the K-1 before it are requested at once, unconditionally (row index clamped
-    // into the sequence, rows before its start become zeros): one wait instead of one per step
-    Pack<T, VEC> raw[HIST + CONV_CL_STRIP];
-#pragma unroll
-    for (int j = 0; j < HIST + CONV_CL_STRIP; ++j) {
-      const int ts = t_begin - HIST + j;
-      raw[j] = *reinterpret_cast<const Pack<T, VEC> *>(xb + (size_t)min(max(ts, 0), p.len - 1) * p.chans);
-    }
-#pragma unroll
-    for (int j = 0; j < HIST; ++j) {
-      if (t_begin - HIST + j < 0) {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) raw[j].v[i] = from_f32<T>(0.0f);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < CONV_CL_STRIP; ++s) {
-      if (t_begin + s >= t_end) break;
-      float out[VEC];
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        float acc = bias[i];
-#pragma unroll
-        for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[i][m], to_f32(raw[HIST + s - m].v[i]), acc);
-        out[i] = p.silu ? silu_f32(acc) : acc;
-      }
-      store_vec<T, VEC>(yb + (size_t)(t_begin + s) * p.chans, 0, out);
-    }
-    return;
-  }
   // hist[j] holds x at time (t - 1 - j); filled with the K-1 rows before the strip
   float hist[HIST][VEC];
 #pragma unroll
   for (int j = 0; j < HIST; ++j) {
     const int ts = t_begin - 1 - j;
     float v[VEC];
-    if (j < K - 1 && ts >= 0) load_run<T, VEC>(xb + (size_t)ts * p.chans, 0, cw, AL, v);
+    if (j < K - 1 && ts >= 0) load_run<T, VEC>(xb + (size_t)ts * p.chans, 0, cw, false, v);
     else {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) v[i] = 0.0f;
@@ -264,7 +229,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvPar
   }
   for (int t = t_begin; t < t_end; ++t) {
     float cur[VEC], out[VEC];
-    load_run<T, VEC>(xb + (size_t)t * p.chans, 0, cw, AL, cur);
+    load_run<T, VEC>(xb + (size_t)t * p.chans, 0, cw, false, cur);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       float acc = __builtin_fmaf(wrev[i][0], cur[i], bias[i]);
@@ -272,7 +237,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvPar
       for (int j = 0; j < HIST; ++j) acc = __builtin_fmaf(wrev[i][j + 1], hist[j][i], acc);
       out[i] = p.silu ? silu_f32(acc) : acc;
     }
-    store_run<T, VEC>(yb + (size_t)t * p.chans, 0, cw, AL, out);
+    store_run<T, VEC>(yb + (size_t)t * p.chans, 0, cw, false, out);
 #pragma unroll
     for (int j = HIST - 1; j > 0; --j)
 #pragma unroll
@@ -282,33 +247,25 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvPar
   }
 }
 
-// The same forward for aligned rows of sequences of at least a few strips: a thread walks CONV_CL_WALK strips in
-// turn.  A launch of one strip per thread runs as a single round of waves that all read, then all compute, then
-// all write.  Walking, a thread requests the rows of its next strip before it computes the present one and keeps
-// the present strip's last K-1 rows as the next one's history (no row is read twice): 25.4 -> 24.1 us at
-// 8 x 2048 x 1536 bf16, whatever the number of strips walked (2 to 16).  What remains is not the shape of the
-// walk: the channels-first kernel does the same arithmetic per element in 19.5 us on rows that are contiguous
-// in time.
-constexpr int CONV_CL_WALK = 4, CONV_CL_WALK_STRIP = 8;   // strips of 8 steps: 24.1 us against 25.4 with 16 and 27.9 with 32
-constexpr int CONV_CL_WALK_THREADS = 64;
+// The same forward for aligned rows: a thread takes a strip of 8 steps of its channels and requests all of its rows, and the
+// taps, at once.  Bound by memory where the call is large, by the latency of one such chain where it is not: a thread that
+// walked four strips in turn, asking for the next one's rows ahead, took 22.6 us for 8 x 2048 x 1536 bf16, 13.9 for 4 x 2048 x
+// 1536, 8.0 for 4 x 2048 x 256 and 7.1 for 1 x 300 x 512, where this takes 22.0, 12.9, 5.4 and 3.9; strips of 4 steps 26.6 and 13.8,
+// of 16 21.6 and 14.1.
+constexpr int CONV_CL_ROWS_THREADS = 64, CONV_CL_ROWS_STRIP = 8;
 template <typename T, int TAPS>
-__global__ __launch_bounds__(CONV_CL_WALK_THREADS) void conv_fwd_cl_walk_kernel(const ConvParams p) {
+__global__ __launch_bounds__(CONV_CL_ROWS_THREADS) void conv_fwd_cl_rows_kernel(const ConvParams p) {
   constexpr int VEC = CONV_CL_FWD_BYTES / sizeof(T);
-  constexpr int HIST = TAPS - 1, S = CONV_CL_WALK_STRIP, SPAN = CONV_CL_WALK_STRIP * CONV_CL_WALK;
-  const int cvecs = p.chans / VEC;
-  const int spans = (p.len + SPAN - 1) / SPAN;
-  const size_t total = (size_t)p.batch * spans * cvecs;
+  constexpr int HIST = TAPS - 1, S = CONV_CL_ROWS_STRIP;
+  const int cvecs = p.chans / VEC, strips = (p.len + S - 1) / S;
   const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= total) return;
-  const int cv = (int)(gid % cvecs);
-  const int span = (int)((gid / cvecs) % spans);
-  const int b = (int)(gid / ((size_t)cvecs * spans));
-  const int c0 = cv * VEC;
+  if (gid >= (size_t)p.batch * strips * cvecs) return;
+  const int c0 = (int)(gid % cvecs) * VEC, t_first = (int)((gid / cvecs) % strips) * S;
+  const size_t base = (size_t)(gid / ((size_t)cvecs * strips)) * p.len * p.chans + c0;
   float wrev[VEC][TAPS], bias[VEC];
   load_taps_of<VEC, TAPS>(p.w, p.bias, c0, p.K, p.wide_taps, wrev, bias);
-  const T *xb = reinterpret_cast<const T *>(p.x) + (size_t)b * p.len * p.chans + c0;
-  T *yb = reinterpret_cast<T *>(p.y) + (size_t)b * p.len * p.chans + c0;
-  const int t_first = span * SPAN;
+  const T *xb = reinterpret_cast<const T *>(p.x) + base;
+  T *yb = reinterpret_cast<T *>(p.y) + base;
   Pack<T, VEC> raw[HIST + S];
 #pragma unroll
   for (int j = 0; j < HIST + S; ++j)
@@ -321,32 +278,16 @@ __global__ __launch_bounds__(CONV_CL_WALK_THREADS) void conv_fwd_cl_walk_kernel(
     }
   }
 #pragma unroll
-  for (int w = 0; w < CONV_CL_WALK; ++w) {
-    const int t_begin = t_first + w * S;
-    Pack<T, VEC> nxt[S];
-    if (w + 1 < CONV_CL_WALK) {
+  for (int s = 0; s < S; ++s) {
+    float out[VEC];
 #pragma unroll
-      for (int j = 0; j < S; ++j)
-        nxt[j] = *reinterpret_cast<const Pack<T, VEC> *>(xb + (size_t)min(t_begin + S + j, p.len - 1) * p.chans);
+    for (int i = 0; i < VEC; ++i) {
+      float acc = bias[i];
+#pragma unroll
+      for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[i][m], to_f32(raw[HIST + s - m].v[i]), acc);
+      out[i] = p.silu ? silu_f32(acc) : acc;
     }
-#pragma unroll
-    for (int sidx = 0; sidx < S; ++sidx) {
-      float out[VEC];
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        float acc = bias[i];
-#pragma unroll
-        for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[i][m], to_f32(raw[HIST + sidx - m].v[i]), acc);
-        out[i] = p.silu ? silu_f32(acc) : acc;
-      }
-      if (t_begin + sidx < p.len) store_vec<T, VEC>(yb + (size_t)(t_begin + sidx) * p.chans, 0, out);
-    }
-    if (w + 1 < CONV_CL_WALK) {
-#pragma unroll
-      for (int j = 0; j < HIST; ++j) raw[j] = raw[S + j];
-#pragma unroll
-      for (int j = 0; j < S; ++j) raw[HIST + j] = nxt[j];
-    }
+    if (t_first + s < p.len) store_vec<T, VEC>(yb + (size_t)(t_first + s) * p.chans, 0, out);
   }
 }
 
@@ -602,9 +543,16 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_walk_kernel(const Co
 // 31 here.  The sums for dw and dbias meet in LDS, one partial per (batch, segment of at least 64 steps).
 constexpr int CONV_CL_STEPS = 16, CONV_CL_WAVES = CONV_THREADS / WAVE, CONV_CL_TILE = CONV_CL_STEPS * CONV_CL_WAVES;
 
-__host__ __device__ inline int conv_cl_tiles_per_seg(int len) {
-  const int tiles = (len + CONV_CL_TILE - 1) / CONV_CL_TILE;
-  return (tiles + CONV_CL_SEGS - 1) / CONV_CL_SEGS;
+// Time segments per batch row at most: four workgroups to a CU, between CONV_CL_SEGS and four times as many (1 x 7040 x 128 bf16
+// 15.7 us with 28 segments, 6.8 with 110; 2 x 6592 x 640 20.6 with 26, 16.7 with 52).
+__host__ __device__ inline int conv_cl_segs(int batch, int chans) {
+  const long long wgs = (long long)batch * ((chans + 127) / 128);
+  const int most = (int)(1024 / (wgs < 1024 ? wgs : 1024));
+  return most < CONV_CL_SEGS ? CONV_CL_SEGS : most > 4 * CONV_CL_SEGS ? 4 * CONV_CL_SEGS : most;
+}
+__host__ __device__ inline int conv_cl_tiles_per_seg(int batch, int chans, int len) {
+  const int tiles = (len + CONV_CL_TILE - 1) / CONV_CL_TILE, segs = conv_cl_segs(batch, chans);
+  return (tiles + segs - 1) / segs;
 }
 
 template <typename T, int TAPS>
@@ -613,7 +561,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
   __shared__ float part[CONV_CL_WAVES][SUMS * VEC][WAVE];
   const int wave = wave_id_uniform(), lane = lane_id();
   const int cblocks = (p.chans + WAVE * VEC - 1) / (WAVE * VEC);
-  const int seg_len = conv_cl_tiles_per_seg(p.len) * CONV_CL_TILE, nseg = (p.len + seg_len - 1) / seg_len;
+  const int seg_len = conv_cl_tiles_per_seg(p.batch, p.chans, p.len) * CONV_CL_TILE, nseg = (p.len + seg_len - 1) / seg_len;
   const int cb = (int)(blockIdx.x % cblocks), seg = (int)((blockIdx.x / cblocks) % nseg), b = (int)(blockIdx.x / ((unsigned)cblocks * nseg));
   const int c0 = (cb * WAVE + lane) * VEC;
   const bool live = c0 < p.chans;
@@ -1020,13 +968,11 @@ static int conv_fwd_typed(const ConvParams &p, int layout, bool vec_ok, hipStrea
     constexpr int VECF = CONV_CL_FWD_BYTES / sizeof(T);
     const size_t threads = (size_t)p.batch * strips * ((p.chans + VECF - 1) / VECF);
     const dim3 grid((unsigned)((threads + CONV_THREADS - 1) / CONV_THREADS));
-    if (vec_ok && p.chans % VEC == 0 && p.len >= 2 * CONV_CL_WALK_STRIP * CONV_CL_WALK) {
-      const int spans = (p.len + CONV_CL_WALK_STRIP * CONV_CL_WALK - 1) / (CONV_CL_WALK_STRIP * CONV_CL_WALK);
-      const size_t walkers = (size_t)p.batch * spans * (p.chans / VECF);
-      const dim3 wgrid((unsigned)((walkers + CONV_CL_WALK_THREADS - 1) / CONV_CL_WALK_THREADS));
-      CONV_LAUNCH(conv_fwd_cl_walk_kernel, T, wgrid, dim3(CONV_CL_WALK_THREADS));
-    } else if (vec_ok && p.chans % VEC == 0) CONV_LAUNCH(conv_fwd_cl_kernel, CONV_T_AL(true), grid, dim3(CONV_THREADS));
-    else CONV_LAUNCH(conv_fwd_cl_kernel, CONV_T_AL(false), grid, dim3(CONV_THREADS));
+    if (vec_ok && p.chans % VEC == 0) {
+      const size_t rows_threads = (size_t)p.batch * ((p.len + CONV_CL_ROWS_STRIP - 1) / CONV_CL_ROWS_STRIP) * (p.chans / VECF);
+      const dim3 rgrid((unsigned)((rows_threads + CONV_CL_ROWS_THREADS - 1) / CONV_CL_ROWS_THREADS));
+      CONV_LAUNCH(conv_fwd_cl_rows_kernel, T, rgrid, dim3(CONV_CL_ROWS_THREADS));
+    } else CONV_LAUNCH(conv_fwd_cl_kernel, T, grid, dim3(CONV_THREADS));
   } else {
     const unsigned grid = (unsigned)min((size_t)65535 * 16, (total + CONV_THREADS - 1) / CONV_THREADS);
     hipLaunchKernelGGL(conv_fwd_generic_kernel<T>, dim3(grid), dim3(CONV_THREADS), 0, s, p, channels_last);
@@ -1068,7 +1014,7 @@ static int conv_bwd_typed(const ConvParams &p, int layout, bool vec_ok, float *d
     constexpr int VECB = CONV_CL_BWD_BYTES / sizeof(T);
     // (a strip's rows are addressed by 32-bit offsets)
     const bool dense = vec_ok && p.chans % VEC == 0 && (size_t)p.chans * sizeof(T) * CONV_CL_STEPS < ((size_t)1 << 31);
-    const int seg_len = dense ? conv_cl_tiles_per_seg(p.len) * CONV_CL_TILE : conv_cl_seg_len(p.len);
+    const int seg_len = dense ? conv_cl_tiles_per_seg(p.batch, p.chans, p.len) * CONV_CL_TILE : conv_cl_seg_len(p.len);
     const int nseg = (p.len + seg_len - 1) / seg_len;
     const size_t vecs = (p.chans + VECB - 1) / VECB, walkers = (size_t)p.batch * nseg * vecs;
     const size_t blocks = dense ? (size_t)p.batch * nseg * ((vecs + WAVE - 1) / WAVE) : (walkers + CONV_THREADS - 1) / CONV_THREADS;
@@ -1160,7 +1106,7 @@ extern "C" int ssm_conv1d_fwd(const ssm_conv1d_fwd_args *a, void *hip_stream) {
 extern "C" size_t ssm_conv1d_bwd_workspace_bytes(int batch, int channels, int width) {
   if (batch <= 0 || channels <= 0 || width <= 0) return 0;
   // one partial per batch row, or per (batch row, time segment) in the channels-last kernel
-  return (size_t)batch * ssm::CONV_CL_SEGS * channels * (width + 1) * sizeof(float);
+  return (size_t)batch * ssm::conv_cl_segs(batch, channels) * channels * (width + 1) * sizeof(float);
 }
 
 extern "C" int ssm_conv1d_bwd(const ssm_conv1d_bwd_args *a, void *hip_stream) {

@@ -140,6 +140,27 @@ def test_rows_of_any_length_keep_to_themselves(dtype, length):
         torch.testing.assert_close(a.double().cpu(), r, rtol=tol, atol=4e-6 * length ** 0.5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 1, 8), (2, 7, 16), (3, 8, 8), (1, 9, 136), (2, 129, 264), (1, 8193, 8), (5, 2047, 24)])
+def test_channels_last_strips_and_segments(dtype, shape):
+    """Around the ends of the forward's strips of 8 steps and of the backward's time segments (8193 steps: 65 of two tiles).
+    One rounding to the type of float32 sums of 4 terms; the sums over all steps as above."""
+    B, L, C = shape
+    g = torch.Generator().manual_seed(L)
+    x, go = (torch.randn(shape, generator=g).to(dtype) for _ in range(2))
+    w, b = torch.rand(C, 4, generator=g) - 0.5, torch.randn(C, generator=g) * 0.02
+    xg, wg, bg = (t.cuda().requires_grad_() for t in (x, w, b))
+    y = _ops().dw_causal_conv_channels_last(xg, wg, bg, activation="silu")
+    got = [y, *torch.autograd.grad(y, [xg, wg, bg], go.cuda())]
+    xr, wr, br = (t.double().requires_grad_() for t in (x, w, b))
+    pad = torch.nn.functional.pad(xr.transpose(1, 2), (3, 0))
+    yr = torch.nn.functional.silu(torch.nn.functional.conv1d(pad, wr[:, None], br, groups=C)).transpose(1, 2)
+    want = [yr, *torch.autograd.grad(yr, [xr, wr, br], go.double())]
+    eps = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for a, r, tol in zip(got, want, (eps, eps, 1e-5, 1e-5)):
+        torch.testing.assert_close(a.double().cpu(), r, rtol=tol, atol=4e-6 * (B * L) ** 0.5)
+
+
 def test_config1_shape_bf16():
     """B=8, C=1536, L=2048, K=4, bf16, SiLU: forward + backward at full size against
     the oracle on a channel slice (channels are independent)."""
