@@ -26,30 +26,33 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 //        then one wave per head forms dt' = clamp(softplus(dt + bias)) and the
 //        running sum of dt' A (stored scaled by log2 e, the unit of the kernels'
 //        exponentials).  For the walk the sums start anew every 32 steps (prep_walk_dt_role).
-//  pack: one wave per operand fragment of C and B^T.  Fragment (lane, j) of a
+//  pack: one workgroup per 32 steps of one (b, c, g): their rows of B and C go into LDS once, as 16-byte loads of whole
+//        rows, and come out as operand fragments, transposed ones by ds_read_b64_tr_b16.  Fragment (lane, j) of a
 //        32 x 16 block: row 32 rb + lane % 32, column 16 kb + 8 (lane / 32) + j.
 //          Cblk [(b,c,g)][lb][kn]  from C  (rows = time, columns = state)
 //          Btblk[(b,c,g)][ks][nt]  from B  (rows = state, columns = time)
 //        and, where a backward will follow, Bblk and Ctblk with B and C in each other's place.
-//  CB:   one wave per 32 x 32 block on or below the diagonal of C B^T of a chunk:
-//        MFMA over the state dimension, then through a wave-private LDS tile into
+//  CB:   one wave per 32 x 32 block on or below the diagonal of C B^T of a chunk: both sets of rows as whole rows
+//        through a wave-private LDS tile, MFMA over the state dimension, and through the tile again into
 //          CBblk[(b,c,g)][lb][ks]  (rows = l, columns = s),
 //        with zeros above the diagonal inside the diagonal blocks; for a backward also its transpose,
 //          CBtblk[(b,c,g)][sb][kl]  (rows = s, columns = l).
 // Steps past the end of a last chunk that is no whole one: size zero, rows of B and C zero.
-// What bounds it is the lines of B, C and dt that each workgroup touches: 4 x 2048 steps, 24 heads, everything a backward
-// needs, 14.5 us (17.3 with 64-bit divisions per wave and neighbours on different XCDs); 4 x 4096 steps, 80 heads, for the
-// walk, 14.7 (16.0).
-// The walk takes the last two roles with chunks of 32 steps, and a fragment of C with its states in the order in which
-// an accumulator's registers hold rows: (lane, j) = state 16 kn + 4 (lane / 32) + j, 8 further for j >= 4.
+// What bounds it is latency, and the lines that a load touches: with fragments read straight from the rows (a load touches 32
+// of them, or two bytes of each of eight), a wave each, 4 x 2048 steps, 24 heads, everything a backward needs, took 14.4 us
+// where this takes 8.9; 4 x 4096 steps, 80 heads, for the walk, 14.3 and 8.2; 3 x 4288, 11 heads 12.7 and 7.8; 1 x 3001, 24 heads
+// 6.0 and 4.9.
+// The walk takes the pack role with chunks of 32 steps, the first wave of each workgroup also the block of C B^T, and a
+// fragment of C with its states in the order in which an accumulator's registers hold rows: (lane, j) = state 16 kn +
+// 4 (lane / 32) + j, 8 further for j >= 4.  It is a kernel of its own: blocks of C B^T take 100 registers, without them 64 leave
+// room for all of its workgroups at once (8.2 us against 10.2).
 constexpr int PD_HEADS = 4, PW_HEADS = 32;     // heads of a workgroup of either dt role
 struct SsdPrepParams {
   SsdCumsumParams cs;
   float *dA2;
   const void *Cm, *Bm;                   // element type of the call
   void *Cblk, *Btblk, *CBblk;
-  void *Bblk, *Ctblk, *CBtblk;           // what the backward reads besides (n_kinds = 4), or null
-  unsigned n_kinds;
+  void *Bblk, *Ctblk, *CBtblk;           // what the backward reads besides, or null
   unsigned n_dt, n_pack;                 // workgroups of the first two roles
   const int *seq_idx;                    // (B, L) sequence ids of a packed batch, or null
   float *steps, *ends;                   // what the walk takes from dt (SsdWalkParams); null: the chunks side by side
@@ -169,83 +172,14 @@ __device__ __forceinline__ void prep_walk_dt_role(const SsdPrepParams &pp, unsig
   }
 }
 
+// A 32 x 32 block of C B^T from the fragments of its rows, through `lds` (32 x 33), to CBblk and its transpose's place.
 template <typename E, int KN>
-__device__ __forceinline__ void prep_pack_role(const SsdPrepParams &pp, unsigned wg) {
-  const SsdDims &d = pp.cs.d;
-  const int wave = wave_id_uniform(), lane = lane_id();
-  constexpr int N = 16 * KN, NT = N >> 5;
-  const int Q = d.chunk, nc = d.nchunks, groups = d.groups, len = d.len;
-  const unsigned per_unit = (unsigned)(Q >> 5) * KN;      // = (Q / 16) * NT fragments, whole workgroups of four
-  const unsigned each = (unsigned)d.batch * nc * groups * (per_unit >> 2);
-  const int kind = (int)(wg / each);                      // rows of C, columns of B, rows of B, columns of C
-  wg -= kind * each;
-  const bool rows = kind == 0 || kind == 2, from_c = kind == 0 || kind == 3;
-  const E *src = reinterpret_cast<const E *>(from_c ? pp.Cm : pp.Bm);
-  const size_t stride = from_c ? pp.c_row : pp.b_row;
-  void *dst = kind == 0 ? pp.Cblk : kind == 1 ? pp.Btblk : kind == 2 ? pp.Bblk : pp.Ctblk;
-  const unsigned unit = wg / (per_unit >> 2), bc = unit / (unsigned)groups;
-  const int inner = (int)((wg - unit * (per_unit >> 2)) * 4) + wave;
-  const size_t f = (size_t)unit * per_unit + inner;
-  const int g = (int)(unit - bc * groups), b = (int)(bc / (unsigned)nc), c = (int)bc - b * nc;
-  const int m = lane & 31, g2 = lane >> 5;
-  src += (size_t)b * len * stride + (size_t)g * N;
-  V8<E> v;
-  if (rows) {
-    const int lb = inner / KN, kn = inner % KN;
-    const int t = c * Q + 32 * lb + m;
-    const E *at = src + (size_t)min(t, len - 1) * stride + 16 * kn;
-    if (pp.steps) {                                       // (kind 0 alone)
-      const V4<E> lo = *reinterpret_cast<const V4<E> *>(at + 4 * g2), hi = *reinterpret_cast<const V4<E> *>(at + 8 + 4 * g2);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) { v[j] = lo[j]; v[4 + j] = hi[j]; }
-    } else {
-      v = load_frag_e<E>(at + 8 * g2);
-    }
-    if (t >= len) v = V8<E>{};
-  } else {
-    const int ks = inner / NT, nt = inner % NT;
-    const int t = c * Q + 16 * ks + 8 * g2;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = src[(size_t)min(t + j, len - 1) * stride + 32 * nt + m];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (t + j >= len) v[j] = (E)0.0f;
-  }
-  *reinterpret_cast<V8<E> *>(reinterpret_cast<E *>(dst) + f * FRAG + lane * 8) = v;
-}
-
-template <typename E, int KN>
-__device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned wg, float *lds) {
-  const SsdDims &d = pp.cs.d;
-  const int wave = wave_id_uniform(), lane = lane_id();
-  constexpr int N = 16 * KN;
-  const int Q = d.chunk, groups = d.groups;
-  const int NLB = Q >> 5, KS = Q >> 4;
-  const unsigned per_unit = (unsigned)NLB * (NLB + 1) / 2;
-  const unsigned units = (unsigned)d.batch * d.nchunks * groups;
-  const unsigned blk = wg * 4 + wave, unit32 = blk / per_unit;
-  if (unit32 >= units) return;
-  const size_t unit = unit32;
-  const int idx = (int)(blk - unit32 * per_unit);
-  int lb = 0;
-  while ((lb + 1) * (lb + 2) / 2 <= idx) ++lb;
-  const int sb = idx - lb * (lb + 1) / 2;
-  const unsigned bc = unit32 / (unsigned)groups, b = bc / (unsigned)d.nchunks;
-  const int g = (int)(unit32 - bc * groups), c = (int)(bc - b * d.nchunks);
-  const size_t row0 = (size_t)b * d.len;                  // rows past the end stand for the last one: they meet only zeros
-  const int m = lane & 31, g2 = lane >> 5;
-  const E *crow_p = reinterpret_cast<const E *>(pp.Cm) + (row0 + min(c * Q + 32 * lb + m, d.len - 1)) * pp.c_row + (size_t)g * N + 8 * g2;
-  const E *brow_p = reinterpret_cast<const E *>(pp.Bm) + (row0 + min(c * Q + 32 * sb + m, d.len - 1)) * pp.b_row + (size_t)g * N + 8 * g2;
+__device__ __forceinline__ void prep_cb_block(const SsdPrepParams &pp, size_t unit, int lb, int sb, const V8<E> (&cf)[KN], const V8<E> (&bf)[KN], float *lds) {
+  const int lane = lane_id(), m = lane & 31, g2 = lane >> 5, NLB = pp.cs.d.chunk >> 5, KS = pp.cs.d.chunk >> 4;
   f32x16_t acc = {0};
-  V8<E> cf[KN], bf[KN];
-#pragma unroll
-  for (int i = 0; i < KN; ++i) {
-    cf[i] = load_frag_e<E>(crow_p + 16 * i);
-    bf[i] = load_frag_e<E>(brow_p + 16 * i);
-  }
 #pragma unroll
   for (int i = 0; i < KN; ++i) acc = mma(cf[i], bf[i], acc);
-  float (*tile)[33] = reinterpret_cast<float (*)[33]>(lds + wave * 32 * 33);
+  float (*tile)[33] = reinterpret_cast<float (*)[33]>(lds);
 #pragma unroll
   for (int r = 0; r < 16; ++r) tile[crow(r, g2)][m] = acc[r];
   wave_lds_sync();
@@ -274,18 +208,157 @@ __device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned w
   }
 }
 
+// What the pack role keeps of 32 steps of B and C in LDS: their rows, 16-byte pieces XOR-swizzled by the row.
+template <int KN> struct PackTile {
+  static constexpr int PIECES = 2 * KN, ROW = 16 * PIECES, BYTES = 32 * ROW;
+  static __device__ __forceinline__ int at(int row, int piece) { return row * ROW + ((piece ^ (row & (PIECES - 1))) << 4); }
+};
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4_t;
+
+template <typename E, int KN, bool WALK>
+__device__ __forceinline__ void prep_pack_role(const SsdPrepParams &pp, unsigned wg, unsigned char *lds) {
+  using Tile = PackTile<KN>;
+  const SsdDims &d = pp.cs.d;
+  const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
+  constexpr int N = 16 * KN, NT = N >> 5, EACH = 32 * Tile::PIECES / 256;
+  const int Q = d.chunk, NLB = Q >> 5, len = d.len;
+  const unsigned unit = wg / (unsigned)NLB, bc = unit / (unsigned)d.groups;
+  const int lb = (int)(wg - unit * NLB), g = (int)(unit - bc * d.groups), b = (int)(bc / (unsigned)d.nchunks), c = (int)bc - b * d.nchunks;
+  const int t0 = c * Q + 32 * lb;
+  V8<E> raw[2][EACH];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const size_t stride = k ? pp.c_row : pp.b_row;
+    const E *src = reinterpret_cast<const E *>(k ? pp.Cm : pp.Bm) + (size_t)b * len * stride + (size_t)g * N;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const int e = tid + 256 * i;
+      raw[k][i] = load_frag_e<E>(src + (size_t)min(t0 + e / Tile::PIECES, len - 1) * stride + 8 * (e % Tile::PIECES));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      const int e = tid + 256 * i, row = e / Tile::PIECES;
+      *reinterpret_cast<V8<E> *>(lds + k * Tile::BYTES + Tile::at(row, e % Tile::PIECES)) = t0 + row < len ? raw[k][i] : V8<E>{};
+    }
+  }
+  __syncthreads();
+  const int m = lane & 31, g2 = lane >> 5, k16 = lane & 15;
+  const size_t base = (size_t)unit * NLB * KN;
+  const auto put = [&](void *dst, int inner, const V8<E> &v) { *reinterpret_cast<V8<E> *>(reinterpret_cast<E *>(dst) + (base + inner) * FRAG + lane * 8) = v; };
+  const auto rows = [&](const unsigned char *tile, void *dst, int i) {
+    put(dst, lb * KN + i, load_frag_e<E>(tile + Tile::at(m, 2 * i + g2)));
+  };
+  const auto columns = [&](const unsigned char *tile, void *dst, int i) {
+    typedef __attribute__((address_space(3))) i16x4_t *ptr;
+    const int ks = i / NT, nt = i % NT, row = 16 * ks + 8 * g2 + (k16 >> 2), piece = 4 * nt + 2 * (lane >> 4 & 1) + ((k16 & 3) >> 1);
+    struct { i16x4_t a, b; } r = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(tile + Tile::at(row, piece) + (k16 & 1) * 8)),
+                                  __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(tile + Tile::at(row + 4, piece) + (k16 & 1) * 8))};
+    put(dst, (2 * lb + ks) * NT + nt, __builtin_bit_cast(V8<E>, r));
+  };
+  const unsigned char *tb = lds, *tc = lds + Tile::BYTES;
+#pragma unroll
+  for (int i0 = 0; i0 < KN; i0 += 4) {
+    const int i = i0 + wave;
+    columns(tb, pp.Btblk, i);
+    if constexpr (WALK) {
+      const V4<E> lo = *reinterpret_cast<const V4<E> *>(tc + Tile::at(m, 2 * i) + 8 * g2), hi = *reinterpret_cast<const V4<E> *>(tc + Tile::at(m, 2 * i + 1) + 8 * g2);
+      put(pp.Cblk, i, V8<E>{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+    } else {
+      rows(tc, pp.Cblk, i);
+    }
+    if (!WALK && pp.Bblk) {
+      rows(tb, pp.Bblk, i);
+      columns(tc, pp.Ctblk, i);
+    }
+  }
+  if (WALK && wave == 0) {
+    V8<E> cf[KN], bf[KN];
+#pragma unroll
+    for (int i = 0; i < KN; ++i) {
+      cf[i] = load_frag_e<E>(tc + Tile::at(m, 2 * i + g2));
+      bf[i] = load_frag_e<E>(tb + Tile::at(m, 2 * i + g2));
+    }
+    prep_cb_block<E, KN>(pp, unit, 0, 0, cf, bf, reinterpret_cast<float *>(lds + 2 * Tile::BYTES));
+  }
+}
+
 template <typename E, int KN>
+__device__ __forceinline__ void prep_cb_role(const SsdPrepParams &pp, unsigned wg, unsigned char *lds) {
+  using Tile = PackTile<KN>;
+  const SsdDims &d = pp.cs.d;
+  const int wave = wave_id_uniform(), lane = lane_id();
+  constexpr int N = 16 * KN;
+  const int Q = d.chunk, groups = d.groups;
+  const int NLB = Q >> 5, KS = Q >> 4;
+  const unsigned per_unit = (unsigned)NLB * (NLB + 1) / 2;
+  const unsigned units = (unsigned)d.batch * d.nchunks * groups;
+  const unsigned blk = wg * 4 + wave, unit32 = blk / per_unit;
+  if (unit32 >= units) return;
+  const size_t unit = unit32;
+  const int idx = (int)(blk - unit32 * per_unit);
+  int lb = 0;
+  while ((lb + 1) * (lb + 2) / 2 <= idx) ++lb;
+  const int sb = idx - lb * (lb + 1) / 2;
+  const unsigned bc = unit32 / (unsigned)groups, b = bc / (unsigned)d.nchunks;
+  const int g = (int)(unit32 - bc * groups), c = (int)(bc - b * d.nchunks);
+  const size_t row0 = (size_t)b * d.len;                  // rows past the end stand for the last one: they meet only zeros
+  const int m = lane & 31, g2 = lane >> 5, r0 = lane / Tile::PIECES, piece = lane % Tile::PIECES;
+  const E *C = reinterpret_cast<const E *>(pp.Cm) + row0 * pp.c_row + (size_t)g * N + 8 * piece;
+  const E *B = reinterpret_cast<const E *>(pp.Bm) + row0 * pp.b_row + (size_t)g * N + 8 * piece;
+  unsigned char *tile = lds + wave * std::max(Tile::BYTES, 32 * 33 * 4);
+  V8<E> craw[KN], braw[KN], cf[KN], bf[KN];
+#pragma unroll
+  for (int i = 0; i < KN; ++i) craw[i] = load_frag_e<E>(C + (size_t)min(c * Q + 32 * lb + r0 + 32 / KN * i, d.len - 1) * pp.c_row);
+#pragma unroll
+  for (int i = 0; i < KN; ++i) braw[i] = load_frag_e<E>(B + (size_t)min(c * Q + 32 * sb + r0 + 32 / KN * i, d.len - 1) * pp.b_row);
+#pragma unroll
+  for (int i = 0; i < KN; ++i) *reinterpret_cast<V8<E> *>(tile + Tile::at(r0 + 32 / KN * i, piece)) = craw[i];
+  wave_lds_sync();
+#pragma unroll
+  for (int i = 0; i < KN; ++i) cf[i] = load_frag_e<E>(tile + Tile::at(m, 2 * i + g2));
+  wave_lds_sync();
+#pragma unroll
+  for (int i = 0; i < KN; ++i) *reinterpret_cast<V8<E> *>(tile + Tile::at(r0 + 32 / KN * i, piece)) = braw[i];
+  wave_lds_sync();
+#pragma unroll
+  for (int i = 0; i < KN; ++i) bf[i] = load_frag_e<E>(tile + Tile::at(m, 2 * i + g2));
+  wave_lds_sync();
+  prep_cb_block<E, KN>(pp, unit, lb, sb, cf, bf, reinterpret_cast<float *>(tile));
+}
+
+// Bytes of LDS: of dt 32 x 65 or 4 x 257 floats; of the pack role the rows of B and C and for the walk a tile of float32; of
+// the blocks of C B^T a tile per wave.
+constexpr int prep_lds_bytes(int KN, bool walk) {
+  return walk ? 2 * 32 * 32 * KN + 32 * 33 * 4 : 4 * std::max(32 * 32 * KN, 32 * 33 * 4);
+}
+
+template <typename E, int KN, bool WALK>
 __global__ __launch_bounds__(256) void ssd_fused_prep_kernel(const SsdPrepParams pp) {
-  __shared__ float lds[4 * 32 * 33];
+  extern __shared__ __align__(16) unsigned char prep_lds[];
   const unsigned wg = blockIdx.x;
   // neighbours in a role, which read the same lines, on one XCD
   if (wg < pp.n_dt) {
-    if (pp.steps) prep_walk_dt_role<std::is_same<E, __bf16>::value>(pp, xcd_order(wg, pp.n_dt), lds);
+    float *lds = reinterpret_cast<float *>(prep_lds);
+    if constexpr (WALK) prep_walk_dt_role<std::is_same<E, __bf16>::value>(pp, xcd_order(wg, pp.n_dt), lds);
     else prep_dt_role(pp, xcd_order(wg, pp.n_dt), lds);
-  } else if (wg < pp.n_dt + pp.n_pack) {
-    prep_pack_role<E, KN>(pp, xcd_order(wg - pp.n_dt, pp.n_pack));
+  } else if (WALK || wg < pp.n_dt + pp.n_pack) {
+    prep_pack_role<E, KN, WALK>(pp, xcd_order(wg - pp.n_dt, pp.n_pack), prep_lds);
+  } else if constexpr (!WALK) {
+    prep_cb_role<E, KN>(pp, xcd_order(wg - pp.n_dt - pp.n_pack, gridDim.x - pp.n_dt - pp.n_pack), prep_lds);
+  }
+}
+
+template <bool WALK>
+static void launch_prep(const SsdPrepParams &pp, dim3 grid, size_t lds, bool f16, int nstate, hipStream_t s) {
+  if (nstate == 128) {
+    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 8, WALK>), grid, dim3(256), lds, s, pp);
+    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 8, WALK>), grid, dim3(256), lds, s, pp);
   } else {
-    prep_cb_role<E, KN>(pp, xcd_order(wg - pp.n_dt - pp.n_pack, gridDim.x - pp.n_dt - pp.n_pack), lds);
+    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 4, WALK>), grid, dim3(256), lds, s, pp);
+    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 4, WALK>), grid, dim3(256), lds, s, pp);
   }
 }
 
@@ -382,7 +455,7 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
     units.nchunks = ssd_walk_blocks(d.len);
   }
   const size_t bcg = (size_t)d.batch * units.nchunks * d.groups;
-  const int NLB = units.chunk >> 5, KN = d.nstate >> 4;
+  const int NLB = units.chunk >> 5;
   SsdPrepParams pp{};
   SsdCumsumParams &cp = pp.cs;
   cp.dt = a->dt; cp.A = a->A; cp.bias = a->dt_bias;
@@ -405,24 +478,19 @@ extern "C" int ssm_ssd_combined_fwd(const ssm_ssd_combined_args *a, void *hip_st
   pp.c_row = a->c_row_stride ? (size_t)a->c_row_stride : dense_row;
   void *Cblk = ws + lay.Cblk, *Btblk = ws + lay.Btblk;
   pp.Cblk = Cblk; pp.Btblk = Btblk; pp.CBblk = ws + lay.CBblk;
-  pp.n_kinds = keep ? 4 : 2;
   if (keep) { pp.Bblk = ws + lay.Bblk; pp.Ctblk = ws + lay.Ctblk; pp.CBtblk = ws + lay.CBtblk; }
   const size_t n_dt = side_by_side ? (size_t)d.batch * d.nchunks * ((d.heads + PD_HEADS - 1) / PD_HEADS)
                                    : (size_t)d.batch * (ssd_walk_turns(units.nchunks) / 2) * ((d.heads + PW_HEADS - 1) / PW_HEADS);
-  const size_t n_pack = bcg * NLB * KN * pp.n_kinds / 4;
-  const size_t n_cb = (bcg * (NLB * (NLB + 1) / 2) + 3) / 4;
+  const size_t n_pack = bcg * NLB;
+  const size_t n_cb = side_by_side ? (bcg * (NLB * (NLB + 1) / 2) + 3) / 4 : 0;
   SSM_REQUIRE(n_dt + n_pack + n_cb < ((size_t)1 << 29), SSM_ERR_TOO_LARGE, "ssm_ssd_combined_fwd: too many workgroups");
   pp.n_dt = (unsigned)n_dt; pp.n_pack = (unsigned)n_pack;
   pp.seq_idx = a->seq_idx;
   const bool f16 = a->io_dtype == SSM_F16;
-  const dim3 prep_grid((unsigned)(n_dt + n_pack + n_cb)), prep_block(256);
-  if (d.nstate == 128) {
-    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 8>), prep_grid, prep_block, 0, s, pp);
-    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 8>), prep_grid, prep_block, 0, s, pp);
-  } else {
-    if (f16) hipLaunchKernelGGL((ssd_fused_prep_kernel<_Float16, 4>), prep_grid, prep_block, 0, s, pp);
-    else hipLaunchKernelGGL((ssd_fused_prep_kernel<__bf16, 4>), prep_grid, prep_block, 0, s, pp);
-  }
+  const dim3 prep_grid((unsigned)(n_dt + n_pack + n_cb));
+  const size_t prep_lds = (size_t)prep_lds_bytes(d.nstate >> 4, !side_by_side);
+  if (side_by_side) launch_prep<false>(pp, prep_grid, prep_lds, f16, d.nstate, s);
+  else launch_prep<true>(pp, prep_grid, prep_lds, f16, d.nstate, s);
   SSM_CHECK_LAUNCH("ssm_ssd_combined_fwd(prep)");
   note_mfma_launch(side_by_side ? 16 : 8);
   if (side_by_side) return ssd_chunk_forward(*a, d, lay, s);
