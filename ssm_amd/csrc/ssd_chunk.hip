@@ -46,7 +46,7 @@ static void forward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
                              hipStream_t s) {
   const dim3 units((unsigned)(d.batch * d.nchunks * d.heads)), block(256);
   hipLaunchKernelGGL((ssd_states_kernel<E, Q, N, false>), units, block, 0, s, st);
-  const unsigned carriers = (unsigned)(d.batch * d.heads) * (SSD_P * N / 1024);
+  const unsigned carriers = (unsigned)carry_units(d);
   bool kept = false;
   if constexpr (std::is_same<E, __bf16>::value) {
     kept = ca.low != nullptr;

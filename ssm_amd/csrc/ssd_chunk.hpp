@@ -23,6 +23,8 @@
 #pragma once
 #include "ssd_common.hpp"
 
+#include <algorithm>
+
 namespace ssm {
 
 template <typename E, int C> struct Row { static_assert(sizeof(E) == 2); E v[C]; } __attribute__((aligned(2 * C)));
@@ -174,8 +176,9 @@ struct SsdCarryParams {
   float *last;                   // (B, H, P, N) or null
   const void *entering;          // REV: the forward's states H
   void *turned, *h_turned;       // REV: G and H as rows of 64 channels, (B, nc, H, N, 64): what ssd_dbc_kernel reads
-  float *through;                // REV: (B, H, nc, dim / 1024) partial sums of exp(cs_Q) <G, H>
+  float *through;                // REV: (B, H, nc, dim / 256) partial sums of exp(cs_Q) <G, H>
   int heads, nchunks, chunk, nstate;
+  int run_chunks;                // REV: chunks that a workgroup writes; it carries the state through those in front of them as well
 };
 
 // A float32 as its bfloat16, rounded to nearest, and the 16 bits that complete it: the operands of the matrix products and
@@ -193,99 +196,124 @@ __device__ __forceinline__ float join_f32(uint16_t high, uint16_t low) {
   return __builtin_bit_cast(float, ((unsigned)high << 16) + low - (low > 0x8000 ? 0x10000u : 0u));
 }
 
-// A thread carries 4 states of one channel over all chunks; backwards of four neighbouring channels, whose 4 x 4 it also
-// stores with channels innermost, and those of H with them.  The reads of several chunks are in flight: with no more than
-// one workgroup on most CUs, latency and (backwards) 88 MB set the time of this launch: at 4 x 2048 steps, 24 heads, 128
-// states 9.5 us forwards and 22.2 backwards.  With H in bfloat16 for <G, H>, and its copy with channels innermost left by the
-// forward, they were 12.8 and 17.1 us.
+// The 4 x 4 16-bit values of a quad of lanes, a row of four in each, turned: lane q takes column q.
+__device__ __forceinline__ uint2 quad_turn(uint2 v) {
+  const int q = lane_id() & 3;
+  const unsigned got = __builtin_amdgcn_update_dpp(0, q & 2 ? v.x : v.y, 0x4e, 0xf, 0xf, true);      // lanes 2 3 0 1
+  const unsigned a = q & 2 ? got : v.x, b = q & 2 ? v.y : got, pick = q & 1 ? 0x03020706u : 0x05040100u;
+  const unsigned a1 = __builtin_amdgcn_update_dpp(0, a, 0xb1, 0xf, 0xf, true);                       // lanes 1 0 3 2
+  const unsigned b1 = __builtin_amdgcn_update_dpp(0, b, 0xb1, 0xf, 0xf, true);
+  return make_uint2(__builtin_amdgcn_perm(a1, a, pick), __builtin_amdgcn_perm(b1, b, pick));
+}
+
+// A thread carries 4 states of one channel over the chunks of its run; a quad of lanes holds four neighbouring channels, which
+// turn their 4 x 4 among themselves for the copies with channels innermost that the backward stores, of G and of H.  The reads of
+// eight chunks are in flight together.  Bound: memory where the calls are large (backwards 14 bytes a state and chunk: at 4 x
+// 2048 steps, 24 heads, 128 states 88 MB in 19.3 us; forwards 10 us), one wave's chain from chunk to chunk where they are
+// small.  With the 4 x 4 of a backward in one thread a quarter of the waves had four times the instructions each: there 22.0 us,
+// at 1 x 3456, 34 heads 27.2 (now 16.2), 1 x 7040, 19 heads, 64 states, chunks of 128 87 (now 20), 1 x 569, 62 heads 8.9 (now 4.9).
 template <typename E, bool REV, bool KEEP>                   // KEEP: for a backward
 __global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) {
-  constexpr int C = REV ? 4 : 1, AHEAD = REV ? 4 : 8;
-  typedef Pack<uint16_t, 4> bits4;
-  const int N = p.nstate, dim = SSD_P * N, per = dim / (1024 * C), kn = N >> 4;
-  const unsigned vid = blockIdx.x;
+  constexpr int AHEAD = 8, PASS = 16;
+  const int N = p.nstate, dim = SSD_P * N, per = dim >> 10, kn = N >> 4;
+  // the workgroups with the most chunks in front of theirs start first
+  const int runs = REV ? (p.nchunks + p.run_chunks - 1) / p.run_chunks : 1;
+  const unsigned units = gridDim.x / (unsigned)runs, vid = REV ? blockIdx.x % units : blockIdx.x;
+  const int begin = REV ? (runs - 1 - (int)(blockIdx.x / units)) * p.run_chunks : 0, stop = REV ? min(begin + p.run_chunks, p.nchunks) : p.nchunks;
   const int part = (int)(vid % per), tid = part * 256 + (int)threadIdx.x;
   const size_t bh = vid / per;
   const int h = (int)(bh % p.heads);
   const size_t b = bh / p.heads;
-  // element 4 (tid % 2) of lane fl of fragment frag; backwards of the lanes fl .. fl + 3
-  const int frag = REV ? tid >> 5 : tid >> 7, j = (REV ? tid >> 3 & 1 : tid & 1) * 4;
-  const int fl = REV ? (tid >> 4 & 1) * 32 + (tid & 7) * 4 : tid >> 1 & 63;
+  // element j of lane fl of fragment frag
+  const int q = tid & 3, frag = tid >> 7, j = REV ? tid & 4 : (tid & 1) * 4, fl = REV ? (tid >> 3 & 15) * 4 + q : tid >> 1 & 63;
   const int e = frag * SSD_FRAG + fl * 8 + j, ch = 32 * (frag / kn) + (fl & 31), n = 16 * (frag % kn) + 8 * (fl >> 5) + j;
+  const int turned = (n + q) * SSD_P + ch - q;
   const size_t user = (bh * SSD_P + ch) * N + n;
   const size_t pitch = (size_t)p.heads * dim, at = (b * p.nchunks * p.heads + h) * dim;
   const float *end = p.dA2 + bh * p.nchunks * p.chunk + p.chunk - 1;
-  float run[C][4];
+  const auto chunk_of = [&](int i) { return REV ? p.nchunks - 1 - i : i; };
+  float run[4];
 #pragma unroll
-  for (int i = 0; i < C; ++i) {
+  for (int k = 0; k < 4; ++k) run[k] = p.first ? p.first[user + k] : 0.0f;
+  const auto pass = [&](float f, const float4 &v) {
+    const float add[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) run[i][k] = p.first ? p.first[user + (size_t)i * N + k] : 0.0f;
+    for (int s = 0; s < 4; ++s) run[s] = __builtin_fmaf(run[s], f, add[s]);
+  };
+  for (int i0 = 0; REV && i0 < begin; i0 += PASS) {
+    float4 v[PASS];
+    float a[PASS];
+#pragma unroll
+    for (int k = 0; k < PASS; ++k) {
+      const int c = chunk_of(min(i0 + k, begin - 1));
+      v[k] = *reinterpret_cast<const float4 *>(p.added + at + c * pitch + e);
+      a[k] = end[(size_t)c * p.chunk];
+    }
+#pragma unroll
+    for (int k = 0; k < PASS; ++k)
+      if (i0 + k < begin) pass(exp2_hw(a[k]), v[k]);
   }
-  for (int i0 = 0; i0 < p.nchunks; i0 += AHEAD) {
-    float4 v[AHEAD][C];
-    bits4 high[AHEAD][C], low[AHEAD][C];
+  for (int i0 = begin; i0 < stop; i0 += AHEAD) {
+    float4 v[AHEAD];
+    uint2 high[AHEAD], low[AHEAD];
     float a[AHEAD];
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) {
-      const int i = min(i0 + k, p.nchunks - 1), c = REV ? p.nchunks - 1 - i : i;
+      const int c = chunk_of(min(i0 + k, stop - 1));
       const size_t o = at + c * pitch + e;
-#pragma unroll
-      for (int q = 0; q < C; ++q) {
-        v[k][q] = *reinterpret_cast<const float4 *>(p.added + o + q * 8);
-        if constexpr (REV) {
-          high[k][q] = *reinterpret_cast<const bits4 *>(reinterpret_cast<const uint16_t *>(p.entering) + o + q * 8);
-          low[k][q] = *reinterpret_cast<const bits4 *>(p.low + o + q * 8);
-        }
+      v[k] = *reinterpret_cast<const float4 *>(p.added + o);
+      if constexpr (REV) {
+        high[k] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(p.entering) + o);
+        low[k] = *reinterpret_cast<const uint2 *>(p.low + o);
       }
       a[k] = end[(size_t)c * p.chunk];
     }
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) {
-      const int i = i0 + k, c = REV ? p.nchunks - 1 - i : i;
-      if (i < p.nchunks) {
+      const int i = i0 + k, c = chunk_of(i);
+      if (i < stop) {
         const size_t o = at + c * pitch;
         const float f = exp2_hw(a[k]);
-        float through = 0.0f;
         if constexpr (!REV && KEEP) {
-          bits4 hi, lo;
+          Pack<uint16_t, 4> hi, lo;
 #pragma unroll
-          for (int s = 0; s < 4; ++s) split_f32(run[0][s], hi.v[s], lo.v[s]);
-          *reinterpret_cast<bits4 *>(reinterpret_cast<uint16_t *>(p.states) + o + e) = hi;
-          *reinterpret_cast<bits4 *>(p.low + o + e) = lo;
+          for (int s = 0; s < 4; ++s) split_f32(run[s], hi.v[s], lo.v[s]);
+          *reinterpret_cast<Pack<uint16_t, 4> *>(reinterpret_cast<uint16_t *>(p.states) + o + e) = hi;
+          *reinterpret_cast<Pack<uint16_t, 4> *>(p.low + o + e) = lo;
         } else {
-#pragma unroll
-          for (int q = 0; q < C; ++q) store4_e<E>(reinterpret_cast<E *>(p.states) + o + e + q * 8, run[q]);
+          store4_e<E>(reinterpret_cast<E *>(p.states) + o + e, run);
         }
         if constexpr (REV) {
+          const auto rounded = [](float lo, float hi) {
+            return (unsigned)__builtin_bit_cast(uint16_t, (E)lo) | (unsigned)__builtin_bit_cast(uint16_t, (E)hi) << 16;
+          };
+          *reinterpret_cast<uint2 *>(reinterpret_cast<E *>(p.turned) + o + turned) = quad_turn(make_uint2(rounded(run[0], run[1]), rounded(run[2], run[3])));
+          *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(p.h_turned) + o + turned) = quad_turn(high[k]);
+          const unsigned hs[4] = {high[k].x & 0xffff, high[k].x >> 16, high[k].y & 0xffff, high[k].y >> 16};
+          const unsigned ls[4] = {low[k].x & 0xffff, low[k].x >> 16, low[k].y & 0xffff, low[k].y >> 16};
+          float through = 0.0f;
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            const float t[4] = {run[0][s], run[1][s], run[2][s], run[3][s]};
-            const bits4 ht = {high[k][0].v[s], high[k][1].v[s], high[k][2].v[s], high[k][3].v[s]};
-            store4_e<E>(reinterpret_cast<E *>(p.turned) + o + (n + s) * SSD_P + ch, t);
-            *reinterpret_cast<bits4 *>(reinterpret_cast<uint16_t *>(p.h_turned) + o + (n + s) * SSD_P + ch) = ht;
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < C; ++q) {
-          const float add[4] = {v[k][q].x, v[k][q].y, v[k][q].z, v[k][q].w};
-#pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            if (REV) through = __builtin_fmaf(run[q][s], join_f32(high[k][q].v[s], low[k][q].v[s]), through);
-            run[q][s] = __builtin_fmaf(run[q][s], f, add[s]);
-          }
-        }
-        if (REV) {
+          for (int s = 0; s < 4; ++s) through = __builtin_fmaf(run[s], join_f32((uint16_t)hs[s], (uint16_t)ls[s]), through);
           through = wave_sum(through) * f;
-          if (lane_id() == 0) p.through[(bh * p.nchunks + c) * (dim >> 10) + part * 4 + (threadIdx.x >> 6)] = through;
+          if (lane_id() == 0) p.through[(bh * p.nchunks + c) * (dim >> 8) + part * 4 + (threadIdx.x >> 6)] = through;
         }
+        pass(f, v[k]);
       }
     }
   }
-  if (p.last) {
-#pragma unroll
-    for (int i = 0; i < C; ++i)
-      *reinterpret_cast<float4 *>(p.last + user + (size_t)i * N) = make_float4(run[i][0], run[i][1], run[i][2], run[i][3]);
-  }
+  if (p.last && stop == p.nchunks)
+    *reinterpret_cast<float4 *>(p.last + user) = make_float4(run[0], run[1], run[2], run[3]);
+}
+
+// A backward's workgroup writes the states of a run of chunks; where there are fewer than one workgroup to two CUs the chunks
+// are cut into several runs of at least 8, each of which reads what the chunks in front of it add once more and forms the
+// same numbers.  1 x 4200 steps, 9 heads, 64 states, chunks of 128: 15.7 us in one run, 12.6 in four (11.6 in eight); 1 x 7040, 19 heads
+// 23.2, 21.2 in three (20.0 in six).  More runs gained nothing more there and cost up to twice the time where chunks are few; the
+// forward, which reads and writes less, gained nothing from any.
+inline int carry_units(const SsdDims &d) { return d.batch * d.heads * (SSD_P * d.nstate / 1024); }
+inline int carry_run(const SsdDims &d) {
+  const int runs = std::max(1, std::min(d.nchunks / 8, 256 / carry_units(d)));
+  return (d.nchunks + runs - 1) / runs;
 }
 
 // ---------------------------------------------------------------------- scan

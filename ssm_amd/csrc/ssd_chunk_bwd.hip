@@ -361,7 +361,7 @@ static BwdLayout bwd_layout(const SsdDims &d) {
   f.s2 = take(units * d.chunk * 4);
   f.xu = take(units * d.chunk * 4);
   f.s1 = take(units * d.chunk * 4);
-  f.through = take(units * (SSD_P * d.nstate / 1024) * 4);
+  f.through = take(units * (SSD_P * d.nstate / 256) * 4);
   f.carried = take(units * 4);
   f.dA = take(units * 4);
   f.dbias = take(units * 4);
@@ -399,7 +399,7 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
     return SSM_ERR_LAUNCH;
   }
   hipLaunchKernelGGL((ssd_states_kernel<elem_t, Q, N, true>), units, block, 0, s, st);
-  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(d.batch * d.heads) * (SSD_P * N / 4096)), block, 0, s, ca);
+  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(carry_units(d) * ((d.nchunks + ca.run_chunks - 1) / ca.run_chunks))), block, 0, s, ca);
   if (dz.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, true>), units, block, 0, s, dz);
   else hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, false>), units, block, 0, s, dz);
   hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DX, false>), units, block, 0, s, dx);
@@ -445,6 +445,7 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   st.x = a->dout; st.z = f.z; st.dy = ws + lay.dy; st.frag = kw + kept.Ctblk; st.dA2 = dA2; st.dtv = dtv; st.states = f32(lay.added);
   st.len = d.len; st.heads = d.heads; st.groups = d.groups; st.nchunks = d.nchunks;
   SsdCarryParams ca{};
+  ca.run_chunks = carry_run(d);
   ca.added = f32(lay.added); ca.states = ws + lay.states; ca.turned = ws + lay.turned; ca.dA2 = dA2; ca.first = a->dfinal; ca.last = a->dinitial_states; ca.entering = kw + kept.states; ca.through = f32(lay.through);
   ca.low = const_cast<uint16_t *>(reinterpret_cast<const uint16_t *>(kw + kept.states_low)); ca.h_turned = ws + lay.h_turned;
   ca.heads = d.heads; ca.nchunks = d.nchunks; ca.chunk = d.chunk; ca.nstate = d.nstate;
@@ -466,7 +467,7 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   SsdDtParams dt{};
   dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.through = f32(lay.through); dt.carried = f32(lay.carried); dt.dt_raw = f.dt;
   dt.A = f.A; dt.bias = f.dt_bias; dt.ddt = a->ddt; dt.dA = f32(lay.dA); dt.dbias = f32(lay.dbias);
-  dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.parts = SSD_P * d.nstate / 1024; dt.dt_dtype = f.dt_dtype;
+  dt.len = d.len; dt.heads = d.heads; dt.nchunks = d.nchunks; dt.parts = SSD_P * d.nstate / 256; dt.dt_dtype = f.dt_dtype;
   dt.softplus = f.dt_softplus ? 1 : 0; dt.dt_min = f.dt_min; dt.dt_max = f.dt_max;
 
   int rc = SSM_OK;
