@@ -53,8 +53,8 @@ static void forward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
     if (kept) hipLaunchKernelGGL((ssd_carry_kernel<E, false, true>), dim3(carriers), block, 0, s, ca);
   }
   if (!kept) hipLaunchKernelGGL((ssd_carry_kernel<E, false, false>), dim3(carriers), block, 0, s, ca);
-  if (sc.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, SCAN_Y, true>), units, block, 0, s, sc);
-  else hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, SCAN_Y, false>), units, block, 0, s, sc);
+  if (sc.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, true>), units, block, 0, s, sc);
+  else hipLaunchKernelGGL((ssd_chunk_scan_kernel<E, Q, N, false>), units, block, 0, s, sc);
 }
 
 int ssd_chunk_forward(const ssm_ssd_combined_args &a, const SsdDims &d, const SsdWorkLayout &lay, hipStream_t s) {

@@ -33,8 +33,7 @@ template <typename E, int C> struct Row { static_assert(sizeof(E) == 2); E v[C];
 struct ChunkUnit {
   int b, c, h, g, rows;          // rows: steps of this chunk
   size_t row0, step0, unit, state;
-  __device__ __forceinline__ ChunkUnit(int len, int heads, int groups, int nchunks, int Q, int N) {
-    const unsigned vid = xcd_order(blockIdx.x, gridDim.x);
+  __device__ __forceinline__ ChunkUnit(unsigned vid, int len, int heads, int groups, int nchunks, int Q, int N) {
     h = (int)(vid % heads);
     const unsigned bc = vid / heads;
     c = (int)(bc % nchunks);
@@ -92,7 +91,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
   __shared__ __align__(16) E xT[SSD_P * Q];
   using S = Staging<Q>;
   constexpr int KS = Q >> 4, KN = N >> 4, NT = N >> 5, PW = NT >= 4 ? 2 : 1, AHEAD = BWD || KS < 8 ? 4 : 8;
-  const ChunkUnit u(p.len, p.heads, p.groups, p.nchunks, Q, N);
+  const ChunkUnit u(xcd_order(blockIdx.x, gridDim.x), p.len, p.heads, p.groups, p.nchunks, Q, N);
   const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
   const int m = lane & 31, g2 = lane >> 5;
   const int nt = PW == 2 ? wave : wave & 1, pt0 = PW == 2 ? 0 : wave >> 1;
@@ -347,19 +346,22 @@ struct SsdChunkScanParams {
 // row sums needs both to multiply the same block.
 // SCAN_DZ forms dy from dout and z, which it reads for dz anyway, where reading the states kernel's dy back made it
 // wait for a fourth tensor: 39.5 us before, 36.5 now (2 x 2048 steps, 24 heads, bfloat16).
+template <typename E, int Q, int N, bool GRAD> struct ScanLds {
+  // the carried state is through before the staged rows take its place
+  __align__(16) E tile[SSD_P * (Q > N ? Q : N)];
+  __align__(16) float dAs[Q];
+  __align__(16) float Ps[Q], Rs[Q];                           // decay from the block before to a step, from a step to the end of its block
+  __align__(16) float l2s[GRAD ? 4 : Q];                      // log2 dt
+  float halves[Q < 256 && GRAD ? 4 * Q : 8];                  // row sums of half rows; or sums per wave
+};
+
 template <typename E, int Q, int N, int MODE, bool HAS_Z>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_chunk_scan_kernel(const SsdChunkScanParams p) {
+__device__ __forceinline__ void chunk_scan(const SsdChunkScanParams &p, unsigned vid, ScanLds<E, Q, N, MODE != SCAN_Y> &lds) {
   using S = Staging<Q>;
   constexpr int NLB = Q >> 5, KS = Q >> 4, KN = N >> 4, NPAIR = NLB / 2, PW = NPAIR >= 4 ? 2 : 1;
-  // the carried state is through before the staged rows take its place
-  constexpr int TILE = SSD_P * (Q > N ? Q : N);
-  __shared__ __align__(16) E tile[TILE];
-  E *xT = tile, *hs = tile;
-  __shared__ __align__(16) float dAs[Q];
-  __shared__ __align__(16) float Ps[Q], Rs[Q];                           // decay from the block before to a step, from a step to the end of its block
-  __shared__ __align__(16) float l2s[MODE == SCAN_Y ? Q : 4];            // log2 dt
-  __shared__ float halves[PW == 1 && MODE != SCAN_Y ? 4 * Q : 8];       // row sums of half rows; or sums per wave
-  const ChunkUnit u(p.len, p.heads, p.groups, p.nchunks, Q, N);
+  E *tile = lds.tile, *xT = tile, *hs = tile;
+  float *dAs = lds.dAs, *Ps = lds.Ps, *Rs = lds.Rs, *l2s = lds.l2s, *halves = lds.halves;
+  const ChunkUnit u(vid, p.len, p.heads, p.groups, p.nchunks, Q, N);
   const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
   const int m = lane & 31, g2 = lane >> 5;
   const int pair = PW == 2 ? wave : wave >> 1, pt0 = PW == 2 ? 0 : wave & 1;
@@ -685,6 +687,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void s
     if (tid == 0 && p.dD) p.dD[(size_t)(u.b * p.nchunks + u.c) * p.heads + u.h] = (halves[0] + halves[1]) + (halves[2] + halves[3]);
     if (tid == 0) p.carried[u.step0 / Q] = (halves[4] + halves[5]) + (halves[6] + halves[7]);
   }
+}
+
+template <typename E, int Q, int N, bool HAS_Z>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_chunk_scan_kernel(const SsdChunkScanParams p) {
+  __shared__ ScanLds<E, Q, N, false> lds;
+  chunk_scan<E, Q, N, SCAN_Y, HAS_Z>(p, xcd_order(blockIdx.x, gridDim.x), lds);
+}
+
+// Both scans of a backward in one launch, neighbouring workgroups a unit's dz and dx: neither needs the other, and calls whose units do
+// not fill the chip take little more time for both than for one.  3 x 896 steps, 18 heads, 128 states, chunks of 256: 23.3 us, in
+// two launches 17.5 and 13.7; 1 x 7040, 19 heads, 64 states, chunks of 128 36.5, so 24.5 and 19.9; 4 x 2048, 24 heads 66 either way.
+template <typename E, int Q, int N, bool HAS_Z>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void ssd_grad_scans_kernel(const SsdChunkScanParams dz, const SsdChunkScanParams dx) {
+  __shared__ ScanLds<E, Q, N, true> lds;
+  const unsigned vid = xcd_order(blockIdx.x, gridDim.x);
+  if (vid & 1) chunk_scan<E, Q, N, SCAN_DX, false>(dx, vid >> 1, lds);
+  else chunk_scan<E, Q, N, SCAN_DZ, HAS_Z>(dz, vid >> 1, lds);
 }
 
 }  // namespace ssm

@@ -2,7 +2,7 @@
 //
 //   states  dy = dout silu(z), rounded and kept; what each chunk adds to the adjoint state
 //   carry   the adjoint state leaving each chunk, last to first, and what of <G, H> goes through each chunk
-//   scan    y again for dz and its row sums;  u for dx and its row sums
+//   scans   y again for dz and its row sums;  u for dx and its row sums
 //   dbc     dB and dC, every head of a group (or of a slice of one) in one workgroup
 //   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one launch adds those up
 //
@@ -400,9 +400,9 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
   }
   hipLaunchKernelGGL((ssd_states_kernel<elem_t, Q, N, true>), units, block, 0, s, st);
   hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(carry_units(d) * ((d.nchunks + ca.run_chunks - 1) / ca.run_chunks))), block, 0, s, ca);
-  if (dz.z) hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, true>), units, block, 0, s, dz);
-  else hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DZ, false>), units, block, 0, s, dz);
-  hipLaunchKernelGGL((ssd_chunk_scan_kernel<elem_t, Q, N, SCAN_DX, false>), units, block, 0, s, dx);
+  const dim3 both(2 * units.x);
+  if (dz.z) hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, true>), both, block, 0, s, dz, dx);
+  else hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, false>), both, block, 0, s, dz, dx);
   hipLaunchKernelGGL((ssd_dbc_kernel<Q, N>), dim3(2u * bc.units * bc.slices * (Q / 64)), dim3(64 * DBC_WAVES<Q>), dbc_lds, s, bc);
   hipLaunchKernelGGL((ssd_dt_kernel<Q>), dim3((unsigned)(d.batch * d.nchunks * ((d.heads + DT_HEADS - 1) / DT_HEADS))), block, 0, s, dt);
   return SSM_OK;
