@@ -3,8 +3,8 @@
 //   states  dy = dout silu(z), rounded and kept; what each chunk adds to the adjoint state
 //   carry   the adjoint state leaving each chunk, last to first, and what of <G, H> goes through each chunk
 //   scans   y again for dz and its row sums;  u for dx and its row sums
-//   dbc     dB and dC, every head of a group (or of a slice of one) in one workgroup
-//   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one launch adds those up
+//   dbc     dB and dC, every head of a group (or of a slice of one) in one workgroup; and in the same launch
+//   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one more launch adds those up
 //
 // What the forward prepared (steps, running sums, operand fragments, the states entering the chunks) is read, not formed again.
 #include "ssd_chunk.hpp"
@@ -46,7 +46,7 @@ struct SsdDbcParams {
 // meets as many: 48.7 here, 1.5 % more of a training step at three times the batch.
 template <int Q> constexpr int DBC_WAVES = Q >= 256 ? 16 : 8;
 template <int Q, int N, bool for_b>
-__device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned char *smem) {
+__device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, unsigned char *smem) {
   typedef V8<elem_t> v8;
   typedef const __attribute__((address_space(1))) char *global_bytes;
   typedef const __attribute__((address_space(1))) v8 *global_v8;
@@ -61,7 +61,7 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned char *s
   const int m = lane & 31, g2 = lane >> 5, ot = wave & 1, mw = wave >> 1;
   // the workgroups that meet the most rows start first
   const unsigned same = 2u * p.units * p.slices;
-  const unsigned rank = blockIdx.x / same, rest = blockIdx.x % same;
+  const unsigned rank = block / same, rest = block % same;
   const unsigned unit = (rest >> 1) % p.units, slice = (rest >> 1) / p.units;
   const int r = for_b ? (int)rank : NR - 1 - (int)rank;
   const int meets = (int)(NR - rank);                                  // blocks of 64 rows
@@ -236,13 +236,6 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned char *s
   }
 }
 
-template <int Q, int N>
-__global__ __launch_bounds__(64 * DBC_WAVES<Q>) void ssd_dbc_kernel(const SsdDbcParams p) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  if (blockIdx.x & 1) dbc_rows<Q, N, true>(p, smem);
-  else dbc_rows<Q, N, false>(p, smem);
-}
-
 // ---------------------------------------------------------------------- dt
 
 // With q_t = a_t <G_t, H_{t-1}>:  ddt_t = A q_t + <x_t, u_t>,  dA = sum dt_t q_t.  Inside a chunk q follows from row sums of the
@@ -266,25 +259,23 @@ struct SsdDtParams {
   float dt_min, dt_max;
 };
 
-// A workgroup takes a chunk of 4 heads, a wave one of them, each lane Q / 64 neighbouring steps.  (16 heads per workgroup, a
-// row's 32 bytes together: 64 workgroups and 16 us at batch 4, 2048 steps, 24 heads.)
-constexpr int DT_HEADS = 4;
+// A workgroup takes a chunk of as many heads as it has waves, a wave one of them, each lane Q / 64 neighbouring steps.
 template <int Q>
-__global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
-  constexpr int PER = Q / 64;
-  __shared__ float tile[DT_HEADS][Q + 1];
+__device__ __forceinline__ void dt_rows(const SsdDtParams &p, unsigned block, unsigned char *smem) {
+  constexpr int PER = Q / 64, DT_HEADS = DBC_WAVES<Q>, PITCH = Q + 1;
+  float *tile = reinterpret_cast<float *>(smem);                       // [DT_HEADS][PITCH]
   const int hgroups = (p.heads + DT_HEADS - 1) / DT_HEADS;
-  const int hg = (int)(blockIdx.x % hgroups), bc = (int)(blockIdx.x / hgroups), c = bc % p.nchunks, b = bc / p.nchunks;
+  const int hg = (int)(block % hgroups), bc = (int)(block / hgroups), c = bc % p.nchunks, b = bc / p.nchunks;
   const int h0 = hg * DT_HEADS, rows = min(Q, p.len - c * Q);
   const size_t base = ((size_t)b * p.len + (size_t)c * Q) * p.heads + h0;
   const int hh = (int)threadIdx.x % DT_HEADS, l0 = (int)threadIdx.x / DT_HEADS;
-  for (int l = l0; l < Q; l += 256 / DT_HEADS)
-    tile[hh][l] = h0 + hh < p.heads && l < rows ? load_as_f32(p.dt_raw, p.dt_dtype, base + (size_t)l * p.heads + hh) : 0.0f;
+  for (int l = l0; l < Q; l += 64)
+    tile[hh * PITCH + l] = h0 + hh < p.heads && l < rows ? load_as_f32(p.dt_raw, p.dt_dtype, base + (size_t)l * p.heads + hh) : 0.0f;
   __syncthreads();
   const int wave = wave_id_uniform(), lane = lane_id();
-  for (int k = wave; k < DT_HEADS; k += 4) {
-    const int h = h0 + k;
-    if (h >= p.heads) break;
+  const int h = h0 + wave;
+  float *row = tile + wave * PITCH;
+  if (h < p.heads) {
     const size_t unit = ((size_t)b * p.heads + h) * p.nchunks + c, at = unit * Q + lane * PER;
     float s1[PER], s2[PER], xu[PER], dt[PER], d[PER], tot = 0.0f;
 #pragma unroll
@@ -307,13 +298,13 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
     for (int i = 0; i < PER; ++i) {
       const int l = lane * PER + i;
       const float q = before + d[i];
-      const float raw = tile[k][l] + bias;
+      const float raw = row[l] + bias;
       const float v = p.softplus ? softplus_f32(raw) : raw;
       const float chain = v >= p.dt_min && v <= p.dt_max ? (p.softplus ? sigmoid_f32(raw) : 1.0f) : 0.0f;
       const float g = l < rows ? __builtin_fmaf(A, q, xu[i]) * chain : 0.0f;
       dA = l < rows ? __builtin_fmaf(dt[i], q, dA) : dA;
       db += g;
-      tile[k][l] = g;
+      row[l] = g;
     }
     dA = wave_sum(dA);
     db = wave_sum(db);
@@ -324,7 +315,22 @@ __global__ __launch_bounds__(256) void ssd_dt_kernel(const SsdDtParams p) {
   }
   __syncthreads();
   if (h0 + hh < p.heads)
-    for (int l = l0; l < rows; l += 256 / DT_HEADS) store_any(p.ddt, p.dt_dtype, base + (size_t)l * p.heads + hh, tile[hh][l]);
+    for (int l = l0; l < rows; l += 64) store_any(p.ddt, p.dt_dtype, base + (size_t)l * p.heads + hh, tile[hh * PITCH + l]);
+}
+
+// Both in one launch: the workgroups of dt, of which there are few and short ones, start first, and those of dbc that meet the fewest rows
+// wait for their CUs.  At 4 x 2048 steps, 24 heads, 128 states, chunks of 256 52.6 us, in two launches 51.7 and 7.1; 2 x 2048, 48 heads, 64
+// states 43.3, so 43.1 and 7.0; 3 x 896, 18 heads 27.7, so 26.8 and 5.2.
+template <int Q> constexpr unsigned dt_blocks(const SsdDims &d) {
+  return (unsigned)(d.batch * d.nchunks * ((d.heads + DBC_WAVES<Q> - 1) / DBC_WAVES<Q>));
+}
+template <int Q, int N>
+__global__ __launch_bounds__(64 * DBC_WAVES<Q>) void ssd_dbc_dt_kernel(const SsdDbcParams p, const SsdDtParams t, unsigned first) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x < first) return dt_rows<Q>(t, blockIdx.x, smem);
+  const unsigned block = blockIdx.x - first;
+  if (block & 1) dbc_rows<Q, N, true>(p, block, smem);
+  else dbc_rows<Q, N, false>(p, block, smem);
 }
 
 // ---------------------------------------------------------------------- host
@@ -394,7 +400,8 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
                              hipStream_t s) {
   const dim3 units((unsigned)(d.batch * d.nchunks * d.heads)), block(256);
   constexpr size_t dbc_lds = 2 * ((1 + Q / 64) * 64 * 64 + N * 64) * sizeof(elem_t) + 8 * Q * sizeof(float);
-  if (allow_dynamic_lds(ssd_dbc_kernel<Q, N>, dbc_lds) != hipSuccess) {
+  static_assert(dbc_lds >= DBC_WAVES<Q> * (Q + 1) * sizeof(float));
+  if (allow_dynamic_lds(ssd_dbc_dt_kernel<Q, N>, dbc_lds) != hipSuccess) {
     set_error("ssm_ssd_combined_bwd: cannot reserve %zu bytes of LDS", dbc_lds);
     return SSM_ERR_LAUNCH;
   }
@@ -403,8 +410,8 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
   const dim3 both(2 * units.x);
   if (dz.z) hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, true>), both, block, 0, s, dz, dx);
   else hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, false>), both, block, 0, s, dz, dx);
-  hipLaunchKernelGGL((ssd_dbc_kernel<Q, N>), dim3(2u * bc.units * bc.slices * (Q / 64)), dim3(64 * DBC_WAVES<Q>), dbc_lds, s, bc);
-  hipLaunchKernelGGL((ssd_dt_kernel<Q>), dim3((unsigned)(d.batch * d.nchunks * ((d.heads + DT_HEADS - 1) / DT_HEADS))), block, 0, s, dt);
+  const unsigned first = dt_blocks<Q>(d), all = first + 2u * bc.units * bc.slices * (Q / 64);
+  hipLaunchKernelGGL((ssd_dbc_dt_kernel<Q, N>), dim3(all), dim3(64 * DBC_WAVES<Q>), dbc_lds, s, bc, dt, first);
   return SSM_OK;
 }
 
