@@ -332,8 +332,12 @@ template <typename io_t, int VEC>
 static dim3 onepass_grid(DscanParams &p, bool params, hipStream_t s) {
   const unsigned blocks = (unsigned)(((size_t)p.heads * p.proj + WAVE * VEC - 1) / (WAVE * VEC));
   const int rounds = (p.len + DO_ROUND - 1) / DO_ROUND;
-  // 1.7 us a round: 29 us for the 16 rounds of 2048 steps by 32 workgroups
-  p.seg_rounds = dscan_rounds_per_segment((size_t)blocks * p.batch, rounds, 1.7);
+  // us a round, its tensors and elements a lane: 1.5 and 2.3 for X and Y alone in float32 and in 16 bits, 2.4 and 2.6 with B, C and a
+  // gate.  Fitted with the other figures to times of 1 to 32 segments at 110 sizes (1 to 280 heads over the batch, 200 to 4096
+  // steps); with 1.7 for all, a share of 0.5 and a choice that skipped most segments of two rounds and less those calls took 2.6 % more in the mean:
+  // 1 x 1280 steps, 8 heads, gated bf16 14.7 -> 11.1 us, 4 x 512, 28 heads 18.7 -> 13.4, 2 x 384, 16 heads 13.8 -> 10.5.
+  const double us = params ? (VEC == 2 ? 2.3 : 1.5) : VEC == 2 ? 2.6 : 2.4;
+  p.seg_rounds = dscan_rounds_per_segment((size_t)blocks * p.batch, rounds, us, 3.0, 0.7);
   int nseg = (rounds + p.seg_rounds - 1) / p.seg_rounds;
   if (nseg > p.nseg) p.seg_rounds = rounds, nseg = 1;
   p.maps = nullptr;

@@ -376,7 +376,7 @@ extern "C" int ssm_dscan_bwd(const ssm_dscan_bwd_args *a, void *hip_stream) {
     // per-channel sums of a batch row, (B, HP) each; those that are the caller's gradient already go there
     float *sums = ws + (size_t)Bn * rounds * HP;
     // 2.3 us a round: 75 us for the 32 rounds of 2048 steps by 32 workgroups
-    p.seg_rounds = dscan_rounds_per_segment((size_t)Bn * ((HP + WAVE * vec - 1) / (WAVE * vec)), rounds, 2.3);
+    p.seg_rounds = dscan_rounds_per_segment((size_t)Bn * ((HP + WAVE * vec - 1) / (WAVE * vec)), rounds, 2.3, 4.0, 0.5);
     const int segs = (rounds + p.seg_rounds - 1) / p.seg_rounds, copies = segs * Bn;
     const size_t each = (size_t)copies * HP;
     SSM_REQUIRE((size_t)Bn * rounds * HP + 4 * each + 2 * bhp * std::max(segs, nseg) + 1 <= a->workspace_bytes / 4, SSM_ERR_WORKSPACE, "ssm_dscan_bwd: workspace too small");

@@ -135,20 +135,20 @@ static void launch_dscan_maps(const DscanMapParams &p, hipStream_t s) {
 }
 
 // Segments of a walk of `rounds` rounds by `wgs` workgroups, in rounds per segment.  A workgroup fills a CU, a round takes
-// it `us`, starting a workgroup about two; the maps are a launch of four and about half the walk's own work.
-static int dscan_rounds_per_segment(size_t wgs, int rounds, double us) {
-  int best_n = 1;
+// it `us`, starting a workgroup about two; the maps are a launch of `launch` us and a `share` of the walk's own work.
+static int dscan_rounds_per_segment(size_t wgs, int rounds, double us, double launch, double share) {
+  int best_per = rounds;
   double best = 0.0;
-  for (int n = 1; n <= 32 && n <= rounds; n = n < 8 ? n + 1 : n * 2) {
-    const int per = (rounds + n - 1) / n;
-    const double turns = (double)((wgs * ((rounds + per - 1) / per) + 255) / 256);
-    const double cost = turns * (2.0 + us * per) + (n > 1 ? 4.0 + 0.5 * us * rounds * (double)wgs / 256 : 0.0);
-    if (n == 1 || cost < 0.95 * best) {
+  for (int per = rounds; per >= 1 && (rounds + per - 1) / per <= 32; --per) {
+    const int n = (rounds + per - 1) / per;
+    const double turns = (double)((wgs * n + 255) / 256);
+    const double cost = turns * (2.0 + us * per) + (n > 1 ? launch + share * us * rounds * (double)wgs / 256 : 0.0);
+    if (per == rounds || cost < 0.97 * best) {
       best = cost;
-      best_n = n;
+      best_per = per;
     }
   }
-  return (rounds + best_n - 1) / best_n;
+  return best_per;
 }
 
 }  // namespace ssm
