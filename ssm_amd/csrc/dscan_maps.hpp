@@ -139,11 +139,11 @@ static void launch_dscan_maps(const DscanMapParams &p, hipStream_t s) {
 static int dscan_rounds_per_segment(size_t wgs, int rounds, double us, double launch, double share) {
   int best_per = rounds;
   double best = 0.0;
-  for (int per = rounds; per >= 1 && (rounds + per - 1) / per <= 32; --per) {
-    const int n = (rounds + per - 1) / per;
+  for (int most = 1; most <= 32 && most <= rounds; ++most) {          // at most so many segments, equal but for the last
+    const int per = (rounds + most - 1) / most, n = (rounds + per - 1) / per;
     const double turns = (double)((wgs * n + 255) / 256);
     const double cost = turns * (2.0 + us * per) + (n > 1 ? launch + share * us * rounds * (double)wgs / 256 : 0.0);
-    if (per == rounds || cost < 0.97 * best) {
+    if (most == 1 || cost < 0.97 * best) {
       best = cost;
       best_per = per;
     }
