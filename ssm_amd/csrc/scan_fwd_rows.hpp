@@ -144,7 +144,6 @@ void scan_fwd_rows_kernel(const ScanFwdParams p) {
       float dl[K], du[K], y[K];
       {
         const float bias = p.bias ? p.bias[d] : 0.0f, Dk = p.Dk ? p.Dk[d] : 0.0f;
-        const float D_lo = sub ? 0.0f : Dk, D_hi = sub ? Dk : 0.0f;
         float v[KO];
         if (tail) {
           row_end(t0 + lane_t, L, ur);
@@ -163,8 +162,8 @@ void scan_fwd_rows_kernel(const ScanFwdParams p) {
 #pragma unroll
         for (int i = 0; i < KO; ++i) {
           const float uu = to_f32(ur.v[i]);
-          y[i] = D_lo * uu;              // counted once, by the half that owns the step
-          y[KO + i] = D_hi * uu;
+          y[i] = sub ? 0.0f : Dk * uu;   // counted once, by the half that owns the step: picked, since 0 * u is NaN where u is not
+          y[KO + i] = sub ? Dk * uu : 0.0f;   // finite, and would reach the other half's step, eight earlier or later
           both_halves(v[i], dl[i], dl[KO + i]);
           both_halves(v[i] * uu, du[i], du[KO + i]);
         }
@@ -232,6 +231,14 @@ void scan_fwd_rows_kernel(const ScanFwdParams p) {
       }
       Pack<io_t, KO> zr;
       if (p.z) zr = row_run<io_t, KO>(Z + row * L, t0 + lane_t, L);
+      if (N % 2) {                       // the half that has no such state walks zeros, whatever the row holds
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          dl[i] = n_mine + n_half > N ? 0.0f : dl[i];
+          du[i] = n_mine + n_half > N ? 0.0f : du[i];
+        }
+        dsum = n_mine + n_half > N ? 0.0f : dsum;
+      }
       process(n_half - 1);
 
       float o[KO];

@@ -146,3 +146,24 @@ def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype
     for a, b, what in ((y[:, pick], yr, "y"), (h[:, pick], hr, "last state")):
         scale = float(b.abs().max())
         torch.testing.assert_close(a.double().cpu(), b, rtol=tol["rtol"], atol=tol["atol"] * scale, msg=lambda m: f"{what}: {m}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("length,nstate", [(403, 1), (403, 15), (403, 16), (1031, 3), (200, 9), (200, 16)])
+def test_an_infinite_step_stays_where_it_is(length, nstate, dtype):
+    """An infinite u reaches the outputs from its own step on, as an infinity where nothing cancels it; the steps ahead of it,
+    those in the same lane's run among them, are what they were."""
+    from ssm_amd import ops
+    inp = make_inputs(length, 2, 24 if length < 1031 else 520, length, nstate, dtype=dtype, groups=1)
+    t = {k: v.cuda() for k, v in inp.items()}
+    for k in ("B", "C", "D"):
+        t[k] = t[k].abs() + 0.1
+    call = lambda: ops.selective_scan(*(t[k] for k in NAMES[:5]), D=t["D"], dt_bias=t["dt_bias"], softplus=True)
+    clean = call()
+    rows = torch.arange(t["u"].shape[1], device="cuda")
+    at = 100 + rows % 24                                    # every place in a run of 16
+    t["u"][:, rows, at] = float("inf")
+    y = call()
+    ahead = (torch.arange(length, device="cuda") < at[:, None]).expand_as(y)
+    assert torch.equal(y[ahead], clean[ahead])
+    assert (y[:, rows, at] == float("inf")).all()
