@@ -209,7 +209,7 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, 
         if (sliced) {
           float left[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) left[j] = v[j] - (float)(elem_t)v[j];
+          for (int j = 0; j < 4; ++j) left[j] = fabsf(v[j]) < 3.3e38f ? v[j] - (float)(elem_t)v[j] : 0.0f;     // (inf - inf)
           store4_e<elem_t>(Ls + at, left);
         }
       }
