@@ -3,13 +3,11 @@
 //   states  dy = dout silu(z), rounded and kept; what each chunk adds to the adjoint state
 //   carry   the adjoint state leaving each chunk, last to first, and what of <G, H> goes through each chunk
 //   scans   y again for dz and its row sums;  u for dx and its row sums
-//   dbc     dB and dC, every head of a group (or of a slice of one) in one workgroup; and in the same launch
+//   dbc     dB and dC, every head of a group in one workgroup; and in the same launch
 //   dt      the chain behind ddt, and the partial sums of dA, dD and the bias; one more launch adds those up
 //
 // What the forward prepared (steps, running sums, operand fragments, the states entering the chunks) is read, not formed again.
 #include "ssd_chunk.hpp"
-
-#include <algorithm>
 
 namespace ssm {
 
@@ -26,12 +24,10 @@ struct SsdDbcParams {
   const float *dA2, *dtv;
   const void *Btblk, *Ctblk;
   elem_t *dB, *dC;               // (B, L, G, N)
-  float *dB_parts, *dC_parts;    // (slices, B, L, G, N): what each slice of a group's heads adds, where there are several
   int len, heads, groups, nchunks, units;      // units = batch * nchunks * groups
-  int slices, slice_heads;
 };
 
-// A workgroup takes 64 rows of dC (or of dB) of one (batch, chunk, group) and walks its heads: the 64 own rows, all rows they
+// A workgroup takes 64 rows of dC (or of dB) of one (batch, chunk, group) and walks the heads: the 64 own rows, all rows they
 // meet (s <= l, or l >= s) and the state of the next head are on their way from L2 to registers while those of this head, in
 // LDS, are multiplied (one barrier per head).  Wave w has the own tile w & 1 and, of the tiles it meets, every eighth (every
 // fourth in shorter chunks); M stays in its accumulators, in float32, over all heads and is rounded once, for the product
@@ -60,14 +56,12 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, 
   const int wave = wave_id_uniform(), lane = lane_id(), tid = (int)threadIdx.x;
   const int m = lane & 31, g2 = lane >> 5, ot = wave & 1, mw = wave >> 1;
   // the workgroups that meet the most rows start first
-  const unsigned same = 2u * p.units * p.slices;
-  const unsigned rank = block / same, rest = block % same;
-  const unsigned unit = (rest >> 1) % p.units, slice = (rest >> 1) / p.units;
+  const unsigned rank = block / (2u * p.units), rest = block % (2u * p.units);
+  const unsigned unit = rest >> 1;
   const int r = for_b ? (int)rank : NR - 1 - (int)rank;
   const int meets = (int)(NR - rank);                                  // blocks of 64 rows
   const int g = (int)(unit % p.groups), bc = (int)(unit / p.groups), c = bc % p.nchunks, b = bc / p.nchunks;
-  const int of_group = p.heads / p.groups, first = (int)slice * p.slice_heads;
-  const int per = min(p.slice_heads, of_group - first), h0 = g * of_group + first;
+  const int per = p.heads / p.groups, h0 = g * per;
   const int rows = min(Q, p.len - c * Q);
   if (64 * r >= rows) return;
   const size_t pitch = (size_t)p.heads * SSD_P;
@@ -193,10 +187,8 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, 
     if (h + 1 < per) put(at ^ 1);
     __syncthreads();
   }
-  // ---- M, rounded, as an operand (rows = own, columns = met), times the columns of B (of C); a slice's M with what rounding
-  // took from it as a second operand, so that more roundings of parts do not come to more than the one of the sum
-  elem_t *Ms = bufs, *Ls = bufs + 64 * Q;                              // [64][Q]
-  const bool sliced = p.slices > 1;
+  // ---- M, rounded, as an operand (rows = own, columns = met), times the columns of B (of C)
+  elem_t *Ms = bufs;                                                   // [64][Q]
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int t = mw + MW * i, row = 32 * ot + m;
@@ -204,14 +196,7 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, 
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float v[4] = {M[i][4 * q], M[i][4 * q + 1], M[i][4 * q + 2], M[i][4 * q + 3]};
-        const int at = row * Q + (((4 * t + q) ^ (row & QMASK)) << 3) + 4 * g2;
-        store4_e<elem_t>(Ms + at, v);
-        if (sliced) {
-          float left[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) left[j] = fabsf(v[j]) < 3.3e38f ? v[j] - (float)(elem_t)v[j] : 0.0f;     // (inf - inf)
-          store4_e<elem_t>(Ls + at, left);
-        }
+        store4_e<elem_t>(Ms + row * Q + (((4 * t + q) ^ (row & QMASK)) << 3) + 4 * g2, v);
       }
     }
   }
@@ -219,19 +204,16 @@ __device__ __forceinline__ void dbc_rows(const SsdDbcParams &p, unsigned block, 
   if (mw >= NT) return;
   const elem_t *bt = reinterpret_cast<const elem_t *>(for_b ? p.Ctblk : p.Btblk) + (((size_t)unit * KS + (met0 >> 4)) * NT + mw) * SSD_FRAG + lane * 8;
   for (int ks = 0; ks < 4 * meets; ++ks) {
-    const int row = 32 * ot + m, at = row * Q + (((2 * ks + g2) ^ (row & QMASK)) << 3);
-    const v8 f = load_frag_e<elem_t>(bt + ks * NT * SSD_FRAG);
-    out = mma(f, load_frag_e<elem_t>(Ms + at), out);
-    if (sliced) out = mma(f, load_frag_e<elem_t>(Ls + at), out);
+    const int row = 32 * ot + m;
+    out = mma(load_frag_e<elem_t>(bt + ks * NT * SSD_FRAG),
+              load_frag_e<elem_t>(Ms + row * Q + (((2 * ks + g2) ^ (row & QMASK)) << 3)), out);
   }
   if (own_row < rows) {
-    const size_t row = (size_t)b * p.len + (size_t)c * Q + own_row, dst = (row * p.groups + g) * N + 32 * mw + 4 * g2;
-    float *part = (for_b ? p.dB_parts : p.dC_parts) + (size_t)slice * ((size_t)p.units / p.nchunks * p.len * N) + dst;
+    elem_t *dst = (for_b ? p.dB : p.dC) + (((size_t)b * p.len + (size_t)c * Q + own_row) * p.groups + g) * N + 32 * mw + 4 * g2;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float v[4] = {out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
-      if (sliced) *reinterpret_cast<float4 *>(part + 8 * q) = make_float4(v[0], v[1], v[2], v[3]);
-      else store4_e<elem_t>((for_b ? p.dB : p.dC) + dst + 8 * q, v);
+      store4_e<elem_t>(dst + 8 * q, v);
     }
   }
 }
@@ -320,7 +302,7 @@ __device__ __forceinline__ void dt_rows(const SsdDtParams &p, unsigned block, un
 
 // Both in one launch: the workgroups of dt, of which there are few and short ones, start first, and those of dbc that meet the fewest rows
 // wait for their CUs.  At 4 x 2048 steps, 24 heads, 128 states, chunks of 256 52.6 us, in two launches 51.7 and 7.1; 2 x 2048, 48 heads, 64
-// states 43.3, so 43.1 and 7.0; 3 x 896, 18 heads 27.7, so 26.8 and 5.2.
+// states 43.3, so 43.1 and 7.0.
 template <int Q> constexpr unsigned dt_blocks(const SsdDims &d) {
   return (unsigned)(d.batch * d.nchunks * ((d.heads + DBC_WAVES<Q> - 1) / DBC_WAVES<Q>));
 }
@@ -336,23 +318,8 @@ __global__ __launch_bounds__(64 * DBC_WAVES<Q>) void ssd_dbc_dt_kernel(const Ssd
 // ---------------------------------------------------------------------- host
 
 struct BwdLayout {
-  size_t dy, added, states, turned, h_turned, s2, xu, s1, through, carried, dA, dbias, dD, dB_parts, dC_parts, total;
+  size_t dy, added, states, turned, h_turned, s2, xu, s1, through, carried, dA, dbias, dD, total;
 };
-
-// How the heads of a group are divided among workgroups of dbc: one to a CU is what fits, and a call whose (chunk, group) pairs do
-// not fill the 256 takes as many slices as do.  A slice's rows of dB and dC leave in float32 and the launch of sums adds
-// them up.  At 1 x 569 steps, 62 heads, 64 states, chunks of 256 the kernel takes 16.5 us, so 96.5 with all heads in one
-// workgroup; 3 x 320, 42 heads, 128 states 28.5 and 74.6; 1 x 1635, 76 heads, chunks of 128 34 and 111; 1 x 3456, 34 heads 35.5
-// and 61.  Slices for two rounds of workgroups (384, 512, 768 of them) were 0 to 60 % slower than for one at all of these, and
-// at 4 x 2048, 24 heads, which fills the chip undivided.  Over 24 calls dB and dC of divided groups are off from float64 by
-// 0.0017 of their 2-norm, undivided by 0.0024; by 0.0024 too without the second operand.
-struct DbcCut { int slices, heads; };
-static DbcCut dbc_cut(const SsdDims &d) {
-  const int per = d.heads / d.groups;
-  const size_t workgroups = (size_t)2 * d.batch * d.groups * ((d.len + 63) / 64);
-  const int want = (int)std::max<size_t>(1, 256 / workgroups), heads = (per + want - 1) / want;
-  return {(per + heads - 1) / heads, heads};
-}
 
 static BwdLayout bwd_layout(const SsdDims &d) {
   BwdLayout f;
@@ -372,10 +339,6 @@ static BwdLayout bwd_layout(const SsdDims &d) {
   f.dA = take(units * 4);
   f.dbias = take(units * 4);
   f.dD = take(units * 4);
-  const DbcCut cut = dbc_cut(d);
-  const size_t parts = cut.slices > 1 ? (size_t)cut.slices * d.batch * d.len * d.groups * d.nstate * 4 : 0;
-  f.dB_parts = take(parts);
-  f.dC_parts = take(parts);
   f.total = at;
   return f;
 }
@@ -410,7 +373,7 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
   const dim3 both(2 * units.x);
   if (dz.z) hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, true>), both, block, 0, s, dz, dx);
   else hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, false>), both, block, 0, s, dz, dx);
-  const unsigned first = dt_blocks<Q>(d), all = first + 2u * bc.units * bc.slices * (Q / 64);
+  const unsigned first = dt_blocks<Q>(d), all = first + 2u * bc.units * (Q / 64);
   hipLaunchKernelGGL((ssd_dbc_dt_kernel<Q, N>), dim3(all), dim3(64 * DBC_WAVES<Q>), dbc_lds, s, bc, dt, first);
   return SSM_OK;
 }
@@ -469,8 +432,6 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   bc.dA2 = dA2; bc.dtv = dtv; bc.Btblk = kw + kept.Btblk; bc.Ctblk = kw + kept.Ctblk;
   bc.dB = reinterpret_cast<elem_t *>(a->dB); bc.dC = reinterpret_cast<elem_t *>(a->dC);
   bc.len = d.len; bc.heads = d.heads; bc.groups = d.groups; bc.nchunks = d.nchunks; bc.units = d.batch * d.nchunks * d.groups;
-  const DbcCut cut = dbc_cut(d);
-  bc.slices = cut.slices; bc.slice_heads = cut.heads; bc.dB_parts = f32(lay.dB_parts); bc.dC_parts = f32(lay.dC_parts);
   SsdDtParams dt{};
   dt.s2 = f32(lay.s2); dt.xu = f32(lay.xu); dt.s1 = f32(lay.s1); dt.dtv = dtv; dt.through = f32(lay.through); dt.carried = f32(lay.carried); dt.dt_raw = f.dt;
   dt.A = f.A; dt.bias = f.dt_bias; dt.ddt = a->ddt; dt.dA = f32(lay.dA); dt.dbias = f32(lay.dbias);
@@ -489,11 +450,6 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   jobs.add(f32(lay.dA), a->dA, 1, parts, (size_t)d.heads, SSM_F32);
   if (a->ddt_bias) jobs.add(f32(lay.dbias), a->ddt_bias, 1, parts, (size_t)d.heads, SSM_F32);
   if (a->dD && f.Dskip) jobs.add(f32(lay.dD), a->dD, 1, parts, (size_t)d.heads, SSM_F32);
-  if (cut.slices > 1) {
-    const size_t inner = (size_t)d.batch * d.len * d.groups * d.nstate;
-    jobs.add(f32(lay.dB_parts), a->dB, 1, cut.slices, inner, SSM_BF16);
-    jobs.add(f32(lay.dC_parts), a->dC, 1, cut.slices, inner, SSM_BF16);
-  }
   launch_fold_jobs(jobs, s);
   SSM_CHECK_LAUNCH("ssm_ssd_combined_bwd");
   return SSM_OK;
