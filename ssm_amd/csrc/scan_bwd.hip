@@ -804,16 +804,42 @@ void launch_fold_sum(const float *in, float *out, size_t outer, int count, size_
   hipLaunchKernelGGL(fold_sum_kernel, dim3(fold_grid(outer * inner)), dim3(256), 0, s, in, out, outer, count, inner);
 }
 
-constexpr int BF_MAX_ROWS = 96;          // channels a workgroup of the wave-per-row kernel (scan_bwd_fast.hpp) takes at most
+// The wave-per-row kernel (scan_bwd_fast.hpp): waves of a workgroup, each with a row at a time, and the channels it takes at most.
+constexpr int BF_WAVES = 16, BF_MAX_ROWS = 96;
 
 // How a call is cut into work, from its sizes alone (the workspace is sized before the tensors are known).
 struct BwdPlan {
   int rows_per_wg, nblk;                 // general kernel
   enum { GENERAL, GROUPED, OWN, CONSTANT } route;   // the kernel for whose shape the call has, types permitting
+  int order;                             // GROUPED: neighbouring channels whose sums over the states begin with the same state
   int span, fast_rows, fast_nblk;        // GROUPED: channels that share B and C, those of them to a workgroup, workgroups per batch row
   int nsplit;                            // chunks that may run side by side (1: a unit walks all of them)
   size_t off_dA, off_dD, off_dbias, off_q, off_dB, off_dC, total;   // byte offsets into the workspace
 };
+
+// BwdPlan::order of a call.  Any would do, but a training step repeats to the bit only where it stays: single roundings of
+// du to 16 bits, and behind them 3e-5 of a convolution's float32 weight gradient, change with it.  So it is what it was when a
+// workgroup was 16, 32 or 48 whole rows of a span: the cheapest of these, us that a chunk took a workgroup on few of the
+// CUs and how much more on all of them.
+static int bwd_order(double rows, int span, int nchunks, bool may_split) {
+  const double alone[3] = {29.0, 53.0, 77.0}, crowd[3] = {9.0, 11.6, 15.0}, maps = 12.0 + 0.5 * rows * nchunks / 256;
+  int order = 1;
+  double best = 0.0;
+  for (int k = 3; k >= 1; --k) {
+    if (span % (16 * k)) continue;
+    const auto time = [&](double units) {
+      const double full = (double)(long)(units / 256), rest = units - full * 256;
+      return full * (alone[k - 1] + crowd[k - 1]) + (rest > 0.0 ? alone[k - 1] + crowd[k - 1] * rest / 256 : 0.0);
+    };
+    const double units = rows / (16 * k), in_turn = time(units) * nchunks, side = time(units * nchunks) + maps;
+    const double cost = may_split && side < in_turn ? side : in_turn;
+    if (best == 0.0 || cost < best) {
+      best = cost;
+      order = k;
+    }
+  }
+  return order;
+}
 
 static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int c_kind, int b_groups,
                         int c_groups, bool own_split = true, bool in_turn = false) {
@@ -849,10 +875,11 @@ static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int
     if (own_split && may_split && all <= 1024) pl.nsplit = nchunks;
   } else if (bv && cv && span >= 8 && len >= 8 && len < (1 << 28)) {
     pl.route = BwdPlan::GROUPED;
-    // A chunk takes a workgroup 8 us, 25.5 for every sixteen rows and 12, 17, 21 or 25.5 for the last four, eight, twelve or
-    // sixteen; its start 5 (bf16, us a chunk measured / so: 9 rows 26 / 29, 14 30.5 / 33.5, 16 32.5 / 33.5, 18 44 / 45.5, 48 87 / 84.5,
+    // A chunk takes a workgroup 8 us and a turn 12, 17, 21 or 25.5 with a row to four, eight, twelve or all sixteen waves; its
+    // start 5 (bf16, us a chunk measured / so: 9 rows 26 / 29, 14 30.5 / 33.5, 16 32.5 / 33.5, 18 44 / 45.5, 48 87 / 84.5,
     // 64 rows a chunk each 118 / 115).  Every workgroup leaves a partial sum of dB and dC, which the fold reads.
-    const int units = batch * (dim / span);
+    pl.order = bwd_order(all, span, nchunks, may_split);
+    const int units = batch * (dim / span), step = 4 * pl.order, period = BF_WAVES * pl.order;
     const double part[5] = {0.0, 12.0, 17.0, 21.0, 25.5};
     double best = 0.0;
     for (int side = 0; side < (may_split ? 2 : 1); ++side) {
@@ -861,11 +888,12 @@ static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int
       for (size_t k = least; k < least + 4; ++k) {
         const size_t blocks = k * 256 / pieces;
         int rows = blocks <= 1 ? span : (int)((span + blocks - 1) / blocks);
-        rows = rows < 8 ? 8 : (rows + 3) / 4 * 4;          // rows that cost nothing
+        rows = ((rows < 8 ? 8 : rows) + step - 1) / step * step;          // rows that cost nothing
         if (rows > span) rows = span;
         if (rows > BF_MAX_ROWS) continue;
         const size_t count = (span + rows - 1) / rows;
-        const double chunk = 8.0 + 25.5 * (rows / 16) + part[(rows % 16 + 3) / 4];
+        const int last = (rows % period + pl.order - 1) / pl.order;       // waves with a row in the last turns
+        const double chunk = 8.0 + pl.order * (25.5 * (rows / period) + part[(last + 3) / 4]);
         const double rounds = (double)((pieces * count + 255) / 256);
         double cost = rounds * (5.0 + (side ? chunk : chunk * nchunks)) + (side ? maps : 0.0) + 8.0 * units * count * nstate * len / 4.5e6;
         if (side) cost *= 1.06;            // (where both come out alike: in turn)
@@ -1086,9 +1114,9 @@ extern "C" int ssm_scan_bwd(const ssm_scan_bwd_args *a, void *hip_stream) {
   } else if (route == BwdPlan::GROUPED) {
     p.rows_per_wg = pl.fast_rows;
     p.nblk = pl.fast_nblk;
-    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, s);
-    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, s) : launch_bwd_fast<bf16_t, bf16_t>(p, s);
-    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, s) : launch_bwd_fast<f16_t, f16_t>(p, s);
+    if (a->io_dtype == SSM_F32) rc = launch_bwd_fast<float, float>(p, pl.order, s);
+    else if (a->io_dtype == SSM_BF16) rc = bc32 ? launch_bwd_fast<bf16_t, float>(p, pl.order, s) : launch_bwd_fast<bf16_t, bf16_t>(p, pl.order, s);
+    else rc = bc32 ? launch_bwd_fast<f16_t, float>(p, pl.order, s) : launch_bwd_fast<f16_t, f16_t>(p, pl.order, s);
   } else {
     switch (a->io_dtype) {
       case SSM_F32: rc = launch_bwd<float>(p, s); break;

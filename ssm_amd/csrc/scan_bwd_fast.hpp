@@ -10,7 +10,7 @@
 // sums over states (pre-activation, <gh, B>, the A-term of d delta) never leaves the lane's
 // registers; what sums over the channels of a group (dB, dC) is added into an LDS tile by the
 // 16 wavefronts of the workgroup, which are kept on 16 different states by a skew: wave w works
-// on state (w + slot) mod 16, so a state's part of the tile passes from wave w + 1 to wave w from
+// on state (first + w + slot) mod 16, so a state's part of the tile passes from wave w + 1 to wave w from
 // one slot to the next.  A wave counts its finished slots in LDS and, before it touches the tile
 // (a plain read, add, write at the very end of the slot), waits for the count of the wave it
 // takes over from; the rest of a slot needs no agreement between waves, which may drift apart by
@@ -24,7 +24,6 @@
 
 namespace ssm {
 
-constexpr int BF_WAVES = 16;
 constexpr int BF_THREADS = WAVE * BF_WAVES;
 constexpr int BF_K = 8;
 constexpr int BF_DEP = 1;             // wave w takes a state over from wave w + BF_DEP (-1 measured 2 % slower)
@@ -62,7 +61,7 @@ __device__ __forceinline__ void touch_lines(const void *at, unsigned lds_at) {
 
 // A workgroup walks all chunks of its rows, last to first, or (p.maps: the maps of the chunks are known) one of
 // them; blockIdx then counts chunks fastest, and the per-row sums are left per chunk.
-template <typename io_t, typename bc_t, bool HAS_Z>
+template <typename io_t, typename bc_t, bool HAS_Z, int ORDER>
 __global__ __launch_bounds__(BF_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void scan_bwd_fast_kernel(const ScanBwdParams p) {
   constexpr int K = BF_K, T = FAST_T, NS = FAST_N;
@@ -88,7 +87,12 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
   const int b = unit / p.nblk, blk = unit % p.nblk;
   const int per_span = (p.span + R - 1) / R, in_span = blk % per_span * R;
   const int d_first = blk / per_span * p.span + in_span, count = min(R, p.span - in_span);
-  const int turns = (count + BF_WAVES - 1) / BF_WAVES;
+  // A wave takes ORDER neighbouring rows one after the other, then those 16 sets of neighbours further on.  A row's sums over the
+  // states (ghB, At, pre) begin with the state that its wave begins with, and single roundings of du follow from that: it is
+  // named by the channel's place in its span, however a call is cut into workgroups (of whole sets each).
+  const int first_state = (wave + in_span / ORDER) & (NS - 1);
+  const int turns = (count + BF_WAVES * ORDER - 1) / (BF_WAVES * ORDER) * ORDER;
+  constexpr int FURTHER = (BF_WAVES - 1) * ORDER;
   const int rev_lane = WAVE - 1 - lane;
   const bc_t *Bg = reinterpret_cast<const bc_t *>(p.Bp) + ((size_t)b * p.b_groups + d_first / (p.dim / p.b_groups)) * N * L;
   const bc_t *Cg = reinterpret_cast<const bc_t *>(p.Cp) + ((size_t)b * p.c_groups + d_first / (p.dim / p.c_groups)) * N * L;
@@ -112,8 +116,8 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     row_end(t, L, gr);
     if (HAS_Z) row_end(t, L, zr);
   };
-  if (wave < count) fetch(wave, c_last);
-  for (int r = wave; r < count; r += BF_WAVES) {
+  if (wave * ORDER < count) fetch(wave * ORDER, c_last);
+  for (int r = wave * ORDER, j = 0; r < count; r += ++j % ORDER ? 1 : FURTHER + 1) {
     const int d = d_first + r;
     const size_t row = (size_t)b * p.dim + d;
     if (lane < NS) {
@@ -154,12 +158,17 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     __syncthreads();
 
 #pragma nounroll
-    for (int turn = 0; turn < turns; ++turn) {
-      const int r = turn * BF_WAVES + wave, d = d_first + r;
+    for (int turn = 0, r = wave * ORDER, j = 0, r_after; turn < turns; ++turn, r = r_after) {
+      r_after = r + 1;
+      if (++j == ORDER) {
+        r_after += FURTHER;
+        j = 0;
+      }
+      const int d = d_first + r;
       if (r >= count) {                    // no row: pass the states on
         for (int slot = 0; slot < NS; ++slot) {
           if (!wait_for_slots(done + ((wave + BF_DEP) & (BF_WAVES - 1)), nslots, p.spin_limit)) {
-            const int n = (BF_DEP * wave + slot) & (NS - 1);
+            const int n = (first_state + slot) & (NS - 1);
             accB[n * T + lane * 4] = accC[n * T + lane * 4] = __builtin_nanf("");
           }
           ++nslots;
@@ -170,8 +179,8 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
       }
       const size_t row = (size_t)b * p.dim + d;
       const size_t at = row * L;
-      const bool again = r + BF_WAVES < count;
-      const int r_next = again ? r + BF_WAVES : wave, c_next = again ? c : c - 1;       // the wave's next row and chunk
+      const bool again = r_after < count;
+      const int r_next = again ? r_after : wave * ORDER, c_next = again ? c : c - 1;       // the wave's next row and chunk
       const float A2_lanes = rowA2[r * NS + (lane & (NS - 1))];
       float qcarry = rowq[r * NS + (lane & (NS - 1))], dA_lanes = 0.0f;
       const float Dk = p.Dk ? p.Dk[d] : 0.0f, bias = p.bias ? p.bias[d] : 0.0f;
@@ -207,7 +216,7 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
         dsum += dl[i];
       }
       for (int slot = 0; slot < NS; ++slot) {
-        const int n = (BF_DEP * wave + slot) & (NS - 1);
+        const int n = (first_state + slot) & (NS - 1);
         if (sizeof(io_t) == 2 && slot == 1 && c_next >= c_first) {
           // (not ahead of the first slot, whose wait for the entering states would wait for these too; float32 rows are twice
           // as many lines, which the L2 does not hold for all CUs: 397 us without, 405 with)
@@ -358,7 +367,7 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
     }
   }
 
-  for (int r = wave; r < count; r += BF_WAVES) {
+  for (int r = wave * ORDER, j = 0; r < count; r += ++j % ORDER ? 1 : FURTHER + 1) {
     const size_t row = ((size_t)(p.maps ? part : 0) * p.batch + b) * p.dim + d_first + r;
     if (lane < N) p.dA_rows[row * N + lane] = rowdA[r * NS + lane];
     if (lane == 0) {
@@ -369,10 +378,12 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
 }
 
 template <typename io_t, typename bc_t>
-static int launch_bwd_fast(const ScanBwdParams &p, hipStream_t s) {
+static int launch_bwd_fast(const ScanBwdParams &p, int order, hipStream_t s) {
   const size_t ldsb = ((size_t)4 * FAST_N * FAST_T + BF_THREADS + (size_t)p.rows_per_wg * (3 * FAST_N + 2) + BF_WAVES) * sizeof(float);
   const unsigned grid = (unsigned)((size_t)p.batch * p.nblk * (p.maps ? (p.len + FAST_T - 1) / FAST_T : 1));
-  auto kernel = p.z ? scan_bwd_fast_kernel<io_t, bc_t, true> : scan_bwd_fast_kernel<io_t, bc_t, false>;
+  auto kernel = order == 1 ? (p.z ? scan_bwd_fast_kernel<io_t, bc_t, true, 1> : scan_bwd_fast_kernel<io_t, bc_t, false, 1>)
+              : order == 2 ? (p.z ? scan_bwd_fast_kernel<io_t, bc_t, true, 2> : scan_bwd_fast_kernel<io_t, bc_t, false, 2>)
+                           : (p.z ? scan_bwd_fast_kernel<io_t, bc_t, true, 3> : scan_bwd_fast_kernel<io_t, bc_t, false, 3>);
   if (allow_dynamic_lds(kernel, ldsb) != hipSuccess) {
     (void)hipGetLastError();
     set_error("ssm_scan_bwd: cannot reserve %zu bytes of LDS", ldsb);

@@ -404,6 +404,32 @@ def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype
         torch.testing.assert_close(f, r, **tol, msg=lambda m, k=k: f"grad {k}: {m}")
 
 
+@pytest.mark.parametrize("batch,dim,length,groups,neighbours", [
+    (8, 1536, 64, 1, 3), (8, 1536, 2048, 1, 3), (5, 928, 1472, 1, 2), (7, 1248, 139, 1, 3), (6, 1600, 1541, 1, 2),
+    (2, 752, 204, 1, 1), (3, 912, 3072, 1, 1), (4, 192, 520, 4, 1), (8, 616, 131, 1, 1)])
+def test_the_state_a_sum_begins_with(batch, dim, length, groups, neighbours):
+    """A channel's sums over the states begin with a state that its place among the channels of its group names, and with
+    no other: neighbours share one, the next neighbours begin with the next.  At the last step du is the sum of B alone, of
+    which two large terms take what comes between them: exact float32 numbers that differ from start to start."""
+    values = torch.tensor([2.0 ** 30] + [2.0 ** k for k in range(7)] + [-2.0 ** 30] + [3.0 * 2.0 ** k for k in range(7)])
+    B, C = (torch.zeros(batch, groups, 16, length, device="cuda") for _ in range(2))
+    B[..., -1], C[..., -1] = values.cuda(), 1.0
+    u = torch.zeros(batch, dim, length, device="cuda", requires_grad=True)
+    go = torch.zeros(batch, dim, length, device="cuda")
+    go[..., -1] = 1.0
+    y = _ops().selective_scan(u, torch.ones_like(go), torch.full((dim, 16), -1.0, device="cuda"), B, C)
+    du = torch.autograd.grad(y, u, go)[0][..., -1].cpu()
+    sums = []
+    for start in range(16):
+        acc = torch.zeros(())
+        for k in range(16):
+            acc = acc + values[(start + k) % 16]
+        sums.append(float(acc))
+    assert len(set(sums)) == 16
+    want = torch.tensor([sums[d % (dim // groups) % (16 * neighbours) // neighbours] for d in range(dim)])
+    assert torch.equal(du, want.expand(batch, dim))
+
+
 def test_a_wave_that_gives_up_its_wait_poisons_dB_and_dC():
     """The wave-per-row kernel bounds its wait for the neighbouring wave's slot count; a wave that gives up
     writes NaN into its sums so that the caller cannot take them for gradients.  The test-hooks build cuts the
