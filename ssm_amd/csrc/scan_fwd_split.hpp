@@ -61,18 +61,23 @@ void scan_fwd_split_kernel(const ScanFwdParams p) {
     const int c = c0 + wave;                                 // beyond the end: a wave of identity maps
     const int t = c * T + lane * K;
     const bool tail = (c + 1) * T > L;
+    // A run's 32-bit offset counts from the chunk's first step, or from the row's last run where the chunk lies beyond the end.
+    const int origin = RAGGED ? min(c * T, L - K) : 0;
+    const auto run_of = [&](const auto *row) {
+      return lane_run<RAGGED, std::remove_const_t<std::remove_pointer_t<decltype(row)>>, K>(row + origin, t - origin, L - origin);
+    };
     Pack<bc_t, K> braw[2], craw[2];
     auto fetch = [&](int n) {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
         const size_t at = (size_t)min(n + w, N - 1) * L;
-        braw[w] = lane_run<RAGGED, bc_t, K>(Bg + at, t, L);
-        craw[w] = lane_run<RAGGED, bc_t, K>(Cg + at, t, L);
+        braw[w] = run_of(Bg + at);
+        craw[w] = run_of(Cg + at);
       }
     };
     if constexpr (!CONST_BC) fetch(0);
-    Pack<io_t, K> ur = lane_run<RAGGED, io_t, K>(U, t, L), dr = lane_run<RAGGED, io_t, K>(DT, t, L), zr;
-    if (p.z) zr = lane_run<RAGGED, io_t, K>(Z, t, L);
+    Pack<io_t, K> ur = run_of(U), dr = run_of(DT), zr;
+    if (p.z) zr = run_of(Z);
     if (RAGGED && tail) {
       row_end(t, L, ur);
       row_end(t, L, dr);

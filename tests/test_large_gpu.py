@@ -178,3 +178,27 @@ def test_ssd_combined_beyond_2_31_elements():
         # at the usual level; a wrapped address gives errors of the order of the values themselves everywhere
         half_close(y[:, :, h0:h0 + 2].cpu(), ys.cpu(), what=f"y heads {h0}..", atol_rms=0.3)
         half_close(final[:, h0:h0 + 2].cpu(), fs.cpu(), what=f"final states heads {h0}..", atol_rms=0.3)
+
+
+@pytest.mark.parametrize("varying", [False, True])
+def test_one_row_of_more_than_2_32_bytes(varying):
+    """Two rows of float32 whose ends lie more than 2**32 bytes behind their starts, few enough for their chunks to run side by
+    side.  The state forgets within tens of steps (it falls by e^-1 and e^-2 at each), so from 300 steps before 2**30 on the
+    outputs are those of a call that begins 724 steps earlier, a whole number of chunks into the row, up to the rounding of
+    sums of float32."""
+    ops = _ops()
+    dim, length, cut = 2, 2 ** 30 + 4 * 512 + 5, 2 ** 30 - 1024
+    g = _gen(3)
+    u = torch.empty(1, dim, length, device="cuda").normal_(generator=g)
+    delta = torch.empty(1, dim, length, device="cuda").fill_(1.0)
+    A = -torch.tensor([[1.0, 2.0]], device="cuda").repeat(dim, 1)
+    if varying:
+        B, C = (torch.empty(1, 1, 2, length, device="cuda").normal_(generator=g) for _ in range(2))
+    else:
+        B, C = (torch.randn(dim, 2, generator=g, device="cuda") for _ in range(2))
+    y, last = ops.selective_scan(u, delta, A, B, C, return_last_state=True)
+    part = lambda t: t[..., cut:].contiguous()
+    ys, lasts = ops.selective_scan(part(u), part(delta), A, part(B) if varying else B, part(C) if varying else C,
+                                   return_last_state=True)
+    torch.testing.assert_close(y[..., cut + 724:], ys[..., 724:], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(last, lasts, rtol=1e-5, atol=1e-5)
