@@ -251,6 +251,22 @@ def test_shipped_library_has_no_test_hooks_and_the_hooks_build_does():
     assert L.load() is lib
 
 
+@pytest.mark.parametrize("selector", [111120, 113082, 111162])
+def test_a_selector_is_refused_rows_that_its_kernel_cannot_read(selector):
+    """The kernel for any number of channels to a workgroup reads four steps of a row at a time, from 32-bit offsets: a selector
+    of the test-hooks build that asks for it with rows shorter or longer than that is refused before anything is launched."""
+    L = _lib()
+    hooks = L.load_test_hooks()
+    buf = (ctypes.c_float * 64)()
+    p = ctypes.addressof(buf)
+    p += (-p) % 16
+    for length in (1, 3, 1 << 28):
+        a = L.ScanFwdArgs(u=p, delta=p, A=p, Bproj=p, Cproj=p, out=p, batch=1, dim=24, seqlen=length, nstate=2, b_kind=2, c_kind=2,
+                          b_groups=1, c_groups=1, reserved=selector)
+        assert hooks.ssm_scan_fwd(ctypes.byref(a), None) in (-2, -4), length
+        assert b"selector" in hooks.ssm_amd_last_error()
+
+
 def test_without_the_host_module_calls_take_the_long_way(tmp_path):
     """``_host.so`` saves host time only: where it cannot be loaded a warning says so, it answers every form with None, and
     the library is bound and used without it."""
