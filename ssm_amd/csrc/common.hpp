@@ -366,11 +366,22 @@ __device__ __forceinline__ float wave_read_lane(float v, int lane) {
 
 // Sum over the 64 lanes, result valid in every lane (uniform).  Six DPP additions (a running
 // sum inside each row of 16, then the row totals passed on: lane 63 ends with everything) and
-// one read of lane 63: no trip through the LDS crossbar as with shuffles.  Written out: lanes whose source does not exist,
-// or whose row is masked off, keep their value, where the compiler moves a zero in first (ten instructions).
+// one read of lane 63: no trip through the LDS crossbar as with shuffles.  Neighbouring sums fill each other's waits.
 __device__ __forceinline__ float wave_sum(float v) {
-  asm volatile(
-      "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+  v += dpp_move<DPP_ROW_SHR1, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR2, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR4, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_SHR8, 0xf>(0.0f, v);
+  v += dpp_move<DPP_ROW_BCAST15, 0xa>(0.0f, v);
+  v += dpp_move<DPP_ROW_BCAST31, 0xc>(0.0f, v);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
+}
+// The same sum where it stands alone, with other waves to fill its waits: lanes whose source does not exist, or whose row is
+// masked off, keep their value, where the compiler moves a zero in first (ten instructions for six, and a wait of two cycles in
+// front of each either way).  One per state of the grouped scan's backward: 0.5 % of 161 training calls; three side by side, as
+// where projections are constant in time, took 4 % more of such a call than the form above (1 x 793 x 3292 117 us, so 112).
+__device__ __forceinline__ float wave_sum_alone(float v) {
+  asm("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
       "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
       "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
       "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"

@@ -287,7 +287,7 @@ void scan_bwd_fast_kernel(const ScanBwdParams p) {
             At[i] = __builtin_fmaf(qh, A2, At[i]);
             sA = __builtin_fmaf(qh, dl[i], sA);
           }
-          const float tot = wave_sum(sA);
+          const float tot = wave_sum_alone(sA);
           dA_lanes += lane == n ? tot : 0.0f;
           // The skew gives this wave the state's part of both tiles to itself for the slot (plain read, add,
           // write), once the wave that had it in the slot before is through with it.
