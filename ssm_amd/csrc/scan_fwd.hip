@@ -148,20 +148,25 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
     int pick = 0;
     // (rows of at most 256 steps and few states: the general kernel, 3 x 1024 x 64 bf16 with 5 states 7.2 us against 8.5)
     if (p.span >= ROWS_MIN && a->seqlen >= 4 && a->seqlen < (1 << 28) && (a->seqlen > FAST_T / 2 || a->nstate > 8)) {
-      // Any number of channels to a workgroup, but where two rows to a wave at once come out even (aligned 16-bit rows, 48 channels
-      // to a workgroup on every CU in every round: 109.6 us against 111.0 at the headline shape), or where so few states leave
-      // little but the reads, for which more waves do better (aligned, 8 x 1536 x 2048, at most 8 states: bf16 42 to 75 us
-      // against 49 to 77, float32 with 24 channels 88 to 103 against 102 to 109).
+      // Any number of channels to a workgroup, but where
+      //   few states leave little but the reads.  16-bit, aligned runs: a row to a wave, at most 9 states 0.82 of the time over 165
+      //   random calls, 10 states 0.99, 12 1.03 (float32 1.02 to 1.14).  16-bit runs of any start: workgroups of 8 channels, at most
+      //   4 states 0.91 over 44 calls of up to 4096 rows and three chunks (one state: any number of chunks), more rows 1.0.  Float32: 24
+      //   channels on every CU 88 to 103 us against 102 to 109 (8 x 1536 x 2048), or workgroups of 8 (3 x 1072 x 640, one state, 9.6 / 12.4);
+      //   two rows to a wave at once come out even (aligned 16-bit rows, 48 channels to a workgroup on every CU in every round:
+      //   109.6 us against 111.0 at the headline shape);
+      //   a single chunk would take a second turn for its last rows, or has no more than 8 on a CU: workgroups of 8 channels, two
+      //   to a CU (aligned: 2 x 1984 x 448 f16 16.3 / 19.0, 8 x 384 x 448 bf16, 12 on a CU, 15.4 / 13.9, 8 x 256 x 448 10.4 / 12.2).
       pick = p.split ? 31041 : ROWS_VARIANT;
       const int even = half ? 48 : 24;
       const size_t wgs = rows_total / even;
-      if (!p.split && whole16 && a->seqlen > FAST_T / 2 && p.span % even == 0 && wgs >= 256 &&
-          (a->nstate <= 8 || (half && wgs % 256 == 0))) pick = half ? 22123 : 12121;
-      // workgroups of 8 channels, two to a CU: for so few states (5 x 320 x 2304 f16, one state, 13.8 us against 17.5; 1648 x 1408
-      // bf16, two, 9.7 / 12.4; 3 x 1072 x 640 float32, one, 9.6 / 12.4), and where a single chunk would take a second turn for its last rows, or has no more than 8 on a
-      // CU (aligned, one chunk: 2 x 1984 x 448 f16 16.3 / 19.0, 8 x 384 x 448 bf16, 12 on a CU, 15.4 / 13.9, 8 x 256 x 448 10.4 / 12.2)
-      else if (!p.split && whole16 && a->seqlen > FAST_T / 2 && p.span % 8 == 0 &&
-               ((a->nstate <= 2 && (half || nchunks <= 4)) || (nchunks == 1 && rows_total <= 4096 && (rows_total <= 2048 || rows_total > 3072)))) pick = 11082;
+      if (!p.split && a->seqlen > FAST_T / 2) {
+        if (half && whole8 && aligned_to(a->Bproj, 16) && aligned_to(a->Cproj, 16) && a->nstate <= 9) pick = 31041;
+        else if (half && !whole8 && p.span % 8 == 0 && a->nstate <= 4 && rows_total <= 4096 && (nchunks <= 3 || a->nstate == 1)) pick = 11082;
+        else if (whole16 && p.span % even == 0 && wgs >= 256 && (half ? wgs % 256 == 0 : a->nstate <= 8)) pick = half ? 22123 : 12121;
+        else if (whole16 && p.span % 8 == 0 && ((!half && a->nstate <= 2 && nchunks <= 4) ||
+                                                (nchunks == 1 && rows_total <= 4096 && (rows_total <= 2048 || rows_total > 3072)))) pick = 11082;
+      }
     } else if (per_b % 8 == 0 && per_c % 8 == 0 && a->seqlen > 256) {
       pick = p.split ? 31041 : 11082;
     } else if (a->seqlen > 256 || (per_b == 1 && per_c == 1)) {
