@@ -119,10 +119,30 @@ __device__ __forceinline__ void store_any(T *row, int t, int len, const float (&
 
 // ---------------------------------------------------------------- forward, (B,C,L)
 
-// AL: rows start on 16-byte boundaries and are a whole number of vectors long.  Otherwise vectors are read and written at
-// their elements' own addresses, and only what crosses a row's end goes element by element: with every element an access of
-// its own, 8 x 1536 x 2047 bf16 took 60 us, 30 so (2044 steps 27); 2048 steps take 20 on that card.
-template <typename T, bool AL, int TAPS>
+// How a row is read and written.  CF_ALIGNED: rows start on 16-byte boundaries and are a whole number of vectors long.
+// CF_ANY: vectors at their elements' own addresses, and only what crosses a row's end goes element by element: with every
+// element an access of its own, 8 x 1536 x 2047 bf16 took 60 us, 30 so (2044 steps 27); 2048 steps take 20 on that card.
+// CF_ELEMENTS: an access per element, the fewer instructions in rows of less than a 16-bit vector (14 x 2720 x 2 bf16 16.9 us,
+// as CF_ANY 21.7) or a float32 wave (6 x 1836 x 6, two taps, forward and backward 18.4 / 22.3; 3 x 2168 x 218 18.1 / 19.5).
+enum { CF_ALIGNED, CF_ANY, CF_ELEMENTS };
+template <typename T>
+static int conv_cf_form(int len, bool vec_ok) {
+  constexpr int VEC = 16 / sizeof(T);
+  if (vec_ok && len % VEC == 0) return CF_ALIGNED;
+  return len < (sizeof(T) == 4 ? WAVE * VEC : VEC) ? CF_ELEMENTS : CF_ANY;
+}
+// A run of a row in the last form, zeros ahead of the row and past its end.
+template <typename T, int VEC>
+__device__ __forceinline__ void load_elements_or_zero(const T *row, int t, int len, float (&out)[VEC]) {
+  if (t >= 0) {
+    load_run<T, VEC>(row, t, len, false, out);
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) out[i] = 0.0f;
+  }
+}
+
+template <typename T, int FORM, int TAPS>
 __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cf_kernel(const ConvParams p) {
   constexpr int VEC = 16 / sizeof(T);
   const int row = blockIdx.x;                       // b * C + c
@@ -137,9 +157,12 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cf_kernel(const ConvPar
   const float bias = bias1[0];
   for (int t0 = threadIdx.x * VEC; t0 < p.len; t0 += CONV_THREADS * VEC) {
     float win[2 * VEC], prev[VEC], cur[VEC];
-    if constexpr (AL) {
+    if constexpr (FORM == CF_ALIGNED) {
       load_vec_or_zero<T, VEC>(xr, t0 - VEC, p.len, prev);
       load_vec_or_zero<T, VEC>(xr, t0, p.len, cur);
+    } else if constexpr (FORM == CF_ELEMENTS) {
+      load_elements_or_zero<T, VEC>(xr, t0 - VEC, p.len, prev);
+      load_elements_or_zero<T, VEC>(xr, t0, p.len, cur);
     } else {
       const bool tail = t0 + (WAVE - lane) * VEC > p.len;         // the same for the whole wave
       load_any_or_zero<T, VEC>(xr, t0 - VEC, p.len, tail, room, prev);
@@ -158,7 +181,8 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cf_kernel(const ConvPar
       for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[m], win[VEC + i - m], acc);
       out[i] = p.silu ? silu_f32(acc) : acc;
     }
-    if constexpr (AL) store_vec<T, VEC>(yr, t0, out);
+    if constexpr (FORM == CF_ALIGNED) store_vec<T, VEC>(yr, t0, out);
+    else if constexpr (FORM == CF_ELEMENTS) store_run<T, VEC>(yr, t0, p.len, false, out);
     else store_any<T, VEC>(yr, t0, p.len, out);
   }
 }
@@ -293,8 +317,8 @@ __global__ __launch_bounds__(CONV_CL_ROWS_THREADS) void conv_fwd_cl_rows_kernel(
 
 // --------------------------------------------------------------- backward, (B,C,L)
 
-// AL: as in the forward.  8 x 1536 x 2047 bf16 119 us with an access per element, 55 so (2044 steps 47); 2048 steps 36.
-template <typename T, bool AL, int TAPS>
+// FORM: as in the forward.  8 x 1536 x 2047 bf16 119 us with an access per element, 55 as CF_ANY (2044 steps 47); 2048 steps 36.
+template <typename T, int FORM, int TAPS>
 __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cf_kernel(const ConvParams p) {
   constexpr int VEC = 16 / sizeof(T);
   const int lane = lane_id();
@@ -320,7 +344,13 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cf_kernel(const ConvPar
   for (int t0 = threadIdx.x * VEC; t0 < p.len; t0 += CONV_THREADS * VEC) {
     // x over [t0-VEC, t0+2*VEC), dout over [t0, t0+2*VEC)
     float xw[3 * VEC], g[2 * VEC], v0[VEC], v1[VEC], v2[VEC], g0[VEC], g1[VEC];
-    if constexpr (AL) {
+    if constexpr (FORM == CF_ELEMENTS) {
+      load_elements_or_zero<T, VEC>(xr, t0 - VEC, p.len, v0);
+      load_elements_or_zero<T, VEC>(xr, t0, p.len, v1);
+      load_elements_or_zero<T, VEC>(xr, t0 + VEC, p.len, v2);
+      load_elements_or_zero<T, VEC>(gr, t0, p.len, g0);
+      load_elements_or_zero<T, VEC>(gr, t0 + VEC, p.len, g1);
+    } else if constexpr (FORM == CF_ALIGNED) {
       load_vec_or_zero<T, VEC>(xr, t0 - VEC, p.len, v0);
       load_vec_or_zero<T, VEC>(xr, t0, p.len, v1);
       load_vec_or_zero<T, VEC>(xr, t0 + VEC, p.len, v2);
@@ -363,7 +393,8 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cf_kernel(const ConvPar
 #pragma unroll
       for (int m = 0; m < TAPS; ++m) dwrev[m] = __builtin_fmaf(g[i], xw[VEC + i - m], dwrev[m]);
     }
-    if constexpr (AL) store_vec<T, VEC>(dxr, t0, dx);
+    if constexpr (FORM == CF_ALIGNED) store_vec<T, VEC>(dxr, t0, dx);
+    else if constexpr (FORM == CF_ELEMENTS) store_run<T, VEC>(dxr, t0, p.len, false, dx);
     else store_any<T, VEC>(dxr, t0, p.len, dx);
   }
   }
@@ -961,8 +992,11 @@ static int conv_fwd_typed(const ConvParams &p, int layout, bool vec_ok, hipStrea
     if (p.len % VEC == 0) CONV_LAUNCH(conv_fwd_tr_kernel, CONV_T_AL(true), dim3((unsigned)blocks), dim3(CONV_TR_FWD_THREADS));
     else CONV_LAUNCH(conv_fwd_tr_kernel, CONV_T_AL(false), dim3((unsigned)blocks), dim3(CONV_TR_FWD_THREADS));
   } else if (p.K <= CONV_TAPS && !channels_last) {
-    if (vec_ok && p.len % VEC == 0) CONV_LAUNCH(conv_fwd_cf_kernel, CONV_T_AL(true), dim3(p.batch * p.chans), dim3(CONV_THREADS));
-    else CONV_LAUNCH(conv_fwd_cf_kernel, CONV_T_AL(false), dim3(p.batch * p.chans), dim3(CONV_THREADS));
+    switch (conv_cf_form<T>(p.len, vec_ok)) {
+      case CF_ALIGNED: CONV_LAUNCH(conv_fwd_cf_kernel, CONV_T_AL(CF_ALIGNED), dim3(p.batch * p.chans), dim3(CONV_THREADS)); break;
+      case CF_ANY: CONV_LAUNCH(conv_fwd_cf_kernel, CONV_T_AL(CF_ANY), dim3(p.batch * p.chans), dim3(CONV_THREADS)); break;
+      default: CONV_LAUNCH(conv_fwd_cf_kernel, CONV_T_AL(CF_ELEMENTS), dim3(p.batch * p.chans), dim3(CONV_THREADS));
+    }
   } else if (p.K <= CONV_TAPS && channels_last) {
     const int strips = (p.len + CONV_CL_STRIP - 1) / CONV_CL_STRIP;
     constexpr int VECF = CONV_CL_FWD_BYTES / sizeof(T);
@@ -1003,8 +1037,11 @@ static int conv_bwd_typed(const ConvParams &p, int layout, bool vec_ok, float *d
     const dim3 grid(q.whole_batch ? p.chans : p.batch * p.chans);
     {
       const ConvParams &p = q;
-      if (vec_ok && p.len % VEC == 0) CONV_LAUNCH(conv_bwd_cf_kernel, CONV_T_AL(true), grid, dim3(CONV_THREADS));
-      else CONV_LAUNCH(conv_bwd_cf_kernel, CONV_T_AL(false), grid, dim3(CONV_THREADS));
+      switch (conv_cf_form<T>(p.len, vec_ok)) {
+        case CF_ALIGNED: CONV_LAUNCH(conv_bwd_cf_kernel, CONV_T_AL(CF_ALIGNED), grid, dim3(CONV_THREADS)); break;
+        case CF_ANY: CONV_LAUNCH(conv_bwd_cf_kernel, CONV_T_AL(CF_ANY), grid, dim3(CONV_THREADS)); break;
+        default: CONV_LAUNCH(conv_bwd_cf_kernel, CONV_T_AL(CF_ELEMENTS), grid, dim3(CONV_THREADS));
+      }
     }
     if (q.whole_batch) {
       SSM_CHECK_LAUNCH("ssm_conv1d_bwd");

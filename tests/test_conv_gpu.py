@@ -141,6 +141,12 @@ def test_rows_of_any_length_keep_to_themselves(dtype, length):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("length", [2, 5, 8, 253, 255, 257, 259])
+def test_rows_on_both_sides_of_an_access_per_element(dtype, length):
+    test_rows_of_any_length_keep_to_themselves(dtype, length)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(1, 1, 8), (2, 7, 16), (3, 8, 8), (1, 9, 136), (2, 129, 264), (1, 8193, 8), (5, 2047, 24)])
 def test_channels_last_strips_and_segments(dtype, shape):
     """Around the ends of the forward's strips of 8 steps and of the backward's time segments (8193 steps: 65 of two tiles).
