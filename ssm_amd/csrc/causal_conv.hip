@@ -272,20 +272,23 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_cl_kernel(const ConvPar
 }
 
 // The same forward for aligned rows: a thread takes a strip of 8 steps of its channels and requests all of its rows, and the
-// taps, at once.  Bound by memory where the call is large, by the latency of one such chain where it is not: a thread that
-// walked four strips in turn, asking for the next one's rows ahead, took 22.6 us for 8 x 2048 x 1536 bf16, 13.9 for 4 x 2048 x
-// 1536, 8.0 for 4 x 2048 x 256 and 7.1 for 1 x 300 x 512, where this takes 22.0, 12.9, 5.4 and 3.9; strips of 4 steps 26.6 and 13.8,
-// of 16 21.6 and 14.1.
-constexpr int CONV_CL_ROWS_THREADS = 64, CONV_CL_ROWS_STRIP = 8;
-template <typename T, int TAPS>
+// taps, at once.  Bound by the latency of one such chain where the call is small: a thread that walked four strips in turn,
+// asking for the next one's rows ahead, took 8.4 us for 4 x 2048 x 256 bf16 and 15.2 for 4 x 2048 x 1536, where one strip takes
+// 5.9 and 13.4 (float32 7.7 / 6.3 and, 53 MB, 13.4 / 12.8).  Bound by memory where it is large, and there the walk does better, which
+// reads no row twice: 8 x 2048 x 1536 bf16 20.2 us against 21.8 in single strips, float32 33.9 against 37.2.  The line lies where
+// the walk is 1792 waves, 59 MB read and written in either type: float32 62 MB 12.7 / 14.4, 68 MB 14.9 / 15.4, bf16 60 MB 15.8 / 16.2,
+// 54 MB 15.5 / 14.9.
+// Single strips of 4 steps took 26.6 us for 8 x 2048 x 1536 bf16 and 13.8 for half of it, of 16 21.6 and 14.1.
+constexpr int CONV_CL_ROWS_THREADS = 64, CONV_CL_ROWS_STRIP = 8, CONV_CL_WALK = 4;
+template <typename T, int WALK, int TAPS>
 __global__ __launch_bounds__(CONV_CL_ROWS_THREADS) void conv_fwd_cl_rows_kernel(const ConvParams p) {
   constexpr int VEC = CONV_CL_FWD_BYTES / sizeof(T);
-  constexpr int HIST = TAPS - 1, S = CONV_CL_ROWS_STRIP;
-  const int cvecs = p.chans / VEC, strips = (p.len + S - 1) / S;
+  constexpr int HIST = TAPS - 1, S = CONV_CL_ROWS_STRIP, SPAN = S * WALK;
+  const int cvecs = p.chans / VEC, spans = (p.len + SPAN - 1) / SPAN;
   const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (size_t)p.batch * strips * cvecs) return;
-  const int c0 = (int)(gid % cvecs) * VEC, t_first = (int)((gid / cvecs) % strips) * S;
-  const size_t base = (size_t)(gid / ((size_t)cvecs * strips)) * p.len * p.chans + c0;
+  if (gid >= (size_t)p.batch * spans * cvecs) return;
+  const int c0 = (int)(gid % cvecs) * VEC, t_first = (int)((gid / cvecs) % spans) * SPAN;
+  const size_t base = (size_t)(gid / ((size_t)cvecs * spans)) * p.len * p.chans + c0;
   float wrev[VEC][TAPS], bias[VEC];
   load_taps_of<VEC, TAPS>(p.w, p.bias, c0, p.K, p.wide_taps, wrev, bias);
   const T *xb = reinterpret_cast<const T *>(p.x) + base;
@@ -302,16 +305,32 @@ __global__ __launch_bounds__(CONV_CL_ROWS_THREADS) void conv_fwd_cl_rows_kernel(
     }
   }
 #pragma unroll
-  for (int s = 0; s < S; ++s) {
-    float out[VEC];
+  for (int w = 0; w < WALK; ++w) {
+    const int t_begin = t_first + w * S;
+    Pack<T, VEC> next[S];
+    if (w + 1 < WALK) {
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-      float acc = bias[i];
-#pragma unroll
-      for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[i][m], to_f32(raw[HIST + s - m].v[i]), acc);
-      out[i] = p.silu ? silu_f32(acc) : acc;
+      for (int j = 0; j < S; ++j)
+        next[j] = *reinterpret_cast<const Pack<T, VEC> *>(xb + (size_t)min(t_begin + S + j, p.len - 1) * p.chans);
     }
-    if (t_first + s < p.len) store_vec<T, VEC>(yb + (size_t)(t_first + s) * p.chans, 0, out);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      float out[VEC];
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        float acc = bias[i];
+#pragma unroll
+        for (int m = 0; m < TAPS; ++m) acc = __builtin_fmaf(wrev[i][m], to_f32(raw[HIST + s - m].v[i]), acc);
+        out[i] = p.silu ? silu_f32(acc) : acc;
+      }
+      if (t_begin + s < p.len) store_vec<T, VEC>(yb + (size_t)(t_begin + s) * p.chans, 0, out);
+    }
+    if (w + 1 < WALK) {
+#pragma unroll
+      for (int j = 0; j < HIST; ++j) raw[j] = raw[S + j];
+#pragma unroll
+      for (int j = 0; j < S; ++j) raw[HIST + j] = next[j];
+    }
   }
 }
 
@@ -980,7 +999,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_fold_kernel(const float
     if (p.K <= 4) hipLaunchKernelGGL((kernel<targs, 4>), grid, block, 0, s, p);                        \
     else hipLaunchKernelGGL((kernel<targs, 5>), grid, block, 0, s, p);                                 \
   } while (0)
-#define CONV_T_AL(al) T, al
+#define CONV_T_AL(form) T, form
 
 template <typename T>
 static int conv_fwd_typed(const ConvParams &p, int layout, bool vec_ok, hipStream_t s) {
@@ -1003,9 +1022,11 @@ static int conv_fwd_typed(const ConvParams &p, int layout, bool vec_ok, hipStrea
     const size_t threads = (size_t)p.batch * strips * ((p.chans + VECF - 1) / VECF);
     const dim3 grid((unsigned)((threads + CONV_THREADS - 1) / CONV_THREADS));
     if (vec_ok && p.chans % VEC == 0) {
-      const size_t rows_threads = (size_t)p.batch * ((p.len + CONV_CL_ROWS_STRIP - 1) / CONV_CL_ROWS_STRIP) * (p.chans / VECF);
-      const dim3 rgrid((unsigned)((rows_threads + CONV_CL_ROWS_THREADS - 1) / CONV_CL_ROWS_THREADS));
-      CONV_LAUNCH(conv_fwd_cl_rows_kernel, T, rgrid, dim3(CONV_CL_ROWS_THREADS));
+      const auto threads_of = [&](int steps) { return (size_t)p.batch * ((p.len + steps - 1) / steps) * (p.chans / VECF); };
+      const auto blocks_of = [](size_t n) { return dim3((unsigned)((n + CONV_CL_ROWS_THREADS - 1) / CONV_CL_ROWS_THREADS)); };
+      const size_t walkers = threads_of(CONV_CL_ROWS_STRIP * CONV_CL_WALK), strips_all = threads_of(CONV_CL_ROWS_STRIP);
+      if (walkers >= (size_t)1792 * WAVE) CONV_LAUNCH(conv_fwd_cl_rows_kernel, CONV_T_AL(CONV_CL_WALK), blocks_of(walkers), dim3(CONV_CL_ROWS_THREADS));
+      else CONV_LAUNCH(conv_fwd_cl_rows_kernel, CONV_T_AL(1), blocks_of(strips_all), dim3(CONV_CL_ROWS_THREADS));
     } else CONV_LAUNCH(conv_fwd_cl_kernel, T, grid, dim3(CONV_THREADS));
   } else {
     const unsigned grid = (unsigned)min((size_t)65535 * 16, (total + CONV_THREADS - 1) / CONV_THREADS);

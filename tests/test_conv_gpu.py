@@ -167,6 +167,18 @@ def test_channels_last_strips_and_segments(dtype, shape):
         torch.testing.assert_close(a.double().cpu(), r, rtol=tol, atol=4e-6 * (B * L) ** 0.5)
 
 
+@pytest.mark.parametrize("dtype,chans", [(torch.float32, 1024), (torch.bfloat16, 2048), (torch.float16, 2056)])
+@pytest.mark.parametrize("length", [1023, 1025, 1031, 1033])
+def test_channels_last_strips_in_turn(dtype, chans, length):
+    """A call large enough that a thread walks four strips of 8 steps, around the ends of strips and of walks: the same bits as
+    its batch entries alone, whose threads take a strip each."""
+    x, w, b = (torch.randn(8, length, chans, device="cuda").to(dtype), torch.rand(chans, 4, device="cuda") - 0.5,
+               torch.randn(chans, device="cuda"))
+    y = _ops().dw_causal_conv_channels_last(x, w, b, activation="silu")
+    for i in (0, 7):
+        assert torch.equal(y[i], _ops().dw_causal_conv_channels_last(x[i:i + 1].contiguous(), w, b, activation="silu")[0])
+
+
 def test_config1_shape_bf16():
     """B=8, C=1536, L=2048, K=4, bf16, SiLU: forward + backward at full size against
     the oracle on a channel slice (channels are independent)."""
