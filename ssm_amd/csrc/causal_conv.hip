@@ -593,15 +593,17 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_walk_kernel(const Co
 // 31 here.  The sums for dw and dbias meet in LDS, one partial per (batch, segment of at least 64 steps).
 constexpr int CONV_CL_STEPS = 16, CONV_CL_WAVES = CONV_THREADS / WAVE, CONV_CL_TILE = CONV_CL_STEPS * CONV_CL_WAVES;
 
-// Time segments per batch row at most: four workgroups to a CU, between CONV_CL_SEGS and four times as many (1 x 7040 x 128 bf16
-// 15.7 us with 28 segments, 6.8 with 110; 2 x 6592 x 640 20.6 with 26, 16.7 with 52).
-__host__ __device__ inline int conv_cl_segs(int batch, int chans) {
-  const long long wgs = (long long)batch * ((chans + 127) / 128);
+// Time segments per batch row at most: four workgroups (of `block` channels each) to a CU, between CONV_CL_SEGS and four times as
+// many (1 x 7040 x 128 bf16 15.7 us with 28 segments, 6.8 with 110; 2 x 6592 x 640 20.6 with 26, 16.7 with 52).  Counted as if float32 had
+// as few workgroups as 16 bits, 3 x 3160 x 616 was cut into 50: forward and backward 35.2 us, of 25 segments 33.1.
+constexpr int CONV_CL_BLOCK = WAVE * CONV_CL_BWD_BYTES / 2;           // channels of a workgroup at most
+__host__ __device__ inline int conv_cl_segs(int batch, int chans, int block) {
+  const long long wgs = (long long)batch * ((chans + block - 1) / block);
   const int most = (int)(1024 / (wgs < 1024 ? wgs : 1024));
   return most < CONV_CL_SEGS ? CONV_CL_SEGS : most > 4 * CONV_CL_SEGS ? 4 * CONV_CL_SEGS : most;
 }
-__host__ __device__ inline int conv_cl_tiles_per_seg(int batch, int chans, int len) {
-  const int tiles = (len + CONV_CL_TILE - 1) / CONV_CL_TILE, segs = conv_cl_segs(batch, chans);
+__host__ __device__ inline int conv_cl_tiles_per_seg(int batch, int chans, int len, int block) {
+  const int tiles = (len + CONV_CL_TILE - 1) / CONV_CL_TILE, segs = conv_cl_segs(batch, chans, block);
   return (tiles + segs - 1) / segs;
 }
 
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_bwd_cl_kernel(const ConvPar
   __shared__ float part[CONV_CL_WAVES][SUMS * VEC][WAVE];
   const int wave = wave_id_uniform(), lane = lane_id();
   const int cblocks = (p.chans + WAVE * VEC - 1) / (WAVE * VEC);
-  const int seg_len = conv_cl_tiles_per_seg(p.batch, p.chans, p.len) * CONV_CL_TILE, nseg = (p.len + seg_len - 1) / seg_len;
+  const int seg_len = conv_cl_tiles_per_seg(p.batch, p.chans, p.len, WAVE * VEC) * CONV_CL_TILE, nseg = (p.len + seg_len - 1) / seg_len;
   const int cb = (int)(blockIdx.x % cblocks), seg = (int)((blockIdx.x / cblocks) % nseg), b = (int)(blockIdx.x / ((unsigned)cblocks * nseg));
   const int c0 = (cb * WAVE + lane) * VEC;
   const bool live = c0 < p.chans;
@@ -1072,7 +1074,7 @@ static int conv_bwd_typed(const ConvParams &p, int layout, bool vec_ok, float *d
     constexpr int VECB = CONV_CL_BWD_BYTES / sizeof(T);
     // (a strip's rows are addressed by 32-bit offsets)
     const bool dense = vec_ok && p.chans % VEC == 0 && (size_t)p.chans * sizeof(T) * CONV_CL_STEPS < ((size_t)1 << 31);
-    const int seg_len = dense ? conv_cl_tiles_per_seg(p.batch, p.chans, p.len) * CONV_CL_TILE : conv_cl_seg_len(p.len);
+    const int seg_len = dense ? conv_cl_tiles_per_seg(p.batch, p.chans, p.len, WAVE * VECB) * CONV_CL_TILE : conv_cl_seg_len(p.len);
     const int nseg = (p.len + seg_len - 1) / seg_len;
     const size_t vecs = (p.chans + VECB - 1) / VECB, walkers = (size_t)p.batch * nseg * vecs;
     const size_t blocks = dense ? (size_t)p.batch * nseg * ((vecs + WAVE - 1) / WAVE) : (walkers + CONV_THREADS - 1) / CONV_THREADS;
@@ -1163,8 +1165,8 @@ extern "C" int ssm_conv1d_fwd(const ssm_conv1d_fwd_args *a, void *hip_stream) {
 
 extern "C" size_t ssm_conv1d_bwd_workspace_bytes(int batch, int channels, int width) {
   if (batch <= 0 || channels <= 0 || width <= 0) return 0;
-  // one partial per batch row, or per (batch row, time segment) in the channels-last kernel
-  return (size_t)batch * ssm::conv_cl_segs(batch, channels) * channels * (width + 1) * sizeof(float);
+  // one partial per batch row, or per (batch row, time segment) in the channels-last kernel (float32 has no more segments than 16 bits)
+  return (size_t)batch * ssm::conv_cl_segs(batch, channels, ssm::CONV_CL_BLOCK) * channels * (width + 1) * sizeof(float);
 }
 
 extern "C" int ssm_conv1d_bwd(const ssm_conv1d_bwd_args *a, void *hip_stream) {
