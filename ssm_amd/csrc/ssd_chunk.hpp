@@ -177,7 +177,7 @@ struct SsdCarryParams {
   void *turned, *h_turned;       // REV: G and H as rows of 64 channels, (B, nc, H, N, 64): what ssd_dbc_kernel reads
   float *through;                // REV: (B, H, nc, dim / 256) partial sums of exp(cs_Q) <G, H>
   int heads, nchunks, chunk, nstate;
-  int run_chunks;                // REV: chunks that a workgroup writes; it carries the state through those in front of them as well
+  int runs;                      // REV: runs of chunks, a workgroup each; it carries the state through those in front of its own as well
 };
 
 // A float32 as its bfloat16, rounded to nearest, and the 16 bits that complete it: the operands of the matrix products and
@@ -216,9 +216,10 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) 
   constexpr int AHEAD = 8, PASS = 16;
   const int N = p.nstate, dim = SSD_P * N, per = dim >> 10, kn = N >> 4;
   // the workgroups with the most chunks in front of theirs start first
-  const int runs = REV ? (p.nchunks + p.run_chunks - 1) / p.run_chunks : 1;
-  const unsigned units = gridDim.x / (unsigned)runs, vid = REV ? blockIdx.x % units : blockIdx.x;
-  const int begin = REV ? (runs - 1 - (int)(blockIdx.x / units)) * p.run_chunks : 0, stop = REV ? min(begin + p.run_chunks, p.nchunks) : p.nchunks;
+  const unsigned units = gridDim.x / (unsigned)(REV ? p.runs : 1), vid = REV ? blockIdx.x % units : blockIdx.x;
+  const int run_at = REV ? p.runs - 1 - (int)(blockIdx.x / units) : 0;
+  const int begin = REV ? (int)((long long)run_at * p.nchunks / p.runs) : 0;
+  const int stop = REV ? (int)((long long)(run_at + 1) * p.nchunks / p.runs) : p.nchunks;
   const int part = (int)(vid % per), tid = part * 256 + (int)threadIdx.x;
   const size_t bh = vid / per;
   const int h = (int)(bh % p.heads);
@@ -310,10 +311,7 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(const SsdCarryParams p) 
 // 23.2, 21.2 in three (20.0 in six).  More runs gained nothing more there and cost up to twice the time where chunks are few; the
 // forward, which reads and writes less, gained nothing from any.
 inline int carry_units(const SsdDims &d) { return d.batch * d.heads * (SSD_P * d.nstate / 1024); }
-inline int carry_run(const SsdDims &d) {
-  const int runs = std::max(1, std::min(d.nchunks / 8, 256 / carry_units(d)));
-  return (d.nchunks + runs - 1) / runs;
-}
+inline int carry_runs(const SsdDims &d) { return std::max(1, std::min(d.nchunks / 8, 256 / carry_units(d))); }
 
 // ---------------------------------------------------------------------- scan
 

@@ -369,7 +369,7 @@ static int backward_launches(const SsdStatesParams &st, const SsdCarryParams &ca
     return SSM_ERR_LAUNCH;
   }
   hipLaunchKernelGGL((ssd_states_kernel<elem_t, Q, N, true>), units, block, 0, s, st);
-  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(carry_units(d) * ((d.nchunks + ca.run_chunks - 1) / ca.run_chunks))), block, 0, s, ca);
+  hipLaunchKernelGGL((ssd_carry_kernel<elem_t, true, true>), dim3((unsigned)(carry_units(d) * ca.runs)), block, 0, s, ca);
   const dim3 both(2 * units.x);
   if (dz.z) hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, true>), both, block, 0, s, dz, dx);
   else hipLaunchKernelGGL((ssd_grad_scans_kernel<elem_t, Q, N, false>), both, block, 0, s, dz, dx);
@@ -415,7 +415,7 @@ extern "C" int ssm_ssd_combined_bwd(const ssm_ssd_combined_bwd_args *a, void *hi
   st.x = a->dout; st.z = f.z; st.dy = ws + lay.dy; st.frag = kw + kept.Ctblk; st.dA2 = dA2; st.dtv = dtv; st.states = f32(lay.added);
   st.len = d.len; st.heads = d.heads; st.groups = d.groups; st.nchunks = d.nchunks;
   SsdCarryParams ca{};
-  ca.run_chunks = carry_run(d);
+  ca.runs = carry_runs(d);
   ca.added = f32(lay.added); ca.states = ws + lay.states; ca.turned = ws + lay.turned; ca.dA2 = dA2; ca.first = a->dfinal; ca.last = a->dinitial_states; ca.entering = kw + kept.states; ca.through = f32(lay.through);
   ca.low = const_cast<uint16_t *>(reinterpret_cast<const uint16_t *>(kw + kept.states_low)); ca.h_turned = ws + lay.h_turned;
   ca.heads = d.heads; ca.nchunks = d.nchunks; ca.chunk = d.chunk; ca.nstate = d.nstate;
