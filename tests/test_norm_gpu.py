@@ -57,6 +57,31 @@ def check(pair, tol, ptol=None):
             torch.testing.assert_close(got[k].float(), want[k].float(), **(ptol or tol))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,hidden", [(5001, 768), (5001, 704), (4097, 64), (2051, 1536), (1030, 4096), (517, 8192)])
+@pytest.mark.parametrize("residual,bias,is_rms", [(False, False, True), (True, True, False), (True, False, True)])
+def test_sums_over_rows_read_ahead(rows, hidden, dtype, residual, bias, is_rms):
+    """More rows than owners, so that each walks several and asks for the next one ahead: the gradients against float64 of the same
+    16-bit values.  Rows: one rounding of float32.  Weight and bias: sums of `rows` float32 terms of size about 1, whose rounding
+    errors (2^-24 of a partial sum each) add up like a random walk, at most a few times 2^-24 x rows."""
+    g = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, go = r(1, rows, hidden).to(dtype).requires_grad_(), r(1, rows, hidden).to(dtype)
+    w, b = (r(hidden) + 1.0).requires_grad_(), r(hidden).requires_grad_() if bias else None
+    res = r(1, rows, hidden).to(dtype).requires_grad_() if residual else None
+    leaves = [t for t in (x, w, b, res) if t is not None]
+    got = torch.autograd.grad(_ops().fused_layer_norm(x, w, b, residual=res, is_rms=is_rms, eps=1e-5), leaves, go)
+    wide = [t.detach().double().requires_grad_() for t in leaves]
+    v = wide[0] + wide[-1] if residual else wide[0]
+    v = v if is_rms else v - v.mean(-1, keepdim=True)
+    y = v * torch.rsqrt((v * v).mean(-1, keepdim=True) + 1e-5) * wide[1]
+    want = torch.autograd.grad(y + wide[2] if bias else y, wide, go.double())
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for t, a, e in zip(leaves, got, want):
+        tol = dict(rtol=eps, atol=1e-5) if t.dtype == dtype else dict(rtol=1e-5, atol=8 * 2.0 ** -24 * rows)
+        torch.testing.assert_close(a.double(), e, **tol)
+
+
 def test_upstream_layer_norm_prenorm():
     rec = fx.upstream("layer_norms", "layer_norm_prenorm")
     i = rec["inputs"]
