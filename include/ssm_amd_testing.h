@@ -5,7 +5,7 @@
  * `reserved` field.  The test suite also needs to run a chosen kernel where the library would pick another
  * (to compare two implementations of one operator on the same inputs) and to learn which kernel a call
  * took.  A second build of the same sources with -DSSM_TEST_HOOKS (libssm_amd_testhooks.so) reads the
- * `reserved` fields as the selectors below and exports one more function.  Nothing here has a counterpart
+ * `reserved` fields as the selectors below and exports three more functions.  Nothing here has a counterpart
  * in the reference and nothing here is part of the backend's interface.
  *
  *   ssm_scan_fwd_args.reserved        0 = automatic; 100 * steps-per-lane + states-per-LDS-pass (408, 808, 816);
@@ -44,6 +44,11 @@ extern "C" {
  * bit 4 the same with its chunks side by side.
  * Resets on read. */
 int ssm_ssd_mfma_launches(void);
+
+/* Channels that a call with time-varying projections gives to a workgroup where its rows go many to a workgroup: the forward's
+ * kernel for any number of channels, the backward's wave-per-row kernel (0: the call's shape is not for that). */
+int ssm_scan_fwd_rows_per_workgroup(int batch, int dim, int seqlen, int b_groups, int c_groups);
+int ssm_scan_bwd_rows_per_workgroup(int batch, int dim, int seqlen, int nstate, int b_groups, int c_groups);
 
 #ifdef __cplusplus
 }

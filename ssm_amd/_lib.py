@@ -410,6 +410,8 @@ PLAIN_SYMBOLS = {
 # exported by the test-hooks build only (include/ssm_amd_testing.h)
 HOOKS_SYMBOLS = {
     "ssm_ssd_mfma_launches": (C.c_int, []),
+    "ssm_scan_fwd_rows_per_workgroup": (C.c_int, [C.c_int] * 5),
+    "ssm_scan_bwd_rows_per_workgroup": (C.c_int, [C.c_int] * 6),
 }
 HOOKS_LIB_PATH = LIB_PATH.with_name("libssm_amd_testhooks.so")
 

@@ -21,6 +21,7 @@
 // There are no atomics: results are bit-reproducible.
 #include "common.hpp"
 
+#include <numeric>
 #include <type_traits>
 #include <utility>
 
@@ -859,12 +860,7 @@ static BwdPlan plan_bwd(int batch, int dim, int len, int nstate, int b_kind, int
   const int nchunks = (len + BW_T - 1) / BW_T;
   const bool may_split = nchunks > 1 && !in_turn;
   const double all = (double)batch * dim;
-  int span = per_b;                      // channels that share a B group and a C group
-  for (int r = per_c; r;) {
-    const int q = span % r;
-    span = r;
-    r = q;
-  }
+  const int span = std::gcd(per_b, per_c);
   pl.span = span;
   // Side by side, the chunks fill the chip better and cost a launch more (scan_bwd_maps.hpp), us.
   const double maps = 7.0 + 0.5 * all * nchunks / 256;
@@ -965,6 +961,12 @@ extern "C" size_t ssm_scan_bwd_workspace_bytes(int batch, int dim, int seqlen, i
   if (c_kind == SSM_PROJ_BGNL && (c_groups <= 0 || dim % c_groups)) return 0;
   return plan_bwd(batch, dim, seqlen, nstate, b_kind, c_kind, b_groups, c_groups).total;
 }
+
+#ifdef SSM_TEST_HOOKS
+extern "C" int ssm_scan_bwd_rows_per_workgroup(int batch, int dim, int seqlen, int nstate, int b_groups, int c_groups) {
+  return ssm::plan_bwd(batch, dim, seqlen, nstate, SSM_PROJ_BGNL, SSM_PROJ_BGNL, b_groups, c_groups).fast_rows;
+}
+#endif
 
 namespace ssm {
 template <typename io_t>

@@ -3,6 +3,8 @@
 // instantiated per activation dtype in scan_fwd_{f32,bf16,f16}.hip.
 #include "scan_fwd_fast.hpp"
 
+#include <numeric>
+
 namespace ssm {
 
 extern template int scan_fwd_dispatch<float>(const ScanFwdParams &, int, int, hipStream_t);
@@ -68,6 +70,13 @@ static bool valid_kind(int k) { return k == SSM_PROJ_DN || k == SSM_PROJ_BDN || 
 }  // namespace ssm
 
 extern "C" int ssm_scan_chunk_len(void) { return 512; }
+
+#ifdef SSM_TEST_HOOKS
+extern "C" int ssm_scan_fwd_rows_per_workgroup(int batch, int dim, int seqlen, int b_groups, int c_groups) {
+  const int span = std::gcd(dim / b_groups, dim / c_groups);
+  return ssm::scan_fwd_rows_per_wg(batch, dim / span, span, (seqlen + ssm::FAST_T - 1) / ssm::FAST_T);
+}
+#endif
 
 extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   using namespace ssm;
@@ -136,12 +145,7 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
   const bool in_turn = tune >= 200000;      // a selector of 200000 + v: variant v, a row's chunks in turn however few the rows are
   if (in_turn) tune -= 100000;
   const bool half = a->io_dtype != SSM_F32;
-  p.span = per_b;
-  for (int r = per_c; r;) {                 // channels that share a group of B and one of C
-    const int q = p.span % r;
-    p.span = r;
-    r = q;
-  }
+  p.span = std::gcd(per_b, per_c);          // channels that share a group of B and one of C
   const int spans = a->dim / p.span, nchunks = (a->seqlen + FAST_T - 1) / FAST_T;
   p.split = !in_turn && scan_fwd_splits(rows_total, a->seqlen, !const_ok, p.span >= ROWS_MIN, half, p.ragged);
   if (tune == 0 && fast_ok) {

@@ -404,6 +404,37 @@ def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype
         torch.testing.assert_close(f, r, **tol, msg=lambda m, k=k: f"grad {k}: {m}")
 
 
+@pytest.mark.parametrize("batch,dim,length,dtype,rows", [
+    (8, 3072, 40, torch.float16, 96), (8, 3060, 40, torch.bfloat16, 96), (8, 3040, 520, torch.bfloat16, 96),
+    (8, 3072, 520, torch.float32, 96), (8, 616, 131, torch.float32, 20)])
+def test_the_largest_workgroups(batch, dim, length, dtype, rows):
+    """Workgroups of as many channels as fit (the most turns and LDS), a group's last one with fewer: against the general kernel."""
+    from ssm_amd import _lib
+    assert _lib.load_test_hooks().ssm_scan_bwd_rows_per_workgroup(batch, dim, length, 16, 1, 1) == rows
+    test_any_number_of_channels_to_a_workgroup(batch, dim, length, 16, dtype, dtype, (1, 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_groups_that_share_runs_of_four_channels(dtype):
+    """B and C in groups that have four channels in common: no run of eight that a wave-per-row kernel takes.  Against float64
+    autograd through the oracle."""
+    batch, dim, length, nstate = 2, 60, 1065, 16
+    inp = make_inputs(length, batch, dim, length, nstate, dtype=dtype, groups=1)
+    g = torch.Generator().manual_seed(5)
+    inp["B"], inp["C"] = (torch.randn(batch, n, nstate, length, generator=g).to(dtype) for n in (5, 3))
+    go = torch.randn(batch, dim, length, generator=g).to(dtype)
+    got = _bwd_direct(inp, go, None, 0)
+    w = {k: v.double().requires_grad_() for k, v in inp.items()}
+    out = O.selective_scan(w["u"], w["delta"], w["A"], w["B"], w["C"], D=w["D"], z=w["z"], dt_bias=w["dt_bias"], softplus=True,
+                           acc=torch.float64)
+    (out * go.double()).sum().backward()
+    for k, f in zip(NAMES, got):
+        scale = float(w[k].grad.abs().max())
+        half = k in ("u", "delta", "z") and dtype != torch.float32
+        tol = dict(rtol=2e-2, atol=4e-3 * scale) if half else dict(rtol=1e-3, atol=1e-4 * scale)
+        torch.testing.assert_close(f.double().cpu(), w[k].grad, **tol, msg=lambda m, k=k: f"grad {k}: {m}")
+
+
 @pytest.mark.parametrize("batch,dim,length,groups,neighbours", [
     (8, 1536, 64, 1, 3), (8, 1536, 2048, 1, 3), (5, 928, 1472, 1, 2), (7, 1248, 139, 1, 3), (6, 1600, 1541, 1, 2),
     (2, 752, 204, 1, 1), (3, 912, 3072, 1, 1), (4, 192, 520, 4, 1), (8, 616, 131, 1, 1)])

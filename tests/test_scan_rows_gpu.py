@@ -148,6 +148,16 @@ def test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype
         torch.testing.assert_close(a.double().cpu(), b, rtol=tol["rtol"], atol=tol["atol"] * scale, msg=lambda m: f"{what}: {m}")
 
 
+@pytest.mark.parametrize("batch,dim,length,nstate,dtype,bc_dtype,groups,rows", [
+    (8, 3072, 265, 16, torch.float32, torch.float32, (1, 1), 96), (8, 3072, 277, 15, torch.bfloat16, torch.float32, (1, 1), 96),
+    (16, 1440, 64, 16, torch.float16, torch.float16, (1, 1), 90), (9, 2720, 264, 16, torch.float32, torch.float32, (2, 1), 49)])
+def test_the_largest_workgroups(batch, dim, length, nstate, dtype, bc_dtype, groups, rows):
+    """Workgroups of as many channels as fit (the most rows to a wave and LDS), and of a size that leaves one over."""
+    from ssm_amd import _lib
+    assert _lib.load_test_hooks().ssm_scan_fwd_rows_per_workgroup(batch, dim, length, *groups) == rows
+    test_any_number_of_channels_to_a_workgroup(batch, dim, length, nstate, dtype, bc_dtype, groups)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("length,nstate", [(403, 1), (403, 15), (403, 16), (1031, 3), (200, 9), (200, 16)])
 def test_an_infinite_step_stays_where_it_is(length, nstate, dtype):
