@@ -12,8 +12,8 @@
  *                                     1616, 2416, 3216, 4816 = 816 with two, three, four, six channels per wave;
  *                                     100000 + v = variant v of the kernel for grouped time-varying projections
  *                                     (131041: the row-per-wave kernel; 131042: that for projections constant in time;
- *                                     113082, 111162, 122121, 121081: the kernel for any number of channels to a
- *                                     workgroup with 24, 8, 48, 16);
+ *                                     111120: the kernel for any number of channels to a workgroup; 113082, 111162, 122121,
+ *                                     121081: that with 24, 8, 48, 16);
  *                                     200000 + v = the same with a row's chunks one after the other however few rows
  *   ssm_scan_bwd_args.reserved        1 = the general kernel also where a wave-per-row kernel applies (grouped
  *                                     projections, projections of their own per channel, or projections that are

@@ -204,7 +204,7 @@ extern "C" int ssm_scan_fwd(const ssm_scan_fwd_args *a, void *hip_stream) {
       SSM_REQUIRE(per_wg == 1 || whole16, SSM_ERR_BAD_KIND, "ssm_scan_fwd: selector %d is for aligned rows of whole 16-step runs", tune);
       SSM_REQUIRE(v == 31041 || (a->seqlen >= 4 && a->seqlen < (1 << 28)), SSM_ERR_BAD_SHAPE,
                   "ssm_scan_fwd: selector %d is for rows of 4 to 2^28 - 1 steps", tune);
-      p.rows_per_wg = per_wg;
+      p.rows_per_wg = v == ROWS_VARIANT ? scan_fwd_rows_per_wg(a->batch, spans, p.span, nchunks) : per_wg;
     }
     const bool bc32 = a->bc_dtype == SSM_F32;
     switch (a->io_dtype) {
