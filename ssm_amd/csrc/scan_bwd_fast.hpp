@@ -1,5 +1,5 @@
 // Selective scan, backward: the kernel for the common call shape (time-varying grouped B and C,
-// at most 16 states, activations of any supported type; rows of any length and start in its RAGGED form).  Included by
+// at most 16 states, activations of any supported type; rows of at least 8 steps, of any length and start).  Included by
 // scan_bwd.hip after ScanBwdParams.
 //
 // A wavefront owns one row at a time and walks its states one after the other, lanes split
@@ -18,7 +18,8 @@
 // atomics, which take the 64 lanes one by one on this chip, eight times the whole kernel.)
 // Every element is added to by one wave at a time in a fixed order, so results are the same bits
 // on every run.  The tile goes to memory once per chunk as one partial per workgroup.
-// 128 KB of LDS: one workgroup of 16 waves per CU, four waves per SIMD.
+// 128 KB of LDS for the slabs and the tiles, 4 to dump what touch_lines reads, 200 bytes for every row: one workgroup of 16
+// waves per CU, four waves per SIMD.
 #pragma once
 #include "scan_fwd_fast.hpp"
 

@@ -29,6 +29,10 @@ extern template int scan_fwd_fast_dispatch<f16_t, float>(const ScanFwdParams &, 
 //   1024 x 2045 31.1 / 26.6, 512 x 8111 71 / 84, 768 x 8111 104 / 85.
 //   Few channels to a group (a row per wave in turn): 1024 x 2048 float32 71 / 48, bf16 29 / 27, 1536 x 2048 38.5 / 37.9.
 //   Constant projections: 256 x 2048 18.4 / 10.2, 512 x 8192 68 / 43, 512 x 1024 10.6 / 10.9, 1024 x 4096 41 / 43.
+// (A single chunk has none beside it: up to those rows such a call goes a row to a wave, of which the x 504 figures are.)
+// Over 1200 random grouped calls (1 to 8 x 12 to 2560 channels, 256 to 6000 steps, 1 to 16 states) what is chosen here and below
+// took 1.9 % more in the mean than the fastest of the kernels that could have been, 6 % or less in nine calls of ten, 17 % in 99 of
+// 100, 42 % at worst (2 x 402 x 2176 bf16: 39.8 side by side, 28.1 a row to a wave in turn).
 static bool scan_fwd_splits(size_t rows, int len, bool varying, bool grouped, bool half, bool ragged) {
   const int chunks = (len + FAST_T - 1) / FAST_T;
   if (!varying) return chunks > 1 && rows <= (chunks > 2 ? 512 : 384);

@@ -174,7 +174,7 @@ struct SsdCarryParams {
   const float *first;            // (B, H, P, N): the state before the first chunk (after the last one), or null
   float *last;                   // (B, H, P, N) or null
   const void *entering;          // REV: the forward's states H
-  void *turned, *h_turned;       // REV: G and H as rows of 64 channels, (B, nc, H, N, 64): what ssd_dbc_kernel reads
+  void *turned, *h_turned;       // REV: G and H as rows of 64 channels, (B, nc, H, N, 64): what ssd_dbc_dt_kernel reads
   float *through;                // REV: (B, H, nc, dim / 256) partial sums of exp(cs_Q) <G, H>
   int heads, nchunks, chunk, nstate;
   int runs;                      // REV: runs of chunks, a workgroup each; it carries the state through those in front of its own as well
